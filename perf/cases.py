@@ -68,28 +68,28 @@ def _step(name, model, layers, prompts=0, tokens=(0, 0), past=(0, 0), decodes=0,
 def listed():
     return [
         # one analyst chatting: the latency of a token of the agent model
-        _step("chat token, 1 sequence", "llama3-8b", 16, decodes=1, context=(777, 777)),
+        _step("chat token of 1 sequence", "llama3-8b", 16, decodes=1, context=(777, 777)),
         # many investigations at once, a few turns into their contexts
-        _step("decode, 96 investigations", "llama3-8b", 16, decodes=96, context=(500, 2900)),
+        _step("decode of 96 investigations", "llama3-8b", 16, decodes=96, context=(500, 2900)),
         # the small triage model with the eight-bit cache that doubles its capacity
-        _step("decode, 23 triages, fp8 cache", "llama3.2-1b", 16, decodes=23,
+        _step("decode of 23 triages with fp8 cache", "llama3.2-1b", 16, decodes=23,
               context=(300, 5000), cache="fp8"),
         # first prompts of new investigations, packed into one batch
         _step("8 first prompts", "llama3-8b", 8, prompts=8, tokens=(400, 1100)),
         # one portion of a long log pasted behind an already long context
-        _step("long context, one portion", "llama3-8b", 4, prompts=1, tokens=(4096, 4096),
+        _step("one portion behind a long context", "llama3-8b", 4, prompts=1, tokens=(4096, 4096),
               past=(22000, 22000)),
         # tool results of three investigations join a running batch of a routed model
         _step("tool results beside decodes", "mixtral-8x7b", 2, prompts=3, tokens=(350, 650),
               past=(800, 2200), decodes=41, context=(700, 2600)),
         # routed decoding: every expert's weights for a few tokens each
-        _step("routed decode, 32 sequences", "mixtral-8x7b", 2, decodes=32,
+        _step("routed decode of 32 sequences", "mixtral-8x7b", 2, decodes=32,
               context=(600, 2500)),
         # a prompt batch of a layer-listed decoder: window attention, recurrences, experts
-        _step("4 prompts, recurrent and routed", "kikalix-4096", 4, prompts=4,
+        _step("4 prompts recurrent and routed", "kikalix-4096", 4, prompts=4,
               tokens=(1900, 2048)),
         # the same design with many narrow experts, decoding
-        _step("recurrent decode, 64 sequences", "kikalix-2048", 4, decodes=64,
+        _step("recurrent decode of 64 sequences", "kikalix-2048", 4, decodes=64,
               context=(1500, 2500)),
         # latent attention: prompt portions behind a context beside decoding sequences
         _step("latent portions beside decodes", "senotar-4096", 4, prompts=2,
