@@ -298,6 +298,9 @@ def _prepare_step(case, seed):
             del os.environ["AURORA_KV_FP8"]
         else:
             os.environ["AURORA_KV_FP8"] = before
+    # rows of a captured batch that no sequence fills decode token 0, not what an engine of
+    # another vocabulary may have left in the pinned memory
+    engine._host_i64.zero_()
     vocab, seqs, nexts = _sizes(case["model"])[1], [], []
     for i, ((past, new), p) in enumerate(zip(portions, pages)):
         ids = _tokens(seed, f"ids{i}", past + max(new, DECODE_CYCLE), vocab).tolist()
