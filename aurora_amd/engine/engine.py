@@ -221,7 +221,8 @@ class LLMEngine:
             self._scratch_page = self.kv.alloc(1)[0]
             self._scratch_slot = self._scratch_page * self.kv.page_size
             maxb = self._BUCKETS[-1]
-            self._host_i64 = torch.empty(maxb, dtype=torch.int64, pin_memory=True)
+            # zeros: rows that no sequence has filled yet are idle rows' token ids
+            self._host_i64 = torch.zeros(maxb, dtype=torch.int64, pin_memory=True)
             self._host_i32 = torch.empty(maxb, 4, dtype=torch.int32, pin_memory=True)
             self._host_bt = torch.full((maxb, mp), self._scratch_page,
                                        dtype=torch.int32, pin_memory=True)
@@ -764,7 +765,8 @@ class LLMEngine:
             self._scratch_page = self.kv.alloc(1)[0]
             self._scratch_slot = self._scratch_page * self.kv.page_size
             maxb = self._BUCKETS[-1]
-            self._host_i64 = torch.empty(maxb, dtype=torch.int64, pin_memory=True)
+            # zeros: rows that no sequence has filled yet are idle rows' token ids
+            self._host_i64 = torch.zeros(maxb, dtype=torch.int64, pin_memory=True)
             self._host_i32 = torch.empty(maxb, 4, dtype=torch.int32, pin_memory=True)
             self._host_bt = torch.full((maxb, mp), self._scratch_page,
                                        dtype=torch.int32, pin_memory=True)
