@@ -1,24 +1,33 @@
 // Flash-style causal prefill attention over the paged KV cache (gfx950).
 //
-// MFMA structure (CDNA4, v_mfma_f32_32x32x16_bf16):
-//  * swapped QK^T — compute S^T = mfma(A=K-tile, B=Q^T-tile) so each lane
-//    owns ONE q column (q = lane&31) and the softmax row-reduce is
-//    per-lane over registers + one shfl_xor(32) with its half-wave partner
-//    (no cross-lane softmax, no P staging through LDS);
-//  * P -> PV A-fragments in-register via bf16 packing + v_permlane32_swap
-//    (the cvt_pk/permlane redistribution idiom);
-//  * K tile staged in LDS row-major with the ((row&15)<<4) XOR byte-swizzle
-//    (ds_read_b128 would otherwise be up-to-16-way bank-conflicted at
-//    D=128); V staged TRANSPOSED [D][KVBLK+8] so the PV B-fragment read is
-//    a contiguous 16-B ds_read per lane;
-//  * O accumulates in registers (col d = lane&31 per d-tile); the epilogue
-//    transposes through LDS so global stores are coalesced 16-B rows.
+// A wave owns 32 query rows of one head and computes S^T = K Q^T and O^T = V^T P^T
+// (v_mfma_f32_32x32x16_bf16), so a lane owns one query row: maxima, sums and the
+// rescaling of O are its own numbers and nothing of the softmax goes through LDS.
+//  * P needs no exchange either: an accumulator of S^T holds keys 4 half + {0..3, 8..11}
+//    of every 16, and V^T is read with its keys in just that order, four rows at a
+//    time, by the transposing ds_read_b64_tr_b16.
+//  * K and V tiles of 64 keys lie in LDS as they do in the cache, filled by
+//    direct-to-LDS loads (an 8-bit cache goes through registers) into a ring of three
+//    tiles: one barrier a tile, and a tile has a whole tile's computation to arrive.
+//    16-byte units are XOR-swizzled by row, K's so that 16 rows of a column and V's so
+//    that 4 neighbouring rows of 32 columns spread over the banks.
+//  * The scores of the next 32 keys are computed among the exponentials of the current
+//    ones, so the matrix cores and the vector unit work side by side within a wave.
+//  * Weights are taken against a reference that need not be the maximum: it moves, and
+//    O is rescaled, only when a score exceeds it by PRE_SLACK powers of two.
 //
-// Geometry: 8 waves/WG (512 threads); the WG covers HG = min(G, 4) query
-// heads of ONE kv head x (8/HG)*32 query rows, so every staged K/V tile
-// feeds 8 waves of MFMA (GQA heads share the stage — staging bandwidth was
-// the 156-TF bound of the 4-wave/1-head structure).  KV tiles of 64 keys,
-// two 32-key MFMA steps each.
+// What bounds it: 4096 rows behind 22000, 32 heads of 128 on 8 cached ones, keep the matrix
+// units busy 54% of the cycles and the vector unit 50%; the clock falls to 1.9 GHz under
+// them. 4135 us before (values transposed by 2-byte stores, nothing in flight, O rescaled
+// through LDS), now 1480 us = 1090 TF/s; 4 x 2048 fresh rows 712 and 157 us = 877 TF/s;
+// 8 x 800 fresh 230 and 74 us; heads of 64, 4 x 2048, 372 and 98 us; 8-bit cache, 2 x 2048
+// behind 4000, 1070 and 363 us. Tried and slower: the values of a step delayed into the next
+// one's exponentials (registers spill: 887 TF/s), a raised wave priority for the values.
+//
+// Geometry: 8 waves, HG = min(G, 4) query heads of ONE kv head x (8/HG)*32 query rows,
+// so a staged tile serves all of them. Workgroups run through the head groups first:
+// neighbours lie on different XCDs, and the workgroups of one XCD read the same heads'
+// keys.
 // BIAS adds a per-head distance penalty, linear, logarithmic or none, and a sliding
 // window or chunks of positions (tiles and MFMA steps wholly outside of what a wave
 // sees are skipped), lets keys and values differ in width, and writes scaled columns
@@ -32,18 +41,19 @@
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
+#include <type_traits>
+
 #define CUR_STREAM c10::hip::getCurrentHIPStream().stream()
 
-typedef __attribute__((ext_vector_type(4))) float f32x4;
-
-DEVINL unsigned int pack2_bf16(float lo, float hi) {
-  return ((unsigned int)f32_to_bf16(hi) << 16) | f32_to_bf16(lo);
-}
-
-#define LN2 0.69314718f  // the hardware's logarithm has base 2
+#define LOG2E 1.44269504f
+#define PRE_KEYS 64     // keys per tile
+#define PRE_STAGES 3    // tiles in LDS
+#define PRE_SLACK 10.f  // weights stay below 2^PRE_SLACK
 enum { NO_BIAS = 0, LINEAR_BIAS = 1, LOG_BIAS = 2, FLAT_BIAS = 3 };
 enum { PLAIN = 0, GATED = 1, TAILED = 2, TURNED = 3 };
-#define TURN_STRIDE 40  // row stride of a wave's 32 x 32 results in LDS
+
+typedef const __attribute__((address_space(1))) void* gptr_t;
+typedef __attribute__((address_space(3))) void* lptr_t;
 
 // shared last dimensions of the keys: key t's are row t, its own come first in kc
 struct KeyTail {
@@ -54,19 +64,80 @@ struct KeyTail {
 };
 
 union frag_u {
+  shortx8 s;
+  shortx4 h[2];
   unsigned int u[4];
   bf16x8 v;
 };
 
-template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA>  // HG = query heads per workgroup
+template <int N, typename F>
+DEVINL void static_for(F&& f) {
+  if constexpr (N > 0) {
+    static_for<N - 1>(f);
+    f(std::integral_constant<int, N - 1>{});
+  }
+}
+
+DEVINL unsigned int cvt2_bf16(float lo, float hi) {
+  const floatx2 f = {lo, hi};
+  const bf16x2 b = __builtin_convertvector(f, bf16x2);
+  return __builtin_bit_cast(unsigned int, b);
+}
+
+// Transposing reads of two V^T fragments, of each the halves HALF bytes apart. Written out
+// because the compiler puts a wait for all global loads in flight, the next tiles' among
+// them, before the builtin form. Nothing may touch v before await_values: no branch and
+// nothing that could run out of registers stands between the two.
+template <int AT, int HALF>
+DEVINL void read_values(shortx4 (&v)[4], unsigned a0, unsigned a1) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %4 offset:%6\n\t"
+      "ds_read_b64_tr_b16 %1, %4 offset:%7\n\t"
+      "ds_read_b64_tr_b16 %2, %5 offset:%6\n\t"
+      "ds_read_b64_tr_b16 %3, %5 offset:%7"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
+      : "v"(a0), "v"(a1), "n"(AT), "n"(AT + HALF)
+      : "memory");
+}
+
+DEVINL void await_values(shortx4 (&v)[4]) {
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])::"memory");
+}
+
+// Sequence and first row of the nb-th block of ``rows`` rows, counted through the
+// sequences; false past the last. A lane per sequence.
+DEVINL bool find_block(const int* cu, int S, int rows, int nb, int lane, int& seq, int& off) {
+  for (int s0 = 0; s0 < S; s0 += WAVE) {
+    const int s = s0 + lane;
+    const int n = s < S ? (cu[s + 1] - cu[s] + rows - 1) / rows : 0;
+    int end = n;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+      const int before = __shfl_up(end, d, WAVE);
+      if (lane >= d) end += before;
+    }
+    const unsigned long long past = __ballot(end > nb);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      seq = s0 + at;
+      off = (nb - __builtin_amdgcn_readlane(end - n, at)) * rows;
+      return true;
+    }
+    nb -= __builtin_amdgcn_readlane(end, WAVE - 1);
+  }
+  return false;
+}
+
+// HG: query heads per workgroup; PAGED: pages are whole tiles
+template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED>
 __global__ __launch_bounds__(512, 1) void prefill_kernel(
     const __hip_bfloat16* __restrict__ q,   // [T, qstride], heads D apart
     const void* __restrict__ kc,  // [NP, Hkv, P, D] bf16 | fp8 e4m3
     const void* __restrict__ vc,
     __hip_bfloat16* __restrict__ out,       // [T, ostride], heads dv apart
-    const int* __restrict__ block_seq,      // [NB] seq index of this q-block
+    const int* __restrict__ block_seq,      // [NB] seq index of this q-block, or null:
     const int* __restrict__ block_qoff,     // [NB] q-row offset within the seq
-    const int* __restrict__ cu_q,           // [S+1]
+    const int* __restrict__ cu_q, int S,    // [S+1]
     const int* __restrict__ block_tables,   // [S, MP]
     const int* __restrict__ ctx_lens,       // [S]
     int Hq, int Hkv, int P, int MP, float scale,
@@ -75,57 +146,61 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
     int chunk, const float* __restrict__ sink,  // [Hq], or null unless GATED
     const __hip_bfloat16* __restrict__ gate, long gstride,  // [T, gstride]
     KeyTail tail, HeadTurn turn) {
-  constexpr int KVB = 64;           // keys staged per tile
-  constexpr int NC = D / 16;        // Q^T fragments (MFMA K-chunks of QK^T)
-  constexpr int NDT = DV / 32;      // 32-wide d-tiles of O
-  constexpr int VROW = KVB + 8;     // padded V^T row length (elements)
-  // K-tile XOR swizzle mask: a row has D/8 16-B slots, so the swizzle may
-  // only permute within that many slots (at D=64, (row&15)<<4 would escape
-  // the 128-B row)
-  // (at D=192 a row is 1.5 times all banks: pairs of rows share a permutation)
-  constexpr int SWZ = D == 192 ? 7 : (D / 8) - 1;
-  constexpr int SWZ_SHIFT = D == 192 ? 1 : 0;
+  constexpr int NC = D / 16;        // Q^T fragments (MFMA K-chunks of K Q^T)
+  constexpr int NDT = DV / 32;      // 32-wide d-tiles of O^T
+  constexpr int KU = D / 8, VU = DV / 8;         // 16-B units of a key's, a value's row
+  constexpr int LK = PRE_KEYS * KU / 512, LV = PRE_KEYS * VU / 512;  // loads per thread
+  constexpr int KBYTES = PRE_KEYS * D * 2, STAGE = PRE_KEYS * (D + DV) * 2;
+  // units of K's row r are XORed with (r >> KSHIFT) & KMASK; a row of 192 is one and a
+  // half times 256 bytes, so pairs of rows share a permutation
+  constexpr int KMASK = D == 128 ? 15 : 7, KSHIFT = D == 192 ? 1 : 0;
   constexpr int QS = 8 / HG;          // 32-row q sub-blocks per WG
-  const int nb = gridDim.x - 1 - blockIdx.x;  // late rows see most keys: first
-  const int seq = block_seq[nb];
-  const int qoff = block_qoff[nb];
+  const int groups = Hq / HG;
+  // late rows see most keys: first
+  const int nb = gridDim.x / groups - 1 - blockIdx.x / groups;
+  const int lane = threadIdx.x % WAVE;
+  int seq, qoff;
+  if (block_seq) {
+    seq = block_seq[nb];
+    qoff = block_qoff[nb];
+  } else if (!find_block(cu_q, S, QS * 32, nb, lane, seq, qoff)) {
+    return;
+  }
   const int q_start = cu_q[seq];
   const int qlen = cu_q[seq + 1] - q_start;
   const int ctx = ctx_lens[seq];
   const int* bt = block_tables + (long)seq * MP;
 
   const int tid = threadIdx.x;
-  const int wave = tid / WAVE;
-  const int lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int col = lane & 31;   // q column owned by this lane (within wave's 32)
   const int half = lane >> 5;  // half-wave
   // wave -> (query head, q sub-block): heads vary fastest so the HG heads
   // of one sub-block sit on consecutive waves
-  const int h = blockIdx.y * HG + (wave % HG);
-  const int kvh = h / (Hq / Hkv);
+  const int h0 = blockIdx.x % groups * HG;
+  const int h = h0 + (wave % HG);
+  const int kvh = h0 / (Hq / Hkv);
   const int qsub = wave / HG;
 
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  short* kbuf = (short*)smem;                       // [KVB][D] XOR-swizzled
-  short* vtbuf = (short*)(smem + KVB * D * 2);      // [D][VROW] transposed
-  // [8][32] after K, V^T and the epilogue's four 32 x DV tiles
-  float* scratch = (float*)(smem + max(KVB * D * 2 + DV * VROW * 2, 256 * DV));
-  float* wsc = scratch + wave * 32;
+  const unsigned smem_at = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
 
-  // ---- Q fragments (B-operand of swapped QK^T): held for the whole block
+  // ---- Q fragments (B operand of K Q^T): held for the whole block. A scale that is
+  // not positive goes into them: the reference below compares unscaled scores
   const int qrow = qoff + qsub * 32 + col;  // local q row in this seq
   const bool qvalid = qrow < qlen;
   const long qbase = (q_start + (qvalid ? qrow : 0)) * qstride + (long)h * D;
+  const unsigned flip = scale < 0.f ? 0x80008000u : 0u;
+  const float c2 = scale == 0.f ? 1.f : fabsf(scale) * LOG2E;  // scores in units of log 2
   frag_u qf[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    if (qvalid) {
-      const shortx8 v =
-          *reinterpret_cast<const shortx8*>(q + qbase + c * 16 + half * 8);
-      qf[c].u[0] = ((const unsigned int*)&v)[0];
-      qf[c].u[1] = ((const unsigned int*)&v)[1];
-      qf[c].u[2] = ((const unsigned int*)&v)[2];
-      qf[c].u[3] = ((const unsigned int*)&v)[3];
+    bool there = qvalid && scale != 0.f;
+    if constexpr (EXTRA == TAILED) there = there && c * 16 + half * 8 < tail.own + tail.width;
+    if (there) {
+      qf[c].s = *reinterpret_cast<const shortx8*>(q + qbase + c * 16 + half * 8);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) qf[c].u[k] ^= flip;
     } else {
       qf[c].u[0] = qf[c].u[1] = qf[c].u[2] = qf[c].u[3] = 0u;
     }
@@ -133,7 +208,9 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
 
   const int q_abs = ctx - qlen + qrow;  // absolute position of this lane's q
   const bool has_sink = EXTRA == GATED || (BIAS && sink);
-  float m = has_sink ? sink[h] : -1e30f, l = has_sink ? 1.f : 0.f;
+  // reference and this lane's part of the sum (its half of the keys)
+  float m = has_sink ? fmaxf(sink[h] * LOG2E, -1e30f) : -1e30f;
+  float l = has_sink && half == 0 ? 1.f : 0.f;
   floatx16 o[NDT];
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt)
@@ -143,14 +220,14 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
   // keys needed by this q block: up to the last row's absolute position
   const int blk_rows = min(qlen - qoff, QS * 32);
   const int kend = min(ctx, ctx - qlen + qoff + blk_rows);
-  const int ntiles = (kend + KVB - 1) / KVB;
+  const int ntiles = (kend + PRE_KEYS - 1) / PRE_KEYS;
   // absolute position of the wave's first (smallest) q row
   const int q_abs_min = ctx - qlen + qoff + qsub * 32;
 
-  // this head's penalty per token of distance, or of ln(1 + rate * distance);
-  // first key any row here sees
-  const float slope = BIAS && BIAS != FLAT_BIAS
-                          ? slopes[h] * (BIAS == LOG_BIAS ? LN2 : 1.f) : 0.f;
+  // this head's penalty per token of distance, or per doubling of 1 + rate * distance,
+  // in units of log 2; first key any row here sees
+  const float slope = BIAS == LINEAR_BIAS ? slopes[h] * LOG2E
+                      : BIAS == LOG_BIAS  ? slopes[h] : 0.f;
   const float rate = BIAS == LOG_BIAS ? rates[h] : 0.f;
   const int win = BIAS && window > 0 ? window : 0x3fffffff;
   // first key a query at position x sees (negative: all)
@@ -158,288 +235,381 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
     const int lo = x - win + 1;
     return BIAS && chunk > 0 ? max(lo, x - x % chunk) : lo;
   };
-  const int tile0 = BIAS ? max(0, first_seen(ctx - qlen + qoff)) / KVB : 0;
+  const int tile0 = BIAS ? max(0, first_seen(ctx - qlen + qoff)) / PRE_KEYS : 0;
   const int lo = BIAS ? first_seen(q_abs) : 0;
-  const int lo_min = BIAS ? first_seen(q_abs_min) : 0;
   const int lo_max = BIAS ? first_seen(q_abs_min + 31) : 0;
+  // tiles that the wave's rows see; the first of its workgroup's where there are no rows
+  const bool rows = qoff + qsub * 32 < qlen;
+  const int first = rows && BIAS ? max(first_seen(q_abs_min), 0) / PRE_KEYS : tile0;
+  const int end = rows ? (min(kend, q_abs_min + 32) + PRE_KEYS - 1) / PRE_KEYS : tile0;
 
-  for (int tile = tile0; tile < ntiles; ++tile) {
-    const int kbase = tile * KVB;
-    // ---- stage K (swizzled) and V^T cooperatively: 512 threads
-    __syncthreads();
-    auto load8 = [&](const void* cache, long base) -> shortx8 {
-      if constexpr (FP8)
-        return fp8x8_to_bf16x8(
-            *reinterpret_cast<const u64b*>((const unsigned char*)cache + base));
-      else
-        return *reinterpret_cast<const shortx8*>((const __hip_bfloat16*)cache + base);
-    };
+  // ---- tiles. A thread's unit x of a tile is unit tid + 512 x in LDS and takes what the
+  // swizzle puts there. Pages are looked up a tile before the loads that need them (by
+  // vector loads: with a scalar one under way every wait for LDS is for all of it); nothing
+  // is computed from them until then, so nothing waits for them.
+  constexpr int NP = PAGED ? 1 : D == DV ? LK : LK + LV;
+  constexpr int EB = FP8 ? 1 : 2;  // bytes of a cached number
+  int page[NP];
+  auto key_column = [&](int x) {
+    const unsigned row = (tid + x * 512u) / KU, slot = (tid + x * 512u) % KU;
+    return (slot ^ ((row >> KSHIFT) & KMASK)) * 8;
+  };
+  auto value_column = [&](int x) {
+    const unsigned row = (tid + x * 512u) / VU, slot = (tid + x * 512u) % VU;
+    return (slot ^ (DV == 64 ? (row & 2) << 1 : (row & 3) << 2)) * 8;
+  };
+  auto unit_row = [&](int x) -> int {  // of K's units, then V's
+    return x < LK ? (tid + x * 512u) / KU : (tid + (x - LK) * 512u) / VU;
+  };
+  const unsigned per = 0xffffffffu / P;  // t / P without a division
+  auto page_of = [&](int t, int& in) {
+    int pg = __umulhi((unsigned)t, per);
+    in = t - pg * P;
+    if (in >= P) { in -= P; ++pg; }
+    return pg;
+  };
+  auto lookup = [&](int tile) {
+    if (tile >= ntiles) return;
+    int in;
+    if constexpr (PAGED) {
+      int at = page_of(tile * PRE_KEYS, in);
+      asm("" : "+v"(at));
+      page[0] = bt[at];
+    } else {
 #pragma unroll
-    for (int i = 0; i < KVB * (D > DV ? D : DV) / (512 * 8); ++i) {
-      const int c = tid + i * 512;
-      constexpr int W8 = (D > DV ? D : DV) / 8;
-      const int row = c / W8;
-      const int d0 = (c % W8) * 8;
-      const int t = kbase + row;
-      shortx8 kv8 = {0, 0, 0, 0, 0, 0, 0, 0};
-      shortx8 vv8 = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (t < ctx) {
-        const long slot = ((long)bt[t / P] * Hkv + kvh) * P + (t % P);
-        if constexpr (EXTRA == TAILED) {
-          const long key = (long)bt[t / P] * P + t % P;
-          if (d0 < tail.own)
-            kv8 = load8(kc, slot * tail.own + d0);
-          else if (d0 < D && d0 - tail.own < tail.width)
-            kv8 = load8(tail.rows, key * tail.stride + d0 - tail.own);
-        } else {
-          if (D >= DV || d0 < D) kv8 = load8(kc, slot * D + d0);
-        }
-        if (DV >= D || d0 < DV) vv8 = load8(vc, slot * DV + d0);
-      }
-      if (D >= DV || d0 < D) {
-        const int kb = (row * D * 2 + ((d0 * 2) ^ (((row >> SWZ_SHIFT) & SWZ) << 4))) / 2;
-        *reinterpret_cast<shortx8*>(kbuf + kb) = kv8;
-      }
-      if (DV >= D || d0 < DV) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) vtbuf[(d0 + j) * VROW + row] = vv8[j];
-      }
+      for (int x = 0; x < NP; ++x)
+        page[x] = bt[page_of(min(tile * PRE_KEYS + unit_row(x), ctx - 1), in)];
     }
-    __syncthreads();
-
-    // ---- two 32-key MFMA steps (waves skip steps beyond their causal bound)
-    const int wave_kend = min(kend, q_abs_min + 32);
+  };
+  // Where unit x comes from, handed to ``load``. Past the end the last key stands again.
+  // PAGED: the tile's place is a scalar and a thread's own offset is the same in all tiles
+  // but the last.
+  unsigned offset[2];  // of a thread's first unit of K and V; the others' rows follow
+  constexpr int KSTEP = 512 / KU, VSTEP = 512 / VU;
+  offset[0] = (unit_row(0) * D + key_column(0)) * EB;
+  offset[1] = (unit_row(LK) * DV + value_column(0)) * EB;
+  auto units = [&](int tile, auto load) {
+    if constexpr (PAGED) {
+      static_assert(512 % KU == 0 && KSTEP % 16 == 0 && VSTEP % 16 == 0);
+      int in;
+      page_of(tile * PRE_KEYS, in);
+      const unsigned row =
+          ((unsigned)__builtin_amdgcn_readfirstlane(page[0]) * Hkv + kvh) * P + in;
+      const char* kt = (const char*)kc + (u64b)row * (D * EB);
+      const char* vt = (const char*)vc + (u64b)row * (DV * EB);
+      if (tile * PRE_KEYS + PRE_KEYS <= ctx) {
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int ks = kbase + s * 32;  // absolute key base of this step
-      if (ks >= wave_kend) break;
-      if (BIAS && ks + 31 < lo_min) continue;  // before all that the wave sees
-      // S^T = K * Q^T : rows k, cols q
-      floatx16 st;
+        for (int x = 0; x < LK; ++x) load(x, kt + x * KSTEP * D * EB + offset[0]);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) st[r] = 0.f;
-      const int krow = s * 32 + col;  // this lane's A-row in the K tile
+        for (int x = 0; x < LV; ++x) load(LK + x, vt + x * VSTEP * DV * EB + offset[1]);
+      } else {
+        const int last = ctx - 1 - tile * PRE_KEYS;
 #pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        const int kb =
-            (krow * D * 2 +
-             (((c * 16 + half * 8) * 2) ^ (((krow >> SWZ_SHIFT) & SWZ) << 4))) / 2;
-        frag_u kf;
-        const shortx8 kv = *reinterpret_cast<const shortx8*>(kbuf + kb);
-        kf.u[0] = ((const unsigned int*)&kv)[0];
-        kf.u[1] = ((const unsigned int*)&kv)[1];
-        kf.u[2] = ((const unsigned int*)&kv)[2];
-        kf.u[3] = ((const unsigned int*)&kv)[3];
-        st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf.v, qf[c].v, st, 0, 0, 0);
+        for (int x = 0; x < LK; ++x)
+          load(x, kt + (unsigned)(min(unit_row(x), last) * D + key_column(x)) * EB);
+#pragma unroll
+        for (int x = 0; x < LV; ++x)
+          load(LK + x, vt + (unsigned)(min(unit_row(LK + x), last) * DV + value_column(x)) * EB);
       }
-      // ---- mask + scale (S^T reg r holds key row R = (r&3)+8*(r>>2)+4*half)
-      float p[16];
+    } else {
+      // a cache holds fewer than 2^32 rows: it fits the card
+      unsigned rows[NP], token[NP];
+#pragma unroll
+      for (int x = 0; x < NP; ++x) {
+        int in;
+        page_of(min(tile * PRE_KEYS + unit_row(x), ctx - 1), in);
+        rows[x] = ((unsigned)page[x] * Hkv + kvh) * P + in;
+        token[x] = (unsigned)page[x] * P + in;  // in a cache of one head
+      }
+#pragma unroll
+      for (int x = 0; x < LK; ++x) {
+        const unsigned d0 = key_column(x);
+        const char* src = (const char*)kc + ((u64b)rows[x] * D + d0) * EB;
+        if constexpr (EXTRA == TAILED) {
+          // columns past the tail's are not there: the queries hold zeros for them
+          const int past = (int)d0 - tail.own;
+          if (past < 0) src = (const char*)kc + ((u64b)rows[x] * tail.own + d0) * EB;
+          else if (tail.width > 0)
+            src = (const char*)(tail.rows + token[x] * tail.stride +
+                                (past < tail.width ? past : 0));
+          else src = (const char*)kc + (u64b)rows[x] * tail.own * EB;
+        }
+        load(x, src);
+      }
+#pragma unroll
+      for (int x = 0; x < LV; ++x)
+        load(LK + x, (const char*)vc + ((u64b)rows[NP - LV + x] * DV + value_column(x)) * EB);
+    }
+  };
+  auto issue = [&](int tile) {  // bf16: straight to LDS
+    char* st = smem + (tile % PRE_STAGES) * STAGE + wave * 64 * 16;
+    units(tile, [&](int x, const char* src) {
+      char* dst = st + (x < LK ? x * 512 * 16 : KBYTES + (x - LK) * 512 * 16);
+      __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)dst, 16, 0, 0);
+    });
+  };
+  u64b u8[LK + LV];
+  auto fetch8 = [&](int tile) {  // fp8: to registers, then (store8) converted to LDS
+    units(tile, [&](int x, const char* src) { u8[x] = *reinterpret_cast<const u64b*>(src); });
+  };
+  auto store8 = [&](int tile) {
+    char* st = smem + (tile % PRE_STAGES) * STAGE + tid * 16;
+#pragma unroll
+    for (int x = 0; x < LK + LV; ++x)
+      *reinterpret_cast<shortx8*>(st + (x < LK ? x * 512 * 16 : KBYTES + (x - LK) * 512 * 16)) =
+          fp8x8_to_bf16x8(u8[x]);
+  };
+
+  // ---- one step: 32 keys
+  // this lane's K row (A operand: row col, contraction 8 half + j) and V^T addresses:
+  // lane i of 16 reads 8 bytes of row i / 4; dt's columns move by 64 bytes
+  // addresses in the tile at hand, K's one tile ahead; a tile's second step is a constant
+  // further
+  unsigned kat[NC], vat[NDT];
+  {
+    const int i = lane & 15, r = i >> 2;
+    const int swz = DV == 64 ? (r & 2) << 1 : r << 2;
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) {
+      const int unit = dt * 4 + ((lane >> 4) & 1) * 2 + ((i & 3) >> 1);
+      vat[dt] = smem_at + KBYTES + (4 * half + r) * DV * 2 + (unit ^ swz) * 16 + (i & 1) * 8;
+    }
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      kat[c] = smem_at + col * D * 2 + (((c * 2 + half) ^ ((col >> KSHIFT) & KMASK)) << 4);
+  }
+  auto load_keys = [&](frag_u (&kf)[NC], int second, int from, int to) {
+#pragma unroll
+    for (int c = from; c < to; ++c)
+      kf[c].s = *(const __attribute__((address_space(3))) shortx8*)(kat[c] + second * 32 * D * 2);
+  };
+  // O^T += V^T P^T, product j of 2 NDT: 16 keys j / NDT, d-tile j % NDT; fragments in pairs
+  auto product = [&](const frag_u (&w)[2], const shortx4 (&v)[NDT][4], int j) {
+    frag_u vf;
+    vf.h[0] = v[j / 2][j % 2 * 2];
+    vf.h[1] = v[j / 2][j % 2 * 2 + 1];
+    o[j % NDT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, w[j / NDT].v, o[j % NDT], 0, 0, 0);
+  };
+  // pair I of the step AT bytes into its tile
+  auto fetch_values = [&](shortx4 (&v)[NDT][4], auto AT, auto I) {
+    constexpr int i = decltype(I)::value, ROW8 = 8 * DV * 2;
+    constexpr int at = decltype(AT)::value + i / (NDT / 2) * 2 * ROW8, dt = i % (NDT / 2) * 2;
+    read_values<at, ROW8>(v[i], vat[dt], vat[dt + 1]);
+  };
+  using ZERO = std::integral_constant<int, 0>;
+  using ONE = std::integral_constant<int, 1>;
+  // penalty and mask of a step's scores
+  auto mask = [&](floatx16& st, int step) {
+    const int ks = step * 32;
+    if constexpr (BIAS == LINEAR_BIAS || BIAS == LOG_BIAS) {
       // distance of key row 4 * half, and the logarithm's argument there
       const float dist0 = (float)(q_abs - ks - 4 * half);
       const float arg0 = 1.f + rate * dist0;
-      const bool need_mask = (ks + 31 > q_abs_min) || (ks + 31 >= ctx) ||
-                             (BIAS && ks < lo_max);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float away = (float)((r & 3) + 8 * (r >> 2));
+        st[r] = st[r] * c2 - slope * (BIAS == LOG_BIAS ? __builtin_amdgcn_logf(arg0 - rate * away)
+                                                       : dist0 - away);
+      }
+    }
+    // (a row that has seen only masked keys yet keeps its first reference)
+    if ((ks + 31 > q_abs_min) || (ks + 31 >= ctx) || (BIAS && ks < lo_max)) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const int k_abs = ks + (r & 3) + 8 * (r >> 2) + 4 * half;
-        float sv = st[r] * scale;
-        if constexpr (BIAS != NO_BIAS) {
-          // a row that has seen only masked keys yet holds weights of
-          // exp(0); its first visible key rescales them to zero
-          const float step = (float)((r & 3) + 8 * (r >> 2));
-          if constexpr (BIAS != FLAT_BIAS)
-            sv -= slope * (BIAS == LOG_BIAS ? __builtin_amdgcn_logf(arg0 - rate * step)
-                                            : dist0 - step);
-          if (need_mask && (k_abs > q_abs || k_abs >= ctx || k_abs < lo))
-            sv = -1e30f;
-        } else {
-          if (need_mask && (k_abs > q_abs || k_abs >= ctx)) sv = -3.0e4f;
-        }
-        p[r] = sv;
-      }
-      // ---- online softmax (per-lane column view)
-      float tmax = p[0];
-#pragma unroll
-      for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, p[r]);
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-      const float mn = fmaxf(m, tmax);
-      const float alpha = __expf(m - mn);
-      m = mn;
-      float psum = 0.f;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        p[r] = __expf(p[r] - mn);
-        psum += p[r];
-      }
-      psum += __shfl_xor(psum, 32, WAVE);
-      l = l * alpha + psum;
-      // ---- rescale O by alpha of each O-row's q (broadcast via LDS)
-      if (half == 0) wsc[col] = alpha;
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x4 av = *reinterpret_cast<const f32x4*>(wsc + 4 * half + 8 * g);
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) o[dt][4 * g + j] *= av[j];
-        }
-      }
-      // ---- P -> bf16 A-fragments (pack + permlane32_swap)
-      frag_u pf[2];
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        unsigned int a0 = pack2_bf16(p[c * 8 + 0], p[c * 8 + 1]);
-        unsigned int a1 = pack2_bf16(p[c * 8 + 2], p[c * 8 + 3]);
-        unsigned int b0 = pack2_bf16(p[c * 8 + 4], p[c * 8 + 5]);
-        unsigned int b1 = pack2_bf16(p[c * 8 + 6], p[c * 8 + 7]);
-        {
-          auto r0 = __builtin_amdgcn_permlane32_swap(a0, b0, false, false);
-          a0 = r0[0];
-          b0 = r0[1];
-          auto r1 = __builtin_amdgcn_permlane32_swap(a1, b1, false, false);
-          a1 = r1[0];
-          b1 = r1[1];
-        }
-        pf[c].u[0] = a0;
-        pf[c].u[1] = a1;
-        pf[c].u[2] = b0;
-        pf[c].u[3] = b1;
-      }
-      // ---- PV: O[dt] += P * V  (B-frag = 16-B row read of transposed V)
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) {
-          const int d = dt * 32 + col;
-          const int kloc = s * 32 + c * 16 + half * 8;
-          frag_u vf;
-          const shortx8 vv =
-              *reinterpret_cast<const shortx8*>(vtbuf + d * VROW + kloc);
-          vf.u[0] = ((const unsigned int*)&vv)[0];
-          vf.u[1] = ((const unsigned int*)&vv)[1];
-          vf.u[2] = ((const unsigned int*)&vv)[2];
-          vf.u[3] = ((const unsigned int*)&vv)[3];
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(pf[c].v, vf.v, o[dt], 0, 0, 0);
-        }
+        if (k_abs > q_abs || k_abs >= ctx || (BIAS && k_abs < lo)) st[r] = -INFINITY;
       }
     }
+  };
+
+  // Softmax and values of ``step``, whose scores S^T (rows keys, columns queries) are in
+  // ``cur``, and the scores of the step after it. A row's last step computes scores of
+  // whatever lies in LDS, which nobody uses.
+  auto advance = [&](floatx16& cur, floatx16& next, int step, auto SECOND) {
+    constexpr bool SCALED = BIAS == LINEAR_BIAS || BIAS == LOG_BIAS;
+    constexpr int second = decltype(SECOND)::value;
+    using AT = std::integral_constant<int, second * 32 * DV * 2>;
+    mask(cur, step);
+    frag_u kf[NC];
+    shortx4 v[NDT][4];
+    constexpr int EARLY = NC < 8 ? NC : 8;  // the others when registers are free again
+    load_keys(kf, 1 - second, 0, EARLY);
+    float mx = cur[0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) mx = fmaxf(mx, cur[r]);
+    if constexpr (!SCALED) mx *= c2;
+    if (__any(mx > m + PRE_SLACK)) {
+      mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+      const float mn = fmaxf(m, mx);
+      const float alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) next[r] = 0.f;
+    frag_u pf[2];
+    float sum = 0.f;
+    // an eighth of the scores and of the softmax at a time
+    static_for<8>([&](auto E) {
+      constexpr int e = decltype(E)::value;
+#pragma unroll
+      for (int c = NC * e / 8; c < NC * (e + 1) / 8; ++c)
+        next = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[c].v, qf[c].v, next, 0, 0, 0);
+      float p[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        p[k] = __builtin_amdgcn_exp2f(SCALED ? cur[2 * e + k] - m
+                                             : __builtin_fmaf(cur[2 * e + k], c2, -m));
+      sum += p[0] + p[1];
+      pf[e >> 2].u[e & 3] = cvt2_bf16(p[0], p[1]);
+      if constexpr (EARLY < NC && e == 2) load_keys(kf, 1 - second, EARLY, NC);
+      if constexpr (e == 6) fetch_values(v, AT{}, ZERO{});
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    l += sum;
+    await_values(v[0]);
+    static_for<NDT>([&](auto I) {  // O^T += V^T P^T
+      constexpr int i = decltype(I)::value;
+      if constexpr (i + 1 < NDT) fetch_values(v, AT{}, std::integral_constant<int, i + 1>{});
+      product(pf, v, 2 * i);
+      product(pf, v, 2 * i + 1);
+      if constexpr (i + 1 < NDT) await_values(v[i + 1]);
+    });
+  };
+
+  // before and after the computation of a tile: the next one is there for all, and nobody
+  // reads the one before it any more
+  auto begin = [&](int tile) {
+    if constexpr (FP8) {
+      if (tile + 1 < ntiles) fetch8(tile + 1);
+      lookup(tile + 2);
+    }
+  };
+  auto turn_over = [&](int tile) {
+    if constexpr (FP8) {
+      if (tile + 1 < ntiles) store8(tile + 1);
+      __syncthreads();
+    } else {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      if (tile + 2 < ntiles) issue(tile + 2);
+      lookup(tile + 3);
+    }
+  };
+  lookup(tile0);
+  if constexpr (FP8) {
+    fetch8(tile0);
+    store8(tile0);
+    lookup(tile0 + 1);
+    __syncthreads();
+  } else {
+    issue(tile0);
+    lookup(tile0 + 1);
+    if (tile0 + 1 < ntiles) {
+      issue(tile0 + 1);
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LK + LV) : "memory");
+    } else {
+      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    lookup(tile0 + 2);
+  }
+  int tile = tile0;
+  for (; tile < first; ++tile) {
+    begin(tile);
+    turn_over(tile);
+  }
+  floatx16 even, odd;
+  unsigned stage = tile % PRE_STAGES * STAGE;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) kat[c] += stage;
+#pragma unroll
+  for (int dt = 0; dt < NDT; ++dt) vat[dt] += stage;
+  {  // the first scores
+    frag_u kf[NC];
+    load_keys(kf, 0, 0, NC);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) even[r] = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      even = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[c].v, qf[c].v, even, 0, 0, 0);
+  }
+  for (; tile < end; ++tile) {
+    begin(tile);
+    advance(even, odd, tile * 2, ZERO{});
+    turn_over(tile);
+    const unsigned move = stage == (PRE_STAGES - 1) * STAGE ? -(PRE_STAGES - 1) * STAGE : STAGE;
+    stage += move;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) kat[c] += move;
+    advance(odd, even, tile * 2 + 1, ONE{});
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt) vat[dt] += move;
+  }
+  for (; tile < ntiles; ++tile) {  // other waves' rows see more
+    begin(tile);
+    turn_over(tile);
   }
 
-  // ---- epilogue: divide by l (per q row), transpose via LDS, store rows
+  // ---- epilogue: a lane holds channels 4 half + {0..3} of every 8 of its row
+  l += __shfl_xor(l, 32, WAVE);
+  const long row = q_start + qrow;
   if constexpr (EXTRA == GATED) {  // divided by l, times the gate
     const long grow = (q_start + (qvalid ? qrow : 0)) * gstride + h;
     l *= 1.f + __expf(-bf16_to_f32(((const unsigned short*)gate)[grow]));
   }
-  if (half == 0) wsc[col] = l;
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  __builtin_amdgcn_sched_barrier(0);
-  float linv[4][4];
+  const float inv = oscale / l;
+  bf16_t* orow = (bf16_t*)out + row * ostride + (long)h * dv;
+  const float* cs = EXTRA == TURNED && turn.cs ? turn.cs + (long)q_abs * dv : nullptr;
+  const bf16_t* gp = EXTRA == TURNED && turn.gate
+                         ? (const bf16_t*)turn.gate + row * turn.gstride + h * dv : nullptr;
+  const bool vec = !BIAS || ((dv | ostride | ((long)out >> 1) |
+                              (EXTRA == TURNED ? turn.gstride | ((long)turn.gate >> 1) : 0)) &
+                             7) == 0;
 #pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const f32x4 lv = *reinterpret_cast<const f32x4*>(wsc + 4 * half + 8 * g);
+  for (int dt = 0; dt < NDT; ++dt) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) linv[g][j] = oscale / lv[j];
-  }
-  if constexpr (EXTRA == TURNED) {
-    // 32 x 32 results at a time through the wave's own LDS; a lane then holds 16
-    // neighbouring channels of one row
-    __syncthreads();
-    float* ob = (float*)smem + wave * (32 * TURN_STRIDE);
-    const int r = lane >> 1, c0 = (lane & 1) * 16, qr = qoff + qsub * 32 + r;
-    const long row = q_start + qr;
-    const float* cs = turn.cs ? turn.cs + (long)(ctx - qlen + qr) * dv : nullptr;
-    const bf16_t* gp = turn.gate ? (const bf16_t*)turn.gate + row * turn.gstride + h * dv
-                                 : nullptr;
-    bf16_t* orow = (bf16_t*)out + row * ostride + (long)h * dv;
-    const bool vec = ((dv | ostride | turn.gstride | ((long)out >> 1) |
-                       ((long)turn.gate >> 1)) & 7) == 0;
+    for (int g = 0; g < 4; g += 2) {
+      unsigned int y[2][2];
 #pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
+      for (int k = 0; k < 2; ++k) {
+        const int d = dt * 32 + 8 * (g + k) + 4 * half;
+        float v[4];
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
+        for (int j = 0; j < 4; ++j) v[j] = o[dt][4 * (g + k) + j] * inv;
+        if constexpr (EXTRA == TURNED) {
+          if (qvalid && d < dv) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          ob[(j + 8 * g + 4 * half) * TURN_STRIDE + col] = o[dt][4 * g + j] * linv[g][j];
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
+            for (int j = 0; j < 4; j += 2)
+              if (cs && d + j < dv)
+                turn_pair(v[j], v[j + 1], cs[(d + j) / 2], -cs[(dv + d + j) / 2]);
 #pragma unroll
-      for (int i = 0; i < 16; i += 8) {
-        const int d = dt * 32 + c0 + i;
-        if (qr >= qlen || d >= dv) continue;
-        float y[8];
-        const float* src = ob + r * TURN_STRIDE + c0 + i;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) y[k] = src[k];
-        if (vec) {
-          if (cs) {
-            const floatx4 c = ld4(cs + d / 2), sn = ld4(cs + (dv + d) / 2);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) turn_pair(y[2 * k], y[2 * k + 1], c[k], -sn[k]);
-          }
-          if (gp) {
-            const shortx8 gv = *reinterpret_cast<const shortx8*>(gp + d);
-#pragma unroll
-            for (int k = 0; k < 8; ++k) y[k] *= sigmoid_f(bf16_to_f32((unsigned short)gv[k]));
-          }
-          shortx8 v;
-#pragma unroll
-          for (int k = 0; k < 8; ++k) v[k] = (short)f32_to_bf16(y[k]);
-          *reinterpret_cast<shortx8*>(orow + d) = v;
-        } else {
-#pragma unroll
-          for (int k = 0; k < 8; k += 2) {
-            if (cs && d + k < dv)
-              turn_pair(y[k], y[k + 1], cs[(d + k) / 2], -cs[(dv + d + k) / 2]);
-#pragma unroll
-            for (int x = k; x < k + 2; ++x)
-              if (d + x < dv) stf(orow + d + x, gp ? y[x] * sigmoid_f(ldf(gp + d + x)) : y[x]);
+            for (int j = 0; j < 4; ++j)
+              if (gp && d + j < dv) v[j] *= sigmoid_f(ldf(gp + d + j));
           }
         }
-      }
-    }
-    return;
-  }
-  // everyone done with K/V buffers; reuse as O staging in two rounds of
-  // 4 waves (8 waves' staging would not fit the K+V area)
+        if (!vec && qvalid) {  // head width or column not a multiple of 8
 #pragma unroll
-  for (int round = 0; round < 2; ++round) {
-    __syncthreads();
-    if ((wave >> 2) != round) continue;
-    short* obuf = (short*)smem + (wave & 3) * 32 * DV;
-#pragma unroll
-    for (int dt = 0; dt < NDT; ++dt) {
-      const int d = dt * 32 + col;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int r = (j) + 8 * g + 4 * half;  // q row within the wave's 32
-          obuf[r * DV + d] = (short)f32_to_bf16(o[dt][4 * g + j] * linv[g][j]);
+          for (int j = 0; j < 4; ++j)
+            if (d + j < dv) stf(orow + d + j, v[j]);
         }
+        y[k][0] = cvt2_bf16(v[0], v[1]);
+        y[k][1] = cvt2_bf16(v[2], v[3]);
       }
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    __builtin_amdgcn_sched_barrier(0);
-    // each lane stores half a row (DV/2 elems = DV bytes) with 16-B stores
-    const int r = lane >> 1;            // 0..31
-    const int seg = (lane & 1) * (DV / 2);
-    const int qr = qoff + qsub * 32 + r;
-    if (qr < qlen) {
-      __hip_bfloat16* orow = out + (long)(q_start + qr) * ostride + (long)h * dv;
-      if (!BIAS || ((dv | ostride | ((long)out >> 1)) & 7) == 0) {
+      if (!vec) continue;
+      // halves trade: this lane's half of 16 channels in one piece
+      frag_u w;
 #pragma unroll
-        for (int i = 0; i < DV / 16; ++i) {
-          if (BIAS && seg + i * 8 >= dv) break;
-          const shortx8 v =
-              *reinterpret_cast<const shortx8*>(obuf + r * DV + seg + i * 8);
-          *reinterpret_cast<shortx8*>(orow + seg + i * 8) = v;
-        }
-      } else {  // head width or column not a multiple of 8
-        for (int i = seg; i < min(dv, seg + DV / 2); ++i)
-          *(short*)(orow + i) = obuf[r * DV + i];
+      for (int j = 0; j < 2; ++j) {
+        const auto r = __builtin_amdgcn_permlane32_swap(y[0][j], y[1][j], false, false);
+        w.u[j] = r[0];
+        w.u[2 + j] = r[1];
       }
+      const int d = dt * 32 + 8 * (g + half);
+      if (qvalid && (!BIAS || d < dv)) *reinterpret_cast<shortx8*>(orow + d) = w.s;
     }
   }
 }
@@ -447,13 +617,16 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
 // query heads per workgroup: the GQA group shares each staged K/V tile
 static int heads_per_block(int G) { return G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1; }
 
-template <int D, int DV>
-static size_t prefill_lds() {
-  return std::max<size_t>(64 * D * 2 + DV * (64 + 8) * 2, 256 * DV) + 8 * 32 * 4;
-}
-template <int D, int DV>
-static size_t turned_lds() {
-  return std::max<size_t>(prefill_lds<D, DV>(), 8 * 32 * TURN_STRIDE * 4);
+template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED, typename... Args>
+static void prefill_launch(int blocks, int Hq, Args... args) {
+  constexpr int lds = PRE_STAGES * PRE_KEYS * (D + DV) * 2;
+  const auto kern = prefill_kernel<D, DV, HG, FP8, BIAS, EXTRA, PAGED>;
+  if (lds > 64 * 1024) {
+    static const hipError_t once = hipFuncSetAttribute(
+        (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    TORCH_CHECK(once == hipSuccess, "attention prefill: LDS");
+  }
+  hipLaunchKernelGGL(kern, dim3(blocks * (Hq / HG)), dim3(512), lds, CUR_STREAM, args...);
 }
 
 torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
@@ -469,39 +642,24 @@ torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
   TORCH_CHECK(Hq % Hkv == 0, "GQA requires Hq % Hkv == 0");
   const int HG = heads_per_block(Hq / Hkv);
   const int QROWS = 32 * (8 / HG);  // q rows covered per workgroup
-  // host-side q-block map (cu_q is tiny; engine built it on CPU this step)
-  auto cu_cpu = cu_q.to(torch::kCPU);
-  const int* cu = cu_cpu.data_ptr<int>();
-  const int S = cu_cpu.numel() - 1;
-  std::vector<int> bseq, boff;
-  for (int s = 0; s < S; ++s) {
-    const int qlen = cu[s + 1] - cu[s];
-    for (int off = 0; off < qlen; off += QROWS) {
-      bseq.push_back(s);
-      boff.push_back(off);
-    }
-  }
-  const int NB = bseq.size();
-  auto opts = torch::TensorOptions().dtype(torch::kInt32).device(q.device());
-  auto bseq_t = torch::from_blob(bseq.data(), {NB}, torch::kInt32).to(opts.device());
-  auto boff_t = torch::from_blob(boff.data(), {NB}, torch::kInt32).to(opts.device());
-
+  // as many blocks as there can be; each finds its rows, so that nothing is read back
+  const int S = cu_q.numel() - 1, NB = T / QROWS + S;
   const bool fp8 = kc.dtype() == torch::kFloat8_e4m3fn;
-  dim3 grid(NB, Hq / HG), block(512);
-  auto stream = CUR_STREAM;
-#define PLAUNCH1(DD, HGV, F8)                                                 \
-  hipLaunchKernelGGL((prefill_kernel<DD, DD, HGV, F8, NO_BIAS, PLAIN>), grid, block,   \
-                     (prefill_lds<DD, DD>()), stream,                         \
+#define PLAUNCH1(DD, HGV, F8, PG)                                               \
+  prefill_launch<DD, DD, HGV, F8, NO_BIAS, PLAIN, PG>(NB, Hq,                      \
                      (const __hip_bfloat16*)q.data_ptr(),                     \
                      kc.data_ptr(), vc.data_ptr(),                            \
                      (__hip_bfloat16*)out.data_ptr(),                         \
-                     bseq_t.data_ptr<int>(), boff_t.data_ptr<int>(),          \
-                     cu_q.data_ptr<int>(), bt.data_ptr<int>(),                \
+                     nullptr, nullptr, cu_q.data_ptr<int>(), S, bt.data_ptr<int>(),                \
                      ctx.data_ptr<int>(), Hq, Hkv, P, MP, (float)scale,       \
                      (long)Hq * D, (long)Hq * D, D, 1.f, nullptr, nullptr, 0, \
                      0, nullptr, nullptr, 0, KeyTail{}, HeadTurn{})
 #define PLAUNCH(DD, HGV)                                                      \
-  if (fp8) { PLAUNCH1(DD, HGV, true); } else { PLAUNCH1(DD, HGV, false); }
+  if (P % PRE_KEYS == 0) {                                                    \
+    if (fp8) { PLAUNCH1(DD, HGV, true, true); }                               \
+    else { PLAUNCH1(DD, HGV, false, true); }                                  \
+  } else if (fp8) { PLAUNCH1(DD, HGV, true, false); }                         \
+  else { PLAUNCH1(DD, HGV, false, false); }
 #define PLAUNCH_D(DD)                                                         \
   switch (HG) {                                                               \
     case 1: PLAUNCH(DD, 1); break;                                            \
@@ -549,24 +707,25 @@ void biased_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
   const int NB = bseq.numel();
   if (T == 0 || NB == 0) return;
   const int HG = heads_per_block(Hq / Hkv);
-  dim3 grid(NB, Hq / HG), block(512);
   const float* rp = rates ? rates->data_ptr<float>() : nullptr;
   const float* sp = slopes ? slopes->data_ptr<float>() : nullptr;
   const float* snk = sink ? sink->data_ptr<float>() : nullptr;
-#define BLAUNCH1(DD, DVV, HGV, BB, XX, LDS)                                     \
-  hipLaunchKernelGGL((prefill_kernel<DD, DVV, HGV, false, BB, XX>), grid, block, \
-                     (LDS<DD, DVV>()), CUR_STREAM,                              \
+#define BLAUNCH2(DD, DVV, HGV, BB, XX, PG)                                      \
+  prefill_launch<DD, DVV, HGV, false, BB, XX, PG>(NB, Hq,                            \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr() + col,      \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
-                     cu_q.data_ptr<int>(), bt.data_ptr<int>(),                  \
+                     cu_q.data_ptr<int>(), (int)ctx.numel(), bt.data_ptr<int>(), \
                      ctx.data_ptr<int>(), Hq, Hkv, P, MP, (float)scale,         \
                      (long)Hq * D, out.stride(0), (int)dv, (float)oscale,       \
                      sp, rp, (int)window, (int)chunk, snk, nullptr, 0, KeyTail{}, ht)
+#define BLAUNCH1(DD, DVV, HGV, BB, XX)                                          \
+  if (P % PRE_KEYS == 0) { BLAUNCH2(DD, DVV, HGV, BB, XX, true); }              \
+  else { BLAUNCH2(DD, DVV, HGV, BB, XX, false); }
 #define BLAUNCH(DD, DVV, HGV)                                                   \
-  if (!sp) { BLAUNCH1(DD, DVV, HGV, FLAT_BIAS, TURNED, turned_lds); }           \
-  else if (rp) { BLAUNCH1(DD, DVV, HGV, LOG_BIAS, PLAIN, prefill_lds); }        \
-  else { BLAUNCH1(DD, DVV, HGV, LINEAR_BIAS, PLAIN, prefill_lds); }
+  if (!sp) { BLAUNCH1(DD, DVV, HGV, FLAT_BIAS, TURNED); }           \
+  else if (rp) { BLAUNCH1(DD, DVV, HGV, LOG_BIAS, PLAIN); }        \
+  else { BLAUNCH1(DD, DVV, HGV, LINEAR_BIAS, PLAIN); }
 #define BLAUNCH_HG(DD, DVV)                    \
   switch (HG) {                                \
     case 1: BLAUNCH(DD, DVV, 1); break;        \
@@ -581,6 +740,7 @@ void biased_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
 #undef BLAUNCH_HG
 #undef BLAUNCH
 #undef BLAUNCH1
+#undef BLAUNCH2
   HIP_CHECK_KERNEL();
 }
 
@@ -609,14 +769,12 @@ void sink_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
               cu_q.numel() == ctx.numel() + 1 && bt.size(0) == ctx.numel());
   const int NB = bseq.numel();
   if (T == 0 || NB == 0) return;
-  dim3 grid(NB, H), block(512);
 #define SLAUNCH(DD, DVV)                                                        \
-  hipLaunchKernelGGL((prefill_kernel<DD, DVV, 1, false, NO_BIAS, GATED>), grid,    \
-                     block, (prefill_lds<DD, DVV>()), CUR_STREAM,               \
+  prefill_launch<DD, DVV, 1, false, NO_BIAS, GATED, false>(NB, H,                       \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr(),            \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
-                     cu_q.data_ptr<int>(), bt.data_ptr<int>(),                  \
+                     cu_q.data_ptr<int>(), (int)ctx.numel(), bt.data_ptr<int>(), \
                      ctx.data_ptr<int>(), H, H, P, MP, (float)scale,            \
                      q.stride(0), out.stride(0), DV, 1.f, nullptr, nullptr, 0,  \
                      0, sink.data_ptr<float>(),                                 \
@@ -659,16 +817,14 @@ void tailed_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
               cu_q.numel() == ctx.numel() + 1 && bt.size(0) == ctx.numel());
   const int NB = bseq.numel();
   if (T == 0 || NB == 0) return;
-  dim3 grid(NB, H), block(512);
   const KeyTail kt = {(const __hip_bfloat16*)tail.data_ptr(), tail.stride(0),
                       (int)tail.size(1), own};
 #define TLAUNCH(DD, DVV)                                                        \
-  hipLaunchKernelGGL((prefill_kernel<DD, DVV, 1, false, FLAT_BIAS, TAILED>), grid, \
-                     block, (prefill_lds<DD, DVV>()), CUR_STREAM,               \
+  prefill_launch<DD, DVV, 1, false, FLAT_BIAS, TAILED, false>(NB, H,                    \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr(),            \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
-                     cu_q.data_ptr<int>(), bt.data_ptr<int>(),                  \
+                     cu_q.data_ptr<int>(), (int)ctx.numel(), bt.data_ptr<int>(), \
                      ctx.data_ptr<int>(), H, H, 1, MP, (float)scale,            \
                      q.stride(0), out.stride(0), DV, 1.f, nullptr, nullptr,     \
                      (int)window, 0, nullptr, nullptr, 0, kt, HeadTurn{})
