@@ -170,8 +170,9 @@ class MoEMLP(nn.Module):
 
     Experts are TP-sharded like the dense MLP (each expert's gate_up column-
     sharded, down row-sharded) so the expert compute stays local and the
-    row-parallel all-reduce doubles as the TP combine.  Token->expert
-    dispatch is a host-side gather for prompts, a grouped GEMM for decoding.
+    row-parallel all-reduce doubles as the TP combine.  On the GPU tokens are
+    sorted by expert on the device and run through grouped products; elsewhere
+    dispatch is a host-side gather for prompts, a batched product for small batches.
     """
 
     def __init__(self, spec: ModelSpec, dtype):
@@ -194,8 +195,28 @@ class MoEMLP(nn.Module):
             self.experts = nn.ModuleList(
                 [LlamaMLP(spec, dtype) for _ in range(spec.n_experts)]
             )
-        self._w_gu = None  # lazy stacked-weight cache for the batched path
-        self._w_dn = None
+        self._w_gu = None  # all experts' weights in one tensor each, of which the
+        self._w_dn = None  # experts' own are views
+        if self.ep_size == 1:
+            gu, dn = self.experts[0].gate_up.weight, self.experts[0].down.weight
+            self._share(gu.new_empty((self.n_experts, *gu.shape)),
+                        dn.new_empty((self.n_experts, *dn.shape)))
+
+    def _share(self, w_gu: torch.Tensor, w_dn: torch.Tensor) -> None:
+        for e, ex in enumerate(self.experts):
+            ex.gate_up.weight.data, ex.down.weight.data = w_gu[e], w_dn[e]
+        self._w_gu, self._w_dn = w_gu, w_dn
+
+    def _apply(self, fn, recurse: bool = True):
+        self._w_gu = self._w_dn = None  # a move leaves every expert's weights apart
+        return super()._apply(fn, recurse)
+
+    def _stacked(self) -> Tuple[torch.Tensor, torch.Tensor]:
+        if self._w_gu is None:
+            with torch.inference_mode(False):
+                self._share(torch.stack([ex.gate_up.weight.data for ex in self.experts]),
+                            torch.stack([ex.down.weight.data for ex in self.experts]))
+        return self._w_gu, self._w_dn
 
     def _local_expert_fn(self, xp: torch.Tensor,
                          local_sel: torch.Tensor) -> torch.Tensor:
@@ -208,6 +229,9 @@ class MoEMLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         T, H = x.shape
+        if self.ep_size == 1 and ops.has_moe_grouped(x):
+            out = ops.moe_silu_glu(x, self.router.weight, self.top_k, *self._stacked())
+            return pdist.tp_all_reduce(out) if pdist.tp_world_size() > 1 else out
         logits = self.router(x).float()  # [T, E]
         weights, sel = logits.topk(self.top_k, dim=-1)
         weights = weights.softmax(-1).to(x.dtype)  # [T, k]
@@ -229,13 +253,9 @@ class MoEMLP(nn.Module):
 
     def _forward_batched(self, x: torch.Tensor, weights: torch.Tensor,
                          sel: torch.Tensor) -> torch.Tensor:
-        """Decode path: tokens sorted by expert into a PACKED buffer
-        (no capacity padding), then per-expert grouped GEMMs via the
-        streaming moe_grouped_gemm kernel — unrouted experts skip their
-        whole weight stream, activations/silu run over A = T*top_k rows
-        instead of E*C. Static shapes + device-read
-        counts keep the step hipGraph-capturable. CPU / no-extension
-        fallback: a fixed-capacity bmm dispatch."""
+        """Small batches without the grouped kernels: tokens sorted by expert into a
+        fixed-capacity buffer, batched products over all experts. Static shapes, nothing
+        read back."""
         T, H = x.shape
         E, k = self.n_experts, self.top_k
         flat = sel.reshape(-1)  # [T*k]
@@ -245,33 +265,19 @@ class MoEMLP(nn.Module):
         counts = torch.zeros(E, dtype=torch.long, device=x.device).scatter_add_(
             0, flat, torch.ones_like(flat))
         starts = torch.cumsum(counts, 0) - counts
-        if self._w_gu is None:  # stacked expert weights, cached (constant)
-            self._w_gu = torch.stack([ex.gate_up.weight for ex in self.experts])
-            self._w_dn = torch.stack([ex.down.weight for ex in self.experts])
-        w_gu, w_dn = self._w_gu, self._w_dn
+        w_gu, w_dn = self._stacked()
         wflat = weights.reshape(-1)[order].unsqueeze(1).to(x.dtype)
-        if ops.has_moe_grouped(x):
-            xp = x[tok_of]  # [A, H] packed, expert-sorted
-            st32 = starts.to(torch.int32)
-            ct32 = counts.to(torch.int32)
-            gu = ops.moe_grouped_gemm(xp, w_gu, st32, ct32)     # [A, 2I']
-            act = ops.silu_mul(gu)                              # [A, I']
-            ye = ops.moe_grouped_gemm(act, w_dn, st32, ct32)    # [A, H]
-            out = torch.zeros_like(x)
-            out.index_add_(0, tok_of, ye * wflat)
-        else:
-            C = T
-            rank = torch.arange(T * k, device=x.device) - starts[flat[order]]
-            slot_idx = flat[order] * C + rank  # rank < C always
-            xe = x.new_zeros(E * C, H)
-            xe[slot_idx] = x[tok_of]
-            xe = xe.view(E, C, H)
-            gu = torch.bmm(xe, w_gu.transpose(1, 2).contiguous())  # [E, C, 2I']
-            act = ops.silu_mul(gu.reshape(E * C, -1)).view(E, C, -1)
-            ye = torch.bmm(act, w_dn.transpose(1, 2).contiguous()).view(E * C, H)
-            out = torch.zeros_like(x)
-            out.index_add_(0, tok_of, ye[slot_idx] * wflat)
-        from ..parallel import dist as pdist
+        C = T
+        rank = torch.arange(T * k, device=x.device) - starts[flat[order]]
+        slot_idx = flat[order] * C + rank  # rank < C always
+        xe = x.new_zeros(E * C, H)
+        xe[slot_idx] = x[tok_of]
+        xe = xe.view(E, C, H)
+        gu = torch.bmm(xe, w_gu.transpose(1, 2).contiguous())  # [E, C, 2I']
+        act = ops.silu_mul(gu.reshape(E * C, -1)).view(E, C, -1)
+        ye = torch.bmm(act, w_dn.transpose(1, 2).contiguous()).view(E * C, H)
+        out = torch.zeros_like(x)
+        out.index_add_(0, tok_of, ye[slot_idx] * wflat)
         return pdist.tp_all_reduce(out) if pdist.tp_world_size() > 1 else out
 
 

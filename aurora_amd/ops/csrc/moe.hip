@@ -2,7 +2,8 @@
 //     act = g sigmoid(alpha g) (u + shift),  g = min(gate, limit), u = clamp(up)
 // (without a limit, alpha 1 and shift 0: silu(gate) up), or a squared relu, act =
 // max(up, 0)^2, chosen by one of three routers:
-//     z = W_r h + b (fp32), the ``top`` largest, softmax over the chosen;
+//     z = W_r h + b (fp32; without b rounded to the weights' type, as such models' plain
+//     product leaves it), the ``top`` largest, softmax over the chosen;
 //     s = sigmoid(W_r h) (fp32), the ``top`` largest of s + c among the best groups of
 //     neighbours (by the sum of their two largest), weights s / sum s * scale;
 //     s = softmax(W_r h) (fp32) over all, the ``top`` largest among the best groups (by
@@ -88,7 +89,10 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(
       float z = 0.f;
 #pragma unroll
       for (int v = 0; v < 16; ++v) z += part[v][t][x];
-      if (e < E) logits[t * E + e] = GROUPED ? z : z + bias[e];
+      // without a bias the logits are those of a product in the model's own type
+      if (ROUTER == CHOSEN_SOFTMAX)
+        z = bias ? z + bias[min(e, E - 1)] : sizeof(T) == 2 ? bf16_to_f32(f32_to_bf16(z)) : z;
+      if (e < E) logits[t * E + e] = z;
     }
     __syncthreads();
   }
@@ -177,8 +181,9 @@ static std::vector<torch::Tensor> route(const torch::Tensor& h, const torch::Ten
               router.is_contiguous() && router.dtype() == h.dtype());
   const long T_ = h.size(0), W = h.size(1), E = router.size(0);
   TORCH_CHECK(router.size(1) == W);
-  TORCH_CHECK(ROUTER == GROUPED_SOFTMAX ? !bias : bias && bias->numel() == E &&
-              bias->dtype() == torch::kFloat32, "router bias");
+  TORCH_CHECK(bias ? ROUTER != GROUPED_SOFTMAX && bias->numel() == E &&
+                         bias->dtype() == torch::kFloat32
+                   : ROUTER != GROUPED_SIGMOID, "router bias");
   TORCH_CHECK(top >= 1 && top <= E && E <= 512, "1 <= top <= experts <= 512");
   auto sel = torch::empty({T_, top}, h.options().dtype(torch::kInt32));
   auto gate = torch::empty({T_, top}, h.options().dtype(torch::kFloat32));
@@ -200,7 +205,7 @@ static std::vector<torch::Tensor> route(const torch::Tensor& h, const torch::Ten
 }
 
 std::vector<torch::Tensor> moe_route(torch::Tensor h, torch::Tensor router,
-                                     torch::Tensor bias, long top) {
+                                     c10::optional<torch::Tensor> bias, long top) {
   return route<CHOSEN_SOFTMAX>(h, router, bias, top, 1, 1, 1.0);
 }
 
@@ -549,4 +554,47 @@ std::vector<torch::Tensor> moe_clamped_glu(torch::Tensor h, torch::Tensor sel,
 std::vector<torch::Tensor> moe_relu2(torch::Tensor h, torch::Tensor sel, torch::Tensor w_up,
                                      torch::Tensor w_dn) {
   return experts<RELU2_ACT>(h, sel, w_up, w_dn, 0.0, 0.0, 0.0);
+}
+
+// ------------------------------------------------------------------ combine
+
+// Every token's expert rows, weighted and summed in fp32; a thread owns 8 columns. Bound
+// by memory: 1580 tokens of 4096 with two experts each, 39 MB.
+__global__ __launch_bounds__(256) void moe_combine_kernel(
+    const bf16_t* __restrict__ y, const int* __restrict__ place,
+    const float* __restrict__ gate, bf16_t* __restrict__ out, long T_, int W, int top) {
+  const long x = blockIdx.x * 256L + threadIdx.x;
+  const int w8 = W / 8;
+  const long t = x / w8;
+  if (t >= T_) return;
+  const int c = x % w8 * 8;
+  float acc[8] = {};
+  for (int k = 0; k < top; ++k) {
+    const float g = gate[t * top + k];
+    const shortx8 v = *reinterpret_cast<const shortx8*>(y + (long)place[t * top + k] * W + c);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] += g * bf16_to_f32((unsigned short)v[j]);
+  }
+  shortx8 r;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) r[j] = (short)f32_to_bf16(acc[j]);
+  *reinterpret_cast<shortx8*>(out + t * W + c) = r;
+}
+
+// y [T * top, W] rows of the sorted batch, place and gate [T, top] -> [T, W]
+torch::Tensor moe_combine(torch::Tensor y, torch::Tensor place, torch::Tensor gate) {
+  TORCH_CHECK(y.is_cuda() && y.dtype() == torch::kBFloat16 && y.is_contiguous() &&
+              place.is_contiguous() && place.dtype() == torch::kInt32 &&
+              gate.is_contiguous() && gate.dtype() == torch::kFloat32 &&
+              place.sizes() == gate.sizes() && y.size(0) == place.numel());
+  const long T_ = place.size(0), W = y.size(1);
+  TORCH_CHECK(W % 8 == 0, "rows of a multiple of 8");
+  auto out = torch::empty({T_, W}, y.options());
+  if (T_ == 0) return out;
+  hipLaunchKernelGGL(moe_combine_kernel, dim3((T_ * (W / 8) + 255) / 256), dim3(256), 0,
+                     CUR_STREAM, (const bf16_t*)y.data_ptr(), place.data_ptr<int>(),
+                     gate.data_ptr<float>(), (bf16_t*)out.data_ptr(), T_, (int)W,
+                     (int)place.size(1));
+  HIP_CHECK_KERNEL();
+  return out;
 }
