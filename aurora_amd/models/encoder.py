@@ -37,16 +37,20 @@ class EncoderLayer(nn.Module):
             p.requires_grad_(False)
         self.eps = spec.rms_eps
 
-    def forward(self, x, cos_sin, positions, cu):
+    def forward(self, x, delta, cos_sin, positions, cu):
+        """The stream ``x``, to which ``delta`` (the layer before's result) is still to be
+        added -> the stream and this layer's."""
         T = x.shape[0]
-        h = ops.rmsnorm(x, self.norm1, self.eps)
+        if delta is None:
+            h = ops.rmsnorm(x, self.norm1, self.eps)
+        else:
+            h, x = ops.rmsnorm_residual(delta, x, self.norm1, self.eps)
         qkv = self.qkv(h).view(T, 3 * self.n_heads, self.head_dim)
         q, k, v = qkv.split(self.n_heads, dim=1)
-        q, k = ops.rope_apply(q.contiguous(), k.contiguous(), positions, cos_sin)
-        o = ops.attention_prefill(q, k, v.contiguous(), cu, self.scale, causal=False)
-        x = x + self.o(o.reshape(T, -1))
-        h = ops.rmsnorm(x, self.norm2, self.eps)
-        return x + self.down(ops.silu_mul(self.gate_up(h)))
+        ops.rope_apply_(q, k, positions, cos_sin)
+        o = ops.attention_prefill(q, k, v, cu, self.scale, causal=False)
+        h, x = ops.rmsnorm_residual(self.o(o.reshape(T, -1)), x, self.norm2, self.eps)
+        return x, self.down(ops.silu_mul(self.gate_up(h)))
 
 
 class SentenceEncoder(nn.Module):
@@ -91,7 +95,8 @@ class SentenceEncoder(nn.Module):
         cu_t = torch.tensor(cu, dtype=torch.int32, device=dev)
         pos_t = torch.tensor(pos, dtype=torch.int32, device=dev)
         x = self.embed(ids)
+        delta = None
         for layer in self.layers:
-            x = layer(x, self.cos_sin, pos_t, cu_t)
-        x = ops.rmsnorm(x, self.final_norm, self.spec.rms_eps)
+            x, delta = layer(x, delta, self.cos_sin, pos_t, cu_t)
+        x = ops.rmsnorm_residual(delta, x, self.final_norm, self.spec.rms_eps)[0]
         return ops.embed_pool(x, cu_t)

@@ -75,6 +75,17 @@ def rope_apply(
     return torch_ref.rope_apply(q, k, positions, cos_sin)
 
 
+def rope_apply_(
+    q: torch.Tensor, k: torch.Tensor, positions: torch.Tensor, cos_sin: torch.Tensor
+) -> None:
+    """``rope_apply`` in place, on rows that may be strided (columns of a projection)."""
+    if q.is_cuda:
+        _require_hip("rope_apply_").rope_apply_(q, k, positions.to(torch.int32), cos_sin)
+        return
+    for x, y in zip((q, k), torch_ref.rope_apply(q, k, positions, cos_sin)):
+        x.copy_(y)
+
+
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     if gate_up.is_cuda:
         return _require_hip("silu_mul").silu_mul(gate_up.contiguous())
@@ -91,10 +102,9 @@ def attention_prefill(
 ) -> torch.Tensor:
     if q.is_cuda:
         m = _require_hip("attention_prefill", aux=True)
-        return m.attention_prefill(
-            q.contiguous(), k.contiguous(), v.contiguous(),
-            cu_seqlens.to(torch.int32), float(scale), bool(causal),
-        )
+        # rows may be strided
+        return m.attention_prefill(q, k, v, cu_seqlens.to(torch.int32).contiguous(),
+                                   float(scale), bool(causal))
     return torch_ref.attention_prefill(q, k, v, cu_seqlens, scale, causal)
 
 

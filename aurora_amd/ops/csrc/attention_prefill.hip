@@ -37,23 +37,18 @@
 // result back and gates its channels, in fp32 (head_turn.h).
 // Covers fresh prefill and append-prefill (chunked agent turns) since K/V
 // are read from the paged cache with an absolute-position causal bound.
+#include "flash_tiles.h"
 #include "head_turn.h"
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
-#include <type_traits>
-
 #define CUR_STREAM c10::hip::getCurrentHIPStream().stream()
 
-#define LOG2E 1.44269504f
 #define PRE_KEYS 64     // keys per tile
 #define PRE_STAGES 3    // tiles in LDS
 #define PRE_SLACK 10.f  // weights stay below 2^PRE_SLACK
 enum { NO_BIAS = 0, LINEAR_BIAS = 1, LOG_BIAS = 2, FLAT_BIAS = 3 };
 enum { PLAIN = 0, GATED = 1, TAILED = 2, TURNED = 3 };
-
-typedef const __attribute__((address_space(1))) void* gptr_t;
-typedef __attribute__((address_space(3))) void* lptr_t;
 
 // shared last dimensions of the keys: key t's are row t, its own come first in kc
 struct KeyTail {
@@ -62,71 +57,6 @@ struct KeyTail {
   int width;  // columns there are; the rest of D is zeros
   int own;    // dimensions in kc, a multiple of 8
 };
-
-union frag_u {
-  shortx8 s;
-  shortx4 h[2];
-  unsigned int u[4];
-  bf16x8 v;
-};
-
-template <int N, typename F>
-DEVINL void static_for(F&& f) {
-  if constexpr (N > 0) {
-    static_for<N - 1>(f);
-    f(std::integral_constant<int, N - 1>{});
-  }
-}
-
-DEVINL unsigned int cvt2_bf16(float lo, float hi) {
-  const floatx2 f = {lo, hi};
-  const bf16x2 b = __builtin_convertvector(f, bf16x2);
-  return __builtin_bit_cast(unsigned int, b);
-}
-
-// Transposing reads of two V^T fragments, of each the halves HALF bytes apart. Written out
-// because the compiler puts a wait for all global loads in flight, the next tiles' among
-// them, before the builtin form. Nothing may touch v before await_values: no branch and
-// nothing that could run out of registers stands between the two.
-template <int AT, int HALF>
-DEVINL void read_values(shortx4 (&v)[4], unsigned a0, unsigned a1) {
-  asm volatile(
-      "ds_read_b64_tr_b16 %0, %4 offset:%6\n\t"
-      "ds_read_b64_tr_b16 %1, %4 offset:%7\n\t"
-      "ds_read_b64_tr_b16 %2, %5 offset:%6\n\t"
-      "ds_read_b64_tr_b16 %3, %5 offset:%7"
-      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3])
-      : "v"(a0), "v"(a1), "n"(AT), "n"(AT + HALF)
-      : "memory");
-}
-
-DEVINL void await_values(shortx4 (&v)[4]) {
-  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])::"memory");
-}
-
-// Sequence and first row of the nb-th block of ``rows`` rows, counted through the
-// sequences; false past the last. A lane per sequence.
-DEVINL bool find_block(const int* cu, int S, int rows, int nb, int lane, int& seq, int& off) {
-  for (int s0 = 0; s0 < S; s0 += WAVE) {
-    const int s = s0 + lane;
-    const int n = s < S ? (cu[s + 1] - cu[s] + rows - 1) / rows : 0;
-    int end = n;
-#pragma unroll
-    for (int d = 1; d < WAVE; d <<= 1) {
-      const int before = __shfl_up(end, d, WAVE);
-      if (lane >= d) end += before;
-    }
-    const unsigned long long past = __ballot(end > nb);
-    if (past) {
-      const int at = __builtin_ctzll(past);
-      seq = s0 + at;
-      off = (nb - __builtin_amdgcn_readlane(end - n, at)) * rows;
-      return true;
-    }
-    nb -= __builtin_amdgcn_readlane(end, WAVE - 1);
-  }
-  return false;
-}
 
 // HG: query heads per workgroup; PAGED: pages are whole tiles
 template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED>
