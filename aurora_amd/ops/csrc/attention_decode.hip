@@ -1,203 +1,372 @@
 // Paged-KV decode attention for gfx950 (one new token per sequence).
 //
-// Memory-bound by the KV read; the kernel streams each (seq, kv_head)'s
-// pages once at 16 B/lane and amortises the read over all G grouped query
-// heads (GQA).  Two levers keep it at streaming rate:
-//  * token-group software pipelining: each D/8-lane group prefetches K/V
-//    for 4 tokens before the (serial) online-softmax updates, so the
-//    memory system always has 8 x 16 B loads in flight per lane-group
-//    (the naive one-token loop is latency-bound through the o-rescale
-//    dependency chain: measured 1.07 TB/s at B=16 -> this structure);
-//  * flash-decode context splits: grid.z partitions the context into
-//    contiguous chunks so small batches still put >=512 workgroups on the
-//    256-CU chip; per-chunk (m, l, o) partials combine in a second kernel.
+// Memory-bound by the KV read; a workgroup streams a stretch of one (sequence, kv head)
+// once for up to 16 query heads of the group, four waves taking 32 keys in turn:
+//  * scores are S^T = K Q^T and results O^T = V^T P^T on the matrix cores, so a lane owns
+//    a head and maxima, sums and rescaling need no exchange. Keys come from the cache
+//    straight as A fragments; values through registers and the wave's own LDS, from where
+//    transposing reads give V^T with its keys in the order in which the scores lie. Nothing
+//    is shared between waves until the end, so there is no barrier in the loop;
+//  * the next 32 keys and values are under way while 32 are computed (16 KB a wave);
+//  * weights keep their 32 bits: each is the sum of two bf16 numbers and meets the values
+//    twice; O is rescaled only when a score exceeds the reference by DEC_SLACK powers
+//    of two;
+//  * contexts are cut into stretches of equal length, found on the device from all context
+//    lengths (``split_length``), so that a few long ones do not keep the others waiting
+//    and few sequences still fill the chip; a second kernel merges the stretches of a
+//    sequence that has several.
+// Measured in a graph, before and now (vector dot products, 64 keys at a time, as many
+// stretches for every sequence): 96 sequences of 500 to 2900 keys, 32 heads over 8,
+// 128 wide, 210 and 136 us (4.9 TB/s; a large read reaches 5.5 to 5.8), the same in fp8 211
+// and 90; 256 of 1600 326 and 289 (5.8 TB/s); 32 of 600 to 2500 66 and 43; one of 12000 102
+// and 26, one of 777 20 and 13; 7 heads over one, 40 of 300 to 3000, 90 and 37; fp8 64 wide,
+// 23 of 300 to 5000, 44 and 24. fp8 is bound by widening its values; a single sequence by
+// the two launches and one round trip to memory.
 //
 // Replaces the per-token provider round-trip of the reference agent loop
 // (reference: server/chat/backend/agent/llm.py:192) with an in-process
 // batched decode step.
+#include "flash_tiles.h"
 #include "head_turn.h"
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
 #define CUR_STREAM c10::hip::getCurrentHIPStream().stream()
 
-#ifndef TUNR
-#define TUNR 4  // tokens prefetched per group iteration (8 measured neutral)
-#endif
+#define DEC_KEYS 32       // keys a wave takes at a time
+#define DEC_WAVES 4
+#define DEC_HEADS 16      // query heads of a workgroup
+#define DEC_SLACK 10.f    // weights stay below 2^DEC_SLACK
+#define DEC_TARGET 1024   // workgroups that the contexts are cut into
 
 enum { NO_BIAS = 0, LINEAR_BIAS = 1, LOG_BIAS = 2, FLAT_BIAS = 3 };
 
+// keys of a sequence that its query sees: [first, L)
+struct Seen {
+  int window, chunk;
+  DEVINL int first(int L) const {
+    int lo = window > 0 ? max(0, L - window) : 0;
+    if (chunk > 0 && L > 0) lo = max(lo, L - 1 - (L - 1) % chunk);
+    return lo;
+  }
+};
+
+// Keys per stretch, a multiple of 128 (one round of the waves): what leaves about ``target``
+// stretches over all sequences and head tiles. All lanes of a wave.
+DEVINL int split_length(const int* ctx, int B, int tiles, int target, const Seen& seen,
+                        int lane) {
+  long sum = 0;
+  for (int s = lane; s < B; s += WAVE) sum += ctx[s] - seen.first(ctx[s]);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, WAVE);
+  const long per = (sum * tiles + target - 1) / target;
+  return (int)max(128L, (per + 127) / 128 * 128);
+}
+
+DEVINL int splits_of(int seen, int length) { return max(1, (seen + length - 1) / length); }
+
+// sequence and place of stretch ``idx``, the sequence's first stretch and their number
+DEVINL bool find_split(const int* ctx, int B, int length, const Seen& seen, int idx, int lane,
+                       int& b, int& s, int& n) {
+  for (int b0 = 0; b0 < B; b0 += WAVE) {
+    const int x = b0 + lane;
+    const int c = x < B ? splits_of(ctx[x] - seen.first(ctx[x]), length) : 0;
+    int end = c;
+#pragma unroll
+    for (int d = 1; d < WAVE; d <<= 1) {
+      const int before = __shfl_up(end, d, WAVE);
+      if (lane >= d) end += before;
+    }
+    const unsigned long long past = __ballot(end > idx);
+    if (past) {
+      const int at = __builtin_ctzll(past);
+      b = b0 + at;
+      n = __builtin_amdgcn_readlane(c, at);
+      s = idx - (__builtin_amdgcn_readlane(end, at) - n);
+      return true;
+    }
+    idx -= __builtin_amdgcn_readlane(end, WAVE - 1);
+  }
+  return false;
+}
+
+// Four V^T fragments at once: rows 4 g .. and 16 + 4 g .. of d-tiles at four addresses.
+template <int SECOND>
+DEVINL void read_value_tiles(shortx4 (&v)[8], unsigned a0, unsigned a1, unsigned a2,
+                             unsigned a3) {
+  asm volatile(
+      "ds_read_b64_tr_b16 %0, %8\n\t"
+      "ds_read_b64_tr_b16 %1, %8 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %2, %9\n\t"
+      "ds_read_b64_tr_b16 %3, %9 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %4, %10\n\t"
+      "ds_read_b64_tr_b16 %5, %10 offset:%12\n\t"
+      "ds_read_b64_tr_b16 %6, %11\n\t"
+      "ds_read_b64_tr_b16 %7, %11 offset:%12\n\t"
+      "s_waitcnt lgkmcnt(0)"
+      : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]),
+        "=&v"(v[6]), "=&v"(v[7])
+      : "v"(a0), "v"(a1), "v"(a2), "v"(a3), "n"(SECOND)
+      : "memory");
+}
+
 // BIAS: a distance penalty per head or none (see attention_prefill.hip), a window or
 // chunks of positions; sink: one more term of the denominator per head, or null;
-// FLAT_BIAS results may be turned back and gated
-template <int D, int DV, int G, bool FP8, int BIAS>
+// FLAT_BIAS results may be turned back and gated. PAGED: pages are whole tiles.
+// Without ``cut`` a workgroup takes a whole context.
+template <int D, int DV, bool FP8, int BIAS, bool PAGED>
 __global__ __launch_bounds__(256) void paged_decode_kernel(
     const __hip_bfloat16* __restrict__ q,   // [B, Hq, D]
-    const void* __restrict__ kc,  // [NP, Hkv, P, D] bf16 | fp8 e4m3
-    const void* __restrict__ vc,
-    __hip_bfloat16* __restrict__ out,       // [B, ostride], heads dv apart (CS==1)
-    float* __restrict__ part,               // [CS, B, Hq, DV+2] (CS>1)
+    // (not __restrict__: loads of them must stay before the waits that count them)
+    const void* kc,  // [NP, Hkv, P, D] bf16 | fp8 e4m3
+    const void* vc,
+    __hip_bfloat16* out,                    // [B, ostride], heads dv apart
+    float* part,                            // [stretches, Hq, DV + 2], where a context has several
     const int* __restrict__ block_tables,   // [B, MP]
     const int* __restrict__ ctx_lens,       // [B]
-    int Hkv, int NG,                        // NG: head groups per kv head
-    int P, int MP, int CS, float scale,
+    int B, int Hq, int Hkv, int P, int MP, int cut, float scale,
     long ostride, int dv, float oscale,
-    const float* __restrict__ slopes, const float* __restrict__ rates, int window,
-    int chunk_of, const float* __restrict__ sink, HeadTurn turn) {
-  constexpr int GL = (D > DV ? D : DV) / 8;  // lanes per token-group
-  constexpr int TPW = WAVE / GL;   // token-groups per wave
-  constexpr int NW = 4;            // waves per workgroup
-  constexpr int NPART = NW * TPW;  // in-block partials to combine
-
-  const int b = blockIdx.x;
-  const int kvh = blockIdx.y / NG;
-  const int h0 = blockIdx.y * G;  // first query head of this workgroup
-  const int Hq = gridDim.y * G;
-  const int cs = blockIdx.z;
-  const int L = ctx_lens[b];
-  // contiguous chunk of the visible context for this split
-  int first = BIAS && window > 0 ? max(0, L - window) : 0;
-  if (BIAS && chunk_of > 0) first = max(first, L - 1 - (L - 1) % chunk_of);
-  const int chunk = (L - first + CS - 1) / CS;
-  const int t_lo = first + cs * chunk;
-  const int t_hi = min(L, t_lo + chunk);
-  const int tid = threadIdx.x;
-  const int wave = tid / WAVE;
-  const int lane = tid % WAVE;
-  const int grp = lane / GL;   // token-group within the wave
-  const int sub = lane % GL;   // 16-B slot within the token row
-
-  shortx8 qf[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    if (DV > D && sub * 8 >= D)
-      qf[g] = shortx8{0, 0, 0, 0, 0, 0, 0, 0};
-    else
-      qf[g] = *reinterpret_cast<const shortx8*>(
-          q + ((long)b * Hq + h0 + g) * D + sub * 8);
+    const float* __restrict__ slopes, const float* __restrict__ rates, Seen seen,
+    const float* __restrict__ sink, HeadTurn turn) {
+  constexpr int NC = D / 32, NDT = DV / 16;
+  constexpr int EB = FP8 ? 1 : 2;
+  constexpr int VU = DV / 8, LV = DEC_KEYS * VU / WAVE;  // 16-B units of a value, a lane's
+  constexpr int STAGE = DEC_KEYS * DV * 2;
+  const int lane = threadIdx.x % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int G = Hq / Hkv, NG = (G + DEC_HEADS - 1) / DEC_HEADS;
+  const int tiles = Hkv * NG, idx = blockIdx.x / tiles, tile = blockIdx.x % tiles;
+  const int kvh = tile / NG, h0 = kvh * G + tile % NG * DEC_HEADS;
+  const int GT = min(DEC_HEADS, kvh * G + G - h0);
+  int b = idx, split = 0, nsplits = 1, length = 0x7fffffff;
+  if (cut) {
+    length = split_length(ctx_lens, B, tiles, DEC_TARGET, seen, lane);
+    if (!find_split(ctx_lens, B, length, seen, idx, lane, b, split, nsplits)) return;
+    // the same in all lanes, which the compiler cannot see
+    b = __builtin_amdgcn_readfirstlane(b);
+    split = __builtin_amdgcn_readfirstlane(split);
+    nsplits = __builtin_amdgcn_readfirstlane(nsplits);
+    length = __builtin_amdgcn_readfirstlane(length);
   }
-  float slope[G], rate[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    slope[g] = BIAS && BIAS != FLAT_BIAS ? slopes[h0 + g] : 0.f;
-    rate[g] = BIAS == LOG_BIAS ? rates[h0 + g] : 0.f;
-  }
-  // 16-B column of a key / value row this lane reads (lanes past the narrower
-  // of the two re-read its last column and contribute nothing)
-  const int ksub = min(sub * 8, D - 8), vsub = min(sub * 8, DV - 8);
-
-  float m[G], l[G], o[G][8];
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    m[g] = -1e30f;
-    l[g] = 0.f;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) o[g][j] = 0.f;
-  }
-
+  const int L = ctx_lens[b], first = seen.first(L);
+  const int t_lo = first + (cut ? split * length : 0);
+  const int t_hi = cut ? min(L, t_lo + length) : L;
   const int* bt = block_tables + (long)b * MP;
-  const int stride = NW * TPW;
-  // groups stride the chunk; TUNR tokens prefetched per iteration
-  for (int t0 = t_lo + (wave * TPW + grp) * TUNR; t0 < t_hi;
-       t0 += stride * TUNR) {
-    shortx8 kf[TUNR], vf[TUNR];
-    int nt = 0;
-    if constexpr (FP8) {
-      // fp8 cache: half the KV stream bytes (the kernel is KV-bound at
-      // ~6.15 TB/s in bf16); 8-byte loads, convert
-      // to bf16 fragments in-register
-      u64b k8[TUNR], v8[TUNR];
+  const int head = lane & 15, g = lane >> 4;
+  const bool mine = head < GT;
+
+  // LDS: a tile of values per wave; at the end the waves' results
+  __shared__ __attribute__((aligned(16))) char smem[DEC_WAVES * STAGE];
+  __shared__ float s_m[DEC_WAVES][DEC_HEADS], s_l[DEC_WAVES][DEC_HEADS];
+  static_assert(sizeof(smem) >= DEC_WAVES * DEC_HEADS * DV * 4);
+  char* ring = smem + wave * STAGE;
+  const unsigned ring_at =
+      (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring;
+
+  frag_u qf[NC];
 #pragma unroll
-      for (int u = 0; u < TUNR; ++u) {
-        const int t = t0 + u;
-        const int tc = min(t, t_hi - 1);
-        const long row = ((long)bt[tc / P] * Hkv + kvh) * P + (tc % P);
-        k8[u] = *reinterpret_cast<const u64b*>((const unsigned char*)kc + row * D + ksub);
-        v8[u] = *reinterpret_cast<const u64b*>((const unsigned char*)vc + row * DV + vsub);
-      }
+  for (int c = 0; c < NC; ++c) {
+    qf[c].s = shortx8{0, 0, 0, 0, 0, 0, 0, 0};
+    if (mine)
+      qf[c].s = *reinterpret_cast<const shortx8*>(q + ((long)b * Hq + h0 + head) * D + c * 32 +
+                                                  g * 8);
+  }
+  const float c2 = scale * LOG2E;  // scores in units of log 2
+  const float slope = BIAS == LINEAR_BIAS && mine ? slopes[h0 + head] * LOG2E
+                      : BIAS == LOG_BIAS && mine  ? slopes[h0 + head] : 0.f;
+  const float rate = BIAS == LOG_BIAS && mine ? rates[h0 + head] : 0.f;
+
+  float m = -1e30f, l = 0.f;
+  floatx4 o[NDT];
 #pragma unroll
-      for (int u = 0; u < TUNR; ++u) {
-        kf[u] = fp8x8_to_bf16x8(k8[u]);
-        vf[u] = fp8x8_to_bf16x8(v8[u]);
-      }
-    } else {
+  for (int dt = 0; dt < NDT; ++dt) o[dt] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+  // this wave's tiles: t0 + 128 i. Row of key t in a head's cache; past the end the last
+  // key again
+  auto row_of = [&](int t) -> long {
+    t = min(t, t_hi - 1);
+    return ((long)bt[t / P] * Hkv + kvh) * P + t % P;
+  };
+  auto value_unit = [&](int x, int& row, int& col) {
+    const unsigned u = lane + x * WAVE;
+    row = u / VU;
+    col = ((u % VU) ^ (DV == 64 ? (row >> 1 & 3) << 1 : (row & 7) << 1)) * 8;
+  };
+  // (Through registers and not straight to LDS: beside direct-to-LDS loads the compiler
+  // turns every wait for a register into a wait for all loads.)
+  using raw = std::conditional_t<FP8, u64b, shortx8>;
+  raw kr[2][2][NC], vr[LV];   // K: [parity][16 keys][32 dimensions]
+  // Rows of a tile: past the end the last tile again, so that every round has as many
+  // loads. PAGED: its first row is looked up a tile ahead.
+  long page_row = 0;
+  auto tile_at = [&](int t0) { return min(t0, (t_hi - 1) & -DEC_KEYS); };
+  auto lookup = [&](int t0) {
+    if constexpr (PAGED) page_row = row_of(tile_at(t0));
+  };
+  auto source = [&](int t0, int key, long first_row) -> long {
+    t0 = tile_at(t0);
+    if constexpr (!PAGED) return row_of(t0 + key);
+    return first_row + (t0 + DEC_KEYS <= t_hi ? key : min(key, t_hi - 1 - t0));
+  };
+  auto load_keys = [&](int t0, long first_row, auto PARITY) {
+    constexpr int parity = decltype(PARITY)::value;
 #pragma unroll
-      for (int u = 0; u < TUNR; ++u) {
-        const int t = t0 + u;
-        const int tc = min(t, t_hi - 1);  // clamped prefetch (masked below)
-        const long row = ((long)bt[tc / P] * Hkv + kvh) * P + (tc % P);
-        kf[u] = *reinterpret_cast<const shortx8*>((const __hip_bfloat16*)kc + row * D + ksub);
-        vf[u] = *reinterpret_cast<const shortx8*>((const __hip_bfloat16*)vc + row * DV + vsub);
+    for (int k = 0; k < 2; ++k) {
+      const char* src = (const char*)kc + (source(t0, k * 16 + head, first_row) * D + g * 8) * EB;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        kr[parity][k][c] = *reinterpret_cast<const raw*>(src + c * 32 * EB);
+    }
+  };
+  auto load_values = [&](int t0, long first_row) {
+#pragma unroll
+    for (int x = 0; x < LV; ++x) {
+      int row, col;
+      value_unit(x, row, col);
+      vr[x] = *reinterpret_cast<const raw*>(
+          (const char*)vc + (source(t0, row, first_row) * DV + col) * EB);
+    }
+  };
+  auto widen = [](raw x) -> shortx8 {
+    if constexpr (FP8) return fp8x8_to_bf16x8(x);
+    else return x;
+  };
+  // where a lane's values lie: lane i of 16 reads 8 bytes of row 4 g + i / 4
+  const int vrow = 4 * g + (head >> 2);
+  const unsigned vat = ring_at + vrow * DV * 2, vcol =
+      ((((head & 3) >> 1) ^ (DV == 64 ? (vrow >> 1 & 3) << 1 : (vrow & 7) << 1)) << 4) +
+      (head & 1) * 8;
+
+  // one round: the tile at t0, whose keys are in kr[parity] and whose values in vr; the
+  // wave's next tile is requested as soon as its registers are free
+  constexpr int ROUND = DEC_WAVES * DEC_KEYS;
+  auto compute = [&](int t0, auto PARITY) {
+    constexpr int parity = decltype(PARITY)::value;
+    const long next_row = page_row;
+    load_keys(t0 + ROUND, next_row, std::integral_constant<int, 1 - parity>{});
+    lookup(t0 + 2 * ROUND);
+    __builtin_amdgcn_sched_barrier(0);
+    floatx4 st[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      st[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        frag_u kf;
+        kf.s = widen(kr[parity][k][c]);
+        st[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.v, qf[c].v, st[k], 0, 0, 0);
       }
     }
+    float x[8];  // scores of keys 16 k + 4 g + r
+    float mx = -INFINITY;
 #pragma unroll
-    for (int u = 0; u < TUNR; ++u) {
-      if (t0 + u >= t_hi) break;
-      float s[G];
+    for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int g = 0; g < G; ++g) {
-        s[g] = group_sum<GL>(dot8_bf16_fast(kf[u], qf[g])) * scale;
+      for (int r = 0; r < 4; ++r) {
+        const int t = t0 + k * 16 + 4 * g + r;
+        float y = st[k][r] * c2;
         if constexpr (BIAS == LINEAR_BIAS || BIAS == LOG_BIAS) {
-          const float dist = (float)(L - 1 - t0 - u);
-          s[g] -= slope[g] * (BIAS == LOG_BIAS ? __logf(1.f + rate[g] * dist) : dist);
+          const float dist = (float)(L - 1 - t);
+          y -= slope * (BIAS == LOG_BIAS ? __builtin_amdgcn_logf(1.f + rate * dist) : dist);
         }
-        // defer-style rescale: the running max rarely grows, so the O/l
-        // rescale (8*G VALU per token) is branch-skipped when it does not
-        if (s[g] > m[g]) {
-          const float alpha = __expf(m[g] - s[g]);
-          m[g] = s[g];
-          l[g] *= alpha;
-#pragma unroll
-          for (int j = 0; j < 8; ++j) o[g][j] *= alpha;
-        }
-        const float pv = __expf(s[g] - m[g]);
-        l[g] += pv;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          o[g][j] += pv * bf16_to_f32((unsigned short)vf[u][j]);
+        if (t >= t_hi || (BIAS && t < t_lo)) y = -INFINITY;
+        x[k * 4 + r] = y;
+        mx = fmaxf(mx, y);
       }
+    if (__any(mx > m + DEC_SLACK)) {
+      mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE));
+      const float mn = fmaxf(m, mx), alpha = __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
+    }
+    frag_u hi, lo;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float p0 = __builtin_amdgcn_exp2f(x[2 * j] - m);
+      const float p1 = __builtin_amdgcn_exp2f(x[2 * j + 1] - m);
+      l += p0 + p1;
+      hi.u[j] = cvt2_bf16(p0, p1);
+      lo.u[j] = cvt2_bf16(p0 - __builtin_bit_cast(float, hi.u[j] << 16),
+                          p1 - __builtin_bit_cast(float, hi.u[j] & 0xffff0000u));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < LV; ++x)
+      *reinterpret_cast<shortx8*>(ring + (lane + x * WAVE) * 16) = widen(vr[x]);
+    load_values(t0 + ROUND, next_row);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int d4 = 0; d4 < NDT; d4 += 4) {
+      shortx4 v[8];
+      read_value_tiles<16 * DV * 2>(v, vat + (vcol ^ (d4 * 32)), vat + (vcol ^ (d4 * 32 + 32)),
+                                    vat + (vcol ^ (d4 * 32 + 64)), vat + (vcol ^ (d4 * 32 + 96)));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        frag_u vf;
+        vf.h[0] = v[2 * j];
+        vf.h[1] = v[2 * j + 1];
+        o[d4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, lo.v, o[d4 + j], 0, 0, 0);
+        o[d4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, hi.v, o[d4 + j], 0, 0, 0);
+      }
+    }
+  };
+  using EVEN = std::integral_constant<int, 0>;
+  using ODD = std::integral_constant<int, 1>;
+  // tiles lie within pages, so the first may begin before the stretch
+  int t0 = t_lo - (BIAS ? t_lo % DEC_KEYS : 0) + wave * DEC_KEYS;
+  if (t0 < t_hi) {
+    lookup(t0);
+    load_keys(t0, page_row, EVEN{});
+    load_values(t0, page_row);
+    lookup(t0 + ROUND);
+    for (;;) {
+      compute(t0, EVEN{});
+      if ((t0 += ROUND) >= t_hi) break;
+      compute(t0, ODD{});
+      if ((t0 += ROUND) >= t_hi) break;
     }
   }
 
-  // ---- combine the NPART in-block partials per head through LDS ----
-  __shared__ float s_m[G][NPART];
-  __shared__ float s_l[G][NPART];
-  __shared__ float s_o[G][NPART][DV];
-  const int pidx = wave * TPW + grp;
-#pragma unroll
-  for (int g = 0; g < G; ++g) {
-    if (sub == 0) {
-      s_m[g][pidx] = m[g];
-      s_l[g][pidx] = l[g];
+  // ---- the waves' results
+  l += __shfl_xor(l, 16, WAVE);
+  l += __shfl_xor(l, 32, WAVE);
+  __syncthreads();
+  float* so = (float*)smem;  // [waves][heads][DV]
+  if (mine) {
+    if (g == 0) {
+      s_m[wave][head] = m;
+      s_l[wave][head] = l;
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      if (DV >= D || sub * 8 < DV) s_o[g][pidx][sub * 8 + j] = o[g][j];
+    for (int dt = 0; dt < NDT; ++dt)
+      *reinterpret_cast<floatx4*>(so + (wave * DEC_HEADS + head) * DV + dt * 16 + 4 * g) = o[dt];
   }
   __syncthreads();
-  for (int gd = tid; gd < G * DV; gd += blockDim.x) {
-    const int g = gd / DV, d = gd % DV;
-    const bool ends = BIAS && CS == 1 && sink;  // the sink counts once
-    const float first = ends ? sink[h0 + g] : -1e30f;
-    float M = first;
-#pragma unroll 4
-    for (int i = 0; i < NPART; ++i) M = fmaxf(M, s_m[g][i]);
-    float Lsum = ends ? __expf(first - M) : 0.f, O = 0.f;
-#pragma unroll 4
-    for (int i = 0; i < NPART; ++i) {
-      const float w = __expf(s_m[g][i] - M);
-      Lsum += w * s_l[g][i];
-      O += w * s_o[g][i][d];
+  for (int gd = threadIdx.x; gd < GT * DV; gd += blockDim.x) {
+    const int hh = gd / DV, d = gd % DV;
+    const bool ends = BIAS && nsplits == 1 && sink;  // the sink counts once
+    const float s0 = ends ? fmaxf(sink[h0 + hh] * LOG2E, -1e30f) : -1e30f;
+    float M = s0;
+#pragma unroll
+    for (int w = 0; w < DEC_WAVES; ++w) M = fmaxf(M, s_m[w][hh]);
+    float Lsum = ends ? __builtin_amdgcn_exp2f(s0 - M) : 0.f, O = 0.f;
+#pragma unroll
+    for (int w = 0; w < DEC_WAVES; ++w) {
+      const float f = __builtin_amdgcn_exp2f(s_m[w][hh] - M);
+      Lsum += f * s_l[w][hh];
+      O += f * so[(w * DEC_HEADS + hh) * DV + d];
     }
-    const long hq = (long)b * Hq + h0 + g;
-    if (CS == 1) {
+    if (nsplits == 1) {
       float y = O / Lsum * oscale;
-      if constexpr (BIAS == FLAT_BIAS) y = turned<bf16_t>(turn, y, b, L - 1, h0 + g, d, dv);
+      if constexpr (BIAS == FLAT_BIAS) y = turned<bf16_t>(turn, y, b, L - 1, h0 + hh, d, dv);
       if (!BIAS || d < dv)
-        *(unsigned short*)(out + b * ostride + (long)(h0 + g) * dv + d) = f32_to_bf16(y);
+        *(unsigned short*)(out + b * ostride + (long)(h0 + hh) * dv + d) = f32_to_bf16(y);
     } else {
-      // emit an un-normalised chunk partial: {o*w-sum, m, l}
-      float* dst = part + ((long)cs * gridDim.x * Hq + hq) * (DV + 2);
+      // an un-normalised partial result, its reference and its sum
+      float* dst = part + ((long)idx * Hq + h0 + hh) * (DV + 2);
       dst[d] = O;
       if (d == 0) {
         dst[DV] = M;
@@ -207,41 +376,50 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
   }
 }
 
-// combine CS chunk partials -> out; one wave per (b, h)
-template <int D>
-__global__ void decode_combine_kernel(const float* __restrict__ part,
-                                      __hip_bfloat16* __restrict__ out,
-                                      int CS, long BH, int Hq, long ostride,
-                                      int dv, float oscale,
-                                      const float* __restrict__ sink, HeadTurn turn,
-                                      const int* __restrict__ ctx_lens) {
-  const long bh = blockIdx.x * (blockDim.x / WAVE) + threadIdx.x / WAVE;
-  if (bh >= BH) return;
-  const int lane = threadIdx.x % WAVE;
-  const float first = sink ? sink[bh % Hq] : -1e30f;
-  float M = first;
-  for (int s = 0; s < CS; ++s)
-    M = fmaxf(M, part[((long)s * BH + bh) * (D + 2) + D]);
-  float Lsum = sink ? __expf(first - M) : 0.f;
-  for (int s = 0; s < CS; ++s) {
-    const float* p = part + ((long)s * BH + bh) * (D + 2);
-    Lsum += __expf(p[D] - M) * p[D + 1];
+// Merges the stretches of a sequence that has several; a wave per (sequence, head). All
+// references are read at once, then the results in groups of independent loads.
+template <int DV>
+__global__ __launch_bounds__(256) void decode_combine_kernel(
+    const float* __restrict__ part, __hip_bfloat16* __restrict__ out,
+    const int* __restrict__ ctx_lens, int B, int Hq, int tiles, long ostride, int dv,
+    float oscale, const float* __restrict__ sink, HeadTurn turn, Seen seen) {
+  const long bh = blockIdx.x * 4L + threadIdx.x / WAVE;
+  if (bh >= (long)B * Hq) return;
+  const int lane = threadIdx.x % WAVE, b = bh / Hq, h = bh % Hq;
+  const int length = split_length(ctx_lens, B, tiles, DEC_TARGET, seen, lane);
+  const int n = splits_of(ctx_lens[b] - seen.first(ctx_lens[b]), length);
+  if (n == 1) return;
+  int before = 0;  // stretches of the sequences before this
+  for (int s = lane; s < b; s += WAVE)
+    before += splits_of(ctx_lens[s] - seen.first(ctx_lens[s]), length);
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) before += __shfl_xor(before, d, WAVE);
+  const float* src = part + ((long)before * Hq + h) * (DV + 2);
+  const long step = (long)Hq * (DV + 2);
+  const float s0 = sink ? fmaxf(sink[h] * LOG2E, -1e30f) : -1e30f;
+  float M = s0;
+  for (int s = lane; s < n; s += WAVE) M = fmaxf(M, src[s * step + DV]);
+  M = wave_max(M);
+  float Lsum = 0.f;
+  for (int s = lane; s < n; s += WAVE)
+    Lsum += __builtin_amdgcn_exp2f(src[s * step + DV] - M) * src[s * step + DV + 1];
+  Lsum = wave_sum(Lsum) + (sink ? __builtin_amdgcn_exp2f(s0 - M) : 0.f);
+  constexpr int N = DV / WAVE;
+  float O[N] = {};
+#pragma unroll 8
+  for (int s = 0; s < n; ++s) {
+    const float f = __builtin_amdgcn_exp2f(src[s * step + DV] - M);
+#pragma unroll
+    for (int j = 0; j < N; ++j) O[j] += f * src[s * step + lane + j * WAVE];
   }
-  for (int d = lane; d < dv; d += WAVE) {
-    float O = 0.f;
-    for (int s = 0; s < CS; ++s) {
-      const float* p = part + ((long)s * BH + bh) * (D + 2);
-      O += __expf(p[D] - M) * p[d];
-    }
-    float y = O / Lsum * oscale;
-    if (turn.cs || turn.gate)
-      y = turned<bf16_t>(turn, y, bh / Hq, ctx_lens[bh / Hq] - 1, bh % Hq, d, dv);
-    *(unsigned short*)(out + bh / Hq * ostride + bh % Hq * dv + d) = f32_to_bf16(y);
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int d = lane + j * WAVE;
+    float y = O[j] / Lsum * oscale;
+    if (turn.cs || turn.gate) y = turned<bf16_t>(turn, y, b, ctx_lens[b] - 1, h, d, dv);
+    if (d < dv) *(unsigned short*)(out + b * ostride + (long)h * dv + d) = f32_to_bf16(y);
   }
 }
-
-// query heads sharing one K/V stream: the largest tile that divides the group
-static int head_tile(int G) { return G % 8 == 0 ? 8 : G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1; }
 
 template <int D, int DV, bool FP8, int BIAS>
 static void decode_launch(const torch::Tensor& q, const torch::Tensor& kc,
@@ -249,35 +427,37 @@ static void decode_launch(const torch::Tensor& q, const torch::Tensor& kc,
                           const torch::Tensor& ctx, __hip_bfloat16* out, long ostride,
                           int dv, float scale, float oscale, const float* slopes,
                           const float* rates, int window, int chunk, const float* sink,
-                          const HeadTurn& turn, int CS) {
+                          const HeadTurn& turn) {
   const int B = q.size(0), Hq = q.size(1);
   const int Hkv = kc.size(1), P = kc.size(2), MP = bt.size(1);
-  const int G = Hq / Hkv, GT = head_tile(G);
+  const int tiles = Hkv * ((Hq / Hkv + DEC_HEADS - 1) / DEC_HEADS);
+  // Contexts stay whole while the longest that can be seen is short or the workgroups are
+  // many: cutting costs its search and the second kernel, and evens out little then. Whole
+  // and cut, 128 wide, 8 kv heads: 64 sequences of 2000 keys 100 and 110 us, 100 of 50 keys
+  // 7 and 13; behind a window of 1024, 32 sequences 30 and 40, 16 sequences 19 and 27, 2
+  // sequences (outside the rule) 16 and 13. What it gives up: 64 sequences of 300 to 8000
+  // keys 229 and 215.
+  long longest = (long)MP * P;
+  if (window > 0) longest = std::min<long>(longest, window);
+  if (chunk > 0) longest = std::min<long>(longest, chunk);
+  const bool cut = longest > std::max<long>(256, (long)B * tiles * B * tiles / 16);
+  const long most = cut ? B + DEC_TARGET / tiles + 1 : B;  // stretches there can be
   torch::Tensor part;
-  if (CS > 1)
-    part = torch::empty({CS, (long)B * Hq, DV + 2}, q.options().dtype(torch::kFloat32));
-  float* pp = CS > 1 ? part.data_ptr<float>() : nullptr;
-  dim3 grid(B, Hkv * (G / GT), CS), block(256);
-  auto stream = CUR_STREAM;
-#define LAUNCH(GG)                                                              \
-  hipLaunchKernelGGL((paged_decode_kernel<D, DV, GG, FP8, BIAS>), grid, block,  \
-                     0, stream, (const __hip_bfloat16*)q.data_ptr(),            \
-                     kc.data_ptr(), vc.data_ptr(), out, pp, bt.data_ptr<int>(), \
-                     ctx.data_ptr<int>(), Hkv, G / GT, P, MP, CS, scale,        \
-                     ostride, dv, oscale, slopes, rates, window, chunk, sink, turn)
-  switch (GT) {
-    case 8: LAUNCH(8); break;
-    case 4: LAUNCH(4); break;
-    case 2: LAUNCH(2); break;
-    default: LAUNCH(1); break;
-  }
-#undef LAUNCH
-  if (CS > 1) {
-    const long BH = (long)B * Hq;
-    hipLaunchKernelGGL((decode_combine_kernel<DV>), dim3((BH + 3) / 4), dim3(256), 0,
-                       stream, pp, out, CS, BH, Hq, ostride, dv, oscale, sink, turn,
-                       ctx.data_ptr<int>());
-  }
+  if (cut) part = torch::empty({most, Hq, DV + 2}, q.options().dtype(torch::kFloat32));
+  float* pp = cut ? part.data_ptr<float>() : nullptr;
+  const Seen seen = {window, chunk};
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(most * tiles), dim3(256), 0, CUR_STREAM,
+                       (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out,
+                       pp, bt.data_ptr<int>(), ctx.data_ptr<int>(), B, Hq, Hkv, P, MP,
+                       cut ? 1 : 0, scale, ostride, dv, oscale, slopes, rates, seen, sink, turn);
+  };
+  if (P % DEC_KEYS == 0) launch(paged_decode_kernel<D, DV, FP8, BIAS, true>);
+  else launch(paged_decode_kernel<D, DV, FP8, BIAS, false>);
+  if (cut)
+    hipLaunchKernelGGL((decode_combine_kernel<DV>), dim3(((long)B * Hq + 3) / 4), dim3(256), 0,
+                       CUR_STREAM, pp, out, ctx.data_ptr<int>(), B, Hq, tiles, ostride, dv,
+                       oscale, sink, turn, seen);
   HIP_CHECK_KERNEL();
 }
 
@@ -290,15 +470,12 @@ torch::Tensor paged_attention_decode(torch::Tensor q, torch::Tensor kc,
   TORCH_CHECK(D == 128 || D == 64, "unsupported head_dim ", D);
   auto out = torch::empty_like(q);
   if (B == 0) return out;
-  // context splits: fill target ~1024 WGs. At B=64 the LDS-bound residency
-  // is only 2 WGs/CU, so deeper splits buy memory-level parallelism
-  const int CS = std::max(1, std::min(8, 1024 / std::max(B * Hkv, 1)));
   auto* o = (__hip_bfloat16*)out.data_ptr();
   const long stride = (long)Hq * D;
   const bool fp8 = kc.dtype() == torch::kFloat8_e4m3fn;
 #define RUN(DD, F8) \
   decode_launch<DD, DD, F8, NO_BIAS>(q, kc, vc, bt, ctx, o, stride, D, (float)scale, \
-                                     1.f, nullptr, nullptr, 0, 0, nullptr, HeadTurn{}, CS)
+                                     1.f, nullptr, nullptr, 0, 0, nullptr, HeadTurn{})
   if (D == 128) { if (fp8) RUN(128, true); else RUN(128, false); }
   else { if (fp8) RUN(64, true); else RUN(64, false); }
 #undef RUN
@@ -328,10 +505,6 @@ void biased_attention_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc
   TORCH_CHECK(ctx.numel() == B && bt.size(0) == B && bt.dtype() == torch::kInt32 &&
               ctx.dtype() == torch::kInt32);
   if (B == 0) return;
-  // a split of fewer than 64 visible keys is not worth its combine
-  int CS = std::max(1, std::min(8, 1024 / std::max(B * Hkv, 1)));
-  for (long seen : {window, chunk})
-    if (seen > 0) CS = std::max(1, std::min(CS, (int)((seen + 63) / 64)));
   auto* o = (__hip_bfloat16*)out.data_ptr() + col;
   const float* rp = rates ? rates->data_ptr<float>() : nullptr;
   const float* sp = slopes ? slopes->data_ptr<float>() : nullptr;
@@ -339,7 +512,7 @@ void biased_attention_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc
 #define RUN1(DD, DVV, BB)                                                        \
   decode_launch<DD, DVV, false, BB>(q, kc, vc, bt, ctx, o, out.stride(0),        \
                                     (int)dv, (float)scale, (float)oscale,        \
-                                    sp, rp, (int)window, (int)chunk, snk, ht, CS)
+                                    sp, rp, (int)window, (int)chunk, snk, ht)
 #define RUN(DD, DVV)                         \
   if (!sp) RUN1(DD, DVV, FLAT_BIAS);         \
   else if (rp) RUN1(DD, DVV, LOG_BIAS);      \
