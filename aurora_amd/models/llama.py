@@ -107,12 +107,12 @@ class LlamaAttention(nn.Module):
         meta: AttnMetadata,
     ) -> torch.Tensor:
         T = x.shape[0]
-        qkv = self.qkv_proj(x)
+        qkv = self.qkv_proj.parts(x)
         k_cache, v_cache = kv_cache
-        # fused split + RoPE + paged K/V scatter (one kernel on GPU)
+        # fused split + bias + RoPE + paged K/V scatter (one kernel on GPU)
         q = ops.fused_rope_kv_write(qkv, meta.positions, meta.slot_mapping,
                                     cos_sin, k_cache, v_cache,
-                                    self.n_heads, self.n_kv_heads)
+                                    self.n_heads, self.n_kv_heads, self.qkv_proj.bias)
         if meta.mode == "prefill":
             o = ops.attention_prefill_paged(
                 q, k_cache, v_cache, meta.block_tables,
@@ -135,7 +135,7 @@ class LlamaAttention(nn.Module):
                 meta.dec_context_lens, self.scale,
             ) if T > Tp else q[:0]
             o = torch.cat([o_pre, o_dec]) if (Tp and T > Tp) else (o_pre if Tp else o_dec)
-        return self.o_proj(o.reshape(T, self.n_heads * self.head_dim))
+        return self.o_proj.parts(o.reshape(T, self.n_heads * self.head_dim))
 
 
 class LlamaMLP(nn.Module):
@@ -145,7 +145,11 @@ class LlamaMLP(nn.Module):
         self.down = RowParallelLinear(spec.intermediate_size, spec.hidden_size, dtype=dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down(ops.silu_mul(self.gate_up(x)))
+        return self.down(ops.linear_silu_mul(x, self.gate_up.weight))
+
+    def parts(self, x: torch.Tensor) -> torch.Tensor:
+        """As ``forward``, possibly in parts (``ops.linear_parts``)."""
+        return self.down.parts(ops.linear_silu_mul(x, self.gate_up.weight))
 
 
 class _FullWidthMLP(nn.Module):
@@ -162,7 +166,7 @@ class _FullWidthMLP(nn.Module):
             requires_grad=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return ops.linear(ops.silu_mul(ops.linear(x, self.gate_up)), self.down)
+        return ops.linear(ops.linear_silu_mul(x, self.gate_up), self.down)
 
 
 class MoEMLP(nn.Module):
@@ -298,8 +302,8 @@ class LlamaDecoderLayer(nn.Module):
             h, residual = ops.rmsnorm_residual(x, residual, self.input_norm, self.eps)
         a = self.attn(h, cos_sin, kv_cache, meta)
         h, residual = ops.rmsnorm_residual(a, residual, self.post_attn_norm, self.eps)
-        m = self.mlp(h)
-        return m, residual
+        m = self.mlp(h) if isinstance(self.mlp, MoEMLP) else self.mlp.parts(h)
+        return m, residual  # m is read by rmsnorm_residual, which adds up parts
 
 
 class LlamaForCausalLM(nn.Module):

@@ -159,15 +159,18 @@ def paged_attention_decode(
 
 
 def fused_rope_kv_write(qkv, positions, slots, cos_sin, k_cache, v_cache,
-                        n_heads: int, n_kv_heads: int):
+                        n_heads: int, n_kv_heads: int, bias=None):
     """Split fused qkv output, RoPE q/k, scatter k/v into the paged cache;
     returns contiguous roped q [T, Hq, D].  One kernel on GPU; composed
-    reference ops on CPU."""
+    reference ops on CPU. ``qkv`` may be a product in parts (``linear_parts``);
+    ``bias`` is added to it first."""
     if qkv.is_cuda:
         m = _require_hip("fused_rope_kv_write")
         return m.fused_rope_kv_write(qkv.contiguous(), positions.to(torch.int32),
                                      slots.to(torch.int32), cos_sin,
-                                     k_cache, v_cache, n_heads, n_kv_heads)
+                                     k_cache, v_cache, n_heads, n_kv_heads, bias)
+    if bias is not None:
+        qkv = qkv + bias
     T = qkv.shape[0]
     D = k_cache.shape[3]
     q = qkv[:, : n_heads * D].reshape(T, n_heads, D)
@@ -190,31 +193,42 @@ def knn_topk(query: torch.Tensor, docs: torch.Tensor, k: int):
     return torch_ref.knn_topk(query, docs, k)
 
 
-def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """Bias-free linear: custom skinny GEMM on the GPU decode path (M<=64),
-    hipBLASLt otherwise.  Dispatch thresholds are measured
-    (profiles/kernel_perf_r01_*.json): hipBLASLt wins at very large N
-    (lm-head shapes), the skinny kernel at mid-size per-layer shapes."""
-    import torch.nn.functional as F
-    if (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= 64
-            and x.shape[1] % 128 == 0 and x.dtype == torch.bfloat16
-            and _hip is not None):
-        w_bytes = weight.shape[0] * weight.shape[1] * 2
-        # measured crossover (tools/sweep_skinny2.py, COLD weights rotated
-        # past the 256 MB LLC — the in-engine regime): the LDS-staged v2
-        # kernel beats hipBLASLt up to ~128 MB of W (o 15.0 vs 21.4 us,
-        # down 34.1 vs 42.2 us at M=64); above that (gate_up 235 MB,
-        # lm-head) blaslt's large-N kernels reach ~5 TB/s and win.
+def _few_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """True for products that the kernel of few rows takes."""
+    return (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= 128 and x.shape[1] % 64 == 0
+            and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
+            and _hip is not None and weight.is_contiguous()
+            and weight.data_ptr() % 16 == 0
+            and not (x.is_contiguous() and x.data_ptr() % 16))
+
+
+def _few_rows_win(x: torch.Tensor, weight: torch.Tensor, raw: bool) -> bool:
+    """True where that kernel beats the library's (us, cold weights): up to 32 rows always
+    (28672 x 4096, 23 rows 50 and 56, 128256 x 2048 101 and 120); up to 64 while the weights
+    are at most 128 MB (16384 x 2048 18 and 19, but 37888 x 3584 66 and 62); above that up to
+    8192 outputs with parts that their reader adds up (3072 x 2048, 96 rows, 8 and 13), or
+    with K long enough to pay for adding them (4096 x 4096 15 and 22, 6144 x 4096 22 and 23,
+    but 2048 x 2048 11 and 9)."""
+    M, K, N = x.shape[0], x.shape[1], weight.shape[0]
+    if M <= 32:
+        return True
+    if M <= 64:
         import os
         max_mb = int(os.environ.get("AURORA_SKINNY_MAX_MB", "128"))
-        if w_bytes <= max_mb * 1024 * 1024:
-            s_target = 256 if w_bytes <= 40 * 1024 * 1024 else 512
-            return _hip.skinny_gemm2_ex(x.contiguous(), weight, s_target)
-    elif (x.is_cuda and x.dim() == 2 and 64 < x.shape[0] <= 256
+        return N * K * 2 <= max_mb * 1024 * 1024
+    return N <= 8192 and (raw or K >= 3072)
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """Bias-free linear: own kernels for up to 256 rows on the GPU where they win,
+    hipBLASLt otherwise."""
+    import torch.nn.functional as F
+    if _few_rows(x, weight) and _few_rows_win(x, weight, False):
+        return _hip.linear_few_rows(x.contiguous(), weight, False)
+    if (x.is_cuda and x.dim() == 2 and 64 < x.shape[0] <= 256
             and x.shape[1] % 64 == 0 and weight.shape[0] % 64 == 0
             and x.dtype == torch.bfloat16 and _hip is not None):
-        # M=65..256 (the B=128-256 decode regime): measured per-shape
-        # dispatch (cold rotated weights) —
+        # measured per-shape dispatch (cold rotated weights) —
         # the glds v3 kernel wins the qkv shape at M>128 (1.36 vs 1.18
         # TB/s) and deep-K at M<=128 (down128 2.18 vs 1.59); hipBLASLt
         # keeps o / gate_up / lm-head. Gated off with AURORA_SKINNY3=0.
@@ -225,6 +239,23 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
                                             and M > 128):
                 return _hip.skinny_gemm3_ex(x.contiguous(), weight, 384)
     return F.linear(x, weight)
+
+
+def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """As ``linear``, but where the product of few rows is cut along K its parts
+    [S, T, N] in float32, for a reader that adds and rounds them itself
+    (``rmsnorm_residual``, ``fused_rope_kv_write``)."""
+    if _few_rows(x, weight) and _few_rows_win(x, weight, True):
+        return _hip.linear_few_rows(x.contiguous(), weight, True)
+    return linear(x, weight)
+
+
+def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up of the products with gate's rows, then up's; in one kernel for few
+    rows."""
+    if _few_rows(x, weight) and weight.shape[0] % 2 == 0:
+        return _hip.silu_few_rows(x.contiguous(), weight)
+    return silu_mul(linear(x, weight))
 
 
 def has_moe_grouped(x: torch.Tensor) -> bool:

@@ -20,8 +20,11 @@ torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w);
 torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
                                   torch::Tensor slots, torch::Tensor cos_sin,
                                   torch::Tensor kc, torch::Tensor vc,
-                                  long Hq, long Hkv);
-torch::Tensor skinny_gemm_ex(torch::Tensor x, torch::Tensor w, long s_target, long unroll);
+                                  long Hq, long Hkv,
+                                  c10::optional<torch::Tensor> bias);
+torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts);
+torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
+torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor skinny_gemm2_ex(torch::Tensor x, torch::Tensor w, long s_target);
 torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target);
 torch::Tensor moe_grouped_gemm(torch::Tensor xp, torch::Tensor w,
@@ -168,8 +171,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "decode-path skinny GEMM (M<=64)");
   m.def("fused_rope_kv_write", &fused_rope_kv_write,
         "fused qkv split + RoPE + paged KV scatter");
-  m.def("skinny_gemm_ex", &skinny_gemm_ex, "skinny GEMM with tuning knobs");
-  m.def("skinny_gemm2_ex", &skinny_gemm2_ex, "LDS-staged skinny GEMM (M<=64)");
+  m.def("few_rows", &few_rows, "products of at most 128 rows, K in parts");
+  m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows");
+  m.def("silu_few_rows", &silu_few_rows, "gate and up of at most 128 rows, silu(gate) * up");
+  m.def("skinny_gemm2_ex", &skinny_gemm2_ex, "products of at most 256 rows");
   m.def("skinny_gemm3_ex", &skinny_gemm3_ex, "glds double-buffered projection GEMM (M<=256)");
   m.def("moe_grouped_gemm", &moe_grouped_gemm,
         "packed per-expert grouped GEMM (skips unrouted experts)");

@@ -5,6 +5,8 @@
 // tensor is read exactly once.  These replace the reference's CPU-side
 // text plumbing with the engine's per-layer hot path (no reference analog;
 // SURVEY.md preamble table row 1).
+#include <type_traits>
+
 #include "common.h"
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
@@ -13,16 +15,39 @@
 
 // ---------------------------------------------------------------- rmsnorm
 
+// Eight results of a product in parts, each rounded to bf16 as the product would be
+DEVINL void add_parts8(float (&y)[8], const float* x, int parts, long step) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) y[j] = 0.f;
+#pragma unroll 4
+  for (int p = 0; p < parts; ++p) {
+    const floatx4 a = *reinterpret_cast<const floatx4*>(x + p * step);
+    const floatx4 b = *reinterpret_cast<const floatx4*>(x + p * step + 4);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      y[j] += a[j];
+      y[4 + j] += b[j];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) y[j] = bf16_to_f32(f32_to_bf16(y[j]));
+}
+
+
 // One workgroup per row; 256 threads; row length H must be a multiple of 8.
 // RESIDUAL: also adds `res` first and writes the sum back to res_out.
-template <bool RESIDUAL>
-__global__ void rmsnorm_kernel(
-    const __hip_bfloat16* __restrict__ x,
+// PARTS: x is the sum, rounded to bf16, of `parts` fp32 terms that lie `step` apart. A
+// product left in parts is so added up where it is read anyway: 96 rows of 4096 in 4 parts
+// 3.5 us, 23 rows of 2048 in 8 parts 3.3; of a whole product 3.4 and 2.6, after a kernel to
+// add its parts that takes 2.4 to 4.7.
+template <bool RESIDUAL, bool PARTS = false>
+__global__ __launch_bounds__(1024) void rmsnorm_kernel(
+    const std::conditional_t<PARTS, float, __hip_bfloat16>* __restrict__ x,
     const __hip_bfloat16* __restrict__ res,
     __hip_bfloat16* __restrict__ out,
     __hip_bfloat16* __restrict__ res_out,
     const __hip_bfloat16* __restrict__ weight,
-    int H, float eps) {
+    int H, float eps, int parts = 1, long step = 0) {
   const int row = blockIdx.x;
   const long base = (long)row * H;
   const int tid = threadIdx.x;
@@ -33,10 +58,14 @@ __global__ void rmsnorm_kernel(
   float ss = 0.f;
   // each thread strides over the row in 8-element vectors
   for (int i = tid * 8; i < H; i += nthr * 8) {
-    shortx8 v = *reinterpret_cast<const shortx8*>(x + base + i);
     float vals[8];
+    if constexpr (PARTS) {
+      add_parts8(vals, x + base + i, parts, step);
+    } else {
+      shortx8 v = *reinterpret_cast<const shortx8*>(x + base + i);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) vals[j] = bf16_to_f32((unsigned short)v[j]);
+      for (int j = 0; j < 8; ++j) vals[j] = bf16_to_f32((unsigned short)v[j]);
+    }
     if (RESIDUAL) {
       shortx8 r = *reinterpret_cast<const shortx8*>(res + base + i);
       shortx8 sum;
@@ -61,7 +90,7 @@ __global__ void rmsnorm_kernel(
   }
   __syncthreads();
   const float inv = s_inv;
-  const __hip_bfloat16* src = RESIDUAL ? res_out : x;
+  const __hip_bfloat16* src = RESIDUAL ? res_out : (const __hip_bfloat16*)x;
   for (int i = tid * 8; i < H; i += nthr * 8) {
     shortx8 v = *reinterpret_cast<const shortx8*>(src + base + i);
     shortx8 w = *reinterpret_cast<const shortx8*>(weight + i);
@@ -133,9 +162,9 @@ static void rmsnorm_launch(const torch::Tensor& x, const void* res, const torch:
                        CUR_STREAM, xp, (const __hip_bfloat16*)res, op,
                        (__hip_bfloat16*)res_out, wp, T, H, (float)eps);
   else
-    hipLaunchKernelGGL(rmsnorm_kernel<RESIDUAL>, dim3(T), dim3(256), 0, CUR_STREAM, xp,
+    hipLaunchKernelGGL((rmsnorm_kernel<RESIDUAL>), dim3(T), dim3(256), 0, CUR_STREAM, xp,
                        (const __hip_bfloat16*)res, op, (__hip_bfloat16*)res_out, wp, H,
-                       (float)eps);
+                       (float)eps, 1, 0L);
   HIP_CHECK_KERNEL();
 }
 
@@ -152,6 +181,23 @@ torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor weight, double eps) {
 
 std::vector<torch::Tensor> rmsnorm_residual(torch::Tensor x, torch::Tensor res,
                                             torch::Tensor weight, double eps) {
+  if (x.dtype() == torch::kFloat32 && x.dim() == 3) {  // a product in parts
+    const long S = x.size(0), T = x.size(1), H = x.size(2);
+    TORCH_CHECK(x.is_cuda() && x.is_contiguous() && res.dtype() == torch::kBFloat16 &&
+                    res.numel() == T * H && weight.numel() == H && H % 8 == 0,
+                "parts [S, T, H] and residual [T, H]");
+    const auto rc = res.contiguous();
+    auto out = torch::empty_like(rc), res_out = torch::empty_like(rc);
+    if (T == 0) return {out, res_out};
+    const int threads = (int)std::min(1024L, (H / 8 + 63) / 64 * 64);
+    hipLaunchKernelGGL((rmsnorm_kernel<true, true>), dim3(T), dim3(threads), 0, CUR_STREAM,
+                       x.data_ptr<float>(), (const __hip_bfloat16*)rc.data_ptr(),
+                       (__hip_bfloat16*)out.data_ptr(), (__hip_bfloat16*)res_out.data_ptr(),
+                       (const __hip_bfloat16*)weight.data_ptr(), (int)H, (float)eps, (int)S,
+                       T * H);
+    HIP_CHECK_KERNEL();
+    return {out, res_out};
+  }
   TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kBFloat16, "bf16 GPU only");
   auto out = torch::empty_like(x);
   auto res_out = torch::empty_like(x);
@@ -343,14 +389,18 @@ void kv_cache_write(torch::Tensor k, torch::Tensor v, torch::Tensor kc,
 // rocprof showed those as ~5 launches + 3 copies per layer of pure launch
 // floor in the decode step (profiles/decode_kernel_stats_r01.csv).
 // qkv: [T, (Hq+2*Hkv)*D] -> writes q_out [T, Hq, D] (roped), kc/vc slots.
-template <bool FP8>
+// PARTS: qkv is a product in `parts` fp32 terms `step` apart, see rmsnorm_kernel: 96
+// rows of 6144 in 2 parts 3.3 us and whole 3.0, 23 of 3072 in 5 parts 2.8 and 2.4.
+// bias: one term more per column or null, added to the rounded product.
+template <bool FP8, bool PARTS>
 __global__ void fused_rope_kv_write_kernel(
-    const __hip_bfloat16* __restrict__ qkv,
+    const std::conditional_t<PARTS, float, unsigned short>* __restrict__ qkv,
+    const unsigned short* __restrict__ bias,
     __hip_bfloat16* __restrict__ q_out,
     void* __restrict__ kc, void* __restrict__ vc,
     const int* __restrict__ positions, const int* __restrict__ slots,
     const float* __restrict__ cos_sin,
-    int T, int Hq, int Hkv, int D, int P) {
+    int T, int Hq, int Hkv, int D, int P, int parts, long step) {
   const int half = D / 2;
   const int HT = Hq + 2 * Hkv;
   const int waves_per_block = blockDim.x / WAVE;
@@ -359,7 +409,8 @@ __global__ void fused_rope_kv_write_kernel(
   if (wave_id >= (long)T * HT) return;
   const int t = wave_id / HT;
   const int h = wave_id % HT;
-  const __hip_bfloat16* src = qkv + ((long)t * HT + h) * D;
+  const auto* src = qkv + ((long)t * HT + h) * D;
+  if (bias) bias += (long)h * D;
   if (h < Hq + Hkv) {
     // roped write (q -> q_out, k -> cache)
     const int pos = positions[t];
@@ -375,8 +426,24 @@ __global__ void fused_rope_kv_write_kernel(
     for (int i = lane; i < half; i += WAVE) {
       const float c = cos_sin[(long)pos * D + i];
       const float s = cos_sin[(long)pos * D + half + i];
-      const float x1 = bf16_to_f32(*(const unsigned short*)(src + i));
-      const float x2 = bf16_to_f32(*(const unsigned short*)(src + half + i));
+      float x1, x2;
+      if constexpr (PARTS) {
+        x1 = x2 = 0.f;
+#pragma unroll 4
+        for (int p = 0; p < parts; ++p) {
+          x1 += src[p * step + i];
+          x2 += src[p * step + half + i];
+        }
+        x1 = bf16_to_f32(f32_to_bf16(x1));
+        x2 = bf16_to_f32(f32_to_bf16(x2));
+      } else {
+        x1 = bf16_to_f32(src[i]);
+        x2 = bf16_to_f32(src[half + i]);
+      }
+      if (bias) {
+        x1 = bf16_to_f32(f32_to_bf16(x1 + bf16_to_f32(bias[i])));
+        x2 = bf16_to_f32(f32_to_bf16(x2 + bf16_to_f32(bias[half + i])));
+      }
       const float r1 = x1 * c - x2 * s;
       const float r2 = x2 * c + x1 * s;
       if (is_q) {
@@ -399,12 +466,26 @@ __global__ void fused_rope_kv_write_kernel(
     const long dst_row =
         ((((long)(slot / P) * Hkv + (h - Hq - Hkv)) * P + slot % P)) * D;
     for (int i = lane * 8; i < D; i += WAVE * 8) {
-      if constexpr (FP8) {
-        *reinterpret_cast<u64b*>((unsigned char*)vc + dst_row + i) =
-            bf16x8_to_fp8x8(*reinterpret_cast<const shortx8*>(src + i));
+      shortx8 v;
+      if constexpr (PARTS) {
+        float y[8];
+        add_parts8(y, src + i, parts, step);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = (short)f32_to_bf16(y[j]);
       } else {
-        *reinterpret_cast<shortx8*>((__hip_bfloat16*)vc + dst_row + i) =
-            *reinterpret_cast<const shortx8*>(src + i);
+        v = *reinterpret_cast<const shortx8*>(src + i);
+      }
+      if (bias) {
+        const shortx8 b = *reinterpret_cast<const shortx8*>(bias + i);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          v[j] = (short)f32_to_bf16(bf16_to_f32((unsigned short)v[j]) +
+                                    bf16_to_f32((unsigned short)b[j]));
+      }
+      if constexpr (FP8) {
+        *reinterpret_cast<u64b*>((unsigned char*)vc + dst_row + i) = bf16x8_to_fp8x8(v);
+      } else {
+        *reinterpret_cast<shortx8*>((__hip_bfloat16*)vc + dst_row + i) = v;
       }
     }
   }
@@ -413,32 +494,38 @@ __global__ void fused_rope_kv_write_kernel(
 torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
                                   torch::Tensor slots, torch::Tensor cos_sin,
                                   torch::Tensor kc, torch::Tensor vc,
-                                  long Hq, long Hkv) {
-  TORCH_CHECK(qkv.is_cuda() && qkv.dtype() == torch::kBFloat16, "bf16 GPU only");
-  const int T = qkv.size(0);
+                                  long Hq, long Hkv, c10::optional<torch::Tensor> bias) {
+  const bool raw = qkv.dtype() == torch::kFloat32 && qkv.dim() == 3;  // a product in parts
+  TORCH_CHECK(qkv.is_cuda() && (raw ? qkv.is_contiguous() : qkv.dtype() == torch::kBFloat16),
+              "bf16 GPU only");
+  const int T = qkv.size(raw ? 1 : 0);
   const int P = kc.size(2), D = kc.size(3);
-  TORCH_CHECK(qkv.size(1) == (Hq + 2 * Hkv) * D, "qkv width mismatch");
-  auto q_out = torch::empty({(long)T, Hq, (long)D}, qkv.options());
+  const long width = (Hq + 2 * Hkv) * D;
+  TORCH_CHECK(qkv.size(-1) == width, "qkv width mismatch");
+  TORCH_CHECK(!bias || (bias->is_cuda() && bias->dtype() == torch::kBFloat16 &&
+                        bias->is_contiguous() && bias->numel() == width),
+              "a contiguous bf16 bias per column");
+  auto q_out = torch::empty({(long)T, Hq, (long)D}, qkv.options().dtype(torch::kBFloat16));
   if (T == 0) return q_out;
   const long waves = (long)T * (Hq + 2 * Hkv);
   const int wpb = 4;
-  const bool fp8 = kc.dtype() == torch::kFloat8_e4m3fn;
-  if (fp8)
-    hipLaunchKernelGGL(fused_rope_kv_write_kernel<true>,
-                       dim3((waves + wpb - 1) / wpb), dim3(wpb * WAVE), 0,
-                       CUR_STREAM, (const __hip_bfloat16*)qkv.data_ptr(),
-                       (__hip_bfloat16*)q_out.data_ptr(), kc.data_ptr(),
-                       vc.data_ptr(), positions.data_ptr<int>(),
-                       slots.data_ptr<int>(), cos_sin.data_ptr<float>(),
-                       T, (int)Hq, (int)Hkv, D, P);
-  else
-    hipLaunchKernelGGL(fused_rope_kv_write_kernel<false>,
-                       dim3((waves + wpb - 1) / wpb), dim3(wpb * WAVE), 0,
-                       CUR_STREAM, (const __hip_bfloat16*)qkv.data_ptr(),
-                       (__hip_bfloat16*)q_out.data_ptr(), kc.data_ptr(),
-                       vc.data_ptr(), positions.data_ptr<int>(),
-                       slots.data_ptr<int>(), cos_sin.data_ptr<float>(),
-                       T, (int)Hq, (int)Hkv, D, P);
+  auto launch = [&](auto kern, auto* src) {
+    hipLaunchKernelGGL(kern, dim3((waves + wpb - 1) / wpb), dim3(wpb * WAVE), 0, CUR_STREAM,
+                       src, bias ? (const unsigned short*)bias->data_ptr() : nullptr,
+                       (__hip_bfloat16*)q_out.data_ptr(), kc.data_ptr(), vc.data_ptr(),
+                       positions.data_ptr<int>(), slots.data_ptr<int>(),
+                       cos_sin.data_ptr<float>(), T, (int)Hq, (int)Hkv, D, P,
+                       raw ? (int)qkv.size(0) : 1, T * width);
+  };
+  const auto* f = (const float*)qkv.data_ptr();
+  const auto* h = (const unsigned short*)qkv.data_ptr();
+  if (kc.dtype() == torch::kFloat8_e4m3fn) {
+    if (raw) launch(fused_rope_kv_write_kernel<true, true>, f);
+    else launch(fused_rope_kv_write_kernel<true, false>, h);
+  } else {
+    if (raw) launch(fused_rope_kv_write_kernel<false, true>, f);
+    else launch(fused_rope_kv_write_kernel<false, false>, h);
+  }
   HIP_CHECK_KERNEL();
   return q_out;
 }

@@ -1,0 +1,232 @@
+// Products of few rows for gfx950: out[M <= 128, N] = x[M, K] @ W[N, K]^T, what a decoding
+// step does with every dense weight, and silu(gate) * up of such products.
+//
+// Bound by reading W once. A workgroup takes 64 rows of W (128 for the wide form) and all
+// rows of x, in steps of 64 of K through a ring of LDS stages that direct-to-LDS loads fill
+// several steps ahead: two workgroups of 72 to 80 KB fit a CU and have 48 to 80 KB of W
+// under way. A wave multiplies 16 rows of W with all of x: a lane ends with four outputs
+// that lie side by side. Reading W straight into fragments instead, with K split over the
+// waves of a workgroup and no LDS, came to the same at one row and lost at 16 and more
+// (x is then read as often as W's tiles of 16 rows: 28672 x 4096, 32 rows, 86 us).
+//
+// Few tiles of W leave the chip idle, so K is cut into parts as well (``parts_of``). Their
+// fp32 sums are added by whatever reads the product next (norm or rotation, 0.1 to 0.7 us)
+// or by a kernel of their own (2.4 to 4.7 us).
+//
+// Cold weights in a graph, with the parts not yet added; before are the kernel of shallow
+// stages that this replaced, its combining kernel included, or the library's from 65 rows:
+//   N x K          rows: 1            23           64           96           128
+//   4096 x 4096    14.4 ->  8.0   14.2 ->  8.9  15.6 -> 10.0  22.2 -> 11.5  24.4 -> 13.6 us
+//   6144 x 4096    15.4 -> 12.3   16.2 -> 13.4  20.1 -> 16.3  23.3 -> 18.7  25.8 -> 21.6
+//   4096 x 14336   28.2 -> 23.0   29.0 -> 24.1  33.5 -> 27.4  52.3 -> 32.1  55.5 -> 38.1
+//   2048 x 2048     8.3 ->  3.8    9.0 ->  4.0  10.4 ->  5.5   8.5 ->  6.4   8.5 ->  7.2
+//   2048 x 8192    15.1 ->  8.6   15.8 ->  9.3  16.7 -> 10.4  25.0 -> 12.2  25.2 -> 14.4
+//   28672 x 4096, with silu (two kernels before)
+//                  66.3 -> 48.5   58.2 -> 48.0  56.8 -> 53.3  60.1 -> 56.1  62.8 -> 59.3
+// (4096 x 14336 is 21 us at the 5.6 TB/s of a large read, 28672 x 4096 42 us). What is left
+// at 64 rows and more is x on its way to every CU.
+#include "flash_tiles.h"
+#include <torch/extension.h>
+#include <c10/hip/HIPStream.h>
+
+#define CUR_STREAM c10::hip::getCurrentHIPStream().stream()
+
+#define FEW_K 64      // K of a stage: eight 16-byte units a row, XOR-swizzled by row
+#define FEW_MOST 128  // rows of x
+
+// This wave's loads but the last L have landed, its reads are done, and so for all waves.
+template <int L>
+DEVINL void await_stage() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(L) : "memory");
+}
+
+// WN rows of W, 16 MT rows of x, NS stages. SILU: W is gate's N rows, then up's; a wave's 16
+// rows are 8 of each. Outputs are bf16, or with ``part`` sums over ``span`` of K.
+template <int WN, int MT, int NS, bool SILU>
+__global__ __launch_bounds__(WN * 4) void few_rows_kernel(
+    const unsigned short* x, const unsigned short* w, unsigned short* out, float* part, int M,
+    int N, int K, int span) {
+  constexpr int NT = WN * 4;
+  constexpr int L = (WN * 8 + MT * 128 + NT - 1) / NT;  // loads of a thread per stage
+  constexpr int STAGE = L * NT * 16;
+  __shared__ __attribute__((aligned(16))) char lds[NS * STAGE];
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int at = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * (SILU ? WN / 2 : WN);
+  const int k0 = blockIdx.y * span, steps = (min(K, k0 + span) - k0) / FEW_K;
+  const unsigned short* src[L];
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    const int r = (tid + l * NT) >> 3, unit = (tid & 7) ^ (r & 7);
+    long row;  // rows past the end are the last again
+    if (l >= WN * 8 / NT) row = min(r - WN, M - 1);
+    else if constexpr (SILU) row = min(n0 + r / 16 * 8 + r % 8, N - 1) + (long)(r % 16 / 8) * N;
+    else row = min(n0 + r, N - 1);
+    src[l] = (l >= WN * 8 / NT ? x : w) + row * K + k0 + unit * 8;
+  }
+  auto issue = [&](int s) {
+    char* stage = lds + s % NS * STAGE;
+#pragma unroll
+    for (int l = 0; l < L; ++l)
+      __builtin_amdgcn_global_load_lds((gptr_t)(src[l] + (long)s * FEW_K),
+                                       (lptr_t)(stage + (l * NT + wave * WAVE) * 16), 16, 0, 0);
+  };
+  floatx4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int s) {
+    const char* stage = lds + s % NS * STAGE;
+    frag_u wf[2], xf[2][MT];  // all read before the first product: one latency a step
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int unit = ((h * 4 + g) ^ (at & 7)) * 16;
+      wf[h].s = *reinterpret_cast<const shortx8*>(stage + (wave * 16 + at) * 128 + unit);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        xf[h][m].s = *reinterpret_cast<const shortx8*>(stage + (WN + m * 16 + at) * 128 + unit);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h].v, xf[h][m].v, acc[m], 0, 0, 0);
+  };
+  for (int s = 0; s < min(steps, NS - 1); ++s) issue(s);
+  int s = 0;
+  for (; s + NS - 1 < steps; ++s) {
+    await_stage<(NS - 2) * L>();
+    issue(s + NS - 1);  // over the stage before this, which all waves have left
+    compute(s);
+  }
+  await_stage<0>();
+  for (; s < steps; ++s) compute(s);
+
+  const int n = n0 + (SILU ? wave * 8 + (g & 1) * 4 : wave * 16 + g * 4);
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    floatx4 y = acc[m];
+    if constexpr (SILU) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float up = __shfl_xor(y[j], 32, WAVE);
+        y[j] = y[j] / (1.f + __expf(-y[j])) * up;
+      }
+      if (g >= 2) continue;
+    }
+    const int row = m * 16 + at;
+    if (row >= M) continue;
+    const bool whole = n + 4 <= N && N % 4 == 0;
+    if (!SILU && part) {
+      float* dst = part + ((long)blockIdx.y * M + row) * N + n;
+      if (whole) *reinterpret_cast<floatx4*>(dst) = y;
+      else
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (n + j < N) dst[j] = y[j];
+    } else {
+      unsigned short* dst = out + (long)row * N + n;
+      if (whole)
+        *reinterpret_cast<u64b*>(dst) =
+            (u64b)cvt2_bf16(y[2], y[3]) << 32 | cvt2_bf16(y[0], y[1]);
+      else
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (n + j < N) dst[j] = f32_to_bf16(y[j]);
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void add_parts_kernel(const float* __restrict__ part,
+                                                        unsigned short* __restrict__ out, int S,
+                                                        long MN) {
+  for (long i = blockIdx.x * 256L + threadIdx.x; i < MN; i += gridDim.x * 256L) {
+    float sum = 0.f;
+    for (int s = 0; s < S; ++s) sum += part[s * MN + i];
+    out[i] = f32_to_bf16(sum);
+  }
+}
+
+// K's parts: a workgroup per CU or a few less, of two stages at least (one CU takes in some
+// 50 GB/s whatever is under way, so more workgroups than CUs only even out badly). 4096 x
+// 14336, 23 rows: 1 part 52 us, 2 35, 4 23, 8 25; 2048 x 8192: 4 11.8, 8 9.3, 16 10.3; 4608
+// x 3584: 2 11.1, 3 (216 workgroups) 9.3, 4 (288) 11.3.
+static long parts_of(long N, long K) {
+  const long tiles = (N + 63) / 64;
+  return std::max(1L, std::min({256 / tiles, K / FEW_K / 2, 16L}));
+}
+
+static void check(const torch::Tensor& x, const torch::Tensor& w) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dtype() == torch::kBFloat16 &&
+                  w.dtype() == torch::kBFloat16 && x.is_contiguous() && w.is_contiguous(),
+              "contiguous bf16 GPU only");
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && x.size(0) <= FEW_MOST &&
+                  x.size(1) % FEW_K == 0,
+              "at most ", FEW_MOST, " rows and K a multiple of ", FEW_K);
+}
+
+template <int WN, int MT, int NS, bool SILU>
+static void launch(const torch::Tensor& x, const torch::Tensor& w, unsigned short* out,
+                   float* part, long N, long S, long span) {
+  constexpr int tile = SILU ? WN / 2 : WN;
+  hipLaunchKernelGGL((few_rows_kernel<WN, MT, NS, SILU>), dim3((N + tile - 1) / tile, S),
+                     dim3(WN * 4), 0, CUR_STREAM, (const unsigned short*)x.data_ptr(),
+                     (const unsigned short*)w.data_ptr(), out, part, (int)x.size(0), (int)N,
+                     (int)x.size(1), (int)span);
+  HIP_CHECK_KERNEL();
+}
+
+// [M, N] in bf16, or with ``raw`` where K is cut [S, M, N] in fp32, S terms to be added.
+torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts) {
+  check(x, w);
+  const long M = x.size(0), K = x.size(1), N = w.size(0);
+  torch::Tensor out, part;
+  if (M == 0 || N == 0 || K == 0) return torch::zeros({M, N}, x.options());
+  const long steps = K / FEW_K;
+  const long per = (steps + std::max(parts, 1L) - 1) / std::max(parts, 1L);
+  const long S = (steps + per - 1) / per, span = per * FEW_K;
+  if (S > 1) part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
+  if (S == 1 || !raw) out = torch::empty({M, N}, x.options());
+  auto* op = S > 1 ? nullptr : (unsigned short*)out.data_ptr();
+  float* pp = S > 1 ? part.data_ptr<float>() : nullptr;
+  if (M <= 32) launch<64, 2, 6, false>(x, w, op, pp, N, S, span);
+  else if (M <= 64) launch<64, 4, 5, false>(x, w, op, pp, N, S, span);
+  else if (M <= 96) launch<64, 6, 4, false>(x, w, op, pp, N, S, span);
+  else launch<64, 8, 3, false>(x, w, op, pp, N, S, span);
+  if (S == 1) return out;
+  if (raw) return part;
+  hipLaunchKernelGGL(add_parts_kernel, dim3(std::min((M * N + 255) / 256, 2048L)), dim3(256), 0,
+                     CUR_STREAM, pp, (unsigned short*)out.data_ptr(), (int)S, M * N);
+  HIP_CHECK_KERNEL();
+  return out;
+}
+
+torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw) {
+  // A kernel to add the parts pays off where a tile's steps take much longer than it: 2048
+  // x 2048, 23 rows, 8.2 us whole, 4.0 and 4.7 in parts; 4096 x 4096 16.7, 8.9 and 2.4; 2048
+  // x 2048, 64 rows, 11.7, 5.5 and 4.2.
+  const bool cut = raw || x.size(1) * (x.size(0) > 32 ? 2 : 1) >= 4096;
+  return few_rows(x, w, raw, cut ? parts_of(w.size(0), x.size(1)) : 1);
+}
+
+// silu(x @ gate^T) * (x @ up^T), rounded once; w: gate's rows, then up's
+torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w) {
+  check(x, w);
+  TORCH_CHECK(w.size(0) % 2 == 0);
+  const long M = x.size(0), K = x.size(1), N = w.size(0) / 2;
+  auto out = torch::empty({M, N}, x.options());
+  if (M == 0 || N == 0) return out;
+  auto* op = (unsigned short*)out.data_ptr();
+  // From 65 rows on x is as much to move as W: tiles of 128 halve it where there are enough
+  // for the chip. 28672 x 4096, 96 rows, 59.9 and 56.1 us; 16384 x 2048 21.8 and 27.6; 28672
+  // x 4096, 64 rows, 53.3 and 53.6.
+  const bool wide = N / 64 >= 192;
+  if (M <= 32) launch<64, 2, 6, true>(x, w, op, nullptr, N, 1, K);
+  else if (M <= 64) launch<64, 4, 5, true>(x, w, op, nullptr, N, 1, K);
+  else if (M <= 96 && wide) launch<128, 6, 5, true>(x, w, op, nullptr, N, 1, K);
+  else if (M <= 96) launch<64, 6, 4, true>(x, w, op, nullptr, N, 1, K);
+  else if (wide) launch<128, 8, 5, true>(x, w, op, nullptr, N, 1, K);
+  else launch<64, 8, 3, true>(x, w, op, nullptr, N, 1, K);
+  return out;
+}

@@ -1,16 +1,5 @@
-// Skinny GEMM for the decode path: out[M<=64, N] = x[M, K] @ W[N, K]^T.
-//
-// Decode serving is bound by streaming the weight matrices once per token
-// step (llama3-8b: 16 GB/step); hipBLASLt's skinny kernels measured only
-// 2.55 TB/s on [16, 6144x4096] (profiles/kernel_perf_r01_v1.json), far off
-// the ~6.3 TB/s the chip streams.  This kernel reads W exactly once at
-// 16 B/lane as direct MFMA B-fragments (v_mfma_f32_16x16x32_bf16: lane
-// holds B[k=(l>>4)*8+j][col=l&15] = 16 contiguous bf16 of one W row), so
-// the matrix pipe is free and the kernel runs at the W-streaming limit.
-// x ([M,K] <= 0.5 MB) stays L1/L2-resident and is re-read as the A
-// fragment.  Split-K keeps >=512 workgroups on the 256-CU / 8-XCD chip;
-// f32 partials combine in a second tiny kernel (deterministic, no
-// atomics).
+// Products of 129 to 256 rows, and of rows packed by expert, for gfx950: out = x @ W^T with
+// W streamed once past all rows (products of fewer rows: few_rows.hip).
 #include "common.h"
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
@@ -23,312 +12,6 @@ union sfrag {
   unsigned int u[4];
   bf16x8 v;
 };
-
-// MT = number of 16-row M tiles (M <= 16*MT); SPLIT: write f32 partials.
-template <int MT, bool SPLIT, int UNR>
-__global__ __launch_bounds__(256) void skinny_gemm_kernel(
-    const __hip_bfloat16* __restrict__ x,  // [M, K]
-    const __hip_bfloat16* __restrict__ w,  // [N, K]
-    __hip_bfloat16* __restrict__ out,      // [M, N] (SPLIT=false)
-    float* __restrict__ part,              // [S, M, N] (SPLIT=true)
-    int M, int N, int K, int KS) {
-  const int lane = threadIdx.x % WAVE;
-  const int wave = threadIdx.x / WAVE;
-  const int n0 = blockIdx.x * 64 + wave * 16;  // this wave's 16 W rows
-  if (n0 >= N) return;
-  const int split = blockIdx.y;
-  const int k_begin = split * KS;
-  const int k_end = min(K, k_begin + KS);
-
-  const int col = lane & 15;          // n offset / m row (A)
-  const int krow = (lane >> 4) * 8;   // k offset of this lane's 8 elements
-
-  const int n = n0 + col;
-  const bool nvalid = n < N;
-  // branchless k-loop: clamp out-of-range rows to a safe address and mask
-  // at the store instead (a runtime guard inside the loop makes hipcc
-  // branch around each load and drain vmcnt per element)
-  const long wbase = (long)min(n, N - 1) * K;
-
-  f32x4 acc[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[t][r] = 0.f;
-
-  long xbase[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-    xbase[t] = (long)min(t * 16 + col, M - 1) * K;  // clamped (masked at store)
-
-  // UNR k-steps per iteration: UNR W loads (+UNR*MT x loads) in flight
-  for (int k = k_begin; k < k_end; k += 32 * UNR) {
-    shortx8 wv[UNR];
-    sfrag bf[UNR], af[UNR][MT];
-#pragma unroll
-    for (int u = 0; u < UNR; ++u)
-      wv[u] = *reinterpret_cast<const shortx8*>(w + wbase + k + u * 32 + krow);
-#pragma unroll
-    for (int u = 0; u < UNR; ++u)
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const shortx8 xv =
-            *reinterpret_cast<const shortx8*>(x + xbase[t] + k + u * 32 + krow);
-        __builtin_memcpy(&af[u][t], &xv, 16);
-      }
-#pragma unroll
-    for (int u = 0; u < UNR; ++u) {
-      __builtin_memcpy(&bf[u], &wv[u], 16);
-#pragma unroll
-      for (int t = 0; t < MT; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[u][t].v, bf[u].v,
-                                                         acc[t], 0, 0, 0);
-    }
-  }
-
-  if (!nvalid) return;
-  // C layout (16x16): lane holds col j = lane&15 (= n), rows (lane>>4)*4+r
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = t * 16 + (lane >> 4) * 4 + r;
-      if (m >= M) continue;
-      if (SPLIT) {
-        part[((long)split * M + m) * N + n] = acc[t][r];
-      } else {
-        *(unsigned short*)(out + (long)m * N + n) = f32_to_bf16(acc[t][r]);
-      }
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
-// v2: LDS-staged variant for M <= 64 (the dispatched decode path).
-// v1's per-lane 16 B fragment
-// loads are row-gathers (consecutive lanes touch lines K*2 bytes apart);
-// at MT=4 that is 5 gathered loads per 32-k step and caps the kernel at
-// ~1.3 TB/s cold (tools/sweep_skinny2.py).  Here a WG cooperatively
-// streams W and x tiles with 64 B-per-thread coalesced loads into
-// XOR-swizzled LDS ([64 rows][128 k] bf16, unit16 ^= row&15 -- conflict-
-// free per 16-lane phase for both the b128 stores and the fragment
-// reads), double-buffered so the global stream overlaps the MFMAs.
-// ---------------------------------------------------------------------------
-#define SG2_BK 128                 // k elements per staged chunk
-#define SG2_TILE_B (64 * SG2_BK * 2)  // one tile: 16 KB
-
-__device__ __forceinline__ int sg2_addr(int row, int unit) {
-  return row * (SG2_BK * 2) + ((unit ^ (row & 15)) << 4);
-}
-
-template <bool SPLIT>
-__global__ __launch_bounds__(256, 2) void skinny_gemm2_kernel(
-    const __hip_bfloat16* __restrict__ x,  // [M, K]
-    const __hip_bfloat16* __restrict__ w,  // [N, K]
-    __hip_bfloat16* __restrict__ out,      // [M, N] (SPLIT=false)
-    float* __restrict__ part,              // [S, M, N] (SPLIT=true)
-    int M, int N, int K, int KS) {
-  __shared__ char lds[2][2 * SG2_TILE_B];  // [buf][W tile | X tile]
-  const int lane = threadIdx.x % WAVE;
-  const int wave = threadIdx.x / WAVE;
-  const int n0 = blockIdx.x * 64;
-  const int split = blockIdx.y;
-  const int k_begin = split * KS;
-  const int k_end = min(K, k_begin + KS);
-  const int nchunks = (k_end - k_begin + SG2_BK - 1) / SG2_BK;
-  if (nchunks <= 0 || n0 >= N) return;
-
-  // cooperative load mapping: thread -> (row = t>>2, 64B segment = t&3)
-  const int lrow = threadIdx.x >> 2;
-  const int lseg = threadIdx.x & 3;
-  const long wrow = (long)min(n0 + lrow, N - 1) * K;  // clamped
-  const long xrow = (long)min(lrow, M - 1) * K;       // clamped
-
-  float4 gw0, gw1, gw2, gw3, gx0, gx1, gx2, gx3;
-#define SG2_GLOAD(c)                                                        \
-  {                                                                         \
-    const long kc = k_begin + (long)(c)*SG2_BK + lseg * 32;                 \
-    gw0 = *reinterpret_cast<const float4*>(w + wrow + kc);                  \
-    gw1 = *reinterpret_cast<const float4*>(w + wrow + kc + 8);              \
-    gw2 = *reinterpret_cast<const float4*>(w + wrow + kc + 16);             \
-    gw3 = *reinterpret_cast<const float4*>(w + wrow + kc + 24);             \
-    gx0 = *reinterpret_cast<const float4*>(x + xrow + kc);                  \
-    gx1 = *reinterpret_cast<const float4*>(x + xrow + kc + 8);              \
-    gx2 = *reinterpret_cast<const float4*>(x + xrow + kc + 16);             \
-    gx3 = *reinterpret_cast<const float4*>(x + xrow + kc + 24);             \
-  }
-#define SG2_STORE(b)                                                        \
-  {                                                                         \
-    char* wt = lds[b];                                                      \
-    char* xt = lds[b] + SG2_TILE_B;                                         \
-    *reinterpret_cast<float4*>(wt + sg2_addr(lrow, lseg * 4 + 0)) = gw0;    \
-    *reinterpret_cast<float4*>(wt + sg2_addr(lrow, lseg * 4 + 1)) = gw1;    \
-    *reinterpret_cast<float4*>(wt + sg2_addr(lrow, lseg * 4 + 2)) = gw2;    \
-    *reinterpret_cast<float4*>(wt + sg2_addr(lrow, lseg * 4 + 3)) = gw3;    \
-    *reinterpret_cast<float4*>(xt + sg2_addr(lrow, lseg * 4 + 0)) = gx0;    \
-    *reinterpret_cast<float4*>(xt + sg2_addr(lrow, lseg * 4 + 1)) = gx1;    \
-    *reinterpret_cast<float4*>(xt + sg2_addr(lrow, lseg * 4 + 2)) = gx2;    \
-    *reinterpret_cast<float4*>(xt + sg2_addr(lrow, lseg * 4 + 3)) = gx3;    \
-  }
-
-  f32x4 acc[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[t][r] = 0.f;
-
-  const int bcol = lane & 15;    // W-tile row / x-tile row offset
-  const int kg = lane >> 4;      // unit offset of this lane's 16 B
-
-  SG2_GLOAD(0);
-  SG2_STORE(0);
-  if (nchunks > 1) SG2_GLOAD(1);
-  __syncthreads();
-
-  for (int c = 0; c < nchunks; ++c) {
-    const int buf = c & 1;
-    if (c + 1 < nchunks) {
-      SG2_STORE(!buf);                    // stage next chunk
-      if (c + 2 < nchunks) SG2_GLOAD(c + 2);  // start chunk after next
-    }
-    const char* wt = lds[buf];
-    const char* xt = lds[buf] + SG2_TILE_B;
-    const int klim = min(SG2_BK, k_end - k_begin - c * SG2_BK);
-#pragma unroll
-    for (int s = 0; s < SG2_BK / 32; ++s) {
-      if (s * 32 >= klim) break;
-      const shortx8 bv = *reinterpret_cast<const shortx8*>(
-          wt + sg2_addr(wave * 16 + bcol, s * 4 + kg));
-      sfrag bfr;
-      __builtin_memcpy(&bfr, &bv, 16);
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const shortx8 av = *reinterpret_cast<const shortx8*>(
-            xt + sg2_addr(t * 16 + bcol, s * 4 + kg));
-        sfrag afr;
-        __builtin_memcpy(&afr, &av, 16);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr.v, bfr.v,
-                                                         acc[t], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-
-  const int n = n0 + wave * 16 + bcol;
-  if (n >= N) return;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = t * 16 + (lane >> 4) * 4 + r;
-      if (m >= M) continue;
-      if (SPLIT) {
-        part[((long)split * M + m) * N + n] = acc[t][r];
-      } else {
-        *(unsigned short*)(out + (long)m * N + n) = f32_to_bf16(acc[t][r]);
-      }
-    }
-  }
-}
-#undef SG2_GLOAD
-#undef SG2_STORE
-
-// ---------------------------------------------------------------------------
-// v2 mid-M variant (65 <= M <= 256, MT = 8 or 16 m-tiles): hipBLASLt's
-// skinny-M kernels measured 1.2-1.8 TB/s cold on the B=256 decode shapes
-// (tools/sweep_skinny2.py).  Only the x tile is LDS-staged (it is L2-hot:
-// every workgroup re-reads the same [M,K] activations, so the staging
-// loads return in ~100 cycles); W streams straight into MFMA B-fragments
-// as 16 B per-lane row-gathers exactly like v1 -- at MT tiles per wave
-// each W fragment feeds MT MFMAs, so the gather instruction rate that
-// capped v1 at MT=4 is amortized 2-4x further.  Single-buffered; cross-
-// chunk latency hides behind the other 2-5 workgroups on the CU.
-// ---------------------------------------------------------------------------
-template <int MT, bool SPLIT>
-__global__ __launch_bounds__(256, 2) void skinny_gemm2m_kernel(
-    const __hip_bfloat16* __restrict__ x,  // [M, K]
-    const __hip_bfloat16* __restrict__ w,  // [N, K]
-    __hip_bfloat16* __restrict__ out,      // [M, N] (SPLIT=false)
-    float* __restrict__ part,              // [S, M, N] (SPLIT=true)
-    int M, int N, int K, int KS) {
-  __shared__ char xt[MT * 16 * SG2_BK * 2];  // x tile, XOR-swizzled
-  const int lane = threadIdx.x % WAVE;
-  const int wave = threadIdx.x / WAVE;
-  const int n0 = blockIdx.x * 64;
-  const int split = blockIdx.y;
-  const int k_begin = split * KS;
-  const int k_end = min(K, k_begin + KS);
-  const int nchunks = (k_end - k_begin + SG2_BK - 1) / SG2_BK;
-  if (nchunks <= 0 || n0 >= N) return;
-
-  // X tile staging: 16/MT threads per row, MT 16B units each
-  constexpr int TPR = 16 / MT;          // threads per X row
-  const int xlrow = threadIdx.x / TPR;
-  const int xuseg = (threadIdx.x % TPR) * MT;  // first unit of this thread
-  const long xrow = (long)min(xlrow, M - 1) * K;
-
-  const int bcol = lane & 15;
-  const int kg = lane >> 4;
-  const int n = n0 + wave * 16 + bcol;
-  const long wbase = (long)min(n, N - 1) * K;  // clamped, masked at store
-
-  f32x4 acc[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) acc[t][r] = 0.f;
-
-  for (int c = 0; c < nchunks; ++c) {
-    const long kc = k_begin + (long)c * SG2_BK;
-    __syncthreads();  // all waves done reading the tile of chunk c-1
-    {
-      const long kcx = kc + xuseg * 8;
-#pragma unroll
-      for (int b = 0; b < MT / 4; ++b) {
-        float4 x0 = *reinterpret_cast<const float4*>(x + xrow + kcx + b * 32);
-        float4 x1 = *reinterpret_cast<const float4*>(x + xrow + kcx + b * 32 + 8);
-        float4 x2 = *reinterpret_cast<const float4*>(x + xrow + kcx + b * 32 + 16);
-        float4 x3 = *reinterpret_cast<const float4*>(x + xrow + kcx + b * 32 + 24);
-        *reinterpret_cast<float4*>(xt + sg2_addr(xlrow, xuseg + b * 4)) = x0;
-        *reinterpret_cast<float4*>(xt + sg2_addr(xlrow, xuseg + b * 4 + 1)) = x1;
-        *reinterpret_cast<float4*>(xt + sg2_addr(xlrow, xuseg + b * 4 + 2)) = x2;
-        *reinterpret_cast<float4*>(xt + sg2_addr(xlrow, xuseg + b * 4 + 3)) = x3;
-      }
-    }
-    __syncthreads();  // tile of chunk c visible
-#pragma unroll
-    for (int s = 0; s < SG2_BK / 32; ++s) {
-      const shortx8 bv =
-          *reinterpret_cast<const shortx8*>(w + wbase + kc + s * 32 + kg * 8);
-      sfrag bfr;
-      __builtin_memcpy(&bfr, &bv, 16);
-#pragma unroll
-      for (int t = 0; t < MT; ++t) {
-        const shortx8 av = *reinterpret_cast<const shortx8*>(
-            xt + sg2_addr(t * 16 + bcol, s * 4 + kg));
-        sfrag afr;
-        __builtin_memcpy(&afr, &av, 16);
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(afr.v, bfr.v,
-                                                         acc[t], 0, 0, 0);
-      }
-    }
-  }
-
-  if (n >= N) return;
-#pragma unroll
-  for (int t = 0; t < MT; ++t) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = t * 16 + (lane >> 4) * 4 + r;
-      if (m >= M) continue;
-      if (SPLIT) {
-        part[((long)split * M + m) * N + n] = acc[t][r];
-      } else {
-        *(unsigned short*)(out + (long)m * N + n) = f32_to_bf16(acc[t][r]);
-      }
-    }
-  }
-}
 
 // ---------------------------------------------------------------------------
 // v3: the M = 128-256 decode-batch projection GEMM (the headline B=256
@@ -617,70 +300,6 @@ __global__ void skinny_combine_kernel(const float* __restrict__ part,
   }
 }
 
-torch::Tensor skinny_gemm_ex(torch::Tensor x, torch::Tensor w, long s_target, long unroll) {
-  TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kBFloat16, "bf16 GPU only");
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1));
-  const int M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(M <= 64, "skinny_gemm is for M <= 64");
-  TORCH_CHECK(K % 64 == 0, "K must be a multiple of 64");
-  auto out = torch::empty({M, N}, x.options());
-  if (M == 0 || N == 0) return out;
-  const int nblocks = (N + 63) / 64;
-  const int target = s_target > 0 ? (int)s_target : 1024;
-  const int kquant = 32 * (int)unroll;
-  int S = std::max(1, std::min(32, target / std::max(nblocks, 1)));
-  int KS = ((K / S + kquant - 1) / kquant) * kquant;
-  S = (K + KS - 1) / KS;  // actual split count after rounding
-  TORCH_CHECK(K % kquant == 0, "K must be a multiple of ", kquant);
-  const int MT = (M + 15) / 16;
-  auto stream = CUR_STREAM;
-  torch::Tensor part;
-  if (S > 1)
-    part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
-  dim3 grid(nblocks, S), block(256);
-#define SG_LAUNCH(MTV, SPLITV)                                               \
-  if (unroll == 4)                                                           \
-    hipLaunchKernelGGL((skinny_gemm_kernel<MTV, SPLITV, 4>), grid, block, 0, \
-                     stream, (const __hip_bfloat16*)x.data_ptr(),            \
-                     (const __hip_bfloat16*)w.data_ptr(),                    \
-                     (__hip_bfloat16*)out.data_ptr(),                        \
-                     SPLITV ? part.data_ptr<float>() : nullptr, M, N, K, KS);\
-  else                                                                       \
-    hipLaunchKernelGGL((skinny_gemm_kernel<MTV, SPLITV, 2>), grid, block, 0, \
-                     stream, (const __hip_bfloat16*)x.data_ptr(),            \
-                     (const __hip_bfloat16*)w.data_ptr(),                    \
-                     (__hip_bfloat16*)out.data_ptr(),                        \
-                     SPLITV ? part.data_ptr<float>() : nullptr, M, N, K, KS)
-  if (S > 1) {
-    switch (MT) {
-      case 1: SG_LAUNCH(1, true); break;
-      case 2: SG_LAUNCH(2, true); break;
-      case 3: SG_LAUNCH(3, true); break;
-      default: SG_LAUNCH(4, true); break;
-    }
-    const long MN = (long)M * N;
-    int cblocks = (int)std::min<long>((MN + 255) / 256, 1024);
-    hipLaunchKernelGGL(skinny_combine_kernel, dim3(cblocks), dim3(256), 0,
-                       stream, part.data_ptr<float>(),
-                       (__hip_bfloat16*)out.data_ptr(), S, MN);
-  } else {
-    switch (MT) {
-      case 1: SG_LAUNCH(1, false); break;
-      case 2: SG_LAUNCH(2, false); break;
-      case 3: SG_LAUNCH(3, false); break;
-      default: SG_LAUNCH(4, false); break;
-    }
-  }
-#undef SG_LAUNCH
-  HIP_CHECK_KERNEL();
-  return out;
-}
-
-
-torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w) {
-  return skinny_gemm_ex(x, w, 0, 2);
-}
-
 torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target) {
   TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kBFloat16, "bf16 GPU only");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1));
@@ -723,54 +342,20 @@ torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target) {
   return out;
 }
 
+// defined in few_rows.hip
+torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts);
+torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
+
+torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w) {
+  TORCH_CHECK(x.dim() == 2 && x.size(0) <= 64, "skinny_gemm is for M <= 64");
+  return linear_few_rows(x, w, false);
+}
+
 torch::Tensor skinny_gemm2_ex(torch::Tensor x, torch::Tensor w, long s_target) {
-  TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kBFloat16, "bf16 GPU only");
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1));
-  const int M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(M <= 256, "skinny_gemm2 is for M <= 256");
-  TORCH_CHECK(K % SG2_BK == 0, "K must be a multiple of ", SG2_BK);
-  auto out = torch::empty({M, N}, x.options());
-  if (M == 0 || N == 0) return out;
-  const int nblocks = (N + 63) / 64;
-  const int target = s_target > 0 ? (int)s_target : 768;
-  int S = std::max(1, std::min(16, target / std::max(nblocks, 1)));
-  int KS = ((K / S + SG2_BK - 1) / SG2_BK) * SG2_BK;
-  S = (K + KS - 1) / KS;
-  auto stream = CUR_STREAM;
-  torch::Tensor part;
-  dim3 grid(nblocks, S), block(256);
-  float* pptr = nullptr;
-  if (S > 1) {
-    part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
-    pptr = part.data_ptr<float>();
-  }
-#define SG2_DISPATCH(SPLITV)                                                 \
-  if (M <= 64)                                                               \
-    hipLaunchKernelGGL((skinny_gemm2_kernel<SPLITV>), grid, block, 0,        \
-                       stream, (const __hip_bfloat16*)x.data_ptr(),          \
-                       (const __hip_bfloat16*)w.data_ptr(),                  \
-                       (__hip_bfloat16*)out.data_ptr(), pptr, M, N, K, KS);  \
-  else if (M <= 128)                                                         \
-    hipLaunchKernelGGL((skinny_gemm2m_kernel<8, SPLITV>), grid, block, 0,    \
-                       stream, (const __hip_bfloat16*)x.data_ptr(),          \
-                       (const __hip_bfloat16*)w.data_ptr(),                  \
-                       (__hip_bfloat16*)out.data_ptr(), pptr, M, N, K, KS);  \
-  else                                                                       \
-    hipLaunchKernelGGL((skinny_gemm2m_kernel<16, SPLITV>), grid, block, 0,   \
-                       stream, (const __hip_bfloat16*)x.data_ptr(),          \
-                       (const __hip_bfloat16*)w.data_ptr(),                  \
-                       (__hip_bfloat16*)out.data_ptr(), pptr, M, N, K, KS)
-  if (S > 1) {
-    SG2_DISPATCH(true);
-    const long MN = (long)M * N;
-    int cblocks = (int)std::min<long>((MN + 255) / 256, 2048);
-    hipLaunchKernelGGL(skinny_combine_kernel, dim3(cblocks), dim3(256), 0,
-                       stream, part.data_ptr<float>(),
-                       (__hip_bfloat16*)out.data_ptr(), S, MN);
-  } else {
-    SG2_DISPATCH(false);
-  }
-#undef SG2_DISPATCH
-  HIP_CHECK_KERNEL();
-  return out;
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(0) <= 256,
+              "skinny_gemm2 is for M <= 256");
+  TORCH_CHECK(x.size(1) % 128 == 0, "K must be a multiple of 128");
+  if (x.size(0) > 128) return skinny_gemm3_ex(x, w, s_target);
+  const long tiles = (w.size(0) + 63) / 64, target = s_target > 0 ? s_target : 768;
+  return few_rows(x, w, false, std::max(1L, std::min(16L, target / std::max(tiles, 1L))));
 }

@@ -45,6 +45,10 @@ class ColumnParallelLinear(nn.Module):
             y = pdist.tp_all_gather(y, dim=-1)
         return y
 
+    def parts(self, x: torch.Tensor) -> torch.Tensor:
+        """This rank's product without its bias, possibly in parts (``ops.linear_parts``)."""
+        return ops.linear_parts(x, self.weight)
+
 
 class RowParallelLinear(nn.Module):
     """Y = all_reduce(X_local @ W_local^T), W_local = W[rank-th input shard]."""
@@ -63,6 +67,10 @@ class RowParallelLinear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         y = ops.linear(x, self.weight)
         return pdist.tp_all_reduce(y)
+
+    def parts(self, x: torch.Tensor) -> torch.Tensor:
+        """As ``forward``, possibly in parts (``ops.linear_parts``) where nothing is reduced."""
+        return self(x) if pdist.tp_world_size() > 1 else ops.linear_parts(x, self.weight)
 
 
 class QKVParallelLinear(ColumnParallelLinear):

@@ -16,7 +16,7 @@ CSRC = "aurora_amd/ops/csrc/"
 EXTENSIONS = {
     # decoder kernels
     "_hip_ops": ["bindings.cpp", "elementwise.hip", "attention_decode.hip",
-                 "attention_prefill.hip", "skinny_gemm.hip", "residual_norm.hip",
+                 "attention_prefill.hip", "skinny_gemm.hip", "few_rows.hip", "residual_norm.hip",
                  "attention_rows.hip", "recurrence.hip", "moe.hip", "sublayer.hip",
                  "latent_attention.hip", "output_norm.hip", "conv_heads.hip"],
     # sentence encoder, vector search, one-shot all-reduce
