@@ -338,17 +338,3 @@ torch::Tensor embed_pool(torch::Tensor hidden, torch::Tensor cu) {
   HIP_CHECK_KERNEL();
   return out;
 }
-
-// ---- brute-force kNN over the HBM-resident doc matrix --------------------
-// Scores via hipBLASLt GEMM (a plain library GEMM) + torch topk; the win on
-// MI355X is that the whole corpus lives in 288 GB HBM.  A fused
-// score+select kernel is a later optimisation (profiles will say if the
-// [Q, N] score materialisation ever matters).
-
-std::vector<torch::Tensor> knn_topk(torch::Tensor query, torch::Tensor docs, long k) {
-  TORCH_CHECK(query.is_cuda(), "GPU only");
-  auto scores = torch::mm(query.to(docs.dtype()), docs.t()).to(torch::kFloat32);
-  k = std::min<long>(k, docs.size(0));
-  auto [vals, idx] = scores.topk(k, -1);
-  return {vals, idx};
-}

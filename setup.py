@@ -20,7 +20,7 @@ EXTENSIONS = {
                  "attention_rows.hip", "recurrence.hip", "moe.hip", "sublayer.hip",
                  "latent_attention.hip", "output_norm.hip", "conv_heads.hip"],
     # sentence encoder, vector search, one-shot all-reduce
-    "_hip_aux": ["bindings_aux.cpp", "encoder.hip", "allreduce.hip"],
+    "_hip_aux": ["bindings_aux.cpp", "encoder.hip", "knn.hip", "allreduce.hip"],
 }
 wanted = os.environ.get("AURORA_EXTENSIONS", "").split(",")
 names = [n for n in EXTENSIONS if n in wanted] or list(EXTENSIONS)
