@@ -16,6 +16,7 @@
 // row tile) in a device table; blocks past its end leave at once, so experts
 // nobody chose cost no weight traffic.
 #include "elem.h"
+#include "flash_tiles.h"
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
@@ -288,6 +289,13 @@ DEVINL float clamped_glu(float g, float u, const GroupArgs& p) {
   return g * (u + p.shift) / (1.f + expf(-p.alpha * g));
 }
 
+// The same to a few units in the last place of fp32, for results in bf16
+DEVINL float clamped_glu_fast(float g, float u, const GroupArgs& p) {
+  g = fminf(g, p.limit);
+  u = fminf(fmaxf(u, -p.limit), p.limit);
+  return g * (u + p.shift) * __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-p.alpha * LOG2E * g));
+}
+
 // Any size and float32: 32 rows x 64 columns, 16 of K at a time, through LDS as
 // fp32 (GLU: 32 gate and the matching 32 up columns).
 template <typename T, int ACT>
@@ -468,6 +476,180 @@ __global__ __launch_bounds__(NTHR) void grouped_bf16_kernel(GroupArgs p) {
     }
 }
 
+// The same for well filled experts: 256 rows x 256 weight rows, eight waves of 128 x 64, two
+// stages of 64 of K. While the products of 32 of K run, the fragments of the next 32 are
+// read between them; a stage is requested as soon as all have read its predecessor but one,
+// a stage's products ahead, and costs one barrier. Rows of a stage are whole cache lines
+// (half lines halve what the L2 delivers, 72 and 136 GB/s a CU). A fifth slot of the ring
+// lets w, which comes from further away than x, be asked for two stages ahead; requests go
+// out between the first products of a half, where they cost the least.
+// Two products of 8 experts of 4096 x 14336 for 8000 tokens, two experts each: 5.66 ms (996
+// TFLOP/s, one stage ahead and no reads or requests between products) and now 4.48 ms
+// (1260); 64 of 2048 x 1408, 16000 tokens, 1.98 and 1.61 ms. Matrix cores are busy two
+// thirds of the time at the 1.85 GHz this load leaves; the rest is waiting for the slowest
+// of a stage's lines.
+template <int ACT>
+__global__ __launch_bounds__(512) void grouped_large_kernel(GroupArgs p, int tiles, int cols) {
+  constexpr bool GLU = ACT == GLU_ACT;
+  constexpr int BN = GLU ? 128 : 256, SLOT = 256 * GK * 2, RING = 5 * SLOT, L = 4;
+  // Bands of eight row tiles, down and then across; an XCD takes a contiguous eighth of
+  // each, so that its blocks share rows and columns in its L2.
+  const int band = blockIdx.x / 8 / cols, at = blockIdx.x % 8 * cols + blockIdx.x / 8 % cols;
+  const int rt = band * 8 + at % 8, ct = at / 8;
+  if (rt >= tiles) return;
+  const int* tb = p.table + rt * 3;
+  const int e = tb[0];
+  if (e < 0) return;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int row0 = tb[1], cnt = tb[2], n0 = ct * BN, K = p.K;
+  const int tid = threadIdx.x, lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  const int i = lane & 15, g = lane >> 4;
+  const bf16_t* w = (const bf16_t*)p.w + (long)e * (GLU ? 2 : 1) * p.N * K;
+
+  // source of each 16-byte unit this thread fills: rows of x, then of w
+  const bf16_t *xs[L], *ws[L];
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    const int r = (tid + l * 512) >> 3, unit = (tid & 7) ^ (r & 7);
+    const int row = row0 + min(r, cnt - 1);
+    xs[l] = (const bf16_t*)p.x + (long)(p.gather ? p.gather[row] : row) * K + unit * 8;
+    long wr;
+    if constexpr (GLU)  // of a wave's 64 columns half are gate's, half up's
+      wr = min(n0 + r / 64 * 32 + r % 32, p.N - 1) + (long)(r % 64 / 32) * p.N;
+    else
+      wr = min(n0 + r, p.N - 1);
+    ws[l] = w + wr * K + unit * 8;
+  }
+  // the ring's slots take w's and x's blocks of 64 of K in turn
+  int to = 0;
+  auto request = [&](const bf16_t* const (&from)[L], int stage, int l) {
+    __builtin_amdgcn_global_load_lds((gptr_t)(from[l] + (long)stage * GK),
+                                     (lptr_t)(lds + to + (l * 512 + wave * WAVE) * 16), 16, 0, 0);
+  };
+  auto advance = [&] { to = to == RING - SLOT ? 0 : to + SLOT; };
+  const int wm = wave / 4 * 128, wn = wave % 4 * 64;
+  const int unit = (g ^ (i & 7)) * 16;  // of the first 32 of K; of the second ^ 64
+  const int xa = (wm + i) * 128, wb = (wn + i) * 128;
+  frag_u a[2][8], b[2][4];
+  floatx4 acc[8][4];
+#pragma unroll
+  for (int m = 0; m < 8; ++m)
+#pragma unroll
+    for (int n = 0; n < 4; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+  auto read = [&](int at, auto HALF, int x) {  // of w's block at ``at`` and x's behind it
+    constexpr int h = decltype(HALF)::value;
+    const char* st = lds + (unit ^ h * 64);
+    const int behind = at == RING - SLOT ? 0 : at + SLOT;
+    if (x < 4) b[h][x].s = *reinterpret_cast<const shortx8*>(st + at + wb + x * 2048);
+    else a[h][x - 4].s = *reinterpret_cast<const shortx8*>(st + behind + xa + (x - 4) * 2048);
+  };
+  auto multiply = [&](auto HALF) {
+    constexpr int h = decltype(HALF)::value;
+#pragma unroll
+    for (int m = 0; m < 8; ++m)
+#pragma unroll
+      for (int n = 0; n < 4; ++n)
+        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[h][n].v, a[h][m].v, acc[m][n],
+                                                            0, 0, 0);
+  };
+  // The products of a half; between them the next half's fragments and, with ``from``, a
+  // block's requests, in this order.
+  auto half = [&](auto HALF, int at, const bf16_t* const (*from)[L], int stage) {
+    constexpr int h = decltype(HALF)::value;
+    if (from)
+#pragma unroll
+      for (int l = 0; l < L; ++l) request(*from, stage, l);
+#pragma unroll
+    for (int x = 0; x < 12; ++x) read(at, std::integral_constant<int, 1 - h>{}, x);
+    if (from) advance();
+    multiply(HALF);
+    if (from)
+#pragma unroll
+      for (int l = 0; l < L; ++l) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // products
+        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);  // a request
+      }
+#pragma unroll
+    for (int x = 0; x < 12; ++x) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a read
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  using FIRST = std::integral_constant<int, 0>;
+  using SECOND = std::integral_constant<int, 1>;
+  const int steps = K / GK;
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+    if (x / 2 < steps) {
+#pragma unroll
+      for (int l = 0; l < L; ++l) request(x % 2 ? xs : ws, x / 2, l);
+      advance();
+    }
+  if (steps > 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * L) : "memory");
+  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+  int at_w = 0;  // slot of w's block of this stage
+  auto next = [&] { at_w = at_w >= 3 * SLOT ? at_w - 3 * SLOT : at_w + 2 * SLOT; };
+#pragma unroll
+  for (int x = 0; x < 12; ++x) read(0, FIRST{}, x);
+  __builtin_amdgcn_sched_barrier(0);
+  int s = 0;
+  for (; s + 2 < steps; ++s) {
+    half(FIRST{}, at_w, &ws, s + 2);
+    // the next stage has landed and all have read this one
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(L) : "memory");
+    next();
+    half(SECOND{}, at_w, &xs, s + 2);
+  }
+  for (; s < steps; ++s) {
+    half(FIRST{}, at_w, nullptr, 0);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    next();
+    half(SECOND{}, at_w, nullptr, 0);  // reads past the end what lies there, for nothing
+  }
+
+  // a lane has four outputs of a row side by side
+  bf16_t* y = (bf16_t*)p.y;
+  constexpr int NO = GLU ? 2 : 4;
+#pragma unroll
+  for (int m = 0; m < 8; ++m) {
+    const int row = wm + m * 16 + i;
+    if (row >= cnt) continue;
+#pragma unroll
+    for (int n = 0; n < NO; ++n) {
+      const int c = n0 + (GLU ? wn / 2 : wn) + n * 16 + 4 * g;
+      float v[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        v[r] = GLU ? clamped_glu_fast(acc[m][n][r], acc[m][n + (GLU ? NO : 0)][r], p)
+                   : acc[m][n][r];
+        if constexpr (ACT == RELU2_ACT) v[r] = v[r] > 0.f ? v[r] * v[r] : 0.f;
+      }
+      bf16_t* dst = y + (long)(row0 + row) * p.N + c;
+      if (c + 4 <= p.N && p.N % 4 == 0)
+        *reinterpret_cast<u64b*>(dst) =
+            (u64b)cvt2_bf16(v[2], v[3]) << 32 | cvt2_bf16(v[0], v[1]);
+      else
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (c + r < p.N) dst[r] = f32_to_bf16(v[r]);
+    }
+  }
+}
+
+template <int ACT>
+static void grouped_large(const GroupArgs& p, int tiles) {
+  constexpr int BN = ACT == GLU_ACT ? 128 : 256, lds = 5 * 256 * GK * 2;
+  auto kern = grouped_large_kernel<ACT>;
+  static const hipError_t once = hipFuncSetAttribute(
+      (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+  (void)once;
+  const int cols = (p.N + BN - 1) / BN;
+  hipLaunchKernelGGL(kern, dim3(8 * cols * ((tiles + 7) / 8)), dim3(512), lds,
+                     CUR_STREAM, p, tiles, cols);
+}
+
 template <int TM, int TB, int NS, int NTHR, int ACT>
 static void grouped_bf16(const GroupArgs& p, int tiles) {
   constexpr int BN = ACT == GLU_ACT ? TB / 2 : TB;
@@ -486,7 +668,7 @@ static void grouped(const GroupArgs& p, bool bf16, int tiles, int TM, long busy)
   constexpr bool GLU = ACT == GLU_ACT;
   if (bf16 && p.K % GK == 0) {
     const long blocks = (p.N + (GLU ? 63 : 127)) / (GLU ? 64 : 128) * busy;
-    if (TM == 256) grouped_bf16<256, 256, 2, 512, ACT>(p, tiles);
+    if (TM == 256) grouped_large<ACT>(p, tiles);
     else if (TM == 128) grouped_bf16<128, 128, 2, 256, ACT>(p, tiles);
     else if (TM == 64) grouped_bf16<64, 128, 3, 256, ACT>(p, tiles);
     // few rows: the weights' stream counts. Two workgroups per CU with four
@@ -518,12 +700,19 @@ static std::vector<torch::Tensor> experts(const torch::Tensor& h, const torch::T
   auto y = torch::empty({A, W}, h.options()), place = torch::empty({T_, top}, i32);
   if (A == 0) return {y, place};
   const bool bf16 = h.dtype() == torch::kBFloat16;
-  // row tile: enough rows per weight read when experts are well filled
+  // Row tile: enough rows per weight read. 256 from 80 rows an expert on, where there are
+  // blocks for a good part of the chip: the kernel of that tile is the fastest by so much
+  // that even rows of padding pay. 256 and the next best: 8 experts of 4096 x 14336, two
+  // each, 300 tokens (75 rows) 744 and 746 us, 500 767 and 927, 3000 1959 and 2675; 64 of
+  // 2048 x 1408, six each, 1000 tokens 284 and 329, 8000 946 and 1249; 16 of 1024 x 512,
+  // two each, 2000 tokens (64 blocks) 51 and 46, 4000 (125) 58 and 71.
   const bool matrix = bf16 && W % GK == 0 && F % GK == 0;
-  // and the large tile only where it leaves enough blocks for the chip
   const long cols = ACT == GLU_ACT ? 128 : 256;
-  const bool large = A >= 512 * E && A / 256 * ((F + cols - 1) / cols) >= 1024;
-  const int TM = !matrix || A < 48 * E ? 32 : A < 160 * E ? 64 : large ? 256 : 128;
+  const long blocks = std::max(std::min(E, A), A / 256) *
+                      std::min((F + cols - 1) / cols, (W + 255) / 256);
+  const int TM = !matrix || A < 48 * E          ? 32
+                 : A >= 80 * E && blocks >= 96  ? 256
+                 : A < 160 * E                  ? 64 : 128;
   const int tiles = (int)(A / TM + std::min(E, A));
   auto token = torch::empty({A}, i32), table = torch::empty({tiles, 3}, i32);
   auto act = torch::empty({A, F}, h.options());

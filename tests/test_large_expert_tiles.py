@@ -1,0 +1,49 @@
+"""The grouped product of 256-row tiles: stages, ragged tiles of rows and columns."""
+import pytest
+import torch
+
+from aurora_amd.ops.sequence import _hip
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows_of(E, top, least):
+    """Rows of experts at the edges of a tile, the rest evenly, ``least`` each on average."""
+    edges = [0, 1, 255, 256, 257, 600, 16, 0]
+    left = least * E - sum(edges)
+    rows = edges + [left // (E - len(edges))] * (E - len(edges))
+    rows[-1] += -sum(rows) % top
+    return rows
+
+
+#: width, ff, experts: 1, 2 and 3, 5 and 7, 16 and 9 stages; columns of a tile and less
+@pytest.mark.parametrize("W,F,E,top", [(64, 64, 128, 1), (128, 192, 100, 2), (320, 448, 48, 1),
+                                       (1024, 576, 24, 3)])
+@pytest.mark.parametrize("kind", ["glu", "relu2"])
+def test_tiles(W, F, E, top, kind):
+    g = torch.Generator(device="cuda").manual_seed(W)
+    rows = torch.tensor(_rows_of(E, top, 84), device="cuda")
+    sel = torch.repeat_interleave(torch.arange(E, device="cuda"), rows)
+    sel = sel[torch.randperm(len(sel), generator=g, device="cuda")].int().view(-1, top).contiguous()
+    T = len(sel)
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    h, dn = n(T, W).bfloat16(), (n(E, W, F) * F ** -0.5).bfloat16()
+    up = (n(E, (2 if kind == "glu" else 1) * F, W) * W ** -0.5).bfloat16()
+    if kind == "glu":
+        y, place = _hip("moe_clamped_glu").moe_clamped_glu(h, sel, up, dn, 0.9, 1.702, 1.0)
+    else:
+        y, place = _hip("moe_relu2").moe_relu2(h, sel, up, dn)
+    assert sorted(place.flatten().tolist()) == list(range(T * top))
+    for e in range(E):
+        t, k = (sel == e).nonzero(as_tuple=True)
+        z = h[t].double() @ up[e].double().t()
+        if kind == "glu":
+            a, b = z[:, :F].clamp(max=0.9), z[:, F:].clamp(-0.9, 0.9)
+            z = a * torch.sigmoid(1.702 * a) * (b + 1)
+        else:
+            z = z.clamp(min=0) ** 2
+        want = z @ dn[e].double().t()
+        # activations and then results are rounded, each by up to 2^-8 of itself
+        err = (y[place[t, k].long()].double() - want).norm(dim=-1)
+        through = torch.linalg.matrix_norm(dn[e].double(), 2) * z.norm(dim=-1)
+        assert (err <= 2 ** -8 * (want.norm(dim=-1) + through) + 1e-9).all()
