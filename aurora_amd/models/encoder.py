@@ -50,7 +50,7 @@ class EncoderLayer(nn.Module):
         ops.rope_apply_(q, k, positions, cos_sin)
         o = ops.attention_prefill(q, k, v, cu, self.scale, causal=False)
         h, x = ops.rmsnorm_residual(self.o(o.reshape(T, -1)), x, self.norm2, self.eps)
-        return x, self.down(ops.silu_mul(self.gate_up(h)))
+        return x, self.down(ops.linear_silu_mul(h, self.gate_up.weight))
 
 
 class SentenceEncoder(nn.Module):

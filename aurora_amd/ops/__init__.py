@@ -193,13 +193,38 @@ def knn_topk(query: torch.Tensor, docs: torch.Tensor, k: int):
     return torch_ref.knn_topk(query, docs, k)
 
 
-def _few_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """True for products that the kernel of few rows takes."""
-    return (x.is_cuda and x.dim() == 2 and 0 < x.shape[0] <= 128 and x.shape[1] % 64 == 0
+def _own_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """True for products that the own kernels can take."""
+    return (x.is_cuda and x.dim() == 2 and x.shape[0] > 0 and x.shape[1] > 0
+            and x.shape[1] % 64 == 0 and x.shape[1] == weight.shape[1]
             and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
             and _hip is not None and weight.is_contiguous()
             and weight.data_ptr() % 16 == 0
             and not (x.is_contiguous() and x.data_ptr() % 16))
+
+
+def _few_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    return x.dim() == 2 and x.shape[0] <= 128 and _own_product(x, weight)
+
+
+def _many_rows_win(x: torch.Tensor, weight: torch.Tensor, silu: bool) -> bool:
+    """True for more than 128 rows where the kernel of 256-row tiles beats the library's
+    product (with ``silu``, product and activation), us. With silu: any number of tiles up to
+    1024 of K (6144 x 768, 300 rows 22 and 25, 27000 rows 250 and 349), else those that fill
+    the chip's rounds (16384 x 2048, 600 rows 45 and 48, 6172 rows 330 and 411; 28672 x 4096,
+    2048 rows 371 and 376, 6172 rows 1132 and 1224; not full: 1600 rows 346 and 341, 12288 x
+    4096, 3000 rows 255 and 248). Without: only where the tiles nearly fill the chip twice
+    and K is long, where the library falls to 0.75 to 1.2 PFLOP/s (4096 x 14336, 6172 rows
+    594 and 807, 7000 rows 630 and 696; 3584 x 18944, 7500 rows 798 and 1184; outside: 6144
+    rows of 4096 x 14336 586 and 565, 8000 rows 677 and 629)."""
+    T, K, N = x.shape[0], x.shape[1], weight.shape[0]
+    tiles = -(-T // 256) * -(-N // 256)
+    if not silu:
+        return K >= 14336 and 384 < tiles < 512
+    if K <= 1024:
+        return T >= 256 and tiles >= 48
+    full = tiles / (-(-tiles // 256) * 256)
+    return tiles >= 192 and full >= (0.75 if K <= 2048 else 0.78)
 
 
 def _few_rows_win(x: torch.Tensor, weight: torch.Tensor, raw: bool) -> bool:
@@ -220,11 +245,13 @@ def _few_rows_win(x: torch.Tensor, weight: torch.Tensor, raw: bool) -> bool:
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """Bias-free linear: own kernels for up to 256 rows on the GPU where they win,
-    hipBLASLt otherwise."""
+    """Bias-free linear: own kernels on the GPU where they win, hipBLASLt otherwise."""
     import torch.nn.functional as F
     if _few_rows(x, weight) and _few_rows_win(x, weight, False):
         return _hip.linear_few_rows(x.contiguous(), weight, False)
+    if (x.dim() == 2 and x.shape[0] > 128 and _own_product(x, weight)
+            and _many_rows_win(x, weight, False)):
+        return _hip.many_rows(x.contiguous(), weight, False)
     if (x.is_cuda and x.dim() == 2 and 64 < x.shape[0] <= 256
             and x.shape[1] % 64 == 0 and weight.shape[0] % 64 == 0
             and x.dtype == torch.bfloat16 and _hip is not None):
@@ -251,10 +278,13 @@ def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 
 
 def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """silu(gate) * up of the products with gate's rows, then up's; in one kernel for few
-    rows."""
-    if _few_rows(x, weight) and weight.shape[0] % 2 == 0:
-        return _hip.silu_few_rows(x.contiguous(), weight)
+    """silu(gate) * up of the products with gate's rows, then up's; in one kernel where that
+    is faster."""
+    if weight.shape[0] % 16 == 0 and _own_product(x, weight):
+        if x.shape[0] <= 128:
+            return _hip.silu_few_rows(x.contiguous(), weight)
+        if _many_rows_win(x, weight, True):
+            return _hip.many_rows(x.contiguous(), weight, True)
     return silu_mul(linear(x, weight))
 
 

@@ -22,6 +22,7 @@ torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
                                   torch::Tensor kc, torch::Tensor vc,
                                   long Hq, long Hkv,
                                   c10::optional<torch::Tensor> bias);
+torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
 torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts);
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
@@ -171,6 +172,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "decode-path skinny GEMM (M<=64)");
   m.def("fused_rope_kv_write", &fused_rope_kv_write,
         "fused qkv split + RoPE + paged KV scatter");
+  m.def("many_rows", &many_rows, "products of many rows, with silu(gate) * up");
   m.def("few_rows", &few_rows, "products of at most 128 rows, K in parts");
   m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows");
   m.def("silu_few_rows", &silu_few_rows, "gate and up of at most 128 rows, silu(gate) * up");

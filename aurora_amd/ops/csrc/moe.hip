@@ -278,9 +278,10 @@ struct GroupArgs {
   const int* gather;   // null: x itself is sorted
   const void* w;       // [E, N, K]; GLU: [E, 2N, K], gate rows then up rows
   void* y;             // [A, N]
-  const int* table;
+  const int* table;    // null: one expert for all ``rows``
   int N, K;
   float limit, alpha, shift;
+  int rows = 0;
 };
 
 DEVINL float clamped_glu(float g, float u, const GroupArgs& p) {
@@ -497,11 +498,15 @@ __global__ __launch_bounds__(512) void grouped_large_kernel(GroupArgs p, int til
   const int band = blockIdx.x / 8 / cols, at = blockIdx.x % 8 * cols + blockIdx.x / 8 % cols;
   const int rt = band * 8 + at % 8, ct = at / 8;
   if (rt >= tiles) return;
-  const int* tb = p.table + rt * 3;
-  const int e = tb[0];
-  if (e < 0) return;
+  int e = 0, row0 = rt * 256, cnt = min(256, p.rows - row0);
+  if (p.table) {
+    e = p.table[rt * 3];
+    row0 = p.table[rt * 3 + 1];
+    cnt = p.table[rt * 3 + 2];
+    if (e < 0) return;
+  }
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int row0 = tb[1], cnt = tb[2], n0 = ct * BN, K = p.K;
+  const int n0 = ct * BN, K = p.K;
   const int tid = threadIdx.x, lane = tid % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int i = lane & 15, g = lane >> 4;
@@ -738,6 +743,25 @@ std::vector<torch::Tensor> moe_clamped_glu(torch::Tensor h, torch::Tensor sel,
                                            torch::Tensor w_gu, torch::Tensor w_dn,
                                            double limit, double alpha, double shift) {
   return experts<GLU_ACT>(h, sel, w_gu, w_dn, limit, alpha, shift);
+}
+
+// x [T, K] @ w^T, with ``silu`` silu(gate) * up of the products with w's halves
+torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu) {
+  TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dtype() == torch::kBFloat16 &&
+                  w.dtype() == torch::kBFloat16 && x.is_contiguous() && w.is_contiguous() &&
+                  x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) &&
+                  x.size(1) % GK == 0 && x.size(1) > 0 && (!silu || w.size(0) % 2 == 0),
+              "contiguous bf16 on the GPU, K a multiple of ", GK);
+  const long T_ = x.size(0), N = w.size(0) / (silu ? 2 : 1);
+  auto y = torch::empty({T_, N}, x.options());
+  if (T_ == 0 || N == 0) return y;
+  GroupArgs p = {x.data_ptr(), nullptr, w.data_ptr(), y.data_ptr(), nullptr, (int)N,
+                 (int)x.size(1), INFINITY, 1.f, 0.f, (int)T_};
+  const int tiles = (int)((T_ + 255) / 256);
+  if (silu) grouped_large<GLU_ACT>(p, tiles);
+  else grouped_large<NO_ACT>(p, tiles);
+  HIP_CHECK_KERNEL();
+  return y;
 }
 
 std::vector<torch::Tensor> moe_relu2(torch::Tensor h, torch::Tensor sel, torch::Tensor w_up,

@@ -47,7 +47,10 @@ def test_silu(m, n, k):
     x, w = _inputs(m, 2 * n, k)
     y = x.double() @ w.double().t()
     want = torch.nn.functional.silu(y[:, :n]) * y[:, n:]
-    _check(ops.linear_silu_mul(x, w), want, k)
+    from aurora_amd import _hip_ops
+    _check(_hip_ops.silu_few_rows(x, w), want, k)
+    if n % 8 == 0:  # as silu_mul by itself
+        _check(ops.linear_silu_mul(x, w), want, k)
 
 
 @pytest.mark.parametrize("m", [1, 33, 128])

@@ -47,3 +47,19 @@ def test_tiles(W, F, E, top, kind):
         err = (y[place[t, k].long()].double() - want).norm(dim=-1)
         through = torch.linalg.matrix_norm(dn[e].double(), 2) * z.norm(dim=-1)
         assert (err <= 2 ** -8 * (want.norm(dim=-1) + through) + 1e-9).all()
+
+
+@pytest.mark.parametrize("T", [1, 129, 255, 256, 257, 2100])
+@pytest.mark.parametrize("N,K", [(16, 64), (200, 128), (258, 192), (1000, 448), (2080, 1024)])
+@pytest.mark.parametrize("silu", [False, True])
+def test_dense(T, N, K, silu):
+    """The same tiles without experts; 2100 rows of 2080 columns make a second band."""
+    g = torch.Generator(device="cuda").manual_seed(T + N)
+    x = torch.randn(T, K, generator=g, device="cuda").bfloat16()
+    w = (torch.randn(N * (1 + silu), K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    got = _hip("many_rows").many_rows(x, w, silu).double()
+    want = x.double() @ w.double().t()
+    if silu:
+        want = torch.nn.functional.silu(want[:, :N]) * want[:, N:]
+    # rounded by up to 2^-8 of itself; fp32 sums of K terms stay below 2^-16 of the largest
+    assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2 ** -16 * want.abs().max()).all()
