@@ -392,8 +392,11 @@ void kv_cache_write(torch::Tensor k, torch::Tensor v, torch::Tensor kc,
 // PARTS: qkv is a product in `parts` fp32 terms `step` apart, see rmsnorm_kernel: 96
 // rows of 6144 in 2 parts 3.3 us and whole 3.0, 23 of 3072 in 5 parts 2.8 and 2.4.
 // bias: one term more per column or null, added to the rounded product.
-template <bool FP8, bool PARTS>
-__global__ void fused_rope_kv_write_kernel(
+// A thread per VEC columns of a head and their partners half a head on (16-byte accesses
+// at 8): bound by memory. 6172 rows of 48 heads of 128 took 58 us in 2-byte accesses,
+// now 26; 3000 rows of 48 heads of 64 27 and 8.5.
+template <bool FP8, bool PARTS, int VEC>
+__global__ __launch_bounds__(256) void fused_rope_kv_write_kernel(
     const std::conditional_t<PARTS, float, unsigned short>* __restrict__ qkv,
     const unsigned short* __restrict__ bias,
     __hip_bfloat16* __restrict__ q_out,
@@ -401,92 +404,71 @@ __global__ void fused_rope_kv_write_kernel(
     const int* __restrict__ positions, const int* __restrict__ slots,
     const float* __restrict__ cos_sin,
     int T, int Hq, int Hkv, int D, int P, int parts, long step) {
-  const int half = D / 2;
-  const int HT = Hq + 2 * Hkv;
-  const int waves_per_block = blockDim.x / WAVE;
-  const long wave_id = (long)blockIdx.x * waves_per_block + threadIdx.x / WAVE;
-  const int lane = threadIdx.x % WAVE;
-  if (wave_id >= (long)T * HT) return;
-  const int t = wave_id / HT;
-  const int h = wave_id % HT;
-  const auto* src = qkv + ((long)t * HT + h) * D;
-  if (bias) bias += (long)h * D;
-  if (h < Hq + Hkv) {
-    // roped write (q -> q_out, k -> cache)
-    const int pos = positions[t];
-    const bool is_q = h < Hq;
-    long dst_row;
-    if (is_q) {
-      dst_row = ((long)t * Hq + h) * D;
-    } else {
-      const int slot = slots[t];
-      if (slot < 0) return;
-      dst_row = ((((long)(slot / P) * Hkv + (h - Hq)) * P + slot % P)) * D;
-    }
-    for (int i = lane; i < half; i += WAVE) {
-      const float c = cos_sin[(long)pos * D + i];
-      const float s = cos_sin[(long)pos * D + half + i];
-      float x1, x2;
-      if constexpr (PARTS) {
-        x1 = x2 = 0.f;
-#pragma unroll 4
-        for (int p = 0; p < parts; ++p) {
-          x1 += src[p * step + i];
-          x2 += src[p * step + half + i];
-        }
-        x1 = bf16_to_f32(f32_to_bf16(x1));
-        x2 = bf16_to_f32(f32_to_bf16(x2));
-      } else {
-        x1 = bf16_to_f32(src[i]);
-        x2 = bf16_to_f32(src[half + i]);
-      }
-      if (bias) {
-        x1 = bf16_to_f32(f32_to_bf16(x1 + bf16_to_f32(bias[i])));
-        x2 = bf16_to_f32(f32_to_bf16(x2 + bf16_to_f32(bias[half + i])));
-      }
-      const float r1 = x1 * c - x2 * s;
-      const float r2 = x2 * c + x1 * s;
-      if (is_q) {
-        __hip_bfloat16* dq = q_out + dst_row;
-        *(unsigned short*)(dq + i) = f32_to_bf16(r1);
-        *(unsigned short*)(dq + half + i) = f32_to_bf16(r2);
-      } else if constexpr (FP8) {
-        unsigned char* dk = (unsigned char*)kc + dst_row;
-        dk[i] = f32_to_fp8(r1);
-        dk[half + i] = f32_to_fp8(r2);
-      } else {
-        __hip_bfloat16* dk = (__hip_bfloat16*)kc + dst_row;
-        *(unsigned short*)(dk + i) = f32_to_bf16(r1);
-        *(unsigned short*)(dk + half + i) = f32_to_bf16(r2);
-      }
-    }
-  } else {
+  const int half = D / 2, HT = Hq + 2 * Hkv;
+  const unsigned units = half / VEC, x = blockIdx.x * 256u + threadIdx.x;
+  const unsigned unit_row = x / units;
+  if (unit_row >= (unsigned)T * HT) return;
+  const int i = (x - unit_row * units) * VEC, t = unit_row / HT, h = unit_row - t * HT;
+  const long row = unit_row;
+  const bool is_q = h < Hq, is_v = h >= Hq + Hkv;
+  long dst = ((long)t * Hq + h) * D + i;
+  if (!is_q) {
     const int slot = slots[t];
     if (slot < 0) return;
-    const long dst_row =
-        ((((long)(slot / P) * Hkv + (h - Hq - Hkv)) * P + slot % P)) * D;
-    for (int i = lane * 8; i < D; i += WAVE * 8) {
-      shortx8 v;
-      if constexpr (PARTS) {
-        float y[8];
-        add_parts8(y, src + i, parts, step);
+    const int head = h - Hq - (is_v ? Hkv : 0);
+    dst = (((long)(slot / P) * Hkv + head) * P + slot % P) * D + i;
+  }
+  float y[2][VEC];  // columns i.. and half + i..
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (short)f32_to_bf16(y[j]);
-      } else {
-        v = *reinterpret_cast<const shortx8*>(src + i);
-      }
-      if (bias) {
-        const shortx8 b = *reinterpret_cast<const shortx8*>(bias + i);
+  for (int z = 0; z < 2; ++z) {
+    const auto* src = qkv + row * D + z * half + i;
+    if constexpr (PARTS && VEC == 8) {
+      add_parts8(y[z], src, parts, step);
+    } else if constexpr (PARTS) {
+      float sum = 0.f;
+#pragma unroll 4
+      for (int p = 0; p < parts; ++p) sum += src[p * step];
+      y[z][0] = bf16_to_f32(f32_to_bf16(sum));
+    } else if constexpr (VEC == 8) {
+      const shortx8 v = *reinterpret_cast<const shortx8*>(src);
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          v[j] = (short)f32_to_bf16(bf16_to_f32((unsigned short)v[j]) +
-                                    bf16_to_f32((unsigned short)b[j]));
-      }
-      if constexpr (FP8) {
-        *reinterpret_cast<u64b*>((unsigned char*)vc + dst_row + i) = bf16x8_to_fp8x8(v);
-      } else {
-        *reinterpret_cast<shortx8*>((__hip_bfloat16*)vc + dst_row + i) = v;
-      }
+      for (int j = 0; j < 8; ++j) y[z][j] = bf16_to_f32((unsigned short)v[j]);
+    } else {
+      y[z][0] = bf16_to_f32(src[0]);
+    }
+    if (bias) {
+      const unsigned short* b = bias + (long)h * D + z * half + i;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+        y[z][j] = bf16_to_f32(f32_to_bf16(y[z][j] + bf16_to_f32(b[j])));
+    }
+  }
+  if (!is_v) {
+    const float* cs = cos_sin + (long)positions[t] * D + i;
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      const float c = cs[j], s = cs[half + j], x1 = y[0][j], x2 = y[1][j];
+      y[0][j] = x1 * c - x2 * s;
+      y[1][j] = x2 * c + x1 * s;
+    }
+  }
+  void* to = is_q ? (void*)q_out : is_v ? vc : kc;
+#pragma unroll
+  for (int z = 0; z < 2; ++z) {
+    const long at = dst + z * half;
+    if (FP8 && !is_q) {
+      unsigned char out[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) out[j] = f32_to_fp8(y[z][j]);
+      if constexpr (VEC == 8) *reinterpret_cast<u64b*>((unsigned char*)to + at) = *(u64b*)out;
+      else ((unsigned char*)to)[at] = out[0];
+    } else {
+      unsigned short out[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) out[j] = f32_to_bf16(y[z][j]);
+      if constexpr (VEC == 8)
+        *reinterpret_cast<shortx8*>((unsigned short*)to + at) = *(shortx8*)out;
+      else ((unsigned short*)to)[at] = out[0];
     }
   }
 }
@@ -507,10 +489,18 @@ torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
               "a contiguous bf16 bias per column");
   auto q_out = torch::empty({(long)T, Hq, (long)D}, qkv.options().dtype(torch::kBFloat16));
   if (T == 0) return q_out;
-  const long waves = (long)T * (Hq + 2 * Hkv);
-  const int wpb = 4;
+  TORCH_CHECK(D % 2 == 0, "head width");
+  uintptr_t bits = 0;
+  for (const void* p : {(const void*)qkv.data_ptr(), (const void*)q_out.data_ptr(),
+                        (const void*)kc.data_ptr(), (const void*)vc.data_ptr()})
+    bits |= (uintptr_t)p;
+  // few rows leave the chip idle with eight columns a thread: 23 rows of 3072 in 5 parts
+  // 3.5 us and 2.8, but 300 rows of 4608 6.2 us both ways
+  const int vec = D % 16 == 0 && bits % 16 == 0 && T * width >= 1 << 20 ? 8 : 1;
+  const long threads = (long)T * (Hq + 2 * Hkv) * (D / 2 / vec);
+  TORCH_CHECK(threads < 1L << 32, "more rows than a launch can index");
   auto launch = [&](auto kern, auto* src) {
-    hipLaunchKernelGGL(kern, dim3((waves + wpb - 1) / wpb), dim3(wpb * WAVE), 0, CUR_STREAM,
+    hipLaunchKernelGGL(kern, dim3((threads + 255) / 256), dim3(256), 0, CUR_STREAM,
                        src, bias ? (const unsigned short*)bias->data_ptr() : nullptr,
                        (__hip_bfloat16*)q_out.data_ptr(), kc.data_ptr(), vc.data_ptr(),
                        positions.data_ptr<int>(), slots.data_ptr<int>(),
@@ -519,13 +509,15 @@ torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
   };
   const auto* f = (const float*)qkv.data_ptr();
   const auto* h = (const unsigned short*)qkv.data_ptr();
+#define ROPE(F8, VEC)                                               \
+  if (raw) launch(fused_rope_kv_write_kernel<F8, true, VEC>, f);    \
+  else launch(fused_rope_kv_write_kernel<F8, false, VEC>, h)
   if (kc.dtype() == torch::kFloat8_e4m3fn) {
-    if (raw) launch(fused_rope_kv_write_kernel<true, true>, f);
-    else launch(fused_rope_kv_write_kernel<true, false>, h);
+    if (vec == 8) { ROPE(true, 8); } else { ROPE(true, 1); }
   } else {
-    if (raw) launch(fused_rope_kv_write_kernel<false, true>, f);
-    else launch(fused_rope_kv_write_kernel<false, false>, h);
+    if (vec == 8) { ROPE(false, 8); } else { ROPE(false, 1); }
   }
+#undef ROPE
   HIP_CHECK_KERNEL();
   return q_out;
 }

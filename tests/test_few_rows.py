@@ -100,3 +100,27 @@ def test_rotation_of_parts(D, dtype, parts, biased):
         q = ops.fused_rope_kv_write(plain, at, slots, cs, *caches, hq, hkv, bias)
         for a, b in zip([q] + [c.float() for c in caches], results[0]):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("D,T", [(128, 230), (64, 460), (72, 3), (24, 5), (128, 2000)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_rotation_widths(D, T, dtype):
+    """Eight columns a thread from 2^20 values on, one below and for other widths."""
+    g = torch.Generator().manual_seed(D)
+    hq, hkv, P = 32, 2, 16
+    qkv = torch.randn(T, (hq + 2 * hkv) * D, generator=g).bfloat16()
+    cs = ops.torch_ref.rope_cos_sin_cache(D, T, 10000.0, dtype=torch.float32)
+    at = torch.arange(T, dtype=torch.int32)
+    slots = torch.randperm(-(-T // P) * P, generator=g)[:T].int()
+    slots[T // 2] = -1
+    kc, vc = (torch.zeros(-(-T // P), hkv, P, D).to(dtype).cuda() for _ in range(2))
+    q = ops.fused_rope_kv_write(qkv.cuda(), at.cuda(), slots.cuda(), cs.cuda(), kc, vc, hq, hkv)
+    k_want, v_want = torch.zeros(kc.shape), torch.zeros(kc.shape)
+    keep = slots >= 0
+    q_want = ops.fused_rope_kv_write(qkv[keep].float(), at[keep], slots[keep], cs, k_want,
+                                     v_want, hq, hkv)
+    # rounded once, to 2^-8 or to 2^-4 of itself (or half the 8-bit type's smallest step)
+    for got, want, step in ((q.cpu()[keep], q_want, 2 ** -8),
+                            (kc.cpu(), k_want, 2 ** -8 if dtype == torch.bfloat16 else 2 ** -4),
+                            (vc.cpu(), v_want, 2 ** -8 if dtype == torch.bfloat16 else 2 ** -4)):
+        assert ((got.float() - want).abs() <= step * want.abs() + 2 ** -10).all()
