@@ -87,6 +87,7 @@ def test_windows(window, chunk, bias, D, DV):
     _check(out.cpu().view(-1, H, DV), want.double().view(-1, H, DV))
 
 
+@torch.inference_mode()  # as the engine captures: the generator is shared
 def test_replay():
     """The stretches of a captured launch follow the contexts of each replay."""
     H, G, D, P = 8, 4, 128, 64

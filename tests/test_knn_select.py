@@ -55,6 +55,7 @@ def test_special_values():
     assert values[0, 1] == float("inf") and torch.isfinite(values[0, 2:]).all()
 
 
+@torch.inference_mode()  # as the engine captures: the generator is shared
 def test_replay():
     docs, queries = _unit(40000, 128, 4), _unit(2, 128, 5)
     ops.knn_topk(queries, docs, 20)
