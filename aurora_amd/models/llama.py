@@ -169,6 +169,15 @@ class _FullWidthMLP(nn.Module):
         return ops.linear(ops.linear_silu_mul(x, self.gate_up), self.down)
 
 
+def _are_slices(whole: Optional[torch.Tensor], weights: List[torch.Tensor]) -> bool:
+    """True where ``weights`` are ``whole[0]``, ``whole[1]`` and so on themselves."""
+    if whole is None or whole.is_meta:
+        return False
+    at, step, shape = whole.data_ptr(), whole.stride(0) * whole.element_size(), whole.shape[1:]
+    return all(w.data_ptr() == at + i * step and w.shape == shape and w.dtype == whole.dtype
+               and w.is_contiguous() for i, w in enumerate(weights))
+
+
 class MoEMLP(nn.Module):
     """Mixtral-style sparse MoE block (top-k routing over dense experts).
 
@@ -216,10 +225,14 @@ class MoEMLP(nn.Module):
         return super()._apply(fn, recurse)
 
     def _stacked(self) -> Tuple[torch.Tensor, torch.Tensor]:
-        if self._w_gu is None:
-            with torch.inference_mode(False):
-                self._share(torch.stack([ex.gate_up.weight.data for ex in self.experts]),
-                            torch.stack([ex.down.weight.data for ex in self.experts]))
+        """All experts' weights, put together anew if one has got another storage
+        (``load_state_dict(assign=True)``, a copy of the module, ``weight.data``)."""
+        gu = [ex.gate_up.weight for ex in self.experts]
+        dn = [ex.down.weight for ex in self.experts]
+        if not (_are_slices(self._w_gu, gu) and _are_slices(self._w_dn, dn)):
+            with torch.inference_mode(gu[0].is_inference()):
+                self._share(torch.stack([w.data for w in gu]),
+                            torch.stack([w.data for w in dn]))
         return self._w_gu, self._w_dn
 
     def _local_expert_fn(self, xp: torch.Tensor,

@@ -1,0 +1,93 @@
+"""Routed experts read the weights that their modules hold now, however they got there."""
+import copy
+
+import pytest
+import torch
+
+from aurora_amd.models.config import get_spec
+from aurora_amd.models.llama import MoEMLP
+
+SPEC = get_spec("tiny-moe")
+
+
+def _fill(m, seed):
+    g = torch.Generator().manual_seed(seed)
+    for p in m.parameters():
+        p.data.copy_(torch.randn(p.shape, generator=g) * 0.1)
+    return m
+
+
+def _by_expert(m, x):
+    weights, sel = m.router(x).topk(SPEC.experts_per_token, dim=-1)
+    weights = weights.softmax(-1)
+    out = torch.zeros_like(x)
+    for e, expert in enumerate(m.experts):
+        tok, slot = (sel == e).nonzero(as_tuple=True)
+        out.index_add_(0, tok, expert(x[tok]) * weights[tok, slot, None])
+    return out
+
+
+def _assign(m, x):
+    m.load_state_dict(_fill(MoEMLP(SPEC, torch.float32), 7).state_dict(), assign=True)
+    return m
+
+
+def _copy_then_load(m, x):
+    m = copy.deepcopy(m)
+    m.load_state_dict(_fill(MoEMLP(SPEC, torch.float32), 7).state_dict())
+    return m
+
+
+def _data(m, x):
+    for p in list(m.experts[1].parameters()):
+        p.data = p.data * 2 + 0.01
+    return m
+
+
+def _parameter(m, x):
+    down = m.experts[0].down
+    down.weight = torch.nn.Parameter(-down.weight.data, requires_grad=False)
+    return m
+
+
+def _in_place(m, x):
+    m.load_state_dict(_fill(MoEMLP(SPEC, torch.float32), 7).state_dict())
+    return m
+
+
+def _other_layout(m, x):
+    w = m.experts[2].gate_up.weight
+    w.data = w.data.t().contiguous().t()
+    return m
+
+
+@pytest.mark.parametrize("change", [_assign, _copy_then_load, _data, _parameter, _in_place,
+                                    _other_layout])
+@pytest.mark.parametrize("after_a_pass", [False, True])
+def test_replaced_weights_are_read(change, after_a_pass):
+    m = _fill(MoEMLP(SPEC, torch.float32), 3)
+    x = torch.randn(33, SPEC.hidden_size)
+    if after_a_pass:
+        m(x)
+    m = change(m, x)
+    for _ in range(2):
+        # fp32 sums of at most 256 terms of another order
+        torch.testing.assert_close(m(x), _by_expert(m, x), rtol=1e-4, atol=1e-5)
+
+
+def test_built_without_memory():
+    with torch.device("meta"):
+        m = MoEMLP(SPEC, torch.float32)
+    m.load_state_dict(_fill(MoEMLP(SPEC, torch.float32), 5).state_dict(), assign=True)
+    x = torch.randn(9, SPEC.hidden_size)
+    torch.testing.assert_close(m(x), _by_expert(m, x), rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.parametrize("inside", [False, True])
+def test_built_in_inference_mode(inside):
+    with torch.inference_mode():
+        m = _fill(MoEMLP(SPEC, torch.float32), 5)
+        _data(m, None)
+    x = torch.randn(9, SPEC.hidden_size)
+    with torch.inference_mode(inside):
+        torch.testing.assert_close(m(x), _by_expert(m, x), rtol=1e-4, atol=1e-5)
