@@ -246,7 +246,7 @@ class MoEMLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         T, H = x.shape
-        if self.ep_size == 1 and ops.has_moe_grouped(x):
+        if self.ep_size == 1 and ops.has_moe_grouped(x, self.router.weight):
             out = ops.moe_silu_glu(x, self.router.weight, self.top_k, *self._stacked())
             return pdist.tp_all_reduce(out) if pdist.tp_world_size() > 1 else out
         logits = self.router(x).float()  # [T, E]
@@ -270,9 +270,10 @@ class MoEMLP(nn.Module):
 
     def _forward_batched(self, x: torch.Tensor, weights: torch.Tensor,
                          sel: torch.Tensor) -> torch.Tensor:
-        """Small batches without the grouped kernels: tokens sorted by expert into a
-        fixed-capacity buffer, batched products over all experts. Static shapes, nothing
-        read back."""
+        """Small batches without the router kernel: tokens sorted by expert and packed for
+        one product per expert that was chosen, or without the extension in a buffer of
+        fixed capacity for batched products over all experts. Static shapes, nothing read
+        back."""
         T, H = x.shape
         E, k = self.n_experts, self.top_k
         flat = sel.reshape(-1)  # [T*k]
@@ -284,6 +285,12 @@ class MoEMLP(nn.Module):
         starts = torch.cumsum(counts, 0) - counts
         w_gu, w_dn = self._stacked()
         wflat = weights.reshape(-1)[order].unsqueeze(1).to(x.dtype)
+        out = torch.zeros_like(x)
+        if ops.has_moe_grouped(x):
+            st, ct = starts.to(torch.int32), counts.to(torch.int32)
+            act = ops.silu_mul(ops.moe_grouped_gemm(x[tok_of], w_gu, st, ct))  # [T*k, I']
+            out.index_add_(0, tok_of, ops.moe_grouped_gemm(act, w_dn, st, ct) * wflat)
+            return pdist.tp_all_reduce(out) if pdist.tp_world_size() > 1 else out
         C = T
         rank = torch.arange(T * k, device=x.device) - starts[flat[order]]
         slot_idx = flat[order] * C + rank  # rank < C always
@@ -293,7 +300,6 @@ class MoEMLP(nn.Module):
         gu = torch.bmm(xe, w_gu.transpose(1, 2).contiguous())  # [E, C, 2I']
         act = ops.silu_mul(gu.reshape(E * C, -1)).view(E, C, -1)
         ye = torch.bmm(act, w_dn.transpose(1, 2).contiguous()).view(E * C, H)
-        out = torch.zeros_like(x)
         out.index_add_(0, tok_of, ye[slot_idx] * wflat)
         return pdist.tp_all_reduce(out) if pdist.tp_world_size() > 1 else out
 

@@ -288,13 +288,16 @@ def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return silu_mul(linear(x, weight))
 
 
-def has_moe_grouped(x: torch.Tensor) -> bool:
-    """True when the grouped expert kernels serve this tensor. Eight experts of 4096 x
+def has_moe_grouped(x: torch.Tensor, router: Optional[torch.Tensor] = None) -> bool:
+    """True when the grouped expert kernels serve this tensor, with ``router`` the router
+    kernel too: 512 experts at most, weights of the tensor's type. Eight experts of 4096 x
     14336, two each: 32 rows 833 -> 516 us against products packed for decoding, 300 rows
     1600 -> 730 and 8192 rows 6210 -> 5740 us against a library product per expert."""
     import os
     return (x.is_cuda and x.dtype == torch.bfloat16 and _hip is not None
             and x.shape[1] % 64 == 0
+            and (router is None or (router.shape[0] <= 512 and router.dtype == x.dtype
+                                    and router.is_contiguous()))
             and os.environ.get("AURORA_MOE_GROUPED", "1") != "0")
 
 

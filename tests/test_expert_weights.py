@@ -1,5 +1,6 @@
 """Routed experts read the weights that their modules hold now, however they got there."""
 import copy
+from dataclasses import replace
 
 import pytest
 import torch
@@ -19,7 +20,7 @@ def _fill(m, seed):
 
 def _by_expert(m, x):
     weights, sel = m.router(x).topk(SPEC.experts_per_token, dim=-1)
-    weights = weights.softmax(-1)
+    weights = weights.float().softmax(-1).to(x.dtype)
     out = torch.zeros_like(x)
     for e, expert in enumerate(m.experts):
         tok, slot = (sel == e).nonzero(as_tuple=True)
@@ -91,3 +92,18 @@ def test_built_in_inference_mode(inside):
     x = torch.randn(9, SPEC.hidden_size)
     with torch.inference_mode(inside):
         torch.testing.assert_close(m(x), _by_expert(m, x), rtol=1e-4, atol=1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 9, 256, 257])
+@pytest.mark.parametrize("experts,strided", [(513, False), (1030, False), (8, True)])
+def test_routers_that_the_kernel_does_not_take(T, experts, strided):
+    """More experts than it has room for, a router stored by columns."""
+    spec = replace(SPEC, hidden_size=64, intermediate_size=64, n_experts=experts)
+    m = _fill(MoEMLP(spec, torch.bfloat16), 11).cuda()
+    x = torch.randn(T, 64).bfloat16().cuda()
+    if strided:
+        m.router.weight.data = m.router.weight.data.t().contiguous().t()
+    got, want = m(x).double(), _by_expert(m, x).double()
+    # products, activations and sums are each rounded to 2^-9 of themselves
+    assert (got - want).norm() <= 2 ** -6 * want.norm()
