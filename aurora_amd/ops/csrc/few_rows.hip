@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void add_parts_kernel(const float* __restrict_
 // 14336, 23 rows: 1 part 52 us, 2 35, 4 23, 8 25; 2048 x 8192: 4 11.8, 8 9.3, 16 10.3; 4608
 // x 3584: 2 11.1, 3 (216 workgroups) 9.3, 4 (288) 11.3.
 static long parts_of(long N, long K) {
-  const long tiles = (N + 63) / 64;
+  const long tiles = std::max(1L, (N + 63) / 64);
   return std::max(1L, std::min({256 / tiles, K / FEW_K / 2, 16L}));
 }
 
