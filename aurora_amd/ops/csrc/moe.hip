@@ -300,9 +300,11 @@ DEVINL float over_1_plus_exp(float x, float z) {
 }
 
 DEVINL float clamped_glu(float g, float u, const GroupArgs& p) {
-  g = fminf(g, p.limit);
-  u = fminf(fmaxf(u, -p.limit), p.limit);
-  return over_1_plus_exp(g * (u + p.shift), p.alpha * g);
+  // (fminf and fmaxf would drop a NaN)
+  g = __builtin_elementwise_minimum(g, p.limit);
+  u = __builtin_elementwise_minimum(__builtin_elementwise_maximum(u, -p.limit), p.limit);
+  // the gate first: a closed one makes nothing of however large an ``up``
+  return over_1_plus_exp(g, p.alpha * g) * (u + p.shift);
 }
 
 // Any size and float32: 32 rows x 64 columns, 16 of K at a time, through LDS as

@@ -20,15 +20,16 @@ def _products(T, F, W, gates, ups):
     return x.cuda(), w.cuda()
 
 
-def _activations(x, w, kernel, limit, alpha, shift):
+def _activations(x, w, kernel, limit, alpha, shift, down=None):
     F = w.shape[0] // 2
     if kernel == "prompt":
         from aurora_amd import _hip_ops
         return _hip_ops.many_rows(x, w, True)
-    eye = torch.eye(x.shape[1], F).bfloat16().cuda()  # what the second product reads
+    down = torch.eye(x.shape[1], F) if down is None else down  # gives what it reads
+    down = down.bfloat16().cuda()
     sel = torch.zeros(x.shape[0], 1, dtype=torch.int32, device="cuda")
     from aurora_amd import _hip_ops
-    y, place = _hip_ops.moe_clamped_glu(x, sel, w[None].contiguous(), eye[None].contiguous(),
+    y, place = _hip_ops.moe_clamped_glu(x, sel, w[None].contiguous(), down[None].contiguous(),
                                         limit, alpha, shift)
     return y[place[:, 0].long(), :F]
 
@@ -56,3 +57,32 @@ def test_rounded_once(kernel, T, F, W, limit, alpha, shift):
     slack = 2.0 ** -21 + (alpha != 1) * z.abs() * 2.0 ** -24
     lo, hi = ((want * (1 + s * slack)).float().bfloat16() for s in (-1, 1))
     assert ((got == lo) | (got == hi)).all()
+
+
+@pytest.mark.parametrize("kernel,T,F,W", SIZES + [("few", 40, 192, 64)])
+@pytest.mark.parametrize("limit", [INF, 7.0])
+def test_special_values(kernel, T, F, W, limit):
+    """NaN stays NaN with and without a limit, a closed gate gives 0 beside any finite
+    number, infinities act as in the formula."""
+    if kernel in ("prompt", "few") and limit < INF:
+        pytest.skip("prompts have no limit")
+    x, w = torch.zeros(T, W).bfloat16().cuda(), torch.zeros(2 * F, W).bfloat16().cuda()
+    x[:, :2] = 1
+    nan = float("nan")
+    for a, b in [(nan, 1), (1, nan), (-2e4, 3e38), (-3e38, 3e38), (3, 2), (3e38, 2), (INF, 1),
+                 (3, INF), (3, -INF), (-INF, 1), (0, INF)]:
+        w[:F, 0], w[F:, 1] = a, b
+        if kernel == "few":
+            got = ops.linear_silu_mul(x, w).double()
+        else:  # the second product adds them up: a row of unlike ones would be NaN
+            got = _activations(x, w, kernel, limit, 1.0, 0.0,
+                               down=torch.ones(W, F)).double() / (1 if kernel == "prompt" else F)
+        g, u = (torch.tensor(v, dtype=torch.float64) for v in (a, b))
+        g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+        want = (g / (1 + torch.exp(-g)) * u).float().double().item()
+        if want != want:
+            assert got.isnan().all(), (a, b)
+        elif abs(want) == INF:
+            assert (got == want).all(), (a, b)
+        else:  # rounded to bf16 twice at most
+            assert ((got - want).abs() <= abs(want) * 2 ** -7).all(), (a, b)
