@@ -181,10 +181,12 @@ torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor weight, double eps) {
 
 std::vector<torch::Tensor> rmsnorm_residual(torch::Tensor x, torch::Tensor res,
                                             torch::Tensor weight, double eps) {
-  if (x.dtype() == torch::kFloat32 && x.dim() == 3) {  // a product in parts
+  // A product in parts: several, each of the residual's two dimensions. Nothing else is
+  // float32: an activation has its residual's shape.
+  if (x.dtype() == torch::kFloat32 && x.dim() == 3 && x.size(0) > 1) {
     const long S = x.size(0), T = x.size(1), H = x.size(2);
     TORCH_CHECK(x.is_cuda() && x.is_contiguous() && res.dtype() == torch::kBFloat16 &&
-                    res.numel() == T * H && weight.numel() == H && H % 8 == 0,
+                    res.dim() == 2 && res.size(0) == T && res.size(1) == H && weight.numel() == H && H % 8 == 0,
                 "parts [S, T, H] and residual [T, H]");
     const auto rc = res.contiguous();
     auto out = torch::empty_like(rc), res_out = torch::empty_like(rc);
