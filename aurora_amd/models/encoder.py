@@ -17,6 +17,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
+from ..parallel.tp import is_plain
 from .config import ModelSpec, get_spec
 
 
@@ -37,7 +38,11 @@ class EncoderLayer(nn.Module):
             p.requires_grad_(False)
         self.eps = spec.rms_eps
 
-    def forward(self, x, delta, cos_sin, positions, cu):
+    def forward(self, x, cos_sin, positions, cu):
+        x, delta = self.step(x, None, cos_sin, positions, cu)
+        return x + delta
+
+    def step(self, x, delta, cos_sin, positions, cu):
         """The stream ``x``, to which ``delta`` (the layer before's result) is still to be
         added -> the stream and this layer's."""
         T = x.shape[0]
@@ -50,7 +55,11 @@ class EncoderLayer(nn.Module):
         ops.rope_apply_(q, k, positions, cos_sin)
         o = ops.attention_prefill(q, k, v, cu, self.scale, causal=False)
         h, x = ops.rmsnorm_residual(self.o(o.reshape(T, -1)), x, self.norm2, self.eps)
-        return x, self.down(ops.linear_silu_mul(h, self.gate_up.weight))
+        if is_plain(self.gate_up, nn.Linear) and self.gate_up.bias is None:
+            act = ops.linear_silu_mul(h, self.gate_up.weight)
+        else:
+            act = ops.silu_mul(self.gate_up(h))
+        return x, self.down(act)
 
 
 class SentenceEncoder(nn.Module):
@@ -97,6 +106,13 @@ class SentenceEncoder(nn.Module):
         x = self.embed(ids)
         delta = None
         for layer in self.layers:
-            x, delta = layer(x, delta, self.cos_sin, pos_t, cu_t)
-        x = ops.rmsnorm_residual(delta, x, self.final_norm, self.spec.rms_eps)[0]
+            if is_plain(layer, EncoderLayer):
+                x, delta = layer.step(x, delta, self.cos_sin, pos_t, cu_t)
+            else:  # somebody watches it or has replaced it
+                x, delta = x if delta is None else x + delta, None
+                x = layer(x, self.cos_sin, pos_t, cu_t)
+        if delta is None:
+            x = ops.rmsnorm(x, self.final_norm, self.spec.rms_eps)
+        else:
+            x = ops.rmsnorm_residual(delta, x, self.final_norm, self.spec.rms_eps)[0]
         return ops.embed_pool(x, cu_t)

@@ -26,6 +26,10 @@ from ..parallel.tp import (
     MergedColumnParallelLinear,
     QKVParallelLinear,
     RowParallelLinear,
+    column_parts,
+    column_silu_mul,
+    is_plain,
+    row_parts,
 )
 from .config import ModelSpec
 
@@ -106,13 +110,21 @@ class LlamaAttention(nn.Module):
         kv_cache: Tuple[torch.Tensor, torch.Tensor],
         meta: AttnMetadata,
     ) -> torch.Tensor:
+        return self.o_proj(self._heads(x, cos_sin, kv_cache, meta))
+
+    def parts(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
+        """As ``forward``, possibly in parts (``ops.linear_parts``)."""
+        return row_parts(self.o_proj, self._heads(x, cos_sin, kv_cache, meta))
+
+    def _heads(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
+        """The heads' results side by side, [T, heads * width]."""
         T = x.shape[0]
-        qkv = self.qkv_proj.parts(x)
+        qkv, bias = column_parts(self.qkv_proj, x)
         k_cache, v_cache = kv_cache
         # fused split + bias + RoPE + paged K/V scatter (one kernel on GPU)
         q = ops.fused_rope_kv_write(qkv, meta.positions, meta.slot_mapping,
                                     cos_sin, k_cache, v_cache,
-                                    self.n_heads, self.n_kv_heads, self.qkv_proj.bias)
+                                    self.n_heads, self.n_kv_heads, bias)
         if meta.mode == "prefill":
             o = ops.attention_prefill_paged(
                 q, k_cache, v_cache, meta.block_tables,
@@ -135,7 +147,7 @@ class LlamaAttention(nn.Module):
                 meta.dec_context_lens, self.scale,
             ) if T > Tp else q[:0]
             o = torch.cat([o_pre, o_dec]) if (Tp and T > Tp) else (o_pre if Tp else o_dec)
-        return self.o_proj.parts(o.reshape(T, self.n_heads * self.head_dim))
+        return o.reshape(T, self.n_heads * self.head_dim)
 
 
 class LlamaMLP(nn.Module):
@@ -145,11 +157,11 @@ class LlamaMLP(nn.Module):
         self.down = RowParallelLinear(spec.intermediate_size, spec.hidden_size, dtype=dtype)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down(ops.linear_silu_mul(x, self.gate_up.weight))
+        return self.down(column_silu_mul(self.gate_up, x))
 
     def parts(self, x: torch.Tensor) -> torch.Tensor:
         """As ``forward``, possibly in parts (``ops.linear_parts``)."""
-        return self.down.parts(ops.linear_silu_mul(x, self.gate_up.weight))
+        return row_parts(self.down, column_silu_mul(self.gate_up, x))
 
 
 class _FullWidthMLP(nn.Module):
@@ -235,6 +247,12 @@ class MoEMLP(nn.Module):
                             torch.stack([w.data for w in dn]))
         return self._w_gu, self._w_dn
 
+    def _experts_plain(self) -> bool:
+        """True where router and experts are what this class made them and nobody watches."""
+        return is_plain(self.router, nn.Linear) and all(
+            is_plain(ex, LlamaMLP) and is_plain(ex.gate_up, ColumnParallelLinear)
+            and is_plain(ex.down, RowParallelLinear) for ex in self.experts)
+
     def _local_expert_fn(self, xp: torch.Tensor,
                          local_sel: torch.Tensor) -> torch.Tensor:
         y = torch.empty_like(xp)
@@ -246,7 +264,8 @@ class MoEMLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         T, H = x.shape
-        if self.ep_size == 1 and ops.has_moe_grouped(x, self.router.weight):
+        if (self.ep_size == 1 and self._experts_plain()
+                and ops.has_moe_grouped(x, self.router.weight)):
             out = ops.moe_silu_glu(x, self.router.weight, self.top_k, *self._stacked())
             return pdist.tp_all_reduce(out) if pdist.tp_world_size() > 1 else out
         logits = self.router(x).float()  # [T, E]
@@ -314,15 +333,21 @@ class LlamaDecoderLayer(nn.Module):
         self.mlp = MoEMLP(spec, dtype) if spec.n_experts > 0 else LlamaMLP(spec, dtype)
 
     def forward(self, x, residual, cos_sin, kv_cache, meta):
+        return self.step(x, residual, cos_sin, kv_cache, meta, False)
+
+    def step(self, x, residual, cos_sin, kv_cache, meta, in_parts: bool):
+        """As ``forward``; with ``in_parts`` the result may be in parts, which
+        ``rmsnorm_residual`` adds up, and so may ``x``."""
         if residual is None:
             residual = x
             h = ops.rmsnorm(x, self.input_norm, self.eps)
         else:
             h, residual = ops.rmsnorm_residual(x, residual, self.input_norm, self.eps)
-        a = self.attn(h, cos_sin, kv_cache, meta)
+        attn = self.attn.parts if is_plain(self.attn, LlamaAttention) else self.attn
+        a = attn(h, cos_sin, kv_cache, meta)
         h, residual = ops.rmsnorm_residual(a, residual, self.post_attn_norm, self.eps)
-        m = self.mlp(h) if isinstance(self.mlp, MoEMLP) else self.mlp.parts(h)
-        return m, residual  # m is read by rmsnorm_residual, which adds up parts
+        mlp = self.mlp.parts if in_parts and is_plain(self.mlp, LlamaMLP) else self.mlp
+        return mlp(h), residual
 
 
 class LlamaForCausalLM(nn.Module):
@@ -367,8 +392,11 @@ class LlamaForCausalLM(nn.Module):
     ) -> torch.Tensor:
         x = self.embed(input_ids)
         residual = None
-        for layer, cache in zip(self.layers, kv_caches):
-            x, residual = layer(x, residual, self.cos_sin, cache, meta)
+        # layers that somebody watches or has replaced are called and get no parts
+        plain = [is_plain(layer, LlamaDecoderLayer) for layer in self.layers] + [True]
+        for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):
+            args = x, residual, self.cos_sin, cache, meta
+            x, residual = layer.step(*args, plain[i + 1]) if plain[i] else layer(*args)
         x = ops.rmsnorm_residual(x, residual, self.final_norm, self.spec.rms_eps)[0]
         return x  # hidden states [T, H]
 

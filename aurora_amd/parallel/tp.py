@@ -8,12 +8,33 @@ loader shards checkpoints the same way.
 """
 from __future__ import annotations
 
+from typing import Optional, Tuple
+
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.nn.modules.module import (
+    _global_backward_hooks,
+    _global_backward_pre_hooks,
+    _global_forward_hooks,
+    _global_forward_pre_hooks,
+)
 
 from .. import ops
 from . import dist as pdist
+
+_CALL = nn.Module.__call__
+
+
+def is_plain(module: nn.Module, kind: type) -> bool:
+    """True where a call of ``module`` is ``kind.forward`` and nothing else: no hook, no
+    other class's or its own forward. Only then may its work be done without the call."""
+    own, cls = module.__dict__, type(module)
+    return not (cls.forward is not kind.forward or cls.__call__ is not _CALL
+                or "forward" in own or own["_forward_hooks"] or own["_forward_pre_hooks"]
+                or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                or _global_forward_hooks or _global_forward_pre_hooks
+                or _global_backward_hooks or _global_backward_pre_hooks)
 
 
 class ColumnParallelLinear(nn.Module):
@@ -45,10 +66,6 @@ class ColumnParallelLinear(nn.Module):
             y = pdist.tp_all_gather(y, dim=-1)
         return y
 
-    def parts(self, x: torch.Tensor) -> torch.Tensor:
-        """This rank's product without its bias, possibly in parts (``ops.linear_parts``)."""
-        return ops.linear_parts(x, self.weight)
-
 
 class RowParallelLinear(nn.Module):
     """Y = all_reduce(X_local @ W_local^T), W_local = W[rank-th input shard]."""
@@ -67,10 +84,6 @@ class RowParallelLinear(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         y = ops.linear(x, self.weight)
         return pdist.tp_all_reduce(y)
-
-    def parts(self, x: torch.Tensor) -> torch.Tensor:
-        """As ``forward``, possibly in parts (``ops.linear_parts``) where nothing is reduced."""
-        return self(x) if pdist.tp_world_size() > 1 else ops.linear_parts(x, self.weight)
 
 
 class QKVParallelLinear(ColumnParallelLinear):
@@ -102,3 +115,25 @@ class MergedColumnParallelLinear(ColumnParallelLinear):
     def __init__(self, hidden: int, intermediate: int, dtype=None):
         super().__init__(hidden, 2 * intermediate, dtype=dtype)
         self.intermediate_local = intermediate // pdist.tp_world_size()
+
+
+def column_parts(m: nn.Module, x: torch.Tensor) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    """``m(x)`` of a column-parallel layer as a product possibly in parts
+    (``ops.linear_parts``) and the bias still to be added."""
+    if is_plain(m, ColumnParallelLinear) and not m.gather_output:
+        return ops.linear_parts(x, m.weight), m.bias
+    return m(x), None
+
+
+def row_parts(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``m(x)`` of a row-parallel layer, possibly in parts where nothing is reduced."""
+    if is_plain(m, RowParallelLinear) and pdist.tp_world_size() == 1:
+        return ops.linear_parts(x, m.weight)
+    return m(x)
+
+
+def column_silu_mul(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``silu_mul(m(x))`` of a merged gate and up layer, in one kernel where that is faster."""
+    if is_plain(m, ColumnParallelLinear) and m.bias is None and not m.gather_output:
+        return ops.linear_silu_mul(x, m.weight)
+    return ops.silu_mul(m(x))
