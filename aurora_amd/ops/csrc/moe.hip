@@ -271,7 +271,7 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
 // ------------------------------------------------------------ grouped product
 
 // what the product's epilogue does
-enum { NO_ACT = 0, GLU_ACT = 1, RELU2_ACT = 2 };
+enum { NO_ACT = 0, GLU_ACT = 1, RELU2_ACT = 2, SILU_ACT = 3 };
 
 struct GroupArgs {
   const void* x;       // rows [*, K]; row r of the sorted batch is x[gather[r]]
@@ -284,19 +284,23 @@ struct GroupArgs {
   int rows = 0;
 };
 
-// x / (1 + e^-z) to two units in the last place, as expf and a division give it but in half
-// their instructions: e^a is 2^t with what the rounding of t = a log2 e left over, the
-// quotient is x times the denominator's reciprocal, corrected once. (The 256-row tile has
-// nothing to hide them behind: 4 prompts of 2000 tokens, 8 experts of 4096 x 14336, spend
-// 2% of a layer more with expf and a division. exp2f and rcpf alone are off by 2^-18 at
-// z = -60.) Below z = -87 it gives 0 for results under 2^-120 of x.
-DEVINL float over_1_plus_exp(float x, float z) {
-  const float t = -z * LOG2E;
-  float rest = __builtin_fmaf(-z, 1.92596303e-8f, __builtin_fmaf(-z, LOG2E, -t));
-  rest = __builtin_amdgcn_fmed3f(rest, -1.f, 1.f);  // infinite t leaves none
-  const float d = 1.f + __builtin_amdgcn_exp2f(t) * __builtin_fmaf(rest, 0.693147181f, 1.f);
+// What replaces expf and a division in the activations, with half their instructions: in
+// the 256-row tile there is nothing to hide them behind (4 prompts of 2000 tokens, 8 experts
+// of 4096 x 14336, took 2% longer with expf and a division).
+
+// x / d for d >= 1, once corrected. 0 where d is 2^126 or more.
+DEVINL float over(float x, float d) {
   const float r = __builtin_amdgcn_rcpf(d), q = x * r;
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, x), r, q), d, x);
+}
+
+// e^x to two units in the last place: 2^t with what the rounding of t = x log2 e left over.
+// (2^t alone is off by 2^-18 at x = 60.)
+DEVINL float exp_whole(float x) {
+  const float t = x * LOG2E;
+  float rest = __builtin_fmaf(x, 1.92596303e-8f, __builtin_fmaf(x, LOG2E, -t));
+  rest = __builtin_amdgcn_fmed3f(rest, -1.f, 1.f);  // infinite t leaves none
+  return __builtin_amdgcn_exp2f(t) * __builtin_fmaf(rest, 0.693147181f, 1.f);
 }
 
 DEVINL float clamped_glu(float g, float u, const GroupArgs& p) {
@@ -304,7 +308,12 @@ DEVINL float clamped_glu(float g, float u, const GroupArgs& p) {
   g = __builtin_elementwise_minimum(g, p.limit);
   u = __builtin_elementwise_minimum(__builtin_elementwise_maximum(u, -p.limit), p.limit);
   // the gate first: a closed one makes nothing of however large an ``up``
-  return over_1_plus_exp(g, p.alpha * g) * (u + p.shift);
+  return over(g, 1.f + exp_whole(-p.alpha * g)) * (u + p.shift);
+}
+
+// silu(g) u with the exponential of silu_mul and the products of few rows
+DEVINL float silu_glu(float g, float u) {
+  return over(g, 1.f + __builtin_amdgcn_exp2f(-LOG2E * g)) * u;
 }
 
 // Any size and float32: 32 rows x 64 columns, 16 of K at a time, through LDS as
@@ -501,7 +510,7 @@ __global__ __launch_bounds__(NTHR) void grouped_bf16_kernel(GroupArgs p) {
 // of a stage's lines.
 template <int ACT>
 __global__ __launch_bounds__(512) void grouped_large_kernel(GroupArgs p, int tiles, int cols) {
-  constexpr bool GLU = ACT == GLU_ACT;
+  constexpr bool GLU = ACT == GLU_ACT || ACT == SILU_ACT;
   constexpr int BN = GLU ? 128 : 256, SLOT = 256 * GK * 2, RING = 5 * SLOT, L = 4;
   // Bands of eight row tiles, down and then across; an XCD takes a contiguous eighth of
   // each, so that its blocks share rows and columns in its L2.
@@ -637,8 +646,8 @@ __global__ __launch_bounds__(512) void grouped_large_kernel(GroupArgs p, int til
       float v[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        v[r] = GLU ? clamped_glu(acc[m][n][r], acc[m][n + (GLU ? NO : 0)][r], p)
-                   : acc[m][n][r];
+        const float x = acc[m][n][r], up = acc[m][n + (GLU ? NO : 0)][r];
+        v[r] = ACT == SILU_ACT ? silu_glu(x, up) : GLU ? clamped_glu(x, up, p) : x;
         if constexpr (ACT == RELU2_ACT) v[r] = v[r] > 0.f ? v[r] * v[r] : 0.f;
       }
       bf16_t* dst = y + (long)(row0 + row) * p.N + c;
@@ -655,7 +664,7 @@ __global__ __launch_bounds__(512) void grouped_large_kernel(GroupArgs p, int til
 
 template <int ACT>
 static void grouped_large(const GroupArgs& p, int tiles) {
-  constexpr int BN = ACT == GLU_ACT ? 128 : 256, lds = 5 * 256 * GK * 2;
+  constexpr int BN = ACT == GLU_ACT || ACT == SILU_ACT ? 128 : 256, lds = 5 * 256 * GK * 2;
   auto kern = grouped_large_kernel<ACT>;
   static const hipError_t once = hipFuncSetAttribute(
       (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -768,7 +777,7 @@ torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu) {
   GroupArgs p = {x.data_ptr(), nullptr, w.data_ptr(), y.data_ptr(), nullptr, (int)N,
                  (int)x.size(1), INFINITY, 1.f, 0.f, (int)T_};
   const int tiles = (int)((T_ + 255) / 256);
-  if (silu) grouped_large<GLU_ACT>(p, tiles);
+  if (silu) grouped_large<SILU_ACT>(p, tiles);
   else grouped_large<NO_ACT>(p, tiles);
   HIP_CHECK_KERNEL();
   return y;
