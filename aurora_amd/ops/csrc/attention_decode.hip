@@ -8,8 +8,8 @@
 //    transposing reads give V^T with its keys in the order in which the scores lie. Nothing
 //    is shared between waves until the end, so there is no barrier in the loop;
 //  * the next 32 keys and values are under way while 32 are computed (16 KB a wave);
-//  * weights keep their 32 bits: each is the sum of two bf16 numbers and meets the values
-//    twice; O is rescaled only when a score exceeds the reference by DEC_SLACK powers
+//  * weights keep their 32 bits: each is the sum of three bf16 numbers (``split3``) and
+//    meets the values three times; O is rescaled only when a score exceeds the reference by DEC_SLACK powers
 //    of two;
 //  * contexts are cut into stretches of equal length, found on the device from all context
 //    lengths (``split_length``), so that a few long ones do not keep the others waiting
@@ -282,20 +282,31 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) o[dt] *= alpha;
     }
-    frag_u hi, lo;
+    frag_u pf[3];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const float p0 = __builtin_amdgcn_exp2f(x[2 * j] - m);
       const float p1 = __builtin_amdgcn_exp2f(x[2 * j + 1] - m);
       l += p0 + p1;
-      hi.u[j] = cvt2_bf16(p0, p1);
-      lo.u[j] = cvt2_bf16(p0 - __builtin_bit_cast(float, hi.u[j] << 16),
-                          p1 - __builtin_bit_cast(float, hi.u[j] & 0xffff0000u));
+      unsigned u[3];
+      split3(p0, p1, u);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) pf[k].u[j] = u[k];
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int x = 0; x < LV; ++x)
       *reinterpret_cast<shortx8*>(ring + (lane + x * WAVE) * 16) = widen(vr[x]);
+    if (t0 + DEC_KEYS > t_hi || (BIAS && t0 < t_lo)) {
+      // keys that nobody sees: what stands in their place may be infinite
+#pragma unroll
+      for (int x = 0; x < LV; ++x) {
+        const int t = t0 + (lane + x * WAVE) / VU;
+        if (t >= t_hi || (BIAS && t < t_lo))
+          *reinterpret_cast<shortx8*>(ring + (lane + x * WAVE) * 16) =
+              shortx8{0, 0, 0, 0, 0, 0, 0, 0};
+      }
+    }
     load_values(t0 + ROUND, next_row);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -308,8 +319,9 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
         frag_u vf;
         vf.h[0] = v[2 * j];
         vf.h[1] = v[2 * j + 1];
-        o[d4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, lo.v, o[d4 + j], 0, 0, 0);
-        o[d4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, hi.v, o[d4 + j], 0, 0, 0);
+#pragma unroll
+        for (int k = 2; k >= 0; --k)
+          o[d4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf[k].v, o[d4 + j], 0, 0, 0);
       }
     }
   };
