@@ -115,7 +115,7 @@ DEVINL void read_value_tiles(shortx4 (&v)[8], unsigned a0, unsigned a1, unsigned
 // FLAT_BIAS results may be turned back and gated. PAGED: pages are whole tiles.
 // Without ``cut`` a workgroup takes a whole context.
 template <int D, int DV, bool FP8, int BIAS, bool PAGED>
-__global__ __launch_bounds__(256) void paged_decode_kernel(
+__global__ __launch_bounds__(256, 2) void paged_decode_kernel(
     const __hip_bfloat16* __restrict__ q,   // [B, Hq, D]
     // (not __restrict__: loads of them must stay before the waits that count them)
     const void* kc,  // [NP, Hkv, P, D] bf16 | fp8 e4m3
@@ -315,14 +315,14 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(
       read_value_tiles<16 * DV * 2>(v, vat + (vcol ^ (d4 * 32)), vat + (vcol ^ (d4 * 32 + 32)),
                                     vat + (vcol ^ (d4 * 32 + 64)), vat + (vcol ^ (d4 * 32 + 96)));
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        frag_u vf;
-        vf.h[0] = v[2 * j];
-        vf.h[1] = v[2 * j + 1];
+      for (int k = 2; k >= 0; --k)
 #pragma unroll
-        for (int k = 2; k >= 0; --k)
+        for (int j = 0; j < 4; ++j) {
+          frag_u vf;
+          vf.h[0] = v[2 * j];
+          vf.h[1] = v[2 * j + 1];
           o[d4 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf[k].v, o[d4 + j], 0, 0, 0);
-      }
+        }
     }
   };
   using EVEN = std::integral_constant<int, 0>;

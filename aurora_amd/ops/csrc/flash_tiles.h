@@ -33,19 +33,27 @@ DEVINL unsigned int cvt2_bf16(float lo, float hi) {
   return __builtin_bit_cast(unsigned int, b);
 }
 
+typedef __attribute__((ext_vector_type(2))) unsigned short ushortx2;
+DEVINL unsigned max_halves(unsigned a, unsigned b) {
+  return __builtin_bit_cast(unsigned, __builtin_elementwise_max(__builtin_bit_cast(ushortx2, a),
+                                                                __builtin_bit_cast(ushortx2, b)));
+}
+
 // Two weights p >= 0 (or NaN) as three bf16 numbers each whose sum is p to its last bit: the
 // first eight, the next eight and the last eight bits. A term that would be 0 beside p > 0 is
 // 2^-126, so that a weight times an infinite value is that infinity, as in fp32.
 DEVINL void split3(float p0, float p1, unsigned (&u)[3]) {
-  const float t0 = fminf(p0, 0x1p-126f), t1 = fminf(p1, 0x1p-126f);
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const unsigned a = __builtin_bit_cast(unsigned, p0), b = __builtin_bit_cast(unsigned, p1);
     u[k] = __builtin_amdgcn_perm(b, a, 0x07060302);  // the upper halves
-    if (k == 2) break;
-    p0 = fmaxf(p0 - __builtin_bit_cast(float, a & 0xffff0000u), t0);
-    p1 = fmaxf(p1 - __builtin_bit_cast(float, b & 0xffff0000u), t1);
+    p0 -= __builtin_bit_cast(float, a & 0xffff0000u);
+    p1 -= __builtin_bit_cast(float, b & 0xffff0000u);
   }
+  const ushortx2 least = __builtin_elementwise_min(__builtin_bit_cast(ushortx2, u[0]),
+                                                   ushortx2{0x80, 0x80});
+  u[1] = max_halves(u[1], __builtin_bit_cast(unsigned, least));
+  u[2] = max_halves(u[2], __builtin_bit_cast(unsigned, least));
 }
 
 // Transposing reads of two V^T fragments, of each the halves HALF bytes apart. Written out
