@@ -16,12 +16,12 @@
 // One head of 128 query rows per workgroup, 32 per wave, in the manner of the paged
 // prompt kernel: S^T = K Q^T and O^T = V^T P^T, so a lane owns a row. Two tiles of 64 keys
 // in LDS, the next one loaded while one is computed. Weights keep their 32 bits: each is
-// the sum of two bf16 numbers and meets the values twice.
+// the sum of three bf16 numbers (``split3``) and meets the values three times.
 // Bound by memory and by the start of its many short sequences: 200 texts of 20 to 256
 // tokens, 12 heads of 64 (170 MB) 676 us as a wave per row and head over scalar dot
 // products, now 69 us.
 template <int D>
-__global__ __launch_bounds__(256) void packed_attn_kernel(
+__global__ __launch_bounds__(256, 2) void packed_attn_kernel(
     const __hip_bfloat16* __restrict__ q,  // rows of Hq heads, D apart
     const __hip_bfloat16* __restrict__ k,  // rows of Hkv heads
     const __hip_bfloat16* __restrict__ v,
@@ -116,7 +116,8 @@ __global__ __launch_bounds__(256) void packed_attn_kernel(
                                                                    second * 32 * D * 2);
         s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf.v, qf[c].v, s, 0, 0, 0);
       }
-      if (ks + 31 >= n || (causal && ks + 31 > row0)) {
+      const bool partly = ks + 31 >= n || (causal && ks + 31 > row0);
+      if (partly) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
           const int key = ks + (r & 3) + 8 * (r >> 2) + 4 * half;
@@ -137,22 +138,50 @@ __global__ __launch_bounds__(256) void packed_attn_kernel(
 #pragma unroll
           for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
       }
-      frag_u hi[2], lo[2];
+      frag_u pf[3][2];
       float sum = 0.f;
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
-        float p[2], rest[2];
+        float p[2];
 #pragma unroll
         for (int j = 0; j < 2; ++j)
           p[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[2 * r + j], c2, -m));
         sum += p[0] + p[1];
-        const unsigned u = cvt2_bf16(p[0], p[1]);
-        rest[0] = p[0] - __builtin_bit_cast(float, u << 16);
-        rest[1] = p[1] - __builtin_bit_cast(float, u & 0xffff0000u);
-        hi[r >> 2].u[r & 3] = u;
-        lo[r >> 2].u[r & 3] = cvt2_bf16(rest[0], rest[1]);
+        unsigned u[3];
+        split3(p[0], p[1], u);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) pf[k][r >> 2].u[r & 3] = u[k];
       }
       l += sum;
+      // Where rows do not see all keys, infinite values stay out of the products, which
+      // would make NaN of them and the others' 0, and are added to those who see them.
+      const char* const vt = smem + st + KBYTES + second * 32 * D * 2;
+      bool wild = false;
+      if (partly) {
+        unsigned most = 0;
+#pragma unroll
+        for (int x = 0; x < 32 * U / WAVE; ++x) {
+          frag_u f;
+          f.s = *reinterpret_cast<const shortx8*>(vt + (lane + x * WAVE) * 16);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) most = max_halves(most, f.u[j] & 0x7fff7fffu);
+        }
+        wild = __any(most >= 0x7f800000u || (most & 0xffffu) >= 0x7f80u);
+        if (wild)
+          for (int t = 0; t < 32; ++t) {
+            if (ks + t >= n || (causal && ks + t > row)) continue;
+            const unsigned swz = D == 64 ? (t & 2) << 1 : (t & 3) << 2;
+#pragma unroll
+            for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+              for (int r = 0; r < 16; ++r) {
+                const unsigned unit = dt * 4 + (r >> 2);
+                const unsigned short y = *reinterpret_cast<const unsigned short*>(
+                    vt + t * D * 2 + ((unit ^ swz) * 8 + 4 * half + (r & 3)) * 2);
+                if ((y & 0x7f80u) == 0x7f80u) o[dt][r] += bf16_to_f32(y);
+              }
+          }
+      }
       __builtin_amdgcn_sched_barrier(0);
       // pair i of V^T fragments: 16 keys i / (NDT / 2), d-tiles i % (NDT / 2) * 2 + {0, 1}
       shortx4 vf[NDT][4];
@@ -166,14 +195,23 @@ __global__ __launch_bounds__(256) void packed_attn_kernel(
       static_for<NDT>([&](auto I) {
         constexpr int i = decltype(I)::value, c = i / (NDT / 2), dt = i % (NDT / 2) * 2;
         if constexpr (i + 1 < NDT) fetch(std::integral_constant<int, i + 1>{});
+        frag_u f[2];
 #pragma unroll
         for (int x = 0; x < 2; ++x) {
-          frag_u f;
-          f.h[0] = vf[i][2 * x];
-          f.h[1] = vf[i][2 * x + 1];
-          o[dt + x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.v, lo[c].v, o[dt + x], 0, 0, 0);
-          o[dt + x] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.v, hi[c].v, o[dt + x], 0, 0, 0);
+          f[x].h[0] = vf[i][2 * x];
+          f[x].h[1] = vf[i][2 * x + 1];
+          if (wild)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              f[x].u[j] &= ((f[x].u[j] & 0x7f80u) == 0x7f80u ? 0u : 0xffffu) |
+                           ((f[x].u[j] & 0x7f800000u) == 0x7f800000u ? 0u : 0xffff0000u);
         }
+#pragma unroll
+        for (int k = 2; k >= 0; --k)
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+            o[dt + x] =
+                __builtin_amdgcn_mfma_f32_32x32x16_bf16(f[x].v, pf[k][c].v, o[dt + x], 0, 0, 0);
         if constexpr (i + 1 < NDT) await_values(vf[i + 1]);
       });
     });

@@ -104,3 +104,44 @@ def test_decoding_behind_a_window(L, window):
             c[:, first // 64, :, :first % 64] = INF  # rows before the window
             c[:, -1, :, (L - 1) % 64 + 1:] = -INF
     _check(*_decode(L, 64, 64, bias=True, window=window, spoil=spoil))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+def test_packed_rows_keep_32_bits(D, causal):
+    k, v, want = _near(D)
+    q = torch.zeros(128 * 3, 1, D).bfloat16()
+    q[:, :, 0] = 1
+    cu = torch.arange(129, dtype=torch.int32) * 3
+    out = ops.attention_prefill(q.cuda(), k.reshape(-1, 1, D).cuda(), v.reshape(-1, 1, D).cuda(),
+                                cu.cuda(), 1.0, causal=causal)
+    _check_near(out.view(128, 3, D)[:, 2:], want)  # the last row sees all three
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("value", [INF, -INF, NAN])
+def test_packed_rows_over_infinite_values(D, causal, value):
+    """Only rows that see an infinite value are infinite in its channel, in every place of
+    a tile, at a sequence's end and beside other sequences."""
+    g = torch.Generator().manual_seed(D)
+    lens = [1, 31, 40, 64, 65, 100, 130, 200]
+    at = [0, 30, 39, 17, 64, 70, 33, 131]  # the spoiled row of each
+    cu = torch.tensor([0] + lens).cumsum(0)
+    T = int(cu[-1])
+    q, k, v = (torch.randn(T, h, D, generator=g).bfloat16() for h in (4, 2, 2))
+    for s, a in enumerate(at):
+        v[cu[s] + a, s % 2, (7 * s) % D] = value
+    out = ops.attention_prefill(*(x.cuda() for x in (q, k, v)), cu.int().cuda(), D ** -0.5,
+                                causal=causal).double().cpu()
+    want = torch.empty(T, 4, D, dtype=torch.float64)
+    for s, n in enumerate(lens):
+        rows = slice(int(cu[s]), int(cu[s + 1]))
+        x, keys, values = (t[rows].double().transpose(0, 1) for t in (
+            q, k.repeat_interleave(2, 1), v.repeat_interleave(2, 1)))
+        w = x @ keys.transpose(1, 2) * D ** -0.5
+        for r in range(n):
+            sees = r + 1 if causal else n
+            p = w[:, r, :sees].softmax(-1)
+            want[rows.start + r] = (p[:, :, None] * values[:, :sees]).sum(1)
+    _check(out, want)
