@@ -12,6 +12,8 @@
 // were rounded to bf16 before. What is left is the start and end of two kernels, some 20 us,
 // and at a million the rate of a read.
 #include "flash_tiles.h"
+#include "plain.h"
+#include <c10/core/DeviceGuard.h>
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
@@ -283,6 +285,7 @@ template <typename T>
 static std::vector<torch::Tensor> nearest(const torch::Tensor& query, const torch::Tensor& docs,
                                           int k) {
   const long Q = query.size(0), D = query.size(1), N = docs.size(0);
+  const c10::DeviceGuard on(docs.device());
   // about two workgroups per CU, which hold 1024 at most: 400000 documents, 768 floats, 256
   // 298 us, 512 264, 1024 306
   const long share = std::min<long>(KNN_DOCS, std::max<long>(128, (N / 512 + 127) / 128 * 128));
@@ -315,8 +318,9 @@ std::vector<torch::Tensor> knn_topk(torch::Tensor query, torch::Tensor docs, lon
   // and as many neighbours as a wave has lanes. Within
   // that the kernels won at every size tried, most narrowly with 3 queries and 1 neighbour:
   // 607 and 667 us at a million in fp32, 27 and 31 at 5000; 16 queries and 40 neighbours 649
-  // and 852. The library's product serves the rest.
-  if (docs.is_cuda() && query.dim() == 2 && docs.dim() == 2 && query.size(1) == docs.size(1) &&
+  // and 852. The library's product serves the rest, and all that autograd, a transform or a
+  // trace follows.
+  if (plain(query) && plain(docs) && docs.is_cuda() && query.dim() == 2 && docs.dim() == 2 && query.size(1) == docs.size(1) &&
       (f32 || docs.dtype() == torch::kBFloat16) && docs.is_contiguous() &&
       query.is_contiguous() && query.size(1) > 0 && query.size(1) * size % 256 == 0 &&
       query.size(1) * size <= 4096 && query.size(0) > 0 && query.size(0) <= KNN_QUERIES &&
