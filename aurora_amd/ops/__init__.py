@@ -194,12 +194,13 @@ def knn_topk(query: torch.Tensor, docs: torch.Tensor, k: int):
 
 
 def _own_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """True for products that the own kernels can take."""
+    """True for products that the own kernels can take: not what autograd, a transform or a
+    trace follows, which passes through the library's."""
     return (x.is_cuda and x.dim() == 2 and x.shape[0] > 0 and x.shape[1] > 0
             and x.shape[1] % 64 == 0 and x.shape[1] == weight.shape[1]
             and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
-            and _hip is not None and weight.is_contiguous()
-            and weight.data_ptr() % 16 == 0
+            and x.device == weight.device and _hip is not None and _hip.plain(x, weight)
+            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
             and not (x.is_contiguous() and x.data_ptr() % 16))
 
 

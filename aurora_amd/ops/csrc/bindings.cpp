@@ -1,4 +1,5 @@
 // Python bindings of the decoder kernels (gfx950).
+#include "plain.h"
 #include <torch/extension.h>
 
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor weight, double eps);
@@ -172,6 +173,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "decode-path skinny GEMM (M<=64)");
   m.def("fused_rope_kv_write", &fused_rope_kv_write,
         "fused qkv split + RoPE + paged KV scatter");
+  m.def("plain", [](const torch::Tensor& x, const torch::Tensor& w) { return plain(x) && plain(w); },
+        "whether nobody follows what is done with two tensors");
   m.def("many_rows", &many_rows, "products of many rows, with silu(gate) * up");
   m.def("few_rows", &few_rows, "products of at most 128 rows, K in parts");
   m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows");

@@ -44,3 +44,36 @@ def test_search_traced():
     q, d = _search_inputs()
     traced = torch.jit.trace(lambda x: ops.knn_topk(x, d, 5)[0], q, check_trace=False)
     torch.testing.assert_close(traced(-q), ops.knn_topk(-q, d, 5)[0], rtol=1e-5, atol=1e-4)
+
+
+#: rows, outputs, K: what the kernels of few rows, of many and of prompts take otherwise
+PRODUCTS = [(40, 256, 192), (100, 256, 3072), (300, 64, 64), (6400, 4096, 14336)]
+
+
+@pytest.mark.parametrize("m,n,k", PRODUCTS)
+def test_product_gradients(m, n, k):
+    x = torch.randn(m, k, device="cuda").bfloat16().requires_grad_()
+    w = (torch.randn(n, k, device="cuda") * k ** -0.5).bfloat16()
+    y = ops.linear(x, w)
+    y.backward(torch.ones_like(y))
+    want = w.double().sum(0).expand(m, k)
+    # sums of n terms, rounded to bf16
+    assert (x.grad.double() - want).norm() <= 2 ** -7 * want.norm()
+
+
+@pytest.mark.parametrize("m,n,k", PRODUCTS[:3])
+def test_product_transforms(m, n, k):
+    x = torch.randn(3, m, k, device="cuda").bfloat16()
+    w = (torch.randn(n, k, device="cuda") * k ** -0.5).bfloat16()
+    want = x.double() @ w.double().t()
+    for f in (ops.linear, ops.linear_parts):
+        got = torch.func.vmap(f, in_dims=(0, None))(x, w)
+        assert (got.double() - want).norm() <= 2 ** -8 * want.norm()
+    traced = torch.jit.trace(lambda a: ops.linear(a, w), x[0], check_trace=False)
+    got = traced(x[1])
+    assert (got.double() - want[1]).norm() <= 2 ** -8 * want[1].norm()
+
+
+def test_products_of_two_devices():
+    with pytest.raises(RuntimeError):
+        ops.linear(torch.ones(4, 64, device="cuda").bfloat16(), torch.ones(8, 64).bfloat16())
