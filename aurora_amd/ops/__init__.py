@@ -16,6 +16,7 @@ from __future__ import annotations
 from typing import Optional, Tuple
 
 import torch
+import torch.nn.functional as F
 
 from . import torch_ref
 
@@ -193,100 +194,26 @@ def knn_topk(query: torch.Tensor, docs: torch.Tensor, k: int):
     return torch_ref.knn_topk(query, docs, k)
 
 
-def _own_product(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    """True for products that the own kernels can take: not what autograd, a transform or a
-    trace follows, which passes through the library's."""
-    return (x.is_cuda and x.dim() == 2 and x.shape[0] > 0 and x.shape[1] > 0
-            and x.shape[1] % 64 == 0 and x.shape[1] == weight.shape[1]
-            and x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16
-            and x.device == weight.device and _hip is not None and _hip.plain(x, weight)
-            and weight.is_contiguous() and weight.data_ptr() % 16 == 0
-            and not (x.is_contiguous() and x.data_ptr() % 16))
-
-
-def _few_rows(x: torch.Tensor, weight: torch.Tensor) -> bool:
-    return x.dim() == 2 and x.shape[0] <= 128 and _own_product(x, weight)
-
-
-def _many_rows_win(x: torch.Tensor, weight: torch.Tensor, silu: bool) -> bool:
-    """True for more than 128 rows where the kernel of 256-row tiles beats the library's
-    product (with ``silu``, product and activation), us. With silu: any number of tiles up to
-    1024 of K (6144 x 768, 300 rows 22 and 25, 27000 rows 250 and 349), else those that fill
-    the chip's rounds (16384 x 2048, 600 rows 45 and 48, 6172 rows 330 and 411; 28672 x 4096,
-    2048 rows 371 and 376, 6172 rows 1132 and 1224; not full: 1600 rows 346 and 341, 12288 x
-    4096, 3000 rows 255 and 248). Without: only where the tiles nearly fill the chip twice
-    and K is long, where the library falls to 0.75 to 1.2 PFLOP/s (4096 x 14336, 6172 rows
-    594 and 807, 7000 rows 630 and 696; 3584 x 18944, 7500 rows 798 and 1184; outside: 6144
-    rows of 4096 x 14336 586 and 565, 8000 rows 677 and 629)."""
-    T, K, N = x.shape[0], x.shape[1], weight.shape[0]
-    tiles = -(-T // 256) * -(-N // 256)
-    if not silu:
-        return K >= 14336 and 384 < tiles < 512
-    if K <= 1024:
-        return T >= 256 and tiles >= 48
-    full = tiles / (-(-tiles // 256) * 256)
-    return tiles >= 192 and full >= (0.75 if K <= 2048 else 0.78)
-
-
-def _few_rows_win(x: torch.Tensor, weight: torch.Tensor, raw: bool) -> bool:
-    """True where that kernel beats the library's (us, cold weights): up to 32 rows always
-    (28672 x 4096, 23 rows 50 and 56, 128256 x 2048 101 and 120); up to 64 while the weights
-    are at most 128 MB (16384 x 2048 18 and 19, but 37888 x 3584 66 and 62); above that up to
-    8192 outputs with parts that their reader adds up (3072 x 2048, 96 rows, 8 and 13), or
-    with K long enough to pay for adding them (4096 x 4096 15 and 22, 6144 x 4096 22 and 23,
-    but 2048 x 2048 11 and 9)."""
-    M, K, N = x.shape[0], x.shape[1], weight.shape[0]
-    if M <= 32:
-        return True
-    if M <= 64:
-        import os
-        max_mb = int(os.environ.get("AURORA_SKINNY_MAX_MB", "128"))
-        return N * K * 2 <= max_mb * 1024 * 1024
-    return N <= 8192 and (raw or K >= 3072)
-
-
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
-    """Bias-free linear: own kernels on the GPU where they win, hipBLASLt otherwise."""
-    import torch.nn.functional as F
-    if _few_rows(x, weight) and _few_rows_win(x, weight, False):
-        return _hip.linear_few_rows(x.contiguous(), weight, False)
-    if (x.dim() == 2 and x.shape[0] > 128 and _own_product(x, weight)
-            and _many_rows_win(x, weight, False)):
-        return _hip.many_rows(x.contiguous(), weight, False)
-    if (x.is_cuda and x.dim() == 2 and 64 < x.shape[0] <= 256
-            and x.shape[1] % 64 == 0 and weight.shape[0] % 64 == 0
-            and x.dtype == torch.bfloat16 and _hip is not None):
-        # measured per-shape dispatch (cold rotated weights) —
-        # the glds v3 kernel wins the qkv shape at M>128 (1.36 vs 1.18
-        # TB/s) and deep-K at M<=128 (down128 2.18 vs 1.59); hipBLASLt
-        # keeps o / gate_up / lm-head. Gated off with AURORA_SKINNY3=0.
-        import os
-        if os.environ.get("AURORA_SKINNY3", "1") != "0":
-            M, K, N = x.shape[0], x.shape[1], weight.shape[0]
-            if (K >= 8192 and M <= 128) or (4096 < N <= 8192 and K <= 4096
-                                            and M > 128):
-                return _hip.skinny_gemm3_ex(x.contiguous(), weight, 384)
-    return F.linear(x, weight)
+    """Bias-free linear: own kernels on the GPU where they win (``own_product``),
+    hipBLASLt otherwise."""
+    y = _hip.own_product(x, weight, 0) if x.is_cuda and _hip is not None else None
+    return F.linear(x, weight) if y is None else y
 
 
 def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """As ``linear``, but where the product of few rows is cut along K its parts
     [S, T, N] in float32, for a reader that adds and rounds them itself
     (``rmsnorm_residual``, ``fused_rope_kv_write``)."""
-    if _few_rows(x, weight) and _few_rows_win(x, weight, True):
-        return _hip.linear_few_rows(x.contiguous(), weight, True)
-    return linear(x, weight)
+    y = _hip.own_product(x, weight, 1) if x.is_cuda and _hip is not None else None
+    return F.linear(x, weight) if y is None else y
 
 
 def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up of the products with gate's rows, then up's; in one kernel where that
     is faster."""
-    if weight.shape[0] % 16 == 0 and _own_product(x, weight):
-        if x.shape[0] <= 128:
-            return _hip.silu_few_rows(x.contiguous(), weight)
-        if _many_rows_win(x, weight, True):
-            return _hip.many_rows(x.contiguous(), weight, True)
-    return silu_mul(linear(x, weight))
+    y = _hip.own_product(x, weight, 2) if x.is_cuda and _hip is not None else None
+    return silu_mul(linear(x, weight)) if y is None else y
 
 
 def has_moe_grouped(x: torch.Tensor, router: Optional[torch.Tensor] = None) -> bool:

@@ -1,5 +1,4 @@
 // Python bindings of the decoder kernels (gfx950).
-#include "plain.h"
 #include <torch/extension.h>
 
 torch::Tensor rmsnorm(torch::Tensor x, torch::Tensor weight, double eps);
@@ -23,6 +22,8 @@ torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
                                   torch::Tensor kc, torch::Tensor vc,
                                   long Hq, long Hkv,
                                   c10::optional<torch::Tensor> bias);
+c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Tensor& w,
+                                         long form);
 torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
 torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts);
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
@@ -173,8 +174,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("skinny_gemm", &skinny_gemm, "decode-path skinny GEMM (M<=64)");
   m.def("fused_rope_kv_write", &fused_rope_kv_write,
         "fused qkv split + RoPE + paged KV scatter");
-  m.def("plain", [](const torch::Tensor& x, const torch::Tensor& w) { return plain(x) && plain(w); },
-        "whether nobody follows what is done with two tensors");
+  m.def("own_product", &own_product, "a product by the own kernels where they win");
   m.def("many_rows", &many_rows, "products of many rows, with silu(gate) * up");
   m.def("few_rows", &few_rows, "products of at most 128 rows, K in parts");
   m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows");

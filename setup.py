@@ -15,7 +15,7 @@ from torch.utils.cpp_extension import BuildExtension, CUDAExtension
 CSRC = "aurora_amd/ops/csrc/"
 EXTENSIONS = {
     # decoder kernels
-    "_hip_ops": ["bindings.cpp", "elementwise.hip", "attention_decode.hip",
+    "_hip_ops": ["bindings.cpp", "products.cpp", "elementwise.hip", "attention_decode.hip",
                  "attention_prefill.hip", "skinny_gemm.hip", "few_rows.hip", "residual_norm.hip",
                  "attention_rows.hip", "recurrence.hip", "moe.hip", "sublayer.hip",
                  "latent_attention.hip", "output_norm.hip", "conv_heads.hip"],
