@@ -14,35 +14,80 @@ torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target);
 
 enum { WHOLE = 0, PARTS = 1, SILU = 2 };
 
-// Up to 128 rows, where the kernel beats the library's (us, cold weights): up to 32 rows
-// always (28672 x 4096, 23 rows 50 and 56, 128256 x 2048 101 and 120); up to 64 while the
-// weights are at most 128 MB (16384 x 2048 18 and 19, but 37888 x 3584 66 and 62); above that
-// up to 8192 outputs with parts that their reader adds up (3072 x 2048, 96 rows, 8 and 13),
-// or with K long enough to pay for adding them (4096 x 4096 15 and 22, 6144 x 4096 22 and 23,
-// but 2048 x 2048 11 and 9).
-static bool few_rows_win(long M, long N, long K, bool parts) {
-  if (M <= 32) return true;
-  if (M <= 64) {
-    const char* mb = std::getenv("AURORA_SKINNY_MAX_MB");
-    return N * K * 2 <= (mb ? std::atol(mb) : 128) * 1024 * 1024;
-  }
-  return N <= 8192 && (parts || K >= 3072);
+static long megabytes(long N, long K) { return (N * K * 2) >> 20; }
+
+// Weights up to here are read in one go by the kernel of few rows, whatever their shape.
+static long small_megabytes() {
+  const char* mb = std::getenv("AURORA_SKINNY_MAX_MB");
+  return mb ? std::atol(mb) : 128;
 }
 
-// More than 128 rows, where the kernel of 256-row tiles beats the library's product (with
-// silu, product and activation), us. With silu: any number of tiles up to 1024 of K (6144 x
-// 768, 300 rows 22 and 25, 27000 rows 250 and 349), else those that fill the chip's rounds
-// (16384 x 2048, 600 rows 45 and 48, 6172 rows 330 and 411; 28672 x 4096, 2048 rows 371 and
-// 376, 6172 rows 1132 and 1224; not full: 1600 rows 346 and 341, 12288 x 4096, 3000 rows 255
-// and 248). Without: only where the tiles nearly fill the chip twice and K is long, where the
-// library falls to 0.75 to 1.2 PFLOP/s (4096 x 14336, 6172 rows 594 and 807, 7000 rows 630 and
-// 696; 3584 x 18944, 7500 rows 798 and 1184; outside: 6144 rows of 4096 x 14336 586 and 565,
-// 8000 rows 677 and 629).
+// Up to 128 rows: where the kernel beats the library's. us with cold weights, ours and the
+// library's. Small weights up to 64 rows (4096 x 14336, 23 rows 24 and 33). Larger ones up to
+// 32 rows while K is short, up to 512 MB of them to 4096 (1 and 32 rows: 152064 x 3584 195
+// and 233, 208 and 264; 32000 x 4096 54 and 60, 56 and 66; but 128256 x 4096 204 and 187, 207
+// and 201; 57344 x 8192 213 and 181; 16384 x 8192 66 and 62, 65 and 54; the other way, given
+// up, 28672 x 8192 105 and 131). Above 64 rows up to 8192 outputs with parts that their
+// reader adds up (3072 x 2048, 96 rows, 8 and 13), or with K long enough to pay for adding
+// them, few outputs with longer ones (96 rows: 4608 x 4096 16 and 22, 2048 x 4096 13.3 and
+// 12.8, 2048 x 8192 15 and 21, 1024 x 8192 15.2 and 15.0, 1024 x 14336 17 and 25, 8192 x 28672
+// 123 and 124; but 4608 x 2048 13.1 and 13.5, 128 rows 15.9 and 15.0; 10240 x 8192 57 and 55).
+static bool few_rows_win(long M, long N, long K, bool parts) {
+  if (M > 64)
+    return N <= 8192 &&
+           (parts || K >= 14336 || (K >= 3072 && N >= (K < 8192 ? 3072 : 2048)));
+  const long size = megabytes(N, K);
+  return size <= small_megabytes() ||
+         (M <= 32 && (K < 4096 || (K == 4096 && size <= 512)));
+}
+
+// The same with silu, N outputs of 2 N rows of weights, against a library product and an
+// activation: K is not cut here, so a tile of 32 outputs takes its K's time and long K wants
+// tiles for all CUs, above 32 rows as many for each (``even``). Library's time over ours at
+// 1, 23, 64, 96 and 128 rows:
+//   K     tiles 16                  56                       112
+//   2048  1.25 1.26 0.93 0.75 0.60  1.23 1.24 1.01 1.02 0.90  1.20 1.20 1.01 1.05 0.92
+//   3072  1.18 1.11 0.79 0.58 0.47  1.17 0.99 0.80 0.73 0.65  1.05 0.96 1.00 0.91 0.84
+//   4096  0.80 0.82 0.70 0.54 0.43  0.84 0.83 0.66 0.60 0.54  1.02 0.94 0.87 0.89 0.76
+//   8192  0.51 0.51 0.42 0.36 0.28  0.66 0.68 0.54 0.47 0.43  0.83 0.79 0.78 0.78 0.67
+//         tiles 160                 224                      296
+//   2048  1.17 1.16 1.16 1.08 1.01  1.11 1.15 1.13 1.15 0.97  1.09 1.11 1.03 1.07 0.96
+//   3072  1.13 1.10 1.09 1.10 0.97  1.08 1.12 1.05 1.08 1.03  1.08 1.02 0.98 0.87 0.79
+//   4096  1.04 1.06 1.08 1.09 0.95  1.02 1.05 0.98 1.07 0.97  1.02 0.99 0.93 0.86 0.79
+//   8192  0.93 0.98 0.90 0.99 0.89  0.91 0.94 0.90 1.01 0.91  0.86 1.01 0.87 0.83 0.75
+// K 1024 1.05 to 1.55, but 0.95 at 16 tiles and 128 rows; 4096 with 448 tiles 1.40 1.21 1.07
+// 1.02 1.01, with 384 1.05 1.07 0.96 1.01 0.97; 3584 with 592 1.03 1.04 1.00 0.89 0.84; 8192
+// with 896 0.96 0.92 0.94 1.00 0.98.
+static bool silu_few_rows_win(long M, long N, long K) {
+  const long tiles = (N + 31) / 32;
+  const bool even = tiles <= 256 || (tiles >= 410 && tiles <= 512);
+  if (K <= 1024) return true;
+  if (M <= 32)
+    return K <= 3072 || (K <= 4096 && tiles >= 88) || (K <= 5120 && tiles >= 160);
+  if (M <= 64)
+    return K <= 3072 ? tiles >= (K <= 2048 ? 32 : 88) : K <= 4096 && tiles >= 160 && even;
+  if (M <= 96) return K <= 2048 ? tiles >= 56 : K <= 4096 && tiles >= 160 && even;
+  return K <= 2048 && tiles >= 160;
+}
+
+// More than 128 rows: where the kernel of 256-row tiles beats the library's product (with
+// silu, product and activation). Library's time over ours, at rows of 256 r, - 57 and - 200.
+// With silu, K up to 1024: everywhere tried from 256 rows on (2048 to 6144 x 768 and 1024, 1.07
+// to 2.1). To 2048: from r = 3 on (4096 to 17920 x 1536 and 2048: mostly 1.1 to 1.6; least
+// 5632, r 11, 0.90, 11264, r 5, 9 and 10, 0.92 to 0.97; r 2 0.75 to 1.2). Longer: where the
+// library falls behind, r 4, 7, 8 and from 11 on (8192 to 37888 x 3584 to 5120 1.0 to 1.5;
+// 57344 x 8192 0.92 to 1.15); elsewhere it is the library's (28672 x 4096, r 2 0.84, 5 0.88, 6
+// 0.92, 9 0.84, 10 0.92; 24576 x 4096, r 5 0.90).
+// Without: only where the tiles fill the chip twice but for a part, where the library takes
+// three rounds (2048 to 8192 outputs, by tiles: K 11008, 350 to 432 0.91 to 1.59, 470 to 512
+// 0.86 to 0.96; K 14336 to 28672, 350 to 480 1.1 to 1.65 but for 8192 at 448, 1.0, 500 to 512
+// 0.86 to 1.0; K 8192, 350 to 512 0.9 to 0.98, 300 0.85).
 static bool many_rows_win(long M, long N, long K, bool silu) {
-  const long tiles = (M + 255) / 256 * ((N + 255) / 256), rounds = (tiles + 255) / 256;
-  if (!silu) return K >= 14336 && tiles > 384 && tiles < 512;
+  const long rows = (M + 255) / 256, tiles = rows * ((N + 255) / 256);
+  if (!silu) return K >= 11008 && tiles >= 350 && tiles <= (K >= 14336 ? 480 : 432);
   if (K <= 1024) return M >= 256 && tiles >= 48;
-  return tiles >= 192 && tiles >= (K <= 2048 ? 0.75 : 0.78) * 256 * rounds;
+  if (tiles < 96) return false;
+  return K <= 2048 ? rows >= 3 : rows == 4 || rows == 7 || rows == 8 || rows >= 11;
 }
 
 // x @ w^T in ``form``, or nothing: the library's product serves better or is followed by
@@ -60,7 +105,10 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
   const c10::DeviceGuard on(x.device());
   if (form == SILU) {
     if (N % 16) return {};
-    if (M <= 128) return silu_few_rows(x.contiguous(), w);
+    if (M <= 128) {
+      if (!silu_few_rows_win(M, N / 2, K)) return {};
+      return silu_few_rows(x.contiguous(), w);
+    }
     if (many_rows_win(M, N, K, true)) return many_rows(x.contiguous(), w, true);
     return {};
   }
@@ -71,11 +119,11 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
   } else if (many_rows_win(M, N, K, false)) {
     return many_rows(x.contiguous(), w, false);
   }
-  // Cold weights: W streamed once past up to 256 rows wins for 4096 to 8192 outputs above 128
-  // rows (6144 x 4096 1.36 and 1.18 TB/s), and up to there for long K and more outputs than
-  // the kernel above takes. AURORA_SKINNY3=0 leaves them to the library.
-  if (M > 64 && M <= 256 && N % 64 == 0 &&
-      (M <= 128 ? K >= 8192 : N > 4096 && N <= 8192 && K <= 4096)) {
+  // Cold weights: W streamed once past up to 256 rows, ours and the library's, 192 and 256
+  // rows: 6144 x 4096 33 and 34, 38 and 42; 4608 x 3584 30 and 30, 32 and 36. Fewer rows, more
+  // outputs and shorter K are the library's (160 rows 32 and 29, 29 and 25; 192 of 8192 x 4096
+  // 38 and 36, 6144 x 2048 26 and 22). AURORA_SKINNY3=0 leaves them all to it.
+  if (M >= 192 && M <= 256 && N % 64 == 0 && N > 4096 && N <= 6144 && K > 2048 && K <= 4096) {
     const char* off = std::getenv("AURORA_SKINNY3");
     if (!off || std::strcmp(off, "0")) return skinny_gemm3_ex(x.contiguous(), w, 384);
   }
