@@ -306,8 +306,9 @@ void rope_apply_(torch::Tensor q, torch::Tensor k, torch::Tensor positions,
               "bf16 GPU only");
   const long T = q.size(0);
   const int Hq = q.size(1), D = q.size(2), Hkv = k.size(1);
-  for (auto* t : {&q, &k})
-    TORCH_CHECK(t->stride(2) == 1 && t->stride(1) == D && t->size(0) == T && t->size(2) == D,
+  for (auto* t : {&q, &k})  // (the stride of a single head says nothing)
+    TORCH_CHECK(t->stride(2) == 1 && (t->stride(1) == D || t->size(1) == 1) &&
+                    t->size(0) == T && t->size(2) == D,
                 "heads of a row lie side by side");
   if (T == 0) return;
   auto cs = cos_sin.to(torch::kFloat32).contiguous();
