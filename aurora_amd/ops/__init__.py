@@ -223,7 +223,7 @@ def has_moe_grouped(x: torch.Tensor, router: Optional[torch.Tensor] = None) -> b
     1600 -> 730 and 8192 rows 6210 -> 5740 us against a library product per expert."""
     import os
     return (x.is_cuda and x.dtype == torch.bfloat16 and _hip is not None
-            and x.shape[1] % 64 == 0
+            and x.shape[1] % 64 == 0 and not (x.is_contiguous() and x.data_ptr() % 16)
             and (router is None or (router.shape[0] <= 512 and router.dtype == x.dtype
                                     and router.is_contiguous()))
             and os.environ.get("AURORA_MOE_GROUPED", "1") != "0")

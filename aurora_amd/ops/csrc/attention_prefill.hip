@@ -547,6 +547,12 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
 // query heads per workgroup: the GQA group shares each staged K/V tile
 static int heads_per_block(int G) { return G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1; }
 
+// A cache as loads straight to LDS can read it: 16-byte units at 16-byte addresses
+static torch::Tensor unit_aligned(const torch::Tensor& cache) {
+  const bool ok = (reinterpret_cast<uintptr_t>(cache.data_ptr()) & 15) == 0;
+  return ok ? cache : cache.clone();
+}
+
 template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED, typename... Args>
 static void prefill_launch(int blocks, int Hq, Args... args) {
   constexpr int lds = PRE_STAGES * PRE_KEYS * (D + DV) * 2;
@@ -569,6 +575,8 @@ torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
   TORCH_CHECK(D == 128 || D == 64, "head_dim must be 64 or 128, got ", D);
   auto out = torch::empty_like(q);
   if (T == 0) return out;
+  kc = unit_aligned(kc);
+  vc = unit_aligned(vc);
   TORCH_CHECK(Hq % Hkv == 0, "GQA requires Hq % Hkv == 0");
   const int HG = heads_per_block(Hq / Hkv);
   const int QROWS = 32 * (8 / HG);  // q rows covered per workgroup
@@ -636,6 +644,8 @@ void biased_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
               cu_q.numel() == ctx.numel() + 1 && bt.size(0) == ctx.numel());
   const int NB = bseq.numel();
   if (T == 0 || NB == 0) return;
+  kc = unit_aligned(kc);
+  vc = unit_aligned(vc);
   const int HG = heads_per_block(Hq / Hkv);
   const float* rp = rates ? rates->data_ptr<float>() : nullptr;
   const float* sp = slopes ? slopes->data_ptr<float>() : nullptr;
@@ -699,6 +709,8 @@ void sink_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
               cu_q.numel() == ctx.numel() + 1 && bt.size(0) == ctx.numel());
   const int NB = bseq.numel();
   if (T == 0 || NB == 0) return;
+  kc = unit_aligned(kc);
+  vc = unit_aligned(vc);
 #define SLAUNCH(DD, DVV)                                                        \
   prefill_launch<DD, DVV, 1, false, NO_BIAS, GATED, false>(NB, H,                       \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
@@ -747,6 +759,8 @@ void tailed_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
               cu_q.numel() == ctx.numel() + 1 && bt.size(0) == ctx.numel());
   const int NB = bseq.numel();
   if (T == 0 || NB == 0) return;
+  kc = unit_aligned(kc);
+  vc = unit_aligned(vc);
   const KeyTail kt = {(const __hip_bfloat16*)tail.data_ptr(), tail.stride(0),
                       (int)tail.size(1), own};
 #define TLAUNCH(DD, DVV)                                                        \

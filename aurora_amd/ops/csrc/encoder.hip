@@ -244,9 +244,11 @@ __global__ __launch_bounds__(256, 2) void packed_attn_kernel(
 
 // [T, H, D] whose rows may be strided, as 16-byte loads can read it
 static torch::Tensor row_readable(const torch::Tensor& t) {
-  const bool ok = t.stride(2) == 1 && t.stride(1) == t.size(2) && t.stride(0) % 8 == 0 &&
+  const bool ok = t.stride(2) == 1 && (t.stride(1) == t.size(2) || t.size(1) == 1) &&
+                  (t.stride(0) % 8 == 0 || t.size(0) == 1) &&
                   (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
-  return ok ? t : t.contiguous();
+  // (contiguous() gives the same tensor back where only its address is odd)
+  return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
 torch::Tensor attention_prefill(torch::Tensor q_, torch::Tensor k_, torch::Tensor v_,

@@ -33,3 +33,50 @@ def test_rotation_of_one_head(T):
     got = ops.rope_apply(q, k, at.cuda(), cs.cuda())
     for a, b in zip(got, want):
         assert ((a.cpu().float() - b).abs() <= b.abs() * 2 ** -8 + 2 ** -12).all()
+
+
+@pytest.mark.parametrize("H,G,D", [(4, 2, 64), (1, 1, 128), (3, 1, 64)])
+@pytest.mark.parametrize("layout", ["off", "one head"])
+@pytest.mark.parametrize("lens", [[1], [5, 70, 33]])
+def test_packed_attention(H, G, D, layout, lens):
+    if layout == "one head" and (H, G) != (1, 1):
+        pytest.skip("of one head")
+    g = torch.Generator().manual_seed(D)
+    cu = torch.tensor([0] + lens).cumsum(0).int()
+    T = int(cu[-1])
+    if layout == "off":
+        q, k, v = (_off(torch.randn(T, h, D, generator=g).bfloat16()) for h in (H, G, G))
+    else:
+        q, k, v = (_one_head(T, D, g) for _ in range(3))
+    got = ops.attention_prefill(q, k, v, cu.cuda(), D ** -0.5, causal=False)
+    want = torch_ref.attention_prefill(q.cpu().float(), k.cpu().float(), v.cpu().float(), cu,
+                                       D ** -0.5, False)
+    assert (got.cpu().float() - want).norm() <= 2 ** -7.5 * want.norm()
+
+
+@pytest.mark.parametrize("P", [16, 64])
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("elements", [1, 3, 4])
+def test_prompts_over_a_cache_at_an_odd_address(P, cache, elements):
+    g = torch.Generator().manual_seed(P)
+    D, L, n = 64, 150, 40
+    k, v = (_off(torch.randn(-(-L // P), 2, P, D, generator=g).to(cache), elements)
+            for _ in range(2))
+    q = torch.randn(n, 4, D, generator=g).bfloat16()
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32)  # noqa: E731
+    args = torch.arange(-(-L // P), dtype=torch.int32)[None], i32(0, n), i32(L)
+    got = ops.attention_prefill_paged(q.cuda(), k, v, *(a.cuda() for a in args), D ** -0.5)
+    want = ops.attention_prefill_paged(q.cuda(), k.clone(), v.clone(),
+                                       *(a.cuda() for a in args), D ** -0.5)
+    assert torch.equal(got, want)
+
+
+def test_experts_of_rows_at_an_odd_address():
+    from aurora_amd.models.config import get_spec
+    from aurora_amd.models.llama import MoEMLP
+    m = MoEMLP(get_spec("smoke-moe"), torch.bfloat16).cuda()
+    for p in m.parameters():
+        p.data.normal_(0, p.shape[-1] ** -0.5)
+    x = torch.randn(300, 512, device="cuda").bfloat16()
+    got, want = m(_off(x)), m(x)
+    assert (got.float() - want.float()).norm() <= 2 ** -6 * want.float().norm()
