@@ -18,6 +18,7 @@ from typing import List, Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.utils.dlpack import from_dlpack, to_dlpack
 
 from .. import ops
 from ..parallel import dist as pdist
@@ -190,6 +191,12 @@ def _are_slices(whole: Optional[torch.Tensor], weights: List[torch.Tensor]) -> b
                and w.is_contiguous() for i, w in enumerate(weights))
 
 
+def _apart(x: torch.Tensor) -> torch.Tensor:
+    """The same memory with a storage of its own: whoever saves ``x`` saves no more, and
+    does not find it to be a part of something."""
+    return x if x.is_meta else from_dlpack(to_dlpack(x))
+
+
 class MoEMLP(nn.Module):
     """Mixtral-style sparse MoE block (top-k routing over dense experts).
 
@@ -220,8 +227,8 @@ class MoEMLP(nn.Module):
             self.experts = nn.ModuleList(
                 [LlamaMLP(spec, dtype) for _ in range(spec.n_experts)]
             )
-        self._w_gu = None  # all experts' weights in one tensor each, of which the
-        self._w_dn = None  # experts' own are views
+        self._w_gu = None  # all experts' weights in one tensor each, in whose memory the
+        self._w_dn = None  # experts' own lie
         if self.ep_size == 1:
             gu, dn = self.experts[0].gate_up.weight, self.experts[0].down.weight
             self._share(gu.new_empty((self.n_experts, *gu.shape)),
@@ -229,7 +236,7 @@ class MoEMLP(nn.Module):
 
     def _share(self, w_gu: torch.Tensor, w_dn: torch.Tensor) -> None:
         for e, ex in enumerate(self.experts):
-            ex.gate_up.weight.data, ex.down.weight.data = w_gu[e], w_dn[e]
+            ex.gate_up.weight.data, ex.down.weight.data = _apart(w_gu[e]), _apart(w_dn[e])
         self._w_gu, self._w_dn = w_gu, w_dn
 
     def _apply(self, fn, recurse: bool = True):

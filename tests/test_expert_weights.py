@@ -94,6 +94,22 @@ def test_built_in_inference_mode(inside):
         torch.testing.assert_close(m(x), _by_expert(m, x), rtol=1e-4, atol=1e-5)
 
 
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)])
+@pytest.mark.parametrize("after_a_pass", [False, True])
+def test_saved_as_weights_of_their_own(device, after_a_pass, tmp_path):
+    m = _fill(MoEMLP(SPEC, torch.bfloat16 if device == "cuda" else torch.float32), 3).to(device)
+    if after_a_pass:
+        m(torch.randn(9, SPEC.hidden_size, device=device).to(m.router.weight.dtype))
+    safetensors = pytest.importorskip("safetensors.torch")
+    safetensors.save_model(m, str(tmp_path / "m.safetensors"))
+    torch.save(m.experts[0].state_dict(), tmp_path / "e.pt")
+    size = sum(p.numel() * p.element_size() for p in m.experts[0].parameters())
+    assert (tmp_path / "e.pt").stat().st_size < size + 8192
+    read = safetensors.load_file(str(tmp_path / "m.safetensors"))
+    for name, p in m.named_parameters():
+        assert torch.equal(read[name], p.cpu())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("T", [1, 9, 256, 257])
 @pytest.mark.parametrize("experts,strided", [(513, False), (1030, False), (8, True)])
