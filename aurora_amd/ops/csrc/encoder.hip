@@ -256,8 +256,8 @@ torch::Tensor attention_prefill(torch::Tensor q_, torch::Tensor k_, torch::Tenso
   TORCH_CHECK(q_.is_cuda() && q_.dtype() == torch::kBFloat16, "bf16 GPU only");
   const int T = q_.size(0), Hq = q_.size(1), D = q_.size(2), Hkv = k_.size(1);
   TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64/128");
-  TORCH_CHECK(k_.dtype() == q_.dtype() && v_.dtype() == q_.dtype() && k_.size(0) == T &&
-              v_.size(0) == T && v_.size(1) == Hkv && k_.size(2) == D && v_.size(2) == D &&
+  TORCH_CHECK(k_.dtype() == q_.dtype() && v_.dtype() == q_.dtype() && k_.size(0) >= T &&
+              v_.size(0) >= T && v_.size(1) == Hkv && k_.size(2) == D && v_.size(2) == D &&
               Hq % Hkv == 0 && cu.dtype() == torch::kInt32 && cu.is_contiguous(),
               "queries, keys and values");
   auto out = torch::empty({T, Hq, D}, q_.options());

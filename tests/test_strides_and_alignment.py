@@ -54,6 +54,14 @@ def test_packed_attention(H, G, D, layout, lens):
     assert (got.cpu().float() - want).norm() <= 2 ** -7.5 * want.norm()
 
 
+def test_packed_attention_of_a_longer_buffer():
+    """Keys and values may have rows past the queries' last."""
+    q, k, v = (torch.randn(n, 2, 64, device="cuda").bfloat16() for n in (40, 64, 50))
+    cu = torch.tensor([0, 15, 40], dtype=torch.int32, device="cuda")
+    got = ops.attention_prefill(q, k, v, cu, 0.125, causal=True)
+    assert torch.equal(got, ops.attention_prefill(q, k[:40], v[:40], cu, 0.125, causal=True))
+
+
 @pytest.mark.parametrize("P", [16, 64])
 @pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e4m3fn])
 @pytest.mark.parametrize("elements", [1, 3, 4])
