@@ -1,7 +1,7 @@
-"""Cold-weight skinny-GEMM sweep: rotates >LLC-sized W copies so every
-iteration streams W from HBM (the in-engine regime; the earlier sweep kept
-one W hot in LLC and mistuned s_target).  Prints TB/s per config vs
-hipBLASLt on the llama3-8b decode shapes."""
+"""Sweep of the products of few rows over the parts of K, on weights that come from memory:
+copies larger than the last-level cache are used in turn, as an engine's layers are. Prints
+TB/s of the weights per number of parts, of the rule's own choice and of hipBLASLt for
+llama3-8b's decode shapes; SHAPES overrides them, BLASLT_ONLY=1 leaves ours out."""
 import os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch
@@ -36,19 +36,17 @@ for tag, M, K, N in SHAPES:
     iters = max(20, min(60, 3 * ncopy))
     res = {}
     only_blaslt = os.environ.get("BLASLT_ONLY") == "1"
-    for st in () if (only_blaslt or M > 64) else (256, 512, 1024, 2048):
-        for unr in (2, 4):
-            dt = timeit(lambda i: hip.skinny_gemm_ex(x, ws[i % ncopy], st, unr), iters)
-            res[f"sk_s{st}_u{unr}"] = dt
-    if K % 128 == 0 and not only_blaslt:
-        for st in (256, 512, 768, 1024, 2048):
-            dt = timeit(lambda i: hip.skinny_gemm2_ex(x, ws[i % ncopy], st), iters)
-            res[f"v2_s{st}"] = dt
-        # numerics: v2 vs fp32 reference on the last W
+    if M <= 128 and K % 64 == 0 and not only_blaslt:
+        for parts in (1, 2, 4, 8, 16):
+            res[f"parts_{parts}"] = timeit(
+                lambda i: hip.few_rows(x, ws[i % ncopy], False, parts), iters)
+        res["own_choice"] = timeit(lambda i: hip.linear_few_rows(x, ws[i % ncopy], False), iters)
+        res["left_in_parts"] = timeit(lambda i: hip.linear_few_rows(x, ws[i % ncopy], True), iters)
+        # numerics against fp32 on the last W
         ref = (x.float() @ ws[0].float().t())
-        got = hip.skinny_gemm2_ex(x, ws[0], 768).float()
+        got = hip.linear_few_rows(x, ws[0], False).float()
         err = (got - ref).abs().max().item() / max(ref.abs().max().item(), 1e-6)
-        assert err < 2e-2, f"v2 numerics off: rel {err}"
+        assert err < 2e-2, f"numerics off: rel {err}"
     res["blaslt"] = timeit(lambda i: torch.matmul(x, ws[i % ncopy].t()), iters)
     best = min(res, key=res.get)
     print(f"== {tag} M={M} K={K} N={N} W={wb/1e6:.0f}MB (x{ncopy} copies)")

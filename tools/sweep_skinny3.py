@@ -1,5 +1,5 @@
 """Cold-weight sweep for the v3 (M=128-256) projection GEMM: numerics vs
-fp32 torch reference, then TB/s vs hipBLASLt and v2m on the llama3-8b
+fp32 torch reference, then TB/s vs hipBLASLt and the other own kernel on the llama3-8b
 decode shapes with W copies rotated past the 256 MB LLC."""
 import json
 import os
@@ -56,8 +56,10 @@ for tag, M, K, N in SHAPES:
     for st in (256, 384, 512, 640, 896):
         dt = timeit(lambda i: hip.skinny_gemm3_ex(x, ws[i % ncopy], st), iters)
         res[f"v3_s{st}"] = dt
-    dt = timeit(lambda i: hip.skinny_gemm2_ex(x, ws[i % ncopy], 512), iters)
-    res["v2m_s512"] = dt
+    if M > 128:
+        res["many_rows"] = timeit(lambda i: hip.many_rows(x, ws[i % ncopy], False), iters)
+    else:
+        res["few_rows"] = timeit(lambda i: hip.linear_few_rows(x, ws[i % ncopy], False), iters)
     res["blaslt"] = timeit(lambda i: torch.matmul(x, ws[i % ncopy].t()), iters)
     best = min(res, key=res.get)
     print(f"== {tag} M={M} K={K} N={N} W={wb/1e6:.0f}MB (x{ncopy} copies)")
