@@ -237,7 +237,7 @@ def moe_silu_glu(x: torch.Tensor, router: torch.Tensor, top: int, w_gate_up: tor
     m = _require_hip("moe_silu_glu")
     x = x.contiguous()
     sel, weights = m.moe_route(x, router, None, top)
-    y, place = m.moe_clamped_glu(x, sel, w_gate_up, w_down, float("inf"), 1.0, 0.0)
+    y, place = m.moe_silu_glu(x, sel, w_gate_up, w_down)
     return m.moe_combine(y, place, weights)
 
 

@@ -117,6 +117,8 @@ void retention_decode(torch::Tensor proj, torch::Tensor decay, torch::Tensor cos
 std::vector<torch::Tensor> moe_route(torch::Tensor h, torch::Tensor router,
                                      c10::optional<torch::Tensor> bias, long top);
 torch::Tensor moe_combine(torch::Tensor y, torch::Tensor place, torch::Tensor gate);
+std::vector<torch::Tensor> moe_silu_glu(torch::Tensor h, torch::Tensor sel, torch::Tensor w_gu,
+                                        torch::Tensor w_dn);
 std::vector<torch::Tensor> moe_clamped_glu(torch::Tensor h, torch::Tensor sel,
                                            torch::Tensor w_gu, torch::Tensor w_dn,
                                            double limit, double alpha, double shift);
@@ -221,6 +223,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("retention_prefill", &retention_prefill, "retention, chunked");
   m.def("retention_decode", &retention_decode, "retention, one token per sequence");
   m.def("moe_route", &moe_route, "fp32 router, top choice, softmax over the chosen");
+  m.def("moe_silu_glu", &moe_silu_glu, "sorted grouped silu GLU experts");
   m.def("moe_combine", &moe_combine, "weighted sum of every token's expert rows");
   m.def("moe_route_grouped", &moe_route_grouped,
         "fp32 sigmoid or softmax router, top choice among the best groups");

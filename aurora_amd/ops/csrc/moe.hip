@@ -282,33 +282,28 @@ struct GroupArgs {
   int N, K;
   float limit, alpha, shift;
   int rows = 0;
+  bool silu = false;   // no limit, alpha 1 and shift 0, with silu_mul's exponential
 };
 
-// What replaces expf and a division in the activations, with half their instructions: in
-// the 256-row tile there is nothing to hide them behind (4 prompts of 2000 tokens, 8 experts
-// of 4096 x 14336, took 2% longer with expf and a division).
-
-// x / d for d >= 1, once corrected. 0 where d is 2^126 or more.
+// x / d for d >= 1, once corrected: what replaces a division in the 256-row tile, whose
+// results are bf16 and which has nothing to hide it behind. silu is as near to 64 bits with it
+// as with a division (off by 1.75e-7 of itself at most, 3.7e-8 rms, -85 to 20), and 4 prompts
+// of 2000 tokens, 8 experts of 4096 x 14336, lose half of the 2% that a division costs. (2^(x
+// log2 e) in place of expf saves another 1% and is off by 3.9e-6; with the product's rounding
+// brought in by 2.3e-7.) 0 where d is 2^126 or more.
 DEVINL float over(float x, float d) {
   const float r = __builtin_amdgcn_rcpf(d), q = x * r;
   return __builtin_amdgcn_div_fixupf(__builtin_fmaf(__builtin_fmaf(-d, q, x), r, q), d, x);
 }
 
-// e^x to two units in the last place: 2^t with what the rounding of t = x log2 e left over.
-// (2^t alone is off by 2^-18 at x = 60.)
-DEVINL float exp_whole(float x) {
-  const float t = x * LOG2E;
-  float rest = __builtin_fmaf(x, 1.92596303e-8f, __builtin_fmaf(x, LOG2E, -t));
-  rest = __builtin_amdgcn_fmed3f(rest, -1.f, 1.f);  // infinite t leaves none
-  return __builtin_amdgcn_exp2f(t) * __builtin_fmaf(rest, 0.693147181f, 1.f);
-}
-
+template <bool TILE256 = false>
 DEVINL float clamped_glu(float g, float u, const GroupArgs& p) {
   // (fminf and fmaxf would drop a NaN)
   g = __builtin_elementwise_minimum(g, p.limit);
   u = __builtin_elementwise_minimum(__builtin_elementwise_maximum(u, -p.limit), p.limit);
+  const float d = 1.f + expf(-p.alpha * g);
   // the gate first: a closed one makes nothing of however large an ``up``
-  return over(g, 1.f + exp_whole(-p.alpha * g)) * (u + p.shift);
+  return (TILE256 ? over(g, d) : g / d) * (u + p.shift);
 }
 
 // silu(g) u with the exponential of silu_mul and the products of few rows
@@ -647,7 +642,7 @@ __global__ __launch_bounds__(512) void grouped_large_kernel(GroupArgs p, int til
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const float x = acc[m][n][r], up = acc[m][n + (GLU ? NO : 0)][r];
-        v[r] = ACT == SILU_ACT ? silu_glu(x, up) : GLU ? clamped_glu(x, up, p) : x;
+        v[r] = ACT == SILU_ACT ? silu_glu(x, up) : GLU ? clamped_glu<true>(x, up, p) : x;
         if constexpr (ACT == RELU2_ACT) v[r] = v[r] > 0.f ? v[r] * v[r] : 0.f;
       }
       bf16_t* dst = y + (long)(row0 + row) * p.N + c;
@@ -692,7 +687,8 @@ static void grouped(const GroupArgs& p, bool bf16, int tiles, int TM, long busy)
   constexpr bool GLU = ACT == GLU_ACT;
   if (bf16 && p.K % GK == 0) {
     const long blocks = (p.N + (GLU ? 63 : 127)) / (GLU ? 64 : 128) * busy;
-    if (TM == 256) grouped_large<ACT>(p, tiles);
+    if (TM == 256 && ACT == GLU_ACT && p.silu) grouped_large<SILU_ACT>(p, tiles);
+    else if (TM == 256) grouped_large<ACT>(p, tiles);
     else if (TM == 128) grouped_bf16<128, 128, 2, 256, ACT>(p, tiles);
     else if (TM == 64) grouped_bf16<64, 128, 3, 256, ACT>(p, tiles);
     // few rows: the weights' stream counts. Two workgroups per CU with four
@@ -712,7 +708,8 @@ static void grouped(const GroupArgs& p, bool bf16, int tiles, int TM, long busy)
 template <int ACT>
 static std::vector<torch::Tensor> experts(const torch::Tensor& h, const torch::Tensor& sel,
                                           const torch::Tensor& w_up, const torch::Tensor& w_dn,
-                                          double limit, double alpha, double shift) {
+                                          double limit, double alpha, double shift,
+                                          bool silu = false) {
   TORCH_CHECK(h.is_cuda() && h.dim() == 2 && h.is_contiguous() && sel.is_contiguous() &&
               sel.dtype() == torch::kInt32 && sel.size(0) == h.size(0));
   const long T_ = h.size(0), W = h.size(1), top = sel.size(1), A = T_ * top;
@@ -745,7 +742,7 @@ static std::vector<torch::Tensor> experts(const torch::Tensor& h, const torch::T
                      place.data_ptr<int>(), token.data_ptr<int>(), table.data_ptr<int>());
   GroupArgs p = {h.data_ptr(), token.data_ptr<int>(), w_up.data_ptr(), act.data_ptr(),
                  table.data_ptr<int>(), (int)F, (int)W, (float)limit, (float)alpha,
-                 (float)shift};
+                 (float)shift, 0, silu};
   grouped<ACT>(p, bf16, tiles, TM, std::min(E, A));
   p.x = act.data_ptr();
   p.gather = nullptr;
@@ -762,6 +759,12 @@ std::vector<torch::Tensor> moe_clamped_glu(torch::Tensor h, torch::Tensor sel,
                                            torch::Tensor w_gu, torch::Tensor w_dn,
                                            double limit, double alpha, double shift) {
   return experts<GLU_ACT>(h, sel, w_gu, w_dn, limit, alpha, shift);
+}
+
+// silu(gate) up, in the 256-row tile with silu_mul's exponential
+std::vector<torch::Tensor> moe_silu_glu(torch::Tensor h, torch::Tensor sel, torch::Tensor w_gu,
+                                        torch::Tensor w_dn) {
+  return experts<GLU_ACT>(h, sel, w_gu, w_dn, INFINITY, 1.0, 0.0, true);
 }
 
 // x [T, K] @ w^T, with ``silu`` silu(gate) * up of the products with w's halves

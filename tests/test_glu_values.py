@@ -29,15 +29,17 @@ def _activations(x, w, kernel, limit, alpha, shift, down=None):
     down = down.bfloat16().cuda()
     sel = torch.zeros(x.shape[0], 1, dtype=torch.int32, device="cuda")
     from aurora_amd import _hip_ops
-    y, place = _hip_ops.moe_clamped_glu(x, sel, w[None].contiguous(), down[None].contiguous(),
-                                        limit, alpha, shift)
+    w, down = w[None].contiguous(), down[None].contiguous()
+    y, place = _hip_ops.moe_silu_glu(x, sel, w, down) if kernel == "silu experts" else \
+        _hip_ops.moe_clamped_glu(x, sel, w, down, limit, alpha, shift)
     return y[place[:, 0].long(), :F]
 
 
 #: rows, outputs, width: the tiles of 32, 64, 128 and 256 rows of the experts' kernel, the
 #: kernel of any size, prompts
 SIZES = [("experts", 40, 192, 192), ("experts", 90, 192, 192), ("experts", 200, 192, 192),
-         ("experts", 2100, 1536, 3072), ("experts", 40, 72, 72), ("prompt", 300, 320, 64)]
+         ("experts", 2100, 1536, 3072), ("experts", 40, 72, 72), ("prompt", 300, 320, 64),
+         ("silu experts", 40, 192, 192), ("silu experts", 2100, 1536, 3072)]
 
 
 @pytest.mark.parametrize("kernel,T,F,W", SIZES)
@@ -45,17 +47,17 @@ SIZES = [("experts", 40, 192, 192), ("experts", 90, 192, 192), ("experts", 200, 
 def test_rounded_once(kernel, T, F, W, limit, alpha, shift):
     """Results are bf16 roundings of fp32 numbers that a handful of correctly rounded
     operations keep within 2^-21 of the exact value. Where the gate is scaled first, by
-    alpha or by log2 e for prompts (as in silu_mul), the exponential multiplies that
+    alpha or by log2 e where silu_mul stood before, the exponential multiplies that
     product's and the factor's rounding, 2^-24 each, by its argument."""
-    if kernel == "prompt" and limit < INF:
-        pytest.skip("prompts have no limit")
+    if kernel in ("prompt", "silu experts") and limit < INF:
+        pytest.skip("of experts with a limit")
     x, w = _products(T, F, W, (-85.0 / alpha, 20.0), (-9.0, 9.0))
     got = _activations(x, w, kernel, limit, alpha, shift)
     y = x.double() @ w.double().t()
     g, u = y[:, :F].clamp(max=limit), y[:, F:].clamp(-limit, limit) + shift
     z = torch.tensor(alpha, dtype=torch.float32).double().item() * g  # as the kernel has it
     want = g * torch.sigmoid(z) * u
-    scaled = 2 if kernel == "prompt" else alpha != 1
+    scaled = 2 if kernel in ("prompt", "silu experts") else alpha != 1
     slack = 2.0 ** -21 + scaled * z.abs() * 2.0 ** -24
     lo, hi = ((want * (1 + s * slack)).float().bfloat16() for s in (-1, 1))
     assert ((got == lo) | (got == hi)).all()
@@ -66,8 +68,8 @@ def test_rounded_once(kernel, T, F, W, limit, alpha, shift):
 def test_special_values(kernel, T, F, W, limit):
     """NaN stays NaN with and without a limit, a closed gate gives 0 beside any finite
     number, infinities act as in the formula."""
-    if kernel in ("prompt", "few") and limit < INF:
-        pytest.skip("prompts have no limit")
+    if kernel in ("prompt", "few", "silu experts") and limit < INF:
+        pytest.skip("of experts with a limit")
     x, w = torch.zeros(T, W).bfloat16().cuda(), torch.zeros(2 * F, W).bfloat16().cuda()
     x[:, :2] = 1
     nan = float("nan")
