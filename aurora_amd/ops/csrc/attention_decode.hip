@@ -18,9 +18,9 @@
 // Measured in a graph, before and now (vector dot products, 64 keys at a time, as many
 // stretches for every sequence): 96 sequences of 500 to 2900 keys, 32 heads over 8,
 // 128 wide, 210 and 136 us (4.9 TB/s; a large read reaches 5.5 to 5.8), the same in fp8 211
-// and 90; 256 of 1600 326 and 289 (5.8 TB/s); 32 of 600 to 2500 66 and 43; one of 12000 102
+// and 91; 256 of 1600 326 and 289 (5.8 TB/s); 32 of 600 to 2500 66 and 43; one of 12000 102
 // and 26, one of 777 20 and 13; 7 heads over one, 40 of 300 to 3000, 90 and 37; fp8 64 wide,
-// 23 of 300 to 5000, 44 and 24. fp8 is bound by widening its values; a single sequence by
+// 23 of 300 to 5000, 44 and 25. fp8 is bound by widening its values; a single sequence by
 // the two launches and one round trip to memory.
 //
 // Replaces the per-token provider round-trip of the reference agent loop

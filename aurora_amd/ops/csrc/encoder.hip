@@ -19,7 +19,7 @@
 // the sum of three bf16 numbers (``split3``) and meets the values three times.
 // Bound by memory and by the start of its many short sequences: 200 texts of 20 to 256
 // tokens, 12 heads of 64 (170 MB) 676 us as a wave per row and head over scalar dot
-// products, now 69 us.
+// products, now 70 us.
 template <int D>
 __global__ __launch_bounds__(256, 2) void packed_attn_kernel(
     const __hip_bfloat16* __restrict__ q,  // rows of Hq heads, D apart

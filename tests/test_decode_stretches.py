@@ -42,7 +42,7 @@ def _reference(q, k, v, bt, ctx, scale):
 
 def _check(got, want):
     """Results are those in 64 bits, rounded to bf16: scores of fp32 sums of D products of
-    bf16 numbers and weights of 16 bits or more add less than 2^-12 to the errors of that
+    bf16 numbers and weights of 32 bits add less than 2^-12 to the errors of that
     rounding, which moves some of them to the other neighbour: twice that."""
     def errors(x):
         return (x.double() - want).norm(dim=-1) / want.norm(dim=-1)

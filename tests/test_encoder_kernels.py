@@ -33,7 +33,7 @@ def test_attention_edges(D, H, G, causal, scale):
                               float("-inf"))
         want = (torch.softmax(w, -1) @ vv).transpose(0, 1)
         err = (got[a:b] - want).norm(dim=-1) / want.norm(dim=-1)
-        # weights are good to 2^-16, results are rounded once to 2^-9 of themselves
+        # weights are good to 2^-22, results are rounded once to 2^-9 of themselves
         assert err.max() < 2 ** -8, (b - a, float(err.max()))
 
 
