@@ -205,7 +205,8 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
   };
   auto source = [&](int t0, int key, long first_row) -> long {
     t0 = tile_at(t0);
-    if constexpr (!PAGED) return row_of(t0 + key);
+    // (the table need not name pages behind a window)
+    if constexpr (!PAGED) return row_of(BIAS ? max(t0 + key, t_lo) : t0 + key);
     return first_row + (t0 + DEC_KEYS <= t_hi ? key : min(key, t_hi - 1 - t0));
   };
   auto load_keys = [&](int t0, long first_row, auto PARITY) {

@@ -106,6 +106,26 @@ def test_decoding_behind_a_window(L, window):
     _check(*_decode(L, 64, 64, bias=True, window=window, spoil=spoil))
 
 
+@pytest.mark.parametrize("P", [16, 48, 64])
+@pytest.mark.parametrize("L,window", [(100, 1), (200, 70), (203, 120)])
+def test_decoding_without_the_pages_behind_a_window(P, L, window):
+    """The block table need not name pages that nobody sees."""
+    g = torch.Generator().manual_seed(L)
+    n = -(-L // P)
+    kc, vc = (torch.randn(n, 2, P, 64, generator=g).bfloat16().cuda() for _ in range(2))
+    q = torch.randn(1, 4, 64, generator=g).bfloat16().cuda()
+    ctx = torch.tensor([L], dtype=torch.int32, device="cuda")
+    results = []
+    for hidden in (0, -1):
+        bt = torch.arange(n, dtype=torch.int32, device="cuda")[None].clone()
+        bt[:, :(L - window) // P] = hidden
+        seg = Segment(rows=slice(0, 1), block_tables=bt, context_lens=ctx, starts=ctx - 1,
+                      state_slots=None)
+        results.append(torch.empty(1, 256, dtype=torch.bfloat16, device="cuda"))
+        biased_attention(q, kc, vc, seg, 0.125, window, None, results[-1], 0, 64, 1.0)
+    assert torch.equal(*results) and results[0].isfinite().all()
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
 def test_packed_rows_keep_32_bits(D, causal):
