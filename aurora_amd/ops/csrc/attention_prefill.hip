@@ -430,22 +430,25 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
       lookup(tile + 3);
     }
   };
-  lookup(tile0);
-  if constexpr (FP8) {
-    fetch8(tile0);
-    store8(tile0);
-    lookup(tile0 + 1);
-    __syncthreads();
-  } else {
-    issue(tile0);
-    lookup(tile0 + 1);
-    if (tile0 + 1 < ntiles) {
-      issue(tile0 + 1);
-      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LK + LV) : "memory");
+  // (a context shorter than its rows can leave a block without a key)
+  if (tile0 < ntiles) {
+    lookup(tile0);
+    if constexpr (FP8) {
+      fetch8(tile0);
+      store8(tile0);
+      lookup(tile0 + 1);
+      __syncthreads();
     } else {
-      asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      issue(tile0);
+      lookup(tile0 + 1);
+      if (tile0 + 1 < ntiles) {
+        issue(tile0 + 1);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LK + LV) : "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      }
+      lookup(tile0 + 2);
     }
-    lookup(tile0 + 2);
   }
   int tile = tile0;
   for (; tile < first; ++tile) {

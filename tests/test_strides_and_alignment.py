@@ -79,6 +79,21 @@ def test_prompts_over_a_cache_at_an_odd_address(P, cache, elements):
     assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("cache", [torch.bfloat16, torch.float8_e4m3fn])
+@pytest.mark.parametrize("P", [16, 64])
+def test_prompts_beside_rows_without_keys(P, cache):
+    """Rows whose context says that there are none read nothing and disturb nobody."""
+    g = torch.Generator().manual_seed(P)
+    n = -(-40 // P)
+    k, v = (torch.randn(n, 1, P, 64, generator=g).to(cache).cuda() for _ in range(2))
+    q = torch.randn(80, 4, 64, generator=g).bfloat16().cuda()
+    bt = torch.arange(n, dtype=torch.int32, device="cuda").expand(2, n).contiguous()
+    i32 = lambda *x: torch.tensor(x, dtype=torch.int32, device="cuda")  # noqa: E731
+    got = ops.attention_prefill_paged(q, k, v, bt, i32(0, 40, 80), i32(40, 0), 0.125)
+    want = ops.attention_prefill_paged(q[:40], k, v, bt[:1], i32(0, 40), i32(40), 0.125)
+    assert torch.equal(got[:40], want)
+
+
 def test_experts_of_rows_at_an_odd_address():
     from aurora_amd.models.config import get_spec
     from aurora_amd.models.llama import MoEMLP
