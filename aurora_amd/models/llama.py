@@ -2,7 +2,7 @@
 built on the aurora_amd op set.
 
 Every hot op routes through aurora_amd.ops (HIP/CDNA4 kernels on GPU, fp32
-torch reference on CPU); plain projections stay on hipBLASLt via F.linear.
+torch reference on CPU), plain projections through ops.linear.
 The forward is engine-shaped: packed varlen tokens + paged KV metadata, no
 [B, S] padding anywhere.
 

@@ -224,7 +224,9 @@ std::vector<torch::Tensor> moe_route_grouped(torch::Tensor h, torch::Tensor rout
 // --------------------------------------------------------------------- sort
 
 // place[a]: sorted row of choice a; token[row]: its token; table: (expert, first
-// row, rows) of every row tile, then expert -1
+// row, rows) of every row tile, then expert -1; behind ``tiles`` of them their number.
+// Tiles of 256 rows share an expert's rows evenly, 32 at a time: their kernel multiplies no
+// more of those than there are.
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
     const int* __restrict__ sel, int A, int E, int top, int TM, int tiles,
     int* __restrict__ place, int* __restrict__ token, int* __restrict__ table) {
@@ -250,14 +252,18 @@ __global__ __launch_bounds__(1024) void moe_sort_kernel(
       nt += __shfl(sk, WAVE - 1, WAVE);
     }
     for (int t = nt + tid; t < tiles; t += WAVE) table[t * 3] = -1;
+    if (tid == 0) table[tiles * 3] = nt;
   }
   __syncthreads();
   for (int e = tid; e < E; e += 1024) {
-    for (int k = 0, r = 0; r < count[e]; ++k, r += TM) {
+    const int c = count[e], n = (c + TM - 1) / TM, parts = (c + 31) / 32;
+    for (int k = 0; k < n; ++k) {
+      const int r = TM == 256 ? k * parts / n * 32 : k * TM;
+      const int end = TM == 256 ? (k + 1) * parts / n * 32 : r + TM;
       int* t = table + (tbase[e] + k) * 3;
       t[0] = e;
       t[1] = base[e] + r;
-      t[2] = min(TM, count[e] - r);
+      t[2] = min(end, c) - r;
     }
   }
   __syncthreads();
@@ -278,11 +284,12 @@ struct GroupArgs {
   const int* gather;   // null: x itself is sorted
   const void* w;       // [E, N, K]; GLU: [E, 2N, K], gate rows then up rows
   void* y;             // [A, N]
-  const int* table;    // null: one expert for all ``rows``
+  const int* table;    // of moe_sort_kernel; null: one expert for all ``rows``
   int N, K;
   float limit, alpha, shift;
-  int rows = 0;
+  int rows = 0;        // of x
   bool silu = false;   // no limit, alpha 1 and shift 0, with silu_mul's exponential
+  int ldx = 0;         // from row to row of x where that is not K (256-row tile only)
 };
 
 // x / d for d >= 1, once corrected: what replaces a division in the 256-row tile, whose
@@ -375,9 +382,13 @@ __global__ __launch_bounds__(256) void grouped_any_kernel(GroupArgs p) {
 template <int TM, int TB, int NS, int NTHR, int ACT>
 __global__ __launch_bounds__(NTHR) void grouped_bf16_kernel(GroupArgs p) {
   constexpr bool GLU = ACT == GLU_ACT;
-  const int* tb = p.table + blockIdx.y * 3;
-  const int e = tb[0];
-  if (e < 0) return;
+  int e = 0, row0 = blockIdx.y * TM, cnt = min(TM, p.rows - row0);
+  if (p.table) {
+    const int* tb = p.table + blockIdx.y * 3;
+    e = tb[0];
+    if (e < 0) return;
+    row0 = tb[1], cnt = tb[2];
+  }
   constexpr int MW = TM >= 64 ? 2 : 1;        // waves along rows
   constexpr int NW = NTHR / 64 / MW;          // waves along columns
   constexpr int WM = TM / MW, WN = TB / NW;   // a wave's tile
@@ -385,7 +396,6 @@ __global__ __launch_bounds__(NTHR) void grouped_bf16_kernel(GroupArgs p) {
   constexpr int LA = TM * 8 / NTHR, LB = TB * 8 / NTHR;  // loads per thread
   constexpr int STAGE = (TM + TB) * GK * 2;
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int row0 = tb[1], cnt = tb[2];
   const int tid = threadIdx.x, lane = tid % WAVE, wave = tid / WAVE;
   const int i = lane & 15, g = lane >> 4;
   constexpr int BN = GLU ? TB / 2 : TB;
@@ -491,170 +501,257 @@ __global__ __launch_bounds__(NTHR) void grouped_bf16_kernel(GroupArgs p) {
     }
 }
 
-// The same for well filled experts: 256 rows x 256 weight rows, eight waves of 128 x 64, two
-// stages of 64 of K. While the products of 32 of K run, the fragments of the next 32 are
-// read between them; a stage is requested as soon as all have read its predecessor but one,
-// a stage's products ahead, and costs one barrier. Rows of a stage are whole cache lines
-// (half lines halve what the L2 delivers, 72 and 136 GB/s a CU). A fifth slot of the ring
-// lets w, which comes from further away than x, be asked for two stages ahead; requests go
-// out between the first products of a half, where they cost the least.
-// Two products of 8 experts of 4096 x 14336 for 8000 tokens, two experts each: 5.66 ms (996
-// TFLOP/s, one stage ahead and no reads or requests between products) and now 4.48 ms
-// (1260); 64 of 2048 x 1408, 16000 tokens, 1.98 and 1.61 ms. Matrix cores are busy two
-// thirds of the time at the 1.85 GHz this load leaves; the rest is waiting for the slowest
-// of a stage's lines.
+// The same for well filled experts and for products of many rows: up to 256 rows x 256 weight
+// rows, eight waves of half the rows and 64 columns each, two stages of 64 of K. While the
+// products of 32 of K run, the fragments of the next 32 are read between them; a stage is
+// requested as soon as all have read its predecessor but one, a stage's products ahead, and
+// costs one barrier. Rows of a stage are whole cache lines (half lines halve what the L2
+// delivers, 72 and 136 GB/s a CU). A fifth slot of the ring lets w, which comes from further
+// away than x, be asked for two stages ahead; requests go out between the first products of
+// a half, where they cost the least.
+// The bound is power: the matrix cores are busy nine tenths of a stage, at the 1.7 GHz that
+// this load leaves (8192^3 1.52 PFLOP/s, the stages alone 1.60; products of 32 x 32 leave 1.55
+// GHz). What is left are the ends of tiles, and rows that are not there. So a workgroup stays
+// on its CU and takes a tile of every round, with the next tile's first two stages on their
+// way while it finishes one; outputs leave as whole lines and past the caches (4096 x 28672 x
+// 1024: 250 us, with 32-byte pieces from a new workgroup for each tile, and now 198; 27700 x
+// 2304 x 768: 123 and 85); and a tile has as many rows as its table says, 32 of them a step,
+// of which a wave multiplies half (6176 x 4096 x 14336: 575 and 531).
 template <int ACT>
 __global__ __launch_bounds__(512) void grouped_large_kernel(GroupArgs p, int tiles, int cols) {
+#ifdef __HIP_DEVICE_COMPILE__  // (the host pass does not know a buffer's descriptor)
   constexpr bool GLU = ACT == GLU_ACT || ACT == SILU_ACT;
   constexpr int BN = GLU ? 128 : 256, SLOT = 256 * GK * 2, RING = 5 * SLOT, L = 4;
-  // Bands of eight row tiles, down and then across; an XCD takes a contiguous eighth of
-  // each, so that its blocks share rows and columns in its L2.
-  const int band = blockIdx.x / 8 / cols, at = blockIdx.x % 8 * cols + blockIdx.x / 8 % cols;
-  const int rt = band * 8 + at % 8, ct = at / 8;
-  if (rt >= tiles) return;
-  int e = 0, row0 = rt * 256, cnt = min(256, p.rows - row0);
-  if (p.table) {
-    e = p.table[rt * 3];
-    row0 = p.table[rt * 3 + 1];
-    cnt = p.table[rt * 3 + 2];
-    if (e < 0) return;
-  }
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int n0 = ct * BN, K = p.K;
-  const int tid = threadIdx.x, lane = tid % WAVE;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  const int i = lane & 15, g = lane >> 4;
-  const bf16_t* w = (const bf16_t*)p.w + (long)e * (GLU ? 2 : 1) * p.N * K;
+  const int K = p.K, steps = K / GK;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
+  const int wr = wave / 4 * 16, wn = wave % 4 * 64;  // rows 32 m + wr + 0..15, columns
 
-  // source of each 16-byte unit this thread fills: rows of x, then of w
-  const bf16_t *xs[L], *ws[L];
+  // The tile that is multiplied and the next. A round's tiles lie in bands of up to eight row
+  // tiles, down and then across; an XCD takes neighbours, which share rows and columns in
+  // its L2.
+  const int nt = p.table ? __builtin_amdgcn_readfirstlane(p.table[tiles * 3]) : tiles;
+  const int bands = (nt + 7) / 8, high = bands ? (nt + bands - 1) / bands : 1;
+  int e = 0, row0 = 0, cnt = 0, n0 = 0, row_now = 0, cnt_now = 0, n_now = 0;
+  auto locate = [&](int round) {  // false: there is none
+    const long left = (long)nt * cols - round * 256L;
+    const int share = (int)(min(left, 256L) + 7) / 8, at = blockIdx.x / 8;
+    if (left <= 0 || at >= share || (int)(blockIdx.x % 8) * share + at >= left) return false;
+    const unsigned v = round * 256 + blockIdx.x % 8 * share + at, band = v / (high * cols);
+    const unsigned in = v - band * high * cols, h = min(high, nt - (int)band * high);
+    const int rt = band * high + in % h;
+    n0 = in / h * BN;
+    if (p.table) {
+      e = p.table[rt * 3];
+      row0 = p.table[rt * 3 + 1];
+      cnt = p.table[rt * 3 + 2];
+    } else {
+      const long parts = (p.rows + 31) / 32;
+      row0 = (int)(rt * parts / nt) * 32;
+      cnt = min((int)((rt + 1) * parts / nt) * 32, p.rows) - row0;
+    }
+    return true;
+  };
+  if (!locate(0)) return;
+
+  const unsigned wbytes = (unsigned)((GLU ? 2 : 1) * p.N) * (unsigned)(K * 2);
+  auto weights = [&] {
+    return __builtin_amdgcn_make_buffer_rsrc((char*)p.w + e * (long)wbytes, 0, wbytes, 0x00027000);
+  };
+  const unsigned xrow = (p.ldx ? p.ldx : K) * 2;
+  const auto xres = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)p.x, 0, (unsigned)(p.rows - 1) * xrow + (unsigned)(K * 2), 0x00027000);
+  auto wres = weights();
+  // offsets of the 16-byte units this thread fills: rows of x, then of w
+  unsigned xo[L], wo[L];
+  auto aim = [&] {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));  // nothing of this is kept through the products
+    const int unit = (tid & 7) ^ (tid >> 3 & 7);
 #pragma unroll
-  for (int l = 0; l < L; ++l) {
-    const int r = (tid + l * 512) >> 3, unit = (tid & 7) ^ (r & 7);
-    const int row = row0 + min(r, cnt - 1);
-    xs[l] = (const bf16_t*)p.x + (long)(p.gather ? p.gather[row] : row) * K + unit * 8;
-    long wr;
-    if constexpr (GLU)  // of a wave's 64 columns half are gate's, half up's
-      wr = min(n0 + r / 64 * 32 + r % 32, p.N - 1) + (long)(r % 64 / 32) * p.N;
-    else
-      wr = min(n0 + r, p.N - 1);
-    ws[l] = w + wr * K + unit * 8;
-  }
+    for (int l = 0; l < L; ++l) {
+      const int r = (tid >> 3) + l * 64, row = row0 + min(r, cnt - 1);
+      xo[l] = (unsigned)(p.gather ? p.gather[row] : row) * xrow + unit * 16;
+      int wrow;
+      if constexpr (GLU)  // of a wave's 64 columns half are gate's, half up's
+        wrow = min(n0 + l * 32 + (r & 31), p.N - 1) + (r >> 5 & 1) * p.N;
+      else
+        wrow = min(n0 + r, p.N - 1);
+      wo[l] = (unsigned)wrow * (unsigned)(K * 2) + unit * 16;
+    }
+    wres = weights();
+  };
+  aim();
   // the ring's slots take w's and x's blocks of 64 of K in turn
   int to = 0;
-  auto request = [&](const bf16_t* const (&from)[L], int stage, int l) {
-    __builtin_amdgcn_global_load_lds((gptr_t)(from[l] + (long)stage * GK),
-                                     (lptr_t)(lds + to + (l * 512 + wave * WAVE) * 16), 16, 0, 0);
+  auto request_w = [&](int stage, int l) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        wres, (lptr_t)(lds + to + (l * 512 + wave * WAVE) * 16), 16, wo[l], stage * (GK * 2), 0, 0);
+  };
+  auto request_x = [&](int stage, int l) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        xres, (lptr_t)(lds + to + (l * 512 + wave * WAVE) * 16), 16, xo[l], stage * (GK * 2), 0, 0);
   };
   auto advance = [&] { to = to == RING - SLOT ? 0 : to + SLOT; };
-  const int wm = wave / 4 * 128, wn = wave % 4 * 64;
-  const int unit = (g ^ (i & 7)) * 16;  // of the first 32 of K; of the second ^ 64
-  const int xa = (wm + i) * 128, wb = (wn + i) * 128;
-  frag_u a[2][8], b[2][4];
-  floatx4 acc[8][4];
-#pragma unroll
-  for (int m = 0; m < 8; ++m)
-#pragma unroll
-    for (int n = 0; n < 4; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
-  auto read = [&](int at, auto HALF, int x) {  // of w's block at ``at`` and x's behind it
-    constexpr int h = decltype(HALF)::value;
-    const char* st = lds + (unit ^ h * 64);
-    const int behind = at == RING - SLOT ? 0 : at + SLOT;
-    if (x < 4) b[h][x].s = *reinterpret_cast<const shortx8*>(st + at + wb + x * 2048);
-    else a[h][x - 4].s = *reinterpret_cast<const shortx8*>(st + behind + xa + (x - 4) * 2048);
-  };
-  auto multiply = [&](auto HALF) {
-    constexpr int h = decltype(HALF)::value;
-#pragma unroll
-    for (int m = 0; m < 8; ++m)
-#pragma unroll
-      for (int n = 0; n < 4; ++n)
-        acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[h][n].v, a[h][m].v, acc[m][n],
-                                                            0, 0, 0);
-  };
-  // The products of a half; between them the next half's fragments and, with ``from``, a
-  // block's requests, in this order.
-  auto half = [&](auto HALF, int at, const bf16_t* const (*from)[L], int stage) {
-    constexpr int h = decltype(HALF)::value;
-    if (from)
-#pragma unroll
-      for (int l = 0; l < L; ++l) request(*from, stage, l);
-#pragma unroll
-    for (int x = 0; x < 12; ++x) read(at, std::integral_constant<int, 1 - h>{}, x);
-    if (from) advance();
-    multiply(HALF);
-    if (from)
-#pragma unroll
-      for (int l = 0; l < L; ++l) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);  // products
-        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);  // a request
-      }
-#pragma unroll
-    for (int x = 0; x < 12; ++x) {
-      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a read
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  };
-  using FIRST = std::integral_constant<int, 0>;
-  using SECOND = std::integral_constant<int, 1>;
-  const int steps = K / GK;
-#pragma unroll
-  for (int x = 0; x < 4; ++x)
-    if (x / 2 < steps) {
-#pragma unroll
-      for (int l = 0; l < L; ++l) request(x % 2 ? xs : ws, x / 2, l);
-      advance();
-    }
-  if (steps > 1) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * L) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
   int at_w = 0;  // slot of w's block of this stage
   auto next = [&] { at_w = at_w >= 3 * SLOT ? at_w - 3 * SLOT : at_w + 2 * SLOT; };
 #pragma unroll
-  for (int x = 0; x < 12; ++x) read(0, FIRST{}, x);
-  __builtin_amdgcn_sched_barrier(0);
-  int s = 0;
-  for (; s + 2 < steps; ++s) {
-    half(FIRST{}, at_w, &ws, s + 2);
-    // the next stage has landed and all have read this one
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(L) : "memory");
-    next();
-    half(SECOND{}, at_w, &xs, s + 2);
+  for (int x = 0; x < 4; ++x) {
+#pragma unroll
+    for (int l = 0; l < L; ++l)
+      if (x % 2) request_x(x / 2, l);
+      else request_w(x / 2, l);
+    advance();
   }
-  for (; s < steps; ++s) {
-    half(FIRST{}, at_w, nullptr, 0);
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    next();
-    half(SECOND{}, at_w, nullptr, 0);  // reads past the end what lies there, for nothing
-  }
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * L) : "memory");
 
-  // a lane has four outputs of a row side by side
-  bf16_t* y = (bf16_t*)p.y;
-  constexpr int NO = GLU ? 2 : 4;
+  using FIRST = std::integral_constant<int, 0>;
+  using SECOND = std::integral_constant<int, 1>;
+  // a tile of up to 32 MI rows, whose first stage has landed
+  auto tile = [&](auto MI_, bool more) {
+    constexpr int MI = decltype(MI_)::value;
+    int lane = threadIdx.x % WAVE;
+    asm volatile("" : "+v"(lane));  // the same
+    const int i = lane & 15, g = lane >> 4;
+    const int unit = (g ^ (i & 7)) * 16;  // of the first 32 of K; of the second ^ 64
+    const int xa = (wr + i) * 128, wb = (wn + i) * 128;
+    frag_u a[2][MI], b[2][4];
+    auto read_b = [&](auto HALF, int n) {
+      constexpr int h = decltype(HALF)::value;
+      b[h][n].s =
+          *reinterpret_cast<const shortx8*>(lds + (unit ^ h * 64) + at_w + wb + n * 2048);
+    };
+    auto read_a = [&](auto HALF, int m) {
+      constexpr int h = decltype(HALF)::value;
+      const int behind = at_w == RING - SLOT ? 0 : at_w + SLOT;
+      a[h][m].s =
+          *reinterpret_cast<const shortx8*>(lds + (unit ^ h * 64) + behind + xa + m * 4096);
+    };
 #pragma unroll
-  for (int m = 0; m < 8; ++m) {
-    const int row = wm + m * 16 + i;
-    if (row >= cnt) continue;
+    for (int n = 0; n < 4; ++n) read_b(FIRST{}, n);
 #pragma unroll
-    for (int n = 0; n < NO; ++n) {
-      const int c = n0 + (GLU ? wn / 2 : wn) + n * 16 + 4 * g;
-      float v[4];
+    for (int m = 0; m < MI; ++m) read_a(FIRST{}, m);
+    floatx4 acc[MI][4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float x = acc[m][n][r], up = acc[m][n + (GLU ? NO : 0)][r];
-        v[r] = ACT == SILU_ACT ? silu_glu(x, up) : GLU ? clamped_glu<true>(x, up, p) : x;
-        if constexpr (ACT == RELU2_ACT) v[r] = v[r] > 0.f ? v[r] * v[r] : 0.f;
+    for (int m = 0; m < MI; ++m)
+#pragma unroll
+      for (int n = 0; n < 4; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // The products of a half; between them ``COUNT`` requests of the block (first w's, then
+    // x's) of ``stage`` and, with AHEAD, the next half's fragments, in this order.
+    auto half = [&](auto HALF, auto COUNT, int stage, auto AHEAD) {
+      constexpr int h = decltype(HALF)::value, count = decltype(COUNT)::value;
+      constexpr int reads = decltype(AHEAD)::value ? 4 + MI : 0;
+      using OTHER = std::integral_constant<int, 1 - h>;
+#pragma unroll
+      for (int l = 0; l < count; ++l)
+        if (h) request_x(stage, l);
+        else request_w(stage, l);
+      advance();
+      if constexpr (reads > 0) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) read_b(OTHER{}, n);
+#pragma unroll
+        for (int m = 0; m < MI; ++m) read_a(OTHER{}, m);
       }
-      bf16_t* dst = y + (long)(row0 + row) * p.N + c;
-      if (c + 4 <= p.N && p.N % 4 == 0)
-        *reinterpret_cast<u64b*>(dst) =
-            (u64b)cvt2_bf16(v[2], v[3]) << 32 | cvt2_bf16(v[0], v[1]);
-      else
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (c + r < p.N) dst[r] = f32_to_bf16(v[r]);
+      for (int m = 0; m < MI; ++m)
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+          acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[h][n].v, a[h][m].v, acc[m][n],
+                                                              0, 0, 0);
+#pragma unroll
+      for (int l = 0; l < count; ++l) {
+        __builtin_amdgcn_sched_group_barrier(0x008, MI > 5 ? 2 : 1, 0);  // products
+        __builtin_amdgcn_sched_group_barrier(0x010, 1, 0);               // a request
+      }
+#pragma unroll
+      for (int x = 0; x < reads; ++x) {
+        if (MI > 3 || x % 2) __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // a read
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // The next stage has landed, which is all that was asked for but the last block of w,
+    // and all have read this one.
+    auto middle = [&] {
+      asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(L) : "memory");
+      next();
+    };
+    using ALL = std::integral_constant<int, L>;
+    using ROWS = std::integral_constant<int, (MI + 1) / 2>;  // requests that hold x's rows
+    for (int s = 2; s < steps; ++s) {
+      half(FIRST{}, ALL{}, s, std::true_type{});
+      middle();
+      half(SECOND{}, ROWS{}, s, std::true_type{});
     }
+    if (more) aim();  // else the same two stages again, for nothing
+    half(FIRST{}, ALL{}, 0, std::true_type{});
+    middle();
+    half(SECOND{}, ALL{}, 0, std::true_type{});
+    half(FIRST{}, ALL{}, 1, std::true_type{});
+    middle();
+    half(SECOND{}, ALL{}, 1, std::false_type{});
+
+    // A lane has four outputs of a row side by side. They become whole lines (GLU: halves of
+    // them) in the ring's free slot, in those parts of it that this wave's own requests fill,
+    // so that nobody waits for another; 16-byte units are xored by row.
+    constexpr int NO = GLU ? 2 : 4, UNITS = NO * 2, ROWS_ = 64 / UNITS;  // of a part of 1 KB
+    constexpr int ONCE = GLU ? 4 : 2;  // m at once
+    char* const part = lds + to + wave * 1024;
+    const int lr = (int)((unsigned)lane / UNITS), lu = (int)((unsigned)lane % UNITS);
+    const int c = n_now + (GLU ? wn / 2 : wn) + lu * 8;
+    bf16_t* const dst = (bf16_t*)p.y + (long)(row_now + wr + lr) * p.N + c;
+#pragma unroll
+    for (int m0 = 0; m0 < MI; m0 += ONCE) {
+#pragma unroll
+      for (int m = m0; m < (m0 + ONCE < MI ? m0 + ONCE : MI); ++m) {
+        const int r = (m - m0) * 16 + i;
+#pragma unroll
+        for (int n = 0; n < NO; ++n) {
+          float v[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float x = acc[m][n][q], up = acc[m][n + (GLU ? NO : 0)][q];
+            v[q] = ACT == SILU_ACT ? silu_glu(x, up) : GLU ? clamped_glu<true>(x, up, p) : x;
+            if constexpr (ACT == RELU2_ACT) v[q] = v[q] > 0.f ? v[q] * v[q] : 0.f;
+          }
+          const int u = (n * 2 + (g >> 1)) ^ (r & (UNITS - 1));
+          *reinterpret_cast<u64b*>(part + r / ROWS_ * 8192 + r % ROWS_ * (UNITS * 16) + u * 16 +
+                                   (g & 1) * 8) =
+              (u64b)cvt2_bf16(v[2], v[3]) << 32 | cvt2_bf16(v[0], v[1]);
+        }
+      }
+      shortx8 v[4];
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+        v[t] = *reinterpret_cast<const shortx8*>(part + t * 8192 + lr * (UNITS * 16) +
+                                                 ((lu ^ lr) & (UNITS - 1)) * 16);
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const int at = (m0 + t * ROWS_ / 16) * 32 + t * ROWS_ % 16;
+        if (at + wr + lr < cnt_now && c < p.N)
+          __builtin_nontemporal_store(v[t], reinterpret_cast<shortx8*>(dst + (long)at * p.N));
+      }
+      asm volatile("" ::: "memory");
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the slot is asked to be filled
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  bool more = true;
+  for (int round = 1; more; ++round) {
+    row_now = row0, cnt_now = cnt, n_now = n0;
+    more = locate(round);
+    const int parts = (cnt_now + 31) / 32;
+    if (parts <= 2) tile(std::integral_constant<int, 2>{}, more);
+    else if (parts <= 4) tile(std::integral_constant<int, 4>{}, more);
+    else if (parts == 5) tile(std::integral_constant<int, 5>{}, more);
+    else if (parts == 6) tile(std::integral_constant<int, 6>{}, more);
+    else if (parts == 7) tile(std::integral_constant<int, 7>{}, more);
+    else tile(std::integral_constant<int, 8>{}, more);
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // requests must not outlive the workgroup
+#endif
 }
 
 template <int ACT>
@@ -664,9 +761,7 @@ static void grouped_large(const GroupArgs& p, int tiles) {
   static const hipError_t once = hipFuncSetAttribute(
       (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
   (void)once;
-  const int cols = (p.N + BN - 1) / BN;
-  hipLaunchKernelGGL(kern, dim3(8 * cols * ((tiles + 7) / 8)), dim3(512), lds,
-                     CUR_STREAM, p, tiles, cols);
+  hipLaunchKernelGGL(kern, dim3(256), dim3(512), lds, CUR_STREAM, p, tiles, (p.N + BN - 1) / BN);
 }
 
 template <int TM, int TB, int NS, int NTHR, int ACT>
@@ -705,6 +800,8 @@ static void grouped(const GroupArgs& p, bool bf16, int tiles, int TM, long busy)
     hipLaunchKernelGGL((grouped_any_kernel<float, ACT>), grid, dim3(256), 0, CUR_STREAM, p);
 }
 
+bool large_takes(long M, long N, long K);
+
 template <int ACT>
 static std::vector<torch::Tensor> experts(const torch::Tensor& h, const torch::Tensor& sel,
                                           const torch::Tensor& w_up, const torch::Tensor& w_dn,
@@ -728,23 +825,25 @@ static std::vector<torch::Tensor> experts(const torch::Tensor& h, const torch::T
   // 2048 x 1408, six each, 1000 tokens 284 and 329, 8000 946 and 1249; 16 of 1024 x 512,
   // two each, 2000 tokens (64 blocks) 51 and 46, 4000 (125) 58 and 71.
   const bool matrix = bf16 && W % GK == 0 && F % GK == 0;
+  const bool large = matrix && large_takes(T_, 2 * F, W) && large_takes(A, W, F);
   const long cols = ACT == GLU_ACT ? 128 : 256;
   const long blocks = std::max(std::min(E, A), A / 256) *
                       std::min((F + cols - 1) / cols, (W + 255) / 256);
   const int TM = !matrix || A < 48 * E          ? 32
-                 : A >= 80 * E && blocks >= 96  ? 256
+                 : A >= 80 * E && blocks >= 96 && large ? 256
                  : A < 160 * E                  ? 64 : 128;
   const int tiles = (int)(A / TM + std::min(E, A));
-  auto token = torch::empty({A}, i32), table = torch::empty({tiles, 3}, i32);
+  auto token = torch::empty({A}, i32), table = torch::empty({tiles + 1, 3}, i32);
   auto act = torch::empty({A, F}, h.options());
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, CUR_STREAM,
                      sel.data_ptr<int>(), (int)A, (int)E, (int)top, TM, tiles,
                      place.data_ptr<int>(), token.data_ptr<int>(), table.data_ptr<int>());
   GroupArgs p = {h.data_ptr(), token.data_ptr<int>(), w_up.data_ptr(), act.data_ptr(),
                  table.data_ptr<int>(), (int)F, (int)W, (float)limit, (float)alpha,
-                 (float)shift, 0, silu};
+                 (float)shift, (int)T_, silu};
   grouped<ACT>(p, bf16, tiles, TM, std::min(E, A));
   p.x = act.data_ptr();
+  p.rows = (int)A;
   p.gather = nullptr;
   p.w = w_dn.data_ptr();
   p.y = y.data_ptr();
@@ -767,21 +866,59 @@ std::vector<torch::Tensor> moe_silu_glu(torch::Tensor h, torch::Tensor sel, torc
   return experts<GLU_ACT>(h, sel, w_gu, w_dn, INFINITY, 1.0, 0.0, true);
 }
 
-// x [T, K] @ w^T, with ``silu`` silu(gate) * up of the products with w's halves
+// Into how many tiles of at most 256 rows a product is cut, evenly: the workgroups, one a
+// CU, take ``cols`` times as many in rounds, a round lasts as its tiles' rows and a constant,
+// and one that does not fill the chip leaves the others a higher clock. (4096 x 28672 x 4096:
+// rounds of 256, 224, 192 and 128 rows 94, 84, 73 and 53 us; 1000 x 4096 x 4096, 64 tiles
+// of 256 rows 70 us, 128 of 128 41.)
+static int row_tiles(long rows, long cols) {
+  const long parts = (rows + 31) / 32, least = (parts + 7) / 8;
+  long best = least;
+  double low = 0;
+  for (long n = least; n <= std::min(parts, least < 8 ? 8 * least : 2 * least); ++n) {
+    const long full = n * cols / 256, rest = n * cols % 256;
+    const double mean = (double)parts / n, most = (double)((parts + n - 1) / n);
+    const double time = full * (mean + 1.25) +
+                        (rest ? (0.75 + 0.25 * rest / 256) * (most + 1.25) : 0);
+    if (n == least || time < low) low = time, best = n;
+  }
+  return (int)best;
+}
+
+// Whether the kernel of 256-row tiles has a form for the product: whole pieces of 16 bytes of
+// an output row, two stages of K, x and w within the 31 bits of their offsets.
+bool large_takes(long M, long N, long K) {
+  return K % GK == 0 && K >= 2 * GK && N % 8 == 0 && M * K < 1l << 30 && N * K < 1l << 30;
+}
+
+// x [T, K], whose rows may be strided, @ w^T, with ``silu`` silu(gate) * up of the products
+// with w's halves
 torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu) {
   TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dtype() == torch::kBFloat16 &&
-                  w.dtype() == torch::kBFloat16 && x.is_contiguous() && w.is_contiguous() &&
+                  w.dtype() == torch::kBFloat16 && w.is_contiguous() &&
                   x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) &&
                   x.size(1) % GK == 0 && x.size(1) > 0 && (!silu || w.size(0) % 2 == 0),
-              "contiguous bf16 on the GPU, K a multiple of ", GK);
+              "bf16 on the GPU, K a multiple of ", GK);
   const long T_ = x.size(0), N = w.size(0) / (silu ? 2 : 1);
   auto y = torch::empty({T_, N}, x.options());
   if (T_ == 0 || N == 0) return y;
+  const bool large = large_takes(T_, w.size(0), x.size(1)) && N % 8 == 0;
+  if (!x.is_contiguous() &&
+      !(large && x.stride(1) == 1 && x.stride(0) % 8 == 0 && x.stride(0) >= x.size(1) &&
+        (uintptr_t)x.data_ptr() % 16 == 0 && T_ * x.stride(0) < 1l << 30))
+    x = x.contiguous();
   GroupArgs p = {x.data_ptr(), nullptr, w.data_ptr(), y.data_ptr(), nullptr, (int)N,
                  (int)x.size(1), INFINITY, 1.f, 0.f, (int)T_};
-  const int tiles = (int)((T_ + 255) / 256);
-  if (silu) grouped_large<SILU_ACT>(p, tiles);
-  else grouped_large<NO_ACT>(p, tiles);
+  if (T_ > 1) p.ldx = (int)x.stride(0);
+  if (large) {
+    const int tiles = row_tiles(T_, silu ? (N + 127) / 128 : (N + 255) / 256);
+    if (silu) grouped_large<SILU_ACT>(p, tiles);
+    else grouped_large<NO_ACT>(p, tiles);
+  } else {
+    const int tiles = (int)((T_ + 127) / 128);
+    if (silu) grouped_bf16<128, 128, 2, 256, GLU_ACT>(p, tiles);
+    else grouped_bf16<128, 128, 2, 256, NO_ACT>(p, tiles);
+  }
   HIP_CHECK_KERNEL();
   return y;
 }

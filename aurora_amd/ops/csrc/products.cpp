@@ -10,6 +10,7 @@
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
+bool large_takes(long M, long N, long K);
 torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target);
 
 enum { WHOLE = 0, PARTS = 1, SILU = 2 };
@@ -71,23 +72,20 @@ static bool silu_few_rows_win(long M, long N, long K) {
 }
 
 // More than 128 rows: where the kernel of 256-row tiles beats the library's product (with
-// silu, product and activation). Library's time over ours, at rows of 256 r, - 57 and - 200.
-// With silu, K up to 1024: everywhere tried from 256 rows on (2048 to 6144 x 768 and 1024, 1.07
-// to 2.1). To 2048: from r = 3 on (4096 to 17920 x 1536 and 2048: mostly 1.1 to 1.6; least
-// 5632, r 11, 0.90, 11264, r 5, 9 and 10, 0.92 to 0.97; r 2 0.75 to 1.2). Longer: where the
-// library falls behind, r 4, 7, 8 and from 11 on (8192 to 37888 x 3584 to 5120 1.0 to 1.5;
-// 57344 x 8192 0.92 to 1.15); elsewhere it is the library's (28672 x 4096, r 2 0.84, 5 0.88, 6
-// 0.92, 9 0.84, 10 0.92; 24576 x 4096, r 5 0.90).
-// Without: only where the tiles fill the chip twice but for a part, where the library takes
-// three rounds (2048 to 8192 outputs, by tiles: K 11008, 350 to 432 0.91 to 1.59, 470 to 512
-// 0.86 to 0.96; K 14336 to 28672, 350 to 480 1.1 to 1.65 but for 8192 at 448, 1.0, 500 to 512
-// 0.86 to 1.0; K 8192, 350 to 512 0.9 to 0.98, 300 0.85).
+// silu, product and activation). Library's time over ours, cold weights, 130 to 27700 rows.
+// With silu: everywhere tried but below 192 rows of long K (K 768 1.5 to 2.6; 1024 1.36 to
+// 1.85; 2048 1.01 to 1.53; 28672 x 4096 from 200 rows on 1.06 to 1.31, 130 and 160 rows 0.93
+// and 0.99; 24576 x 4096 1.01 to 1.30, 0.95 and 0.96; 37888 x 3584 1.06 to 1.55 but for 256
+// rows, 0.81; 57344 x 8192 0.93 to 1.32, the least from 4500 rows on).
+// Without: a CU has one tile at a time and K is not cut, so what counts is whether tiles of
+// 128 rows x 256 columns fill the chip. K up to 1024 everywhere (1.01 to 2.2); to 2048 from
+// 120 tiles on (3072 outputs, 1000 rows 0.99, 6176 1.28; 5632, 640 rows, 110 tiles, 0.93, 769,
+// 154, 1.05, 3500 1.26); longer from 200 on (K 4096 to 28672: 0.94 to 1.97, where the library
+// falls behind by a factor; 100 to 190 tiles 0.7 to 1.07, fewer 0.3 to 0.9).
 static bool many_rows_win(long M, long N, long K, bool silu) {
-  const long rows = (M + 255) / 256, tiles = rows * ((N + 255) / 256);
-  if (!silu) return K >= 11008 && tiles >= 350 && tiles <= (K >= 14336 ? 480 : 432);
-  if (K <= 1024) return M >= 256 && tiles >= 48;
-  if (tiles < 96) return false;
-  return K <= 2048 ? rows >= 3 : rows == 4 || rows == 7 || rows == 8 || rows >= 11;
+  if (silu) return M >= 192 || K <= 2048;
+  const long tiles = (M + 127) / 128 * ((N + 255) / 256);
+  return K <= 1024 || tiles >= (K <= 2048 ? 120 : 200);
 }
 
 // x @ w^T in ``form``, or nothing: the library's product serves better or is followed by
@@ -109,15 +107,16 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
       if (!silu_few_rows_win(M, N / 2, K)) return {};
       return silu_few_rows(x.contiguous(), w);
     }
-    if (many_rows_win(M, N, K, true)) return many_rows(x.contiguous(), w, true);
+    if (large_takes(M, N, K) && many_rows_win(M, N, K, true))
+      return many_rows(x, w, true);
     return {};
   }
   if (M <= 128) {
     if (form == PARTS && few_rows_win(M, N, K, true))
       return linear_few_rows(x.contiguous(), w, true);
     if (few_rows_win(M, N, K, false)) return linear_few_rows(x.contiguous(), w, false);
-  } else if (many_rows_win(M, N, K, false)) {
-    return many_rows(x.contiguous(), w, false);
+  } else if (large_takes(M, N, K) && many_rows_win(M, N, K, false)) {
+    return many_rows(x, w, false);
   }
   // Cold weights: W streamed once past up to 256 rows, ours and the library's, 192 and 256
   // rows: 6144 x 4096 33 and 34, 38 and 42; 4608 x 3584 30 and 30, 32 and 36. Fewer rows, more

@@ -63,3 +63,21 @@ def test_dense(T, N, K, silu):
         want = torch.nn.functional.silu(want[:, :N]) * want[:, N:]
     # rounded by up to 2^-8 of itself; fp32 sums of K terms stay below 2^-16 of the largest
     assert ((got - want).abs() <= 2 ** -8 * want.abs() + 2 ** -16 * want.abs().max()).all()
+
+
+#: rows at the edges of 32 and of the tiles that a product is cut into; K of two and three stages
+@pytest.mark.parametrize("T", [31, 33, 64, 65, 128, 160, 161, 192, 224, 225, 513, 1057, 5000])
+@pytest.mark.parametrize("N,K", [(264, 128), (1032, 192), (2048, 512)])
+@pytest.mark.parametrize("silu", [False, True])
+def test_rows_of_a_tile(T, N, K, silu):
+    """Tiles of every height, strided rows of x, and nothing written past the last row."""
+    g = torch.Generator(device="cuda").manual_seed(T + N)
+    x = torch.randn(T, K + 136, generator=g, device="cuda").bfloat16()[:, 64:64 + K]
+    w = (torch.randn(N * (1 + silu), K, generator=g, device="cuda") * K ** -0.5).bfloat16()
+    got = _hip("many_rows").many_rows(x, w, silu)
+    assert got.equal(_hip("many_rows").many_rows(x.contiguous(), w, silu))
+    want = x.double() @ w.double().t()
+    if silu:
+        want = torch.nn.functional.silu(want[:, :N]) * want[:, N:]
+    # rounded by up to 2^-8 of itself; fp32 sums of K terms stay below 2^-16 of the largest
+    assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -16 * want.abs().max()).all()
