@@ -21,6 +21,13 @@ from ..parallel.tp import is_plain
 from .config import ModelSpec, get_spec
 
 
+def _product(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """``m(x)``, through the framework's products where nobody watches or replaced ``m``."""
+    if is_plain(m, nn.Linear) and m.bias is None:
+        return ops.linear(x, m.weight)
+    return m(x)
+
+
 class EncoderLayer(nn.Module):
     def __init__(self, spec: ModelSpec, dtype):
         super().__init__()
@@ -50,16 +57,19 @@ class EncoderLayer(nn.Module):
             h = ops.rmsnorm(x, self.norm1, self.eps)
         else:
             h, x = ops.rmsnorm_residual(delta, x, self.norm1, self.eps)
-        qkv = self.qkv(h).view(T, 3 * self.n_heads, self.head_dim)
+        qkv = _product(self.qkv, h).view(T, 3 * self.n_heads, self.head_dim)
         q, k, v = qkv.split(self.n_heads, dim=1)
-        ops.rope_apply_(q, k, positions, cos_sin)
+        if is_plain(self.qkv, nn.Linear):
+            ops.rope_apply_(q, k, positions, cos_sin)
+        else:  # what somebody else made may be kept by them
+            q, k = ops.rope_apply(q.clone(), k.clone(), positions, cos_sin)
         o = ops.attention_prefill(q, k, v, cu, self.scale, causal=False)
-        h, x = ops.rmsnorm_residual(self.o(o.reshape(T, -1)), x, self.norm2, self.eps)
+        h, x = ops.rmsnorm_residual(_product(self.o, o.reshape(T, -1)), x, self.norm2, self.eps)
         if is_plain(self.gate_up, nn.Linear) and self.gate_up.bias is None:
             act = ops.linear_silu_mul(h, self.gate_up.weight)
         else:
             act = ops.silu_mul(self.gate_up(h))
-        return x, self.down(act)
+        return x, _product(self.down, act)
 
 
 class SentenceEncoder(nn.Module):

@@ -124,3 +124,21 @@ def test_hooks_of_encoders(name, device):
                 torch.arange(43, dtype=torch.int32, device=device),
                 torch.tensor([0, 43], dtype=torch.int32, device=device))
     assert out.shape == x.shape
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("texts", [[[5]], [[5, 6, 7], [8], list(range(1, 30))]])
+def test_encoders_leave_what_is_not_theirs(device, texts):
+    """What a hook keeps of the joint projection stays as it was, and a tensor that somebody
+    hands back on every pass gives the same embeddings on every pass."""
+    m = SentenceEncoder("tiny-encoder" if device == "cpu" else "bge-base", device=device)
+    m.init_random(1)
+    before, kept = m.encode_ids(texts), []
+    hook = m.layers[0].qkv.register_forward_hook(
+        lambda module, args, out: kept.append((out, out.clone())))
+    _same(m.encode_ids(texts), before)
+    assert torch.equal(*kept[0])
+    hook.remove()
+    m.layers[0].qkv.forward = lambda x, made=kept[0][1]: made
+    for _ in range(3):
+        _same(m.encode_ids(texts), before)
