@@ -29,6 +29,7 @@ from typing import Deque, Dict, List, Optional, Tuple
 
 import torch
 
+from .. import ops
 from ..models.config import AnySpec, get_spec, is_checkpoint_dir
 from ..models.llama import AttnMetadata
 from ..models.registry import build_model
@@ -620,6 +621,10 @@ class LLMEngine:
     def _build_batch(self, prefill: List[Sequence], chunks: List[int],
                      decode: List[Sequence]):
         """(input ids, metadata) of [prefill chunks..., decode tokens...]."""
+        if self.device != "cpu":
+            made = self._pack_batch(prefill, chunks, decode)
+            if made is not None:
+                return made
         ids: List[int] = []
         positions: List[int] = []
         slots: List[int] = []
@@ -665,6 +670,39 @@ class LLMEngine:
         input_ids = torch.tensor(ids, dtype=torch.long, device=self.device)
         return input_ids, AttnMetadata(mode=mode, **fields)
 
+    def _pack_batch(self, prefill: List[Sequence], chunks: List[int], decode: List[Sequence]):
+        """``_build_batch`` in native code, one copy to the device; None where it has to be
+        done in Python."""
+        seqs, n = prefill + decode, len(prefill)
+        end = [s.num_cached + c for s, c in zip(prefill, chunks)]
+        end += [s.num_tokens for s in decode]
+        first = [s.num_cached for s in prefill] + [e - 1 for e in end[n:]]
+        made = ops.pack_batch([s.token_ids for s in seqs], first, end, [s.pages for s in seqs],
+                              [s.state_slot for s in seqs], n, self.kv.page_size, self.device)
+        if made is None:
+            return None
+        rows = iter(made[3:])
+
+        def seq_fields(prefix=""):
+            table, ctx, slots = next(rows), next(rows), next(rows)
+            out = {prefix + "block_tables": table, prefix + "context_lens": ctx}
+            if self.states:
+                out[prefix + "state_slots"] = slots
+            return out
+
+        fields = {"positions": made[1], "slot_mapping": made[2]}
+        if self.states:
+            fields["states"] = self.states.states
+        if prefill:
+            cu = [0, *itertools.accumulate(chunks)]
+            fields.update(seq_fields(), cu_seqlens_q=made[-1], cu_host=cu, ctx_host=end[:n])
+            if decode:
+                fields.update(seq_fields("dec_"), num_prefill_tokens=cu[-1])
+        else:
+            fields.update(seq_fields())
+        mode = "decode" if not prefill else "mixed" if decode else "prefill"
+        return made[0], AttnMetadata(mode=mode, **fields)
+
     # ----------------------------------------------------- hipGraph decode
 
     _BUCKETS = (1, 2, 4, 8, 16, 32, 64, 96, 128, 192, 256)
@@ -704,8 +742,8 @@ class LLMEngine:
         if g is None:
             g = self._capture_decode_graph(bucket)
             self._graph_cache[bucket] = g
-        (graph, in_ids, in_pos, in_slot, in_bt, in_ctx, in_state, out_logits) = g
-        mp = in_bt.shape[1]
+        graph, inputs, host_inputs, staged_parts, out_logits = g
+        mp = staged_parts[2].shape[1]
         P = self.kv.page_size
         ids_t = self._host_i64
         ids_t[:B] = torch.tensor([s.token_ids[-1] for s in seqs],
@@ -749,12 +787,12 @@ class LLMEngine:
             if staged[i] is not None:
                 bt_host[i].fill_(self._scratch_page)
                 staged[i] = None
-        in_ids.copy_(ids_t[:bucket], non_blocking=True)
-        in_pos.copy_(pos[:bucket, 0], non_blocking=True)
-        in_slot.copy_(pos[:bucket, 1], non_blocking=True)
-        in_ctx.copy_(pos[:bucket, 2], non_blocking=True)
-        in_state.copy_(pos[:bucket, 3], non_blocking=True)
-        in_bt.copy_(bt_host[:bucket], non_blocking=True)
+        # one copy: ids, positions, slots, contexts, states, tables side by side
+        host_ids, host_rows, host_bt = staged_parts
+        host_ids.copy_(ids_t[:bucket])
+        host_rows.copy_(pos[:bucket].t())
+        host_bt.copy_(bt_host[:bucket])
+        inputs.copy_(host_inputs, non_blocking=True)
         graph.replay()
         return out_logits[:B]
 
@@ -772,14 +810,20 @@ class LLMEngine:
                                        dtype=torch.int32, pin_memory=True)
             self._bt_staged = [None] * maxb
         self._dec_staged_ids = None
-        in_ids = torch.zeros(bucket, dtype=torch.int64, device=dev)
-        in_pos = torch.zeros(bucket, dtype=torch.int32, device=dev)
-        in_slot = torch.full((bucket,), self._scratch_slot, dtype=torch.int32,
-                             device=dev)
-        in_bt = torch.full((bucket, mp), self._scratch_page, dtype=torch.int32,
-                           device=dev)
-        in_ctx = torch.ones(bucket, dtype=torch.int32, device=dev)
-        in_state = torch.full((bucket,), -1, dtype=torch.int32, device=dev)
+
+        def parts(buffer):  # ids; positions, slots, contexts and states; tables
+            ids, rest = buffer[:bucket], buffer[bucket:].view(torch.int32)
+            return (ids, rest[:4 * bucket].view(4, bucket),
+                    rest[4 * bucket:(4 + mp) * bucket].view(bucket, mp))
+
+        size = bucket + ((4 + mp) * bucket + 1) // 2
+        host_inputs = torch.zeros(size, dtype=torch.int64, pin_memory=True)
+        staged_parts = parts(host_inputs)
+        for row, idle in zip(staged_parts[1], (0, self._scratch_slot, 1, -1)):
+            row.fill_(idle)
+        staged_parts[2].fill_(self._scratch_page)
+        inputs = host_inputs.to(dev)
+        in_ids, (in_pos, in_slot, in_ctx, in_state), in_bt = parts(inputs)
         meta = AttnMetadata(mode="decode", positions=in_pos, slot_mapping=in_slot,
                             block_tables=in_bt, context_lens=in_ctx,
                             states=self.states.states, state_slots=in_state)
@@ -806,7 +850,7 @@ class LLMEngine:
                     out_logits = fwd()
         finally:
             gc.enable()
-        return (graph, in_ids, in_pos, in_slot, in_bt, in_ctx, in_state, out_logits)
+        return graph, inputs, host_inputs, staged_parts, out_logits
 
     # --------------------------------------------------------------- sample
 

@@ -103,16 +103,20 @@ class SentenceEncoder(nn.Module):
         """[N, H] L2-normalized embeddings for N token-id lists."""
         dev = self.embed.weight.device
         maxp = self.spec.max_position
-        batches = [b[:maxp] if b else [0] for b in batches]
-        flat = [t for b in batches for t in b]
-        cu = [0]
-        pos: List[int] = []
-        for b in batches:
-            cu.append(cu[-1] + len(b))
-            pos.extend(range(len(b)))
-        ids = torch.tensor(flat, dtype=torch.long, device=dev)
-        cu_t = torch.tensor(cu, dtype=torch.int32, device=dev)
-        pos_t = torch.tensor(pos, dtype=torch.int32, device=dev)
+        packed = ops.pack_texts(list(batches), maxp, dev) if dev.type == "cuda" else None
+        if packed is not None:
+            ids, cu_t, pos_t = packed
+        else:
+            batches = [b[:maxp] if b else [0] for b in batches]
+            flat = [t for b in batches for t in b]
+            cu = [0]
+            pos: List[int] = []
+            for b in batches:
+                cu.append(cu[-1] + len(b))
+                pos.extend(range(len(b)))
+            ids = torch.tensor(flat, dtype=torch.long, device=dev)
+            cu_t = torch.tensor(cu, dtype=torch.int32, device=dev)
+            pos_t = torch.tensor(pos, dtype=torch.int32, device=dev)
         x = self.embed(ids)
         delta = None
         for layer in self.layers:

@@ -250,6 +250,18 @@ def moe_grouped_gemm(xp: torch.Tensor, w: torch.Tensor, starts: torch.Tensor,
         xp.contiguous(), w, starts, counts)
 
 
+def pack_batch(ids, first, end, pages, states, prompts: int, page: int, device):
+    """A step's ids, positions, cache slots and tables on the GPU, or None where its lists
+    hold anything but plain integers (the extension's header has the order)."""
+    return _require_hip("pack_batch").pack_batch(ids, first, end, pages, states, prompts, page,
+                                                 torch.device(device))
+
+
+def pack_texts(texts, most: int, device):
+    """Ids, begins and positions of texts on the GPU, or None as ``pack_batch``."""
+    return _require_hip("pack_texts").pack_texts(texts, most, torch.device(device))
+
+
 def softmax_sample(logits, temperature, top_p, top_k, generator=None):
     # Sampling is [B, V] with B small; keep it in torch on both devices for now
     # (the GPU cost is one softmax over V — negligible next to the forward).

@@ -164,6 +164,11 @@ void memory_decode(torch::Tensor proj, torch::Tensor i_bias, torch::Tensor f_bia
                    torch::Tensor nstate, torch::Tensor mstate, torch::Tensor starts,
                    torch::Tensor slots, torch::Tensor out, long col, double oscale);
 
+py::object pack_batch(py::list ids, std::vector<long> first, std::vector<long> end,
+                      py::list pages, std::vector<long> states, long prompts, long page,
+                      torch::Device device);
+py::object pack_texts(py::list texts, long most, torch::Device device);
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm", &rmsnorm, "fused RMSNorm (bf16, gfx950)");
   m.def("rmsnorm_residual", &rmsnorm_residual, "fused residual-add + RMSNorm");
@@ -240,6 +245,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "final norm");
   m.def("normed_qkv", &normed_qkv,
         "head norms + rotation + temperature + paged KV scatter");
+  m.def("pack_batch", &pack_batch, "a step's batch from lists, in one copy");
+  m.def("pack_texts", &pack_texts, "texts to embed from lists, in one copy");
   m.def("gelu", &gelu, "exact gelu");
   m.def("relu2", &relu2, "squared relu");
   m.def("silu_glu", &silu_glu, "silu(gate) * up");

@@ -15,8 +15,8 @@ from torch.utils.cpp_extension import BuildExtension, CUDAExtension
 CSRC = "aurora_amd/ops/csrc/"
 EXTENSIONS = {
     # decoder kernels
-    "_hip_ops": ["bindings.cpp", "products.cpp", "elementwise.hip", "attention_decode.hip",
-                 "attention_prefill.hip", "skinny_gemm.hip", "few_rows.hip", "residual_norm.hip",
+    "_hip_ops": ["bindings.cpp", "products.cpp", "batch.cpp", "elementwise.hip",
+                 "attention_decode.hip", "attention_prefill.hip", "skinny_gemm.hip", "few_rows.hip", "residual_norm.hip",
                  "attention_rows.hip", "recurrence.hip", "moe.hip", "sublayer.hip",
                  "latent_attention.hip", "output_norm.hip", "conv_heads.hip"],
     # sentence encoder, vector search, one-shot all-reduce
