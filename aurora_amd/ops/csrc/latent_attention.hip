@@ -673,6 +673,53 @@ torch::Tensor gather_latents(torch::Tensor cache, torch::Tensor rows) {
   return out;
 }
 
+// Where the visible context of every portion lies: the cache rows of its tokens, packed, and
+// the place of sequence s's token t among them, table [s, t] (0 where it is not visible). A
+// workgroup per 256 tokens of a sequence adds up what the sequences before it have. (As
+// library operations 16 launches a step, 0.3 ms in which the GPU waited for the host.)
+__global__ __launch_bounds__(256) void latent_places_kernel(
+    const int* __restrict__ block_tables, const int* __restrict__ cu,
+    const int* __restrict__ ctx, int pages, int page, int window, int longest, int total,
+    int* __restrict__ place, int* __restrict__ table) {
+  const int s = blockIdx.y, t = blockIdx.x * 256 + threadIdx.x;
+  auto first = [&](int q) {
+    return window ? max(0, ctx[q] - (cu[q + 1] - cu[q]) - window + 1) : 0;
+  };
+  int before = 0;
+  for (int q = threadIdx.x; q < s; q += 256) before += ctx[q] - first(q);
+  __shared__ int sums[4];
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) before += __shfl_xor(before, d, WAVE);
+  if (threadIdx.x % WAVE == 0) sums[threadIdx.x / WAVE] = before;
+  __syncthreads();
+  before = sums[0] + sums[1] + sums[2] + sums[3];
+  if (t >= longest) return;
+  const int lo = first(s), at = before + t - lo;
+  const bool seen = t >= lo && t < ctx[s] && at < total;
+  table[(long)s * longest + t] = seen ? at : 0;
+  if (seen) place[at] = block_tables[(long)s * pages + t / page] * page + t % page;
+}
+
+// ``total`` visible tokens, the longest context ``longest`` -> (cache rows, table)
+std::vector<torch::Tensor> latent_places(torch::Tensor block_tables, torch::Tensor cu,
+                                         torch::Tensor ctx, long page, long window, long longest,
+                                         long total) {
+  const long S = ctx.numel();
+  for (auto* t : {&block_tables, &cu, &ctx})
+    TORCH_CHECK(t->is_cuda() && t->dtype() == torch::kInt32 && t->is_contiguous(), "tables");
+  TORCH_CHECK(block_tables.dim() == 2 && block_tables.size(0) == S && cu.numel() == S + 1 &&
+              longest > 0 && longest <= block_tables.size(1) * page && total >= 0 && S < 65536,
+              "contexts lie within their pages");
+  auto place = torch::empty({total}, ctx.options()), table = torch::empty({S, longest}, ctx.options());
+  if (S == 0) return {place, table};
+  hipLaunchKernelGGL(latent_places_kernel, dim3((longest + 255) / 256, S), dim3(256), 0,
+                     CUR_STREAM, block_tables.data_ptr<int>(), cu.data_ptr<int>(),
+                     ctx.data_ptr<int>(), (int)block_tables.size(1), (int)page, (int)window,
+                     (int)longest, (int)total, place.data_ptr<int>(), table.data_ptr<int>());
+  HIP_CHECK_KERNEL();
+  return {place, table};
+}
+
 // ------------------------------------------------------------- rotated dimensions
 
 // neighbouring pairs of x's first ``rot`` dimensions turn into out, zeros follow

@@ -287,15 +287,10 @@ class Segment:
         P = cache.shape[2]
         hit = self._maps.get(("context", window))
         if hit is None:
-            dev = cache.device
-            table = torch.zeros(len(self.ctx_host), max(self.ctx_host), dtype=torch.int32)
-            place, n = [], 0
-            for s, (lo, c) in enumerate(zip(self.first_keys(window), self.ctx_host)):
-                table[s, lo:c] = torch.arange(n, n + c - lo, dtype=torch.int32)
-                n += c - lo
-                t = torch.arange(lo, c, device=dev)
-                place.append(self.block_tables[s].long()[t // P] * P + t % P)
-            hit = (torch.cat(place).to(torch.int32), table.to(dev))
+            lo = self.first_keys(window)
+            hit = tuple(_hip("latent_places").latent_places(
+                self.block_tables, self.cu, self.context_lens, P, window, max(self.ctx_host),
+                sum(self.ctx_host) - sum(lo)))
             self._maps["context", window] = hit
         return _hip("gather_latents").gather_latents(cache, hit[0]), hit[1]
 
@@ -303,6 +298,11 @@ class Segment:
 def _hip(op: str):
     from . import _require_hip
     return _require_hip(op)
+
+
+def _linear(x, weight):
+    from . import linear
+    return linear(x, weight)
 
 
 def residual_rmsnorm(x, weight, eps, delta=None, moe=None, step=None,
@@ -482,8 +482,8 @@ def latent_attention(proj, p: LatentParams, cache, seg: Segment, out, q=None,
               and C - R in (0, KEY_PART))
     if matrix and expand_latents(seg, p, R):
         c, rows = seg.latent_rows(cache, p.window)
-        k = torch.nn.functional.linear(c[:, :R], p.uk.flatten(0, 1)).view(-1, H, 1, p.dim)
-        v = torch.nn.functional.linear(c[:, :R], p.uv.flatten(0, 1)).view(-1, H, 1, p.vdim)
+        k = _linear(c[:, :R], p.uk.flatten(0, 1)).view(-1, H, 1, p.dim)
+        v = _linear(c[:, :R], p.uv.flatten(0, 1)).view(-1, H, 1, p.vdim)
         bseq, boff = seg.block_map(m.biased_prefill_rows(1))
         if p.tail:
             rotate_heads(tail, positions, p.cos_sin, tail)
