@@ -223,50 +223,91 @@ std::vector<torch::Tensor> moe_route_grouped(torch::Tensor h, torch::Tensor rout
 
 // --------------------------------------------------------------------- sort
 
-// place[a]: sorted row of choice a; token[row]: its token; table: (expert, first
-// row, rows) of every row tile, then expert -1; behind ``tiles`` of them their number.
-// Tiles of 256 rows share an expert's rows evenly, 32 at a time: their kernel multiplies no
-// more of those than there are.
+// Rounds of the 256-row tile's workgroups, one a CU: as long as their tiles are high, 32 rows
+// a step, and a constant; one that does not fill the chip leaves the others a higher clock.
+// (4096 x 28672 x 4096: rounds of 256, 224, 192 and 128 rows 94, 84, 73 and 53 us; 1000 x 4096
+// x 4096, 64 tiles of 256 rows 70 us, 128 of 128 41.)
+__host__ __device__ inline float rounds_time(long tiles, float mean, int most) {
+  const long full = tiles / 256, rest = tiles % 256;
+  return full * (mean + 1.25f) + (rest ? (0.75f + 0.25f / 256 * rest) * (most + 1.25f) : 0.f);
+}
+
+// place[a]: sorted row of choice a; token[row]: its token; tables of the row tiles of the up
+// and of the down product: (expert, first row, rows) of every tile, then expert -1; behind
+// ``tiles`` of them their number. Tiles of TM rows; where that is 256 (and the tables are
+// two) of at most 256, 32 at a time, an expert's all alike, and so many that the products'
+// rounds, of ``cols`` tiles a row tile, are short (8 experts of 4096 x 14336, two each, 300
+// tokens 711 and 575 us, 1000 tokens 821 to 816: where rows are many, tiles were many before).
 __global__ __launch_bounds__(1024) void moe_sort_kernel(
-    const int* __restrict__ sel, int A, int E, int top, int TM, int tiles,
-    int* __restrict__ place, int* __restrict__ token, int* __restrict__ table) {
+    const int* __restrict__ sel, int A, int E, int top, int TM, int tiles, int cols_up,
+    int cols_dn, int* __restrict__ place, int* __restrict__ token, int* __restrict__ table) {
   __shared__ int count[MAX_EXPERTS], base[MAX_EXPERTS], tbase[MAX_EXPERTS];
+  __shared__ int s_high[2];
   const int tid = threadIdx.x;
+  const bool even = TM == 256;
   for (int e = tid; e < E; e += 1024) count[e] = 0;
   __syncthreads();
   for (int a = tid; a < A; a += 1024) atomicAdd(&count[sel[a]], 1);
   __syncthreads();
-  if (tid < WAVE) {  // exclusive sums over experts, one wave
-    int rows = 0, nt = 0;
-    for (int e0 = 0; e0 < E; e0 += WAVE) {
-      const int e = e0 + tid;
-      const int c = e < E ? count[e] : 0, k = (c + TM - 1) / TM;
-      int sc = c, sk = k;
-#pragma unroll
-      for (int off = 1; off < WAVE; off <<= 1) {
-        const int a = __shfl_up(sc, off, WAVE), b = __shfl_up(sk, off, WAVE);
-        if (tid >= off) { sc += a; sk += b; }
+  if (even && tid < WAVE) {  // a lane per height
+    const int high = 4 + tid;
+    int parts = 0, nt = 0, most = 0;
+    if (high <= 8)
+      for (int e = 0; e < E; ++e) {
+        const int u = (count[e] + 31) / 32, n = (u + high - 1) / high;
+        parts += u;
+        nt += n;
+        if (n) most = max(most, (u + n - 1) / n);
       }
-      if (e < E) { base[e] = rows + sc - c; tbase[e] = nt + sk - k; }
-      rows += __shfl(sc, WAVE - 1, WAVE);
-      nt += __shfl(sk, WAVE - 1, WAVE);
-    }
-    for (int t = nt + tid; t < tiles; t += WAVE) table[t * 3] = -1;
-    if (tid == 0) table[tiles * 3] = nt;
-  }
-  __syncthreads();
-  for (int e = tid; e < E; e += 1024) {
-    const int c = count[e], n = (c + TM - 1) / TM, parts = (c + 31) / 32;
-    for (int k = 0; k < n; ++k) {
-      const int r = TM == 256 ? k * parts / n * 32 : k * TM;
-      const int end = TM == 256 ? (k + 1) * parts / n * 32 : r + TM;
-      int* t = table + (tbase[e] + k) * 3;
-      t[0] = e;
-      t[1] = base[e] + r;
-      t[2] = min(end, c) - r;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const float time =
+          rounds_time((long)nt * (k ? cols_dn : cols_up), (float)parts / max(nt, 1), most);
+      float low = __shfl(time, 4, WAVE);
+      int best = 8;
+#pragma unroll
+      for (int x = 3; x >= 0; --x) {
+        const float t = __shfl(time, x, WAVE);
+        if (t < low) low = t, best = 4 + x;
+      }
+      if (tid == 0) s_high[k] = best;
     }
   }
   __syncthreads();
+  for (int k = 0; k < (even ? 2 : 1); ++k, table += (tiles + 1) * 3) {
+    const int step = even ? s_high[k] * 32 : TM;
+    if (tid < WAVE) {  // exclusive sums over experts, one wave
+      int rows = 0, nt = 0;
+      for (int e0 = 0; e0 < E; e0 += WAVE) {
+        const int e = e0 + tid;
+        const int c = e < E ? count[e] : 0, n = (c + step - 1) / step;
+        int sc = c, sk = n;
+#pragma unroll
+        for (int off = 1; off < WAVE; off <<= 1) {
+          const int a = __shfl_up(sc, off, WAVE), b = __shfl_up(sk, off, WAVE);
+          if (tid >= off) { sc += a; sk += b; }
+        }
+        if (e < E) { base[e] = rows + sc - c; tbase[e] = nt + sk - n; }
+        rows += __shfl(sc, WAVE - 1, WAVE);
+        nt += __shfl(sk, WAVE - 1, WAVE);
+      }
+      for (int t = nt + tid; t < tiles; t += WAVE) table[t * 3] = -1;
+      if (tid == 0) table[tiles * 3] = nt;
+    }
+    __syncthreads();
+    for (int e = tid; e < E; e += 1024) {
+      const int c = count[e], n = (c + step - 1) / step, parts = (c + 31) / 32;
+      for (int x = 0; x < n; ++x) {
+        const int r = even ? x * parts / n * 32 : x * TM;
+        const int end = even ? (x + 1) * parts / n * 32 : r + TM;
+        int* t = table + (tbase[e] + x) * 3;
+        t[0] = e;
+        t[1] = base[e] + r;
+        t[2] = min(end, c) - r;
+      }
+    }
+    __syncthreads();
+  }
   for (int a = tid; a < A; a += 1024) {
     const int row = atomicAdd(&base[sel[a]], 1);
     place[a] = row;
@@ -818,25 +859,30 @@ static std::vector<torch::Tensor> experts(const torch::Tensor& h, const torch::T
   auto y = torch::empty({A, W}, h.options()), place = torch::empty({T_, top}, i32);
   if (A == 0) return {y, place};
   const bool bf16 = h.dtype() == torch::kBFloat16;
-  // Row tile: enough rows per weight read. 256 from 80 rows an expert on, where there are
-  // blocks for a good part of the chip: the kernel of that tile is the fastest by so much
-  // that even rows of padding pay. 256 and the next best: 8 experts of 4096 x 14336, two
-  // each, 300 tokens (75 rows) 744 and 746 us, 500 767 and 927, 3000 1959 and 2675; 64 of
-  // 2048 x 1408, six each, 1000 tokens 284 and 329, 8000 946 and 1249; 16 of 1024 x 512,
-  // two each, 2000 tokens (64 blocks) 51 and 46, 4000 (125) 58 and 71.
+  // Row tile, us of tiles of 32, 64, 128 and 256 (both products, uneven experts). Below some
+  // 18 rows an expert the weights' stream counts: 8 experts of 4096 x 14336, 16 rows on average
+  // 512 517 615 538, 25 rows 644 515 621 548; 32 of 2048 x 2816, 16 rows 230 216 225 220; but 16
+  // of 1024 x 512, 25 rows 22 24 36 37. From 36 on the 256-row tile, where there are blocks for
+  // a good part of the chip: 8 of 4096 x 14336, 38 rows (160 blocks) 721 618 628 568, 250 rows
+  // 2974 1608 1224 816; 64 of 2048 x 1408, 38 rows (656) 289 240 252 245, 84 rows 503 341 305
+  // 278; 8 of 2048 x 8192, 75 rows (96) 258 204 256 244, 125 rows (120) 408 267 266 249; 16 of
+  // 1024 x 512, 162 rows (144) 51 34 39 41, 250 rows (188) 74 48 44 43. Fewer blocks are 64
+  // rows' (8 of 1024 x 3584, 200 rows (80) 144 87 106 102); 128 is what is left to sizes that
+  // the 256-row tile has no form for.
   const bool matrix = bf16 && W % GK == 0 && F % GK == 0;
   const bool large = matrix && large_takes(T_, 2 * F, W) && large_takes(A, W, F);
+  const bool small = W * F < 1l << 20;
   const long cols = ACT == GLU_ACT ? 128 : 256;
-  const long blocks = std::max(std::min(E, A), A / 256) *
-                      std::min((F + cols - 1) / cols, (W + 255) / 256);
-  const int TM = !matrix || A < 48 * E          ? 32
-                 : A >= 80 * E && blocks >= 96 && large ? 256
-                 : A < 160 * E                  ? 64 : 128;
-  const int tiles = (int)(A / TM + std::min(E, A));
-  auto token = torch::empty({A}, i32), table = torch::empty({tiles + 1, 3}, i32);
+  const long blocks = (A / 128 + E) * std::min((F + cols - 1) / cols, (W + 255) / 256);
+  const int TM = !matrix || A < (small ? 48 : 18) * E                      ? 32
+                 : large && A >= 36 * E && blocks >= (small ? 170 : 112)   ? 256
+                 : large || A < 160 * E                                    ? 64 : 128;
+  const int tiles = (int)(A / (TM == 256 ? 128 : TM) + std::min(E, A));
+  auto token = torch::empty({A}, i32), table = torch::empty({2, tiles + 1, 3}, i32);
   auto act = torch::empty({A, F}, h.options());
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(1024), 0, CUR_STREAM,
                      sel.data_ptr<int>(), (int)A, (int)E, (int)top, TM, tiles,
+                     (int)((F + cols - 1) / cols), (int)((W + 255) / 256),
                      place.data_ptr<int>(), token.data_ptr<int>(), table.data_ptr<int>());
   GroupArgs p = {h.data_ptr(), token.data_ptr<int>(), w_up.data_ptr(), act.data_ptr(),
                  table.data_ptr<int>(), (int)F, (int)W, (float)limit, (float)alpha,
@@ -847,6 +893,7 @@ static std::vector<torch::Tensor> experts(const torch::Tensor& h, const torch::T
   p.gather = nullptr;
   p.w = w_dn.data_ptr();
   p.y = y.data_ptr();
+  if (TM == 256) p.table += (tiles + 1) * 3;
   p.N = W;
   p.K = F;
   grouped<NO_ACT>(p, bf16, tiles, TM, std::min(E, A));
@@ -866,20 +913,13 @@ std::vector<torch::Tensor> moe_silu_glu(torch::Tensor h, torch::Tensor sel, torc
   return experts<GLU_ACT>(h, sel, w_gu, w_dn, INFINITY, 1.0, 0.0, true);
 }
 
-// Into how many tiles of at most 256 rows a product is cut, evenly: the workgroups, one a
-// CU, take ``cols`` times as many in rounds, a round lasts as its tiles' rows and a constant,
-// and one that does not fill the chip leaves the others a higher clock. (4096 x 28672 x 4096:
-// rounds of 256, 224, 192 and 128 rows 94, 84, 73 and 53 us; 1000 x 4096 x 4096, 64 tiles
-// of 256 rows 70 us, 128 of 128 41.)
+// Into how many tiles of at most 256 rows, and ``cols`` columns, a product is cut, evenly
 static int row_tiles(long rows, long cols) {
   const long parts = (rows + 31) / 32, least = (parts + 7) / 8;
   long best = least;
-  double low = 0;
+  float low = 0;
   for (long n = least; n <= std::min(parts, least < 8 ? 8 * least : 2 * least); ++n) {
-    const long full = n * cols / 256, rest = n * cols % 256;
-    const double mean = (double)parts / n, most = (double)((parts + n - 1) / n);
-    const double time = full * (mean + 1.25) +
-                        (rest ? (0.75 + 0.25 * rest / 256) * (most + 1.25) : 0);
+    const float time = rounds_time(n * cols, (float)parts / n, (int)((parts + n - 1) / n));
     if (n == least || time < low) low = time, best = n;
   }
   return (int)best;

@@ -81,3 +81,35 @@ def test_rows_of_a_tile(T, N, K, silu):
         want = torch.nn.functional.silu(want[:, :N]) * want[:, N:]
     # rounded by up to 2^-8 of itself; fp32 sums of K terms stay below 2^-16 of the largest
     assert ((got.double() - want).abs() <= 2 ** -8 * want.abs() + 2 ** -16 * want.abs().max()).all()
+
+
+@pytest.mark.parametrize("W,F,E,top", [(128, 256, 180, 1), (192, 320, 180, 2), (520, 448, 64, 1)])
+@pytest.mark.parametrize("kind", ["glu", "relu2"])
+def test_tiles_of_uneven_experts(W, F, E, top, kind):
+    """Enough experts of 36 rows and more for tiles of up to 256: experts cut into two to five
+    alike, those of no and of one row, and the two products' tables."""
+    W = W // 64 * 64
+    g = torch.Generator(device="cuda").manual_seed(E + W)
+    rows = [0, 1, 31, 32, 33, 255, 256, 257, 289, 600, 1100, 16, 0] + [45] * (E - 13)
+    rows[-1] += -sum(rows) % top
+    A = sum(rows)
+    assert A >= 36 * E and (A // 128 + E) * min(-(-F // 256), -(-W // 256)) >= 170
+    sel = torch.repeat_interleave(torch.arange(E, device="cuda"), torch.tensor(rows, device="cuda"))
+    sel = sel[torch.randperm(A, generator=g, device="cuda")].int().view(-1, top).contiguous()
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    h, dn = n(len(sel), W).bfloat16(), (n(E, W, F) * F ** -0.5).bfloat16()
+    up = (n(E, (2 if kind == "glu" else 1) * F, W) * W ** -0.5).bfloat16()
+    if kind == "glu":
+        y, place = _hip("moe_silu_glu").moe_silu_glu(h, sel, up, dn)
+    else:
+        y, place = _hip("moe_relu2").moe_relu2(h, sel, up, dn)
+    assert sorted(place.flatten().tolist()) == list(range(A))
+    for e in range(E):
+        t, k = (sel == e).nonzero(as_tuple=True)
+        z = h[t].double() @ up[e].double().t()
+        z = torch.nn.functional.silu(z[:, :F]) * z[:, F:] if kind == "glu" else z.clamp(min=0) ** 2
+        want = z @ dn[e].double().t()
+        # activations and then results are rounded, each by up to 2^-8 of itself
+        err = (y[place[t, k].long()].double() - want).norm(dim=-1)
+        through = torch.linalg.matrix_norm(dn[e].double(), 2) * z.norm(dim=-1)
+        assert (err <= 2 ** -8 * (want.norm(dim=-1) + through) + 1e-9).all()
