@@ -49,9 +49,10 @@ class EncoderLayer(nn.Module):
         x, delta = self.step(x, None, cos_sin, positions, cu)
         return x + delta
 
-    def step(self, x, delta, cos_sin, positions, cu):
+    def step(self, x, delta, cos_sin, positions, cu, in_order=False):
         """The stream ``x``, to which ``delta`` (the layer before's result) is still to be
-        added -> the stream and this layer's."""
+        added -> the stream and this layer's. ``in_order``: positions are the tokens' places
+        in their texts."""
         T = x.shape[0]
         if delta is None:
             h = ops.rmsnorm(x, self.norm1, self.eps)
@@ -59,11 +60,14 @@ class EncoderLayer(nn.Module):
             h, x = ops.rmsnorm_residual(delta, x, self.norm1, self.eps)
         qkv = _product(self.qkv, h).view(T, 3 * self.n_heads, self.head_dim)
         q, k, v = qkv.split(self.n_heads, dim=1)
-        if is_plain(self.qkv, nn.Linear):
-            ops.rope_apply_(q, k, positions, cos_sin)
-        else:  # what somebody else made may be kept by them
-            q, k = ops.rope_apply(q.clone(), k.clone(), positions, cos_sin)
-        o = ops.attention_prefill(q, k, v, cu, self.scale, causal=False)
+        if in_order:
+            o = ops.attention_prefill_turned(q, k, v, cos_sin, cu, self.scale, causal=False)
+        else:
+            if is_plain(self.qkv, nn.Linear):
+                ops.rope_apply_(q, k, positions, cos_sin)
+            else:  # what somebody else made may be kept by them
+                q, k = ops.rope_apply(q.clone(), k.clone(), positions, cos_sin)
+            o = ops.attention_prefill(q, k, v, cu, self.scale, causal=False)
         h, x = ops.rmsnorm_residual(_product(self.o, o.reshape(T, -1)), x, self.norm2, self.eps)
         if is_plain(self.gate_up, nn.Linear) and self.gate_up.bias is None:
             act = ops.linear_silu_mul(h, self.gate_up.weight)
@@ -121,7 +125,7 @@ class SentenceEncoder(nn.Module):
         delta = None
         for layer in self.layers:
             if is_plain(layer, EncoderLayer):
-                x, delta = layer.step(x, delta, self.cos_sin, pos_t, cu_t)
+                x, delta = layer.step(x, delta, self.cos_sin, pos_t, cu_t, in_order=True)
             else:  # somebody watches it or has replaced it
                 x, delta = x if delta is None else x + delta, None
                 x = layer(x, self.cos_sin, pos_t, cu_t)

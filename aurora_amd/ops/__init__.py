@@ -109,6 +109,27 @@ def attention_prefill(
     return torch_ref.attention_prefill(q, k, v, cu_seqlens, scale, causal)
 
 
+def attention_prefill_turned(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    cos_sin: torch.Tensor,
+    cu_seqlens: torch.Tensor,
+    scale: float,
+    causal: bool = True,
+) -> torch.Tensor:
+    """``attention_prefill`` of queries and keys that are rotated first, each by its place in
+    its sequence; ``cos_sin`` reaches as far as the longest. They stay as they are."""
+    if q.is_cuda:
+        m = _require_hip("attention_prefill_turned", aux=True)
+        return m.attention_prefill_turned(
+            q, k, v, cos_sin.to(torch.float32).contiguous(),
+            cu_seqlens.to(torch.int32).contiguous(), float(scale), bool(causal))
+    begin = torch.repeat_interleave(cu_seqlens[:-1], cu_seqlens.diff())
+    q, k = rope_apply(q, k, torch.arange(q.shape[0], device=q.device) - begin, cos_sin)
+    return torch_ref.attention_prefill(q, k, v, cu_seqlens, scale, causal)
+
+
 def attention_prefill_paged(
     q: torch.Tensor,
     k_cache: torch.Tensor,

@@ -3,6 +3,9 @@
 
 torch::Tensor attention_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
                                 torch::Tensor cu, double scale, bool causal);
+torch::Tensor attention_prefill_turned(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                                       torch::Tensor cos_sin, torch::Tensor cu, double scale,
+                                       bool causal);
 torch::Tensor embed_pool(torch::Tensor hidden, torch::Tensor cu);
 std::vector<torch::Tensor> knn_topk(torch::Tensor query, torch::Tensor docs, long k);
 std::vector<uint8_t> oneshot_init(long world, long rank, long max_bytes);
@@ -14,6 +17,8 @@ void oneshot_destroy();
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("attention_prefill", &attention_prefill, "varlen self-attention (encoder)");
+  m.def("attention_prefill_turned", &attention_prefill_turned,
+        "the same with queries and keys rotated by their places");
   m.def("embed_pool", &embed_pool, "mean-pool + L2 normalize");
   m.def("knn_topk", &knn_topk, "brute-force kNN top-k");
   m.def("oneshot_init", &oneshot_init, "one-shot allreduce: alloc + IPC handle");

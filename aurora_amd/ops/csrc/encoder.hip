@@ -20,14 +20,18 @@
 // Bound by memory and by the start of its many short sequences: 200 texts of 20 to 256
 // tokens, 12 heads of 64 (170 MB) 676 us as a wave per row and head over scalar dot
 // products, now 70 us.
-template <int D>
+// TURN: queries and keys are rotated here by their places in their sequence, a tile of keys
+// in LDS as it arrives, and rounded as the rotation in memory rounds them (which reads and
+// writes both: the same texts 27 us and 71 for the attention, together 82).
+template <int D, bool TURN>
 __global__ __launch_bounds__(256, 2) void packed_attn_kernel(
     const __hip_bfloat16* __restrict__ q,  // rows of Hq heads, D apart
     const __hip_bfloat16* __restrict__ k,  // rows of Hkv heads
     const __hip_bfloat16* __restrict__ v,
     __hip_bfloat16* __restrict__ out,  // [T, Hq, D]
     const int* __restrict__ cu, int S, int Hq, int Hkv, long qstride, long kstride,
-    long vstride, float scale, int causal) {
+    long vstride, float scale, int causal,
+    const float* __restrict__ cos_sin, int places) {  // TURN: [places, D], cosines, then sines
   constexpr int NC = D / 16, NDT = D / 32, U = D / 8;
   constexpr int LU = ENC_KEYS * U / 256;  // loads per thread of K, and of V
   constexpr int KBYTES = ENC_KEYS * D * 2, STAGE = 2 * KBYTES;
@@ -62,6 +66,63 @@ __global__ __launch_bounds__(256, 2) void packed_attn_kernel(
     }
   };
   issue(0);
+  // of a token's rotation the cosines and sines of 8 pairs, from pair i on
+  struct Angles {
+    floatx4 c[2], s[2];
+  };
+  auto angles = [&](int t, int i) {
+    const float* cs = cos_sin + (long)min(t, places - 1) * D + i;
+    Angles y;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      y.c[k] = *reinterpret_cast<const floatx4*>(cs + 4 * k);
+      y.s[k] = *reinterpret_cast<const floatx4*>(cs + D / 2 + 4 * k);
+    }
+    return y;
+  };
+  auto rotate = [](frag_u& u, frag_u& w, const Angles& y) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      float a[2], b[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int e = 2 * j + k;
+        const float c = y.c[e / 4][e % 4], s = y.s[e / 4][e % 4];
+        const float x1 = __builtin_bit_cast(float, k ? u.u[j] & 0xffff0000u : u.u[j] << 16);
+        const float x2 = __builtin_bit_cast(float, k ? w.u[j] & 0xffff0000u : w.u[j] << 16);
+        a[k] = x1 * c - x2 * s;
+        b[k] = x2 * c + x1 * s;
+      }
+      u.u[j] = cvt2_bf16(a[0], a[1]);
+      w.u[j] = cvt2_bf16(b[0], b[1]);
+    }
+  };
+  // a tile's rows have U / 2 pairs of units; a thread's
+  constexpr int PAIRS = TURN ? ENC_KEYS * U / 2 / 256 : 1;
+  Angles turn[PAIRS];
+  auto prepare = [&](int tile) {
+#pragma unroll
+    for (int x = 0; x < PAIRS; ++x) {
+      const int p = tid + x * 256;
+      turn[x] = angles(min(tile * ENC_KEYS + p / (U / 2), n - 1), p % (U / 2) * 8);
+    }
+  };
+  auto turn_keys = [&](int tile) {
+#pragma unroll
+    for (int x = 0; x < PAIRS; ++x) {
+      const unsigned p = tid + x * 256u, r = p / (U / 2), unit = p % (U / 2);
+      char* row = smem + (tile & 1) * STAGE + r * D * 2;
+      shortx8* a = reinterpret_cast<shortx8*>(row + ((unit ^ (r & KMASK)) << 4));
+      shortx8* b = reinterpret_cast<shortx8*>(row + (((unit + U / 2) ^ (r & KMASK)) << 4));
+      frag_u u, w;
+      u.s = *a;
+      w.s = *b;
+      rotate(u, w, turn[x]);
+      *a = u.s;
+      *b = w.s;
+    }
+  };
+  if constexpr (TURN) prepare(0);
 
   // a scale that is not positive goes into the queries: the reference below compares
   // unscaled scores
@@ -74,9 +135,15 @@ __global__ __launch_bounds__(256, 2) void packed_attn_kernel(
     if (valid && scale != 0.f)
       qf[c].s = *reinterpret_cast<const shortx8*>(q + (a + row) * qstride + h * D + c * 16 +
                                                   half * 8);
+  }
+  if constexpr (TURN)
+#pragma unroll
+    for (int c = 0; c < NC / 2; ++c)
+      rotate(qf[c], qf[c + NC / 2], angles(min(row, n - 1), c * 16 + half * 8));
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int j = 0; j < 4; ++j) qf[c].u[j] ^= flip;
-  }
   unsigned kat[NC], vat[NDT];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
@@ -100,7 +167,12 @@ __global__ __launch_bounds__(256, 2) void packed_attn_kernel(
   for (int tile = 0; tile < ntiles; ++tile) {
     // this tile is there for all, and nobody reads the other buffer any more
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-    if (tile + 1 < ntiles) issue(tile + 1);
+    if constexpr (TURN) turn_keys(tile);
+    if (tile + 1 < ntiles) {
+      issue(tile + 1);
+      if constexpr (TURN) prepare(tile + 1);
+    }
+    if constexpr (TURN) asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const unsigned st = (tile & 1) * STAGE;
     static_for<2>([&](auto SECOND) {
       constexpr int second = decltype(SECOND)::value;
@@ -251,8 +323,12 @@ static torch::Tensor row_readable(const torch::Tensor& t) {
   return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
-torch::Tensor attention_prefill(torch::Tensor q_, torch::Tensor k_, torch::Tensor v_,
-                                torch::Tensor cu, double scale, bool causal) {
+// ``cos_sin`` [places, D] fp32: queries and keys, not yet rotated, are turned by their places
+// in their sequences, which must not be longer
+static torch::Tensor packed_attention(const torch::Tensor& q_, const torch::Tensor& k_,
+                                      const torch::Tensor& v_, const torch::Tensor& cu,
+                                      double scale, bool causal,
+                                      const c10::optional<torch::Tensor>& cos_sin) {
   TORCH_CHECK(q_.is_cuda() && q_.dtype() == torch::kBFloat16, "bf16 GPU only");
   const int T = q_.size(0), Hq = q_.size(1), D = q_.size(2), Hkv = k_.size(1);
   TORCH_CHECK(D == 64 || D == 128, "head_dim must be 64/128");
@@ -260,6 +336,11 @@ torch::Tensor attention_prefill(torch::Tensor q_, torch::Tensor k_, torch::Tenso
               v_.size(0) >= T && v_.size(1) == Hkv && k_.size(2) == D && v_.size(2) == D &&
               Hq % Hkv == 0 && cu.dtype() == torch::kInt32 && cu.is_contiguous(),
               "queries, keys and values");
+  TORCH_CHECK(!cos_sin || (cos_sin->is_cuda() && cos_sin->dtype() == torch::kFloat32 &&
+                           cos_sin->is_contiguous() && cos_sin->dim() == 2 &&
+                           cos_sin->size(0) > 0 && cos_sin->size(1) == D &&
+                           (reinterpret_cast<uintptr_t>(cos_sin->data_ptr()) & 15) == 0),
+              "cosines and sines");
   auto out = torch::empty({T, Hq, D}, q_.options());
   const int S = cu.numel() - 1;
   if (T == 0 || S < 1) return out;
@@ -271,12 +352,27 @@ torch::Tensor attention_prefill(torch::Tensor q_, torch::Tensor k_, torch::Tenso
                        (const __hip_bfloat16*)q.data_ptr(), (const __hip_bfloat16*)k.data_ptr(),
                        (const __hip_bfloat16*)v.data_ptr(), (__hip_bfloat16*)out.data_ptr(),
                        cu.data_ptr<int>(), S, Hq, Hkv, q.stride(0), k.stride(0), v.stride(0),
-                       (float)scale, causal ? 1 : 0);
+                       (float)scale, causal ? 1 : 0,
+                       cos_sin ? cos_sin->data_ptr<float>() : nullptr,
+                       cos_sin ? (int)cos_sin->size(0) : 0);
   };
-  if (D == 64) launch(packed_attn_kernel<64>, 2 * 2 * ENC_KEYS * 64 * 2);
-  else launch(packed_attn_kernel<128>, 2 * 2 * ENC_KEYS * 128 * 2);
+  if (D == 64 && cos_sin) launch(packed_attn_kernel<64, true>, 2 * 2 * ENC_KEYS * 64 * 2);
+  else if (D == 64) launch(packed_attn_kernel<64, false>, 2 * 2 * ENC_KEYS * 64 * 2);
+  else if (cos_sin) launch(packed_attn_kernel<128, true>, 2 * 2 * ENC_KEYS * 128 * 2);
+  else launch(packed_attn_kernel<128, false>, 2 * 2 * ENC_KEYS * 128 * 2);
   HIP_CHECK_KERNEL();
   return out;
+}
+
+torch::Tensor attention_prefill(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                                torch::Tensor cu, double scale, bool causal) {
+  return packed_attention(q, k, v, cu, scale, causal, c10::nullopt);
+}
+
+torch::Tensor attention_prefill_turned(torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                                       torch::Tensor cos_sin, torch::Tensor cu, double scale,
+                                       bool causal) {
+  return packed_attention(q, k, v, cu, scale, causal, cos_sin);
 }
 
 // ---- mean-pool + L2 normalize per sequence -------------------------------

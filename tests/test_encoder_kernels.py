@@ -1,5 +1,7 @@
 """The encoder's kernels at the edges of their tiles, over strided rows, and short rows of
 the norms."""
+import itertools
+
 import pytest
 import torch
 
@@ -48,6 +50,27 @@ def test_rotation_in_place_of_strided_rows(D, H, G):
     assert torch.equal(x[:, H + G:], rest)
     for a, b in zip((x[:, :H], x[:, H:H + G]), want):  # at most one rounding the other way
         assert (a.cpu().float() - b.float()).abs().max() <= 2 ** -8 * b.float().abs().max()
+
+
+@pytest.mark.parametrize("scale", [0.125, -0.1])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("D,H,G", [(64, 4, 2), (128, 2, 2)])
+def test_attention_rotates_as_the_rotation_does(D, H, G, causal, scale):
+    lens = [1, 31, 63, 64, 65, 127, 128, 129, 0, 200, 300]  # tiles of 64 keys, 128 rows
+    cu = torch.tensor([0, *itertools.accumulate(lens)], dtype=torch.int32, device="cuda")
+    x = torch.randn(sum(lens), H + 2 * G, D, device="cuda").bfloat16()
+    pos = torch.cat([torch.arange(n) for n in lens]).int().cuda()
+    cs = torch_ref.rope_cos_sin_cache(D, max(lens), 1e4).cuda()
+    q, k, v = x.split([H, G, G], dim=1)
+    before = x.clone()
+    got = ops.attention_prefill_turned(q, k, v, cs, cu, scale, causal)
+    assert torch.equal(x, before)
+    q, k = ops.rope_apply(q.clone(), k.clone(), pos, cs)
+    want = ops.attention_prefill(q, k, v, cu, scale, causal)
+    # a rotated number may be rounded the other way, by 2^-8 of itself: scores of D of them
+    # move by some 2^-8 of their spread of scale sqrt(D)
+    err = (got.float() - want.float()).norm(dim=(1, 2)) / want.float().norm(dim=(1, 2))
+    assert err.max() < 2 ** -7, float(err.max())
 
 
 @pytest.mark.parametrize("T,H", [(1, 8), (5, 64), (4, 504), (3, 512), (7, 520), (9, 768),
