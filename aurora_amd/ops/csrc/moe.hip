@@ -32,6 +32,27 @@ union mfrag {
 
 enum { CHOSEN_SOFTMAX = 0, GROUPED_SIGMOID = 1, GROUPED_SOFTMAX = 2 };
 
+// The largest value of a wave's lanes but NaN, without a trip through LDS. (Choices by
+// butterflies over value and index took 12 such trips each: 64 tokens of 2048 over 64
+// experts, six each, 16.9 and 14.4 us; over 128, eight each, 28.7 and 25.8; 32 of 4096 over 8,
+// two each, 10.5 and 9.6. What is left is a CU's read of the whole router.)
+DEVINL float lanes_max(float x) {
+  auto step = [](float a, auto CTRL) {
+    return fmaxf(a, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(
+        __builtin_bit_cast(int, a), decltype(CTRL)::value, 0xf, 0xf, false)));
+  };
+  x = step(x, std::integral_constant<int, 0xb1>{});   // neighbours
+  x = step(x, std::integral_constant<int, 0x4e>{});   // pairs of a quad
+  x = step(x, std::integral_constant<int, 0x141>{});  // halves of eight
+  x = step(x, std::integral_constant<int, 0x140>{});  // of sixteen
+  const unsigned u = __builtin_bit_cast(unsigned, x);
+  const auto a = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  x = fmaxf(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1]));
+  const unsigned w = __builtin_bit_cast(unsigned, x);
+  const auto b = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
+}
+
 // one workgroup per 16 tokens; its waves split the contraction. GROUPED_SIGMOID: bias
 // is the scores' correction; GROUPED_SOFTMAX: there is none
 template <typename T, bool MATRIX16, int ROUTER>
@@ -142,16 +163,27 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(
       sync();
     }
     float first = 0.f, sum = 0.f;
+    // up to 64 experts: a lane holds its own, the first of the largest is found by lane
+    const bool few = E <= WAVE;
+    float mine = few && lane < E ? z[lane] : -INFINITY;
     for (int n = 0; n < top; ++n) {
       float best = -INFINITY;
       int at = 0x7fffffff;
-      for (int e = lane; e < E; e += WAVE)
-        if (z[e] > best) { best = z[e]; at = e; }
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        const float ob = __shfl_xor(best, off, WAVE);
-        const int oa = __shfl_xor(at, off, WAVE);
-        if (ob > best || (ob == best && oa < at)) { best = ob; at = oa; }
+      if (few) {
+        best = lanes_max(mine);
+        const unsigned long long who = __ballot(mine == best && best > -INFINITY);
+        if (who) at = __builtin_ctzll(who);
+        else best = -INFINITY;
+        if (lane == at) mine = -INFINITY;
+      } else {
+        float own = -INFINITY;
+        int oat = 0;
+        for (int e = lane; e < E; e += WAVE)
+          if (z[e] > own) { own = z[e]; oat = e; }
+        best = lanes_max(own);
+        for (unsigned long long who = __ballot(own == best && best > -INFINITY); who;
+             who &= who - 1)
+          at = min(at, __builtin_amdgcn_readlane(oat, __builtin_ctzll(who)));
       }
       at = min(at, E - 1);  // all logits NaN: still a valid expert
       if (n == 0) first = best;

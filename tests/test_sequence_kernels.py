@@ -320,6 +320,28 @@ def test_retention(dtype, H, d, e, rot):
 
 # ------------------------------------------------------------------ experts
 
+@pytest.mark.parametrize("E,top", [(1, 1), (2, 2), (63, 5), (64, 64), (65, 3), (130, 9),
+                                   (512, 4)])
+def test_choices_among_equal_and_missing_scores(E, top):
+    """Of equal scores the first experts' are chosen, and tokens of NaN get experts that
+    exist."""
+    T = 37
+    z = torch.randint(-2, 3, (T, E)).float()  # many ties, exact in bf16
+    z[1] = -3e38
+    router = torch.zeros(E, max(64, (E + 7) // 8 * 8))
+    router[:, :E] = torch.eye(E)
+    h = torch.zeros(T, router.shape[1])
+    h[:, :E] = z.bfloat16().float()
+    h[5] = float("nan")
+    sel, gate = ops._hip.moe_route(*gpu(h.bfloat16(), router.bfloat16()), None, top)
+    want = torch.sort(h[:, :E], dim=1, descending=True, stable=True).indices[:, :top].int()
+    real = torch.arange(T) != 5
+    assert torch.equal(sel.cpu()[real], want[real])
+    assert ((sel >= 0) & (sel < E)).all()
+    picked = h[:, :E].gather(1, want.long())[real]
+    assert torch.allclose(gate.cpu()[real], torch.softmax(picked, 1), rtol=1e-5, atol=0)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("T,W,F,E,top", [
     (1, 512, 256, 8, 2), (5, 50, 20, 3, 3), (64, 128, 64, 70, 4), (300, 256, 128, 4, 1),
