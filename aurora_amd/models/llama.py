@@ -139,15 +139,17 @@ class LlamaAttention(nn.Module):
             # projections/norms run on the whole packed batch (bigger GEMMs),
             # attention splits per regime
             Tp = meta.num_prefill_tokens
-            o_pre = ops.attention_prefill_paged(
-                q[:Tp], k_cache, v_cache, meta.block_tables,
-                meta.cu_seqlens_q, meta.context_lens, self.scale,
-            ) if Tp else q[:0]
-            o_dec = ops.paged_attention_decode(
-                q[Tp:].contiguous(), k_cache, v_cache, meta.dec_block_tables,
-                meta.dec_context_lens, self.scale,
-            ) if T > Tp else q[:0]
-            o = torch.cat([o_pre, o_dec]) if (Tp and T > Tp) else (o_pre if Tp else o_dec)
+            o = torch.empty_like(q)
+            if Tp:
+                ops.attention_prefill_paged(
+                    q[:Tp], k_cache, v_cache, meta.block_tables,
+                    meta.cu_seqlens_q, meta.context_lens, self.scale, out=o[:Tp],
+                )
+            if T > Tp:
+                ops.paged_attention_decode(
+                    q[Tp:], k_cache, v_cache, meta.dec_block_tables,
+                    meta.dec_context_lens, self.scale, out=o[Tp:],
+                )
         return o.reshape(T, self.n_heads * self.head_dim)
 
 

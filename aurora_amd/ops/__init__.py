@@ -138,16 +138,19 @@ def attention_prefill_paged(
     cu_seqlens_q: torch.Tensor,
     context_lens: torch.Tensor,
     scale: float,
+    out: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
+    """``out``: where the results go, contiguous and shaped as ``q``."""
     if q.is_cuda:
         m = _require_hip("attention_prefill_paged")
         return m.attention_prefill_paged(
             q.contiguous(), k_cache, v_cache, block_tables.to(torch.int32),
-            cu_seqlens_q.to(torch.int32), context_lens.to(torch.int32), float(scale),
+            cu_seqlens_q.to(torch.int32), context_lens.to(torch.int32), float(scale), out,
         )
-    return torch_ref.attention_prefill_paged(
+    y = torch_ref.attention_prefill_paged(
         q, k_cache, v_cache, block_tables, cu_seqlens_q, context_lens, scale
     )
+    return y if out is None else out.copy_(y)
 
 
 def kv_cache_write(
@@ -170,14 +173,17 @@ def paged_attention_decode(
     block_tables: torch.Tensor,
     context_lens: torch.Tensor,
     scale: float,
+    out: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
+    """``out``: where the results go, contiguous and shaped as ``q``."""
     if q.is_cuda:
         m = _require_hip("paged_attention_decode")
         return m.paged_attention_decode(
             q.contiguous(), k_cache, v_cache,
-            block_tables.to(torch.int32), context_lens.to(torch.int32), float(scale),
+            block_tables.to(torch.int32), context_lens.to(torch.int32), float(scale), out,
         )
-    return torch_ref.paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale)
+    y = torch_ref.paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale)
+    return y if out is None else out.copy_(y)
 
 
 def fused_rope_kv_write(qkv, positions, slots, cos_sin, k_cache, v_cache,

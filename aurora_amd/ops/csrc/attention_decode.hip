@@ -476,12 +476,13 @@ static void decode_launch(const torch::Tensor& q, const torch::Tensor& kc,
 
 torch::Tensor paged_attention_decode(torch::Tensor q, torch::Tensor kc,
                                      torch::Tensor vc, torch::Tensor bt,
-                                     torch::Tensor ctx, double scale) {
+                                     torch::Tensor ctx, double scale,
+                                     c10::optional<torch::Tensor> into) {
   TORCH_CHECK(q.is_cuda() && q.dtype() == torch::kBFloat16, "bf16 GPU only");
   const int B = q.size(0), Hq = q.size(1), D = q.size(2), Hkv = kc.size(1);
   TORCH_CHECK(Hq % Hkv == 0, "GQA requires Hq % Hkv == 0");
   TORCH_CHECK(D == 128 || D == 64, "unsupported head_dim ", D);
-  auto out = torch::empty_like(q);
+  auto out = result_like(q, into);
   if (B == 0) return out;
   auto* o = (__hip_bfloat16*)out.data_ptr();
   const long stride = (long)Hq * D;

@@ -571,12 +571,12 @@ static void prefill_launch(int blocks, int Hq, Args... args) {
 torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
                                       torch::Tensor vc, torch::Tensor bt,
                                       torch::Tensor cu_q, torch::Tensor ctx,
-                                      double scale) {
+                                      double scale, c10::optional<torch::Tensor> into) {
   TORCH_CHECK(q.is_cuda() && q.dtype() == torch::kBFloat16, "bf16 GPU only");
   const int T = q.size(0), Hq = q.size(1), D = q.size(2);
   const int Hkv = kc.size(1), P = kc.size(2), MP = bt.size(1);
   TORCH_CHECK(D == 128 || D == 64, "head_dim must be 64 or 128, got ", D);
-  auto out = torch::empty_like(q);
+  auto out = result_like(q, into);
   if (T == 0) return out;
   kc = unit_aligned(kc);
   vc = unit_aligned(vc);

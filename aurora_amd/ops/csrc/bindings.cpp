@@ -11,11 +11,12 @@ void kv_cache_write(torch::Tensor k, torch::Tensor v, torch::Tensor kc,
                     torch::Tensor vc, torch::Tensor slots);
 torch::Tensor paged_attention_decode(torch::Tensor q, torch::Tensor kc,
                                      torch::Tensor vc, torch::Tensor bt,
-                                     torch::Tensor ctx, double scale);
+                                     torch::Tensor ctx, double scale,
+                                     c10::optional<torch::Tensor> into);
 torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
                                       torch::Tensor vc, torch::Tensor bt,
                                       torch::Tensor cu_q, torch::Tensor ctx,
-                                      double scale);
+                                      double scale, c10::optional<torch::Tensor> into);
 torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w);
 torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
                                   torch::Tensor slots, torch::Tensor cos_sin,

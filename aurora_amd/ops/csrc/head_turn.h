@@ -52,3 +52,14 @@ inline HeadTurn head_turn(const c10::optional<torch::Tensor>& turn,
   }
   return t;
 }
+
+// where results of queries q go: ``into``, or a tensor of their own
+inline torch::Tensor result_like(const torch::Tensor& q,
+                                 const c10::optional<torch::Tensor>& into) {
+  if (!into) return torch::empty_like(q);
+  TORCH_CHECK(into->device() == q.device() && into->dtype() == q.dtype() &&
+                  into->sizes() == q.sizes() && into->is_contiguous() &&
+                  (reinterpret_cast<uintptr_t>(into->data_ptr()) & 15) == 0,
+              "results lie as the queries do");
+  return *into;
+}

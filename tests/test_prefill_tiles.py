@@ -91,3 +91,23 @@ def test_block_search_over_many_sequences():
           for t in (q, k, v, bt, cu, ctx)), 0.125)
     err = (got - want).norm(dim=-1) / want.norm(dim=-1)
     assert err.max() < 2 ** -7
+
+
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.bfloat16),
+                                     (128, torch.float8_e4m3fn)])
+def test_results_into_a_buffer(D, dtype):
+    """Prompts and decoding rows of one batch write their parts of one tensor."""
+    q, k, v, bt, cu, ctx = _case(64, 8, 4, D, dtype)
+    one = q[:len(ctx)].contiguous()
+    want = ops.attention_prefill_paged(q, k, v, bt, cu, ctx, 0.1)
+    last = ops.paged_attention_decode(one, k, v, bt, ctx, 0.1)
+    both = torch.full((len(q) + len(one) + 1, *q.shape[1:]), 7.0, device="cuda").bfloat16()
+    ops.attention_prefill_paged(q, k, v, bt, cu, ctx, 0.1, out=both[:len(q)])
+    ops.paged_attention_decode(one, k, v, bt, ctx, 0.1, out=both[len(q):-1])
+    assert torch.equal(both[:len(q)], want) and torch.equal(both[len(q):-1], last)
+    assert (both[-1] == 7).all()
+    for wrong in (both[1:], both[:len(q)].float(), both[:len(q), ::2]):
+        with pytest.raises(RuntimeError):
+            ops.attention_prefill_paged(q, k, v, bt, cu, ctx, 0.1, out=wrong)
+        with pytest.raises(RuntimeError):
+            ops.paged_attention_decode(one, k, v, bt, ctx, 0.1, out=wrong)
