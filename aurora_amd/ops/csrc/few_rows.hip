@@ -45,7 +45,7 @@ DEVINL void await_stage() {
 template <int WN, int MT, int NS, bool SILU>
 __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
     const unsigned short* x, const unsigned short* w, unsigned short* out, float* part, int M,
-    int N, int K, int span) {
+    int N, int K, int span, long ldx) {
   constexpr int NT = WN * 4;
   constexpr int L = (WN * 8 + MT * 128 + NT - 1) / NT;  // loads of a thread per stage
   constexpr int STAGE = L * NT * 16;
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
     if (l >= WN * 8 / NT) row = min(r - WN, M - 1);
     else if constexpr (SILU) row = min(n0 + r / 16 * 8 + r % 8, N - 1) + (long)(r % 16 / 8) * N;
     else row = min(n0 + r, N - 1);
-    src[l] = (l >= WN * 8 / NT ? x : w) + row * K + k0 + unit * 8;
+    src[l] = (l >= WN * 8 / NT ? x + row * ldx : w + row * K) + k0 + unit * 8;
   }
   auto issue = [&](int s) {
     char* stage = lds + s % NS * STAGE;
@@ -160,11 +160,21 @@ static long parts_of(long N, long K) {
 
 static void check(const torch::Tensor& x, const torch::Tensor& w) {
   TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dtype() == torch::kBFloat16 &&
-                  w.dtype() == torch::kBFloat16 && x.is_contiguous() && w.is_contiguous(),
+                  w.dtype() == torch::kBFloat16 && w.is_contiguous(),
               "contiguous bf16 GPU only");
   TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && x.size(0) <= FEW_MOST &&
                   x.size(1) % FEW_K == 0,
               "at most ", FEW_MOST, " rows and K a multiple of ", FEW_K);
+}
+
+// x as 16-byte loads can read its rows, which may be strided (a part of a joint projection,
+// 64 rows of 256, copied first took 4.5 us more)
+static torch::Tensor readable(const torch::Tensor& x) {
+  const bool ok = x.dim() == 2 && (x.stride(1) == 1 || x.size(1) == 1) &&
+                  (x.size(0) == 1 || (x.stride(0) >= x.size(1) && x.stride(0) % 8 == 0)) &&
+                  (uintptr_t)x.data_ptr() % 16 == 0;
+  // (contiguous() gives the same tensor back where only its address is odd)
+  return ok ? x : x.clone(at::MemoryFormat::Contiguous);
 }
 
 template <int WN, int MT, int NS, bool SILU>
@@ -174,13 +184,14 @@ static void launch(const torch::Tensor& x, const torch::Tensor& w, unsigned shor
   hipLaunchKernelGGL((few_rows_kernel<WN, MT, NS, SILU>), dim3((N + tile - 1) / tile, S),
                      dim3(WN * 4), 0, CUR_STREAM, (const unsigned short*)x.data_ptr(),
                      (const unsigned short*)w.data_ptr(), out, part, (int)x.size(0), (int)N,
-                     (int)x.size(1), (int)span);
+                     (int)x.size(1), (int)span, x.size(0) > 1 ? x.stride(0) : 0L);
   HIP_CHECK_KERNEL();
 }
 
 // [M, N] in bf16, or with ``raw`` where K is cut [S, M, N] in fp32, S terms to be added.
 torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts) {
   check(x, w);
+  x = readable(x);
   const long M = x.size(0), K = x.size(1), N = w.size(0);
   torch::Tensor out, part;
   if (M == 0 || N == 0 || K == 0) return torch::zeros({M, N}, x.options());
@@ -214,6 +225,7 @@ torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw) {
 // silu(x @ gate^T) * (x @ up^T), rounded once; w: gate's rows, then up's
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w) {
   check(x, w);
+  x = readable(x);
   TORCH_CHECK(w.size(0) % 2 == 0);
   const long M = x.size(0), K = x.size(1), N = w.size(0) / 2;
   auto out = torch::empty({M, N}, x.options());

@@ -105,7 +105,7 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
     if (N % 16) return {};
     if (M <= 128) {
       if (!silu_few_rows_win(M, N / 2, K)) return {};
-      return silu_few_rows(x.contiguous(), w);
+      return silu_few_rows(x, w);
     }
     if (large_takes(M, N, K) && many_rows_win(M, N, K, true))
       return many_rows(x, w, true);
@@ -113,8 +113,8 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
   }
   if (M <= 128) {
     if (form == PARTS && few_rows_win(M, N, K, true))
-      return linear_few_rows(x.contiguous(), w, true);
-    if (few_rows_win(M, N, K, false)) return linear_few_rows(x.contiguous(), w, false);
+      return linear_few_rows(x, w, true);
+    if (few_rows_win(M, N, K, false)) return linear_few_rows(x, w, false);
   } else if (large_takes(M, N, K) && many_rows_win(M, N, K, false)) {
     return many_rows(x, w, false);
   }

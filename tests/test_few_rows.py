@@ -124,3 +124,20 @@ def test_rotation_widths(D, T, dtype):
                             (kc.cpu(), k_want, 2 ** -8 if dtype == torch.bfloat16 else 2 ** -4),
                             (vc.cpu(), v_want, 2 ** -8 if dtype == torch.bfloat16 else 2 ** -4)):
         assert ((got.float() - want).abs() <= step * want.abs() + 2 ** -10).all()
+
+
+@pytest.mark.parametrize("M", [1, 2, 33, 65, 128])
+@pytest.mark.parametrize("step,first", [(256, 64), (200, 8), (136, 0), (131, 0), (256, 3)])
+def test_strided_rows(M, step, first):
+    """Columns of a wider tensor, at distances and addresses that 16-byte loads can read and
+    at others."""
+    from aurora_amd import _hip_ops
+    K, N = 128, 96
+    x = torch.randn(M, step + 64, device="cuda").bfloat16().as_strided((M, K), (step, 1), first)
+    w = torch.randn(2 * N, K, device="cuda").bfloat16()
+    whole = x.contiguous().clone()
+    for parts in (1, 2):
+        assert torch.equal(_hip_ops.few_rows(x, w, False, parts),
+                           _hip_ops.few_rows(whole, w, False, parts))
+    assert torch.equal(_hip_ops.silu_few_rows(x, w), _hip_ops.silu_few_rows(whole, w))
+    assert torch.equal(ops.linear(x, w), ops.linear(whole, w))
