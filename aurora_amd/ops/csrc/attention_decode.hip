@@ -17,7 +17,7 @@
 //    sequence that has several.
 // Measured in a graph, before and now (vector dot products, 64 keys at a time, as many
 // stretches for every sequence): 96 sequences of 500 to 2900 keys, 32 heads over 8,
-// 128 wide, 210 and 136 us (4.9 TB/s; a large read reaches 5.5 to 5.8), the same in fp8 211
+// 128 wide, 210 and 124 us (5.4 TB/s; a large read reaches 5.5 to 5.8), the same in fp8 211
 // and 91; 256 of 1600 326 and 289 (5.8 TB/s); 32 of 600 to 2500 66 and 43; one of 12000 102
 // and 26, one of 777 20 and 13; 7 heads over one, 40 of 300 to 3000, 90 and 37; fp8 64 wide,
 // 23 of 300 to 5000, 44 and 25. fp8 is bound by widening its values; a single sequence by
@@ -90,6 +90,72 @@ DEVINL bool find_split(const int* ctx, int B, int length, const Seen& seen, int 
   return false;
 }
 
+// Workgroups that each take a whole context start by length, longest first: the last to start
+// are short. (32 heads over 8, 128 wide, in the order of the batch and so: 96 sequences of 500 to
+// 2900 keys 143 and 124 us, all of their mean 119; 128 of 50 to 1500 87 and 80; 64 of 300 to 8000
+// 232 and 220; 41 of 700 to 2600 74 and 66; 100 of 600 56.2 and 57.1, of 50 16.2 and 16.6.) The
+// sequence whose context is the idx-th longest to a 64th of the longest, in the
+// batch's order where they are alike, and its length; of at most 64 N. All lanes of a wave.
+template <int N>
+DEVINL int ranked(const int* ctx, int B, int idx, int lane, int& length) {
+  int n[N], most = 0;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const int s = lane + k * WAVE;
+    n[k] = s < B ? ctx[s] : 0;
+    most = max(most, n[k]);
+  }
+  auto take = [&](int at) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if (at >> 6 == k) length = __builtin_amdgcn_readlane(n[k], at & 63);
+    return at;
+  };
+  idx = __builtin_amdgcn_readfirstlane(idx);
+  if (!__any(most > 512)) return take(idx);  // an order costs half a microsecond
+  // the highest bit of any
+  int bits = 0;
+#pragma unroll
+  for (int step = 16; step > 0; step >>= 1)
+    if (__any(most >> (bits + step) != 0)) bits += step;
+  const int shift = max(bits - 5, 0);
+  unsigned long long in[N];
+  bool less = false, two = false, three = false;  // quarters of that bit's double
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    in[k] = __ballot(lane + k * WAVE < B);
+    const int v = n[k] >> (shift + 4);
+    if (lane + k * WAVE < B) less |= v < 2, two |= v == 2, three |= v == 3;
+  }
+  if (!__any(less) && !(__any(two) && __any(three))) return take(idx);  // alike
+#pragma unroll
+  for (int bit = 5; bit >= 0; --bit) {
+    unsigned long long one[N];
+    int count = 0;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      one[k] = __ballot(n[k] >> (shift + bit) & 1) & in[k];
+      count += __popcll(one[k]);
+    }
+    const bool here = idx < count;
+    if (!here) idx -= count;
+#pragma unroll
+    for (int k = 0; k < N; ++k) in[k] = here ? one[k] : in[k] & ~one[k];
+  }
+  int at = 0;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const int c = __popcll(in[k]);
+    if (idx >= 0 && idx < c) {
+      const unsigned long long below = (1ull << lane) - 1;
+      const bool is = (in[k] >> lane & 1) && __popcll(in[k] & below) == idx;
+      at = k * WAVE + __builtin_ctzll(__ballot(is));
+    }
+    idx -= c;
+  }
+  return take(__builtin_amdgcn_readfirstlane(at));
+}
+
 // Four V^T fragments at once: rows 4 g .. and 16 + 4 g .. of d-tiles at four addresses.
 template <int SECOND>
 DEVINL void read_value_tiles(shortx4 (&v)[8], unsigned a0, unsigned a1, unsigned a2,
@@ -138,7 +204,11 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
   const int tiles = Hkv * NG, idx = blockIdx.x / tiles, tile = blockIdx.x % tiles;
   const int kvh = tile / NG, h0 = kvh * G + tile % NG * DEC_HEADS;
   const int GT = min(DEC_HEADS, kvh * G + G - h0);
-  int b = idx, split = 0, nsplits = 1, length = 0x7fffffff;
+  int b = idx, split = 0, nsplits = 1, length = 0x7fffffff, L = -1;
+  if (!cut && seen.window <= 0 && seen.chunk <= 0) {
+    if (B <= 2 * WAVE) b = ranked<2>(ctx_lens, B, idx, lane, L);
+    else if (B <= 4 * WAVE) b = ranked<4>(ctx_lens, B, idx, lane, L);
+  }
   if (cut) {
     length = split_length(ctx_lens, B, tiles, DEC_TARGET, seen, lane);
     if (!find_split(ctx_lens, B, length, seen, idx, lane, b, split, nsplits)) return;
@@ -148,7 +218,8 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
     nsplits = __builtin_amdgcn_readfirstlane(nsplits);
     length = __builtin_amdgcn_readfirstlane(length);
   }
-  const int L = ctx_lens[b], first = seen.first(L);
+  if (L < 0) L = ctx_lens[b];
+  const int first = seen.first(L);
   const int t_lo = first + (cut ? split * length : 0);
   const int t_hi = cut ? min(L, t_lo + length) : L;
   const int* bt = block_tables + (long)b * MP;
