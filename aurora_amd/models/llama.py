@@ -12,7 +12,7 @@ model the engine steps directly.
 """
 from __future__ import annotations
 
-from dataclasses import dataclass
+from dataclasses import dataclass, replace
 from typing import List, Optional, Tuple
 
 import torch
@@ -63,6 +63,7 @@ class AttnMetadata:
     dec_state_slots: Optional[torch.Tensor] = None
     cu_host: Optional[List[int]] = None  # cu_seqlens_q without a device read
     ctx_host: Optional[List[int]] = None  # context_lens of the prompt portions
+    marks: Optional[torch.Tensor] = None  # ``ops.decode_marks`` of the single tokens
 
     def segments(self, T: int) -> List[ops.Segment]:
         """The step's prompt portions and its single-token rows, each with its
@@ -133,7 +134,8 @@ class LlamaAttention(nn.Module):
             )
         elif meta.mode == "decode":
             o = ops.paged_attention_decode(
-                q, k_cache, v_cache, meta.block_tables, meta.context_lens, self.scale
+                q, k_cache, v_cache, meta.block_tables, meta.context_lens, self.scale,
+                marks=meta.marks,
             )
         else:  # mixed: prefill chunks + decode tokens in one forward — the
             # projections/norms run on the whole packed batch (bigger GEMMs),
@@ -148,7 +150,7 @@ class LlamaAttention(nn.Module):
             if T > Tp:
                 ops.paged_attention_decode(
                     q[Tp:], k_cache, v_cache, meta.dec_block_tables,
-                    meta.dec_context_lens, self.scale, out=o[Tp:],
+                    meta.dec_context_lens, self.scale, out=o[Tp:], marks=meta.marks,
                 )
         return o.reshape(T, self.n_heads * self.head_dim)
 
@@ -401,6 +403,10 @@ class LlamaForCausalLM(nn.Module):
     ) -> torch.Tensor:
         x = self.embed(input_ids)
         residual = None
+        tables = {"decode": meta.block_tables, "mixed": meta.dec_block_tables}.get(meta.mode)
+        if tables is not None and kv_caches:
+            meta = replace(meta, marks=ops.decode_marks(
+                self.spec.n_heads // pdist.tp_world_size(), kv_caches[0][0], tables))
         # layers that somebody watches or has replaced are called and get no parts
         plain = [is_plain(layer, LlamaDecoderLayer) for layer in self.layers] + [True]
         for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):

@@ -174,16 +174,32 @@ def paged_attention_decode(
     context_lens: torch.Tensor,
     scale: float,
     out: Optional[torch.Tensor] = None,
+    marks: Optional[torch.Tensor] = None,
 ) -> torch.Tensor:
-    """``out``: where the results go, contiguous and shaped as ``q``."""
+    """``out``: where the results go, contiguous and shaped as ``q``; ``marks``: of
+    ``decode_marks`` for this batch."""
     if q.is_cuda:
         m = _require_hip("paged_attention_decode")
         return m.paged_attention_decode(
             q.contiguous(), k_cache, v_cache,
             block_tables.to(torch.int32), context_lens.to(torch.int32), float(scale), out,
+            marks,
         )
     y = torch_ref.paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale)
     return y if out is None else out.copy_(y)
+
+
+def decode_marks(heads: int, k_cache: torch.Tensor, block_tables: torch.Tensor,
+                 window: int = 0, chunk: int = 0) -> Optional[torch.Tensor]:
+    """Zeros by which decode attention finds out that all stretches of a context are done.
+    It leaves zeros behind, so the layers of a step, which follow each other on one stream,
+    share them. None where contexts stay whole."""
+    if not k_cache.is_cuda:
+        return None
+    n = _require_hip("decode_marks").decode_marks(
+        block_tables.shape[0], heads, k_cache.shape[1],
+        block_tables.shape[1] * k_cache.shape[2], window, chunk)
+    return torch.zeros(n, dtype=torch.int32, device=k_cache.device) if n else None
 
 
 def fused_rope_kv_write(qkv, positions, slots, cos_sin, k_cache, v_cache,

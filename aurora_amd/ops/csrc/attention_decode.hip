@@ -13,15 +13,15 @@
 //    of two;
 //  * contexts are cut into stretches of equal length, found on the device from all context
 //    lengths (``split_length``), so that a few long ones do not keep the others waiting
-//    and few sequences still fill the chip; a second kernel merges the stretches of a
-//    sequence that has several.
-// Measured in a graph, before and now (vector dot products, 64 keys at a time, as many
-// stretches for every sequence): 96 sequences of 500 to 2900 keys, 32 heads over 8,
-// 128 wide, 210 and 124 us (5.4 TB/s; a large read reaches 5.5 to 5.8), the same in fp8 211
-// and 91; 256 of 1600 326 and 289 (5.8 TB/s); 32 of 600 to 2500 66 and 43; one of 12000 102
-// and 26, one of 777 20 and 13; 7 heads over one, 40 of 300 to 3000, 90 and 37; fp8 64 wide,
-// 23 of 300 to 5000, 44 and 25. fp8 is bound by widening its values; a single sequence by
-// the two launches and one round trip to memory.
+//    and few sequences still fill the chip; the last workgroup to end merges the stretches
+//    of a sequence that has several.
+// Measured in a graph, before and now (a second kernel that merges, whole contexts in the order of
+// the batch): 96 sequences of 500 to 2900 keys, 32 heads over 8, 128 wide, 143 and 124 us (5.4
+// TB/s; a large read reaches 5.5 to 5.8), the same in fp8 86 and 82; 256 of 1600 292 (5.8 TB/s);
+// one of 12000 29.5 and 19.0, one of 777 13.3 and 10.2, 8 of 200 to 600 15.8 and 12.2; 7 heads
+// over one, 4 fp8 sequences of 3000 to 9000 27.7 and 18.8; fp8 64 wide, 23 of 300 to 5000, 27.6
+// and 24.4. A single sequence is bound by trips to memory one behind the other: lengths, pages,
+// keys, and to merge a mark and the other stretches.
 //
 // Replaces the per-token provider round-trip of the reference agent loop
 // (reference: server/chat/backend/agent/llm.py:192) with an in-process
@@ -37,7 +37,8 @@
 #define DEC_WAVES 4
 #define DEC_HEADS 16      // query heads of a workgroup
 #define DEC_SLACK 10.f    // weights stay below 2^DEC_SLACK
-#define DEC_TARGET 1024   // workgroups that the contexts are cut into
+#define DEC_TARGET 1024   // stretches that the contexts are cut into
+#define DEC_LEAST 160     // of few keys each
 
 enum { NO_BIAS = 0, LINEAR_BIAS = 1, LOG_BIAS = 2, FLAT_BIAS = 3 };
 
@@ -51,16 +52,20 @@ struct Seen {
   }
 };
 
-// Keys per stretch, a multiple of 128 (one round of the waves): what leaves about ``target``
-// stretches over all sequences and head tiles. All lanes of a wave.
-DEVINL int split_length(const int* ctx, int B, int tiles, int target, const Seen& seen,
-                        int lane) {
+// Keys per stretch, a multiple of 128 (one round of the waves): what leaves about DEC_TARGET
+// stretches over all sequences and head tiles; of less than 512 only to have DEC_LEAST of them, as
+// a stretch takes its start and many take longer to merge than they save. 8 kv heads, us with
+// stretches of at least 128, 256, 384 and 512: one sequence of 777 keys 10.1 11.0 12.0 13.0, of
+// 4000 16.1 13.2 14.0 13.9, of 12000 33 23 20 19; 8 of 300 to 1500 15.7 16.5 14.2 14.9; 16 of 1024
+// 28 21 23 21; 16 of 100 to 3000 34 34 34 30. All lanes of a wave.
+DEVINL int split_length(const int* ctx, int B, int tiles, const Seen& seen, int lane) {
   long sum = 0;
   for (int s = lane; s < B; s += WAVE) sum += ctx[s] - seen.first(ctx[s]);
 #pragma unroll
   for (int d = 32; d > 0; d >>= 1) sum += __shfl_xor(sum, d, WAVE);
-  const long per = (sum * tiles + target - 1) / target;
-  return (int)max(128L, (per + 127) / 128 * 128);
+  const long per = (sum * tiles + DEC_TARGET - 1) / DEC_TARGET;
+  const long least = min(max(sum * tiles / DEC_LEAST, 1L), 512L);
+  return (int)((max(per, least) + 127) / 128 * 128);
 }
 
 DEVINL int splits_of(int seen, int length) { return max(1, (seen + length - 1) / length); }
@@ -176,11 +181,74 @@ DEVINL void read_value_tiles(shortx4 (&v)[8], unsigned a0, unsigned a1, unsigned
       : "memory");
 }
 
+// Numbers that workgroups on different XCDs hand each other go past the L2s, each of which
+// knows only its own: made known by a fence instead, every workgroup would write its whole L2
+// back and drop it (23 sequences of 300 to 5000 keys 27 and 60 us).
+DEVINL void hand_over(float* p, float x) {
+  __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+DEVINL float handed(const float* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Results of two heads, h by half a wave, from the n stretches of their sequence, ``src`` the
+// first one's. 32 references and sums are read at once, and the first results with them.
+template <int DV, bool TURNS>
+DEVINL void merge_stretches(const float* src, long step, int n, int lane, __hip_bfloat16* out,
+                            int b, int h, int L, long ostride, int dv, float oscale,
+                            const float* sink, const HeadTurn& turn) {
+  constexpr int N = DV / 32, AT_ONCE = 8;
+  const int col = lane & 31;
+  float M = sink ? fmaxf(sink[h] * LOG2E, -1e30f) : -1e30f, Lsum = sink ? 1.f : 0.f, O[N] = {};
+  for (int s0 = 0; s0 < n; s0 += 32) {
+    float o[AT_ONCE][N];
+    auto read = [&](int first) {
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k)
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          o[k][j] = handed(src + min(first + k, n - 1) * step + col + j * 32);
+    };
+    const float* ref = src + min(s0 + col, n - 1) * step + DV;
+    const float m = s0 + col < n ? handed(ref) : -1e30f, l = s0 + col < n ? handed(ref + 1) : 0.f;
+    read(s0);
+    float most = m;
+#pragma unroll
+    for (int d = 16; d > 0; d >>= 1) most = fmaxf(most, __shfl_xor(most, d, WAVE));
+    const float Mn = fmaxf(M, most), alpha = __builtin_amdgcn_exp2f(M - Mn);
+    M = Mn;
+    const float f = s0 + col < n ? __builtin_amdgcn_exp2f(m - M) : 0.f;
+    float sum = f * l;
+#pragma unroll
+    for (int d = 16; d > 0; d >>= 1) sum += __shfl_xor(sum, d, WAVE);
+    Lsum = Lsum * alpha + sum;
+#pragma unroll
+    for (int j = 0; j < N; ++j) O[j] *= alpha;
+    for (int s = s0; s < min(s0 + 32, n); s += AT_ONCE) {
+      if (s > s0) read(s);
+#pragma unroll
+      for (int k = 0; k < AT_ONCE; ++k) {
+        const float fk = __shfl(f, (lane & 32) + (s - s0 + k), WAVE);
+#pragma unroll
+        for (int j = 0; j < N; ++j)
+          if (s + k < n) O[j] += fk * o[k][j];
+      }
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    const int d = col + j * 32;
+    float y = O[j] / Lsum * oscale;
+    if constexpr (TURNS) y = turned<bf16_t>(turn, y, b, L - 1, h, d, dv);
+    if (d < dv) *(unsigned short*)(out + b * ostride + (long)h * dv + d) = f32_to_bf16(y);
+  }
+}
+
 // BIAS: a distance penalty per head or none (see attention_prefill.hip), a window or
 // chunks of positions; sink: one more term of the denominator per head, or null;
 // FLAT_BIAS results may be turned back and gated. PAGED: pages are whole tiles.
-// Without ``cut`` a workgroup takes a whole context.
-template <int D, int DV, bool FP8, int BIAS, bool PAGED>
+// Without CUT a workgroup takes a whole context.
+template <int D, int DV, bool FP8, int BIAS, bool PAGED, bool CUT>
 __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
     const __hip_bfloat16* __restrict__ q,   // [B, Hq, D]
     // (not __restrict__: loads of them must stay before the waits that count them)
@@ -188,9 +256,10 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
     const void* vc,
     __hip_bfloat16* out,                    // [B, ostride], heads dv apart
     float* part,                            // [stretches, Hq, DV + 2], where a context has several
+    int* arrived,                           // [B, head tiles] zeros, and again at the end
     const int* __restrict__ block_tables,   // [B, MP]
     const int* __restrict__ ctx_lens,       // [B]
-    int B, int Hq, int Hkv, int P, int MP, int cut, float scale,
+    int B, int Hq, int Hkv, int P, int MP, float scale,
     long ostride, int dv, float oscale,
     const float* __restrict__ slopes, const float* __restrict__ rates, Seen seen,
     const float* __restrict__ sink, HeadTurn turn) {
@@ -205,12 +274,16 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
   const int kvh = tile / NG, h0 = kvh * G + tile % NG * DEC_HEADS;
   const int GT = min(DEC_HEADS, kvh * G + G - h0);
   int b = idx, split = 0, nsplits = 1, length = 0x7fffffff, L = -1;
-  if (!cut && seen.window <= 0 && seen.chunk <= 0) {
+  // LDS: a tile of values per wave; at the end the waves' results
+  __shared__ __attribute__((aligned(16))) char smem[DEC_WAVES * STAGE];
+  __shared__ float s_m[DEC_WAVES][DEC_HEADS], s_l[DEC_WAVES][DEC_HEADS];
+  static_assert(sizeof(smem) >= DEC_WAVES * DEC_HEADS * DV * 4);
+  if (!CUT && seen.window <= 0 && seen.chunk <= 0) {
     if (B <= 2 * WAVE) b = ranked<2>(ctx_lens, B, idx, lane, L);
     else if (B <= 4 * WAVE) b = ranked<4>(ctx_lens, B, idx, lane, L);
   }
-  if (cut) {
-    length = split_length(ctx_lens, B, tiles, DEC_TARGET, seen, lane);
+  if (CUT) {
+    length = split_length(ctx_lens, B, tiles, seen, lane);
     if (!find_split(ctx_lens, B, length, seen, idx, lane, b, split, nsplits)) return;
     // the same in all lanes, which the compiler cannot see
     b = __builtin_amdgcn_readfirstlane(b);
@@ -220,16 +293,12 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
   }
   if (L < 0) L = ctx_lens[b];
   const int first = seen.first(L);
-  const int t_lo = first + (cut ? split * length : 0);
-  const int t_hi = cut ? min(L, t_lo + length) : L;
+  const int t_lo = first + (CUT ? split * length : 0);
+  const int t_hi = CUT ? min(L, t_lo + length) : L;
   const int* bt = block_tables + (long)b * MP;
   const int head = lane & 15, g = lane >> 4;
   const bool mine = head < GT;
 
-  // LDS: a tile of values per wave; at the end the waves' results
-  __shared__ __attribute__((aligned(16))) char smem[DEC_WAVES * STAGE];
-  __shared__ float s_m[DEC_WAVES][DEC_HEADS], s_l[DEC_WAVES][DEC_HEADS];
-  static_assert(sizeof(smem) >= DEC_WAVES * DEC_HEADS * DV * 4);
   char* ring = smem + wave * STAGE;
   const unsigned ring_at =
       (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring;
@@ -451,58 +520,45 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
     } else {
       // an un-normalised partial result, its reference and its sum
       float* dst = part + ((long)idx * Hq + h0 + hh) * (DV + 2);
-      dst[d] = O;
+      hand_over(dst + d, O);
       if (d == 0) {
-        dst[DV] = M;
-        dst[DV + 1] = Lsum;
+        hand_over(dst + DV, M);
+        hand_over(dst + DV + 1, Lsum);
       }
     }
   }
+  if (nsplits == 1) return;
+  // The last workgroup of the sequence's head tile to come here merges its stretches: all
+  // waves' results have left the CU before one thread makes them known and learns of others'.
+  __shared__ int s_last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int* mark = arrived + (long)b * tiles + tile;
+    const int before =
+        __hip_atomic_fetch_add(mark, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_last = before == nsplits - 1;
+    if (s_last) *mark = 0;
+  }
+  __syncthreads();
+  if (!s_last) return;
+  for (int hh = 2 * wave + lane / 32; hh < GT; hh += 2 * DEC_WAVES)
+    merge_stretches<DV, BIAS == FLAT_BIAS>(part + ((long)(idx - split) * Hq + h0 + hh) * (DV + 2),
+                                           (long)Hq * (DV + 2), nsplits, lane, out, b, h0 + hh, L,
+                                           ostride, dv, oscale, BIAS ? sink : nullptr, turn);
 }
 
-// Merges the stretches of a sequence that has several; a wave per (sequence, head). All
-// references are read at once, then the results in groups of independent loads.
-template <int DV>
-__global__ __launch_bounds__(256) void decode_combine_kernel(
-    const float* __restrict__ part, __hip_bfloat16* __restrict__ out,
-    const int* __restrict__ ctx_lens, int B, int Hq, int tiles, long ostride, int dv,
-    float oscale, const float* __restrict__ sink, HeadTurn turn, Seen seen) {
-  const long bh = blockIdx.x * 4L + threadIdx.x / WAVE;
-  if (bh >= (long)B * Hq) return;
-  const int lane = threadIdx.x % WAVE, b = bh / Hq, h = bh % Hq;
-  const int length = split_length(ctx_lens, B, tiles, DEC_TARGET, seen, lane);
-  const int n = splits_of(ctx_lens[b] - seen.first(ctx_lens[b]), length);
-  if (n == 1) return;
-  int before = 0;  // stretches of the sequences before this
-  for (int s = lane; s < b; s += WAVE)
-    before += splits_of(ctx_lens[s] - seen.first(ctx_lens[s]), length);
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) before += __shfl_xor(before, d, WAVE);
-  const float* src = part + ((long)before * Hq + h) * (DV + 2);
-  const long step = (long)Hq * (DV + 2);
-  const float s0 = sink ? fmaxf(sink[h] * LOG2E, -1e30f) : -1e30f;
-  float M = s0;
-  for (int s = lane; s < n; s += WAVE) M = fmaxf(M, src[s * step + DV]);
-  M = wave_max(M);
-  float Lsum = 0.f;
-  for (int s = lane; s < n; s += WAVE)
-    Lsum += __builtin_amdgcn_exp2f(src[s * step + DV] - M) * src[s * step + DV + 1];
-  Lsum = wave_sum(Lsum) + (sink ? __builtin_amdgcn_exp2f(s0 - M) : 0.f);
-  constexpr int N = DV / WAVE;
-  float O[N] = {};
-#pragma unroll 8
-  for (int s = 0; s < n; ++s) {
-    const float f = __builtin_amdgcn_exp2f(src[s * step + DV] - M);
-#pragma unroll
-    for (int j = 0; j < N; ++j) O[j] += f * src[s * step + lane + j * WAVE];
-  }
-#pragma unroll
-  for (int j = 0; j < N; ++j) {
-    const int d = lane + j * WAVE;
-    float y = O[j] / Lsum * oscale;
-    if (turn.cs || turn.gate) y = turned<bf16_t>(turn, y, b, ctx_lens[b] - 1, h, d, dv);
-    if (d < dv) *(unsigned short*)(out + b * ostride + (long)h * dv + d) = f32_to_bf16(y);
-  }
+// Marks that a call wants for its sequences' head tiles, or 0 where contexts stay whole: while
+// the longest that can be seen is short or the workgroups are many, cutting costs its search
+// and the merge, and evens out little. Whole and cut, 128 wide, 8 kv heads: 64 sequences of 2000
+// keys 100 and 110 us, 100 of 50 keys 7 and 13; behind a window of 1024, 32 sequences 30 and 40,
+// 16 sequences 19 and 27, 2 sequences (outside the rule) 16 and 13. What it gives up: 64
+// sequences of 300 to 8000 keys 229 and 215.
+long decode_marks(long B, long Hq, long Hkv, long longest, long window, long chunk) {
+  const long tiles = Hkv * ((Hq / Hkv + DEC_HEADS - 1) / DEC_HEADS);
+  if (window > 0) longest = std::min(longest, window);
+  if (chunk > 0) longest = std::min(longest, chunk);
+  return longest > std::max<long>(256, B * tiles * B * tiles / 16) ? B * tiles : 0;
 }
 
 template <int D, int DV, bool FP8, int BIAS>
@@ -511,44 +567,42 @@ static void decode_launch(const torch::Tensor& q, const torch::Tensor& kc,
                           const torch::Tensor& ctx, __hip_bfloat16* out, long ostride,
                           int dv, float scale, float oscale, const float* slopes,
                           const float* rates, int window, int chunk, const float* sink,
-                          const HeadTurn& turn) {
+                          const HeadTurn& turn,
+                          const c10::optional<torch::Tensor>& marks) {
   const int B = q.size(0), Hq = q.size(1);
   const int Hkv = kc.size(1), P = kc.size(2), MP = bt.size(1);
   const int tiles = Hkv * ((Hq / Hkv + DEC_HEADS - 1) / DEC_HEADS);
-  // Contexts stay whole while the longest that can be seen is short or the workgroups are
-  // many: cutting costs its search and the second kernel, and evens out little then. Whole
-  // and cut, 128 wide, 8 kv heads: 64 sequences of 2000 keys 100 and 110 us, 100 of 50 keys
-  // 7 and 13; behind a window of 1024, 32 sequences 30 and 40, 16 sequences 19 and 27, 2
-  // sequences (outside the rule) 16 and 13. What it gives up: 64 sequences of 300 to 8000
-  // keys 229 and 215.
-  long longest = (long)MP * P;
-  if (window > 0) longest = std::min<long>(longest, window);
-  if (chunk > 0) longest = std::min<long>(longest, chunk);
-  const bool cut = longest > std::max<long>(256, (long)B * tiles * B * tiles / 16);
+  const bool cut = decode_marks(B, Hq, Hkv, (long)MP * P, window, chunk) > 0;
   const long most = cut ? B + DEC_TARGET / tiles + 1 : B;  // stretches there can be
-  torch::Tensor part;
-  if (cut) part = torch::empty({most, Hq, DV + 2}, q.options().dtype(torch::kFloat32));
+  torch::Tensor part, arrived;
+  if (cut) {
+    part = torch::empty({most, Hq, DV + 2}, q.options().dtype(torch::kFloat32));
+    const bool fit = marks && marks->dtype() == torch::kInt32 && marks->device() == q.device() &&
+                     marks->is_contiguous() && marks->numel() >= (long)B * tiles;
+    arrived = fit ? *marks : torch::zeros({(long)B * tiles}, ctx.options());
+  }
   float* pp = cut ? part.data_ptr<float>() : nullptr;
   const Seen seen = {window, chunk};
   auto launch = [&](auto kern) {
     hipLaunchKernelGGL(kern, dim3(most * tiles), dim3(256), 0, CUR_STREAM,
                        (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out,
-                       pp, bt.data_ptr<int>(), ctx.data_ptr<int>(), B, Hq, Hkv, P, MP,
-                       cut ? 1 : 0, scale, ostride, dv, oscale, slopes, rates, seen, sink, turn);
+                       pp, cut ? arrived.data_ptr<int>() : nullptr, bt.data_ptr<int>(),
+                       ctx.data_ptr<int>(), B, Hq, Hkv, P, MP,
+                       scale, ostride, dv, oscale, slopes, rates, seen, sink, turn);
   };
-  if (P % DEC_KEYS == 0) launch(paged_decode_kernel<D, DV, FP8, BIAS, true>);
-  else launch(paged_decode_kernel<D, DV, FP8, BIAS, false>);
-  if (cut)
-    hipLaunchKernelGGL((decode_combine_kernel<DV>), dim3(((long)B * Hq + 3) / 4), dim3(256), 0,
-                       CUR_STREAM, pp, out, ctx.data_ptr<int>(), B, Hq, tiles, ostride, dv,
-                       oscale, sink, turn, seen);
+  const bool paged = P % DEC_KEYS == 0;
+  if (paged && cut) launch(paged_decode_kernel<D, DV, FP8, BIAS, true, true>);
+  else if (paged) launch(paged_decode_kernel<D, DV, FP8, BIAS, true, false>);
+  else if (cut) launch(paged_decode_kernel<D, DV, FP8, BIAS, false, true>);
+  else launch(paged_decode_kernel<D, DV, FP8, BIAS, false, false>);
   HIP_CHECK_KERNEL();
 }
 
 torch::Tensor paged_attention_decode(torch::Tensor q, torch::Tensor kc,
                                      torch::Tensor vc, torch::Tensor bt,
                                      torch::Tensor ctx, double scale,
-                                     c10::optional<torch::Tensor> into) {
+                                     c10::optional<torch::Tensor> into,
+                                     c10::optional<torch::Tensor> marks) {
   TORCH_CHECK(q.is_cuda() && q.dtype() == torch::kBFloat16, "bf16 GPU only");
   const int B = q.size(0), Hq = q.size(1), D = q.size(2), Hkv = kc.size(1);
   TORCH_CHECK(Hq % Hkv == 0, "GQA requires Hq % Hkv == 0");
@@ -560,7 +614,7 @@ torch::Tensor paged_attention_decode(torch::Tensor q, torch::Tensor kc,
   const bool fp8 = kc.dtype() == torch::kFloat8_e4m3fn;
 #define RUN(DD, F8) \
   decode_launch<DD, DD, F8, NO_BIAS>(q, kc, vc, bt, ctx, o, stride, D, (float)scale, \
-                                     1.f, nullptr, nullptr, 0, 0, nullptr, HeadTurn{})
+                                     1.f, nullptr, nullptr, 0, 0, nullptr, HeadTurn{}, marks)
   if (D == 128) { if (fp8) RUN(128, true); else RUN(128, false); }
   else { if (fp8) RUN(64, true); else RUN(64, false); }
 #undef RUN
@@ -574,7 +628,8 @@ void biased_attention_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc
                              c10::optional<torch::Tensor> sink,
                              c10::optional<torch::Tensor> turn,
                              c10::optional<torch::Tensor> gate, torch::Tensor out,
-                             long col, long dv, double oscale) {
+                             long col, long dv, double oscale,
+                             c10::optional<torch::Tensor> marks) {
   TORCH_CHECK(q.is_cuda() && q.dtype() == torch::kBFloat16 && q.is_contiguous());
   const int B = q.size(0), Hq = q.size(1), D = q.size(2);
   const int Hkv = kc.size(1), DV = vc.size(3);
@@ -597,7 +652,7 @@ void biased_attention_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc
 #define RUN1(DD, DVV, BB)                                                        \
   decode_launch<DD, DVV, false, BB>(q, kc, vc, bt, ctx, o, out.stride(0),        \
                                     (int)dv, (float)scale, (float)oscale,        \
-                                    sp, rp, (int)window, (int)chunk, snk, ht)
+                                    sp, rp, (int)window, (int)chunk, snk, ht, marks)
 #define RUN(DD, DVV)                         \
   if (!sp) RUN1(DD, DVV, FLAT_BIAS);         \
   else if (rp) RUN1(DD, DVV, LOG_BIAS);      \

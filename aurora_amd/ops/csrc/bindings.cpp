@@ -12,7 +12,9 @@ void kv_cache_write(torch::Tensor k, torch::Tensor v, torch::Tensor kc,
 torch::Tensor paged_attention_decode(torch::Tensor q, torch::Tensor kc,
                                      torch::Tensor vc, torch::Tensor bt,
                                      torch::Tensor ctx, double scale,
-                                     c10::optional<torch::Tensor> into);
+                                     c10::optional<torch::Tensor> into,
+                                     c10::optional<torch::Tensor> marks);
+long decode_marks(long B, long Hq, long Hkv, long longest, long window, long chunk);
 torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
                                       torch::Tensor vc, torch::Tensor bt,
                                       torch::Tensor cu_q, torch::Tensor ctx,
@@ -91,7 +93,8 @@ void biased_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
 void biased_attention_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
                              torch::Tensor bt, torch::Tensor ctx, double scale, long window,
                              long chunk, OptT slopes, OptT rates, OptT sink, OptT turn,
-                             OptT gate, torch::Tensor out, long col, long dv, double oscale);
+                             OptT gate, torch::Tensor out, long col, long dv, double oscale,
+                             OptT marks);
 void biased_attention_rows(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
                            torch::Tensor bt, OptT cu, torch::Tensor ctx, OptT row_seq,
                            OptT row_off, double scale, long window, long chunk, OptT slopes,
@@ -179,7 +182,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("silu_mul", &silu_mul, "fused SiLU(gate)*up");
   m.def("rope_apply_", &rope_apply_, "in-place RoPE on q/k");
   m.def("kv_cache_write", &kv_cache_write, "scatter K/V into paged cache");
-  m.def("paged_attention_decode", &paged_attention_decode, "paged GQA decode attention");
+  m.def("paged_attention_decode", &paged_attention_decode, "paged GQA decode attention",
+        py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("bt"), py::arg("ctx"),
+        py::arg("scale"), py::arg("into") = py::none(), py::arg("marks") = py::none());
+  m.def("decode_marks", &decode_marks,
+        "zeros that decode attention wants to merge stretches of contexts, 0 for none");
   m.def("attention_prefill_paged", &attention_prefill_paged,
         "MFMA flash prefill over paged KV");
   m.def("skinny_gemm", &skinny_gemm, "decode-path skinny GEMM (M<=64)");
@@ -224,7 +231,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("biased_attention_prefill", &biased_attention_prefill,
         "MFMA flash prefill with distance bias, window or chunks, sink, turn and gate");
   m.def("biased_attention_decode", &biased_attention_decode,
-        "paged decode with distance bias, window or chunks, sink, turn and gate");
+        "paged decode with distance bias, window or chunks, sink, turn and gate",
+        py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("bt"), py::arg("ctx"),
+        py::arg("scale"), py::arg("window"), py::arg("chunk"), py::arg("slopes"),
+        py::arg("rates"), py::arg("sink"), py::arg("turn"), py::arg("gate"), py::arg("out"),
+        py::arg("col"), py::arg("dv"), py::arg("oscale"), py::arg("marks") = py::none());
   m.def("biased_attention_rows", &biased_attention_rows,
         "any head width / float32 attention with distance bias, window or chunks, sink, "
         "turn and gate");

@@ -219,6 +219,16 @@ class Segment:
     def decode(self) -> bool:
         return self.cu is None
 
+    def decode_marks(self, heads: int, k_cache, window: int, chunk: int):
+        """``ops.decode_marks`` of these rows, the same for all layers alike; a graph that is
+        being captured has its own."""
+        from . import decode_marks
+        key = (heads, k_cache.shape[1:3], window, chunk,
+               k_cache.is_cuda and torch.cuda.is_current_stream_capturing())
+        if key not in self._maps:
+            self._maps[key] = decode_marks(heads, k_cache, self.block_tables, window, chunk)
+        return self._maps[key]
+
     def cu_or_rows(self, n: int) -> torch.Tensor:
         if self.cu is not None:
             return self.cu
@@ -579,7 +589,8 @@ def biased_attention(q, k_cache, v_cache, seg: Segment, scale, window, slopes,
               and v_cache.shape[3] in MATRIX_HEAD_DIMS)
     if matrix and seg.decode:
         m.biased_attention_decode(qs, k_cache, v_cache, seg.block_tables,
-                                  seg.context_lens, *extra)
+                                  seg.context_lens, *extra,
+                                  seg.decode_marks(q.shape[1], k_cache, window, chunk))
     elif matrix:
         rows = m.biased_prefill_rows(q.shape[1] // k_cache.shape[1])
         bseq, boff = seg.block_map(rows, chunk)
