@@ -214,20 +214,11 @@ class LLMEngine:
         self.kv.on_cache_evict = self._drop_page_hash
         self.gen = torch.Generator(device="cpu").manual_seed(config.seed)
         self._graph_cache: Dict[int, tuple] = {}
+        self._staged_keys: Dict[int, torch.Tensor] = {}
         self._graph_pool = None
         if self._graphs_enabled():
-            # reserve the idle-row scratch page + host staging now,
-            # while the cache is guaranteed non-full
-            mp = (self.max_model_len + self.kv.page_size - 1) // self.kv.page_size
-            self._scratch_page = self.kv.alloc(1)[0]
-            self._scratch_slot = self._scratch_page * self.kv.page_size
-            maxb = self._BUCKETS[-1]
-            # zeros: rows that no sequence has filled yet are idle rows' token ids
-            self._host_i64 = torch.zeros(maxb, dtype=torch.int64)
-            self._host_i32 = torch.empty(maxb, 4, dtype=torch.int32)
-            self._host_bt = torch.full((maxb, mp), self._scratch_page, dtype=torch.int32)
-            self._bt_staged = [None] * maxb
-        self._dec_staged_ids = None
+            # now, while the cache is guaranteed non-full
+            self._reserve_scratch()
         # counters (engine observability; surfaced by service.metrics)
         self.counters = {
             "prompt_tokens": 0, "generated_tokens": 0, "prefill_steps": 0,
@@ -599,13 +590,12 @@ class LLMEngine:
                 logits = logits[torch.tensor(rows, dtype=torch.long, device=dev)] \
                     if rows else None
         else:
-            self._dec_staged_ids = None
             input_ids, meta = self._build_batch(prefill, chunks, decode)
             hidden = self.model(input_ids, self.kv.caches, meta)
             logits = None
             if rows:
                 picked = hidden if rows == list(range(hidden.shape[0])) else \
-                    hidden[torch.tensor(rows, dtype=torch.long, device=dev)]
+                    hidden[self._row_index(rows)]
                 logits = self.model.compute_logits(picked)
         if dev != "cpu":
             torch.cuda.synchronize()
@@ -616,6 +606,12 @@ class LLMEngine:
         for seq in decode:
             seq.num_cached = seq.num_tokens
         return logits
+
+    def _row_index(self, rows: List[int]) -> torch.Tensor:
+        # (a copy from ordinary memory would wait for the end of the forward, and the
+        # product behind it would be launched with the GPU idle)
+        made = None if self.device == "cpu" else ops.pack_rows(rows, self.device)
+        return torch.tensor(rows, dtype=torch.long, device=self.device) if made is None else made
 
     def _build_batch(self, prefill: List[Sequence], chunks: List[int],
                      decode: List[Sequence]):
@@ -729,85 +725,55 @@ class LLMEngine:
         and are ignored).  Removes the per-layer kernel-launch host time
         that dominates small-batch decode.
 
-        Staging is incremental: when the batch membership is unchanged
-        since the previous graph decode, position/slot/context rows each
-        advance by exactly one token, so the staging matrix gets a
-        single vectorized += 1 instead of three B-element Python list
-        builds (only page-boundary rows re-derive their slot); any
-        prefill/mixed/eager step invalidates the staged state."""
+        The inputs are staged in native code; a block table's row is
+        rewritten only when its sequence or its pages have changed."""
         B = len(seqs)
         bucket = next(b for b in self._BUCKETS if b >= B)
         g = self._graph_cache.get(bucket)
         if g is None:
             g = self._capture_decode_graph(bucket)
             self._graph_cache[bucket] = g
+            # (serial, page generation, pages) of every table's row; -1: an idle row's
+            self._staged_keys[bucket] = torch.full((bucket, 3), -1, dtype=torch.int64)
         graph, inputs, host_inputs, staged_parts, out_logits = g
-        mp = staged_parts[2].shape[1]
-        P = self.kv.page_size
-        ids_t = self._host_i64
-        ids_t[:B] = torch.tensor([s.token_ids[-1] for s in seqs],
-                                 dtype=torch.int64)
-        pos = self._host_i32
-        batch_ids = [(s.serial, s.page_gen) for s in seqs]
-        if batch_ids == self._dec_staged_ids:
-            pos[:B, :3] += 1  # position, slot and context advance one token
-            for i, s in enumerate(seqs):
-                if (s.num_tokens - 1) % P == 0:  # slot jumped to a new page
-                    pos[i, 1] = self._slot(s, s.num_tokens - 1)
-        else:
-            pos[:B, 0] = torch.tensor([s.num_tokens - 1 for s in seqs],
-                                      dtype=torch.int32)
-            pos[B:bucket, 0] = 0
-            # note: the last token was appended by sampling but its KV is
-            # not yet written; it is this step's input token.
-            pos[:B, 1] = torch.tensor(
-                [self._slot(s, s.num_tokens - 1) for s in seqs],
-                dtype=torch.int32)
-            pos[B:bucket, 1] = self._scratch_slot
-            pos[:B, 2] = torch.tensor([s.num_tokens for s in seqs],
-                                      dtype=torch.int32)
-            pos[B:bucket, 2] = 1
-            pos[:B, 3] = torch.tensor([s.state_slot for s in seqs],
-                                      dtype=torch.int32)
-            pos[B:bucket, 3] = -1  # idle rows touch no state
-            self._dec_staged_ids = batch_ids
-        # block-table rows change only on page append / batch-slot change:
-        # rewrite a staged row only when its (seq, npages) key moved
-        bt_host = self._host_bt
-        staged = self._bt_staged
-        for i, s in enumerate(seqs):
-            key = (s.serial, s.page_gen, len(s.pages))
-            if staged[i] != key:
-                n = min(len(s.pages), mp)
-                bt_host[i, :n] = torch.tensor(s.pages[:n], dtype=torch.int32)
-                bt_host[i, n:] = self._scratch_page
-                staged[i] = key
-        for i in range(len(seqs), bucket):
-            if staged[i] is not None:
-                bt_host[i].fill_(self._scratch_page)
-                staged[i] = None
-        # one copy: ids, positions, slots, contexts, states, tables side by side
-        host_ids, host_rows, host_bt = staged_parts
-        host_ids.copy_(ids_t[:bucket])
-        host_rows.copy_(pos[:bucket].t())
-        host_bt.copy_(bt_host[:bucket])
-        inputs.copy_(host_inputs, non_blocking=True)
+        keys, width = self._staged_keys[bucket], staged_parts[2].shape[1]
+        if not ops.stage_decode(seqs, self._host_i64, host_inputs, keys, inputs, width,
+                                self.kv.page_size, self._scratch_page, self._scratch_slot):
+            self._stage_decode(seqs, staged_parts, keys)
+            inputs.copy_(host_inputs, non_blocking=True)
         graph.replay()
         return out_logits[:B]
+
+    def _stage_decode(self, seqs: List[Sequence], parts, keys: torch.Tensor) -> None:
+        """``ops.stage_decode`` of whatever a sequence may hold."""
+        ids, (pos, slot, ctx, state), tables = parts
+        B, width = len(seqs), tables.shape[1]
+        self._host_i64[:B] = torch.tensor([s.token_ids[-1] for s in seqs], dtype=torch.int64)
+        ids.copy_(self._host_i64[:len(ids)])
+        for row, idle, own in (
+                (pos, 0, [s.num_tokens - 1 for s in seqs]),
+                (slot, self._scratch_slot, [self._slot(s, s.num_tokens - 1) for s in seqs]),
+                (ctx, 1, [s.num_tokens for s in seqs]), (state, -1, [s.state_slot for s in seqs])):
+            row[:B] = torch.tensor(own, dtype=torch.int32)
+            row[B:] = idle
+        tables.fill_(self._scratch_page)
+        for row, s in zip(tables, seqs):
+            n = min(len(s.pages), width)
+            row[:n] = torch.tensor(s.pages[:n], dtype=torch.int32)
+        keys[:B], keys[B:] = -2, -1
+
+    def _reserve_scratch(self) -> None:
+        """The page that idle rows of captured batches write, and the staged token ids."""
+        self._scratch_page = self.kv.alloc(1)[0]
+        self._scratch_slot = self._scratch_page * self.kv.page_size
+        # zeros: rows that no sequence has filled yet are idle rows' token ids
+        self._host_i64 = torch.zeros(self._BUCKETS[-1], dtype=torch.int64)
 
     def _capture_decode_graph(self, bucket: int):
         dev = self.device
         mp = (self.max_model_len + self.kv.page_size - 1) // self.kv.page_size
         if not hasattr(self, "_scratch_page"):
-            self._scratch_page = self.kv.alloc(1)[0]
-            self._scratch_slot = self._scratch_page * self.kv.page_size
-            maxb = self._BUCKETS[-1]
-            # zeros: rows that no sequence has filled yet are idle rows' token ids
-            self._host_i64 = torch.zeros(maxb, dtype=torch.int64)
-            self._host_i32 = torch.empty(maxb, 4, dtype=torch.int32)
-            self._host_bt = torch.full((maxb, mp), self._scratch_page, dtype=torch.int32)
-            self._bt_staged = [None] * maxb
-        self._dec_staged_ids = None
+            self._reserve_scratch()
 
         def parts(buffer):  # ids; positions, slots, contexts and states; tables
             ids, rest = buffer[:bucket], buffer[bucket:].view(torch.int32)

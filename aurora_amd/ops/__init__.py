@@ -300,6 +300,17 @@ def pack_batch(ids, first, end, pages, states, prompts: int, page: int, device):
                                                  torch.device(device))
 
 
+def pack_rows(rows, device):
+    """A list of plain integers on the GPU, without waiting for what runs there, or None."""
+    return _require_hip("pack_rows").pack_rows(list(rows), torch.device(device))
+
+
+def stage_decode(seqs, ids, host, keys, inputs, width, page, scratch_page, scratch_slot) -> bool:
+    """A captured decode step's inputs from its sequences, or False as ``pack_batch``."""
+    return _require_hip("stage_decode").stage_decode(
+        list(seqs), ids, host, keys, inputs, width, page, scratch_page, scratch_slot)
+
+
 def pack_texts(texts, most: int, device):
     """Ids, begins and positions of texts on the GPU, or None as ``pack_batch``."""
     return _require_hip("pack_texts").pack_texts(texts, most, torch.device(device))

@@ -175,6 +175,10 @@ py::object pack_batch(py::list ids, std::vector<long> first, std::vector<long> e
                       py::list pages, std::vector<long> states, long prompts, long page,
                       torch::Device device);
 py::object pack_texts(py::list texts, long most, torch::Device device);
+py::object pack_rows(py::list rows, torch::Device device);
+bool stage_decode(py::list seqs, torch::Tensor ids, torch::Tensor host, torch::Tensor keys,
+                  torch::Tensor inputs, long width, long page, long scratch_page,
+                  long scratch_slot);
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("rmsnorm", &rmsnorm, "fused RMSNorm (bf16, gfx950)");
@@ -263,6 +267,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "head norms + rotation + temperature + paged KV scatter");
   m.def("pack_batch", &pack_batch, "a step's batch from lists, in one copy");
   m.def("pack_texts", &pack_texts, "texts to embed from lists, in one copy");
+  m.def("pack_rows", &pack_rows, "integers to the device without waiting");
+  m.def("stage_decode", &stage_decode, "the inputs of a captured decode step, in one copy");
   m.def("gelu", &gelu, "exact gelu");
   m.def("relu2", &relu2, "squared relu");
   m.def("silu_glu", &silu_glu, "silu(gate) * up");
