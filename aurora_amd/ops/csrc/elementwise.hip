@@ -40,8 +40,10 @@ DEVINL void add_parts8(float (&y)[8], const float* x, int parts, long step) {
 // product left in parts is so added up where it is read anyway: 96 rows of 4096 in 4 parts
 // 3.5 us, 23 rows of 2048 in 8 parts 3.3; of a whole product 3.4 and 2.6, after a kernel to
 // add its parts that takes 2.4 to 4.7.
-template <bool RESIDUAL, bool PARTS = false>
-__global__ __launch_bounds__(1024) void rmsnorm_kernel(
+// N: vectors of eight that a thread holds, so that a row is read once and the weight comes with
+// it; 0 for rows too long for that, which are read again.
+template <bool RESIDUAL, bool PARTS, int N>
+__global__ __launch_bounds__(PARTS ? 1024 : 256) void rmsnorm_kernel(
     const std::conditional_t<PARTS, float, __hip_bfloat16>* __restrict__ x,
     const __hip_bfloat16* __restrict__ res,
     __hip_bfloat16* __restrict__ out,
@@ -53,53 +55,67 @@ __global__ __launch_bounds__(1024) void rmsnorm_kernel(
   const int tid = threadIdx.x;
   const int nthr = blockDim.x;
   __shared__ float s_partial[16];
-  __shared__ float s_inv;
 
+  shortx8 held[N > 0 ? N : 1], scale[N > 0 ? N : 1];
+  if constexpr (N > 0)
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if ((tid + k * nthr) * 8 < H)
+        scale[k] = *reinterpret_cast<const shortx8*>(weight + (tid + k * nthr) * 8);
   float ss = 0.f;
   // each thread strides over the row in 8-element vectors
-  for (int i = tid * 8; i < H; i += nthr * 8) {
+  auto add = [&](int i, shortx8& kept) {
     float vals[8];
     if constexpr (PARTS) {
       add_parts8(vals, x + base + i, parts, step);
     } else {
-      shortx8 v = *reinterpret_cast<const shortx8*>(x + base + i);
+      kept = *reinterpret_cast<const shortx8*>(x + base + i);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) vals[j] = bf16_to_f32((unsigned short)v[j]);
+      for (int j = 0; j < 8; ++j) vals[j] = bf16_to_f32((unsigned short)kept[j]);
     }
     if (RESIDUAL) {
       shortx8 r = *reinterpret_cast<const shortx8*>(res + base + i);
-      shortx8 sum;
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
         vals[j] += bf16_to_f32((unsigned short)r[j]);
-        sum[j] = (short)f32_to_bf16(vals[j]);
+        kept[j] = (short)f32_to_bf16(vals[j]);
       }
-      *reinterpret_cast<shortx8*>(res_out + base + i) = sum;
+      *reinterpret_cast<shortx8*>(res_out + base + i) = kept;
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j) ss += vals[j] * vals[j];
+  };
+  if constexpr (N > 0) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if ((tid + k * nthr) * 8 < H) add((tid + k * nthr) * 8, held[k]);
+  } else {
+    for (int i = tid * 8; i < H; i += nthr * 8) add(i, held[0]);
   }
   ss = wave_sum(ss);
   const int wid = tid / WAVE, lid = tid % WAVE;
   if (lid == 0) s_partial[wid] = ss;
   __syncthreads();
-  if (tid == 0) {
-    float t = 0.f;
-    for (int w = 0; w < nthr / WAVE; ++w) t += s_partial[w];
-    s_inv = rsqrtf(t / H + eps);
-  }
-  __syncthreads();
-  const float inv = s_inv;
-  const __hip_bfloat16* src = RESIDUAL ? res_out : (const __hip_bfloat16*)x;
-  for (int i = tid * 8; i < H; i += nthr * 8) {
-    shortx8 v = *reinterpret_cast<const shortx8*>(src + base + i);
-    shortx8 w = *reinterpret_cast<const shortx8*>(weight + i);
+  float all = 0.f;
+  for (int w = 0; w < nthr / WAVE; ++w) all += s_partial[w];
+  const float inv = rsqrtf(all / H + eps);
+  auto write = [&](int i, const shortx8& v, const shortx8& w) {
     shortx8 o;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       o[j] = (short)f32_to_bf16(bf16_to_f32((unsigned short)v[j]) * inv *
                                 bf16_to_f32((unsigned short)w[j]));
     *reinterpret_cast<shortx8*>(out + base + i) = o;
+  };
+  if constexpr (N > 0) {
+#pragma unroll
+    for (int k = 0; k < N; ++k)
+      if ((tid + k * nthr) * 8 < H) write((tid + k * nthr) * 8, held[k], scale[k]);
+  } else {
+    const __hip_bfloat16* src = RESIDUAL ? res_out : (const __hip_bfloat16*)x;
+    for (int i = tid * 8; i < H; i += nthr * 8)
+      write(i, *reinterpret_cast<const shortx8*>(src + base + i),
+            *reinterpret_cast<const shortx8*>(weight + i));
   }
 }
 
@@ -161,10 +177,17 @@ static void rmsnorm_launch(const torch::Tensor& x, const void* res, const torch:
     hipLaunchKernelGGL(rmsnorm_wave_kernel<RESIDUAL>, dim3((T + 3) / 4), dim3(256), 0,
                        CUR_STREAM, xp, (const __hip_bfloat16*)res, op,
                        (__hip_bfloat16*)res_out, wp, T, H, (float)eps);
-  else
-    hipLaunchKernelGGL((rmsnorm_kernel<RESIDUAL>), dim3(T), dim3(256), 0, CUR_STREAM, xp,
-                       (const __hip_bfloat16*)res, op, (__hip_bfloat16*)res_out, wp, H,
-                       (float)eps, 1, 0L);
+  else {
+    auto launch = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3(T), dim3(256), 0, CUR_STREAM, xp,
+                         (const __hip_bfloat16*)res, op, (__hip_bfloat16*)res_out, wp, H,
+                         (float)eps, 1, 0L);
+    };
+    if (H <= 2048) launch(rmsnorm_kernel<RESIDUAL, false, 1>);
+    else if (H <= 4096) launch(rmsnorm_kernel<RESIDUAL, false, 2>);
+    else if (H <= 8192) launch(rmsnorm_kernel<RESIDUAL, false, 4>);
+    else launch(rmsnorm_kernel<RESIDUAL, false, 0>);
+  }
   HIP_CHECK_KERNEL();
 }
 
@@ -192,8 +215,8 @@ std::vector<torch::Tensor> rmsnorm_residual(torch::Tensor x, torch::Tensor res,
     auto out = torch::empty_like(rc), res_out = torch::empty_like(rc);
     if (T == 0) return {out, res_out};
     const int threads = (int)std::min(1024L, (H / 8 + 63) / 64 * 64);
-    hipLaunchKernelGGL((rmsnorm_kernel<true, true>), dim3(T), dim3(threads), 0, CUR_STREAM,
-                       x.data_ptr<float>(), (const __hip_bfloat16*)rc.data_ptr(),
+    const auto kern = H <= 8192 ? rmsnorm_kernel<true, true, 1> : rmsnorm_kernel<true, true, 0>;
+    hipLaunchKernelGGL(kern, dim3(T), dim3(threads), 0, CUR_STREAM, x.data_ptr<float>(), (const __hip_bfloat16*)rc.data_ptr(),
                        (__hip_bfloat16*)out.data_ptr(), (__hip_bfloat16*)res_out.data_ptr(),
                        (const __hip_bfloat16*)weight.data_ptr(), (int)H, (float)eps, (int)S,
                        T * H);
@@ -414,13 +437,8 @@ __global__ __launch_bounds__(256) void fused_rope_kv_write_kernel(
   const int i = (x - unit_row * units) * VEC, t = unit_row / HT, h = unit_row - t * HT;
   const long row = unit_row;
   const bool is_q = h < Hq, is_v = h >= Hq + Hkv;
-  long dst = ((long)t * Hq + h) * D + i;
-  if (!is_q) {
-    const int slot = slots[t];
-    if (slot < 0) return;
-    const int head = h - Hq - (is_v ? Hkv : 0);
-    dst = (((long)(slot / P) * Hkv + head) * P + slot % P) * D + i;
-  }
+  // (asked for before anything that is read waits for them)
+  const int slot = is_q ? 0 : slots[t], position = is_v ? 0 : positions[t];
   float y[2][VEC];  // columns i.. and half + i..
 #pragma unroll
   for (int z = 0; z < 2; ++z) {
@@ -446,8 +464,14 @@ __global__ __launch_bounds__(256) void fused_rope_kv_write_kernel(
         y[z][j] = bf16_to_f32(f32_to_bf16(y[z][j] + bf16_to_f32(b[j])));
     }
   }
+  if (slot < 0) return;
+  long dst = ((long)t * Hq + h) * D + i;
+  if (!is_q) {
+    const int head = h - Hq - (is_v ? Hkv : 0);
+    dst = (((long)(slot / P) * Hkv + head) * P + slot % P) * D + i;
+  }
   if (!is_v) {
-    const float* cs = cos_sin + (long)positions[t] * D + i;
+    const float* cs = cos_sin + (long)position * D + i;
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
       const float c = cs[j], s = cs[half + j], x1 = y[0][j], x2 = y[1][j];
