@@ -21,6 +21,7 @@ import torch.nn as nn
 
 from .. import ops
 from ..parallel import dist as pdist
+from ..parallel.tp import is_plain
 from .config import (
     DenseSpec,
     FusedMixerSpec,
@@ -37,10 +38,20 @@ from .mixers import (
     GroupedExperts,
     LatentAttention,
     ParallelMixer,
+    Projected,
     RetentionMixer,
     RoutedGLU,
     _param,
 )
+
+
+def _in_parts(module: nn.Module):
+    """What to call for a result that ``residual_rmsnorm`` adds up: ``in_parts`` where the
+    module's call is its class's own and nobody watches it."""
+    for kind in (Projected, DenseXieluMLP, DenseGeluMLP, GroupedExperts):
+        if isinstance(module, kind):
+            return module.in_parts if is_plain(module, kind) else module
+    return module
 
 
 class HybridLayer(nn.Module):
@@ -206,14 +217,15 @@ class HybridForCausalLM(nn.Module):
                 add["step"] = self.loop_step[step]
             h, u, state = read(layer.norm1, layer.conv, state)
             ff_state, state = (state[:1], state[1:]) if layer.ff_conv is not None else ([], state)
-            add = {"delta": layer.mixer(u, meta, segments, kv_caches[kv], state)}
+            mixer = _in_parts(layer.mixer)
+            add = {"delta": mixer(u, meta, segments, kv_caches[kv], state)}
             if layer.gate is not None:
                 add["gate"] = (ops.linear(h, layer.gate), layer.gate_bias)
             if layer.post1 is not None:
                 add["post"] = layer.post1
             if layer.mlp is not None:
                 h, u, _ = read(layer.norm2, layer.ff_conv, ff_state)
-                add = layer.mlp(u)
+                add = _in_parts(layer.mlp)(u)
                 if layer.post2 is not None:
                     add["post"] = layer.post2
             if trail is not None:

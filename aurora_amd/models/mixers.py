@@ -66,7 +66,18 @@ class FusedColumns:
         return {n: weight[a:a + self.width[n]] for n, a in self.at.items()}
 
 
-class ParallelMixer(nn.Module):
+class Projected(nn.Module):
+    """A mixer whose heads' results side by side (``heads``) go through ``out_proj``."""
+
+    def forward(self, h, meta, segments, kv, state):
+        return ops.linear(self.heads(h, meta, segments, kv, state), self.out_proj)
+
+    def in_parts(self, h, meta, segments, kv, state):
+        """As ``forward``, possibly in parts (``ops.linear_parts``)."""
+        return ops.linear_parts(self.heads(h, meta, segments, kv, state), self.out_proj)
+
+
+class ParallelMixer(Projected):
     """Distance-biased window attention beside a gated delta rule. Both write
     their heads, already scaled, into one buffer, so the two output
     projections and their sum are a single product."""
@@ -181,7 +192,7 @@ class ParallelMixer(nn.Module):
                 self.a_log.data, self.dt_bias.data, self.head_norm.data, self.eps)
         return self._delta
 
-    def forward(self, h, meta, segments, kv, state):
+    def heads(self, h, meta, segments, kv, state):
         a, at = self.spec.left, self.cols.at
         (k_cache, v_cache), (S, conv) = kv[0], state[0]
         proj = ops.linear(h, self.in_proj)
@@ -196,10 +207,10 @@ class ParallelMixer(nn.Module):
                                  self.slopes, out, 0, a.vdim, self.spec.left_scale)
             ops.delta_rule(proj, z, self._delta_params(), S, conv, seg, out,
                            a.heads * a.vdim, self.spec.right_scale)
-        return ops.linear(out, self.out_proj)
+        return out
 
 
-class RetentionMixer(nn.Module):
+class RetentionMixer(Projected):
     """Fixed-decay linear attention with rotary positions and an output gate."""
 
     def __init__(self, spec: RetentionSpec, hidden: int, eps: float, dtype,
@@ -243,7 +254,7 @@ class RetentionMixer(nn.Module):
 
         self.load(get)
 
-    def forward(self, h, meta, segments, kv, state):
+    def heads(self, h, meta, segments, kv, state):
         s, at = self.spec, self.cols.at
         if self._p is None or self._p.decay.device != self.decay.device:
             self._p = ops.RetentionParams(
@@ -254,10 +265,10 @@ class RetentionMixer(nn.Module):
                           device=h.device)
         for seg in segments:
             ops.retention(proj, self._p, state[0][0], seg, out)
-        return ops.linear(out, self.out_proj)
+        return out
 
 
-class LatentAttention(nn.Module):
+class LatentAttention(Projected):
     """Attention over one cached latent per token: keys and values are per-head
     linear maps of it, and a part of every key that the heads share may be rotated
     by its position and cached beside it. Queries come straight from the input or
@@ -388,7 +399,7 @@ class LatentAttention(nn.Module):
                 self.cos_sin, s.window), front)
         return self._p
 
-    def forward(self, h, meta, segments, kv, state):
+    def heads(self, h, meta, segments, kv, state):
         p, front = self._params()
         cache, H, width = kv[0][0], self.spec.heads, self.D + self.tail
         proj, q = ops.linear(h, self.in_proj), None
@@ -402,7 +413,7 @@ class LatentAttention(nn.Module):
                           device=h.device)
         for seg in segments:
             ops.latent_attention(proj, p, cache, seg, out, q, meta.positions)
-        return ops.linear(out, self.out_proj)
+        return out
 
 
 class MixerPart(nn.Module):
@@ -616,7 +627,7 @@ class MatrixMemory(MixerPart):
             ops.matrix_memory(proj, p, *state[0], seg, out, col, scale)
 
 
-class FusedMixer(nn.Module):
+class FusedMixer(Projected):
     """Parts side by side. All read one fused input projection and write their
     scaled heads into one buffer, so the output projections and their sum are a
     single product."""
@@ -669,7 +680,7 @@ class FusedMixer(nn.Module):
         self.load(lambda n: made[n] if n in made
                   else randn((self.cols.width[n], hidden)) * hidden ** -0.5)
 
-    def forward(self, h, meta, segments, kv, state):
+    def heads(self, h, meta, segments, kv, state):
         proj = ops.linear(h, self.in_proj)
         out = torch.empty(h.shape[0], self.out_proj.shape[1], dtype=h.dtype,
                           device=h.device)
@@ -679,7 +690,7 @@ class FusedMixer(nn.Module):
             s1 = s0 + len(part.state_layout(h.dtype))
             part(proj, at, self.eps, meta, segments, kv[k0:k1], state[s0:s1], out, col, scale)
             col, k0, s0 = col + part.out_width, k1, s1
-        return ops.linear(out, self.out_proj)
+        return out
 
 
 class DenseXieluMLP(nn.Module):
@@ -720,10 +731,17 @@ class DenseXieluMLP(nn.Module):
                   lambda n: randn((hidden,)) if n else randn((hidden, hidden)) * hidden ** -0.5)
 
     def forward(self, h) -> Dict[str, object]:
+        return self._add(h, ops.linear)
+
+    def in_parts(self, h) -> Dict[str, object]:
+        """As ``forward``, a delta possibly in parts (``ops.linear_parts``)."""
+        return self._add(h, ops.linear_parts)
+
+    def _add(self, h, product) -> Dict[str, object]:
         at, ff = self.cols.at, self.spec.ff
         z = ops.linear(h, self.in_proj)
         add: Dict[str, object] = {
-            "delta": ops.linear(ops.xielu(z[:, at["up"]:at["up"] + ff], self.act), self.down)}
+            "delta": product(ops.xielu(z[:, at["up"]:at["up"] + ff], self.act), self.down)}
         if self.gate_bias is not None:
             add["gate"] = (z[:, :h.shape[1]], self.gate_bias)
         return add
@@ -749,7 +767,14 @@ class DenseGeluMLP(nn.Module):
                   * getattr(self, n).shape[1] ** -0.5)
 
     def forward(self, h) -> Dict[str, object]:
-        return {"delta": ops.linear(ops.gelu(ops.linear(h, self.up)), self.down)}
+        return self._add(h, ops.linear)
+
+    def in_parts(self, h) -> Dict[str, object]:
+        """As ``forward``, a delta possibly in parts (``ops.linear_parts``)."""
+        return self._add(h, ops.linear_parts)
+
+    def _add(self, h, product) -> Dict[str, object]:
+        return {"delta": product(ops.gelu(ops.linear(h, self.up)), self.down)}
 
 
 class RoutedGLU(nn.Module):
@@ -848,6 +873,13 @@ class GroupedExperts(nn.Module):
                   * (0.1 if n == "correction" else tensors[n].shape[1] ** -0.5))
 
     def forward(self, h) -> Dict[str, object]:
+        return self._add(h, ops.linear)
+
+    def in_parts(self, h) -> Dict[str, object]:
+        """As ``forward``, a delta possibly in parts (``ops.linear_parts``)."""
+        return self._add(h, ops.linear_parts)
+
+    def _add(self, h, product) -> Dict[str, object]:
         s = self.spec
         glu, sf = s.act == "silu_glu", s.shared_ff
         if (s.scores == "sigmoid") != glu:
@@ -859,7 +891,7 @@ class GroupedExperts(nn.Module):
         if sf:
             z = ops.linear(h, self.shared_in)
             a = ops.silu_glu(z, sf) if glu else ops.relu2(z[:, :sf])
-            add["delta"] = ops.linear(a, self.shared_down)
+            add["delta"] = product(a, self.shared_down)
             if s.shared_gate:
                 add["gate"] = z[:, len(self.first) * sf]
         return add

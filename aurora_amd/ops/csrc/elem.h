@@ -38,6 +38,10 @@ DEVINL void st4(bf16_t* p, floatx4 v) {
   *reinterpret_cast<shortx4*>(p) = r;
 }
 
+// a value as an element of that type holds it
+DEVINL float stored(float v, const float*) { return v; }
+DEVINL float stored(float v, const bf16_t*) { return bf16_to_f32(f32_to_bf16(v)); }
+
 DEVINL float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
 DEVINL float silu_f(float x) { return x / (1.f + expf(-x)); }
 // max(x, 0) + log(1 + y), y = e^-|x|; a short series where 1 + y would round y

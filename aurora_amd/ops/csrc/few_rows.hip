@@ -148,6 +148,18 @@ __global__ __launch_bounds__(256) void add_parts_kernel(const float* __restrict_
   }
 }
 
+// [S, M, N] in fp32 -> their sum [M, N], rounded to bf16
+torch::Tensor add_parts(const torch::Tensor& part) {
+  const long S = part.size(0), M = part.size(1), N = part.size(2);
+  auto out = torch::empty({M, N}, part.options().dtype(torch::kBFloat16));
+  if (M * N == 0) return out;
+  hipLaunchKernelGGL(add_parts_kernel, dim3(std::min((M * N + 255) / 256, 2048L)), dim3(256), 0,
+                     CUR_STREAM, part.data_ptr<float>(), (unsigned short*)out.data_ptr(), (int)S,
+                     M * N);
+  HIP_CHECK_KERNEL();
+  return out;
+}
+
 // K's parts: a workgroup per CU or a few less, of two stages at least (of weights that come
 // from memory one CU takes in some 50 GB/s however much is under way, so more workgroups than
 // CUs only even out badly; what lies in the L2 comes at 136 GB/s). 4096 x
@@ -199,7 +211,7 @@ torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts) {
   const long per = (steps + std::max(parts, 1L) - 1) / std::max(parts, 1L);
   const long S = (steps + per - 1) / per, span = per * FEW_K;
   if (S > 1) part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
-  if (S == 1 || !raw) out = torch::empty({M, N}, x.options());
+  if (S == 1) out = torch::empty({M, N}, x.options());
   auto* op = S > 1 ? nullptr : (unsigned short*)out.data_ptr();
   float* pp = S > 1 ? part.data_ptr<float>() : nullptr;
   if (M <= 32) launch<64, 2, 6, false>(x, w, op, pp, N, S, span);
@@ -207,11 +219,7 @@ torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts) {
   else if (M <= 96) launch<64, 6, 4, false>(x, w, op, pp, N, S, span);
   else launch<64, 8, 3, false>(x, w, op, pp, N, S, span);
   if (S == 1) return out;
-  if (raw) return part;
-  hipLaunchKernelGGL(add_parts_kernel, dim3(std::min((M * N + 255) / 256, 2048L)), dim3(256), 0,
-                     CUR_STREAM, pp, (unsigned short*)out.data_ptr(), (int)S, M * N);
-  HIP_CHECK_KERNEL();
-  return out;
+  return raw ? part : add_parts(part);
 }
 
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw) {

@@ -6,9 +6,9 @@
 // separate combine pass exists), and the vector that marks a pass of a repeated
 // span. What the sub-layer and the experts give together may be normed before it is
 // added. In steps of single tokens the kernel also adds the next sublayer's input
-// convolution to the result. One workgroup per row, the row lives in LDS
-// between the sum of squares and the scaling: x is read and written once,
-// everything else once.
+// convolution to the result. One workgroup per row; x is read and written once,
+// everything else once, and the row stays with its threads between the sum of squares
+// and the scaling (rows too long for that, or of odd widths, in LDS).
 //
 // bias_kv_write: splits the fused projection, adds the biases in fp32, and
 // scatters K/V to the paged cache; heads are stored at the cache's width.
@@ -162,6 +162,142 @@ __global__ __launch_bounds__(NTHR) void residual_rmsnorm_kernel(
   }
 }
 
+// the sub-layer's output, or a product's n parts that lie ``step`` apart: their sum,
+// rounded as the product would have been
+template <typename T>
+struct Delta {
+  const T* whole;  // [T, W]
+  const float* parts;
+  int n;
+  long step;
+  DEVINL explicit operator bool() const { return whole || parts; }
+  DEVINL floatx4 at4(long i) const {
+    if (!parts) return ld4(whole + i);
+    floatx4 d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int s = 0; s < n; ++s) d += ld4(parts + s * step + i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) d[j] = stored(d[j], (T*)nullptr);
+    return d;
+  }
+};
+
+// The same for rows of up to N * 4 * NTHR elements, a multiple of 4: a thread holds its N
+// vectors, so that what can be read is asked for at once, the weight and the convolution's
+// past before the sums they wait for, and nothing goes through LDS.
+template <typename T, int NTHR, bool POST, int N, bool CONV>
+__global__ __launch_bounds__(NTHR) void residual_rmsnorm_held_kernel(
+    float* __restrict__ x, const float* __restrict__ weight, Delta<T> delta,
+    ResidualGate<T> rg, const T* __restrict__ y, const int* __restrict__ place,
+    const float* __restrict__ gate, int top, const float* __restrict__ post,
+    const float* __restrict__ step, T* __restrict__ out, ConvTail<T> cv, int W, float eps,
+    float offset) {
+  __shared__ float red[NTHR / WAVE];
+  const long base = (long)blockIdx.x * W;
+  const int* pl = place + (long)blockIdx.x * top;
+  const float* gt = gate + (long)blockIdx.x * top;
+  int at[N];
+  floatx4 a[N], r[N], wt[N];
+  // (threads past the row's end read its last elements and keep nothing)
+  auto in = [&](int k) { return (int)((threadIdx.x + k * NTHR) * 4) < W; };
+#pragma unroll
+  for (int k = 0; k < N; ++k) at[k] = min((int)(threadIdx.x + k * NTHR) * 4, W - 4);
+#pragma unroll
+  for (int k = 0; k < N; ++k) a[k] = ld4(x + base + at[k]);
+  if (!POST) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) r[k] = a[k];
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; ++k) r[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  if (delta) {
+    floatx4 d[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) d[k] = delta.at4(base + at[k]);
+    if (!POST && rg.pre) {
+      const T* pre = rg.pre + blockIdx.x * rg.stride;
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        const floatx4 g = ld4(pre + at[k]) + ld4(rg.bias + at[k]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) d[k][j] *= sigmoid_f(g[j]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < N; ++k) r[k] += d[k];
+  }
+  if (y) {
+#pragma unroll 4
+    for (int j = 0; j < top; ++j) {
+      const T* row = y + (long)pl[j] * W;
+#pragma unroll
+      for (int k = 0; k < N; ++k) r[k] += gt[j] * ld4(row + at[k]);
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) wt[k] = ld4(weight + at[k]);
+  if constexpr (POST) {
+    floatx4 ps[N];
+    float rs = 0.f;
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      ps[k] = ld4(post + at[k]);
+      if (in(k))
+#pragma unroll
+        for (int j = 0; j < 4; ++j) rs += r[k][j] * r[k][j];
+    }
+    const float rinv = rsqrtf(block_sum<NTHR / WAVE>(rs, red) / W + eps);
+#pragma unroll
+    for (int k = 0; k < N; ++k) r[k] = a[k] + r[k] * rinv * ps[k];
+  }
+  if (step) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) r[k] += ld4(step + at[k]);
+  }
+  float ss = 0.f;
+  const bool changed = delta || y || step;
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+    if (in(k)) {
+      if (changed) st4(x + base + at[k], r[k]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ss += r[k][j] * r[k][j];
+    }
+  const int keep = cv.taps - 1;
+  const int slot = CONV ? cv.slots[blockIdx.x] : -1;
+  const int pos = CONV ? cv.pos[blockIdx.x] : 0;
+  T* ring = cv.ring + (long)max(slot, 0) * keep * W;
+  floatx4 past[N], now[N];
+  if constexpr (CONV) {
+    const int known = slot >= 0 ? min(keep, pos) : 0;  // rows of the past
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      const float* w = cv.w + (long)keep * W + at[k];
+      now[k] = ld4(w);
+      past[k] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+      for (int b = 1; b <= known; ++b)
+        past[k] += ld4(w - (long)b * W) * ld4(ring + (long)((pos - b) % keep) * W + at[k]);
+    }
+  }
+  const float inv = rsqrtf(block_sum<NTHR / WAVE>(ss, red) / W + eps);
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    floatx4 v = r[k] * inv * (offset + wt[k]);
+    if (!in(k)) continue;
+    st4(out + base + at[k], v);
+    if constexpr (!CONV) continue;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = stored(v[j], (T*)nullptr);
+    st4(cv.out + base + at[k], v + v * now[k] + past[k]);
+    // the oldest row's place, which this thread has read
+    if (slot >= 0 && keep > 0) st4(ring + (long)(pos % keep) * W + at[k], v);
+  }
+}
+
+torch::Tensor add_parts(const torch::Tensor& part);  // defined in few_rows.hip
+
 std::vector<torch::Tensor> residual_rmsnorm(
     torch::Tensor x, torch::Tensor weight, c10::optional<torch::Tensor> delta,
     c10::optional<torch::Tensor> gate_pre, c10::optional<torch::Tensor> gate_bias,
@@ -177,9 +313,16 @@ std::vector<torch::Tensor> residual_rmsnorm(
   TORCH_CHECK(W <= 32768, "row too wide for LDS");
   const auto dt = to_bf16 ? torch::kBFloat16 : torch::kFloat32;
   std::vector<torch::Tensor> out = {torch::empty({T_, W}, x.options().dtype(dt))};
-  if (delta)
+  // a product in parts: several, each of the residual's two dimensions
+  const bool parts = delta && to_bf16 && delta->dtype() == torch::kFloat32 &&
+                     delta->dim() == 3 && delta->size(0) > 1;
+  if (parts) {
+    TORCH_CHECK(delta->is_contiguous() && delta->size(1) == T_ && delta->size(2) == W &&
+                (reinterpret_cast<uintptr_t>(delta->data_ptr()) & 15) == 0, "delta in parts");
+  } else if (delta) {
     TORCH_CHECK(delta->is_contiguous() && delta->sizes() == x.sizes() &&
                 delta->dtype() == dt, "delta");
+  }
   if (gate_pre)
     TORCH_CHECK(delta && gate_bias && gate_pre->sizes() == x.sizes() &&
                 gate_pre->stride(1) == 1 && gate_pre->dtype() == dt &&
@@ -207,7 +350,7 @@ std::vector<torch::Tensor> residual_rmsnorm(
     out.push_back(torch::empty_like(out[0]));
   }
   if (T_ == 0) return out;
-  const size_t lds = (size_t)W * 4;
+  const size_t row_lds = (size_t)W * 4;
   DISPATCH_ELEM(to_bf16, {
     ResidualGate<T> rg = {nullptr, 0, nullptr};
     if (gate_pre)
@@ -216,27 +359,48 @@ std::vector<torch::Tensor> residual_rmsnorm(
     if (conv_w)
       cv = {conv_w->data_ptr<float>(), (int)conv_w->size(0), (T*)ring->data_ptr(),
             pos->data_ptr<int>(), slots->data_ptr<int>(), (T*)out[1].data_ptr()};
-    auto launch = [&](auto kern, int threads) {
+    auto launch = [&](auto kern, int threads, size_t lds, auto dl) {
       hipLaunchKernelGGL(
           kern, dim3(T_), dim3(threads), lds, CUR_STREAM, x.data_ptr<float>(),
-          weight.data_ptr<float>(), delta ? (const T*)delta->data_ptr() : nullptr, rg,
+          weight.data_ptr<float>(), dl, rg,
           y ? (const T*)y->data_ptr() : nullptr,
           y ? place->data_ptr<int>() : nullptr, y ? gate->data_ptr<float>() : nullptr,
           top, post ? post->data_ptr<float>() : nullptr, step ? step->data_ptr<float>() : nullptr, (T*)out[0].data_ptr(), cv, W,
           (float)eps, (float)offset);
     };
-    const bool vec = W % 4 == 0 && (!gate_pre || (gate_pre->stride(0) % 4 == 0 &&
+    const bool vec = W % 4 == 0 && W > 0 && (!gate_pre || (gate_pre->stride(0) % 4 == 0 &&
                      (reinterpret_cast<uintptr_t>(gate_pre->data_ptr()) & 15) == 0));
     const bool wide = vec && T_ <= 256 && W > 1024;
-    if (post) {
-      if (wide) launch(residual_rmsnorm_kernel<T, 4, 1024, true>, 1024);
-      else if (vec) launch(residual_rmsnorm_kernel<T, 4, 256, true>, 256);
-      else launch(residual_rmsnorm_kernel<T, 1, 256, true>, 256);
-    } else {
-      if (wide) launch(residual_rmsnorm_kernel<T, 4, 1024, false>, 1024);
-      else if (vec) launch(residual_rmsnorm_kernel<T, 4, 256, false>, 256);
-      else launch(residual_rmsnorm_kernel<T, 1, 256, false>, 256);
-    }
+    // Rows that their threads hold, before (through LDS) and after, us: 1 x 4096 3.8 and 2.8,
+    // with a gate 4.4 and 3.5, 64 x 2048 3.4 and 2.8, with 4 experts' rows 4.9 and 3.8, in 8
+    // parts 4.3 (3.4 after 4.7 to add them), 256 x 4096 5.7 and 4.6, 2000 x 1024 9.4 and 8.5,
+    // 7922 x 2048 37.9 and 37.2 (256 threads of two vectors 40.5), with experts' rows 63.5 and
+    // 55.4. Longer rows of many tokens gain where there is more to wait for: 7922 x 4096 with
+    // experts' rows 126 and 116, but 1884 x 4096 without them 18.5 and 19.0, with a gate 24.0
+    // and 23.9, normed 18.0 and 19.8.
+    const bool held = vec && (wide ? W <= (conv_w ? 4096 : 8192)
+                                   : !conv_w && W <= (y ? 4096 : 2048));
+    if (parts && !held) delta = add_parts(*delta);
+    Delta<T> dl = {nullptr, nullptr, 0, 0};
+    if (parts && held) dl = {nullptr, delta->data_ptr<float>(), (int)delta->size(0), (long)T_ * W};
+    else if (delta) dl.whole = (const T*)delta->data_ptr();
+    auto form = [&](auto after) {
+      constexpr bool POST = decltype(after)::value;
+      auto hold = [&](auto kern, int threads) { launch(kern, threads, 0, dl); };
+      auto rows = [&](auto kern, int threads) { launch(kern, threads, row_lds, dl.whole); };
+      if (held && wide && conv_w) hold(residual_rmsnorm_held_kernel<T, 1024, POST, 1, true>, 1024);
+      else if (held && wide && W <= 4096)
+        hold(residual_rmsnorm_held_kernel<T, 1024, POST, 1, false>, 1024);
+      else if (held && wide) hold(residual_rmsnorm_held_kernel<T, 1024, POST, 2, false>, 1024);
+      else if (held && W <= 1024) hold(residual_rmsnorm_held_kernel<T, 256, POST, 1, false>, 256);
+      else if (held && W <= 2048) hold(residual_rmsnorm_held_kernel<T, 512, POST, 1, false>, 512);
+      else if (held) hold(residual_rmsnorm_held_kernel<T, 512, POST, 2, false>, 512);
+      else if (wide) rows(residual_rmsnorm_kernel<T, 4, 1024, POST>, 1024);
+      else if (vec) rows(residual_rmsnorm_kernel<T, 4, 256, POST>, 256);
+      else rows(residual_rmsnorm_kernel<T, 1, 256, POST>, 256);
+    };
+    if (post) form(std::true_type());
+    else form(std::false_type());
   });
   HIP_CHECK_KERNEL();
   return out;

@@ -318,6 +318,8 @@ def _linear(x, weight):
 
 def residual_rmsnorm(x, weight, eps, delta=None, moe=None, step=None,
                      offset: float = 1.0, dtype=None, gate=None, post=None):
+    """``torch_ref.residual_rmsnorm``; on the GPU ``delta`` may be a product in parts
+    (``linear_parts``), which are added up and rounded first."""
     if not x.is_cuda:
         return torch_ref.residual_rmsnorm(x, weight, eps, delta, moe, step, offset,
                                           dtype, gate, post)
