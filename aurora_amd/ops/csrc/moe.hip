@@ -35,7 +35,7 @@ enum { CHOSEN_SOFTMAX = 0, GROUPED_SIGMOID = 1, GROUPED_SOFTMAX = 2 };
 // The largest value of a wave's lanes but NaN, without a trip through LDS. (Choices by
 // butterflies over value and index took 12 such trips each: 64 tokens of 2048 over 64
 // experts, six each, 16.9 and 14.4 us; over 128, eight each, 28.7 and 25.8; 32 of 4096 over 8,
-// two each, 10.5 and 9.6. What is left is a CU's read of the whole router.)
+// two each, 10.5 and 9.6. What was left is a CU's read of the whole router.)
 DEVINL float lanes_max(float x) {
   auto step = [](float a, auto CTRL) {
     return fmaxf(a, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(
@@ -53,14 +53,155 @@ DEVINL float lanes_max(float x) {
   return fmaxf(__builtin_bit_cast(float, (unsigned)b[0]), __builtin_bit_cast(float, (unsigned)b[1]));
 }
 
-// one workgroup per 16 tokens; its waves split the contraction. GROUPED_SIGMOID: bias
-// is the scores' correction; GROUPED_SOFTMAX: there is none
+// A wave chooses token t's experts. z: its logits, which are used up; score: 512 + groups
+// floats for plain scores and the groups'.
+template <int ROUTER>
+DEVINL void choose(float* z, float* score, int lane, const float* bias, int* sel, float* gate,
+                   int t, int E, int top, int groups, int keep, float scale) {
+  constexpr bool GROUPED = ROUTER != CHOSEN_SOFTMAX;
+  if constexpr (GROUPED) {
+    float* gs = score + 512;
+    const int n = E / groups;
+    auto sync = [] {
+      __threadfence_block();
+      __builtin_amdgcn_wave_barrier();
+    };
+    if constexpr (ROUTER == GROUPED_SIGMOID) {
+      for (int e = lane; e < E; e += WAVE) {
+        score[e] = sigmoid_f(z[e]);
+        z[e] = score[e] + bias[e];
+      }
+    } else {
+      float most = -INFINITY, all = 0.f;
+      for (int e = lane; e < E; e += WAVE) most = fmaxf(most, z[e]);
+      most = wave_max(most);
+      for (int e = lane; e < E; e += WAVE) all += score[e] = expf(z[e] - most);
+      all = wave_sum(all);
+      for (int e = lane; e < E; e += WAVE) score[e] /= all;
+    }
+    sync();
+    for (int x = lane; x < groups; x += WAVE) {
+      float a = -INFINITY, b = -INFINITY;  // the two largest
+      for (int e = x * n; e < (x + 1) * n; ++e) {
+        const float c = z[e];
+        b = fmaxf(b, fminf(a, c));
+        a = fmaxf(a, c);
+      }
+      gs[x] = ROUTER == GROUPED_SIGMOID && n > 1 ? a + b : a;
+    }
+    sync();
+    for (int x = lane; x < groups; x += WAVE) {
+      int better = 0;
+      for (int o = 0; o < groups; ++o)
+        better += gs[o] > gs[x] || (gs[o] == gs[x] && o < x);
+      if (better >= keep)
+        for (int e = x * n; e < (x + 1) * n; ++e) z[e] = -INFINITY;
+    }
+    sync();
+  }
+  float first = 0.f, sum = 0.f;
+  // up to 64 experts: a lane holds its own, the first of the largest is found by lane
+  const bool few = E <= WAVE;
+  float mine = few && lane < E ? z[lane] : -INFINITY;
+  // up to 64 choices: a lane holds one (stored one by one, each waited for the one before)
+  const bool hold = top <= WAVE;
+  int my_at = 0;
+  float my_p = 0.f;
+  for (int n = 0; n < top; ++n) {
+    float best = -INFINITY;
+    int at = 0x7fffffff;
+    if (few) {
+      best = lanes_max(mine);
+      const unsigned long long who = __ballot(mine == best && best > -INFINITY);
+      if (who) at = __builtin_ctzll(who);
+      else best = -INFINITY;
+      if (lane == at) mine = -INFINITY;
+    } else {
+      float own = -INFINITY;
+      int oat = 0;
+      for (int e = lane; e < E; e += WAVE)
+        if (z[e] > own) { own = z[e]; oat = e; }
+      best = lanes_max(own);
+      for (unsigned long long who = __ballot(own == best && best > -INFINITY); who;
+           who &= who - 1)
+        at = min(at, __builtin_amdgcn_readlane(oat, __builtin_ctzll(who)));
+    }
+    at = min(at, E - 1);  // all logits NaN: still a valid expert
+    if (n == 0) first = best;
+    const float p = GROUPED ? score[at] : expf(best - first);
+    sum += p;
+    if (lane == n % WAVE) {
+      my_at = at;
+      my_p = p;
+      if (!hold) {
+        sel[(long)t * top + n] = at;
+        gate[(long)t * top + n] = p;
+      }
+    }
+    if (few) continue;
+    if (lane == 0) z[at] = -INFINITY;
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+  }
+  auto scaled = [&](float w) {
+    return ROUTER == GROUPED_SIGMOID ? w / (sum + 1e-20f) * scale
+           : ROUTER == GROUPED_SOFTMAX ? w * scale : w / sum;
+  };
+  if (hold) {
+    if (lane < top) {
+      sel[(long)t * top + lane] = my_at;
+      gate[(long)t * top + lane] = scaled(my_p);
+    }
+    return;
+  }
+  // each lane rescales what it wrote
+  for (int n = lane; n < top; n += WAVE) {
+    float& w = gate[(long)t * top + n];
+    w = scaled(w);
+  }
+}
+
+// a logit as it is chosen by: without a bias those of a product in the model's own type
+template <typename T, int ROUTER>
+DEVINL float whole_logit(float z, const float* bias, int e) {
+  if (ROUTER != CHOSEN_SOFTMAX) return z;
+  return bias ? z + bias[e] : sizeof(T) == 2 ? bf16_to_f32(f32_to_bf16(z)) : z;
+}
+
+// The choices alone, of logits in S parts [S, T, E] to be added: a wave per token.
+template <int ROUTER>
+__global__ __launch_bounds__(WAVE) void moe_choose_kernel(
+    const float* __restrict__ part, int S, const float* __restrict__ bias,
+    int* __restrict__ sel, float* __restrict__ gate, int E, int top, int groups, int keep,
+    float scale) {
+  extern __shared__ float score[];  // [512 + 512], then logits
+  float* z = score + 1024;
+  const int t = blockIdx.x, lane = threadIdx.x;
+  const long step = (long)gridDim.x * E;
+  for (int e = lane; e < E; e += WAVE) {
+    const float* p = part + (long)t * E + e;
+    float sum = 0.f;
+    for (int s = 0; s < S; s += 8) {  // asked for together
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = p[min(s + u, S - 1) * step];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) sum += s + u < S ? v[u] : 0.f;
+    }
+    z[e] = whole_logit<bf16_t, ROUTER>(sum, bias, e);
+  }
+  __threadfence_block();
+  __builtin_amdgcn_wave_barrier();
+  choose<ROUTER>(z, score, lane, bias, sel, gate, t, E, top, groups, keep, scale);
+}
+
+// One workgroup per 16 tokens; its waves split the contraction. GROUPED_SIGMOID: bias
+// is the scores' correction; GROUPED_SOFTMAX: there is none.
 template <typename T, bool MATRIX16, int ROUTER>
 __global__ __launch_bounds__(1024) void moe_route_kernel(
     const T* __restrict__ h, const T* __restrict__ router,
     const float* __restrict__ bias, int* __restrict__ sel, float* __restrict__ gate,
     int T_, int W, int E, int top, int groups, int keep, float scale) {
-  constexpr bool GROUPED = ROUTER != CHOSEN_SOFTMAX;
   extern __shared__ float logits[];  // [16][E]
   __shared__ float part[16][16][64];
   const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
@@ -111,99 +252,37 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(
       float z = 0.f;
 #pragma unroll
       for (int v = 0; v < 16; ++v) z += part[v][t][x];
-      // without a bias the logits are those of a product in the model's own type
-      if (ROUTER == CHOSEN_SOFTMAX)
-        z = bias ? z + bias[min(e, E - 1)] : sizeof(T) == 2 ? bf16_to_f32(f32_to_bf16(z)) : z;
-      if (e < E) logits[t * E + e] = z;
+      if (e < E) logits[t * E + e] = whole_logit<T, ROUTER>(z, bias, e);
     }
     __syncthreads();
   }
-  if (t0 + wave < T_) {
-    const int t = wave;
-    float* z = logits + t * E;
-    float* score = &part[wave][0][0];  // plain scores; from 512 on the groups'
-    if constexpr (GROUPED) {
-      float* gs = score + 512;
-      const int n = E / groups;
-      auto sync = [] {
-        __threadfence_block();
-        __builtin_amdgcn_wave_barrier();
-      };
-      if constexpr (ROUTER == GROUPED_SIGMOID) {
-        for (int e = lane; e < E; e += WAVE) {
-          score[e] = sigmoid_f(z[e]);
-          z[e] = score[e] + bias[e];
-        }
-      } else {
-        float most = -INFINITY, all = 0.f;
-        for (int e = lane; e < E; e += WAVE) most = fmaxf(most, z[e]);
-        most = wave_max(most);
-        for (int e = lane; e < E; e += WAVE) all += score[e] = expf(z[e] - most);
-        all = wave_sum(all);
-        for (int e = lane; e < E; e += WAVE) score[e] /= all;
-      }
-      sync();
-      for (int x = lane; x < groups; x += WAVE) {
-        float a = -INFINITY, b = -INFINITY;  // the two largest
-        for (int e = x * n; e < (x + 1) * n; ++e) {
-          const float c = z[e];
-          b = fmaxf(b, fminf(a, c));
-          a = fmaxf(a, c);
-        }
-        gs[x] = ROUTER == GROUPED_SIGMOID && n > 1 ? a + b : a;
-      }
-      sync();
-      for (int x = lane; x < groups; x += WAVE) {
-        int better = 0;
-        for (int o = 0; o < groups; ++o)
-          better += gs[o] > gs[x] || (gs[o] == gs[x] && o < x);
-        if (better >= keep)
-          for (int e = x * n; e < (x + 1) * n; ++e) z[e] = -INFINITY;
-      }
-      sync();
-    }
-    float first = 0.f, sum = 0.f;
-    // up to 64 experts: a lane holds its own, the first of the largest is found by lane
-    const bool few = E <= WAVE;
-    float mine = few && lane < E ? z[lane] : -INFINITY;
-    for (int n = 0; n < top; ++n) {
-      float best = -INFINITY;
-      int at = 0x7fffffff;
-      if (few) {
-        best = lanes_max(mine);
-        const unsigned long long who = __ballot(mine == best && best > -INFINITY);
-        if (who) at = __builtin_ctzll(who);
-        else best = -INFINITY;
-        if (lane == at) mine = -INFINITY;
-      } else {
-        float own = -INFINITY;
-        int oat = 0;
-        for (int e = lane; e < E; e += WAVE)
-          if (z[e] > own) { own = z[e]; oat = e; }
-        best = lanes_max(own);
-        for (unsigned long long who = __ballot(own == best && best > -INFINITY); who;
-             who &= who - 1)
-          at = min(at, __builtin_amdgcn_readlane(oat, __builtin_ctzll(who)));
-      }
-      at = min(at, E - 1);  // all logits NaN: still a valid expert
-      if (n == 0) first = best;
-      const float p = GROUPED ? score[at] : expf(best - first);
-      sum += p;
-      if (lane == n % WAVE) {
-        sel[(long)(t0 + t) * top + n] = at;
-        gate[(long)(t0 + t) * top + n] = p;
-      }
-      if (lane == 0) z[at] = -INFINITY;
-      __threadfence_block();
-      __builtin_amdgcn_wave_barrier();
-    }
-    // each lane rescales what it wrote
-    for (int n = lane; n < top; n += WAVE) {
-      float& w = gate[(long)(t0 + t) * top + n];
-      w = ROUTER == GROUPED_SIGMOID ? w / (sum + 1e-20f) * scale
-          : ROUTER == GROUPED_SOFTMAX ? w * scale : w / sum;
-    }
-  }
+  if (t0 + wave < T_)
+    choose<ROUTER>(logits + wave * E, &part[wave][0][0], lane, bias, sel, gate, t0 + wave, E,
+                   top, groups, keep, scale);
+}
+
+torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts);
+
+// Few tokens: a workgroup for 16 of them reads the whole router, at some 25 GB/s of a CU, where
+// the products' kernel of few rows spreads it over 16 and more, and a second launch adds the
+// parts and chooses. Cold routers, us, whole and in parts, of 1, 16, 64 and 128 tokens:
+//   E x W       1             16            64            128
+//   8 x 4096    5.7 and 5.2   8.8 and 5.8   9.0 and 6.9   9.0 and 8.4
+//   16 x 2880   6.7 and 6.2   9.5 and 6.3   9.7 and 7.3   9.7 and 8.6
+//   32 x 2048   7.5 and 6.0   9.8 and 6.4   10.0 and 7.1  10.2 and 8.1
+//   64 x 2048   11.2 and 6.0  13.5 and 6.4  13.7 and 7.0  13.9 and 7.8
+//   128 x 4096  34.9 and 8.3  41.1 and 9.2  41.6 and 10.4 41.6 and 11.5
+// and on the other side
+//   8 x 2880    4.9 and 5.1   7.2 and 5.6   7.3 and 6.6   7.3 and 8.0
+//   16 x 2048   5.8 and 6.0   8.1 and 6.3   8.3 and 7.0   8.3 and 8.2
+//   32 x 1024   5.6 and 5.6   7.2 and 5.8   7.4 and 6.6   7.5 and 7.6
+//   64 x 512    5.5 and 5.5   6.8 and 5.9   7.0 and 6.5   7.0 and 7.3
+//   128 x 256   7.3 and 7.1   8.6 and 7.4   8.8 and 8.0   8.8 and 8.9
+static bool route_in_parts(const torch::Tensor& h, const torch::Tensor& router) {
+  const long T_ = h.size(0), W = h.size(1), E = router.size(0);
+  return h.dtype() == torch::kBFloat16 && T_ <= 128 && W % 64 == 0 && W >= 256 &&
+         W * (E + 12) >= 76000 && (uintptr_t)router.data_ptr() % 16 == 0 &&
+         (uintptr_t)h.data_ptr() % 16 == 0;
 }
 
 template <int ROUTER>
@@ -221,6 +300,16 @@ static std::vector<torch::Tensor> route(const torch::Tensor& h, const torch::Ten
   auto sel = torch::empty({T_, top}, h.options().dtype(torch::kInt32));
   auto gate = torch::empty({T_, top}, h.options().dtype(torch::kFloat32));
   if (T_ == 0) return {sel, gate};
+  if (route_in_parts(h, router)) {
+    const auto part = few_rows(h, router, true, std::min(16L, W / 128));
+    hipLaunchKernelGGL(moe_choose_kernel<ROUTER>, dim3(T_), dim3(WAVE), (1024 + E) * 4, CUR_STREAM,
+                       part.template data_ptr<float>(), (int)part.size(0),
+                       bias ? bias->data_ptr<float>() : nullptr, sel.data_ptr<int>(),
+                       gate.data_ptr<float>(), (int)E, (int)top, (int)groups, (int)keep,
+                       (float)scale);
+    HIP_CHECK_KERNEL();
+    return {sel, gate};
+  }
   DISPATCH_ELEM(h.dtype() == torch::kBFloat16, {
     auto launch = [&](auto kern) {
       hipLaunchKernelGGL(kern, dim3((T_ + 15) / 16), dim3(1024), 16 * E * 4, CUR_STREAM,
