@@ -29,6 +29,7 @@ from ..parallel.tp import (
     RowParallelLinear,
     column_parts,
     column_silu_mul,
+    column_weight,
     is_plain,
     row_parts,
 )
@@ -353,12 +354,24 @@ class LlamaDecoderLayer(nn.Module):
             residual = x
             h = ops.rmsnorm(x, self.input_norm, self.eps)
         else:
-            h, residual = ops.rmsnorm_residual(x, residual, self.input_norm, self.eps)
+            h, residual = ops.norm_ahead(x, residual, self.input_norm, self.eps,
+                                         self._reader("attn", x), False)
         attn = self.attn.parts if is_plain(self.attn, LlamaAttention) else self.attn
         a = attn(h, cos_sin, kv_cache, meta)
-        h, residual = ops.rmsnorm_residual(a, residual, self.post_attn_norm, self.eps)
+        h, residual = ops.norm_ahead(a, residual, self.post_attn_norm, self.eps,
+                                     self._reader("mlp", a) if in_parts else None, True)
         mlp = self.mlp.parts if in_parts and is_plain(self.mlp, LlamaMLP) else self.mlp
         return mlp(h), residual
+
+    def _reader(self, what: str, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """The weight whose product alone reads the norm before ``what``, if x, the norm's
+        input, is a single row in parts and nobody watches the product."""
+        if x.dim() != 3 or x.shape[1] != 1:
+            return None
+        if what == "attn":
+            return (column_weight(self.attn.qkv_proj, True)
+                    if is_plain(self.attn, LlamaAttention) else None)
+        return column_weight(self.mlp.gate_up, False) if is_plain(self.mlp, LlamaMLP) else None
 
 
 class LlamaForCausalLM(nn.Module):

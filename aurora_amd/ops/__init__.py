@@ -13,7 +13,7 @@ Build the extensions with ``python setup.py build_ext --inplace`` (hipcc,
 """
 from __future__ import annotations
 
-from typing import Optional, Tuple
+from typing import NamedTuple, Optional, Tuple
 
 import torch
 import torch.nn.functional as F
@@ -244,17 +244,46 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return F.linear(x, weight) if y is None else y
 
 
-def linear_parts(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+class Unnormed(NamedTuple):
+    """A row whose norm is done by the product that reads it (``norm_ahead``)."""
+
+    parts: torch.Tensor
+    residual: torch.Tensor
+    weight: torch.Tensor
+    eps: float
+    sum: torch.Tensor  # the new residual, written by that product
+
+    @property
+    def shape(self):
+        return self.residual.shape
+
+
+def norm_ahead(x, residual, weight, eps, reader: Optional[torch.Tensor], silu: bool):
+    """``rmsnorm_residual`` for ``linear_parts``, or with ``silu`` ``linear_silu_mul``, by
+    ``reader``, the only reader of the rows: a single row in parts is left to it."""
+    if (reader is not None and x.is_cuda and x.dim() == 3 and x.shape[1] == 1
+            and _require_hip("norm_ahead").norms_row(x, residual, weight, reader, silu)):
+        new = torch.empty_like(residual)
+        return Unnormed(x, residual, weight, float(eps), new), new
+    return rmsnorm_residual(x, residual, weight, eps)
+
+
+def linear_parts(x, weight: torch.Tensor) -> torch.Tensor:
     """As ``linear``, but where the product of few rows is cut along K its parts
     [S, T, N] in float32, for a reader that adds and rounds them itself
-    (``rmsnorm_residual``, ``fused_rope_kv_write``)."""
+    (``rmsnorm_residual``, ``fused_rope_kv_write``). ``x``: rows, or one of
+    ``norm_ahead``."""
+    if isinstance(x, Unnormed):
+        return _hip.one_row_product(*x, weight, False)
     y = _hip.own_product(x, weight, 1) if x.is_cuda and _hip is not None else None
     return F.linear(x, weight) if y is None else y
 
 
-def linear_silu_mul(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+def linear_silu_mul(x, weight: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up of the products with gate's rows, then up's; in one kernel where that
-    is faster."""
+    is faster. ``x``: rows, or one of ``norm_ahead``."""
+    if isinstance(x, Unnormed):
+        return _hip.one_row_product(*x, weight, True)
     y = _hip.own_product(x, weight, 2) if x.is_cuda and _hip is not None else None
     return silu_mul(linear(x, weight)) if y is None else y
 

@@ -31,6 +31,10 @@ torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
 torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts);
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
+torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor weight, double eps,
+                              torch::Tensor res_out, torch::Tensor w, bool silu);
+bool norms_row(const torch::Tensor& x, const torch::Tensor& res, const torch::Tensor& weight,
+               const torch::Tensor& w, bool silu);
 torch::Tensor skinny_gemm2_ex(torch::Tensor x, torch::Tensor w, long s_target);
 torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target);
 torch::Tensor moe_grouped_gemm(torch::Tensor xp, torch::Tensor w,
@@ -200,6 +204,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("many_rows", &many_rows, "products of many rows, with silu(gate) * up");
   m.def("few_rows", &few_rows, "products of at most 128 rows, K in parts");
   m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows");
+  m.def("one_row_product", &one_row_product, "a norm and the product of its one row");
+  m.def("norms_row", &norms_row, "whether one_row_product serves");
   m.def("silu_few_rows", &silu_few_rows, "gate and up of at most 128 rows, silu(gate) * up");
   m.def("skinny_gemm2_ex", &skinny_gemm2_ex, "products of at most 256 rows");
   m.def("skinny_gemm3_ex", &skinny_gemm3_ex, "glds double-buffered projection GEMM (M<=256)");

@@ -27,6 +27,7 @@
 // at 64 rows and more is x on its way to every CU.
 #include "flash_tiles.h"
 #include <torch/extension.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
 #define CUR_STREAM c10::hip::getCurrentHIPStream().stream()
@@ -136,6 +137,145 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
           if (n + j < N) dst[j] = f32_to_bf16(y[j]);
     }
   }
+}
+
+// A wait for LDS alone: loads of W on their way to it stay under way.
+DEVINL void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+#define ROW_MOST 8192  // elements of the row below
+
+// The product of one row with the norm before it: x comes as S parts [S, K] to be added to the
+// residual, as rmsnorm_residual does. Every workgroup norms the row for itself: four waves of
+// their own do that while the other four have the first blocks of W on their way, and end. The
+// first workgroup writes the new residual. HV: vectors of four of the row per thread, S at most
+// 16 / HV.
+// Bound by W; what is saved is the norm's launch and its trip to memory, what it costs is the
+// parts' way to every CU (64 KB). A layer of one row, its two norms before and in the products,
+// cold weights: 4096 wide, 28672 and 6144 outputs, 95.3 and 92.0 us; 2048, 16384 and 3072, 41.0
+// and 38.8; 1024, 8192 and 2048, 24.5 and 20.6. With the norm by the waves that load W (its
+// loads are then waited for with W's) 93.7, 38.5 and 21.3.
+template <int HV, bool SILU>
+__global__ __launch_bounds__(512) void one_row_kernel(
+    const float* __restrict__ x, int S, const unsigned short* __restrict__ res,
+    const unsigned short* __restrict__ weight, unsigned short* __restrict__ res_out, float eps,
+    const unsigned short* __restrict__ w, unsigned short* __restrict__ out,
+    float* __restrict__ part, int N, int K, int span) {
+  constexpr int NS = 7, L = 2, STAGE = 64 * 128, PARTS = 16 / HV;
+  // one array: of several the compiler waits for all loads under way before it reads one
+  __shared__ __attribute__((aligned(16))) char lds[NS * STAGE + HV * 2048 + 16];
+  auto* row = reinterpret_cast<unsigned short*>(lds + NS * STAGE);
+  auto* red = reinterpret_cast<float*>(lds + NS * STAGE + HV * 2048);
+  const int tid = threadIdx.x % 256, lane = tid % WAVE;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256) {
+    floatx4 t[PARTS][HV];
+    u64b old[HV], scale[HV];
+#pragma unroll
+    for (int v = 0; v < HV; ++v) {
+      const int c = min((tid + v * 256) * 4, K - 4);
+#pragma unroll
+      for (int p = 0; p < PARTS; ++p)
+        t[p][v] = *reinterpret_cast<const floatx4*>(x + (long)min(p, S - 1) * K + c);
+      old[v] = *reinterpret_cast<const u64b*>(res + c);
+      scale[v] = *reinterpret_cast<const u64b*>(weight + c);
+    }
+    auto four = [](const unsigned short* v) {
+      return (u64b)v[3] << 48 | (u64b)v[2] << 32 | (u64b)v[1] << 16 | v[0];
+    };
+    float ss = 0.f;
+    u64b kept[HV];
+#pragma unroll
+    for (int v = 0; v < HV; ++v) {
+      unsigned short b[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float y = 0.f;
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) y += p < S ? t[p][v][j] : 0.f;
+        y = bf16_to_f32(f32_to_bf16(y)) + bf16_to_f32((unsigned short)(old[v] >> (16 * j)));
+        if ((tid + v * 256) * 4 < K) ss += y * y;
+        b[j] = f32_to_bf16(y);
+      }
+      kept[v] = four(b);
+    }
+    ss = wave_sum(ss);
+    if (lane == 0) red[wave] = ss;
+    meet();
+    const float inv = rsqrtf((red[0] + red[1] + red[2] + red[3]) / K + eps);
+#pragma unroll
+    for (int v = 0; v < HV; ++v) {
+      const int c = (tid + v * 256) * 4;
+      unsigned short b[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        b[j] = f32_to_bf16(bf16_to_f32((unsigned short)(kept[v] >> (16 * j))) * inv *
+                           bf16_to_f32((unsigned short)(scale[v] >> (16 * j))));
+      *reinterpret_cast<u64b*>(row + c) = four(b);  // (past K: not read)
+      if (blockIdx.x == 0 && blockIdx.y == 0 && c < K)
+        *reinterpret_cast<u64b*>(res_out + c) = kept[v];
+    }
+    meet();
+    return;  // barriers wait for the waves that are left
+  }
+  const int at = lane & 15, g = lane >> 4;
+  const int n0 = blockIdx.x * (SILU ? 32 : 64);
+  const int k0 = blockIdx.y * span, steps = (min(K, k0 + span) - k0) / FEW_K;
+  const unsigned short* src[L];
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    const int r = (tid + l * 256) >> 3, unit = (tid & 7) ^ (r & 7);
+    const long n = SILU ? min(n0 + r / 16 * 8 + r % 8, N - 1) + (long)(r % 16 / 8) * N
+                        : min(n0 + r, N - 1);
+    src[l] = w + n * K + k0 + unit * 8;
+  }
+  auto issue = [&](int s) {
+    char* stage = lds + s % NS * STAGE;
+#pragma unroll
+    for (int l = 0; l < L; ++l)
+      __builtin_amdgcn_global_load_lds((gptr_t)(src[l] + (long)s * FEW_K),
+                                       (lptr_t)(stage + (l * 256 + wave * WAVE) * 16), 16, 0, 0);
+  };
+  for (int s = 0; s < min(steps, NS - 1); ++s) issue(s);
+  meet();
+  meet();
+  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int s) {
+    const char* stage = lds + s % NS * STAGE;
+    frag_u wf[2], xf[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      wf[h].s = *reinterpret_cast<const shortx8*>(stage + (wave * 16 + at) * 128 +
+                                                  ((h * 4 + g) ^ (at & 7)) * 16);
+      xf[h].s = *reinterpret_cast<const shortx8*>(row + k0 + s * FEW_K + (h * 4 + g) * 8);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h].v, xf[h].v, acc, 0, 0, 0);
+  };
+  int s = 0;
+  for (; s + NS - 1 < steps; ++s) {
+    await_stage<(NS - 2) * L>();
+    issue(s + NS - 1);  // over the stage before this, which all waves have left
+    compute(s);
+  }
+  await_stage<0>();
+  for (; s < steps; ++s) compute(s);
+  if constexpr (SILU) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float up = __shfl_xor(acc[j], 32, WAVE);
+      acc[j] = acc[j] / (1.f + __expf(-acc[j])) * up;
+    }
+    if (g >= 2) return;
+  }
+  if (at) return;  // all columns of the product are the row's
+  const int n = n0 + (SILU ? wave * 8 + g * 4 : wave * 16 + g * 4);
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    if (n + j < N) {
+      if (!SILU && part) part[(long)blockIdx.y * N + n + j] = acc[j];
+      else out[n + j] = f32_to_bf16(acc[j]);
+    }
 }
 
 __global__ __launch_bounds__(256) void add_parts_kernel(const float* __restrict__ part,
@@ -250,4 +390,55 @@ torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w) {
   else if (wide) launch<128, 8, 5, true>(x, w, op, nullptr, N, 1, K);
   else launch<64, 8, 3, true>(x, w, op, nullptr, N, 1, K);
   return out;
+}
+
+// The kernel above where it has a form: x [S, 1, K] in fp32, S parts.
+bool one_row_fits(long S, long K) {
+  return S > 1 && K % FEW_K == 0 && K <= ROW_MOST &&
+         S <= (K <= 1024 ? 16 : K <= 2048 ? 8 : K <= 4096 ? 4 : 2);
+}
+
+// w @ norm(x's parts + res), with ``silu`` as silu_few_rows, else as linear_few_rows's parts;
+// the sum goes to res_out.
+torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor weight, double eps,
+                              torch::Tensor res_out, torch::Tensor w, bool silu) {
+  TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kFloat32 && x.is_contiguous() && x.dim() == 3 &&
+                  x.size(1) == 1 && one_row_fits(x.size(0), x.size(2)),
+              "a row in parts [S, 1, K]");
+  const long S = x.size(0), K = x.size(2), N = silu ? w.size(0) / 2 : w.size(0);
+  for (const auto& t : {res, weight, res_out, w})
+    TORCH_CHECK(t.device() == x.device() && t.dtype() == torch::kBFloat16 && t.is_contiguous() &&
+                    (uintptr_t)t.data_ptr() % 16 == 0, "bf16 beside the row, contiguous");
+  TORCH_CHECK(res.numel() == K && weight.numel() == K && res_out.numel() == K &&
+                  w.dim() == 2 && w.size(1) == K && w.size(0) % 2 == 0 && N > 0 &&
+                  (uintptr_t)x.data_ptr() % 16 == 0 && res.data_ptr() != res_out.data_ptr(),
+              "rows of K");
+  const c10::DeviceGuard on(x.device());
+  const long steps = K / FEW_K, parts = silu ? 1 : parts_of(N, K);
+  const long per = (steps + parts - 1) / parts, S2 = (steps + per - 1) / per;
+  torch::Tensor out, part;
+  if (S2 > 1) part = torch::empty({S2, 1, N}, x.options());
+  else out = torch::empty({1, N}, w.options());
+  const int tile = silu ? 32 : 64;
+  auto launch = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3((N + tile - 1) / tile, S2), dim3(512), 0, CUR_STREAM,
+                       x.data_ptr<float>(), (int)S, (const unsigned short*)res.data_ptr(),
+                       (const unsigned short*)weight.data_ptr(),
+                       (unsigned short*)res_out.data_ptr(), (float)eps,
+                       (const unsigned short*)w.data_ptr(),
+                       S2 > 1 ? nullptr : (unsigned short*)out.data_ptr(),
+                       S2 > 1 ? part.data_ptr<float>() : nullptr, (int)N, (int)K,
+                       (int)(per * FEW_K));
+    HIP_CHECK_KERNEL();
+  };
+  auto form = [&](auto hv) {
+    constexpr int HV = decltype(hv)::value;
+    if (silu) launch(one_row_kernel<HV, true>);
+    else launch(one_row_kernel<HV, false>);
+  };
+  if (K <= 1024) form(std::integral_constant<int, 1>{});
+  else if (K <= 2048) form(std::integral_constant<int, 2>{});
+  else if (K <= 4096) form(std::integral_constant<int, 4>{});
+  else form(std::integral_constant<int, 8>{});
+  return S2 > 1 ? part : out;
 }

@@ -9,6 +9,7 @@
 // defined in few_rows.hip, moe.hip, skinny_gemm.hip
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
+bool one_row_fits(long S, long K);
 torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
 bool large_takes(long N, long K);
 torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target);
@@ -151,4 +152,22 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
     if (!off || std::strcmp(off, "0")) return skinny_gemm3_ex(x.contiguous(), w, 384);
   }
   return {};
+}
+
+// Whether the norm of x's parts + res by ``weight`` is done by the product with w that reads it,
+// in parts or with ``silu``: one row, where the kernel of few rows would take the product.
+bool norms_row(const torch::Tensor& x, const torch::Tensor& res, const torch::Tensor& weight,
+               const torch::Tensor& w, bool silu) {
+  if (x.dim() != 3 || x.size(1) != 1 || x.dtype() != torch::kFloat32 || !x.is_cuda() ||
+      !plain(x) || !x.is_contiguous() || (uintptr_t)x.data_ptr() % 16)
+    return false;
+  const long K = x.size(2);
+  for (const auto* t : {&res, &weight, &w})
+    if (!plain(*t) || t->device() != x.device() || t->dtype() != torch::kBFloat16 ||
+        !t->is_contiguous() || (uintptr_t)t->data_ptr() % 16)
+      return false;
+  if (!one_row_fits(x.size(0), K) || res.dim() != 2 || res.size(0) != 1 || res.size(1) != K ||
+      weight.numel() != K || w.dim() != 2 || w.size(1) != K || w.size(0) == 0 || w.size(0) % 16)
+    return false;
+  return silu ? silu_few_rows_win(1, w.size(0) / 2, K) : few_rows_win(1, w.size(0), K, true);
 }

@@ -125,6 +125,13 @@ def column_parts(m: nn.Module, x: torch.Tensor) -> Tuple[torch.Tensor, Optional[
     return m(x), None
 
 
+def column_weight(m: nn.Module, bias: bool) -> Optional[torch.Tensor]:
+    """What ``column_parts`` (with ``bias``) or ``column_silu_mul`` multiplies by itself; None
+    where it calls ``m``."""
+    return m.weight if (is_plain(m, ColumnParallelLinear) and not m.gather_output
+                        and (bias or m.bias is None)) else None
+
+
 def row_parts(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
     """``m(x)`` of a row-parallel layer, possibly in parts where nothing is reduced."""
     if is_plain(m, RowParallelLinear) and pdist.tp_world_size() == 1:
