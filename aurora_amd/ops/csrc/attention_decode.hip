@@ -550,10 +550,10 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
 
 // Marks that a call wants for its sequences' head tiles, or 0 where contexts stay whole: while
 // the longest that can be seen is short or the workgroups are many, cutting costs its search
-// and the merge, and evens out little. Whole and cut, 128 wide, 8 kv heads: 64 sequences of 2000
-// keys 100 and 110 us, 100 of 50 keys 7 and 13; behind a window of 1024, 32 sequences 30 and 40,
-// 16 sequences 19 and 27, 2 sequences (outside the rule) 16 and 13. What it gives up: 64
-// sequences of 300 to 8000 keys 229 and 215.
+// and the merge, and evens out little. Whole and cut, 128 wide, 8 kv heads: 32 sequences of 1024
+// keys 31 and 34 us, 96 of 100 to 3000 115 and 132, 16 of 1024 21 and 21; on the other side
+// 4 sequences of 3000 to 9000 keys 93 and 30, 23 of 300 to 5000 73 and 61, 32 of 300 to 8000 126
+// and 114. What it gives up: 64 sequences of 300 to 8000 keys 221 and 215.
 long decode_marks(long B, long Hq, long Hkv, long longest, long window, long chunk) {
   const long tiles = Hkv * ((Hq / Hkv + DEC_HEADS - 1) / DEC_HEADS);
   if (window > 0) longest = std::min(longest, window);

@@ -37,11 +37,12 @@ DEVINL void add_parts8(float (&y)[8], const float* x, int parts, long step) {
 // One workgroup per row; 256 threads; row length H must be a multiple of 8.
 // RESIDUAL: also adds `res` first and writes the sum back to res_out.
 // PARTS: x is the sum, rounded to bf16, of `parts` fp32 terms that lie `step` apart. A
-// product left in parts is so added up where it is read anyway: 96 rows of 4096 in 4 parts
-// 3.5 us, 23 rows of 2048 in 8 parts 3.3; of a whole product 3.4 and 2.6, after a kernel to
-// add its parts that takes 2.4 to 4.7.
+// product left in parts is so added up where it is read anyway: 23 rows of 2048 in 8 parts
+// 3.8 us, 96 rows of 4096 in 4 parts 4.4; a kernel to add the parts takes 2.4 to 4.7 more.
 // N: vectors of eight that a thread holds, so that a row is read once and the weight comes with
-// it; 0 for rows too long for that, which are read again.
+// it; 0 for rows too long for that, which are read again. Read again, and held: 6176 rows of
+// 4096 42.6 and 34.5 us (5.9 TB/s, the bound), 1600 12.7 and 11.9, one row in 4 parts 3.25 and
+// 2.99 (a launch and two trips to memory), 23 of 2048 in 8 parts 4.07 and 3.80.
 template <bool RESIDUAL, bool PARTS, int N>
 __global__ __launch_bounds__(PARTS ? 1024 : 256) void rmsnorm_kernel(
     const std::conditional_t<PARTS, float, __hip_bfloat16>* __restrict__ x,
@@ -416,7 +417,10 @@ void kv_cache_write(torch::Tensor k, torch::Tensor v, torch::Tensor kc,
 // floor in the decode step (profiles/decode_kernel_stats_r01.csv).
 // qkv: [T, (Hq+2*Hkv)*D] -> writes q_out [T, Hq, D] (roped), kc/vc slots.
 // PARTS: qkv is a product in `parts` fp32 terms `step` apart, see rmsnorm_kernel: 96
-// rows of 6144 in 2 parts 3.3 us and whole 3.0, 23 of 3072 in 5 parts 2.8 and 2.4.
+// rows of 6144 in 2 parts 3.3 us and whole 3.0, 23 of 3072 in 5 parts 2.8 and 2.4. Slot and
+// position are asked for before anything else, so that few rows make two trips to memory and
+// not three: 23 of 3072 in 5 parts 3.82 and 3.66, 96 of 6144 in 2 parts 4.46 and 4.18 (of
+// cold cache pages).
 // bias: one term more per column or null, added to the rounded product.
 // A thread per VEC columns of a head and their partners half a head on (16-byte accesses
 // at 8): bound by memory. 6172 rows of 48 heads of 128 took 58 us in 2-byte accesses,
