@@ -144,35 +144,40 @@ DEVINL void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memor
 
 #define ROW_MOST 8192  // elements of the row below
 
+// threads that norm the row, besides the 256 of the product: wider rows want eight waves (4096
+// wide, a layer 92.0 and 91.8 us, 2048 38.8 and 38.1, 1024 20.6 and 21.7)
+constexpr int row_threads(int hv) { return hv > 1 ? 512 : 256; }
+
 // The product of one row with the norm before it: x comes as S parts [S, K] to be added to the
-// residual, as rmsnorm_residual does. Every workgroup norms the row for itself: four waves of
-// their own do that while the other four have the first blocks of W on their way, and end. The
-// first workgroup writes the new residual. HV: vectors of four of the row per thread, S at most
-// 16 / HV.
+// residual, as rmsnorm_residual does. Every workgroup norms the row for itself: four or eight
+// waves of their own do that while four others have the first blocks of W on their way, and end.
+// The first workgroup writes the new residual. HV: vectors of four of the row per 256 threads, S
+// at most 16 / HV.
 // Bound by W; what is saved is the norm's launch and its trip to memory, what it costs is the
 // parts' way to every CU (64 KB). A layer of one row, its two norms before and in the products,
-// cold weights: 4096 wide, 28672 and 6144 outputs, 95.3 and 92.0 us; 2048, 16384 and 3072, 41.0
-// and 38.8; 1024, 8192 and 2048, 24.5 and 20.6. With the norm by the waves that load W (its
+// cold weights: 4096 wide, 28672 and 6144 outputs, 95.9 and 91.8 us; 2048, 16384 and 3072, 41.0
+// and 38.1; 1024, 8192 and 2048, 24.5 and 20.6. With the norm by the waves that load W (its
 // loads are then waited for with W's) 93.7, 38.5 and 21.3.
 template <int HV, bool SILU>
-__global__ __launch_bounds__(512) void one_row_kernel(
+__global__ __launch_bounds__(256 + row_threads(HV)) void one_row_kernel(
     const float* __restrict__ x, int S, const unsigned short* __restrict__ res,
     const unsigned short* __restrict__ weight, unsigned short* __restrict__ res_out, float eps,
     const unsigned short* __restrict__ w, unsigned short* __restrict__ out,
     float* __restrict__ part, int N, int K, int span) {
-  constexpr int NS = 7, L = 2, STAGE = 64 * 128, PARTS = 16 / HV;
+  constexpr int NS = 7, L = 2, STAGE = 64 * 128, RT = row_threads(HV);
+  constexpr int PARTS = 16 / HV, V = HV * 256 / RT > 0 ? HV * 256 / RT : 1;
   // one array: of several the compiler waits for all loads under way before it reads one
-  __shared__ __attribute__((aligned(16))) char lds[NS * STAGE + HV * 2048 + 16];
+  __shared__ __attribute__((aligned(16))) char lds[NS * STAGE + (V * RT * 8) + 64];
   auto* row = reinterpret_cast<unsigned short*>(lds + NS * STAGE);
-  auto* red = reinterpret_cast<float*>(lds + NS * STAGE + HV * 2048);
-  const int tid = threadIdx.x % 256, lane = tid % WAVE;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
+  auto* red = reinterpret_cast<float*>(lds + NS * STAGE + V * RT * 8);
+  const int lane = threadIdx.x % WAVE;
   if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256) {
-    floatx4 t[PARTS][HV];
-    u64b old[HV], scale[HV];
+    const int tid = threadIdx.x - 256, wave = tid / WAVE;
+    floatx4 t[PARTS][V];
+    u64b old[V], scale[V];
 #pragma unroll
-    for (int v = 0; v < HV; ++v) {
-      const int c = min((tid + v * 256) * 4, K - 4);
+    for (int v = 0; v < V; ++v) {
+      const int c = min((tid + v * RT) * 4, K - 4);
 #pragma unroll
       for (int p = 0; p < PARTS; ++p)
         t[p][v] = *reinterpret_cast<const floatx4*>(x + (long)min(p, S - 1) * K + c);
@@ -183,9 +188,9 @@ __global__ __launch_bounds__(512) void one_row_kernel(
       return (u64b)v[3] << 48 | (u64b)v[2] << 32 | (u64b)v[1] << 16 | v[0];
     };
     float ss = 0.f;
-    u64b kept[HV];
+    u64b kept[V];
 #pragma unroll
-    for (int v = 0; v < HV; ++v) {
+    for (int v = 0; v < V; ++v) {
       unsigned short b[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -193,7 +198,7 @@ __global__ __launch_bounds__(512) void one_row_kernel(
 #pragma unroll
         for (int p = 0; p < PARTS; ++p) y += p < S ? t[p][v][j] : 0.f;
         y = bf16_to_f32(f32_to_bf16(y)) + bf16_to_f32((unsigned short)(old[v] >> (16 * j)));
-        if ((tid + v * 256) * 4 < K) ss += y * y;
+        if ((tid + v * RT) * 4 < K) ss += y * y;
         b[j] = f32_to_bf16(y);
       }
       kept[v] = four(b);
@@ -201,10 +206,13 @@ __global__ __launch_bounds__(512) void one_row_kernel(
     ss = wave_sum(ss);
     if (lane == 0) red[wave] = ss;
     meet();
-    const float inv = rsqrtf((red[0] + red[1] + red[2] + red[3]) / K + eps);
+    float all = 0.f;
 #pragma unroll
-    for (int v = 0; v < HV; ++v) {
-      const int c = (tid + v * 256) * 4;
+    for (int i = 0; i < RT / WAVE; ++i) all += red[i];
+    const float inv = rsqrtf(all / K + eps);
+#pragma unroll
+    for (int v = 0; v < V; ++v) {
+      const int c = (tid + v * RT) * 4;
       unsigned short b[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -217,6 +225,8 @@ __global__ __launch_bounds__(512) void one_row_kernel(
     meet();
     return;  // barriers wait for the waves that are left
   }
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int at = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * (SILU ? 32 : 64);
   const int k0 = blockIdx.y * span, steps = (min(K, k0 + span) - k0) / FEW_K;
@@ -420,8 +430,8 @@ torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor 
   if (S2 > 1) part = torch::empty({S2, 1, N}, x.options());
   else out = torch::empty({1, N}, w.options());
   const int tile = silu ? 32 : 64;
-  auto launch = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3((N + tile - 1) / tile, S2), dim3(512), 0, CUR_STREAM,
+  auto launch = [&](auto kern, int threads) {
+    hipLaunchKernelGGL(kern, dim3((N + tile - 1) / tile, S2), dim3(threads), 0, CUR_STREAM,
                        x.data_ptr<float>(), (int)S, (const unsigned short*)res.data_ptr(),
                        (const unsigned short*)weight.data_ptr(),
                        (unsigned short*)res_out.data_ptr(), (float)eps,
@@ -433,8 +443,8 @@ torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor 
   };
   auto form = [&](auto hv) {
     constexpr int HV = decltype(hv)::value;
-    if (silu) launch(one_row_kernel<HV, true>);
-    else launch(one_row_kernel<HV, false>);
+    if (silu) launch(one_row_kernel<HV, true>, 256 + row_threads(HV));
+    else launch(one_row_kernel<HV, false>, 256 + row_threads(HV));
   };
   if (K <= 1024) form(std::integral_constant<int, 1>{});
   else if (K <= 2048) form(std::integral_constant<int, 2>{});
