@@ -265,8 +265,9 @@ class HybridForCausalLM(nn.Module):
 
     @torch.inference_mode()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        logits = ops.linear(hidden, self.lm_head)
-        return logits.float() if self.logit_scale is None else logits * self.logit_scale
+        if self.logit_scale is None:
+            return ops.linear_float(hidden, self.lm_head)
+        return ops.linear(hidden, self.lm_head) * self.logit_scale
 
     @torch.inference_mode()
     def load_tensors(self, get) -> None:

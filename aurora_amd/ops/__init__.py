@@ -244,6 +244,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return F.linear(x, weight) if y is None else y
 
 
+def linear_float(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """``linear(x, weight).float()``, rounded all the same; without a pass of its own where few
+    rows have many outputs."""
+    y = _hip.own_product(x, weight, 3) if x.is_cuda and _hip is not None else None
+    return linear(x, weight).float() if y is None else y
+
+
 class Unnormed(NamedTuple):
     """A row whose norm is done by the product that reads it (``norm_ahead``)."""
 

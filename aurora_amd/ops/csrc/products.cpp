@@ -10,11 +10,13 @@
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 bool one_row_fits(long S, long K);
+bool float_few_rows_fits(long N, long K);
+torch::Tensor float_few_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
 bool large_takes(long N, long K);
 torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target);
 
-enum { WHOLE = 0, PARTS = 1, SILU = 2 };
+enum { WHOLE = 0, PARTS = 1, SILU = 2, FLOAT = 3 };
 
 static long megabytes(long N, long K) { return (N * K * 2) >> 20; }
 
@@ -135,6 +137,10 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
     if (large_takes(N, K) && many_rows_win(M, N, K, true))
       return many_rows(x, w, true);
     return {};
+  }
+  if (form == FLOAT) {
+    if (M > 128 || !few_rows_win(M, N, K, false) || !float_few_rows_fits(N, K)) return {};
+    return float_few_rows(x, w);
   }
   if (M <= 128) {
     if (form == PARTS && few_rows_win(M, N, K, true))
