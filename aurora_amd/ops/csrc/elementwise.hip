@@ -84,7 +84,7 @@ __global__ __launch_bounds__(PARTS ? 1024 : 256) void rmsnorm_kernel(
       *reinterpret_cast<shortx8*>(res_out + base + i) = kept;
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) ss += vals[j] * vals[j];
+    for (int j = 0; j < 8; ++j) ss = fmaf(vals[j], vals[j], ss);  // (one order for every N)
   };
   if constexpr (N > 0) {
 #pragma unroll
