@@ -182,9 +182,43 @@ struct Delta {
   }
 };
 
+// The sum of a row's squares of which a thread holds N vectors of four; every thread gets it. In
+// the order of the kernel above, to the last bit: 512 threads leave it to their upper half, which
+// adds what 256 threads of twice as many vectors would (pass: N vectors of each lower thread).
+template <int NTHR, int N>
+DEVINL float row_squares(const floatx4 (&r)[N], int W, float* red, floatx4 (*pass)[256]) {
+  const int t = threadIdx.x;
+  float ss = 0.f;
+  auto add = [&](const floatx4 v, int i) {
+    if (i < W)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ss = fmaf(v[j], v[j], ss);
+  };
+  if constexpr (NTHR != 512) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) add(r[k], (t + k * NTHR) * 4);
+    return block_sum<NTHR / WAVE>(ss, red);
+  }
+  if (t < 256)
+#pragma unroll
+    for (int k = 0; k < N; ++k) pass[k][t] = r[k];
+  __syncthreads();
+  if (t >= 256) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+      add(pass[k][t - 256], (t - 256 + k * NTHR) * 4);
+      add(r[k], (t + k * NTHR) * 4);
+    }
+    ss = wave_sum(ss);
+    if (t % WAVE == 0) red[t / WAVE] = ss;
+  }
+  __syncthreads();
+  return red[4] + red[5] + red[6] + red[7];
+}
+
 // The same for rows of up to N * 4 * NTHR elements, a multiple of 4: a thread holds its N
 // vectors, so that what can be read is asked for at once, the weight and the convolution's
-// past before the sums they wait for, and nothing goes through LDS.
+// past before the sums they wait for, and nothing but squares goes through LDS.
 template <typename T, int NTHR, bool POST, int N, bool CONV>
 __global__ __launch_bounds__(NTHR) void residual_rmsnorm_held_kernel(
     float* __restrict__ x, const float* __restrict__ weight, Delta<T> delta,
@@ -193,6 +227,7 @@ __global__ __launch_bounds__(NTHR) void residual_rmsnorm_held_kernel(
     const float* __restrict__ step, T* __restrict__ out, ConvTail<T> cv, int W, float eps,
     float offset) {
   __shared__ float red[NTHR / WAVE];
+  __shared__ floatx4 pass[NTHR == 512 ? N : 1][256];
   const long base = (long)blockIdx.x * W;
   const int* pl = place + (long)blockIdx.x * top;
   const float* gt = gate + (long)blockIdx.x * top;
@@ -239,15 +274,9 @@ __global__ __launch_bounds__(NTHR) void residual_rmsnorm_held_kernel(
   for (int k = 0; k < N; ++k) wt[k] = ld4(weight + at[k]);
   if constexpr (POST) {
     floatx4 ps[N];
-    float rs = 0.f;
 #pragma unroll
-    for (int k = 0; k < N; ++k) {
-      ps[k] = ld4(post + at[k]);
-      if (in(k))
-#pragma unroll
-        for (int j = 0; j < 4; ++j) rs += r[k][j] * r[k][j];
-    }
-    const float rinv = rsqrtf(block_sum<NTHR / WAVE>(rs, red) / W + eps);
+    for (int k = 0; k < N; ++k) ps[k] = ld4(post + at[k]);
+    const float rinv = rsqrtf(row_squares<NTHR>(r, W, red, pass) / W + eps);
 #pragma unroll
     for (int k = 0; k < N; ++k) r[k] = a[k] + r[k] * rinv * ps[k];
   }
@@ -255,42 +284,49 @@ __global__ __launch_bounds__(NTHR) void residual_rmsnorm_held_kernel(
 #pragma unroll
     for (int k = 0; k < N; ++k) r[k] += ld4(step + at[k]);
   }
-  float ss = 0.f;
   const bool changed = delta || y || step;
-#pragma unroll
-  for (int k = 0; k < N; ++k)
-    if (in(k)) {
-      if (changed) st4(x + base + at[k], r[k]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) ss += r[k][j] * r[k][j];
-    }
   const int keep = cv.taps - 1;
   const int slot = CONV ? cv.slots[blockIdx.x] : -1;
   const int pos = CONV ? cv.pos[blockIdx.x] : 0;
   T* ring = cv.ring + (long)max(slot, 0) * keep * W;
-  floatx4 past[N], now[N];
+  const int known = slot >= 0 ? min(keep, pos) : 0;  // rows of the past
+  // of which some, and what they are multiplied by, come with the rest; they are added behind
+  // the row itself, as ever
+  constexpr int AHEAD = 3;
+  floatx4 now[N], past[N][AHEAD], tap[N][AHEAD];
+  auto before = [&](int k, int b, floatx4& p, floatx4& w) {
+    w = ld4(cv.w + (long)(keep - b) * W + at[k]);
+    p = ld4(ring + (long)((pos - b) % keep) * W + at[k]);
+  };
   if constexpr (CONV) {
-    const int known = slot >= 0 ? min(keep, pos) : 0;  // rows of the past
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      const float* w = cv.w + (long)keep * W + at[k];
-      now[k] = ld4(w);
-      past[k] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-      for (int b = 1; b <= known; ++b)
-        past[k] += ld4(w - (long)b * W) * ld4(ring + (long)((pos - b) % keep) * W + at[k]);
+      now[k] = ld4(cv.w + (long)keep * W + at[k]);
+#pragma unroll
+      for (int b = 0; b < AHEAD; ++b)
+        if (b < known) before(k, b + 1, past[k][b], tap[k][b]);
     }
   }
-  const float inv = rsqrtf(block_sum<NTHR / WAVE>(ss, red) / W + eps);
+  const float inv = rsqrtf(row_squares<NTHR>(r, W, red, pass) / W + eps);
 #pragma unroll
   for (int k = 0; k < N; ++k) {
     floatx4 v = r[k] * inv * (offset + wt[k]);
     if (!in(k)) continue;
+    if (changed) st4(x + base + at[k], r[k]);
     st4(out + base + at[k], v);
     if constexpr (!CONV) continue;
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = stored(v[j], (T*)nullptr);
-    st4(cv.out + base + at[k], v + v * now[k] + past[k]);
+    floatx4 u = v + v * now[k];
+#pragma unroll
+    for (int b = 0; b < AHEAD; ++b)
+      if (b < known) u += tap[k][b] * past[k][b];
+    for (int b = AHEAD; b < known; ++b) {
+      floatx4 p, w;
+      before(k, b + 1, p, w);
+      u += w * p;
+    }
+    st4(cv.out + base + at[k], u);
     // the oldest row's place, which this thread has read
     if (slot >= 0 && keep > 0) st4(ring + (long)(pos % keep) * W + at[k], v);
   }
