@@ -368,10 +368,15 @@ class LlamaDecoderLayer(nn.Module):
         input, is a single row in parts and nobody watches the product."""
         if x.dim() != 3 or x.shape[1] != 1:
             return None
-        if what == "attn":
-            return (column_weight(self.attn.qkv_proj, True)
-                    if is_plain(self.attn, LlamaAttention) else None)
-        return column_weight(self.mlp.gate_up, False) if is_plain(self.mlp, LlamaMLP) else None
+        module, kind, inner = ((self.attn, LlamaAttention, ("parts", "_heads")) if what == "attn"
+                               else (self.mlp, LlamaMLP, ("parts",)))
+        # (a subclass's own steps are given rows, as they always were)
+        if not is_plain(module, kind) or any(
+                getattr(getattr(module, n), "__func__", None) is not getattr(kind, n)
+                for n in inner):
+            return None
+        return (column_weight(module.qkv_proj, True) if kind is LlamaAttention
+                else column_weight(module.gate_up, False))
 
 
 class LlamaForCausalLM(nn.Module):
