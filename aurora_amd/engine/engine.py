@@ -748,6 +748,7 @@ class LLMEngine:
         """``ops.stage_decode`` of whatever a sequence may hold."""
         ids, (pos, slot, ctx, state), tables = parts
         B, width = len(seqs), tables.shape[1]
+        keys.fill_(-2)  # (of nobody, also where a sequence is refused below)
         self._host_i64[:B] = torch.tensor([s.token_ids[-1] for s in seqs], dtype=torch.int64)
         ids.copy_(self._host_i64[:len(ids)])
         for row, idle, own in (
@@ -760,7 +761,7 @@ class LLMEngine:
         for row, s in zip(tables, seqs):
             n = min(len(s.pages), width)
             row[:n] = torch.tensor(s.pages[:n], dtype=torch.int32)
-        keys[:B], keys[B:] = -2, -1
+        keys[B:] = -1
 
     def _reserve_scratch(self) -> None:
         """The page that idle rows of captured batches write, and the staged token ids."""

@@ -180,8 +180,9 @@ py::object pack_rows(py::list rows, torch::Device device) {
 // int32 positions, cache slots, context lengths, state slots and block tables of ``width``
 // pages. Rows past the sequences are idle: they write the scratch slot and touch no state. A
 // table's row is written again only when its sequence's serial, generation or number of pages,
-// ``keys`` [bucket, 3], has changed; keys of -1 are idle rows'. False, and nothing done, where a
-// sequence holds anything but lists of plain integers that fit.
+// ``keys`` [bucket, 3], has changed; keys of -1 are idle rows', of -2 nobody's. False, and nothing
+// sent, where a sequence holds anything but lists of plain integers that fit: tables before its
+// own may have been written, each with its key.
 bool stage_decode(py::list seqs, torch::Tensor ids, torch::Tensor host, torch::Tensor keys,
                   torch::Tensor inputs, long width, long page, long scratch_page,
                   long scratch_slot) {

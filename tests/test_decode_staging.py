@@ -89,6 +89,26 @@ def test_left_to_python(what):
     assert torch.equal(a.inputs, b.inputs)
 
 
+@pytest.mark.parametrize("what", ["large page", "large slot", "empty"])
+def test_refused_by_both(what):
+    """A sequence that staging in Python refuses as well leaves no row that is taken for staged."""
+    a, b = _Staging(4), _Staging(4)
+    good, other, odd = (_sequence(20, pages) for pages in ([3, 4], [5, 6], [7, 8]))
+    assert a.native([good, other])
+    if what == "large page":
+        odd.pages[0] = 1 << 40
+    elif what == "large slot":
+        odd.pages[1] = 1 << 30
+    else:
+        odd.token_ids = []
+    assert not a.native([odd, other])
+    with pytest.raises((RuntimeError, ValueError, IndexError, OverflowError)):
+        a.python([odd, other])
+    assert a.native([good, other])
+    b.python([good, other])
+    assert torch.equal(a.inputs, b.inputs)
+
+
 @pytest.mark.gpu
 def test_rows_on_the_device():
     assert ops.pack_rows([3, -1, 1 << 40], "cuda").tolist() == [3, -1, 1 << 40]
