@@ -12,7 +12,8 @@ model the engine steps directly.
 """
 from __future__ import annotations
 
-from dataclasses import dataclass, replace
+from copy import copy
+from dataclasses import dataclass
 from typing import List, Optional, Tuple
 
 import torch
@@ -136,7 +137,7 @@ class LlamaAttention(nn.Module):
         elif meta.mode == "decode":
             o = ops.paged_attention_decode(
                 q, k_cache, v_cache, meta.block_tables, meta.context_lens, self.scale,
-                marks=meta.marks,
+                marks=getattr(meta, "marks", None),
             )
         else:  # mixed: prefill chunks + decode tokens in one forward — the
             # projections/norms run on the whole packed batch (bigger GEMMs),
@@ -151,7 +152,8 @@ class LlamaAttention(nn.Module):
             if T > Tp:
                 ops.paged_attention_decode(
                     q[Tp:], k_cache, v_cache, meta.dec_block_tables,
-                    meta.dec_context_lens, self.scale, out=o[Tp:], marks=meta.marks,
+                    meta.dec_context_lens, self.scale, out=o[Tp:],
+                    marks=getattr(meta, "marks", None),
                 )
         return o.reshape(T, self.n_heads * self.head_dim)
 
@@ -421,10 +423,12 @@ class LlamaForCausalLM(nn.Module):
     ) -> torch.Tensor:
         x = self.embed(input_ids)
         residual = None
-        tables = {"decode": meta.block_tables, "mixed": meta.dec_block_tables}.get(meta.mode)
-        if tables is not None and kv_caches:
-            meta = replace(meta, marks=ops.decode_marks(
-                self.spec.n_heads // pdist.tp_world_size(), kv_caches[0][0], tables))
+        if isinstance(meta, AttnMetadata):  # of another kind every layer makes its own marks
+            tables = {"decode": meta.block_tables, "mixed": meta.dec_block_tables}.get(meta.mode)
+            if tables is not None and kv_caches:
+                meta = copy(meta)
+                meta.marks = ops.decode_marks(
+                    self.spec.n_heads // pdist.tp_world_size(), kv_caches[0][0], tables)
         # layers that somebody watches or has replaced are called and get no parts
         plain = [is_plain(layer, LlamaDecoderLayer) for layer in self.layers] + [True]
         for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):

@@ -1,4 +1,8 @@
 """Modules that a user watches or replaces are called, and see whole results."""
+import collections
+import dataclasses
+import types
+
 import pytest
 import torch
 import torch.nn as nn
@@ -31,6 +35,33 @@ def _step(m, T):
                         block_tables=i32(0, 1)[None], context_lens=i32(T),
                         cu_seqlens_q=i32(0, T))
     return m(torch.arange(T, device=dev) % 50, caches, meta)
+
+
+def _decode(m, kind, n=3, past=40):
+    """The hidden states of one token each behind n contexts."""
+    spec, dev, P = m.spec, m.embed.weight.device, 64
+    g = torch.Generator().manual_seed(n)
+    caches = [tuple(torch.randn(2 * n * 8, spec.n_kv_heads, P, spec.head_dim, generator=g)
+                    .to(dev, m.dtype) for _ in range(2)) for _ in range(spec.n_layers)]
+    at = torch.full((n,), past, dtype=torch.int32, device=dev)
+    tables = torch.arange(16 * n, dtype=torch.int32, device=dev).view(n, 16)
+    return m(torch.arange(n, device=dev), caches, kind(
+        mode="decode", positions=at, slot_mapping=tables[:, past // P] * P + past % P,
+        block_tables=tables, context_lens=at + 1))
+
+
+@dataclasses.dataclass
+class _Counted(AttnMetadata):
+    layers: int = dataclasses.field(default=0, init=False)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("kind", [types.SimpleNamespace, _Counted, collections.namedtuple(
+    "Step", "mode positions slot_mapping block_tables context_lens")])
+def test_metadata_of_another_kind(device, kind):
+    """What has the fields that a decoding step reads will do; contexts are cut or may be."""
+    m = _model("tiny-llama", device)
+    _same(_decode(m, kind, past=900), _decode(m, AttnMetadata, past=900))
 
 
 def _same(a, b):
