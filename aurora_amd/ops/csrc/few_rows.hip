@@ -163,7 +163,10 @@ constexpr int row_threads(int hv) { return hv > 1 ? 512 : 256; }
 // parts' way to every CU (64 KB). A layer of one row, its two norms before and in the products,
 // cold weights: 4096 wide, 28672 and 6144 outputs, 95.9 and 91.8 us; 2048, 16384 and 3072, 41.0
 // and 38.1; 1024, 8192 and 2048, 24.5 and 20.6. With the norm by the waves that load W (its
-// loads are then waited for with W's) 93.7, 38.5 and 21.3.
+// loads are then waited for with W's) 93.7, 38.5 and 21.3. The two products alone with their
+// norms, before and in them: 60.8 and 57.8, 27.2 and 24.4, 15.7 and 12.4; 8192 wide, 16384 and
+// 10240 outputs, 106.0 and 102.2 (squares in the order of this kernel's threads: 57.9, 24.5, 12.2
+// and 101.6, but a row in ten thousand with an element off by its last bit).
 template <int HV, bool SILU>
 __global__ __launch_bounds__(256 + row_threads(HV)) void one_row_kernel(
     const float* __restrict__ x, int S, const unsigned short* __restrict__ res,
@@ -179,11 +182,19 @@ __global__ __launch_bounds__(256 + row_threads(HV)) void one_row_kernel(
   const int lane = threadIdx.x % WAVE;
   if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256) {
     const int tid = threadIdx.x - 256, wave = tid / WAVE;
+    // Squares are added as rmsnorm_residual adds them, whose threads hold eight values side by
+    // side: here two vectors of one thread, or those of two lanes, whose pairs are then of every
+    // other thread there, so that two waves end where one wave's last step adds its halves.
+    auto column = [&](int v) {
+      if constexpr (V > 1) return (tid + v / 2 * RT) * 8 + v % 2 * 4;
+      const int eight = wave / 2 * WAVE + (lane & ~1) + wave % 2;
+      return eight * 8 + lane % 2 * 4;
+    };
     floatx4 t[PARTS][V];
     u64b old[V], scale[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
-      const int c = min((tid + v * RT) * 4, K - 4);
+      const int c = min(column(v), K - 4);
 #pragma unroll
       for (int p = 0; p < PARTS; ++p)
         t[p][v] = *reinterpret_cast<const floatx4*>(x + (long)min(p, S - 1) * K + c);
@@ -193,32 +204,52 @@ __global__ __launch_bounds__(256 + row_threads(HV)) void one_row_kernel(
     auto four = [](const unsigned short* v) {
       return (u64b)v[3] << 48 | (u64b)v[2] << 32 | (u64b)v[1] << 16 | v[0];
     };
-    float ss = 0.f;
     u64b kept[V];
+    floatx4 y[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) {
       unsigned short b[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        float y = 0.f;
+        float sum = 0.f;
 #pragma unroll
-        for (int p = 0; p < PARTS; ++p) y += p < S ? t[p][v][j] : 0.f;
-        y = bf16_to_f32(f32_to_bf16(y)) + bf16_to_f32((unsigned short)(old[v] >> (16 * j)));
-        if ((tid + v * RT) * 4 < K) ss += y * y;
-        b[j] = f32_to_bf16(y);
+        for (int p = 0; p < PARTS; ++p) sum += p < S ? t[p][v][j] : 0.f;
+        sum = bf16_to_f32(f32_to_bf16(sum)) + bf16_to_f32((unsigned short)(old[v] >> (16 * j)));
+        b[j] = f32_to_bf16(sum);
+        y[v][j] = column(v) < K ? sum : 0.f;
       }
       kept[v] = four(b);
     }
-    ss = wave_sum(ss);
-    if (lane == 0) red[wave] = ss;
+    auto squares = [&](const floatx4 a, float ss) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) ss = fmaf(a[j], a[j], ss);
+      return ss;
+    };
+    if constexpr (V > 1) {
+#pragma unroll
+      for (int v = 0; v < V; v += 2) {
+        const float ss = wave_sum(squares(y[v + 1], squares(y[v], 0.f)));
+        if (lane == 0) red[v / 2 * (RT / WAVE) + wave] = ss;
+      }
+    } else {
+      float ss = squares(y[0], __shfl_xor(squares(y[0], 0.f), 1, WAVE));  // odd lanes'
+#pragma unroll
+      for (int off = 32; off > 1; off >>= 1) ss += __shfl_xor(ss, off, WAVE);
+      if (lane == 1) red[wave] = ss;
+    }
     meet();
     float all = 0.f;
+    if constexpr (V > 1) {
 #pragma unroll
-    for (int i = 0; i < RT / WAVE; ++i) all += red[i];
+      for (int i = 0; i < V / 2 * (RT / WAVE); ++i) all += red[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < RT / WAVE; i += 2) all += red[i] + red[i + 1];
+    }
     const float inv = rsqrtf(all / K + eps);
 #pragma unroll
     for (int v = 0; v < V; ++v) {
-      const int c = (tid + v * RT) * 4;
+      const int c = column(v);
       unsigned short b[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -428,7 +459,9 @@ torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w) {
   return out;
 }
 
-// The kernel above where it has a form: x [S, 1, K] in fp32, S parts.
+// The kernel above where it has a form: x [S, 1, K] in fp32, S parts, of which a thread holds 64
+// values at most. ``parts_of`` makes more for rows 1088 to 1792, 2112 to 3264 and 4160 to 5440
+// wide, whose norms stay kernels of their own.
 bool one_row_fits(long S, long K) {
   return S > 1 && K % FEW_K == 0 && K <= ROW_MOST &&
          S <= (K <= 1024 ? 16 : K <= 2048 ? 8 : K <= 4096 ? 4 : 2);

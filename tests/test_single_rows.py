@@ -26,6 +26,16 @@ def left(monkeypatch):
     return seen
 
 
+def test_bits_of_separate_norms(left, monkeypatch):
+    m = _model("smoke-llama", "cuda")
+    got = _step(m, 1)
+    # the first layer's first norm reads the embedding, the model's last the last layer's product
+    assert sum(left) == len(left) == 2 * len(m.layers) - 1
+    monkeypatch.setattr(ops, "norm_ahead", lambda x, res, w, eps, *_: ops.rmsnorm_residual(
+        x, res, w, eps))
+    assert torch.equal(_step(m, 1), got)
+
+
 class _Heads(LlamaAttention):
     def _heads(self, x, *args):
         assert isinstance(x, torch.Tensor) and x.dim() == 2

@@ -79,9 +79,10 @@ WATCHED = ["layers.0", "layers.1", "layers.0.attn", "layers.0.attn.qkv_proj",
 
 @pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("name", WATCHED)
-def test_hooks_of_decoders(name, device):
+@pytest.mark.parametrize("T", [21, 1])  # of one row norms may be left to products
+def test_hooks_of_decoders(name, device, T):
     m = _model("tiny-llama", device)
-    T, before = 21, _step(_model("tiny-llama", device), 21)
+    before = _step(_model("tiny-llama", device), T)
     seen = []
 
     def look(module, args, out):
@@ -96,7 +97,8 @@ def test_hooks_of_decoders(name, device):
 
 @pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("name", ["attn.qkv_proj", "attn.o_proj", "mlp.gate_up", "mlp.down"])
-def test_replaced_projections(name, device):
+@pytest.mark.parametrize("T", [21, 1])
+def test_replaced_projections(name, device, T):
     """An adapter in place of a projection, a forward of the instance's own."""
     m, way = _model("tiny-llama", device), _model("tiny-llama", device)
 
@@ -114,11 +116,11 @@ def test_replaced_projections(name, device):
     own.forward = lambda x, f=own.forward: 2 * f(x)
     plain = _model("tiny-llama", device)
     plain.get_submodule(f"{parent}.{child}").weight.data.mul_(2)  # exact
-    want = _step(plain, 21)
-    plain = _step(_model("tiny-llama", device), 21)
+    want = _step(plain, T)
+    plain = _step(_model("tiny-llama", device), T)
     assert (plain - want).norm() > 2 ** -4 * want.norm()
-    _same(_step(m, 21), want)
-    _same(_step(way, 21), want)
+    _same(_step(m, T), want)
+    _same(_step(way, T), want)
 
 
 @pytest.mark.parametrize("device", DEVICES)
