@@ -43,8 +43,9 @@ DEVINL void await_stage() {
 
 // WN rows of W, 16 MT rows of x, NS stages. SILU: W is gate's N rows, then up's; a wave's 16
 // rows are 8 of each. Outputs are bf16, or with ``part`` sums over ``span`` of K; with both they
-// go to ``part``, rounded to bf16 first.
-template <int WN, int MT, int NS, bool SILU>
+// go to ``part``, rounded to bf16 first. ROUTER: a workgroup y of Y takes every Y-th step and keeps
+// the sums of its steps' two halves apart, parts 2 y and 2 y + 1; z are blocks of 16 MT rows of x.
+template <int WN, int MT, int NS, bool SILU, bool ROUTER = false>
 __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
     const unsigned short* x, const unsigned short* w, unsigned short* out, float* part, int M,
     int N, int K, int span, long ldx) {
@@ -56,13 +57,16 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int at = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * (SILU ? WN / 2 : WN);
-  const int k0 = blockIdx.y * span, steps = (min(K, k0 + span) - k0) / FEW_K;
+  const int k0 = blockIdx.y * (ROUTER ? FEW_K : span), m0 = ROUTER ? blockIdx.z * 16 * MT : 0;
+  const int stride = ROUTER ? gridDim.y * FEW_K : FEW_K;
+  const int steps = ROUTER ? max(K - k0 + stride - 1, 0) / stride
+                           : (min(K, k0 + span) - k0) / FEW_K;
   const unsigned short* src[L];
 #pragma unroll
   for (int l = 0; l < L; ++l) {
     const int r = (tid + l * NT) >> 3, unit = (tid & 7) ^ (r & 7);
     long row;  // rows past the end are the last again
-    if (l >= WN * 8 / NT) row = min(r - WN, M - 1);
+    if (l >= WN * 8 / NT) row = min(m0 + r - WN, M - 1);
     else if constexpr (SILU) row = min(n0 + r / 16 * 8 + r % 8, N - 1) + (long)(r % 16 / 8) * N;
     else row = min(n0 + r, N - 1);
     src[l] = (l >= WN * 8 / NT ? x + row * ldx : w + row * K) + k0 + unit * 8;
@@ -71,12 +75,13 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
     char* stage = lds + s % NS * STAGE;
 #pragma unroll
     for (int l = 0; l < L; ++l)
-      __builtin_amdgcn_global_load_lds((gptr_t)(src[l] + (long)s * FEW_K),
+      __builtin_amdgcn_global_load_lds((gptr_t)(src[l] + (long)s * stride),
                                        (lptr_t)(stage + (l * NT + wave * WAVE) * 16), 16, 0, 0);
   };
-  floatx4 acc[MT];
+  constexpr int SUMS = ROUTER ? 2 : 1;
+  floatx4 acc[SUMS][MT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) acc[m] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int m = 0; m < SUMS * MT; ++m) acc[m / MT][m % MT] = floatx4{0.f, 0.f, 0.f, 0.f};
   auto compute = [&](int s) {
     const char* stage = lds + s % NS * STAGE;
     frag_u wf[2], xf[2][MT];  // all read before the first product: one latency a step
@@ -93,7 +98,8 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int m = 0; m < MT; ++m)
-        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h].v, xf[h][m].v, acc[m], 0, 0, 0);
+        acc[h % SUMS][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h].v, xf[h][m].v,
+                                                                   acc[h % SUMS][m], 0, 0, 0);
   };
   for (int s = 0; s < min(steps, NS - 1); ++s) issue(s);
   int s = 0;
@@ -107,8 +113,9 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
 
   const int n = n0 + (SILU ? wave * 8 + (g & 1) * 4 : wave * 16 + g * 4);
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    floatx4 y = acc[m];
+  for (int u = 0; u < SUMS * MT; ++u) {
+    const int m = u % MT;
+    floatx4 y = acc[u / MT][m];
     if constexpr (SILU) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -117,7 +124,7 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
       }
       if (g >= 2) continue;
     }
-    const int row = m * 16 + at;
+    const int row = m0 + m * 16 + at;
     if (row >= M) continue;
     const bool whole = n + 4 <= N && N % 4 == 0;
     if (!SILU && part) {
@@ -126,7 +133,7 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
         y = floatx4{__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u),
                     __uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u)};
       }
-      float* dst = part + ((long)blockIdx.y * M + row) * N + n;
+      float* dst = part + ((long)(blockIdx.y * SUMS + u / MT) * M + row) * N + n;
       if (whole) *reinterpret_cast<floatx4*>(dst) = y;
       else
 #pragma unroll
@@ -407,6 +414,24 @@ torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts) {
   else launch<64, 8, 3, false>(x, w, op, pp, N, S, span);
   if (S == 1) return out;
   return raw ? part : add_parts(part);
+}
+
+// A router's logits in 16 parts [16, M, N] in fp32 that hold what the 16 waves of
+// moe_route_kernel sum up, so that choices and weights do not depend on the number of tokens.
+torch::Tensor router_rows(const torch::Tensor& x, const torch::Tensor& w) {
+  check(x, w);
+  const long M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(x.is_contiguous() && (uintptr_t)x.data_ptr() % 16 == 0 && M > 0 && N > 0,
+              "contiguous tokens");
+  auto part = torch::empty({16, M, N}, x.options().dtype(torch::kFloat32));
+  // A wave takes 16 outputs of 16 rows (32 or 64 of 32 rows, in two or four waves: 64 x 2048, 64
+  // tokens, 6.8 and 7.1 us, the choices included, and 6.5; 128 x 4096 10.4, 11.0 and 9.7).
+  hipLaunchKernelGGL((few_rows_kernel<16, 1, 9, false, true>),
+                     dim3((N + 15) / 16, 8, (M + 15) / 16), dim3(64), 0, CUR_STREAM,
+                     (const unsigned short*)x.data_ptr(), (const unsigned short*)w.data_ptr(),
+                     nullptr, part.data_ptr<float>(), (int)M, (int)N, (int)K, 0, K);
+  HIP_CHECK_KERNEL();
+  return part;
 }
 
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw) {

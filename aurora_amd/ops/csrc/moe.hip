@@ -261,27 +261,30 @@ __global__ __launch_bounds__(1024) void moe_route_kernel(
                    top, groups, keep, scale);
 }
 
-torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts);
+torch::Tensor router_rows(const torch::Tensor& x, const torch::Tensor& w);  // of few_rows.hip
 
 // Few tokens: a workgroup for 16 of them reads the whole router, at some 25 GB/s of a CU, where
-// the products' kernel of few rows spreads it over 16 and more, and a second launch adds the
-// parts and chooses. Cold routers, us, whole and in parts, of 1, 16, 64 and 128 tokens:
-//   E x W       1             16            64            128
-//   8 x 4096    5.7 and 5.2   8.8 and 5.8   9.0 and 6.9   9.0 and 8.4
-//   16 x 2880   6.7 and 6.2   9.5 and 6.3   9.7 and 7.3   9.7 and 8.6
-//   32 x 2048   7.5 and 6.0   9.8 and 6.4   10.0 and 7.1  10.2 and 8.1
-//   64 x 2048   11.2 and 6.0  13.5 and 6.4  13.7 and 7.0  13.9 and 7.8
-//   128 x 4096  34.9 and 8.3  41.1 and 9.2  41.6 and 10.4 41.6 and 11.5
-// and on the other side
-//   8 x 2880    4.9 and 5.1   7.2 and 5.6   7.3 and 6.6   7.3 and 8.0
-//   16 x 2048   5.8 and 6.0   8.1 and 6.3   8.3 and 7.0   8.3 and 8.2
-//   32 x 1024   5.6 and 5.6   7.2 and 5.8   7.4 and 6.6   7.5 and 7.6
-//   64 x 512    5.5 and 5.5   6.8 and 5.9   7.0 and 6.5   7.0 and 7.3
-//   128 x 256   7.3 and 7.1   8.6 and 7.4   8.8 and 8.0   8.8 and 8.9
+// the products' kernel of few rows spreads it and the tokens over 8 and more, and a second launch
+// adds the parts and chooses. Both give the same bits. Cold routers, us, whole and in parts, of 1,
+// 4, 8, 16, 64 and 128 tokens:
+//   E x W       1              4             8             16            64            128
+//   8 x 4096    6.4 and 6.5    7.4 and 6.9   8.1 and 6.8   10.2 and 7.0  10.3 and 7.1  10.3 and 7.1
+//   16 x 2880   6.5 and 6.3    7.2 and 6.6   7.8 and 6.5   9.3 and 6.6   9.5 and 6.8   9.5 and 6.9
+//   64 x 2048   10.9 and 5.8   11.4 and 6.4  12.0 and 6.4  13.3 and 6.4  13.5 and 6.5  13.6 and 6.5
+//   128 x 4096  34.6 and 8.9   36.2 and 9.6  37.5 and 9.8  40.7 and 9.8  41.2 and 9.9  41.3 and 10.4
+//   8 x 2880    5.6 and 6.5    6.4 and 6.6   6.8 and 6.7   8.4 and 6.9   8.7 and 6.9   8.7 and 7.0
+//   16 x 2048   5.6 and 5.8    6.1 and 6.1   6.6 and 6.3   8.0 and 6.3   8.2 and 6.5   8.1 and 6.5
+//   32 x 1024   5.3 and 5.9    5.9 and 6.0   6.2 and 6.0   7.1 and 6.2   7.3 and 6.3   7.3 and 6.3
+//   64 x 512    5.2 and 5.7    5.6 and 5.9   5.9 and 6.0   6.7 and 6.1   6.9 and 6.2   6.9 and 6.2
+//   12 x 1536   4.8 and 6.1    5.4 and 6.3   5.7 and 6.3   6.9 and 6.3   7.1 and 6.5   7.1 and 6.5
+//   16 x 1024   4.6 and 5.6    4.9 and 5.9   5.3 and 6.0   6.2 and 6.1   6.5 and 6.2   6.4 and 6.3
+//   8 x 1024    4.2 and 5.9    4.6 and 6.2   5.0 and 6.3   5.9 and 6.3   6.2 and 6.4   6.2 and 6.4
+// The line is what the first workgroup reads, 40000 values: at it (16 x 2048, 4 tokens; 32 x 1024,
+// 8; 64 x 512, 16) the two are alike or parts ahead; what it gives up is 0.4 us of 128 x 256.
 static bool route_in_parts(const torch::Tensor& h, const torch::Tensor& router) {
   const long T_ = h.size(0), W = h.size(1), E = router.size(0);
   return h.dtype() == torch::kBFloat16 && T_ <= 128 && W % 64 == 0 && W >= 256 &&
-         W * (E + 12) >= 76000 && (uintptr_t)router.data_ptr() % 16 == 0 &&
+         W * (E + std::min(T_, 16L)) >= 40000 && (uintptr_t)router.data_ptr() % 16 == 0 &&
          (uintptr_t)h.data_ptr() % 16 == 0;
 }
 
@@ -301,7 +304,7 @@ static std::vector<torch::Tensor> route(const torch::Tensor& h, const torch::Ten
   auto gate = torch::empty({T_, top}, h.options().dtype(torch::kFloat32));
   if (T_ == 0) return {sel, gate};
   if (route_in_parts(h, router)) {
-    const auto part = few_rows(h, router, true, std::min(16L, W / 128));
+    const auto part = router_rows(h, router);
     hipLaunchKernelGGL(moe_choose_kernel<ROUTER>, dim3(T_), dim3(WAVE), (1024 + E) * 4, CUR_STREAM,
                        part.template data_ptr<float>(), (int)part.size(0),
                        bias ? bias->data_ptr<float>() : nullptr, sel.data_ptr<int>(),
