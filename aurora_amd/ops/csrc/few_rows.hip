@@ -450,15 +450,13 @@ torch::Tensor float_few_rows(torch::Tensor x, torch::Tensor w) {
   check(x, w);
   x = readable(x);
   const long M = x.size(0), K = x.size(1), N = w.size(0);
-  TORCH_CHECK(float_few_rows_fits(N, K), "K is cut for few outputs");
+  TORCH_CHECK(M <= 64 && float_few_rows_fits(N, K), "at most 64 rows, K is cut for few outputs");
   auto out = torch::empty({M, N}, x.options().dtype(torch::kFloat32));
   if (M == 0 || N == 0) return out;
   float* pp = out.data_ptr<float>();
   auto* round = (unsigned short*)pp;
   if (M <= 32) launch<64, 2, 6, false>(x, w, round, pp, N, 1, K);
-  else if (M <= 64) launch<64, 4, 5, false>(x, w, round, pp, N, 1, K);
-  else if (M <= 96) launch<64, 6, 4, false>(x, w, round, pp, N, 1, K);
-  else launch<64, 8, 3, false>(x, w, round, pp, N, 1, K);
+  else launch<64, 4, 5, false>(x, w, round, pp, N, 1, K);
   return out;
 }
 

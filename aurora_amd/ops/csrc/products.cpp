@@ -139,7 +139,8 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
     return {};
   }
   if (form == FLOAT) {
-    if (M > 128 || !few_rows_win(M, N, K, false) || !float_few_rows_fits(N, K)) return {};
+    // (of more than 64 rows none that few_rows_win names has its K whole)
+    if (M > 64 || !few_rows_win(M, N, K, false) || !float_few_rows_fits(N, K)) return {};
     return float_few_rows(x, w);
   }
   if (M <= 128) {

@@ -8,12 +8,14 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M", [1, 17, 32, 33, 64, 65, 96, 97, 128])
-@pytest.mark.parametrize("N", [8256, 16387, 40001])
-@pytest.mark.parametrize("K", [64, 2048, 4160])
+@pytest.mark.parametrize("N,K", [(n, k) for n in (8256, 16387, 40001) for k in (64, 2048, 4160)]
+                         + [(48, 128), (516, 64)])
 def test_bits(M, N, K):
     x = torch.randn(M, K, device="cuda").bfloat16()
     w = torch.randn(N, K, device="cuda").bfloat16()
     x[0, 0] = float("inf")
+    mine = ops._hip.own_product(x, w, 3) is not None
+    assert mine == (M <= 64 and (N * K * 2 >> 20 <= 128 or M <= 32 and K < 4096))
     y = ops.linear_float(x, w)
     assert y.dtype == torch.float32
     assert torch.equal(y.view(torch.int32), ops.linear(x, w).float().view(torch.int32))
