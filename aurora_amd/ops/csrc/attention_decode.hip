@@ -99,8 +99,9 @@ DEVINL bool find_split(const int* ctx, int B, int length, const Seen& seen, int 
 // are short. (32 heads over 8, 128 wide, in the order of the batch and so: 96 sequences of 500 to
 // 2900 keys 143 and 124 us, all of their mean 119; 128 of 50 to 1500 87 and 80; 64 of 300 to 8000
 // 232 and 220; 41 of 700 to 2600 74 and 66; 100 of 600 56.2 and 57.1, of 50 16.2 and 16.6.) The
-// sequence whose context is the idx-th longest to a 64th of the longest, in the
-// batch's order where they are alike, and its length; of at most 64 N. All lanes of a wave.
+// sequence whose context is the idx-th longest, to between a 64th and a 32nd of the
+// longest, in the batch's order where they are alike, and its length; of at most 64 N. All
+// lanes of a wave.
 template <int N>
 DEVINL int ranked(const int* ctx, int B, int idx, int lane, int& length) {
   int n[N], most = 0;

@@ -1,10 +1,8 @@
 // Fused element-wise / normalisation kernels (bf16, gfx950).
 //
-// All memory-bound: the design rule is G13 of the platform guide — bf16
-// loads vectorized as shortx8 (16 B/lane), grid-stride, fused passes so a
-// tensor is read exactly once.  These replace the reference's CPU-side
-// text plumbing with the engine's per-layer hot path (no reference analog;
-// SURVEY.md preamble table row 1).
+// All memory-bound: bf16 loads vectorized as shortx8 (16 B/lane), grid-stride,
+// fused passes so a tensor is read exactly once. The engine's per-layer hot path,
+// without an analog in the reference.
 #include <type_traits>
 
 #include "common.h"
@@ -414,13 +412,13 @@ void kv_cache_write(torch::Tensor k, torch::Tensor v, torch::Tensor kc,
 // One kernel replaces: q/k/v slice copies (the qkv GEMM output is sliced
 // non-contiguously), RoPE on q and k, and the paged-cache K/V scatter —
 // rocprof showed those as ~5 launches + 3 copies per layer of pure launch
-// floor in the decode step (profiles/decode_kernel_stats_r01.csv).
+// floor in the decode step.
 // qkv: [T, (Hq+2*Hkv)*D] -> writes q_out [T, Hq, D] (roped), kc/vc slots.
-// PARTS: qkv is a product in `parts` fp32 terms `step` apart, see rmsnorm_kernel: 96
-// rows of 6144 in 2 parts 3.3 us and whole 3.0, 23 of 3072 in 5 parts 2.8 and 2.4. Slot and
-// position are asked for before anything else, so that few rows make two trips to memory and
-// not three: 23 of 3072 in 5 parts 3.82 and 3.66, 96 of 6144 in 2 parts 4.46 and 4.18 (of
-// cold cache pages).
+// PARTS: qkv is a product in `parts` fp32 terms `step` apart, see rmsnorm_kernel. Beside a
+// whole product that costs 0.3 us for 96 rows of 6144 in 2 parts and 0.4 for 23 of 3072 in 5
+// (warm cache pages). Slot and position are asked for before anything else, so that few
+// rows make two trips to memory and not three: of cold cache pages 23 of 3072 in 5 parts 3.82 us
+// and 3.66, 96 of 6144 in 2 parts 4.46 and 4.18.
 // bias: one term more per column or null, added to the rounded product.
 // A thread per VEC columns of a head and their partners half a head on (16-byte accesses
 // at 8): bound by memory. 6172 rows of 48 heads of 128 took 58 us in 2-byte accesses,
