@@ -173,7 +173,7 @@ constexpr int row_threads(int hv) { return hv > 1 ? 512 : 256; }
 // loads are then waited for with W's) 93.7, 38.5 and 21.3. The two products alone with their
 // norms, before and in them: 60.8 and 57.8, 27.2 and 24.4, 15.7 and 12.4; 8192 wide, 16384 and
 // 10240 outputs, 106.0 and 102.2 (squares in the order of this kernel's threads: 57.9, 24.5, 12.2
-// and 101.6, but a row in ten thousand with an element off by its last bit).
+// and 101.6, but a row in some hundred with an element off by its last bit).
 template <int HV, bool SILU>
 __global__ __launch_bounds__(256 + row_threads(HV)) void one_row_kernel(
     const float* __restrict__ x, int S, const unsigned short* __restrict__ res,
