@@ -1,11 +1,11 @@
 // Products of few rows for gfx950: out[M <= 128, N] = x[M, K] @ W[N, K]^T, what a decoding
 // step does with every dense weight, and silu(gate) * up of such products.
 //
-// Bound by reading W once. A workgroup takes 64 rows of W (128 for the wide form) and all
-// rows of x, in steps of 64 of K through a ring of LDS stages that direct-to-LDS loads fill
+// Bound by reading W once. A workgroup takes 64 rows of W (96 to 128 for the wide forms) and
+// all rows of x, in steps of 64 of K through a ring of LDS stages that direct-to-LDS loads fill
 // several steps ahead: two workgroups of 72 to 80 KB fit a CU and have 48 to 80 KB of W
-// under way. A wave multiplies 16 rows of W with all of x: a lane ends with four outputs
-// that lie side by side. Reading W straight into fragments instead, with K split over the
+// under way. A wave multiplies 16 rows of W with all of x, or from 33 rows of x on 32 with
+// half of it, which takes less from LDS: a lane ends with four outputs that lie side by side. Reading W straight into fragments instead, with K split over the
 // waves of a workgroup and no LDS, came to the same at one row and lost at 16 and more
 // (x is then read as often as W's tiles of 16 rows: 28672 x 4096, 32 rows, 86 us).
 //
@@ -24,7 +24,10 @@
 //   28672 x 4096, with silu (two kernels before)
 //                  66.3 -> 48.5   58.2 -> 48.0  56.8 -> 53.3  60.1 -> 56.1  62.8 -> 59.3
 // (4096 x 14336 is 21 us at the 5.6 TB/s of a large read, 28672 x 4096 42 us). What is left
-// at 64 rows and more is x on its way to every CU.
+// at 64 rows and more is x on its way to every CU. Asking for W ahead of the product, from
+// workgroups beside those of the norm before it, brings nothing (4096 x 14336, norm, 28672 x
+// 4096, 23 rows: 73.5 us, and with 4 to 29 MB asked for 73.2 to 77): what comes from
+// memory and what lies in the cache before it take the same way.
 #include "flash_tiles.h"
 #include <torch/extension.h>
 #include <c10/core/DeviceGuard.h>
@@ -45,17 +48,22 @@ DEVINL void await_stage() {
 // rows are 8 of each. Outputs are bf16, or with ``part`` sums over ``span`` of K; with both they
 // go to ``part``, rounded to bf16 first. ROUTER: a workgroup y of Y takes every Y-th step and keeps
 // the sums of its steps' two halves apart, parts 2 y and 2 y + 1; z are blocks of 16 MT rows of x.
+// A wave's tiles of 16 are RT of W by MW of x. (2 by half of x instead of 1 by all: 64 wide 0.4%
+// faster at 33 to 64 rows, 2.2% at 128, means of 18 weights of 16 MB and more.)
+// (Tiles of one part of K side by side on an XCD, so that its L2 reads that part of x alone: products
+// by themselves 1% faster, steps of 1 to 96 rows of whole models up to 1.5% slower.)
 template <int WN, int MT, int NS, bool SILU, bool ROUTER = false>
 __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
     const unsigned short* x, const unsigned short* w, unsigned short* out, float* part, int M,
     int N, int K, int span, long ldx) {
   constexpr int NT = WN * 4;
+  constexpr int RT = MT >= 4 && WN % 32 == 0 ? 2 : 1, MW = MT / RT, ACROSS = WN / 16 / RT;
   constexpr int L = (WN * 8 + MT * 128 + NT - 1) / NT;  // loads of a thread per stage
   constexpr int STAGE = L * NT * 16;
   __shared__ __attribute__((aligned(16))) char lds[NS * STAGE];
   const int tid = threadIdx.x, lane = tid % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  const int at = lane & 15, g = lane >> 4;
+  const int at = lane & 15, g = lane >> 4, r0 = wave % ACROSS * RT * 16, x0 = wave / ACROSS * MW * 16;
   const int n0 = blockIdx.x * (SILU ? WN / 2 : WN);
   const int k0 = blockIdx.y * (ROUTER ? FEW_K : span), m0 = ROUTER ? blockIdx.z * 16 * MT : 0;
   const int stride = ROUTER ? gridDim.y * FEW_K : FEW_K;
@@ -79,27 +87,34 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
                                        (lptr_t)(stage + (l * NT + wave * WAVE) * 16), 16, 0, 0);
   };
   constexpr int SUMS = ROUTER ? 2 : 1;
-  floatx4 acc[SUMS][MT];
+  floatx4 acc[SUMS][RT][MW];
 #pragma unroll
-  for (int m = 0; m < SUMS * MT; ++m) acc[m / MT][m % MT] = floatx4{0.f, 0.f, 0.f, 0.f};
+  for (int u = 0; u < SUMS * RT * MW; ++u)
+    acc[u / (RT * MW)][u / MW % RT][u % MW] = floatx4{0.f, 0.f, 0.f, 0.f};
   auto compute = [&](int s) {
     const char* stage = lds + s % NS * STAGE;
-    frag_u wf[2], xf[2][MT];  // all read before the first product: one latency a step
+    frag_u wf[2][RT], xf[2][MW];  // all read before the first product: one latency a step
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int unit = ((h * 4 + g) ^ (at & 7)) * 16;
-      wf[h].s = *reinterpret_cast<const shortx8*>(stage + (wave * 16 + at) * 128 + unit);
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-        xf[h][m].s = *reinterpret_cast<const shortx8*>(stage + (WN + m * 16 + at) * 128 + unit);
+      for (int r = 0; r < RT; ++r)
+        wf[h][r].s =
+            *reinterpret_cast<const shortx8*>(stage + (r0 + r * 16 + at) * 128 + unit);
+#pragma unroll
+      for (int m = 0; m < MW; ++m)
+        xf[h][m].s =
+            *reinterpret_cast<const shortx8*>(stage + (WN + x0 + m * 16 + at) * 128 + unit);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-      for (int m = 0; m < MT; ++m)
-        acc[h % SUMS][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[h].v, xf[h][m].v,
-                                                                   acc[h % SUMS][m], 0, 0, 0);
+      for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int m = 0; m < MW; ++m)
+          acc[h % SUMS][r][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              wf[h][r].v, xf[h][m].v, acc[h % SUMS][r][m], 0, 0, 0);
   };
   for (int s = 0; s < min(steps, NS - 1); ++s) issue(s);
   int s = 0;
@@ -111,11 +126,11 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
   await_stage<0>();
   for (; s < steps; ++s) compute(s);
 
-  const int n = n0 + (SILU ? wave * 8 + (g & 1) * 4 : wave * 16 + g * 4);
 #pragma unroll
-  for (int u = 0; u < SUMS * MT; ++u) {
-    const int m = u % MT;
-    floatx4 y = acc[u / MT][m];
+  for (int u = 0; u < SUMS * RT * MW; ++u) {
+    const int m = u % MW, r = u / MW % RT, sum = u / (RT * MW);
+    const int n = n0 + (SILU ? r0 / 2 + r * 8 + (g & 1) * 4 : r0 + r * 16 + g * 4);
+    floatx4 y = acc[sum][r][m];
     if constexpr (SILU) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -124,7 +139,7 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
       }
       if (g >= 2) continue;
     }
-    const int row = m0 + m * 16 + at;
+    const int row = m0 + x0 + m * 16 + at;
     if (row >= M) continue;
     const bool whole = n + 4 <= N && N % 4 == 0;
     if (!SILU && part) {
@@ -133,7 +148,7 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
         y = floatx4{__uint_as_float(a << 16), __uint_as_float(a & 0xffff0000u),
                     __uint_as_float(b << 16), __uint_as_float(b & 0xffff0000u)};
       }
-      float* dst = part + ((long)(blockIdx.y * SUMS + u / MT) * M + row) * N + n;
+      float* dst = part + ((long)(blockIdx.y * SUMS + sum) * M + row) * N + n;
       if (whole) *reinterpret_cast<floatx4*>(dst) = y;
       else
 #pragma unroll
@@ -157,7 +172,7 @@ DEVINL void meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memor
 
 #define ROW_MOST 8192  // elements of the row below
 
-// threads that norm the row, besides the 256 of the product: wider rows want eight waves (4096
+// threads that norm the row, besides those of the product: wider rows want eight waves (4096
 // wide, a layer 92.0 and 91.8 us, 2048 38.8 and 38.1, 1024 20.6 and 21.7)
 constexpr int row_threads(int hv) { return hv > 1 ? 512 : 256; }
 
@@ -174,21 +189,21 @@ constexpr int row_threads(int hv) { return hv > 1 ? 512 : 256; }
 // norms, before and in them: 60.8 and 57.8, 27.2 and 24.4, 15.7 and 12.4; 8192 wide, 16384 and
 // 10240 outputs, 106.0 and 102.2 (squares in the order of this kernel's threads: 57.9, 24.5, 12.2
 // and 101.6, but a row in some hundred with an element off by its last bit).
-template <int HV, bool SILU>
-__global__ __launch_bounds__(256 + row_threads(HV)) void one_row_kernel(
+template <int HV, bool SILU, int WN = 64>
+__global__ __launch_bounds__(WN * 4 + row_threads(HV)) void one_row_kernel(
     const float* __restrict__ x, int S, const unsigned short* __restrict__ res,
     const unsigned short* __restrict__ weight, unsigned short* __restrict__ res_out, float eps,
     const unsigned short* __restrict__ w, unsigned short* __restrict__ out,
     float* __restrict__ part, int N, int K, int span) {
-  constexpr int NS = 7, L = 2, STAGE = 64 * 128, RT = row_threads(HV);
+  constexpr int NT = WN * 4, NS = 7, L = 2, STAGE = WN * 128, RT = row_threads(HV);
   constexpr int PARTS = 16 / HV, V = HV * 256 / RT > 0 ? HV * 256 / RT : 1;
   // one array: of several the compiler waits for all loads under way before it reads one
   __shared__ __attribute__((aligned(16))) char lds[NS * STAGE + (V * RT * 8) + 64];
   auto* row = reinterpret_cast<unsigned short*>(lds + NS * STAGE);
   auto* red = reinterpret_cast<float*>(lds + NS * STAGE + V * RT * 8);
   const int lane = threadIdx.x % WAVE;
-  if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= 256) {
-    const int tid = threadIdx.x - 256, wave = tid / WAVE;
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x) >= NT) {
+    const int tid = threadIdx.x - NT, wave = tid / WAVE;
     // Squares are added as rmsnorm_residual adds them, whose threads hold eight values side by
     // side: here two vectors of one thread, or those of two lanes, whose pairs are then of every
     // other thread there, so that two waves end where one wave's last step adds its halves.
@@ -272,12 +287,12 @@ __global__ __launch_bounds__(256 + row_threads(HV)) void one_row_kernel(
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
   const int at = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (SILU ? 32 : 64);
+  const int n0 = blockIdx.x * (SILU ? WN / 2 : WN);
   const int k0 = blockIdx.y * span, steps = (min(K, k0 + span) - k0) / FEW_K;
   const unsigned short* src[L];
 #pragma unroll
   for (int l = 0; l < L; ++l) {
-    const int r = (tid + l * 256) >> 3, unit = (tid & 7) ^ (r & 7);
+    const int r = (tid + l * NT) >> 3, unit = (tid & 7) ^ (r & 7);
     const long n = SILU ? min(n0 + r / 16 * 8 + r % 8, N - 1) + (long)(r % 16 / 8) * N
                         : min(n0 + r, N - 1);
     src[l] = w + n * K + k0 + unit * 8;
@@ -287,7 +302,7 @@ __global__ __launch_bounds__(256 + row_threads(HV)) void one_row_kernel(
 #pragma unroll
     for (int l = 0; l < L; ++l)
       __builtin_amdgcn_global_load_lds((gptr_t)(src[l] + (long)s * FEW_K),
-                                       (lptr_t)(stage + (l * 256 + wave * WAVE) * 16), 16, 0, 0);
+                                       (lptr_t)(stage + (l * NT + wave * WAVE) * 16), 16, 0, 0);
   };
   for (int s = 0; s < min(steps, NS - 1); ++s) issue(s);
   meet();
@@ -364,6 +379,40 @@ static long parts_of(long N, long K) {
   return std::max(1L, std::min({256 / tiles, K / FEW_K / 2, 16L}));
 }
 
+// Rows of W a workgroup takes and K's parts: what leaves a CU the least to read, of W at 21 GB/s
+// when all read at once and of x at some 125, where the whole W does not take longer anyway
+// (5.3 TB/s), and the reader the fewest parts; 64 rows unless 1.5 us are gained. Of 46 weights, 1
+// to 128 rows each, the norm that reads the parts included, the cut so chosen takes 1.2% longer
+// than the best, 64 rows with the parts above 3.3%. us: 6144 x 4096, 1, 32, 64 and 96 rows, 64
+// wide 16.8 17.3 19.3 21.3, 96 wide in 4 parts 15.0 16.1 17.4 19.1; 8576 x 16064, 32 and 96 rows,
+// 64 wide 76.9 104.3, 128 in 3 parts 56.9 71.4; 4096 x 14336, 96 rows, 64 wide in 4 parts 32.8,
+// 128 in 8 32.2; 5120 x 5120, 64 rows, 19.4 and 19.3.
+struct Cut {
+  int width;
+  long parts;
+};
+static Cut cut_of(long M, long N, long K) {
+  const long steps = K / FEW_K, rows = M <= 32 ? 32 : (M + 31) / 32 * 32;
+  Cut best = {64, 1};
+  // a single row's parts are read by a norm in the next product, which takes few (one_row_fits)
+  if (M == 1 && N <= 4096) return {64, parts_of(N, K)};
+  double low = 0;
+  for (int width : {64, 96, 128}) {
+    if (M == 1 && width > 96) break;  // (one_row_kernel has no wider form)
+    const long tiles = (N + width - 1) / width;
+    const long most = std::max(1L, std::min({256 / tiles, steps / 2, 16L}));
+    for (long parts = most; parts >= std::max(1L, most - 1); --parts) {
+      const long per = (steps + parts - 1) / parts;
+      if ((steps + per - 1) / per != parts) continue;  // the same with fewer
+      const double cu = per * FEW_K * (width * 2 / 21. + rows * 2 * 0.4 / 50);
+      const double time = std::max(cu, N * K * 2 / 5300.) + parts * M * N * 4 / 5000. +
+                          (width > 64 ? 1500 : 0);
+      if (low == 0 || time < low) low = time, best = {width, parts};
+    }
+  }
+  return best;
+}
+
 static void check(const torch::Tensor& x, const torch::Tensor& w) {
   TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dtype() == torch::kBFloat16 &&
                   w.dtype() == torch::kBFloat16 && w.is_contiguous(),
@@ -383,10 +432,12 @@ static torch::Tensor readable(const torch::Tensor& x) {
   return ok ? x : x.clone(at::MemoryFormat::Contiguous);
 }
 
-template <int WN, int MT, int NS, bool SILU>
+template <int WN, int MT, bool SILU>
 static void launch(const torch::Tensor& x, const torch::Tensor& w, unsigned short* out,
                    float* part, long N, long S, long span) {
-  constexpr int tile = SILU ? WN / 2 : WN;
+  // stages: two workgroups of 64 rows on a CU, one of the wide forms
+  constexpr int tile = SILU ? WN / 2 : WN, loads = (WN * 8 + MT * 128 + WN * 4 - 1) / (WN * 4);
+  constexpr int NS = (WN == 64 ? 80 : 160) * 1024 / (loads * WN * 64);
   hipLaunchKernelGGL((few_rows_kernel<WN, MT, NS, SILU>), dim3((N + tile - 1) / tile, S),
                      dim3(WN * 4), 0, CUR_STREAM, (const unsigned short*)x.data_ptr(),
                      (const unsigned short*)w.data_ptr(), out, part, (int)x.size(0), (int)N,
@@ -395,25 +446,37 @@ static void launch(const torch::Tensor& x, const torch::Tensor& w, unsigned shor
 }
 
 // [M, N] in bf16, or with ``raw`` where K is cut [S, M, N] in fp32, S terms to be added.
-torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts) {
+static torch::Tensor cut_rows(torch::Tensor x, torch::Tensor w, bool raw, Cut cut) {
   check(x, w);
   x = readable(x);
   const long M = x.size(0), K = x.size(1), N = w.size(0);
   torch::Tensor out, part;
   if (M == 0 || N == 0 || K == 0) return torch::zeros({M, N}, x.options());
   const long steps = K / FEW_K;
-  const long per = (steps + std::max(parts, 1L) - 1) / std::max(parts, 1L);
+  const long per = (steps + std::max(cut.parts, 1L) - 1) / std::max(cut.parts, 1L);
   const long S = (steps + per - 1) / per, span = per * FEW_K;
   if (S > 1) part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
   if (S == 1) out = torch::empty({M, N}, x.options());
   auto* op = S > 1 ? nullptr : (unsigned short*)out.data_ptr();
   float* pp = S > 1 ? part.data_ptr<float>() : nullptr;
-  if (M <= 32) launch<64, 2, 6, false>(x, w, op, pp, N, S, span);
-  else if (M <= 64) launch<64, 4, 5, false>(x, w, op, pp, N, S, span);
-  else if (M <= 96) launch<64, 6, 4, false>(x, w, op, pp, N, S, span);
-  else launch<64, 8, 3, false>(x, w, op, pp, N, S, span);
+  auto rows = [&](auto MT) {
+    constexpr int mt = decltype(MT)::value;
+    if (cut.width == 64) launch<64, mt, false>(x, w, op, pp, N, S, span);
+    else if (cut.width == 96) launch<96, mt, false>(x, w, op, pp, N, S, span);
+    else launch<128, mt, false>(x, w, op, pp, N, S, span);
+  };
+  if (M <= 32) rows(std::integral_constant<int, 2>{});
+  else if (M <= 64) rows(std::integral_constant<int, 4>{});
+  else if (M <= 96) rows(std::integral_constant<int, 6>{});
+  else rows(std::integral_constant<int, 8>{});
   if (S == 1) return out;
   return raw ? part : add_parts(part);
+}
+
+// The same in a given number of parts and rows of W a workgroup.
+torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width) {
+  TORCH_CHECK(width == 64 || width == 96 || width == 128, "64, 96 or 128 rows of w a workgroup");
+  return cut_rows(x, w, raw, Cut{(int)width, parts});
 }
 
 // A router's logits in 16 parts [16, M, N] in fp32 that hold what the 16 waves of
@@ -438,8 +501,9 @@ torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw) {
   // A kernel to add the parts pays off where a tile's steps take much longer than it: 2048
   // x 2048, 23 rows, 8.2 us whole, 4.0 and 4.7 in parts; 4096 x 4096 16.7, 8.9 and 2.4; 2048
   // x 2048, 64 rows, 11.7, 5.5 and 4.2.
-  const bool cut = raw || x.size(1) * (x.size(0) > 32 ? 2 : 1) >= 4096;
-  return few_rows(x, w, raw, cut ? parts_of(w.size(0), x.size(1)) : 1);
+  // More than 8192 outputs are cut for their reader alone: float_few_rows has their bits.
+  const bool cut = raw || (x.size(1) * (x.size(0) > 32 ? 2 : 1) >= 4096 && parts_of(w.size(0), x.size(1)) > 1);
+  return cut_rows(x, w, raw, cut ? cut_of(x.size(0), w.size(0), x.size(1)) : Cut{64, 1});
 }
 
 // linear_few_rows's result in float32, where K is not cut, without a kernel to convert it: 1 row
@@ -455,8 +519,8 @@ torch::Tensor float_few_rows(torch::Tensor x, torch::Tensor w) {
   if (M == 0 || N == 0) return out;
   float* pp = out.data_ptr<float>();
   auto* round = (unsigned short*)pp;
-  if (M <= 32) launch<64, 2, 6, false>(x, w, round, pp, N, 1, K);
-  else launch<64, 4, 5, false>(x, w, round, pp, N, 1, K);
+  if (M <= 32) launch<64, 2, false>(x, w, round, pp, N, 1, K);
+  else launch<64, 4, false>(x, w, round, pp, N, 1, K);
   return out;
 }
 
@@ -471,19 +535,26 @@ torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w) {
   auto* op = (unsigned short*)out.data_ptr();
   // From 65 rows on x is as much to move as W: tiles of 128 halve it where there are enough
   // for the chip. 28672 x 4096, 96 rows, 59.9 and 56.1 us; 16384 x 2048 21.8 and 27.6; 28672
-  // x 4096, 64 rows, 53.3 and 53.6.
-  const bool wide = N / 64 >= 192;
-  if (M <= 32) launch<64, 2, 6, true>(x, w, op, nullptr, N, 1, K);
-  else if (M <= 64) launch<64, 4, 5, true>(x, w, op, nullptr, N, 1, K);
-  else if (M <= 96 && wide) launch<128, 6, 5, true>(x, w, op, nullptr, N, 1, K);
-  else if (M <= 96) launch<64, 6, 4, true>(x, w, op, nullptr, N, 1, K);
-  else if (wide) launch<128, 8, 5, true>(x, w, op, nullptr, N, 1, K);
-  else launch<64, 8, 3, true>(x, w, op, nullptr, N, 1, K);
+  // x 4096, 64 rows, 53.3 and 53.6. Tiles of 112 where one for every CU is enough (33, 64, 96 and
+  // 128 rows 49.5 51.9 55.3 56.5, and 48.9 49.7 52.5 55.2).
+  const bool wide = N / 64 >= 192, one = wide && (N + 55) / 56 <= 256;
+  auto rows = [&](auto MT) {
+    constexpr int mt = decltype(MT)::value;
+    if constexpr (mt > 2)
+      if (one) return launch<112, mt, true>(x, w, op, nullptr, N, 1, K);
+    if constexpr (mt > 4)
+      if (wide) return launch<128, mt, true>(x, w, op, nullptr, N, 1, K);
+    launch<64, mt, true>(x, w, op, nullptr, N, 1, K);
+  };
+  if (M <= 32) rows(std::integral_constant<int, 2>{});
+  else if (M <= 64) rows(std::integral_constant<int, 4>{});
+  else if (M <= 96) rows(std::integral_constant<int, 6>{});
+  else rows(std::integral_constant<int, 8>{});
   return out;
 }
 
 // The kernel above where it has a form: x [S, 1, K] in fp32, S parts, of which a thread holds 64
-// values at most. ``parts_of`` makes more for rows 1088 to 1792, 2112 to 3264 and 4160 to 5440
+// values at most. ``cut_of`` makes more for rows 1088 to 1792, 2112 to 3264 and 4160 to 6144
 // wide, whose norms stay kernels of their own.
 bool one_row_fits(long S, long K) {
   return S > 1 && K % FEW_K == 0 && K <= ROW_MOST &&
@@ -506,12 +577,13 @@ torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor 
                   (uintptr_t)x.data_ptr() % 16 == 0 && res.data_ptr() != res_out.data_ptr(),
               "rows of K");
   const c10::DeviceGuard on(x.device());
-  const long steps = K / FEW_K, parts = silu ? 1 : parts_of(N, K);
+  const Cut cut = silu ? Cut{64, 1} : cut_of(1, N, K);
+  const long steps = K / FEW_K, parts = cut.parts;
   const long per = (steps + parts - 1) / parts, S2 = (steps + per - 1) / per;
   torch::Tensor out, part;
   if (S2 > 1) part = torch::empty({S2, 1, N}, x.options());
   else out = torch::empty({1, N}, w.options());
-  const int tile = silu ? 32 : 64;
+  const int tile = silu ? 32 : cut.width;
   auto launch = [&](auto kern, int threads) {
     hipLaunchKernelGGL(kern, dim3((N + tile - 1) / tile, S2), dim3(threads), 0, CUR_STREAM,
                        x.data_ptr<float>(), (int)S, (const unsigned short*)res.data_ptr(),
@@ -526,7 +598,8 @@ torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor 
   auto form = [&](auto hv) {
     constexpr int HV = decltype(hv)::value;
     if (silu) launch(one_row_kernel<HV, true>, 256 + row_threads(HV));
-    else launch(one_row_kernel<HV, false>, 256 + row_threads(HV));
+    else if (cut.width == 64) launch(one_row_kernel<HV, false>, 256 + row_threads(HV));
+    else launch(one_row_kernel<HV, false, 96>, 384 + row_threads(HV));
   };
   if (K <= 1024) form(std::integral_constant<int, 1>{});
   else if (K <= 2048) form(std::integral_constant<int, 2>{});

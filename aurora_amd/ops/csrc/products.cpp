@@ -31,17 +31,23 @@ static long small_megabytes() {
 // 32 rows while K is short, up to 512 MB of them to 4096 (1 and 32 rows: 152064 x 3584 195
 // and 233, 208 and 264; 32000 x 4096 54 and 60, 56 and 66; but 128256 x 4096 204 and 187, 207
 // and 201; 57344 x 8192 213 and 181; 16384 x 8192 66 and 62, 65 and 54; the other way, given
-// up, 28672 x 8192 105 and 131). Above 64 rows up to 8192 outputs with parts that their
-// reader adds up (3072 x 2048, 96 rows, 8 and 13), or with K long enough to pay for adding
-// them, few outputs with longer ones (96 rows: 4608 x 4096 16 and 22, 2048 x 4096 13.3 and
-// 12.8, 2048 x 8192 15 and 21, 1024 x 8192 15.2 and 15.0, 1024 x 14336 17 and 25, 8192 x 28672
+// up, 28672 x 8192 105 and 131). Few outputs of long K, which is cut, whatever their size (1, 32
+// and 64 rows with the norm that reads them: 3584 x 18944 30 and 52, 32 and 113, 33 and 94; 5120 x
+// 27648 56 and 141, 56 and 153, 60 and 163; 7168 x 18432 59 and 57, 54 and 61, 58 and 130; 8192 x
+// 28672 96 and 94, 87 and 100, 93 and 142; 10240 x 8192 44 and 42, 41 and 45, 42 and 49; without
+// it 7168 x 18432, 16 and 64 rows, 53 and 110, 56 and 124). Above 64 rows up to 12288 outputs with
+// parts that their reader adds up (3072 x 2048, 96 rows, 8 and 13; with a norm 9216 x 4096 27 and
+// 35, 10240 x 8192 44 and 58, 12288 x 4096 32 and 38; but 16384 x 4096 44 and 44), or up to 8192
+// with K long enough to pay for adding them, few outputs with longer ones (96 rows: 4608 x 4096 16
+// and 22, 2048 x 4096 13.3 and 12.8, 2048 x 8192 15 and 21, 1024 x 8192 15.2 and 15.0, 1024 x 14336 17 and 25, 8192 x 28672
 // 123 and 124; but 4608 x 2048 13.1 and 13.5, 128 rows 15.9 and 15.0; 10240 x 8192 57 and 55).
 static bool few_rows_win(long M, long N, long K, bool parts) {
   if (M > 64)
-    return N <= 8192 &&
+    return N <= (parts ? 12288 : 8192) &&
            (parts || K >= 14336 || (K >= 3072 && N >= (K < 8192 ? 3072 : 2048)));
   const long size = megabytes(N, K);
-  return size <= small_megabytes() ||
+  const long most = M == 1 ? 6144 : !parts ? 7168 : M <= 32 ? 8192 : 10240;
+  return size <= small_megabytes() || (K > 4096 && N <= most) ||
          (M <= 32 && (K < 4096 || (K == 4096 && size <= 512)));
 }
 

@@ -1,0 +1,52 @@
+"""Products of few rows by workgroups of more than 64 rows of weights."""
+import pytest
+import torch
+
+from aurora_amd import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(got, want):
+    """64 bits rounded to bf16, but for fp32 sums whose error is far below 2^-16 of the largest."""
+    slack = 2 ** -16 * want.abs().max()
+    assert ((got.double() - want).abs() <= want.abs() * 2 ** -8 + slack).all()
+
+
+def _inputs(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m + n + k)
+    x, w = (torch.randn(r, k, generator=g, device="cuda").bfloat16() for r in (m, n))
+    return x, w * k ** -0.5
+
+
+@pytest.mark.parametrize("m", [1, 32, 33, 64, 65, 96, 97, 128])
+@pytest.mark.parametrize("n,k", [(8, 64), (95, 128), (97, 192), (129, 448), (1000, 576)])
+@pytest.mark.parametrize("width", [96, 128])
+def test_wide_tiles(m, n, k, width):
+    x, w = _inputs(m, n, k)
+    want = x.double() @ w.double().t()
+    for parts in (1, 3, 16):
+        _check(ops._hip.few_rows(x, w, False, parts, width), want)
+        raw = ops._hip.few_rows(x, w, True, parts, width)
+        _check((raw.sum(0) if raw.dim() == 3 else raw).bfloat16(), want)
+
+
+@pytest.mark.parametrize("m", [33, 65, 97, 128])
+@pytest.mark.parametrize("n", [14336, 14344])  # a tile of 112 for every CU, and one too many
+def test_silu_tiles(m, n):
+    x, w = _inputs(m, 2 * n, 192)
+    y = x.double() @ w.double().t()
+    _check(ops._hip.silu_few_rows(x, w), torch.nn.functional.silu(y[:, :n]) * y[:, n:])
+
+
+@pytest.mark.parametrize("m", [1, 2, 40, 70, 128])
+@pytest.mark.parametrize("n,k", [(6144, 4096), (8576, 4160), (3584, 18944)])
+def test_chosen_cuts(m, n, k):
+    """Sizes whose cuts are wide, and weights beyond 128 MB in parts."""
+    x, w = _inputs(m, n, k)
+    want = x.double() @ w.double().t()
+    y = ops.linear_parts(x, w)
+    _check((y.sum(0) if y.dim() == 3 else y).bfloat16(), want)
+    _check(ops.linear(x, w), want)
+    if n <= 8192 and k > 4096:
+        assert y.dim() == 3
