@@ -663,7 +663,7 @@ class LLMEngine:
             fields.update(seq_fields(decode, dec_ctx))
         mode = "decode" if not prefill else "mixed" if decode else "prefill"
         input_ids = torch.tensor(ids, dtype=torch.long, device=self.device)
-        return input_ids, AttnMetadata(mode=mode, **fields)
+        return input_ids, AttnMetadata(mode=mode, last_tokens=mode == "decode", **fields)
 
     def _pack_batch(self, prefill: List[Sequence], chunks: List[int], decode: List[Sequence]):
         """``_build_batch`` in native code, one copy to the device; None where it has to be
@@ -696,7 +696,7 @@ class LLMEngine:
         else:
             fields.update(seq_fields())
         mode = "decode" if not prefill else "mixed" if decode else "prefill"
-        return made[0], AttnMetadata(mode=mode, **fields)
+        return made[0], AttnMetadata(mode=mode, last_tokens=mode == "decode", **fields)
 
     # ----------------------------------------------------- hipGraph decode
 
@@ -791,7 +791,8 @@ class LLMEngine:
         in_ids, (in_pos, in_slot, in_ctx, in_state), in_bt = parts(inputs)
         meta = AttnMetadata(mode="decode", positions=in_pos, slot_mapping=in_slot,
                             block_tables=in_bt, context_lens=in_ctx,
-                            states=self.states.states, state_slots=in_state)
+                            states=self.states.states, state_slots=in_state,
+                            last_tokens=True)
 
         def fwd():
             hidden = self.model(in_ids, self.kv.caches, meta)

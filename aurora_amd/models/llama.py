@@ -66,6 +66,9 @@ class AttnMetadata:
     cu_host: Optional[List[int]] = None  # cu_seqlens_q without a device read
     ctx_host: Optional[List[int]] = None  # context_lens of the prompt portions
     marks: Optional[torch.Tensor] = None  # ``ops.decode_marks`` of the single tokens
+    # decode: every row is the last token of a sequence that no other row belongs to, at the
+    # position before its context's end and in the slot that its table names for it
+    last_tokens: bool = False
 
     def segments(self, T: int) -> List[ops.Segment]:
         """The step's prompt portions and its single-token rows, each with its
@@ -125,6 +128,12 @@ class LlamaAttention(nn.Module):
         T = x.shape[0]
         qkv, bias = column_parts(self.qkv_proj, x)
         k_cache, v_cache = kv_cache
+        if meta.mode == "decode" and getattr(meta, "last_tokens", False):
+            o = ops.fresh_attention_decode(
+                qkv, bias, meta.positions, meta.slot_mapping, cos_sin, k_cache, v_cache,
+                meta.block_tables, meta.context_lens, self.n_heads, self.scale,
+                getattr(meta, "marks", None))
+            return o.reshape(T, self.n_heads * self.head_dim)
         # fused split + bias + RoPE + paged K/V scatter (one kernel on GPU)
         q = ops.fused_rope_kv_write(qkv, meta.positions, meta.slot_mapping,
                                     cos_sin, k_cache, v_cache,

@@ -225,6 +225,24 @@ def fused_rope_kv_write(qkv, positions, slots, cos_sin, k_cache, v_cache,
     return q
 
 
+def fresh_attention_decode(qkv, bias, positions, slots, cos_sin, k_cache, v_cache, block_tables,
+                           context_lens, n_heads: int, scale: float, marks=None) -> torch.Tensor:
+    """``fused_rope_kv_write`` and ``paged_attention_decode`` of rows that are the last tokens of
+    different sequences, each at the place and position that its table and context say; in one
+    kernel where it has a form."""
+    n_kv_heads = k_cache.shape[1]
+    if qkv.is_cuda:
+        m = _require_hip("fresh_attention_decode")
+        out = m.fresh_attention_decode(qkv, bias, cos_sin, k_cache, v_cache, block_tables,
+                                       context_lens, n_heads, float(scale), marks)
+        if out is not None:
+            return out
+    q = fused_rope_kv_write(qkv, positions, slots, cos_sin, k_cache, v_cache, n_heads,
+                            n_kv_heads, bias)
+    return paged_attention_decode(q, k_cache, v_cache, block_tables, context_lens, scale,
+                                  marks=marks)
+
+
 def embed_pool(hidden: torch.Tensor, cu_seqlens: torch.Tensor) -> torch.Tensor:
     if hidden.is_cuda:
         return _require_hip("embed_pool", aux=True).embed_pool(hidden.contiguous(), cu_seqlens.to(torch.int32))

@@ -40,6 +40,7 @@
 #define DEC_TARGET 1024   // stretches that the contexts are cut into
 #define DEC_LEAST 160     // of few keys each
 
+enum { WHOLE = 1, IN_PARTS = 2 };  // what a kernel that rotates finds
 enum { NO_BIAS = 0, LINEAR_BIAS = 1, LOG_BIAS = 2, FLAT_BIAS = 3 };
 
 // keys of a sequence that its query sees: [first, L)
@@ -245,12 +246,32 @@ DEVINL void merge_stretches(const float* src, long step, int n, int lane, __hip_
   }
 }
 
+// What a step's projection left of its queries and of the new keys and values: rows [B, width] of
+// queries, keys and values side by side, in bf16 or in ``parts`` fp32 terms ``step`` apart, to
+// which a bias is added, and the rotations [positions, D]. A row is the last of its sequence.
+struct Fresh {
+  const void* qkv;
+  const unsigned short* bias;
+  const float* cos_sin;
+  void *kc, *vc;
+  int parts;
+  long step;
+};
+
 // BIAS: a distance penalty per head or none (see attention_prefill.hip), a window or
 // chunks of positions; sink: one more term of the denominator per head, or null;
 // FLAT_BIAS results may be turned back and gated. PAGED: pages are whole tiles.
 // Without CUT a workgroup takes a whole context.
-template <int D, int DV, bool FP8, int BIAS, bool PAGED, bool CUT>
-__global__ __launch_bounds__(256, 2) void paged_decode_kernel(
+// FRESH: the workgroup adds up and rotates its queries itself, and that of the last stretch the
+// new key and value, which it writes to the cache and takes from LDS where the cache would still
+// have what was there before. While parts and rotations are on their way so are its first keys.
+// After a kernel of its own for that and with it in here, 32 heads over 8, us: one sequence of
+// 777, 128 wide, 12.0 and 10.1; 8 of 300 to 1500 17.2 and 14.7; 96 of 500 to 2900 125.3 and
+// 123.2; 41 of 700 to 2600 71.0 and 68.7; 23 of 300 to 5000 in fp8 48.3 and 45.5, 64 wide 27.1
+// and 25.0.
+// (Four columns and partners a lane in all waves, with 64-bit addresses, gave half of that.)
+template <int D, int DV, bool FP8, int BIAS, bool PAGED, bool CUT, int FRESH = 0>
+__global__ __launch_bounds__(256, FRESH && D == 64 ? 4 : 2) void paged_decode_kernel(
     const __hip_bfloat16* __restrict__ q,   // [B, Hq, D]
     // (not __restrict__: loads of them must stay before the waits that count them)
     const void* kc,  // [NP, Hkv, P, D] bf16 | fp8 e4m3
@@ -263,7 +284,8 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
     int B, int Hq, int Hkv, int P, int MP, float scale,
     long ostride, int dv, float oscale,
     const float* __restrict__ slopes, const float* __restrict__ rates, Seen seen,
-    const float* __restrict__ sink, HeadTurn turn) {
+    const float* __restrict__ sink, HeadTurn turn, Fresh fresh) {
+  static_assert(!FRESH || (PAGED && !BIAS && D == DV));
   constexpr int NC = D / 32, NDT = DV / 16;
   constexpr int EB = FP8 ? 1 : 2;
   constexpr int VU = DV / 8, LV = DEC_KEYS * VU / WAVE;  // 16-B units of a value, a lane's
@@ -305,12 +327,14 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
       (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring;
 
   frag_u qf[NC];
+  if constexpr (!FRESH) {
 #pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    qf[c].s = shortx8{0, 0, 0, 0, 0, 0, 0, 0};
-    if (mine)
-      qf[c].s = *reinterpret_cast<const shortx8*>(q + ((long)b * Hq + h0 + head) * D + c * 32 +
-                                                  g * 8);
+    for (int c = 0; c < NC; ++c) {
+      qf[c].s = shortx8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (mine)
+        qf[c].s = *reinterpret_cast<const shortx8*>(q + ((long)b * Hq + h0 + head) * D + c * 32 +
+                                                    g * 8);
+    }
   }
   const float c2 = scale * LOG2E;  // scores in units of log 2
   const float slope = BIAS == LINEAR_BIAS && mine ? slopes[h0 + head] * LOG2E
@@ -324,8 +348,9 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
 
   // this wave's tiles: t0 + 128 i. Row of key t in a head's cache; past the end the last
   // key again
+  const int t_end = FRESH ? max(t_hi, 1) : t_hi;
   auto row_of = [&](int t) -> long {
-    t = min(t, t_hi - 1);
+    t = min(t, t_end - 1);
     return ((long)bt[t / P] * Hkv + kvh) * P + t % P;
   };
   auto value_unit = [&](int x, int& row, int& col) {
@@ -340,7 +365,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
   // Rows of a tile: past the end the last tile again, so that every round has as many
   // loads. PAGED: its first row is looked up a tile ahead.
   long page_row = 0;
-  auto tile_at = [&](int t0) { return min(t0, (t_hi - 1) & -DEC_KEYS); };
+  auto tile_at = [&](int t0) { return min(t0, (t_end - 1) & -DEC_KEYS); };
   auto lookup = [&](int t0) {
     if constexpr (PAGED) page_row = row_of(tile_at(t0));
   };
@@ -348,7 +373,7 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
     t0 = tile_at(t0);
     // (the table need not name pages behind a window)
     if constexpr (!PAGED) return row_of(BIAS ? max(t0 + key, t_lo) : t0 + key);
-    return first_row + (t0 + DEC_KEYS <= t_hi ? key : min(key, t_hi - 1 - t0));
+    return first_row + (t0 + DEC_KEYS <= t_end ? key : min(key, t_end - 1 - t0));
   };
   auto load_keys = [&](int t0, long first_row, auto PARITY) {
     constexpr int parity = decltype(PARITY)::value;
@@ -379,6 +404,11 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
       ((((head & 3) >> 1) ^ (DV == 64 ? (vrow >> 1 & 3) << 1 : (vrow & 7) << 1)) << 4) +
       (head & 1) * 8;
 
+  // FRESH: queries as bf16, the new key and value as the cache has them
+  __shared__ __attribute__((aligned(16))) unsigned short s_q[FRESH ? DEC_HEADS * D : 8];
+  __shared__ __attribute__((aligned(16))) char s_kv[FRESH ? 2 * D * EB : 16];
+  const bool ends = FRESH && t_hi == L;  // this stretch is the last
+
   // one round: the tile at t0, whose keys are in kr[parity] and whose values in vr; the
   // wave's next tile is requested as soon as its registers are free
   constexpr int ROUND = DEC_WAVES * DEC_KEYS;
@@ -388,6 +418,18 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
     load_keys(t0 + ROUND, next_row, std::integral_constant<int, 1 - parity>{});
     lookup(t0 + 2 * ROUND);
     __builtin_amdgcn_sched_barrier(0);
+    const bool newest = ends && t0 + DEC_KEYS >= L;
+    if (FRESH && newest) {
+      int own = lane;
+      asm volatile("" : "+v"(own));  // nothing of this is kept through the rounds
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+        if (t0 + k * 16 + (own & 15) == L - 1)
+#pragma unroll
+          for (int c = 0; c < NC; ++c)
+            kr[parity][k][c] =
+                *reinterpret_cast<const raw*>(s_kv + (c * 32 + (own >> 4) * 8) * EB);
+    }
     floatx4 st[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -449,6 +491,16 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
               shortx8{0, 0, 0, 0, 0, 0, 0, 0};
       }
     }
+    if (FRESH && newest) {
+      int own = lane;
+      asm volatile("" : "+v"(own));  // the same
+      const int row = L - 1 - t0;  // its units lie side by side
+      if (own < VU) {
+        const int turn = DV == 64 ? (row >> 1 & 3) << 1 : (row & 7) << 1;
+        *reinterpret_cast<shortx8*>(ring + (row * VU + own) * 16) =
+            widen(*reinterpret_cast<const raw*>(s_kv + (D + (own ^ turn) * 8) * EB));
+      }
+    }
     load_values(t0 + ROUND, next_row);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -471,10 +523,118 @@ __global__ __launch_bounds__(256, 2) void paged_decode_kernel(
   using ODD = std::integral_constant<int, 1>;
   // tiles lie within pages, so the first may begin before the stretch
   int t0 = t_lo - (BIAS ? t_lo % DEC_KEYS : 0) + wave * DEC_KEYS;
-  if (t0 < t_hi) {
+  if constexpr (FRESH) {
+    // Two columns of a head and their partners half a head on, of all that is new, a lane; waves
+    // that find nothing left ask for their keys alone. (All of a wave's work here stands in the way
+    // of the others on its SIMD: offsets are 32 bits beside addresses that all lanes share.)
+    constexpr int UNITS = D / 4, HALF = D / 2, AHEAD = 8;
+    const int all = (GT + 2 * ends) * UNITS;
     lookup(t0);
-    load_keys(t0, page_row, EVEN{});
-    load_values(t0, page_row);
+    auto request = [&] {  // (waves without a tile ask for the last one too: a branch here
+                          // would make the others wait for all their loads)
+      load_keys(t0, page_row, EVEN{});
+      load_values(t0, page_row);
+    };
+    const long row = (long)b * (Hq + 2 * Hkv) * D;
+    const float* turns = fresh.cos_sin + (long)max(L - 1, 0) * D;
+    const bool keep = ends && L > 0 && tile % NG == 0;
+    long slot = 0;
+    if (keep) slot = (((long)bt[(L - 1) / P] * Hkv + kvh) * P + (L - 1) % P) * D;
+    auto take = [&](int x, auto meanwhile) {
+      const unsigned h = (unsigned)x / UNITS, i = (unsigned)x % UNITS * 2;
+      const bool is_q = h < (unsigned)GT, is_v = h > (unsigned)GT;  // queries, the key, the value
+      const unsigned column = (is_q ? h0 + h : is_v ? Hq + Hkv + kvh : Hq + kvh) * D + i;
+      floatx2 part[AHEAD][2], y[2];
+      unsigned whole[2], bias[2] = {0, 0};
+      if constexpr (FRESH == IN_PARTS) {
+#pragma unroll
+        for (int p = 0; p < AHEAD; ++p) {
+          const float* src = (const float*)fresh.qkv + row + min(p, fresh.parts - 1) * fresh.step;
+#pragma unroll
+          for (int z = 0; z < 2; ++z)
+            part[p][z] = *reinterpret_cast<const floatx2*>(src + (column + z * HALF));
+        }
+      } else {
+        const auto* src = (const bf16_t*)fresh.qkv + row;
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+          whole[z] = *reinterpret_cast<const unsigned*>(src + (column + z * HALF));
+      }
+      const floatx2 cs = *reinterpret_cast<const floatx2*>(turns + i),
+                    sn = *reinterpret_cast<const floatx2*>(turns + (i + HALF));
+      if (fresh.bias)
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+          bias[z] = *reinterpret_cast<const unsigned*>(fresh.bias + (column + z * HALF));
+      meanwhile();
+      __builtin_amdgcn_sched_barrier(0);
+      auto round = [](floatx2 v) {
+        const unsigned u = cvt2_bf16(v[0], v[1]);
+        return floatx2{__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
+      };
+      auto two = [](unsigned u) {
+        return floatx2{__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)};
+      };
+#pragma unroll
+      for (int z = 0; z < 2; ++z)
+        if constexpr (FRESH == IN_PARTS) {
+          y[z] = floatx2{0.f, 0.f};
+#pragma unroll
+          for (int p = 0; p < AHEAD; ++p)
+            if (p < fresh.parts) y[z] += part[p][z];
+        } else {
+          y[z] = two(whole[z]);
+        }
+      if constexpr (FRESH == IN_PARTS) {
+        for (int p = AHEAD; p < fresh.parts; ++p)
+#pragma unroll
+          for (int z = 0; z < 2; ++z)
+            y[z] += *reinterpret_cast<const floatx2*>((const float*)fresh.qkv + row +
+                                                      p * fresh.step + (column + z * HALF));
+        y[0] = round(y[0]), y[1] = round(y[1]);
+      }
+      if (fresh.bias) y[0] = round(y[0] + two(bias[0])), y[1] = round(y[1] + two(bias[1]));
+      if (!is_v)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const float x1 = y[0][j], x2 = y[1][j];
+          y[0][j] = __builtin_fmaf(x1, cs[j], -(x2 * sn[j]));
+          y[1][j] = __builtin_fmaf(x2, cs[j], x1 * sn[j]);
+        }
+      if (is_q) {
+#pragma unroll
+        for (int z = 0; z < 2; ++z)
+          *reinterpret_cast<unsigned*>(s_q + h * D + i + z * HALF) = cvt2_bf16(y[z][0], y[z][1]);
+        return;
+      }
+      using pair = std::conditional_t<FP8, unsigned short, unsigned>;
+      char* cache = (char*)(is_v ? fresh.vc : fresh.kc) + (slot + i) * EB;
+#pragma unroll
+      for (int z = 0; z < 2; ++z) {
+        pair v;
+        if constexpr (FP8) v = (pair)__builtin_amdgcn_cvt_pk_fp8_f32(y[z][0], y[z][1], 0u, false);
+        else v = cvt2_bf16(y[z][0], y[z][1]);
+        *reinterpret_cast<pair*>(s_kv + ((is_v ? D : 0) + i + z * HALF) * EB) = v;
+        if (keep) *reinterpret_cast<pair*>(cache + z * HALF * EB) = v;
+      }
+    };
+    if (wave * WAVE < all) take(min((int)threadIdx.x, all - 1), request);
+    else request();
+    for (int x0 = DEC_WAVES * WAVE; x0 + wave * WAVE < all; x0 += DEC_WAVES * WAVE)
+      take(min(x0 + (int)threadIdx.x, all - 1), [] {});
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (keys stay on their way)
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+      qf[c].s = shortx8{0, 0, 0, 0, 0, 0, 0, 0};
+      if (mine) qf[c].s = *reinterpret_cast<const shortx8*>(s_q + head * D + c * 32 + g * 8);
+    }
+  }
+  if (t0 < t_hi) {
+    if constexpr (!FRESH) {
+      lookup(t0);
+      load_keys(t0, page_row, EVEN{});
+      load_values(t0, page_row);
+    }
     lookup(t0 + ROUND);
     for (;;) {
       compute(t0, EVEN{});
@@ -562,14 +722,14 @@ long decode_marks(long B, long Hq, long Hkv, long longest, long window, long chu
   return longest > std::max<long>(256, B * tiles * B * tiles / 16) ? B * tiles : 0;
 }
 
-template <int D, int DV, bool FP8, int BIAS>
+template <int D, int DV, bool FP8, int BIAS, int FRESH = 0>
 static void decode_launch(const torch::Tensor& q, const torch::Tensor& kc,
                           const torch::Tensor& vc, const torch::Tensor& bt,
                           const torch::Tensor& ctx, __hip_bfloat16* out, long ostride,
                           int dv, float scale, float oscale, const float* slopes,
                           const float* rates, int window, int chunk, const float* sink,
                           const HeadTurn& turn,
-                          const c10::optional<torch::Tensor>& marks) {
+                          const c10::optional<torch::Tensor>& marks, const Fresh& fresh = {}) {
   const int B = q.size(0), Hq = q.size(1);
   const int Hkv = kc.size(1), P = kc.size(2), MP = bt.size(1);
   const int tiles = Hkv * ((Hq / Hkv + DEC_HEADS - 1) / DEC_HEADS);
@@ -589,10 +749,13 @@ static void decode_launch(const torch::Tensor& q, const torch::Tensor& kc,
                        (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(), vc.data_ptr(), out,
                        pp, cut ? arrived.data_ptr<int>() : nullptr, bt.data_ptr<int>(),
                        ctx.data_ptr<int>(), B, Hq, Hkv, P, MP,
-                       scale, ostride, dv, oscale, slopes, rates, seen, sink, turn);
+                       scale, ostride, dv, oscale, slopes, rates, seen, sink, turn, fresh);
   };
   const bool paged = P % DEC_KEYS == 0;
-  if (paged && cut) launch(paged_decode_kernel<D, DV, FP8, BIAS, true, true>);
+  if constexpr (FRESH) {
+    if (cut) launch(paged_decode_kernel<D, DV, FP8, BIAS, true, true, FRESH>);
+    else launch(paged_decode_kernel<D, DV, FP8, BIAS, true, false, FRESH>);
+  } else if (paged && cut) launch(paged_decode_kernel<D, DV, FP8, BIAS, true, true>);
   else if (paged) launch(paged_decode_kernel<D, DV, FP8, BIAS, true, false>);
   else if (cut) launch(paged_decode_kernel<D, DV, FP8, BIAS, false, true>);
   else launch(paged_decode_kernel<D, DV, FP8, BIAS, false, false>);
@@ -619,6 +782,48 @@ torch::Tensor paged_attention_decode(torch::Tensor q, torch::Tensor kc,
   if (D == 128) { if (fp8) RUN(128, true); else RUN(128, false); }
   else { if (fp8) RUN(64, true); else RUN(64, false); }
 #undef RUN
+  return out;
+}
+
+// The same of rows that are the last of their sequences, none of which comes twice: ``qkv`` [B,
+// (Hq + 2 Hkv) D] is the projection, whole or in parts, to which a bias is added; the new keys and
+// values go where the tables have the last of ``ctx`` positions. Nothing where there is no form.
+c10::optional<torch::Tensor> fresh_attention_decode(
+    torch::Tensor qkv, c10::optional<torch::Tensor> bias, torch::Tensor cos_sin, torch::Tensor kc,
+    torch::Tensor vc, torch::Tensor bt, torch::Tensor ctx, long Hq, double scale,
+    c10::optional<torch::Tensor> marks) {
+  const bool raw = qkv.dtype() == torch::kFloat32 && qkv.dim() == 3;
+  if (!qkv.is_cuda() || !qkv.is_contiguous() || (!raw && qkv.dtype() != torch::kBFloat16))
+    return {};
+  const long B = qkv.size(raw ? 1 : 0), Hkv = kc.size(1), P = kc.size(2), D = kc.size(3);
+  const long width = (Hq + 2 * Hkv) * D;
+  const bool fp8 = kc.dtype() == torch::kFloat8_e4m3fn;
+  if (B == 0 || (D != 64 && D != 128) || vc.size(3) != D || Hq % Hkv || P % DEC_KEYS ||
+      qkv.dim() != (raw ? 3 : 2) || qkv.size(-1) != width || vc.dtype() != kc.dtype() ||
+      (!fp8 && kc.dtype() != torch::kBFloat16) || cos_sin.dtype() != torch::kFloat32 ||
+      cos_sin.dim() != 2 || cos_sin.size(1) != D || bt.dim() != 2 || bt.size(0) != B ||
+      ctx.numel() != B ||
+      bt.dtype() != torch::kInt32 || ctx.dtype() != torch::kInt32 ||
+      (bias && (bias->dtype() != torch::kBFloat16 || bias->numel() != width)))
+    return {};
+  for (const torch::Tensor* t : {&qkv, &kc, &vc, &cos_sin, bias ? &*bias : &qkv, &bt, &ctx})
+    if (t->device() != qkv.device() || !t->is_contiguous() ||
+        (t != &bt && t != &ctx && (uintptr_t)t->data_ptr() % 16))
+      return {};
+  auto out = torch::empty({B, Hq, D}, qkv.options().dtype(torch::kBFloat16));
+  const Fresh fresh = {qkv.data_ptr(), bias ? (const unsigned short*)bias->data_ptr() : nullptr,
+                       cos_sin.data_ptr<float>(), kc.data_ptr(), vc.data_ptr(),
+                       raw ? (int)qkv.size(0) : 1, B * width};
+#define RUN1(DD, F8, HOW)                                                                   \
+  decode_launch<DD, DD, F8, NO_BIAS, HOW>(out, kc, vc, bt, ctx, o, Hq* D, DD, (float)scale, \
+                                          1.f, nullptr, nullptr, 0, 0, nullptr, HeadTurn{}, \
+                                          marks, fresh)
+#define RUN(DD, F8) if (raw) RUN1(DD, F8, IN_PARTS); else RUN1(DD, F8, WHOLE)
+  auto* o = (__hip_bfloat16*)out.data_ptr();
+  if (D == 128) { if (fp8) { RUN(128, true); } else { RUN(128, false); } }
+  else { if (fp8) { RUN(64, true); } else { RUN(64, false); } }
+#undef RUN
+#undef RUN1
   return out;
 }
 

@@ -94,6 +94,10 @@ void biased_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
                               long window, long chunk, OptT slopes, OptT rates, OptT sink,
                               OptT turn, OptT gate, torch::Tensor out, long col, long dv,
                               double oscale);
+c10::optional<torch::Tensor> fresh_attention_decode(
+    torch::Tensor qkv, c10::optional<torch::Tensor> bias, torch::Tensor cos_sin, torch::Tensor kc,
+    torch::Tensor vc, torch::Tensor bt, torch::Tensor ctx, long Hq, double scale,
+    c10::optional<torch::Tensor> marks);
 void biased_attention_decode(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
                              torch::Tensor bt, torch::Tensor ctx, double scale, long window,
                              long chunk, OptT slopes, OptT rates, OptT sink, OptT turn,
@@ -241,6 +245,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("biased_prefill_rows", &biased_prefill_rows);
   m.def("biased_attention_prefill", &biased_attention_prefill,
         "MFMA flash prefill with distance bias, window or chunks, sink, turn and gate");
+  m.def("fresh_attention_decode", &fresh_attention_decode,
+        "rotation, cache write and decode attention of rows of different sequences");
   m.def("biased_attention_decode", &biased_attention_decode,
         "paged decode with distance bias, window or chunks, sink, turn and gate",
         py::arg("q"), py::arg("kc"), py::arg("vc"), py::arg("bt"), py::arg("ctx"),

@@ -5,8 +5,9 @@
 // all rows of x, in steps of 64 of K through a ring of LDS stages that direct-to-LDS loads fill
 // several steps ahead: two workgroups of 72 to 80 KB fit a CU and have 48 to 80 KB of W
 // under way. A wave multiplies 16 rows of W with all of x, or from 33 rows of x on 32 with
-// half of it, which takes less from LDS: a lane ends with four outputs that lie side by side. Reading W straight into fragments instead, with K split over the
-// waves of a workgroup and no LDS, came to the same at one row and lost at 16 and more
+// half of it, which takes less from LDS: a lane ends with four outputs that lie side by side.
+// Reading W straight into fragments instead, with K split over the waves of a workgroup and no
+// LDS, came to the same at one row and lost at 16 and more
 // (x is then read as often as W's tiles of 16 rows: 28672 x 4096, 32 rows, 86 us).
 //
 // Few tiles of W leave the chip idle, so K is cut into parts as well (``parts_of``). Their
@@ -50,8 +51,8 @@ DEVINL void await_stage() {
 // the sums of its steps' two halves apart, parts 2 y and 2 y + 1; z are blocks of 16 MT rows of x.
 // A wave's tiles of 16 are RT of W by MW of x. (2 by half of x instead of 1 by all: 64 wide 0.4%
 // faster at 33 to 64 rows, 2.2% at 128, means of 18 weights of 16 MB and more.)
-// (Tiles of one part of K side by side on an XCD, so that its L2 reads that part of x alone: products
-// by themselves 1% faster, steps of 1 to 96 rows of whole models up to 1.5% slower.)
+// (Tiles of one part of K side by side on an XCD, so that its L2 reads that part of x alone:
+// products by themselves 1% faster, steps of 1 to 96 rows of whole models up to 1.5% slower.)
 template <int WN, int MT, int NS, bool SILU, bool ROUTER = false>
 __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
     const unsigned short* x, const unsigned short* w, unsigned short* out, float* part, int M,
@@ -63,7 +64,8 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
   __shared__ __attribute__((aligned(16))) char lds[NS * STAGE];
   const int tid = threadIdx.x, lane = tid % WAVE;
   const int wave = __builtin_amdgcn_readfirstlane(tid / WAVE);
-  const int at = lane & 15, g = lane >> 4, r0 = wave % ACROSS * RT * 16, x0 = wave / ACROSS * MW * 16;
+  const int at = lane & 15, g = lane >> 4;
+  const int r0 = wave % ACROSS * RT * 16, x0 = wave / ACROSS * MW * 16;
   const int n0 = blockIdx.x * (SILU ? WN / 2 : WN);
   const int k0 = blockIdx.y * (ROUTER ? FEW_K : span), m0 = ROUTER ? blockIdx.z * 16 * MT : 0;
   const int stride = ROUTER ? gridDim.y * FEW_K : FEW_K;
@@ -502,7 +504,8 @@ torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw) {
   // x 2048, 23 rows, 8.2 us whole, 4.0 and 4.7 in parts; 4096 x 4096 16.7, 8.9 and 2.4; 2048
   // x 2048, 64 rows, 11.7, 5.5 and 4.2.
   // More than 8192 outputs are cut for their reader alone: float_few_rows has their bits.
-  const bool cut = raw || (x.size(1) * (x.size(0) > 32 ? 2 : 1) >= 4096 && parts_of(w.size(0), x.size(1)) > 1);
+  const bool cut = raw || (x.size(1) * (x.size(0) > 32 ? 2 : 1) >= 4096 &&
+                           parts_of(w.size(0), x.size(1)) > 1);
   return cut_rows(x, w, raw, cut ? cut_of(x.size(0), w.size(0), x.size(1)) : Cut{64, 1});
 }
 
