@@ -58,8 +58,29 @@ struct KeyTail {
   int own;    // dimensions in kc, a multiple of 8
 };
 
+// Few rows behind long contexts have fewer blocks than there are CUs, and a workgroup takes 1.6 us
+// a tile of keys whatever the others do. The tiles of a block, unless they are few, are then cut
+// into up to ``most`` parts, by a workgroup each, whose results [rows, heads, most, DV] and
+// references and sums [.., 2] another kernel merges. 32 heads of 128 over 8, us, whole and cut:
+// 100 rows behind 1500 45.8 and 27.5, behind 8000 199 and 37; 500 behind 1500 57.0 and 40.2, behind
+// 8000 211 and 85; 1000 behind 8000 224 and 157; 4 of 60 behind 4000 106 and 45.
+struct Cut {
+  int most;
+  float *part, *refs;
+};
+#define CUT_LEAST 6  // tiles of a part
+// tiles of a part of a block that has n
+DEVINL int part_tiles(int n, int most) {
+  return n < 2 * CUT_LEAST ? 2 * CUT_LEAST : max(CUT_LEAST, (n + most - 1) / most);
+}
+// tiles of keys that the rows qoff.. of a block see
+DEVINL int block_tiles(int qlen, int ctx, int qoff, int rows) {
+  const int kend = min(ctx, ctx - qlen + qoff + min(qlen - qoff, rows));
+  return (kend + PRE_KEYS - 1) / PRE_KEYS;
+}
+
 // HG: query heads per workgroup; PAGED: pages are whole tiles
-template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED>
+template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED, bool CUT = false>
 __global__ __launch_bounds__(512, 1) void prefill_kernel(
     const __hip_bfloat16* __restrict__ q,   // [T, qstride], heads D apart
     const void* __restrict__ kc,  // [NP, Hkv, P, D] bf16 | fp8 e4m3
@@ -75,7 +96,8 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
     const float* __restrict__ slopes, const float* __restrict__ rates, int window,
     int chunk, const float* __restrict__ sink,  // [Hq], or null unless GATED
     const __hip_bfloat16* __restrict__ gate, long gstride,  // [T, gstride]
-    KeyTail tail, HeadTurn turn) {
+    KeyTail tail, HeadTurn turn, Cut cut) {
+  static_assert(!CUT || (!BIAS && EXTRA == PLAIN));
   constexpr int NC = D / 16;        // Q^T fragments (MFMA K-chunks of K Q^T)
   constexpr int NDT = DV / 32;      // 32-wide d-tiles of O^T
   constexpr int KU = D / 8, VU = DV / 8;         // 16-B units of a key's, a value's row
@@ -87,7 +109,8 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
   constexpr int QS = 8 / HG;          // 32-row q sub-blocks per WG
   const int groups = Hq / HG;
   // late rows see most keys: first
-  const int nb = gridDim.x / groups - 1 - blockIdx.x / groups;
+  const int apart = CUT ? cut.most : 1, part = CUT ? blockIdx.x / groups % apart : 0;
+  const int nb = gridDim.x / groups / apart - 1 - blockIdx.x / groups / apart;
   const int lane = threadIdx.x % WAVE;
   int seq, qoff;
   if (block_seq) {
@@ -150,7 +173,16 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
   // keys needed by this q block: up to the last row's absolute position
   const int blk_rows = min(qlen - qoff, QS * 32);
   const int kend = min(ctx, ctx - qlen + qoff + blk_rows);
-  const int ntiles = (kend + PRE_KEYS - 1) / PRE_KEYS;
+  int ntiles = (kend + PRE_KEYS - 1) / PRE_KEYS;
+  bool whole = true;  // this workgroup sees all of the block's keys
+  int from = 0;       // and the first tile it sees
+  if constexpr (CUT) {
+    const int per = part_tiles(ntiles, cut.most);
+    from = part * per;
+    whole = ntiles <= per;
+    if (part > 0 && from >= ntiles) return;
+    ntiles = min(ntiles, from + per);
+  }
   // absolute position of the wave's first (smallest) q row
   const int q_abs_min = ctx - qlen + qoff + qsub * 32;
 
@@ -165,13 +197,14 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
     const int lo = x - win + 1;
     return BIAS && chunk > 0 ? max(lo, x - x % chunk) : lo;
   };
-  const int tile0 = BIAS ? max(0, first_seen(ctx - qlen + qoff)) / PRE_KEYS : 0;
+  const int tile0 = BIAS ? max(0, first_seen(ctx - qlen + qoff)) / PRE_KEYS : from;
   const int lo = BIAS ? first_seen(q_abs) : 0;
   const int lo_max = BIAS ? first_seen(q_abs_min + 31) : 0;
   // tiles that the wave's rows see; the first of its workgroup's where there are no rows
   const bool rows = qoff + qsub * 32 < qlen;
   const int first = rows && BIAS ? max(first_seen(q_abs_min), 0) / PRE_KEYS : tile0;
-  const int end = rows ? (min(kend, q_abs_min + 32) + PRE_KEYS - 1) / PRE_KEYS : tile0;
+  int end = rows ? (min(kend, q_abs_min + 32) + PRE_KEYS - 1) / PRE_KEYS : tile0;
+  if constexpr (CUT) end = max(tile0, min(end, ntiles));
 
   // ---- tiles. A thread's unit x of a tile is unit tid + 512 x in LDS and takes what the
   // swizzle puts there. Pages are looked up a tile before the loads that need them (by
@@ -490,6 +523,20 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
   // ---- epilogue: a lane holds channels 4 half + {0..3} of every 8 of its row
   l += __shfl_xor(l, 32, WAVE);
   const long row = q_start + qrow;
+  if constexpr (CUT) {
+    if (!whole) {
+      if (!qvalid) return;
+      const long at = (row * Hq + h) * cut.most + part;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<floatx4*>(cut.part + at * DV + dt * 32 + 8 * g + 4 * half) =
+              floatx4{o[dt][4 * g], o[dt][4 * g + 1], o[dt][4 * g + 2], o[dt][4 * g + 3]};
+      if (half == 0) *reinterpret_cast<floatx2*>(cut.refs + at * 2) = floatx2{m, l};
+      return;
+    }
+  }
   if constexpr (EXTRA == GATED) {  // divided by l, times the gate
     const long grow = (q_start + (qvalid ? qrow : 0)) * gstride + h;
     l *= 1.f + __expf(-bf16_to_f32(((const unsigned short*)gate)[grow]));
@@ -547,6 +594,55 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
   }
 }
 
+// A row of every block whose keys were cut: its parts' results put together, a wave per head.
+template <int DV>
+__global__ __launch_bounds__(256) void merge_parts_kernel(
+    Cut cut, __hip_bfloat16* __restrict__ out, const int* __restrict__ cu_q, int S,
+    const int* __restrict__ ctx_lens, int Hq, int rows) {
+  constexpr int N = DV / WAVE;
+  const int row = blockIdx.x, lane = threadIdx.x % WAVE;
+  const int h = blockIdx.y * 4 + threadIdx.x / WAVE;
+  if (h >= Hq) return;
+  int seq = 0;  // sequences that end before the row
+  for (int s0 = 0; s0 < S; s0 += WAVE)
+    seq += __popcll(__ballot(s0 + lane < S && cu_q[min(s0 + lane, S - 1) + 1] <= row));
+  seq = __builtin_amdgcn_readfirstlane(seq);
+  if (seq >= S) return;
+  const int qlen = cu_q[seq + 1] - cu_q[seq], qoff = (row - cu_q[seq]) / rows * rows;
+  const int n = block_tiles(qlen, ctx_lens[seq], qoff, rows), per = part_tiles(n, cut.most);
+  if (n <= per) return;
+  const int parts = (n + per - 1) / per;
+  const long at = ((long)row * Hq + h) * cut.most;
+  constexpr int AT_ONCE = 8;
+  float o[AT_ONCE][N], y[N] = {};
+  auto read = [&](int p0) {
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; ++k)
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        o[k][j] = cut.part[(at + min(p0 + k, parts - 1)) * DV + lane * N + j];
+  };
+  const floatx2 mine =
+      *reinterpret_cast<const floatx2*>(cut.refs + (at + min(lane, parts - 1)) * 2);
+  read(0);
+  const float m = lane < parts ? mine[0] : -1e30f, M = wave_max(m);
+  const float f = lane < parts ? __builtin_amdgcn_exp2f(m - M) : 0.f;
+  const float inv = 1.f / wave_sum(f * mine[1]);
+  for (int p0 = 0; p0 < parts; p0 += AT_ONCE) {
+    if (p0 > 0) read(p0);
+#pragma unroll
+    for (int k = 0; k < AT_ONCE; ++k) {
+      const float fp = __shfl(f, p0 + k, WAVE);
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (p0 + k < parts) y[j] += fp * o[k][j];
+    }
+  }
+  auto* dst = (unsigned short*)out + ((long)row * Hq + h) * DV + lane * N;
+  if constexpr (N == 2) *reinterpret_cast<unsigned*>(dst) = cvt2_bf16(y[0] * inv, y[1] * inv);
+  else dst[0] = f32_to_bf16(y[0] * inv);
+}
+
 // query heads per workgroup: the GQA group shares each staged K/V tile
 static int heads_per_block(int G) { return G % 4 == 0 ? 4 : G % 2 == 0 ? 2 : 1; }
 
@@ -556,16 +652,18 @@ static torch::Tensor unit_aligned(const torch::Tensor& cache) {
   return ok ? cache : cache.clone();
 }
 
-template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED, typename... Args>
-static void prefill_launch(int blocks, int Hq, Args... args) {
+template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED, bool CUT = false,
+          typename... Args>
+static void prefill_launch(const Cut& cut, int blocks, int Hq, Args... args) {
   constexpr int lds = PRE_STAGES * PRE_KEYS * (D + DV) * 2;
-  const auto kern = prefill_kernel<D, DV, HG, FP8, BIAS, EXTRA, PAGED>;
+  const auto kern = prefill_kernel<D, DV, HG, FP8, BIAS, EXTRA, PAGED, CUT>;
   if (lds > 64 * 1024) {
     static const hipError_t once = hipFuncSetAttribute(
         (const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     TORCH_CHECK(once == hipSuccess, "attention prefill: LDS");
   }
-  hipLaunchKernelGGL(kern, dim3(blocks * (Hq / HG)), dim3(512), lds, CUR_STREAM, args...);
+  hipLaunchKernelGGL(kern, dim3(blocks * (CUT ? cut.most : 1) * (Hq / HG)), dim3(512), lds,
+                     CUR_STREAM, args..., cut);
 }
 
 torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
@@ -586,8 +684,25 @@ torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
   // as many blocks as there can be; each finds its rows, so that nothing is read back
   const int S = cu_q.numel() - 1, NB = T / QROWS + S;
   const bool fp8 = kc.dtype() == torch::kFloat8_e4m3fn;
-#define PLAUNCH1(DD, HGV, F8, PG)                                               \
-  prefill_launch<DD, DD, HGV, F8, NO_BIAS, PLAIN, PG>(NB, Hq,                      \
+  // A workgroup for every CU. The parts' way through memory and the merging take what is gained
+  // of few tiles, the more the more blocks there are: 20 rows behind 700 (12 tiles, 8 blocks) 21.3
+  // us whole and 18.1 cut, 300 behind 300 and 700 (10 and 16 tiles, 40 blocks) 23.7 and 29.1, 32.8
+  // and 33.2, 500 behind 300 and 1000 (13 and 24, 64) 28.7 and 35.1, 45.9 and 38.0, 1000 behind 300,
+  // 700 and 1500 (21, 27 and 40, 128) 40.8 and 47.6, 51.0 and 52.8, 70.5 and 63.8. (What the tables
+  // have room for stands for the longest context; short ones of wide tables stay whole all the
+  // same.)
+  const long blocks = (long)NB * (Hq / HG), least = 2 * CUT_LEAST + blocks / 8;
+  Cut cut = {1, nullptr, nullptr};
+  if (P % PRE_KEYS == 0 && (long)MP * P / PRE_KEYS >= least)
+    cut.most = (int)std::max(1L, std::min(256 / blocks, 16L));
+  torch::Tensor part, refs;
+  if (cut.most > 1) {
+    part = torch::empty({(long)T * Hq * cut.most * D}, q.options().dtype(torch::kFloat32));
+    refs = torch::empty({(long)T * Hq * cut.most * 2}, q.options().dtype(torch::kFloat32));
+    cut.part = part.data_ptr<float>(), cut.refs = refs.data_ptr<float>();
+  }
+#define PLAUNCH1(DD, HGV, F8, PG, CT)                                           \
+  prefill_launch<DD, DD, HGV, F8, NO_BIAS, PLAIN, PG, CT>(cut, NB, Hq,             \
                      (const __hip_bfloat16*)q.data_ptr(),                     \
                      kc.data_ptr(), vc.data_ptr(),                            \
                      (__hip_bfloat16*)out.data_ptr(),                         \
@@ -596,11 +711,14 @@ torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
                      (long)Hq * D, (long)Hq * D, D, 1.f, nullptr, nullptr, 0, \
                      0, nullptr, nullptr, 0, KeyTail{}, HeadTurn{})
 #define PLAUNCH(DD, HGV)                                                      \
-  if (P % PRE_KEYS == 0) {                                                    \
-    if (fp8) { PLAUNCH1(DD, HGV, true, true); }                               \
-    else { PLAUNCH1(DD, HGV, false, true); }                                  \
-  } else if (fp8) { PLAUNCH1(DD, HGV, true, false); }                         \
-  else { PLAUNCH1(DD, HGV, false, false); }
+  if (cut.most > 1) {                                                         \
+    if (fp8) { PLAUNCH1(DD, HGV, true, true, true); }                         \
+    else { PLAUNCH1(DD, HGV, false, true, true); }                            \
+  } else if (P % PRE_KEYS == 0) {                                             \
+    if (fp8) { PLAUNCH1(DD, HGV, true, true, false); }                        \
+    else { PLAUNCH1(DD, HGV, false, true, false); }                           \
+  } else if (fp8) { PLAUNCH1(DD, HGV, true, false, false); }                  \
+  else { PLAUNCH1(DD, HGV, false, false, false); }
 #define PLAUNCH_D(DD)                                                         \
   switch (HG) {                                                               \
     case 1: PLAUNCH(DD, 1); break;                                            \
@@ -616,6 +734,13 @@ torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
 #undef PLAUNCH
 #undef PLAUNCH1
   HIP_CHECK_KERNEL();
+  if (cut.most > 1) {
+    const auto merge = D == 128 ? merge_parts_kernel<128> : merge_parts_kernel<64>;
+    hipLaunchKernelGGL(merge, dim3(T, (Hq + 3) / 4), dim3(256), 0, CUR_STREAM, cut,
+                       (__hip_bfloat16*)out.data_ptr(), cu_q.data_ptr<int>(), S,
+                       ctx.data_ptr<int>(), Hq, QROWS);
+    HIP_CHECK_KERNEL();
+  }
   return out;
 }
 
@@ -654,7 +779,7 @@ void biased_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
   const float* sp = slopes ? slopes->data_ptr<float>() : nullptr;
   const float* snk = sink ? sink->data_ptr<float>() : nullptr;
 #define BLAUNCH2(DD, DVV, HGV, BB, XX, PG)                                      \
-  prefill_launch<DD, DVV, HGV, false, BB, XX, PG>(NB, Hq,                            \
+  prefill_launch<DD, DVV, HGV, false, BB, XX, PG>(Cut{}, NB, Hq,                            \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr() + col,      \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
@@ -715,7 +840,7 @@ void sink_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   kc = unit_aligned(kc);
   vc = unit_aligned(vc);
 #define SLAUNCH(DD, DVV)                                                        \
-  prefill_launch<DD, DVV, 1, false, NO_BIAS, GATED, false>(NB, H,                       \
+  prefill_launch<DD, DVV, 1, false, NO_BIAS, GATED, false>(Cut{}, NB, H,                       \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr(),            \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
@@ -767,7 +892,7 @@ void tailed_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
   const KeyTail kt = {(const __hip_bfloat16*)tail.data_ptr(), tail.stride(0),
                       (int)tail.size(1), own};
 #define TLAUNCH(DD, DVV)                                                        \
-  prefill_launch<DD, DVV, 1, false, FLAT_BIAS, TAILED, false>(NB, H,                    \
+  prefill_launch<DD, DVV, 1, false, FLAT_BIAS, TAILED, false>(Cut{}, NB, H,                    \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr(),            \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
