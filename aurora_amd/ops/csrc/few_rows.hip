@@ -396,6 +396,7 @@ struct Cut {
 static Cut cut_of(long M, long N, long K) {
   const long steps = K / FEW_K, rows = M <= 32 ? 32 : (M + 31) / 32 * 32;
   Cut best = {64, 1};
+  if (N == 0 || steps == 0) return best;
   // a single row's parts are read by a norm in the next product, which takes few (one_row_fits)
   if (M == 1 && N <= 4096) return {64, parts_of(N, K)};
   double low = 0;
