@@ -95,6 +95,12 @@ class AttnMetadata:
         return out
 
 
+def _steady(kv_cache, meta) -> bool:
+    """Whether the products' sums keep their order (``ops.linear``): in prompts that fill an
+    8-bit cache, not where each sequence adds one row to its many."""
+    return meta.mode != "decode" and kv_cache[0].element_size() == 1
+
+
 class LlamaAttention(nn.Module):
     def __init__(self, spec: ModelSpec, dtype):
         super().__init__()
@@ -121,12 +127,13 @@ class LlamaAttention(nn.Module):
 
     def parts(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
         """As ``forward``, possibly in parts (``ops.linear_parts``)."""
-        return row_parts(self.o_proj, self._heads(x, cos_sin, kv_cache, meta))
+        return row_parts(self.o_proj, self._heads(x, cos_sin, kv_cache, meta),
+                         _steady(kv_cache, meta))
 
     def _heads(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
         """The heads' results side by side, [T, heads * width]."""
         T = x.shape[0]
-        qkv, bias = column_parts(self.qkv_proj, x)
+        qkv, bias = column_parts(self.qkv_proj, x, _steady(kv_cache, meta))
         k_cache, v_cache = kv_cache
         if meta.mode == "decode" and getattr(meta, "last_tokens", False):
             o = ops.fresh_attention_decode(
@@ -176,9 +183,9 @@ class LlamaMLP(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         return self.down(column_silu_mul(self.gate_up, x))
 
-    def parts(self, x: torch.Tensor) -> torch.Tensor:
+    def parts(self, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
         """As ``forward``, possibly in parts (``ops.linear_parts``)."""
-        return row_parts(self.down, column_silu_mul(self.gate_up, x))
+        return row_parts(self.down, column_silu_mul(self.gate_up, x, steady), steady)
 
 
 class _FullWidthMLP(nn.Module):
@@ -371,8 +378,11 @@ class LlamaDecoderLayer(nn.Module):
         a = attn(h, cos_sin, kv_cache, meta)
         h, residual = ops.norm_ahead(a, residual, self.post_attn_norm, self.eps,
                                      self._reader("mlp", a) if in_parts else None, True)
-        mlp = self.mlp.parts if in_parts and is_plain(self.mlp, LlamaMLP) else self.mlp
-        return mlp(h), residual
+        if not in_parts or not is_plain(self.mlp, LlamaMLP):
+            return self.mlp(h), residual
+        if _steady(kv_cache, meta):
+            return self.mlp.parts(h, True), residual
+        return self.mlp.parts(h), residual
 
     def _reader(self, what: str, x: torch.Tensor) -> Optional[torch.Tensor]:
         """The weight whose product alone reads the norm before ``what``, if x, the norm's

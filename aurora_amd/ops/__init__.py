@@ -255,10 +255,11 @@ def knn_topk(query: torch.Tensor, docs: torch.Tensor, k: int):
     return torch_ref.knn_topk(query, docs, k)
 
 
-def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+def linear(x: torch.Tensor, weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """Bias-free linear: own kernels on the GPU where they win (``own_product``),
-    hipBLASLt otherwise."""
-    y = _hip.own_product(x, weight, 0) if x.is_cuda and _hip is not None else None
+    hipBLASLt otherwise. ``steady``: the sums keep their order, for what an 8-bit cache is
+    filled with, whose bytes show it."""
+    y = _hip.own_product(x, weight, 4 if steady else 0) if x.is_cuda and _hip is not None else None
     return F.linear(x, weight) if y is None else y
 
 
@@ -293,24 +294,24 @@ def norm_ahead(x, residual, weight, eps, reader: Optional[torch.Tensor], silu: b
     return rmsnorm_residual(x, residual, weight, eps)
 
 
-def linear_parts(x, weight: torch.Tensor) -> torch.Tensor:
+def linear_parts(x, weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """As ``linear``, but where the product of few rows is cut along K its parts
     [S, T, N] in float32, for a reader that adds and rounds them itself
     (``rmsnorm_residual``, ``fused_rope_kv_write``). ``x``: rows, or one of
     ``norm_ahead``."""
     if isinstance(x, Unnormed):
         return _hip.one_row_product(*x, weight, False)
-    y = _hip.own_product(x, weight, 1) if x.is_cuda and _hip is not None else None
+    y = _hip.own_product(x, weight, 5 if steady else 1) if x.is_cuda and _hip is not None else None
     return F.linear(x, weight) if y is None else y
 
 
-def linear_silu_mul(x, weight: torch.Tensor) -> torch.Tensor:
+def linear_silu_mul(x, weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """silu(gate) * up of the products with gate's rows, then up's; in one kernel where that
     is faster. ``x``: rows, or one of ``norm_ahead``."""
     if isinstance(x, Unnormed):
         return _hip.one_row_product(*x, weight, True)
     y = _hip.own_product(x, weight, 2) if x.is_cuda and _hip is not None else None
-    return silu_mul(linear(x, weight)) if y is None else y
+    return silu_mul(linear(x, weight, steady)) if y is None else y
 
 
 def has_moe_grouped(x: torch.Tensor, router: Optional[torch.Tensor] = None) -> bool:

@@ -690,10 +690,11 @@ torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
   // and 33.2, 500 behind 300 and 1000 (13 and 24, 64) 28.7 and 35.1, 45.9 and 38.0, 1000 behind 300,
   // 700 and 1500 (21, 27 and 40, 128) 40.8 and 47.6, 51.0 and 52.8, 70.5 and 63.8. (What the tables
   // have room for stands for the longest context; short ones of wide tables stay whole all the
-  // same.)
+  // same.) An 8-bit cache is not cut: the next layers' rows in it are made of these results, and
+  // other sums let one in 20 to 50 of their bytes round the other way.
   const long blocks = (long)NB * (Hq / HG), least = 2 * CUT_LEAST + blocks / 8;
   Cut cut = {1, nullptr, nullptr};
-  if (P % PRE_KEYS == 0 && (long)MP * P / PRE_KEYS >= least)
+  if (!fp8 && P % PRE_KEYS == 0 && (long)MP * P / PRE_KEYS >= least)
     cut.most = (int)std::max(1L, std::min(256 / blocks, 16L));
   torch::Tensor part, refs;
   if (cut.most > 1) {
@@ -712,8 +713,7 @@ torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
                      0, nullptr, nullptr, 0, KeyTail{}, HeadTurn{})
 #define PLAUNCH(DD, HGV)                                                      \
   if (cut.most > 1) {                                                         \
-    if (fp8) { PLAUNCH1(DD, HGV, true, true, true); }                         \
-    else { PLAUNCH1(DD, HGV, false, true, true); }                            \
+    PLAUNCH1(DD, HGV, false, true, true);                                     \
   } else if (P % PRE_KEYS == 0) {                                             \
     if (fp8) { PLAUNCH1(DD, HGV, true, true, false); }                        \
     else { PLAUNCH1(DD, HGV, false, true, false); }                           \

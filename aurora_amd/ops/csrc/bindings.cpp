@@ -29,7 +29,7 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
                                          long form);
 torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
 torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width);
-torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
+torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor weight, double eps,
                               torch::Tensor res_out, torch::Tensor w, bool silu);
@@ -208,7 +208,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("many_rows", &many_rows, "products of many rows, with silu(gate) * up");
   m.def("few_rows", &few_rows, "products of at most 128 rows, K in parts", py::arg("x"),
         py::arg("w"), py::arg("raw"), py::arg("parts"), py::arg("width") = 64);
-  m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows");
+  m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows", py::arg("x"),
+        py::arg("w"), py::arg("raw"), py::arg("steady") = false);
   m.def("one_row_product", &one_row_product, "a norm and the product of its one row");
   m.def("norms_row", &norms_row, "whether one_row_product serves");
   m.def("silu_few_rows", &silu_few_rows, "gate and up of at most 128 rows, silu(gate) * up");

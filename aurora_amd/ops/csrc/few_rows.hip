@@ -500,14 +500,16 @@ torch::Tensor router_rows(const torch::Tensor& x, const torch::Tensor& w) {
   return part;
 }
 
-torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw) {
+// ``steady``: as parts_of has K's parts, for any number of rows
+torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady) {
   // A kernel to add the parts pays off where a tile's steps take much longer than it: 2048
   // x 2048, 23 rows, 8.2 us whole, 4.0 and 4.7 in parts; 4096 x 4096 16.7, 8.9 and 2.4; 2048
   // x 2048, 64 rows, 11.7, 5.5 and 4.2.
   // More than 8192 outputs are cut for their reader alone: float_few_rows has their bits.
   const bool cut = raw || (x.size(1) * (x.size(0) > 32 ? 2 : 1) >= 4096 &&
                            parts_of(w.size(0), x.size(1)) > 1);
-  return cut_rows(x, w, raw, cut ? cut_of(x.size(0), w.size(0), x.size(1)) : Cut{64, 1});
+  const long M = x.size(0), N = w.size(0), K = x.size(1);
+  return cut_rows(x, w, raw, !cut ? Cut{64, 1} : steady ? Cut{64, parts_of(N, K)} : cut_of(M, N, K));
 }
 
 // linear_few_rows's result in float32, where K is not cut, without a kernel to convert it: 1 row

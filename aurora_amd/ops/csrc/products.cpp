@@ -7,7 +7,7 @@
 #include <cstring>
 
 // defined in few_rows.hip, moe.hip, skinny_gemm.hip
-torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
+torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 bool one_row_fits(long S, long K);
 bool float_few_rows_fits(long N, long K);
@@ -16,7 +16,10 @@ torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
 bool large_takes(long N, long K);
 torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target);
 
-enum { WHOLE = 0, PARTS = 1, SILU = 2, FLOAT = 3 };
+// STEADY beside a form: what the rows of prompts go through on their way into an 8-bit cache. They
+// are most of its bytes, and sums in another order let one in 20 to 50 of those round the other
+// way, so such products stay where, and in the parts of K in which, they were first made.
+enum { WHOLE = 0, PARTS = 1, SILU = 2, FLOAT = 3, STEADY = 4 };
 
 static long megabytes(long N, long K) { return (N * K * 2) >> 20; }
 
@@ -41,13 +44,13 @@ static long small_megabytes() {
 // with K long enough to pay for adding them, few outputs with longer ones (96 rows: 4608 x 4096 16
 // and 22, 2048 x 4096 13.3 and 12.8, 2048 x 8192 15 and 21, 1024 x 8192 15.2 and 15.0, 1024 x 14336 17 and 25, 8192 x 28672
 // 123 and 124; but 4608 x 2048 13.1 and 13.5, 128 rows 15.9 and 15.0; 10240 x 8192 57 and 55).
-static bool few_rows_win(long M, long N, long K, bool parts) {
+static bool few_rows_win(long M, long N, long K, bool parts, bool steady) {
   if (M > 64)
-    return N <= (parts ? 12288 : 8192) &&
+    return N <= (parts && !steady ? 12288 : 8192) &&
            (parts || K >= 14336 || (K >= 3072 && N >= (K < 8192 ? 3072 : 2048)));
   const long size = megabytes(N, K);
   const long most = M == 1 ? 6144 : !parts ? 7168 : M <= 32 ? 8192 : 10240;
-  return size <= small_megabytes() || (K > 4096 && N <= most) ||
+  return size <= small_megabytes() || (K > 4096 && N <= most && !steady) ||
          (M <= 32 && (K < 4096 || (K == 4096 && size <= 512)));
 }
 
@@ -124,7 +127,9 @@ static bool many_rows_win(long M, long N, long K, bool silu) {
 // x @ w^T in ``form``, or nothing: the library's product serves better or is followed by
 // autograd, a transform or a trace, or the kernels have no form for it.
 c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Tensor& w,
-                                         long form) {
+                                         long asked) {
+  const long form = asked & ~STEADY;
+  const bool steady = asked & STEADY;
   if (!plain(x) || !plain(w) || x.dim() != 2 || w.dim() != 2 || !x.is_cuda() ||
       x.device() != w.device() || x.dtype() != torch::kBFloat16 ||
       w.dtype() != torch::kBFloat16)
@@ -146,13 +151,13 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
   }
   if (form == FLOAT) {
     // (of more than 64 rows none that few_rows_win names has its K whole)
-    if (M > 64 || !few_rows_win(M, N, K, false) || !float_few_rows_fits(N, K)) return {};
+    if (M > 64 || !few_rows_win(M, N, K, false, steady) || !float_few_rows_fits(N, K)) return {};
     return float_few_rows(x, w);
   }
   if (M <= 128) {
-    if (form == PARTS && few_rows_win(M, N, K, true))
-      return linear_few_rows(x, w, true);
-    if (few_rows_win(M, N, K, false)) return linear_few_rows(x, w, false);
+    if (form == PARTS && few_rows_win(M, N, K, true, steady))
+      return linear_few_rows(x, w, true, steady);
+    if (few_rows_win(M, N, K, false, steady)) return linear_few_rows(x, w, false, steady);
   } else if (large_takes(N, K) && many_rows_win(M, N, K, false)) {
     return many_rows(x, w, false);
   }
@@ -182,5 +187,5 @@ bool norms_row(const torch::Tensor& x, const torch::Tensor& res, const torch::Te
   if (!one_row_fits(x.size(0), K) || res.dim() != 2 || res.size(0) != 1 || res.size(1) != K ||
       weight.numel() != K || w.dim() != 2 || w.size(1) != K || w.size(0) == 0 || w.size(0) % 16)
     return false;
-  return silu ? silu_few_rows_win(1, w.size(0) / 2, K) : few_rows_win(1, w.size(0), K, true);
+  return silu ? silu_few_rows_win(1, w.size(0) / 2, K) : few_rows_win(1, w.size(0), K, true, false);
 }

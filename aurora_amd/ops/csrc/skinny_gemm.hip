@@ -344,11 +344,11 @@ torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target) {
 
 // defined in few_rows.hip
 torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width);
-torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw);
+torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 
 torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w) {
   TORCH_CHECK(x.dim() == 2 && x.size(0) <= 64, "skinny_gemm is for M <= 64");
-  return linear_few_rows(x, w, false);
+  return linear_few_rows(x, w, false, false);
 }
 
 torch::Tensor skinny_gemm2_ex(torch::Tensor x, torch::Tensor w, long s_target) {

@@ -117,11 +117,12 @@ class MergedColumnParallelLinear(ColumnParallelLinear):
         self.intermediate_local = intermediate // pdist.tp_world_size()
 
 
-def column_parts(m: nn.Module, x: torch.Tensor) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+def column_parts(m: nn.Module, x: torch.Tensor,
+                 steady: bool = False) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
     """``m(x)`` of a column-parallel layer as a product possibly in parts
     (``ops.linear_parts``) and the bias still to be added."""
     if is_plain(m, ColumnParallelLinear) and not m.gather_output:
-        return ops.linear_parts(x, m.weight), m.bias
+        return ops.linear_parts(x, m.weight, steady), m.bias
     return m(x), None
 
 
@@ -132,15 +133,17 @@ def column_weight(m: nn.Module, bias: bool) -> Optional[torch.Tensor]:
                         and (bias or m.bias is None)) else None
 
 
-def row_parts(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
+def row_parts(m: nn.Module, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """``m(x)`` of a row-parallel layer, possibly in parts where nothing is reduced."""
     if is_plain(m, RowParallelLinear) and pdist.tp_world_size() == 1:
-        return ops.linear_parts(x, m.weight)
+        return ops.linear_parts(x, m.weight, steady)
+    if is_plain(m, RowParallelLinear) and steady:
+        return pdist.tp_all_reduce(ops.linear(x, m.weight, True))
     return m(x)
 
 
-def column_silu_mul(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
+def column_silu_mul(m: nn.Module, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """``silu_mul(m(x))`` of a merged gate and up layer, in one kernel where that is faster."""
     if is_plain(m, ColumnParallelLinear) and m.bias is None and not m.gather_output:
-        return ops.linear_silu_mul(x, m.weight)
+        return ops.linear_silu_mul(x, m.weight, steady)
     return ops.silu_mul(m(x))

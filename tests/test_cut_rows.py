@@ -50,3 +50,24 @@ def test_chosen_cuts(m, n, k):
     _check(ops.linear(x, w), want)
     if n <= 8192 and k > 4096:
         assert y.dim() == 3
+
+
+@pytest.mark.parametrize("m", [2, 33, 65, 128])
+@pytest.mark.parametrize("n,k,parts", [(6144, 4096, 2), (4096, 14336, 4), (4608, 3584, 3),
+                                       (2048, 2048, 8), (64, 8192, 16)])
+def test_steady(m, n, k, parts):
+    """What fills an 8-bit cache: K in the parts that 64 rows of weights want."""
+    x, w = _inputs(m, n, k)
+    y = ops.linear_parts(x, w, True)
+    assert torch.equal(y, ops._hip.few_rows(x, w, True, parts, 64))
+    whole = ops._hip.own_product(x, w, 4)
+    if whole is not None:
+        cut = k * (2 if m > 32 else 1) >= 4096
+        assert torch.equal(whole, ops._hip.few_rows(x, w, False, parts if cut else 1, 64))
+
+
+def test_steady_leaves_the_library_its_own():
+    for m, n, k in ((16, 3584, 18944), (96, 9216, 4096)):
+        x, w = _inputs(m, n, k)
+        assert ops._hip.own_product(x, w, 5) is None and ops._hip.own_product(x, w, 1) is not None
+        assert torch.equal(ops.linear_parts(x, w, True), torch.nn.functional.linear(x, w))

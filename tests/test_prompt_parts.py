@@ -73,3 +73,38 @@ def test_cut_or_whole():
         torch.arange(41, dtype=torch.int32, device="cuda") * 64, ctx.repeat(40), 128 ** -0.5)
     assert torch.equal(many[:64], many[-64:])
     assert (one.float() - many[:64].float()).norm() <= 2 ** -7 * one.float().norm()
+
+
+def test_eight_bits_stay_whole():
+    """What an 8-bit cache's next rows are made of does not hang on other sequences."""
+    q, kc, vc, bt, cu, ctx = _case([64], [6000], 32, 8, 128, torch.float8_e4m3fn)
+    one = ops.attention_prefill_paged(q, kc, vc, bt, cu, ctx, 128 ** -0.5)
+    many = ops.attention_prefill_paged(
+        q.repeat(40, 1, 1), kc, vc, bt.repeat(40, 1),
+        torch.arange(41, dtype=torch.int32, device="cuda") * 64, ctx.repeat(40), 128 ** -0.5)
+    assert torch.equal(one, many[:64]) and torch.equal(one, many[-64:])
+
+
+@pytest.mark.parametrize("mode,eight,steady", [("prefill", True, True), ("mixed", True, True),
+                                               ("prefill", False, False), ("decode", True, False)])
+def test_prompts_into_eight_bits(mode, eight, steady, monkeypatch):
+    """A step's products keep their order of sums where its prompts fill an 8-bit cache."""
+    from aurora_amd.models.config import ModelSpec
+    from aurora_amd.models.llama import AttnMetadata, LlamaForCausalLM
+    spec = ModelSpec(name="t", vocab_size=64, hidden_size=256, n_layers=2, n_heads=4,
+                     n_kv_heads=2, head_dim=64, intermediate_size=512)
+    model = LlamaForCausalLM(spec, device="cuda")
+    model.init_random(0)
+    dtype = torch.float8_e4m3fn if eight else torch.bfloat16
+    caches = [tuple(torch.zeros(3, 2, P, 64, device="cuda").to(dtype) for _ in "kv")] * 2
+    ints = [torch.tensor(v, dtype=torch.int32, device="cuda")
+            for v in ([0, 1, 2], [P, P + 1, P + 2], [[1, 0]], [3], [0, 3])]
+    if mode == "decode":
+        ints[2], ints[3] = ints[2].repeat(3, 1), ints[3].repeat(3)
+    meta = AttnMetadata(mode, *ints[:4], ints[4], num_prefill_tokens=3,
+                        dec_block_tables=ints[2][:0], dec_context_lens=ints[3][:0])
+    seen, real = [], ops.linear_parts
+    monkeypatch.setattr(ops, "linear_parts",
+                        lambda x, w, s=False: seen.append(s) or real(x, w, s))
+    model(torch.tensor([1, 2, 3], device="cuda"), caches, meta)
+    assert seen == [steady] * 6
