@@ -27,10 +27,11 @@ from .config import ModelSpec, get_spec
 TURNED_TOKENS = 1024
 
 
-def _product(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
-    """``m(x)``, through the framework's products where nobody watches or replaced ``m``."""
+def _product(m: nn.Module, x: torch.Tensor, in_parts: bool = False) -> torch.Tensor:
+    """``m(x)``, through the framework's products where nobody watches or replaced ``m``; with
+    ``in_parts`` possibly in parts (``ops.linear_parts``)."""
     if is_plain(m, nn.Linear) and m.bias is None:
-        return ops.linear(x, m.weight)
+        return (ops.linear_parts if in_parts else ops.linear)(x, m.weight)
     return m(x)
 
 
@@ -55,10 +56,11 @@ class EncoderLayer(nn.Module):
         x, delta = self.step(x, None, cos_sin, positions, cu)
         return x + delta
 
-    def step(self, x, delta, cos_sin, positions, cu, in_order=False):
+    def step(self, x, delta, cos_sin, positions, cu, in_order=False, in_parts=False):
         """The stream ``x``, to which ``delta`` (the layer before's result) is still to be
         added -> the stream and this layer's. ``in_order``: positions are the tokens' places
-        in their texts."""
+        in their texts; with ``in_parts`` the result may be in parts, as ``delta`` may be, which
+        ``rmsnorm_residual`` adds up."""
         T = x.shape[0]
         if delta is None:
             h = ops.rmsnorm(x, self.norm1, self.eps)
@@ -74,12 +76,13 @@ class EncoderLayer(nn.Module):
             else:  # what somebody else made may be kept by them
                 q, k = ops.rope_apply(q.clone(), k.clone(), positions, cos_sin)
             o = ops.attention_prefill(q, k, v, cu, self.scale, causal=False)
-        h, x = ops.rmsnorm_residual(_product(self.o, o.reshape(T, -1)), x, self.norm2, self.eps)
+        h, x = ops.rmsnorm_residual(_product(self.o, o.reshape(T, -1), True), x, self.norm2,
+                                    self.eps)
         if is_plain(self.gate_up, nn.Linear) and self.gate_up.bias is None:
             act = ops.linear_silu_mul(h, self.gate_up.weight)
         else:
             act = ops.silu_mul(self.gate_up(h))
-        return x, _product(self.down, act)
+        return x, _product(self.down, act, in_parts)
 
 
 class SentenceEncoder(nn.Module):
@@ -131,9 +134,10 @@ class SentenceEncoder(nn.Module):
         in_order = maxp <= TURNED_TOKENS or max(map(len, batches), default=0) <= TURNED_TOKENS
         x = self.embed(ids)
         delta = None
-        for layer in self.layers:
-            if is_plain(layer, EncoderLayer):
-                x, delta = layer.step(x, delta, self.cos_sin, pos_t, cu_t, in_order)
+        plain = [is_plain(layer, EncoderLayer) for layer in self.layers] + [True]
+        for i, layer in enumerate(self.layers):
+            if plain[i]:
+                x, delta = layer.step(x, delta, self.cos_sin, pos_t, cu_t, in_order, plain[i + 1])
             else:  # somebody watches it or has replaced it
                 x, delta = x if delta is None else x + delta, None
                 x = layer(x, self.cos_sin, pos_t, cu_t)

@@ -28,7 +28,8 @@ torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
 c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Tensor& w,
                                          long form);
 torch::Tensor many_rows(torch::Tensor x, torch::Tensor w, bool silu);
-torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width);
+torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width,
+                       long rows);
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor weight, double eps,
@@ -207,7 +208,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("own_product", &own_product, "a product by the own kernels where they win");
   m.def("many_rows", &many_rows, "products of many rows, with silu(gate) * up");
   m.def("few_rows", &few_rows, "products of at most 128 rows, K in parts", py::arg("x"),
-        py::arg("w"), py::arg("raw"), py::arg("parts"), py::arg("width") = 64);
+        py::arg("w"), py::arg("raw"), py::arg("parts"), py::arg("width") = 64,
+        py::arg("rows") = 0);
   m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows", py::arg("x"),
         py::arg("w"), py::arg("raw"), py::arg("steady") = false);
   m.def("one_row_product", &one_row_product, "a norm and the product of its one row");

@@ -29,6 +29,9 @@
 // workgroups beside those of the norm before it, brings nothing (4096 x 14336, norm, 28672 x
 // 4096, 23 rows: 73.5 us, and with 4 to 29 MB asked for 73.2 to 77): what comes from
 // memory and what lies in the cache before it take the same way.
+//
+// Up to 1000 rows come in blocks of 64, 96 or 128 (``block_cut``), bound by the stages of the
+// workgroups' tiles: 4096 x 4096, 140 and 512 rows, 18 and 28 us, the library's product 22 and 29.
 #include "flash_tiles.h"
 #include <torch/extension.h>
 #include <c10/core/DeviceGuard.h>
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(WN * 4) void few_rows_kernel(
   const int at = lane & 15, g = lane >> 4;
   const int r0 = wave % ACROSS * RT * 16, x0 = wave / ACROSS * MW * 16;
   const int n0 = blockIdx.x * (SILU ? WN / 2 : WN);
-  const int k0 = blockIdx.y * (ROUTER ? FEW_K : span), m0 = ROUTER ? blockIdx.z * 16 * MT : 0;
+  const int k0 = blockIdx.y * (ROUTER ? FEW_K : span), m0 = blockIdx.z * 16 * MT;
   const int stride = ROUTER ? gridDim.y * FEW_K : FEW_K;
   const int steps = ROUTER ? max(K - k0 + stride - 1, 0) / stride
                            : (min(K, k0 + span) - k0) / FEW_K;
@@ -391,7 +394,7 @@ static long parts_of(long N, long K) {
 // 128 in 8 32.2; 5120 x 5120, 64 rows, 19.4 and 19.3.
 struct Cut {
   int width;
-  long parts;
+  long parts, rows = 0;
 };
 static Cut cut_of(long M, long N, long K) {
   const long steps = K / FEW_K, rows = M <= 32 ? 32 : (M + 31) / 32 * 32;
@@ -416,13 +419,13 @@ static Cut cut_of(long M, long N, long K) {
   return best;
 }
 
-static void check(const torch::Tensor& x, const torch::Tensor& w) {
+static void check(const torch::Tensor& x, const torch::Tensor& w, long most = FEW_MOST) {
   TORCH_CHECK(x.is_cuda() && w.is_cuda() && x.dtype() == torch::kBFloat16 &&
                   w.dtype() == torch::kBFloat16 && w.is_contiguous(),
               "bf16 GPU only, contiguous weights");
-  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && x.size(0) <= FEW_MOST &&
+  TORCH_CHECK(x.dim() == 2 && w.dim() == 2 && x.size(1) == w.size(1) && x.size(0) <= most &&
                   x.size(1) % FEW_K == 0,
-              "at most ", FEW_MOST, " rows and K a multiple of ", FEW_K);
+              "at most ", most, " rows and K a multiple of ", FEW_K);
 }
 
 // x as 16-byte loads can read its rows, which may be strided (a part of a joint projection,
@@ -441,7 +444,8 @@ static void launch(const torch::Tensor& x, const torch::Tensor& w, unsigned shor
   // stages: two workgroups of 64 rows on a CU, one of the wide forms
   constexpr int tile = SILU ? WN / 2 : WN, loads = (WN * 8 + MT * 128 + WN * 4 - 1) / (WN * 4);
   constexpr int NS = (WN == 64 ? 80 : 160) * 1024 / (loads * WN * 64);
-  hipLaunchKernelGGL((few_rows_kernel<WN, MT, NS, SILU>), dim3((N + tile - 1) / tile, S),
+  const long blocks = (x.size(0) + 16 * MT - 1) / (16 * MT);
+  hipLaunchKernelGGL((few_rows_kernel<WN, MT, NS, SILU>), dim3((N + tile - 1) / tile, S, blocks),
                      dim3(WN * 4), 0, CUR_STREAM, (const unsigned short*)x.data_ptr(),
                      (const unsigned short*)w.data_ptr(), out, part, (int)x.size(0), (int)N,
                      (int)x.size(1), (int)span, x.size(0) > 1 ? x.stride(0) : 0L);
@@ -449,8 +453,9 @@ static void launch(const torch::Tensor& x, const torch::Tensor& w, unsigned shor
 }
 
 // [M, N] in bf16, or with ``raw`` where K is cut [S, M, N] in fp32, S terms to be added.
-static torch::Tensor cut_rows(torch::Tensor x, torch::Tensor w, bool raw, Cut cut) {
-  check(x, w);
+static torch::Tensor cut_rows(torch::Tensor x, torch::Tensor w, bool raw, Cut cut,
+                              long most = FEW_MOST) {
+  check(x, w, most);
   x = readable(x);
   const long M = x.size(0), K = x.size(1), N = w.size(0);
   torch::Tensor out, part;
@@ -468,18 +473,58 @@ static torch::Tensor cut_rows(torch::Tensor x, torch::Tensor w, bool raw, Cut cu
     else if (cut.width == 96) launch<96, mt, false>(x, w, op, pp, N, S, span);
     else launch<128, mt, false>(x, w, op, pp, N, S, span);
   };
-  if (M <= 32) rows(std::integral_constant<int, 2>{});
-  else if (M <= 64) rows(std::integral_constant<int, 4>{});
-  else if (M <= 96) rows(std::integral_constant<int, 6>{});
+  const long high = cut.rows ? cut.rows : M;
+  if (high <= 32) rows(std::integral_constant<int, 2>{});
+  else if (high <= 64) rows(std::integral_constant<int, 4>{});
+  else if (high <= 96) rows(std::integral_constant<int, 6>{});
   else rows(std::integral_constant<int, 8>{});
   if (S == 1) return out;
   return raw ? part : add_parts(part);
 }
 
 // The same in a given number of parts and rows of W a workgroup.
-torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width) {
+torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width,
+                       long rows) {
   TORCH_CHECK(width == 64 || width == 96 || width == 128, "64, 96 or 128 rows of w a workgroup");
-  return cut_rows(x, w, raw, Cut{(int)width, parts});
+  return cut_rows(x, w, raw, Cut{(int)width, parts, rows}, rows ? 1 << 16 : FEW_MOST);
+}
+
+// How some hundred rows are cut: into blocks of ``rows``, each of which reads W once more (from
+// the L2 where it is small), tiles of ``width`` and K's parts. A form's time is that of its
+// stages of 64 of K, which depends on nothing but its rows and width while a CU has one
+// workgroup (two of 64 wide share it), and what it takes to bring the parts to their reader.
+// Of 88 sizes from 140 to 1000 rows and 768 x 768 to 4096 x 14336 the form so chosen took 3%
+// longer than the best.
+static Cut block_cut(long M, long N, long K, bool raw) {
+  static const struct {
+    long rows;
+    int width;
+    float stage;  // us
+  } forms[] = {{64, 64, .245f}, {96, 64, .30f}, {64, 128, .366f}, {96, 128, .466f},
+               {128, 128, .556f}};
+  Cut best = {64, 1, 64};
+  float low = 0;
+  const long steps = K / FEW_K;
+  for (const auto& f : forms) {
+    const long tiles = (N + f.width - 1) / f.width * ((M + f.rows - 1) / f.rows);
+    const long most = std::max(1L, std::min({256 / tiles, steps / 2, 16L}));
+    for (long parts : {1L, most}) {
+      const long per = (steps + parts - 1) / parts;
+      if ((steps + per - 1) / per != parts) continue;
+      const long each = tiles * parts;
+      const float rounds =
+          f.width == 64 ? std::max(1.f, each / 256.f) : (float)((each + 255) / 256);
+      const float time = per * f.stage * rounds +
+                         (parts > 1 ? parts * M * N * 2e-6f + (raw ? 0.f : 2.5f) : 0.f);
+      if (low == 0 || time < low) low = time, best = {f.width, parts, f.rows};
+    }
+  }
+  return best;
+}
+
+// linear_few_rows of more rows
+torch::Tensor block_rows(torch::Tensor x, torch::Tensor w, bool raw) {
+  return cut_rows(x, w, raw, block_cut(x.size(0), w.size(0), x.size(1), raw), 1 << 16);
 }
 
 // A router's logits in 16 parts [16, M, N] in fp32 that hold what the 16 waves of
@@ -509,7 +554,8 @@ torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool s
   const bool cut = raw || (x.size(1) * (x.size(0) > 32 ? 2 : 1) >= 4096 &&
                            parts_of(w.size(0), x.size(1)) > 1);
   const long M = x.size(0), N = w.size(0), K = x.size(1);
-  return cut_rows(x, w, raw, !cut ? Cut{64, 1} : steady ? Cut{64, parts_of(N, K)} : cut_of(M, N, K));
+  return cut_rows(x, w, raw,
+                  !cut ? Cut{64, 1} : steady ? Cut{64, parts_of(N, K)} : cut_of(M, N, K));
 }
 
 // linear_few_rows's result in float32, where K is not cut, without a kernel to convert it: 1 row

@@ -9,6 +9,7 @@
 // defined in few_rows.hip, moe.hip, skinny_gemm.hip
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
+torch::Tensor block_rows(torch::Tensor x, torch::Tensor w, bool raw);
 bool one_row_fits(long S, long K);
 bool float_few_rows_fits(long N, long K);
 torch::Tensor float_few_rows(torch::Tensor x, torch::Tensor w);
@@ -124,6 +125,35 @@ static bool many_rows_win(long M, long N, long K, bool silu) {
   return tiles >= (K <= 256 ? 40 : K <= 512 ? 24 : K <= 1024 ? 120 : 144);
 }
 
+// AURORA_SKINNY3=0 leaves 192 to 256 rows to the library.
+static bool left_to_library(long M) {
+  if (M < 192 || M > 256) return false;
+  const char* off = std::getenv("AURORA_SKINNY3");
+  return off && !std::strcmp(off, "0");
+}
+
+// 129 to 1000 rows: where the kernel of few rows, in blocks of rows, beats the library's product.
+// us with cold weights, the library's and ours, whole and in parts with the norm that reads them:
+//   N x K         rows: 140            256            300            512            1000
+//   4096 x 4096     22 18, 26 18   23 22, 27 26   26 24, 30 28   29 28, 34 33   40 41, 47 47
+//   6144 x 4096     40 25, 45 30   40 28, 45 33   29 28, 35 34   36 40, 43 46   52 74, 61 83
+//   4096 x 14336    57 41, 60 40   63 49, 65 50   76 63, 78 63   91 79, 93 80   131 131, 138 138
+//   2048 x 2048     9.1 10, 12 11  9.8 11, 13 12  11 11, 14 13   11 11, 15 15   16 14, 20 18
+//   2048 x 8192     26 18, 29 18   27 22, 30 23   33 25, 36 26   34 32, 37 32   47 48, 53 48
+//   768 x 768       5.8 6.3, 9 8   5.8 6.3, 10 10 5.8 6.3, 9 9   6.7 6.4, 11 11 8.1 6.6, 12 11
+//   768 x 3072      9 10, 12 11    10 11, 13 12   10 12, 13 12   13 13, 16 14   15 17, 19 21
+//   2304 x 768      7 7, 11 10     8 7, 12 11     9 7, 12 11     9 9, 14 13     13 10, 18 15
+// and a call of the library's takes the host 11 us more, which small prompts and texts wait for
+// (a text of 200 tokens 1197 us and 612). The line is work for a quarter of the chip, in tiles of
+// 128 x 256: beyond it both come to the same by themselves (with the norm 520 rows of 4096 x 4096
+// 39 and 36, of 4096 x 14336 111 and 111, 768 of 3584 x 14336 113 and 127) and four layers of
+// 4096, 520 rows, took 1647 and 1746 us. Within it ours falls back by up to 2 us (980 rows of 1024
+// x 4096 22 and 24, 780 of 2048 x 4096 30 and 32).
+static bool block_rows_win(long M, long N, long K) {
+  if (left_to_library(M)) return false;
+  return M <= 1000 && N >= 512 && K > 512 && (M + 127) / 128 * N <= 64 * 256;
+}
+
 // x @ w^T in ``form``, or nothing: the library's product serves better or is followed by
 // autograd, a transform or a trace, or the kernels have no form for it.
 c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Tensor& w,
@@ -160,14 +190,12 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
     if (few_rows_win(M, N, K, false, steady)) return linear_few_rows(x, w, false, steady);
   } else if (large_takes(N, K) && many_rows_win(M, N, K, false)) {
     return many_rows(x, w, false);
-  }
-  // Cold weights: W streamed once past up to 256 rows, ours and the library's, 192 and 256
-  // rows: 6144 x 4096 33 and 34, 38 and 42; 4608 x 3584 30 and 30, 32 and 36. Fewer rows, more
-  // outputs and shorter K are the library's (160 rows 32 and 29, 29 and 25; 192 of 8192 x 4096
-  // 38 and 36, 6144 x 2048 26 and 22). AURORA_SKINNY3=0 leaves them all to it.
-  if (M >= 192 && M <= 256 && N % 64 == 0 && N > 4096 && N <= 6144 && K > 2048 && K <= 4096) {
-    const char* off = std::getenv("AURORA_SKINNY3");
-    if (!off || std::strcmp(off, "0")) return skinny_gemm3_ex(x.contiguous(), w, 384);
+  } else if (steady) {
+    if (M >= 192 && M <= 256 && N % 64 == 0 && N > 4096 && N <= 6144 && K > 2048 && K <= 4096 &&
+        !left_to_library(M))
+      return skinny_gemm3_ex(x.contiguous(), w, 384);
+  } else if (block_rows_win(M, N, K)) {
+    return block_rows(x, w, form == PARTS);
   }
   return {};
 }

@@ -343,7 +343,8 @@ torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target) {
 }
 
 // defined in few_rows.hip
-torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width);
+torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, long width,
+                       long rows);
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 
 torch::Tensor skinny_gemm(torch::Tensor x, torch::Tensor w) {
@@ -357,5 +358,5 @@ torch::Tensor skinny_gemm2_ex(torch::Tensor x, torch::Tensor w, long s_target) {
   TORCH_CHECK(x.size(1) % 128 == 0, "K must be a multiple of 128");
   if (x.size(0) > 128) return skinny_gemm3_ex(x, w, s_target);
   const long tiles = (w.size(0) + 63) / 64, target = s_target > 0 ? s_target : 768;
-  return few_rows(x, w, false, std::max(1L, std::min(16L, target / std::max(tiles, 1L))), 64);
+  return few_rows(x, w, false, std::max(1L, std::min(16L, target / std::max(tiles, 1L))), 64, 0);
 }

@@ -52,6 +52,34 @@ def test_chosen_cuts(m, n, k):
         assert y.dim() == 3
 
 
+@pytest.mark.parametrize("m", [129, 192, 193, 300, 1000])
+@pytest.mark.parametrize("n,k", [(512, 576), (768, 3072), (2048, 2048), (2120, 4160)])
+def test_blocks_of_rows(m, n, k):
+    """129 to 1000 rows: every form, whole and in parts, rows past a block's end."""
+    x, w = _inputs(m, n, k)
+    want = x.double() @ w.double().t()
+    for rows in (64, 96, 128):
+        for width, parts in ((64, 1), (64, 3), (128, 1), (128, 2)):
+            _check(ops._hip.few_rows(x, w, False, parts, width, rows), want)
+            raw = ops._hip.few_rows(x, w, True, parts, width, rows)
+            _check((raw.sum(0) if raw.dim() == 3 else raw).bfloat16(), want)
+    _check(ops.linear(x, w), want)
+    y = ops.linear_parts(x, w)
+    _check((y.sum(0) if y.dim() == 3 else y).bfloat16(), want)
+
+
+@pytest.mark.parametrize("m,n,k,own", [
+    (512, 4096, 4096, True), (1000, 2048, 576, True), (1000, 512, 576, True),
+    (513, 4096, 640, False), (1001, 2048, 576, False), (300, 504, 1024, False),
+    (300, 1024, 512, False)])
+def test_line_to_the_library(m, n, k, own):
+    x, w = _inputs(m, n, k)
+    got = ops._hip.own_product(x, w, 0)
+    assert (got is not None) == own
+    strided = torch.cat([x, x], 1)[:, :k]  # rows apart
+    _check(ops.linear(strided, w), x.double() @ w.double().t())
+
+
 @pytest.mark.parametrize("m", [2, 33, 65, 128])
 @pytest.mark.parametrize("n,k,parts", [(6144, 4096, 2), (4096, 14336, 4), (4608, 3584, 3),
                                        (2048, 2048, 8), (64, 8192, 16)])
