@@ -69,6 +69,8 @@ class AttnMetadata:
     # decode: every row is the last token of a sequence that no other row belongs to, at the
     # position before its context's end and in the slot that its table names for it
     last_tokens: bool = False
+    # prompts that fill an 8-bit cache: the products' sums keep their order (``ops.linear``)
+    steady: bool = False
 
     def segments(self, T: int) -> List[ops.Segment]:
         """The step's prompt portions and its single-token rows, each with its
@@ -93,12 +95,6 @@ class AttnMetadata:
                 starts=self.positions[Tp:],
                 state_slots=self.dec_state_slots if mixed else self.state_slots))
         return out
-
-
-def _steady(kv_cache, meta) -> bool:
-    """Whether the products' sums keep their order (``ops.linear``): in prompts that fill an
-    8-bit cache, not where each sequence adds one row to its many."""
-    return meta.mode != "decode" and kv_cache[0].element_size() == 1
 
 
 class LlamaAttention(nn.Module):
@@ -128,12 +124,12 @@ class LlamaAttention(nn.Module):
     def parts(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
         """As ``forward``, possibly in parts (``ops.linear_parts``)."""
         return row_parts(self.o_proj, self._heads(x, cos_sin, kv_cache, meta),
-                         _steady(kv_cache, meta))
+                         getattr(meta, "steady", False))
 
     def _heads(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
         """The heads' results side by side, [T, heads * width]."""
         T = x.shape[0]
-        qkv, bias = column_parts(self.qkv_proj, x, _steady(kv_cache, meta))
+        qkv, bias = column_parts(self.qkv_proj, x, getattr(meta, "steady", False))
         k_cache, v_cache = kv_cache
         if meta.mode == "decode" and getattr(meta, "last_tokens", False):
             o = ops.fresh_attention_decode(
@@ -380,7 +376,7 @@ class LlamaDecoderLayer(nn.Module):
                                      self._reader("mlp", a) if in_parts else None, True)
         if not in_parts or not is_plain(self.mlp, LlamaMLP):
             return self.mlp(h), residual
-        if _steady(kv_cache, meta):
+        if getattr(meta, "steady", False):
             return self.mlp.parts(h, True), residual
         return self.mlp.parts(h), residual
 
@@ -448,6 +444,9 @@ class LlamaForCausalLM(nn.Module):
                 meta = copy(meta)
                 meta.marks = ops.decode_marks(
                     self.spec.n_heads // pdist.tp_world_size(), kv_caches[0][0], tables)
+            if meta.mode != "decode" and kv_caches and kv_caches[0][0].element_size() == 1:
+                meta = copy(meta)
+                meta.steady = True
         # layers that somebody watches or has replaced are called and get no parts
         plain = [is_plain(layer, LlamaDecoderLayer) for layer in self.layers] + [True]
         for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):
