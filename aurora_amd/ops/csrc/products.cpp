@@ -132,7 +132,7 @@ static bool left_to_library(long M) {
   return off && !std::strcmp(off, "0");
 }
 
-// 129 to 1000 rows: where the kernel of few rows, in blocks of rows, beats the library's product.
+// 65 to 1000 rows: where the kernel of few rows, in blocks of rows, beats the library's product.
 // us with cold weights, the library's and ours, whole and in parts with the norm that reads them:
 //   N x K         rows: 140            256            300            512            1000
 //   4096 x 4096     22 18, 26 18   23 22, 27 26   26 24, 30 28   29 28, 34 33   40 41, 47 47
@@ -149,9 +149,19 @@ static bool left_to_library(long M) {
 // 39 and 36, of 4096 x 14336 111 and 111, 768 of 3584 x 14336 113 and 127) and four layers of
 // 4096, 520 rows, took 1647 and 1746 us. Within it ours falls back by up to 2 us (980 rows of 1024
 // x 4096 22 and 24, 780 of 2048 x 4096 30 and 32).
+// Short K and few rows, whole, 65, 100, 128, 180 and 300 rows, the library's and ours:
+//   256 x 256     8.2 4.4   9.0 4.4   8.8 4.4    11 4.4   5.1 4.5
+//   4096 x 256    5.6 4.5   5.5 4.5   6.2 4.6   5.9 4.7   7.5 5.2
+//   1024 x 512    5.9 5.3   6.0 5.3   7.5 5.3   6.0 5.3   6.8 5.4
+//   3072 x 1024   9.2 7.7, 9.7 7.7, 10 7.8 (65, 100 and 128 rows; 1024 x 1024 6.2 7.3)
+//   6144 x 2048    14 12     14 12     15 13 (2048 x 2048 8.4 8.4, 8.5 9.2, 8.4 9.4)
+//   2816 x 1408   8.5 9.6   8.7 9.5    12 9.6, the one found where the library is ahead
 static bool block_rows_win(long M, long N, long K) {
   if (left_to_library(M)) return false;
-  return M <= 1000 && N >= 512 && K > 512 && (M + 127) / 128 * N <= 64 * 256;
+  if (M <= 128) return N <= 8192 && (K <= 512 ? N >= 64 : K <= 2048 && N >= 2816);
+  const long work = (M + 127) / 128 * N / 256;  // (a little more, many_rows takes)
+  if (K <= 512) return M <= 1000 && N >= 64 && work <= (K <= 256 ? 40 : 16);
+  return M <= 1000 && N >= 512 && (M + 127) / 128 * N <= 64 * 256;
 }
 
 // x @ w^T in ``form``, or nothing: the library's product serves better or is followed by
@@ -188,6 +198,7 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
     if (form == PARTS && few_rows_win(M, N, K, true, steady))
       return linear_few_rows(x, w, true, steady);
     if (few_rows_win(M, N, K, false, steady)) return linear_few_rows(x, w, false, steady);
+    if (!steady && M > 64 && block_rows_win(M, N, K)) return block_rows(x, w, form == PARTS);
   } else if (large_takes(N, K) && many_rows_win(M, N, K, false)) {
     return many_rows(x, w, false);
   } else if (steady) {

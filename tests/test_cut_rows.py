@@ -52,10 +52,11 @@ def test_chosen_cuts(m, n, k):
         assert y.dim() == 3
 
 
-@pytest.mark.parametrize("m", [129, 192, 193, 300, 1000])
-@pytest.mark.parametrize("n,k", [(512, 576), (768, 3072), (2048, 2048), (2120, 4160)])
+@pytest.mark.parametrize("m", [65, 97, 129, 192, 193, 300, 1000])
+@pytest.mark.parametrize("n,k", [(512, 576), (768, 3072), (2048, 2048), (2120, 4160), (72, 64),
+                                 (3400, 1024)])
 def test_blocks_of_rows(m, n, k):
-    """129 to 1000 rows: every form, whole and in parts, rows past a block's end."""
+    """65 to 1000 rows: every form, whole and in parts, rows past a block's end."""
     x, w = _inputs(m, n, k)
     want = x.double() @ w.double().t()
     for rows in (64, 96, 128):
@@ -71,7 +72,9 @@ def test_blocks_of_rows(m, n, k):
 @pytest.mark.parametrize("m,n,k,own", [
     (512, 4096, 4096, True), (1000, 2048, 576, True), (1000, 512, 576, True),
     (513, 4096, 640, False), (1001, 2048, 576, False), (300, 504, 1024, False),
-    (300, 1024, 512, False)])
+    (300, 1024, 512, True), (300, 1456, 512, False), (300, 2824, 256, True), (128, 8192, 64, True),
+    (129, 64, 320, True), (128, 56, 256, False), (65, 2816, 2048, True), (65, 2816, 2112, False),
+    (100, 2808, 576, False), (128, 8192, 1024, True), (64, 64, 64, True)])
 def test_line_to_the_library(m, n, k, own):
     x, w = _inputs(m, n, k)
     got = ops._hip.own_product(x, w, 0)
