@@ -44,7 +44,8 @@ static long small_megabytes() {
 // 35, 10240 x 8192 44 and 58, 12288 x 4096 32 and 38; but 16384 x 4096 44 and 44), or up to 8192
 // with K long enough to pay for adding them, few outputs with longer ones (96 rows: 4608 x 4096 16
 // and 22, 2048 x 4096 13.3 and 12.8, 2048 x 8192 15 and 21, 1024 x 8192 15.2 and 15.0, 1024 x 14336
-// 17 and 25, 8192 x 28672 123 and 124; but 4608 x 2048 13.1 and 13.5, 128 rows 15.9 and 15.0; 10240 x 8192 57 and 55).
+// 17 and 25, 8192 x 28672 123 and 124; but 4608 x 2048 13.1 and 13.5, 128 rows 15.9 and 15.0; 10240
+// x 8192 57 and 55).
 static bool few_rows_win(long M, long N, long K, bool parts, bool steady) {
   if (M > 64)
     return N <= (parts && !steady ? 12288 : 8192) &&
