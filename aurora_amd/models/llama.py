@@ -364,19 +364,20 @@ class LlamaDecoderLayer(nn.Module):
     def step(self, x, residual, cos_sin, kv_cache, meta, in_parts: bool):
         """As ``forward``; with ``in_parts`` the result may be in parts, which
         ``rmsnorm_residual`` adds up, and so may ``x``."""
+        steady = getattr(meta, "steady", False)
         if residual is None:
             residual = x
             h = ops.rmsnorm(x, self.input_norm, self.eps)
         else:
             h, residual = ops.norm_ahead(x, residual, self.input_norm, self.eps,
-                                         self._reader("attn", x), False)
+                                         self._reader("attn", x), False, steady)
         attn = self.attn.parts if is_plain(self.attn, LlamaAttention) else self.attn
         a = attn(h, cos_sin, kv_cache, meta)
         h, residual = ops.norm_ahead(a, residual, self.post_attn_norm, self.eps,
-                                     self._reader("mlp", a) if in_parts else None, True)
+                                     self._reader("mlp", a) if in_parts else None, True, steady)
         if not in_parts or not is_plain(self.mlp, LlamaMLP):
             return self.mlp(h), residual
-        if getattr(meta, "steady", False):
+        if steady:
             return self.mlp.parts(h, True), residual
         return self.mlp.parts(h), residual
 

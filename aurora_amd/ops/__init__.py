@@ -284,11 +284,13 @@ class Unnormed(NamedTuple):
         return self.residual.shape
 
 
-def norm_ahead(x, residual, weight, eps, reader: Optional[torch.Tensor], silu: bool):
+def norm_ahead(x, residual, weight, eps, reader: Optional[torch.Tensor], silu: bool,
+               steady: bool = False):
     """``rmsnorm_residual`` for ``linear_parts``, or with ``silu`` ``linear_silu_mul``, by
-    ``reader``, the only reader of the rows: a single row in parts is left to it."""
+    ``reader``, the only reader of the rows: a single row in parts is left to it. ``steady``
+    as the product is told."""
     if (reader is not None and x.is_cuda and x.dim() == 3 and x.shape[1] == 1
-            and _require_hip("norm_ahead").norms_row(x, residual, weight, reader, silu)):
+            and _require_hip("norm_ahead").norms_row(x, residual, weight, reader, silu, steady)):
         new = torch.empty_like(residual)
         return Unnormed(x, residual, weight, float(eps), new), new
     return rmsnorm_residual(x, residual, weight, eps)
@@ -300,7 +302,7 @@ def linear_parts(x, weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     (``rmsnorm_residual``, ``fused_rope_kv_write``). ``x``: rows, or one of
     ``norm_ahead``."""
     if isinstance(x, Unnormed):
-        return _hip.one_row_product(*x, weight, False)
+        return _hip.one_row_product(*x, weight, False, steady)
     y = _hip.own_product(x, weight, 5 if steady else 1) if x.is_cuda and _hip is not None else None
     return F.linear(x, weight) if y is None else y
 

@@ -33,9 +33,9 @@ torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, l
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor weight, double eps,
-                              torch::Tensor res_out, torch::Tensor w, bool silu);
+                              torch::Tensor res_out, torch::Tensor w, bool silu, bool steady);
 bool norms_row(const torch::Tensor& x, const torch::Tensor& res, const torch::Tensor& weight,
-               const torch::Tensor& w, bool silu);
+               const torch::Tensor& w, bool silu, bool steady);
 torch::Tensor skinny_gemm2_ex(torch::Tensor x, torch::Tensor w, long s_target);
 torch::Tensor skinny_gemm3_ex(torch::Tensor x, torch::Tensor w, long s_target);
 torch::Tensor moe_grouped_gemm(torch::Tensor xp, torch::Tensor w,
@@ -212,8 +212,11 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("rows") = 0);
   m.def("linear_few_rows", &linear_few_rows, "linear of at most 128 rows", py::arg("x"),
         py::arg("w"), py::arg("raw"), py::arg("steady") = false);
-  m.def("one_row_product", &one_row_product, "a norm and the product of its one row");
-  m.def("norms_row", &norms_row, "whether one_row_product serves");
+  m.def("one_row_product", &one_row_product, "a norm and the product of its one row",
+        py::arg("x"), py::arg("res"), py::arg("weight"), py::arg("eps"), py::arg("res_out"),
+        py::arg("w"), py::arg("silu"), py::arg("steady") = false);
+  m.def("norms_row", &norms_row, "whether one_row_product serves", py::arg("x"), py::arg("res"),
+        py::arg("weight"), py::arg("w"), py::arg("silu"), py::arg("steady") = false);
   m.def("silu_few_rows", &silu_few_rows, "gate and up of at most 128 rows, silu(gate) * up");
   m.def("skinny_gemm2_ex", &skinny_gemm2_ex, "products of at most 256 rows");
   m.def("skinny_gemm3_ex", &skinny_gemm3_ex, "glds double-buffered projection GEMM (M<=256)");

@@ -614,9 +614,9 @@ bool one_row_fits(long S, long K) {
 }
 
 // w @ norm(x's parts + res), with ``silu`` as silu_few_rows, else as linear_few_rows's parts;
-// the sum goes to res_out.
+// the sum goes to res_out. ``steady``: K's parts as linear_few_rows then has them.
 torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor weight, double eps,
-                              torch::Tensor res_out, torch::Tensor w, bool silu) {
+                              torch::Tensor res_out, torch::Tensor w, bool silu, bool steady) {
   TORCH_CHECK(x.is_cuda() && x.dtype() == torch::kFloat32 && x.is_contiguous() && x.dim() == 3 &&
                   x.size(1) == 1 && one_row_fits(x.size(0), x.size(2)),
               "a row in parts [S, 1, K]");
@@ -629,7 +629,7 @@ torch::Tensor one_row_product(torch::Tensor x, torch::Tensor res, torch::Tensor 
                   (uintptr_t)x.data_ptr() % 16 == 0 && res.data_ptr() != res_out.data_ptr(),
               "rows of K");
   const c10::DeviceGuard on(x.device());
-  const Cut cut = silu ? Cut{64, 1} : cut_of(1, N, K);
+  const Cut cut = silu ? Cut{64, 1} : steady ? Cut{64, parts_of(N, K)} : cut_of(1, N, K);
   const long steps = K / FEW_K, parts = cut.parts;
   const long per = (steps + parts - 1) / parts, S2 = (steps + per - 1) / per;
   torch::Tensor out, part;

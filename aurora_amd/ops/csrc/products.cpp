@@ -215,7 +215,7 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
 // Whether the norm of x's parts + res by ``weight`` is done by the product with w that reads it,
 // in parts or with ``silu``: one row, where the kernel of few rows would take the product.
 bool norms_row(const torch::Tensor& x, const torch::Tensor& res, const torch::Tensor& weight,
-               const torch::Tensor& w, bool silu) {
+               const torch::Tensor& w, bool silu, bool steady) {
   if (x.dim() != 3 || x.size(1) != 1 || x.dtype() != torch::kFloat32 || !x.is_cuda() ||
       !plain(x) || !x.is_contiguous() || (uintptr_t)x.data_ptr() % 16)
     return false;
@@ -227,5 +227,6 @@ bool norms_row(const torch::Tensor& x, const torch::Tensor& res, const torch::Te
   if (!one_row_fits(x.size(0), K) || res.dim() != 2 || res.size(0) != 1 || res.size(1) != K ||
       weight.numel() != K || w.dim() != 2 || w.size(1) != K || w.size(0) == 0 || w.size(0) % 16)
     return false;
-  return silu ? silu_few_rows_win(1, w.size(0) / 2, K) : few_rows_win(1, w.size(0), K, true, false);
+  return silu ? silu_few_rows_win(1, w.size(0) / 2, K)
+              : few_rows_win(1, w.size(0), K, true, steady);
 }

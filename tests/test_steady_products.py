@@ -1,0 +1,63 @@
+"""Products on their way into an 8-bit cache keep their order of sums, whoever watches them."""
+
+import pytest
+import torch
+
+from aurora_amd import ops
+from aurora_amd.models.config import ModelSpec
+from aurora_amd.models.llama import AttnMetadata, LlamaForCausalLM
+
+P = 64
+GPU = pytest.mark.gpu
+
+
+def _model(width=256, experts=0, device="cuda"):
+    spec = ModelSpec(name="t", vocab_size=64, hidden_size=width, n_layers=2,
+                     n_heads=width // 128 or 1, n_kv_heads=max(width // 512, 1), head_dim=128,
+                     intermediate_size=512, n_experts=experts)
+    m = LlamaForCausalLM(spec, torch.bfloat16 if device == "cuda" else torch.float32, device)
+    m.init_random(0)
+    return m
+
+
+def _parts(m, T, eight=True, kind=AttnMetadata):
+    """What a step of one prompt of T tokens is called with."""
+    s, dev, n = m.spec, m.embed.weight.device, -(-T // P)
+    dtype = torch.float8_e4m3fn if eight else m.dtype
+    caches = [tuple(torch.zeros(n, s.n_kv_heads, P, s.head_dim, device=dev).to(dtype)
+                    for _ in "kv") for _ in range(s.n_layers)]
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=dev)  # noqa: E731
+    at = i32(list(range(T)))
+    return torch.arange(T, device=dev) % 64, caches, kind(
+        mode="prefill", positions=at, slot_mapping=at, block_tables=i32([list(range(n))]),
+        context_lens=i32([T]), cu_seqlens_q=i32([0, T]))
+
+
+@GPU
+def test_a_row_whose_norm_is_left_to_the_product(monkeypatch):
+    """One row 4096 wide: 6144 outputs in the parts that 64 rows of weights want."""
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x = torch.randn(2, 1, 4096, generator=g, device="cuda")
+    res, norm = (torch.randn(n, generator=g, device="cuda").bfloat16()
+                 for n in ((1, 4096), (4096,)))
+    w = (torch.randn(6144, 4096, generator=g, device="cuda") / 64).bfloat16()
+    for steady, parts in ((True, 2), (False, 4)):
+        h, new = ops.norm_ahead(x, res, norm, 1e-5, w, False, steady)
+        assert isinstance(h, ops.Unnormed)
+        y = ops.linear_parts(h, w, steady)
+        assert y.shape == (parts, 1, 6144)
+        if steady:
+            rows, summed = ops.rmsnorm_residual(x, res, norm, 1e-5)
+            assert torch.equal(new, summed)
+            assert torch.equal(y, ops._hip.few_rows(rows, w, True, 2, 64))
+    m, seen, real = _model(4096), [], ops.linear_parts
+
+    def look(h, w, steady=False):
+        y = real(h, w, steady)
+        if w.shape[0] == 6144:
+            seen.append((isinstance(h, ops.Unnormed), y.shape[0]))
+        return y
+
+    monkeypatch.setattr(ops, "linear_parts", look)
+    m(*_parts(m, 1))
+    assert seen == [(False, 2), (True, 2)]
