@@ -33,6 +33,7 @@ from ..parallel.tp import (
     column_weight,
     is_plain,
     row_parts,
+    told,
 )
 from .config import ModelSpec
 
@@ -377,9 +378,7 @@ class LlamaDecoderLayer(nn.Module):
                                      self._reader("mlp", a) if in_parts else None, True, steady)
         if not in_parts or not is_plain(self.mlp, LlamaMLP):
             return self.mlp(h), residual
-        if steady:
-            return self.mlp.parts(h, True), residual
-        return self.mlp.parts(h), residual
+        return told(self.mlp, h, LlamaMLP, steady, "parts"), residual
 
     def _reader(self, what: str, x: torch.Tensor) -> Optional[torch.Tensor]:
         """The weight whose product alone reads the norm before ``what``, if x, the norm's

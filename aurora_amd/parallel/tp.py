@@ -37,6 +37,17 @@ def is_plain(module: nn.Module, kind: type) -> bool:
                 or _global_backward_hooks or _global_backward_pre_hooks)
 
 
+def told(m: nn.Module, x, kind: type, steady: bool, name: str = "") -> torch.Tensor:
+    """``m(x)``, or its method ``name`` of x, which is told ``steady`` (see ``ops.linear``) where
+    it is ``kind``'s, whoever watches it; one of a user's own is given what it always was."""
+    step = getattr(m, name) if name else m
+    if not steady:
+        return step(x)
+    at = name or "forward"
+    own = at in m.__dict__ or getattr(type(m), at, None) is not getattr(kind, at)
+    return step(x) if own else step(x, steady=True)
+
+
 class ColumnParallelLinear(nn.Module):
     """Y_local = X @ W_local^T, W_local = W[rank-th output shard]."""
 

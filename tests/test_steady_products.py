@@ -1,11 +1,10 @@
 """Products on their way into an 8-bit cache keep their order of sums, whoever watches them."""
-
 import pytest
 import torch
 
 from aurora_amd import ops
 from aurora_amd.models.config import ModelSpec
-from aurora_amd.models.llama import AttnMetadata, LlamaForCausalLM
+from aurora_amd.models.llama import AttnMetadata, LlamaForCausalLM, LlamaMLP
 
 P = 64
 GPU = pytest.mark.gpu
@@ -61,3 +60,23 @@ def test_a_row_whose_norm_is_left_to_the_product(monkeypatch):
     monkeypatch.setattr(ops, "linear_parts", look)
     m(*_parts(m, 1))
     assert seen == [(False, 2), (True, 2)]
+
+
+class _Parts(LlamaMLP):
+    def parts(self, x):
+        return super().parts(2 * x)
+
+
+@GPU
+@pytest.mark.parametrize("how", ["class", "instance"])
+def test_parts_of_its_own(how):
+    """A user's own step is given the rows alone, as without an 8-bit cache."""
+    m = _model()
+    want = m(*_parts(m, 3))
+    mlp = m.layers[0].mlp
+    if how == "class":
+        mlp.__class__ = _Parts
+    else:
+        mlp.parts = lambda x: LlamaMLP.parts(mlp, 2 * x)
+    got = m(*_parts(m, 3))
+    assert torch.isfinite(got).all() and not torch.equal(got, want)
