@@ -14,6 +14,7 @@ from __future__ import annotations
 
 from copy import copy
 from dataclasses import dataclass
+from functools import partial
 from typing import List, Optional, Tuple
 
 import torch
@@ -32,6 +33,7 @@ from ..parallel.tp import (
     column_silu_mul,
     column_weight,
     is_plain,
+    row,
     row_parts,
     told,
 )
@@ -120,7 +122,8 @@ class LlamaAttention(nn.Module):
         kv_cache: Tuple[torch.Tensor, torch.Tensor],
         meta: AttnMetadata,
     ) -> torch.Tensor:
-        return self.o_proj(self._heads(x, cos_sin, kv_cache, meta))
+        return row(self.o_proj, self._heads(x, cos_sin, kv_cache, meta),
+                   getattr(meta, "steady", False))
 
     def parts(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
         """As ``forward``, possibly in parts (``ops.linear_parts``)."""
@@ -177,8 +180,8 @@ class LlamaMLP(nn.Module):
         self.gate_up = MergedColumnParallelLinear(spec.hidden_size, spec.intermediate_size, dtype=dtype)
         self.down = RowParallelLinear(spec.intermediate_size, spec.hidden_size, dtype=dtype)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.down(column_silu_mul(self.gate_up, x))
+    def forward(self, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
+        return row(self.down, column_silu_mul(self.gate_up, x, steady), steady)
 
     def parts(self, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
         """As ``forward``, possibly in parts (``ops.linear_parts``)."""
@@ -198,8 +201,8 @@ class _FullWidthMLP(nn.Module):
             spec.hidden_size, spec.intermediate_size, dtype=dtype),
             requires_grad=False)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return ops.linear(ops.linear_silu_mul(x, self.gate_up), self.down)
+    def forward(self, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
+        return ops.linear(ops.linear_silu_mul(x, self.gate_up, steady), self.down, steady)
 
 
 def _are_slices(whole: Optional[torch.Tensor], weights: List[torch.Tensor]) -> bool:
@@ -280,16 +283,16 @@ class MoEMLP(nn.Module):
             is_plain(ex, LlamaMLP) and is_plain(ex.gate_up, ColumnParallelLinear)
             and is_plain(ex.down, RowParallelLinear) for ex in self.experts)
 
-    def _local_expert_fn(self, xp: torch.Tensor,
-                         local_sel: torch.Tensor) -> torch.Tensor:
+    def _local_expert_fn(self, xp: torch.Tensor, local_sel: torch.Tensor,
+                         steady: bool = False) -> torch.Tensor:
         y = torch.empty_like(xp)
         for le in range(self.e_local):
             m = (local_sel == le)
             if m.any():
-                y[m] = self.experts[le](xp[m])
+                y[m] = told(self.experts[le], xp[m], _FullWidthMLP, steady)
         return y
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
         T, H = x.shape
         if (self.ep_size == 1 and self._experts_plain()
                 and ops.has_moe_grouped(x, self.router.weight)):
@@ -301,7 +304,8 @@ class MoEMLP(nn.Module):
         if self.ep_size > 1:
             from ..parallel import ep as pep
             return pep.ep_moe_forward(x, weights, sel, self.n_experts,
-                                      self._local_expert_fn)
+                                      partial(self._local_expert_fn, steady=True) if steady
+                                      else self._local_expert_fn)
         if T <= 256:
             return self._forward_batched(x, weights, sel)
         # prefill: per-expert token batches are large, so plain per-expert
@@ -311,7 +315,8 @@ class MoEMLP(nn.Module):
             tok, slot = (sel == e).nonzero(as_tuple=True)
             if tok.numel() == 0:
                 continue
-            out.index_add_(0, tok, self.experts[e](x[tok]) * weights[tok, slot, None])
+            y = told(self.experts[e], x[tok], LlamaMLP, steady)
+            out.index_add_(0, tok, y * weights[tok, slot, None])
         return out
 
     def _forward_batched(self, x: torch.Tensor, weights: torch.Tensor,
@@ -376,9 +381,10 @@ class LlamaDecoderLayer(nn.Module):
         a = attn(h, cos_sin, kv_cache, meta)
         h, residual = ops.norm_ahead(a, residual, self.post_attn_norm, self.eps,
                                      self._reader("mlp", a) if in_parts else None, True, steady)
-        if not in_parts or not is_plain(self.mlp, LlamaMLP):
-            return self.mlp(h), residual
-        return told(self.mlp, h, LlamaMLP, steady, "parts"), residual
+        if in_parts and is_plain(self.mlp, LlamaMLP):
+            return told(self.mlp, h, LlamaMLP, steady, "parts"), residual
+        kind = MoEMLP if isinstance(self.mlp, MoEMLP) else LlamaMLP
+        return told(self.mlp, h, kind, steady), residual
 
     def _reader(self, what: str, x: torch.Tensor) -> Optional[torch.Tensor]:
         """The weight whose product alone reads the norm before ``what``, if x, the norm's

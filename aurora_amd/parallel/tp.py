@@ -69,8 +69,8 @@ class ColumnParallelLinear(nn.Module):
             torch.empty(self.out_local, dtype=dtype), requires_grad=False
         ) if bias else None
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        y = ops.linear(x, self.weight)
+    def forward(self, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
+        y = ops.linear(x, self.weight, steady)
         if self.bias is not None:
             y = y + self.bias
         if self.gather_output:
@@ -92,8 +92,8 @@ class RowParallelLinear(nn.Module):
             torch.empty(out_features, self.in_local, dtype=dtype), requires_grad=False
         )
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
-        y = ops.linear(x, self.weight)
+    def forward(self, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
+        y = ops.linear(x, self.weight, steady)
         return pdist.tp_all_reduce(y)
 
 
@@ -134,7 +134,7 @@ def column_parts(m: nn.Module, x: torch.Tensor,
     (``ops.linear_parts``) and the bias still to be added."""
     if is_plain(m, ColumnParallelLinear) and not m.gather_output:
         return ops.linear_parts(x, m.weight, steady), m.bias
-    return m(x), None
+    return told(m, x, ColumnParallelLinear, steady), None
 
 
 def column_weight(m: nn.Module, bias: bool) -> Optional[torch.Tensor]:
@@ -148,13 +148,16 @@ def row_parts(m: nn.Module, x: torch.Tensor, steady: bool = False) -> torch.Tens
     """``m(x)`` of a row-parallel layer, possibly in parts where nothing is reduced."""
     if is_plain(m, RowParallelLinear) and pdist.tp_world_size() == 1:
         return ops.linear_parts(x, m.weight, steady)
-    if is_plain(m, RowParallelLinear) and steady:
-        return pdist.tp_all_reduce(ops.linear(x, m.weight, True))
-    return m(x)
+    return row(m, x, steady)
+
+
+def row(m: nn.Module, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
+    """``m(x)`` of a row-parallel layer; ``steady`` as for ``ops.linear``."""
+    return told(m, x, RowParallelLinear, steady)
 
 
 def column_silu_mul(m: nn.Module, x: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """``silu_mul(m(x))`` of a merged gate and up layer, in one kernel where that is faster."""
     if is_plain(m, ColumnParallelLinear) and m.bias is None and not m.gather_output:
         return ops.linear_silu_mul(x, m.weight, steady)
-    return ops.silu_mul(m(x))
+    return ops.silu_mul(told(m, x, ColumnParallelLinear, steady))

@@ -80,3 +80,40 @@ def test_parts_of_its_own(how):
         mlp.parts = lambda x: LlamaMLP.parts(mlp, 2 * x)
     got = m(*_parts(m, 3))
     assert torch.isfinite(got).all() and not torch.equal(got, want)
+
+
+@pytest.fixture
+def forms(monkeypatch):
+    """The forms that products of own kernels were asked in."""
+    seen, real = [], ops._hip.own_product
+    monkeypatch.setattr(ops._hip, "own_product",
+                        lambda x, w, form: seen.append(form) or real(x, w, form))
+    return seen
+
+
+@GPU
+@pytest.mark.parametrize("watched", [
+    "", "layers.1", "layers.0.attn", "layers.1.attn.qkv_proj", "layers.0.attn.o_proj",
+    "layers.0.mlp", "layers.1.mlp", "layers.0.mlp.gate_up", "layers.1.mlp.down"])
+@pytest.mark.parametrize("T", [3, 300])
+def test_whoever_watches(watched, T, forms):
+    """Where a layer, a module or a product is watched, and the layer before it."""
+    m, calls = _model(), []
+    if watched:
+        m.get_submodule(watched).register_forward_hook(lambda *a: calls.append(a[1]))
+    m(*_parts(m, T))
+    assert len(forms) >= 6 and all(f & 4 or f == 2 for f in forms)
+    assert len(calls) == bool(watched) and all(
+        isinstance(t, (torch.Tensor, tuple, AttnMetadata, type(None))) for c in calls for t in c)
+    forms.clear()
+    m(*_parts(m, T, eight=False))
+    assert forms and not any(f & 4 for f in forms)
+
+
+@GPU
+def test_watched_experts(forms):
+    m = _model(experts=2)
+    m.layers[0].mlp.experts[1].register_forward_hook(lambda *a: None)
+    m(*_parts(m, 300))
+    # two layers' attention, one's experts
+    assert len(forms) >= 6 and all(f & 4 or f == 2 for f in forms)
