@@ -72,8 +72,9 @@ class AttnMetadata:
     # decode: every row is the last token of a sequence that no other row belongs to, at the
     # position before its context's end and in the slot that its table names for it
     last_tokens: bool = False
-    # prompts that fill an 8-bit cache: the products' sums keep their order (``ops.linear``)
-    steady: bool = False
+    # prompts that fill an 8-bit cache: the products' sums keep their order (``ops.linear``).
+    # The model finds it out once a step, layers called by themselves each for itself
+    steady: Optional[bool] = None
 
     def segments(self, T: int) -> List[ops.Segment]:
         """The step's prompt portions and its single-token rows, each with its
@@ -100,6 +101,21 @@ class AttnMetadata:
         return out
 
 
+def _eight_bits(kv_cache) -> bool:
+    try:
+        return kv_cache[0].element_size() == 1
+    except (TypeError, LookupError, AttributeError):
+        return False  # what a layer that replaced another may have
+
+
+def _steady(meta, kv_cache) -> bool:
+    """``AttnMetadata.steady`` of metadata of any kind."""
+    known = getattr(meta, "steady", None)
+    if known is None:
+        return getattr(meta, "mode", "decode") != "decode" and _eight_bits(kv_cache)
+    return known
+
+
 class LlamaAttention(nn.Module):
     def __init__(self, spec: ModelSpec, dtype):
         super().__init__()
@@ -122,18 +138,17 @@ class LlamaAttention(nn.Module):
         kv_cache: Tuple[torch.Tensor, torch.Tensor],
         meta: AttnMetadata,
     ) -> torch.Tensor:
-        return row(self.o_proj, self._heads(x, cos_sin, kv_cache, meta),
-                   getattr(meta, "steady", False))
+        return row(self.o_proj, self._heads(x, cos_sin, kv_cache, meta), _steady(meta, kv_cache))
 
     def parts(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
         """As ``forward``, possibly in parts (``ops.linear_parts``)."""
         return row_parts(self.o_proj, self._heads(x, cos_sin, kv_cache, meta),
-                         getattr(meta, "steady", False))
+                         _steady(meta, kv_cache))
 
     def _heads(self, x, cos_sin, kv_cache, meta) -> torch.Tensor:
         """The heads' results side by side, [T, heads * width]."""
         T = x.shape[0]
-        qkv, bias = column_parts(self.qkv_proj, x, getattr(meta, "steady", False))
+        qkv, bias = column_parts(self.qkv_proj, x, _steady(meta, kv_cache))
         k_cache, v_cache = kv_cache
         if meta.mode == "decode" and getattr(meta, "last_tokens", False):
             o = ops.fresh_attention_decode(
@@ -370,7 +385,7 @@ class LlamaDecoderLayer(nn.Module):
     def step(self, x, residual, cos_sin, kv_cache, meta, in_parts: bool):
         """As ``forward``; with ``in_parts`` the result may be in parts, which
         ``rmsnorm_residual`` adds up, and so may ``x``."""
-        steady = getattr(meta, "steady", False)
+        steady = _steady(meta, kv_cache)
         if residual is None:
             residual = x
             h = ops.rmsnorm(x, self.input_norm, self.eps)
@@ -446,13 +461,12 @@ class LlamaForCausalLM(nn.Module):
         residual = None
         if isinstance(meta, AttnMetadata):  # of another kind every layer makes its own marks
             tables = {"decode": meta.block_tables, "mixed": meta.dec_block_tables}.get(meta.mode)
-            if tables is not None and kv_caches:
+            if kv_caches:
                 meta = copy(meta)
-                meta.marks = ops.decode_marks(
-                    self.spec.n_heads // pdist.tp_world_size(), kv_caches[0][0], tables)
-            if meta.mode != "decode" and kv_caches and kv_caches[0][0].element_size() == 1:
-                meta = copy(meta)
-                meta.steady = True
+                meta.steady = meta.mode != "decode" and _eight_bits(kv_caches[0])
+                if tables is not None:
+                    meta.marks = ops.decode_marks(
+                        self.spec.n_heads // pdist.tp_world_size(), kv_caches[0][0], tables)
         # layers that somebody watches or has replaced are called and get no parts
         plain = [is_plain(layer, LlamaDecoderLayer) for layer in self.layers] + [True]
         for i, (layer, cache) in enumerate(zip(self.layers, kv_caches)):

@@ -1,6 +1,9 @@
 """Products on their way into an 8-bit cache keep their order of sums, whoever watches them."""
+import types
+
 import pytest
 import torch
+import torch.nn as nn
 
 from aurora_amd import ops
 from aurora_amd.models.config import ModelSpec
@@ -117,3 +120,34 @@ def test_watched_experts(forms):
     m(*_parts(m, 300))
     # two layers' attention, one's experts
     assert len(forms) >= 6 and all(f & 4 or f == 2 for f in forms)
+
+
+@GPU
+def test_metadata_of_any_kind(forms):
+    m = _model()
+    m(*_parts(m, 3, kind=types.SimpleNamespace))
+    assert len(forms) >= 6 and all(f & 4 or f == 2 for f in forms)
+
+
+@GPU
+@pytest.mark.parametrize("kind", [AttnMetadata, types.SimpleNamespace])
+def test_layers_called_by_themselves(kind, forms):
+    m = _model()
+    ids, caches, meta = _parts(m, 3, kind=kind)
+    m.layers[0](m.embed(ids), None, m.cos_sin, caches[0], meta)
+    assert len(forms) >= 3 and all(f & 4 or f == 2 for f in forms)
+
+
+class _NoCache(nn.Module):
+    def forward(self, x, residual, cos_sin, kv_cache, meta):
+        assert kv_cache is None
+        return x, x if residual is None else residual
+
+
+@pytest.mark.parametrize("device", ["cpu", pytest.param("cuda", marks=GPU)])
+def test_a_first_layer_without_a_cache(device):
+    """What replaces a layer need not have a cache."""
+    m = _model(device=device)
+    m.layers[0] = _NoCache()
+    ids, caches, meta = _parts(m, 3, eight=False)
+    assert torch.isfinite(m(ids, [None, caches[1]], meta)).all()
