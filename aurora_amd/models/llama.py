@@ -70,7 +70,8 @@ class AttnMetadata:
     ctx_host: Optional[List[int]] = None  # context_lens of the prompt portions
     marks: Optional[torch.Tensor] = None  # ``ops.decode_marks`` of the single tokens
     # decode: every row is the last token of a sequence that no other row belongs to, at the
-    # position before its context's end and in the slot that its table names for it
+    # position before its context's end and in the slot that its table names for it. (Rows that
+    # nobody reads may share a page that is nobody's, as a captured batch's idle rows do)
     last_tokens: bool = False
     # prompts that fill an 8-bit cache: the products' sums keep their order (``ops.linear``).
     # The model finds it out once a step, layers called by themselves each for itself

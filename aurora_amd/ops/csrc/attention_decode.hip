@@ -256,7 +256,10 @@ struct Fresh {
   void *kc, *vc;
   int parts;
   long step;
+  bool by_eight;  // the order of sums of the separate kernel's form of many rows
 };
+
+bool rotates_by_eight(long T, long width);  // defined in elementwise.hip
 
 // BIAS: a distance penalty per head or none (see attention_prefill.hip), a window or
 // chunks of positions; sink: one more term of the denominator per head, or null;
@@ -599,7 +602,8 @@ __global__ __launch_bounds__(256, FRESH && D == 64 ? 4 : 2) void paged_decode_ke
         for (int j = 0; j < 2; ++j) {
           const float x1 = y[0][j], x2 = y[1][j];
           y[0][j] = __builtin_fmaf(x1, cs[j], -(x2 * sn[j]));
-          y[1][j] = __builtin_fmaf(x2, cs[j], x1 * sn[j]);
+          y[1][j] = fresh.by_eight ? __builtin_fmaf(x1, sn[j], x2 * cs[j])
+                                   : __builtin_fmaf(x2, cs[j], x1 * sn[j]);
         }
       if (is_q) {
 #pragma unroll
@@ -813,7 +817,7 @@ c10::optional<torch::Tensor> fresh_attention_decode(
   auto out = torch::empty({B, Hq, D}, qkv.options().dtype(torch::kBFloat16));
   const Fresh fresh = {qkv.data_ptr(), bias ? (const unsigned short*)bias->data_ptr() : nullptr,
                        cos_sin.data_ptr<float>(), kc.data_ptr(), vc.data_ptr(),
-                       raw ? (int)qkv.size(0) : 1, B * width};
+                       raw ? (int)qkv.size(0) : 1, B * width, rotates_by_eight(B, width)};
 #define RUN1(DD, F8, HOW)                                                                   \
   decode_launch<DD, DD, F8, NO_BIAS, HOW>(out, kc, vc, bt, ctx, o, Hq* D, DD, (float)scale, \
                                           1.f, nullptr, nullptr, 0, 0, nullptr, HeadTurn{}, \

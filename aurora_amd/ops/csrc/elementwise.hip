@@ -477,8 +477,10 @@ __global__ __launch_bounds__(256) void fused_rope_kv_write_kernel(
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
       const float c = cs[j], s = cs[half + j], x1 = y[0][j], x2 = y[1][j];
-      y[0][j] = x1 * c - x2 * s;
-      y[1][j] = x2 * c + x1 * s;
+      // (the compiler's own choices for the two forms, held fast: decode attention that rotates
+      // by itself has either's bits)
+      y[0][j] = __builtin_fmaf(x1, c, -(x2 * s));
+      y[1][j] = VEC == 8 ? __builtin_fmaf(x1, s, x2 * c) : __builtin_fmaf(x2, c, x1 * s);
     }
   }
   void* to = is_q ? (void*)q_out : is_v ? vc : kc;
@@ -501,6 +503,8 @@ __global__ __launch_bounds__(256) void fused_rope_kv_write_kernel(
     }
   }
 }
+
+bool rotates_by_eight(long T, long width) { return T * width >= 1 << 20; }
 
 torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
                                   torch::Tensor slots, torch::Tensor cos_sin,
@@ -525,7 +529,7 @@ torch::Tensor fused_rope_kv_write(torch::Tensor qkv, torch::Tensor positions,
     bits |= (uintptr_t)p;
   // few rows leave the chip idle with eight columns a thread: 23 rows of 3072 in 5 parts
   // 3.5 us and 2.8, but 300 rows of 4608 6.2 us both ways
-  const int vec = D % 16 == 0 && bits % 16 == 0 && T * width >= 1 << 20 ? 8 : 1;
+  const int vec = D % 16 == 0 && bits % 16 == 0 && rotates_by_eight(T, width) ? 8 : 1;
   const long threads = (long)T * (Hq + 2 * Hkv) * (D / 2 / vec);
   TORCH_CHECK(threads < 1L << 32, "more rows than a launch can index");
   auto launch = [&](auto kern, auto* src) {

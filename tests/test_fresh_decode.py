@@ -63,19 +63,72 @@ def test_as_two_kernels(contexts, hq, hkv, D, parts, biased, dtype):
 
 
 @pytest.mark.gpu
-def test_refused_forms_run_as_two():
-    """Widths, pages and layouts without a form."""
-    args = dict(parts=0, biased=False, dtype=torch.bfloat16, dev="cuda")
-    for D, page in ((96, 32), (64, 16)):
-        qkv, bias, at, slots, cs, kc, vc, bt, ctx = _case(3, [5, 9, 14], 4, 2, D, **args)
-        kc, vc = (c.reshape(-1, 2, page, D).contiguous() if page == 32 else
-                  c[:, :, :page].contiguous() for c in (kc, vc))
-        slots = bt[:, 0] * page + ctx - 1
-        assert ops._hip.fresh_attention_decode(qkv, bias, cs, kc, vc, bt, ctx, 4, 0.1,
-                                               None) is None
-        if D == 64:
-            out = ops.fresh_attention_decode(qkv, bias, at, slots, cs, kc, vc, bt, ctx, 4, 0.1)
-            assert torch.isfinite(out).all()
+@pytest.mark.parametrize("B", [129, 170, 171, 192, 256, 257, 300])
+@pytest.mark.parametrize("hq,hkv,D", [(32, 8, 128), (32, 8, 64), (28, 4, 128)])
+@pytest.mark.parametrize("parts,biased,dtype", [
+    (0, False, torch.bfloat16), (3, True, torch.bfloat16), (2, False, torch.float8_e4m3fn),
+    (0, True, torch.float8_e4m3fn)])
+def test_many_rows_as_two_kernels(B, hq, hkv, D, parts, biased, dtype):
+    """The batches that are captured and more: the separate kernel has another order of sums from
+    a million elements on (171 rows of 6144)."""
+    contexts = [1 + 53 * i % 971 for i in range(B)]
+    qkv, bias, at, slots, cs, kc, vc, bt, ctx = _case(
+        B, contexts, hq, hkv, D, parts, biased, dtype, "cuda")
+    k2, v2 = kc.clone(), vc.clone()
+    out = ops._hip.fresh_attention_decode(qkv, bias, cs, kc, vc, bt, ctx, hq, D ** -0.5, None)
+    q = ops.fused_rope_kv_write(qkv, at, slots, cs, k2, v2, hq, hkv, bias)
+    want = ops.paged_attention_decode(q, k2, v2, bt, ctx, D ** -0.5)
+    bits = torch.uint8 if dtype != torch.bfloat16 else torch.int16
+    assert torch.equal(kc.view(bits), k2.view(bits)) and torch.equal(vc.view(bits), v2.view(bits))
+    assert torch.equal(out, want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("idle", [1, 5, 130])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e4m3fn])
+def test_idle_rows(idle, dtype):
+    """Rows of a captured batch that no sequence fills are all alike, on one page with a context
+    of one: the others and their pages are as without them."""
+    B, hq, hkv, D = 60, 8, 2, 128
+    qkv, _, at, slots, cs, kc, vc, bt, ctx = _case(
+        B, [1, 31, 33, 700, 129], hq, hkv, D, 0, False, dtype, "cuda")
+    k2, v2 = kc.clone(), vc.clone()
+    want = ops.fresh_attention_decode(qkv, None, at, slots, cs, k2, v2, bt, ctx, hq, 0.1)
+    more = lambda t, v: torch.cat([t, t.new_full((idle, *t.shape[1:]), v)])  # noqa: E731
+    scratch = 0  # of the pages that _case gives to nobody
+    out = ops.fresh_attention_decode(more(qkv, 0.5), None, more(at, 0), more(slots, scratch * P), cs,
+                                     kc, vc, more(bt, scratch), more(ctx, 1), hq, 0.1)
+    bits = torch.uint8 if dtype != torch.bfloat16 else torch.int16
+    assert torch.equal(out[:B], want) and torch.isfinite(out).all()
+    assert torch.equal(kc.view(bits)[1:], k2.view(bits)[1:])
+    assert torch.equal(vc.view(bits)[1:], v2.view(bits)[1:])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,page", [(64, 16), (128, 16)])
+def test_refused_forms_run_as_two(D, page):
+    """Pages without a form: the reference's results and cache."""
+    qkv, bias, at, slots, cs, kc, vc, bt, ctx = _case(3, [5, 9, 14], 4, 2, D, 0, True,
+                                                      torch.bfloat16, "cuda")
+    kc, vc = (c[:, :, :page].nan_to_num().contiguous() for c in (kc, vc))
+    slots = bt[:, 0] * page + ctx - 1
+    args = [qkv, bias, at, slots, cs, kc, vc, bt, ctx]
+    host = [t.cpu() for t in args]
+    assert ops._hip.fresh_attention_decode(qkv, bias, cs, kc, vc, bt, ctx, 4, 0.1, None) is None
+    out = ops.fresh_attention_decode(*args, 4, 0.1).float().cpu()
+    want = ops.fresh_attention_decode(*host, 4, 0.1).float()
+    # a row may round the other way in bf16; of results as well, whose weights add up to one
+    for got, held in ((kc, host[5]), (vc, host[6])):
+        got, held = got.float().cpu(), held.float()
+        assert ((got - held).abs() <= 2 ** -7 * held.abs() + 1e-6).all()
+    assert ((out - want).abs() <= 2 ** -6 * host[6].float().abs().max()).all()
+
+
+@pytest.mark.gpu
+def test_refused_width():
+    qkv, bias, _, _, cs, kc, vc, bt, ctx = _case(3, [5, 9, 14], 4, 2, 96, 0, True, torch.bfloat16,
+                                                 "cuda")
+    assert ops._hip.fresh_attention_decode(qkv, bias, cs, kc, vc, bt, ctx, 4, 0.1, None) is None
 
 
 def test_reference():
