@@ -386,12 +386,14 @@ static long parts_of(long N, long K) {
 
 // Rows of W a workgroup takes and K's parts: what leaves a CU the least to read, of W at 21 GB/s
 // when all read at once and of x at some 125, where the whole W does not take longer anyway
-// (5.3 TB/s), and the reader the fewest parts; 64 rows unless 1.5 us are gained. Of 46 weights, 1
-// to 128 rows each, the norm that reads the parts included, the cut so chosen takes 1.2% longer
-// than the best, 64 rows with the parts above 3.3%. us: 6144 x 4096, 1, 32, 64 and 96 rows, 64
-// wide 16.8 17.3 19.3 21.3, 96 wide in 4 parts 15.0 16.1 17.4 19.1; 8576 x 16064, 32 and 96 rows,
-// 64 wide 76.9 104.3, 128 in 3 parts 56.9 71.4; 4096 x 14336, 96 rows, 64 wide in 4 parts 32.8,
-// 128 in 8 32.2; 5120 x 5120, 64 rows, 19.4 and 19.3.
+// (5.3 TB/s), and the reader the fewest parts; 64 rows unless 1.5 us are gained. Parts of a
+// multiple of 2048 of K begin 4 KB apart, which tiles of more than 64 rows show (4608 x 14336, 8
+// rows, 128 wide, 7 parts of 2048 35.7 us, 6 of 2432 29.2, 64 wide 27.9). Of 318 weights of 0.5 to
+// 160 MB, 2 to 128 rows each, the norm that reads the parts included, the cut so chosen takes 1.4%
+// longer than the best, 64 rows with the parts above 3.5%; one call in 90 is 3 to 8% behind the
+// latter. us: 6144 x 4096, 1, 32, 64 and 96 rows, 64 wide 16.8 17.3 19.3 21.3, 96 wide in 4 parts
+// 15.0 16.1 17.4 19.1; 8576 x 16064, 32 and 96 rows, 64 wide 73.7 100.4, 128 in 3 parts 56.2 66.9;
+// 1536 x 1536, 8 parts, 64 and 128 rows 9.0 11.7, 96 wide in 12 10.0 13.4.
 struct Cut {
   int width;
   long parts, rows = 0;
@@ -407,12 +409,11 @@ static Cut cut_of(long M, long N, long K) {
     if (M == 1 && width > 96) break;  // (one_row_kernel has no wider form)
     const long tiles = (N + width - 1) / width;
     const long most = std::max(1L, std::min({256 / tiles, steps / 2, 16L}));
-    for (long parts = most; parts >= std::max(1L, most - 1); --parts) {
-      const long per = (steps + parts - 1) / parts;
-      if ((steps + per - 1) / per != parts) continue;  // the same with fewer
+    for (long asked = most; asked >= std::max(1L, width > 64 ? most - 1 : most); --asked) {
+      const long per = (steps + asked - 1) / asked, parts = (steps + per - 1) / per;
       const double cu = per * FEW_K * (width * 2 / 21. + rows * 2 * 0.4 / 50);
-      const double time = std::max(cu, N * K * 2 / 5300.) + parts * M * N * 4 / 5000. +
-                          (width > 64 ? 1500 : 0);
+      double time = std::max(cu, N * K * 2 / 5300.) + parts * (M * N * 4 / 5000. + 50);
+      if (width > 64) time = time * (parts > 1 && per % 32 == 0 ? 1.15 : 1) + 1500;
       if (low == 0 || time < low) low = time, best = {width, parts};
     }
   }

@@ -52,6 +52,19 @@ def test_chosen_cuts(m, n, k):
         assert y.dim() == 3
 
 
+@pytest.mark.parametrize("m", [2, 40, 70, 128])
+@pytest.mark.parametrize("n", [64, 512, 768, 1024, 1536, 2048])
+def test_steps_that_do_not_divide(m, n):
+    """Every number of steps is cut, into parts that use at least half of what 64 rows of weights
+    leave room for."""
+    for steps in (20, 24, 25, 31, 36, 40, 55, 56, 64, 81):
+        x, w = _inputs(m, n, steps * 64)
+        y = ops.linear_parts(x, w)
+        room = min(256 // (-(-n // 64)), steps // 2, 16)
+        assert y.dim() == 3 and y.shape[0] >= room / 2
+        _check(y.sum(0).bfloat16(), x.double() @ w.double().t())
+
+
 @pytest.mark.parametrize("m", [65, 97, 129, 192, 193, 300, 1000])
 @pytest.mark.parametrize("n,k", [(512, 576), (768, 3072), (2048, 2048), (2120, 4160), (72, 64),
                                  (3400, 1024)])

@@ -96,8 +96,8 @@ def test_idle_rows(idle, dtype):
     want = ops.fresh_attention_decode(qkv, None, at, slots, cs, k2, v2, bt, ctx, hq, 0.1)
     more = lambda t, v: torch.cat([t, t.new_full((idle, *t.shape[1:]), v)])  # noqa: E731
     scratch = 0  # of the pages that _case gives to nobody
-    out = ops.fresh_attention_decode(more(qkv, 0.5), None, more(at, 0), more(slots, scratch * P), cs,
-                                     kc, vc, more(bt, scratch), more(ctx, 1), hq, 0.1)
+    out = ops.fresh_attention_decode(more(qkv, 0.5), None, more(at, 0), more(slots, scratch * P),
+                                     cs, kc, vc, more(bt, scratch), more(ctx, 1), hq, 0.1)
     bits = torch.uint8 if dtype != torch.bfloat16 else torch.int16
     assert torch.equal(out[:B], want) and torch.isfinite(out).all()
     assert torch.equal(kc.view(bits)[1:], k2.view(bits)[1:])
