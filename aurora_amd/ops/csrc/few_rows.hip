@@ -588,9 +588,18 @@ torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w) {
   auto* op = (unsigned short*)out.data_ptr();
   // From 65 rows on x is as much to move as W: tiles of 128 halve it where there are enough
   // for the chip. 28672 x 4096, 96 rows, 59.9 and 56.1 us; 16384 x 2048 21.8 and 27.6; 28672
-  // x 4096, 64 rows, 53.3 and 53.6. Tiles of 112 where one for every CU is enough (33, 64, 96 and
-  // 128 rows 49.5 51.9 55.3 56.5, and 48.9 49.7 52.5 55.2).
-  const bool wide = N / 64 >= 192, one = wide && (N + 55) / 56 <= 256;
+  // x 4096, 64 rows, 53.3 and 53.6. Tiles of 112 where one for every CU is enough: time with the
+  // others over that with them, 33, 48, 64 and 96 rows:
+  //   K      12288 outputs         13312                 14336
+  //   1024   1.09 1.14 1.15 1.03   1.07 1.11 1.14 1.03   1.04 1.08 1.11 1.03
+  //   2048   1.03 1.05 1.07 1.03   0.98 1.00 1.03 1.03   0.96 0.98 1.02 1.03
+  //   3072   1.16 1.19 1.21 1.05   1.15 1.18 1.20 1.05   1.10 1.16 1.18 1.04
+  //   3584   1.18 1.20 1.22 1.05   1.15 1.19 1.21 1.05   1.11 1.16 1.20 1.05
+  //   4096   1.07 1.08 1.09 1.03   1.02 1.05 1.07 1.03   0.95 0.98 1.02 1.02
+  // Rows of W 4 or 8 KB apart hold up tiles of 112 (28672 x 4096 4.6 TB/s, x 3584 5.5), so with
+  // few rows of x and many outputs they stay at 64.
+  const bool wide = N / 64 >= 192,
+             one = wide && (N + 55) / 56 <= 256 && (M > 52 || K % 2048 || N <= 13056);
   auto rows = [&](auto MT) {
     constexpr int mt = decltype(MT)::value;
     if constexpr (mt > 2)

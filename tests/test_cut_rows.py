@@ -39,6 +39,15 @@ def test_silu_tiles(m, n):
     _check(ops._hip.silu_few_rows(x, w), torch.nn.functional.silu(y[:, :n]) * y[:, n:])
 
 
+@pytest.mark.parametrize("m", [52, 53])
+@pytest.mark.parametrize("n", [13056, 13064])
+def test_silu_rows_far_apart(m, n):
+    """Tiles of 64 and 112 on either side of their line."""
+    x, w = _inputs(m, 2 * n, 2048)
+    y = x.double() @ w.double().t()
+    _check(ops._hip.silu_few_rows(x, w), torch.nn.functional.silu(y[:, :n]) * y[:, n:])
+
+
 @pytest.mark.parametrize("m", [1, 2, 40, 70, 128])
 @pytest.mark.parametrize("n,k", [(6144, 4096), (8576, 4160), (3584, 18944)])
 def test_chosen_cuts(m, n, k):
