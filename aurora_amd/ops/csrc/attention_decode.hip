@@ -40,7 +40,7 @@
 #define DEC_TARGET 1024   // stretches that the contexts are cut into
 #define DEC_LEAST 160     // of few keys each
 
-enum { WHOLE = 1, IN_PARTS = 2 };  // what a kernel that rotates finds
+enum { FROM_WHOLE = 1, FROM_PARTS = 2 };  // what a kernel that rotates finds
 enum { NO_BIAS = 0, LINEAR_BIAS = 1, LOG_BIAS = 2, FLAT_BIAS = 3 };
 
 // keys of a sequence that its query sees: [first, L)
@@ -549,7 +549,7 @@ __global__ __launch_bounds__(256, FRESH && D == 64 ? 4 : 2) void paged_decode_ke
       const unsigned column = (is_q ? h0 + h : is_v ? Hq + Hkv + kvh : Hq + kvh) * D + i;
       floatx2 part[AHEAD][2], y[2];
       unsigned whole[2], bias[2] = {0, 0};
-      if constexpr (FRESH == IN_PARTS) {
+      if constexpr (FRESH == FROM_PARTS) {
 #pragma unroll
         for (int p = 0; p < AHEAD; ++p) {
           const float* src = (const float*)fresh.qkv + row + min(p, fresh.parts - 1) * fresh.step;
@@ -580,7 +580,7 @@ __global__ __launch_bounds__(256, FRESH && D == 64 ? 4 : 2) void paged_decode_ke
       };
 #pragma unroll
       for (int z = 0; z < 2; ++z)
-        if constexpr (FRESH == IN_PARTS) {
+        if constexpr (FRESH == FROM_PARTS) {
           y[z] = floatx2{0.f, 0.f};
 #pragma unroll
           for (int p = 0; p < AHEAD; ++p)
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(256, FRESH && D == 64 ? 4 : 2) void paged_decode_ke
         } else {
           y[z] = two(whole[z]);
         }
-      if constexpr (FRESH == IN_PARTS) {
+      if constexpr (FRESH == FROM_PARTS) {
         for (int p = AHEAD; p < fresh.parts; ++p)
 #pragma unroll
           for (int z = 0; z < 2; ++z)
@@ -822,7 +822,7 @@ c10::optional<torch::Tensor> fresh_attention_decode(
   decode_launch<DD, DD, F8, NO_BIAS, HOW>(out, kc, vc, bt, ctx, o, Hq* D, DD, (float)scale, \
                                           1.f, nullptr, nullptr, 0, 0, nullptr, HeadTurn{}, \
                                           marks, fresh)
-#define RUN(DD, F8) if (raw) RUN1(DD, F8, IN_PARTS); else RUN1(DD, F8, WHOLE)
+#define RUN(DD, F8) if (raw) RUN1(DD, F8, FROM_PARTS); else RUN1(DD, F8, FROM_WHOLE)
   auto* o = (__hip_bfloat16*)out.data_ptr();
   if (D == 128) { if (fp8) { RUN(128, true); } else { RUN(128, false); } }
   else { if (fp8) { RUN(64, true); } else { RUN(64, false); } }

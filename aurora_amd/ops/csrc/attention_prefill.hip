@@ -64,7 +64,7 @@ struct KeyTail {
 // references and sums [.., 2] another kernel merges. 32 heads of 128 over 8, us, whole and cut:
 // 100 rows behind 1500 45.8 and 27.5, behind 8000 199 and 37; 500 behind 1500 57.0 and 40.2, behind
 // 8000 211 and 85; 1000 behind 8000 224 and 157; 4 of 60 behind 4000 106 and 45.
-struct Cut {
+struct KeyCut {
   int most;
   float *part, *refs;
 };
@@ -96,7 +96,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
     const float* __restrict__ slopes, const float* __restrict__ rates, int window,
     int chunk, const float* __restrict__ sink,  // [Hq], or null unless GATED
     const __hip_bfloat16* __restrict__ gate, long gstride,  // [T, gstride]
-    KeyTail tail, HeadTurn turn, Cut cut) {
+    KeyTail tail, HeadTurn turn, KeyCut cut) {
   static_assert(!CUT || (!BIAS && EXTRA == PLAIN));
   constexpr int NC = D / 16;        // Q^T fragments (MFMA K-chunks of K Q^T)
   constexpr int NDT = DV / 32;      // 32-wide d-tiles of O^T
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(512, 1) void prefill_kernel(
 // A row of every block whose keys were cut: its parts' results put together, a wave per head.
 template <int DV>
 __global__ __launch_bounds__(256) void merge_parts_kernel(
-    Cut cut, __hip_bfloat16* __restrict__ out, const int* __restrict__ cu_q, int S,
+    KeyCut cut, __hip_bfloat16* __restrict__ out, const int* __restrict__ cu_q, int S,
     const int* __restrict__ ctx_lens, int Hq, int rows) {
   constexpr int N = DV / WAVE;
   const int row = blockIdx.x, lane = threadIdx.x % WAVE;
@@ -654,7 +654,7 @@ static torch::Tensor unit_aligned(const torch::Tensor& cache) {
 
 template <int D, int DV, int HG, bool FP8, int BIAS, int EXTRA, bool PAGED, bool CUT = false,
           typename... Args>
-static void prefill_launch(const Cut& cut, int blocks, int Hq, Args... args) {
+static void prefill_launch(const KeyCut& cut, int blocks, int Hq, Args... args) {
   constexpr int lds = PRE_STAGES * PRE_KEYS * (D + DV) * 2;
   const auto kern = prefill_kernel<D, DV, HG, FP8, BIAS, EXTRA, PAGED, CUT>;
   if (lds > 64 * 1024) {
@@ -693,7 +693,7 @@ torch::Tensor attention_prefill_paged(torch::Tensor q, torch::Tensor kc,
   // same.) An 8-bit cache is not cut: the next layers' rows in it are made of these results, and
   // other sums let one in 20 to 50 of their bytes round the other way.
   const long blocks = (long)NB * (Hq / HG), least = 2 * CUT_LEAST + blocks / 8;
-  Cut cut = {1, nullptr, nullptr};
+  KeyCut cut = {1, nullptr, nullptr};
   if (!fp8 && P % PRE_KEYS == 0 && (long)MP * P / PRE_KEYS >= least)
     cut.most = (int)std::max(1L, std::min(256 / blocks, 16L));
   torch::Tensor part, refs;
@@ -779,7 +779,7 @@ void biased_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
   const float* sp = slopes ? slopes->data_ptr<float>() : nullptr;
   const float* snk = sink ? sink->data_ptr<float>() : nullptr;
 #define BLAUNCH2(DD, DVV, HGV, BB, XX, PG)                                      \
-  prefill_launch<DD, DVV, HGV, false, BB, XX, PG>(Cut{}, NB, Hq,                            \
+  prefill_launch<DD, DVV, HGV, false, BB, XX, PG>(KeyCut{}, NB, Hq,                \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr() + col,      \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
@@ -840,7 +840,7 @@ void sink_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor vc,
   kc = unit_aligned(kc);
   vc = unit_aligned(vc);
 #define SLAUNCH(DD, DVV)                                                        \
-  prefill_launch<DD, DVV, 1, false, NO_BIAS, GATED, false>(Cut{}, NB, H,                       \
+  prefill_launch<DD, DVV, 1, false, NO_BIAS, GATED, false>(KeyCut{}, NB, H,         \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr(),            \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
@@ -892,7 +892,7 @@ void tailed_attention_prefill(torch::Tensor q, torch::Tensor kc, torch::Tensor v
   const KeyTail kt = {(const __hip_bfloat16*)tail.data_ptr(), tail.stride(0),
                       (int)tail.size(1), own};
 #define TLAUNCH(DD, DVV)                                                        \
-  prefill_launch<DD, DVV, 1, false, FLAT_BIAS, TAILED, false>(Cut{}, NB, H,                    \
+  prefill_launch<DD, DVV, 1, false, FLAT_BIAS, TAILED, false>(KeyCut{}, NB, H,       \
                      (const __hip_bfloat16*)q.data_ptr(), kc.data_ptr(),        \
                      vc.data_ptr(), (__hip_bfloat16*)out.data_ptr(),            \
                      bseq.data_ptr<int>(), boff.data_ptr<int>(),                \
