@@ -7,6 +7,7 @@ projection. The kernels between the two take columns of the fused result.
 """
 from __future__ import annotations
 
+from functools import partial
 from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
@@ -73,8 +74,8 @@ class Projected(nn.Module):
         return ops.linear(self.heads(h, meta, segments, kv, state), self.out_proj)
 
     def in_parts(self, h, meta, segments, kv, state):
-        """As ``forward``, possibly in parts (``ops.linear_parts``)."""
-        return ops.linear_parts(self.heads(h, meta, segments, kv, state), self.out_proj)
+        """As ``forward``, possibly in parts (``ops.linear_norm_parts``)."""
+        return ops.linear_norm_parts(self.heads(h, meta, segments, kv, state), self.out_proj)
 
 
 class ParallelMixer(Projected):
@@ -734,8 +735,8 @@ class DenseXieluMLP(nn.Module):
         return self._add(h, ops.linear)
 
     def in_parts(self, h) -> Dict[str, object]:
-        """As ``forward``, a delta possibly in parts (``ops.linear_parts``)."""
-        return self._add(h, ops.linear_parts)
+        """As ``forward``, a delta possibly in parts (``ops.linear_norm_parts``)."""
+        return self._add(h, ops.linear_norm_parts)
 
     def _add(self, h, product) -> Dict[str, object]:
         at, ff = self.cols.at, self.spec.ff
@@ -770,8 +771,8 @@ class DenseGeluMLP(nn.Module):
         return self._add(h, ops.linear)
 
     def in_parts(self, h) -> Dict[str, object]:
-        """As ``forward``, a delta possibly in parts (``ops.linear_parts``)."""
-        return self._add(h, ops.linear_parts)
+        """As ``forward``, a delta possibly in parts (``ops.linear_norm_parts``)."""
+        return self._add(h, ops.linear_norm_parts)
 
     def _add(self, h, product) -> Dict[str, object]:
         return {"delta": product(ops.gelu(ops.linear(h, self.up)), self.down)}
@@ -876,8 +877,8 @@ class GroupedExperts(nn.Module):
         return self._add(h, ops.linear)
 
     def in_parts(self, h) -> Dict[str, object]:
-        """As ``forward``, a delta possibly in parts (``ops.linear_parts``)."""
-        return self._add(h, ops.linear_parts)
+        """As ``forward``, a delta possibly in parts (``ops.linear_norm_parts``)."""
+        return self._add(h, partial(ops.linear_norm_parts, beside_experts=True))
 
     def _add(self, h, product) -> Dict[str, object]:
         s = self.spec

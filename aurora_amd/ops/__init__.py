@@ -307,6 +307,13 @@ def linear_parts(x, weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     return F.linear(x, weight) if y is None else y
 
 
+def linear_norm_parts(x, weight: torch.Tensor, beside_experts: bool = False) -> torch.Tensor:
+    """``linear_parts`` for ``residual_rmsnorm``, which adds parts up itself where its threads
+    hold a row: more than 256 rows up to 2048 wide, ``beside_experts``' rows up to 4096."""
+    held = x.shape[0] <= 256 or weight.shape[0] <= (4096 if beside_experts else 2048)
+    return (linear_parts if held else linear)(x, weight)
+
+
 def linear_silu_mul(x, weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """silu(gate) * up of the products with gate's rows, then up's; in one kernel where that
     is faster. ``x``: rows, or one of ``norm_ahead``."""

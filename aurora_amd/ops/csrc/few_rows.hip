@@ -490,38 +490,49 @@ torch::Tensor few_rows(torch::Tensor x, torch::Tensor w, bool raw, long parts, l
   return cut_rows(x, w, raw, Cut{(int)width, parts, rows}, rows ? 1 << 16 : FEW_MOST);
 }
 
-// How some hundred rows are cut: into blocks of ``rows``, each of which reads W once more (from
-// the L2 where it is small), tiles of ``width`` and K's parts. A form's time is that of its
-// stages of 64 of K, which depends on nothing but its rows and width while a CU has one
-// workgroup (two of 64 wide share it), and what it takes to bring the parts to their reader.
-// Of 88 sizes from 140 to 1000 rows and 768 x 768 to 4096 x 14336 the form so chosen took 3%
-// longer than the best.
+// How some hundred rows are cut: into blocks of ``rows``, each of which reads W once more, tiles
+// of ``width`` and K's parts. A form's time is that of its stages of 64 of K, which depends on
+// nothing but its rows and width while a CU has one workgroup (of 64 wide two share it), or what
+// its XCDs read, if that takes longer: a tile's blocks lie on as many XCDs as their distance
+// leaves over 8, and each of those reads the tile for itself (1408 x 8192, 400 rows, 64 x 128 in 3
+// parts 35.7 us, 96 x 128 in 4, whose blocks share two, 25.1). Then there is what it takes to
+// bring the parts to their reader. Fitted to 3516 sizes from 65 to 1000 rows and 512 x 576 to
+// 8192 x 14336; the form so chosen takes 0.6% longer than the best measured.
 static Cut block_cut(long M, long N, long K, bool raw) {
   static const struct {
     long rows;
     int width;
-    float stage;  // us
-  } forms[] = {{64, 64, .245f}, {96, 64, .30f}, {64, 128, .366f}, {96, 128, .466f},
-               {128, 128, .556f}};
+    float start, stage;  // us
+  } forms[] = {{64, 64, 0.f, .27f}, {96, 64, .35f, .31f}, {64, 128, .7f, .365f},
+               {96, 128, 1.2f, .453f}, {128, 128, 1.6f, .51f}};
   Cut best = {64, 1, 64};
   float low = 0;
   const long steps = K / FEW_K;
   for (const auto& f : forms) {
-    const long tiles = (N + f.width - 1) / f.width * ((M + f.rows - 1) / f.rows);
-    const long most = std::max(1L, std::min({256 / tiles, steps / 2, 16L}));
-    for (long parts : {1L, most}) {
-      const long per = (steps + parts - 1) / parts;
-      if ((steps + per - 1) / per != parts) continue;
-      const long each = tiles * parts;
-      const float rounds =
-          f.width == 64 ? std::max(1.f, each / 256.f) : (float)((each + 255) / 256);
-      const float time = per * f.stage * rounds +
-                         (parts > 1 ? parts * M * N * 2e-6f + (raw ? 0.f : 2.5f) : 0.f);
+    const long across = (N + f.width - 1) / f.width, blocks = (M + f.rows - 1) / f.rows;
+    const long most = std::max(1L, std::min({256 / (across * blocks), steps / 2, 16L}));
+    for (long asked : {1L, most}) {
+      const long per = (steps + asked - 1) / asked, parts = (steps + per - 1) / per;
+      const long each = across * blocks * parts;
+      const float full = each / 256.f;
+      const float rounds = f.width > 64 ? (float)((each + 255) / 256)
+                           : each <= 256 ? 1.f
+                           : std::max(1.35f, full * (each <= 512 ? .92f : 1.15f));
+      const long apart = across * parts % 8;  // blocks of a tile, in workgroups
+      const long xcds = apart == 0 ? 1 : apart == 4 ? 2 : apart % 2 == 0 ? 4 : 8;
+      const float way = N * K * 2e-6f / 7.f * std::min(blocks, xcds) +
+                        M * K * 2e-6f / 12.f * std::min(across, 8L);
+      const float time =
+          f.start + std::max(per * f.stage * rounds, way) +
+          (parts > 1 ? parts * M * N * (raw ? 1.55e-6f : 1.87e-6f) + (raw ? .4f : 3.f) : 0.f);
       if (low == 0 || time < low) low = time, best = {f.width, parts, f.rows};
     }
   }
   return best;
 }
+
+// K's parts of block_rows
+long block_parts(long M, long N, long K, bool raw) { return block_cut(M, N, K, raw).parts; }
 
 // linear_few_rows of more rows
 torch::Tensor block_rows(torch::Tensor x, torch::Tensor w, bool raw) {

@@ -10,6 +10,7 @@
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor block_rows(torch::Tensor x, torch::Tensor w, bool raw);
+long block_parts(long M, long N, long K, bool raw);
 bool one_row_fits(long S, long K);
 bool float_few_rows_fits(long N, long K);
 torch::Tensor float_few_rows(torch::Tensor x, torch::Tensor w);
@@ -136,33 +137,45 @@ static bool left_to_library(long M) {
 // 65 to 1000 rows: where the kernel of few rows, in blocks of rows, beats the library's product.
 // us with cold weights, the library's and ours, whole and in parts with the norm that reads them:
 //   N x K         rows: 140            256            300            512            1000
-//   4096 x 4096     22 18, 26 18   23 22, 27 26   26 24, 30 28   29 28, 34 33   40 41, 47 47
-//   6144 x 4096     40 25, 45 30   40 28, 45 33   29 28, 35 34   36 40, 43 46   52 74, 61 83
-//   4096 x 14336    57 41, 60 40   63 49, 65 50   76 63, 78 63   91 79, 93 80   131 131, 138 138
-//   2048 x 2048     9.1 10, 12 11  9.8 11, 13 12  11 11, 14 13   11 11, 15 15   16 14, 20 18
-//   2048 x 8192     26 18, 29 18   27 22, 30 23   33 25, 36 26   34 32, 37 32   47 48, 53 48
-//   768 x 768       5.8 6.3, 9 8   5.8 6.3, 10 10 5.8 6.3, 9 9   6.7 6.4, 11 11 8.1 6.6, 12 11
-//   768 x 3072      9 10, 12 11    10 11, 13 12   10 12, 13 12   13 13, 16 14   15 17, 19 21
-//   2304 x 768      7 7, 11 10     8 7, 12 11     9 7, 12 11     9 9, 14 13     13 10, 18 15
-// and a call of the library's takes the host 11 us more, which small prompts and texts wait for
-// (a text of 200 tokens 1197 us and 612). The line is work for a quarter of the chip, in tiles of
-// 128 x 256: beyond it both come to the same by themselves (with the norm 520 rows of 4096 x 4096
-// 39 and 36, of 4096 x 14336 111 and 111, 768 of 3584 x 14336 113 and 127) and four layers of
-// 4096, 520 rows, took 1647 and 1746 us. Within it ours falls back by up to 2 us (980 rows of 1024
-// x 4096 22 and 24, 780 of 2048 x 4096 30 and 32).
-// Short K and few rows, whole, 65, 100, 128, 180 and 300 rows, the library's and ours:
-//   256 x 256     8.2 4.4   9.0 4.4   8.8 4.4    11 4.4   5.1 4.5
-//   4096 x 256    5.6 4.5   5.5 4.5   6.2 4.6   5.9 4.7   7.5 5.2
-//   1024 x 512    5.9 5.3   6.0 5.3   7.5 5.3   6.0 5.3   6.8 5.4
-//   3072 x 1024   9.2 7.7, 9.7 7.7, 10 7.8 (65, 100 and 128 rows; 1024 x 1024 6.2 7.3)
-//   6144 x 2048    14 12     14 12     15 13 (2048 x 2048 8.4 8.4, 8.5 9.2, 8.4 9.4)
-//   2816 x 1408   8.5 9.6   8.7 9.5    12 9.6, the one found where the library is ahead
-static bool block_rows_win(long M, long N, long K) {
+//   4096 x 4096     22 18, 26 19   23 23, 27 23   26 26, 30 27   30 30, 35 35   43 43, 50 50
+//   6144 x 4096     39 25, 44 26   37 28, 41 32   29 30, 35 35   38 38, 45 44   54 54, 64 63
+//   4096 x 14336    57 40, 60 40   62 48, 67 49   75 67, 80 67   93 82, 97 84   141 141, 150 148
+//   2048 x 2048     12 11, 15 11   12 12, 15 13   13 12, 16 14   13 13, 17 16   17 16, 22 21
+//   2048 x 8192     26 18, 30 20   27 22, 31 23   33 25, 37 26   35 32, 38 33   52 52, 57 51
+//   768 x 768      6.8 5.7, 10 8  6.8 5.6, 10 8  6.8 5.7, 10 8  7.2 5.8, 11 9  7.5 5.9, 11 10
+//   768 x 3072     9.5 9.6, 13 10  10 11, 14 11   10 12, 13 12   15 12, 19 13   17 17, 20 18
+//   2304 x 768     9.5 6.2, 13 9  9.7 6.6, 13 10 9.8 6.6, 14 10  10 7.3, 15 12  13 13, 18 18
+// and a call of the library's takes the host 11 to 15 us more, which small prompts and texts wait
+// for (a text of 200 tokens 1197 us and 612). The line is work for a quarter of the chip, in tiles
+// of 128 x 256: beyond it both come to the same by themselves (with the norm 520 rows of 4096 x
+// 4096 39 and 36, of 4096 x 14336 111 and 111, 768 of 3584 x 14336 113 and 127) and four layers of
+// 4096, 520 rows, took 1647 and 1746 us. In front of it, more than 256 rows whose long K is not
+// cut, or is for a reader who does not add the parts up, come to 0.98 of the library's time and to
+// 1.16 where its tiles come out even (512 rows of 2816 x 5632 33.6 and 37.5, 1000 of 1536 x 5632
+// 32.4 and 37.7), so those are left to it too. Of 3084 sizes within the lines ours takes 0.83 of
+// the library's time whole, 0.79 with the norm. What falls behind by more than 4% are whole
+// products of 512 to 1536 outputs, K of 1400 to 3100 (10 us where the library takes 9, and the
+// host 20: 512 x 1408 8.5 and 9.1, 1408 x 2816, 140 rows, 9.8 and 11.3, 768 x 3072, 300 rows, 10.0
+// and 11.9).
+// 65 to 128 rows, whole (few_rows_win has those in parts), 65, 96 and 128, the library's and ours:
+//   K      1024 outputs                2304                        2560
+//   768    9.1 6.1, 9.0 6.2, 8.9 6.5   9.0 6.1, 9.2 6.2, 10 6.5    9.1 6.2, 9.1 6.3, 10 6.7
+//   1408   8.3 8.2, 8.7 8.8, 8.6 9.2   8.3 8.8, 8.9 8.9, 15 9.3    9.0 8.9, 9.1 9.0, 15 9.5
+//   2048   11 8.6, 11 9.6, 11 9.5      11 9.7, 11 10, 14 11        11 9.9, 11 10, 14 11
+//          2816                        4096                        8192
+//   768    9.6 6.2, 9.9 6.3, 10 6.6    9.6 6.4, 10 6.4, 10 6.7     10 6.6, 10 6.8, 11 7.1
+//   1408   9.7 8.9, 10 9.0, 15 9.3     9.6 9.1, 10 9.1, 15 9.6     11 9.7, 11 9.8, 16 10
+//   2048   12 11, 13 11, 15 11         12 11, 13 12, 15 12         14 13, 14 13, 16 13
+// and K up to 512 256 x 256 9.2 3.8, 8.4 3.5, 7.9 3.6, 4096 x 256 5.8 3.9, 6.1 4.2, 6.8 4.3, 1024 x
+// 512 7.3 4.7, 6.5 4.5, 7.7 4.5 (65, 100 and 128 rows).
+static bool block_rows_win(long M, long N, long K, bool parts) {
   if (left_to_library(M)) return false;
-  if (M <= 128) return N <= 8192 && (K <= 512 ? N >= 64 : K <= 2048 && N >= 2816);
+  if (M <= 128) return N <= 8192 && (K <= 512 ? N >= 64 : K <= 2048 && N >= 2560);
   const long work = (M + 127) / 128 * N / 256;  // (a little more, many_rows takes)
   if (K <= 512) return M <= 1000 && N >= 64 && work <= (K <= 256 ? 40 : 16);
-  return M <= 1000 && N >= 512 && (M + 127) / 128 * N <= 64 * 256;
+  if (M > 1000 || N < 512 || (M + 127) / 128 * N > 64 * 256) return false;
+  return M <= 256 || K <= 2048 || work < 44 ||
+         ((parts || K > 8192) && block_parts(M, N, K, parts) > 1);
 }
 
 // x @ w^T in ``form``, or nothing: the library's product serves better or is followed by
@@ -199,14 +212,15 @@ c10::optional<torch::Tensor> own_product(const torch::Tensor& x, const torch::Te
     if (form == PARTS && few_rows_win(M, N, K, true, steady))
       return linear_few_rows(x, w, true, steady);
     if (few_rows_win(M, N, K, false, steady)) return linear_few_rows(x, w, false, steady);
-    if (!steady && M > 64 && block_rows_win(M, N, K)) return block_rows(x, w, form == PARTS);
+    if (!steady && M > 64 && block_rows_win(M, N, K, form == PARTS))
+      return block_rows(x, w, form == PARTS);
   } else if (large_takes(N, K) && many_rows_win(M, N, K, false)) {
     return many_rows(x, w, false);
   } else if (steady) {
     if (M >= 192 && M <= 256 && N % 64 == 0 && N > 4096 && N <= 6144 && K > 2048 && K <= 4096 &&
         !left_to_library(M))
       return skinny_gemm3_ex(x.contiguous(), w, 384);
-  } else if (block_rows_win(M, N, K)) {
+  } else if (block_rows_win(M, N, K, form == PARTS)) {
     return block_rows(x, w, form == PARTS);
   }
   return {};

@@ -91,12 +91,33 @@ def test_blocks_of_rows(m, n, k):
     _check((y.sum(0) if y.dim() == 3 else y).bfloat16(), want)
 
 
+@pytest.mark.parametrize("m", [129, 192, 300])
+def test_blocks_whose_steps_do_not_divide(m):
+    """44 steps in 15 parts of three and less, where 16 were asked for."""
+    x, w = _inputs(m, 512, 44 * 64)
+    y = ops.linear_parts(x, w)
+    assert y.dim() == 3 and y.shape[0] >= 5
+    _check(y.sum(0).bfloat16(), x.double() @ w.double().t())
+
+
+@pytest.mark.parametrize("m,n,experts,parts", [(256, 4096, False, True), (257, 4096, False, False),
+                                               (257, 4096, True, True), (300, 2048, False, True),
+                                               (300, 2064, False, False)])
+def test_parts_that_a_norm_holds(m, n, experts, parts):
+    x, w = _inputs(m, n, 14336)
+    assert ops.linear_parts(x, w).dim() == 3
+    y = ops.linear_norm_parts(x, w, experts)
+    assert (y.dim() == 3) == parts
+    _check((y.sum(0) if parts else y).bfloat16(), x.double() @ w.double().t())
+
+
 @pytest.mark.parametrize("m,n,k,own", [
-    (512, 4096, 4096, True), (1000, 2048, 576, True), (1000, 512, 576, True),
+    (512, 4096, 4096, False), (512, 3584, 2048, True), (256, 8192, 4096, True),
+    (1000, 2048, 576, True), (1000, 512, 576, True),
     (513, 4096, 640, False), (1001, 2048, 576, False), (300, 504, 1024, False),
     (300, 1024, 512, True), (300, 1456, 512, False), (300, 2824, 256, True), (128, 8192, 64, True),
-    (129, 64, 320, True), (128, 56, 256, False), (65, 2816, 2048, True), (65, 2816, 2112, False),
-    (100, 2808, 576, False), (128, 8192, 1024, True), (64, 64, 64, True)])
+    (129, 64, 320, True), (128, 56, 256, False), (65, 2560, 2048, True), (65, 2560, 2112, False),
+    (100, 2552, 576, False), (128, 8192, 1024, True), (64, 64, 64, True)])
 def test_line_to_the_library(m, n, k, own):
     x, w = _inputs(m, n, k)
     got = ops._hip.own_product(x, w, 0)
