@@ -531,8 +531,14 @@ static Cut block_cut(long M, long N, long K, bool raw) {
   return best;
 }
 
-// K's parts of block_rows
-long block_parts(long M, long N, long K, bool raw) { return block_cut(M, N, K, raw).parts; }
+// How block_rows takes a product: 2 with K cut, 1 whole in one round of workgroups in which the
+// blocks of a tile of W lie on one or two XCDs, else 0.
+int block_form(long M, long N, long K, bool raw) {
+  const Cut cut = block_cut(M, N, K, raw);
+  if (cut.parts > 1) return 2;
+  const long across = (N + cut.width - 1) / cut.width, blocks = (M + cut.rows - 1) / cut.rows;
+  return across * blocks <= 256 && across % 4 == 0;
+}
 
 // linear_few_rows of more rows
 torch::Tensor block_rows(torch::Tensor x, torch::Tensor w, bool raw) {

@@ -10,7 +10,7 @@
 torch::Tensor linear_few_rows(torch::Tensor x, torch::Tensor w, bool raw, bool steady);
 torch::Tensor silu_few_rows(torch::Tensor x, torch::Tensor w);
 torch::Tensor block_rows(torch::Tensor x, torch::Tensor w, bool raw);
-long block_parts(long M, long N, long K, bool raw);
+int block_form(long M, long N, long K, bool raw);
 bool one_row_fits(long S, long K);
 bool float_few_rows_fits(long N, long K);
 torch::Tensor float_few_rows(torch::Tensor x, torch::Tensor w);
@@ -149,10 +149,12 @@ static bool left_to_library(long M) {
 // for (a text of 200 tokens 1197 us and 612). The line is work for a quarter of the chip, in tiles
 // of 128 x 256: beyond it both come to the same by themselves (with the norm 520 rows of 4096 x
 // 4096 39 and 36, of 4096 x 14336 111 and 111, 768 of 3584 x 14336 113 and 127) and four layers of
-// 4096, 520 rows, took 1647 and 1746 us. In front of it, more than 256 rows whose long K is not
-// cut, or is for a reader who does not add the parts up, come to 0.98 of the library's time and to
-// 1.16 where its tiles come out even (512 rows of 2816 x 5632 33.6 and 37.5, 1000 of 1536 x 5632
-// 32.4 and 37.7), so those are left to it too. Of 3084 sizes within the lines ours takes 0.83 of
+// 4096, 520 rows, took 1647 and 1746 us. In front of it, more than 256 rows of K 2560 to 8192 take
+// as long as the library's where they come whole in one round of workgroups with a tile's blocks
+// on one or two XCDs (0.86 to 1.09, mean of 348 sizes 1.00; 512 rows of 4096 x 4096 28.5 and 29.5
+// us); on four XCDs 1.03 times as long, on eight 1.10, in more rounds 1.11 (512 rows of 2816 x 5632
+// 37.5 and 33.6, 1000 of 1536 x 5632 37.7 and 32.4). Cut for a reader who does not add the parts
+// up they take 1.00 to K 6144 and 0.96 beyond. Of 3084 sizes within the lines ours takes 0.83 of
 // the library's time whole, 0.79 with the norm. What falls behind by more than 4% are whole
 // products of 512 to 1536 outputs, K of 1400 to 3100 (10 us where the library takes 9, and the
 // host 20: 512 x 1408 8.5 and 9.1, 1408 x 2816, 140 rows, 9.8 and 11.3, 768 x 3072, 300 rows, 10.0
@@ -166,16 +168,19 @@ static bool left_to_library(long M) {
 //   768    9.6 6.2, 9.9 6.3, 10 6.6    9.6 6.4, 10 6.4, 10 6.7     10 6.6, 10 6.8, 11 7.1
 //   1408   9.7 8.9, 10 9.0, 15 9.3     9.6 9.1, 10 9.1, 15 9.6     11 9.7, 11 9.8, 16 10
 //   2048   12 11, 13 11, 15 11         12 11, 13 12, 15 12         14 13, 14 13, 16 13
-// and K up to 512 256 x 256 9.2 3.8, 8.4 3.5, 7.9 3.6, 4096 x 256 5.8 3.9, 6.1 4.2, 6.8 4.3, 1024 x
+// where ours is ahead from 2816 outputs on at every K. (Fewer, down to 2304, are even at 1408 and
+// ahead beside it; 1024 falls behind there.)
+// K up to 512: 256 x 256 9.2 3.8, 8.4 3.5, 7.9 3.6, 4096 x 256 5.8 3.9, 6.1 4.2, 6.8 4.3, 1024 x
 // 512 7.3 4.7, 6.5 4.5, 7.7 4.5 (65, 100 and 128 rows).
 static bool block_rows_win(long M, long N, long K, bool parts) {
   if (left_to_library(M)) return false;
-  if (M <= 128) return N <= 8192 && (K <= 512 ? N >= 64 : K <= 2048 && N >= 2560);
+  if (M <= 128) return N <= 8192 && (K <= 512 ? N >= 64 : K <= 2048 && N >= 2816);
   const long work = (M + 127) / 128 * N / 256;  // (a little more, many_rows takes)
   if (K <= 512) return M <= 1000 && N >= 64 && work <= (K <= 256 ? 40 : 16);
   if (M > 1000 || N < 512 || (M + 127) / 128 * N > 64 * 256) return false;
-  return M <= 256 || K <= 2048 || work < 44 ||
-         ((parts || K > 8192) && block_parts(M, N, K, parts) > 1);
+  if (M <= 256 || K <= 2048 || work < 44) return true;
+  const int form = block_form(M, N, K, parts);
+  return form == 1 || (form == 2 && (parts || K > 8192));
 }
 
 // x @ w^T in ``form``, or nothing: the library's product serves better or is followed by

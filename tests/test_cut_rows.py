@@ -112,18 +112,28 @@ def test_parts_that_a_norm_holds(m, n, experts, parts):
 
 
 @pytest.mark.parametrize("m,n,k,own", [
-    (512, 4096, 4096, False), (512, 3584, 2048, True), (256, 8192, 4096, True),
-    (1000, 2048, 576, True), (1000, 512, 576, True),
+    (512, 4096, 4096, True), (1000, 2048, 576, True), (1000, 512, 576, True),
     (513, 4096, 640, False), (1001, 2048, 576, False), (300, 504, 1024, False),
     (300, 1024, 512, True), (300, 1456, 512, False), (300, 2824, 256, True), (128, 8192, 64, True),
-    (129, 64, 320, True), (128, 56, 256, False), (65, 2560, 2048, True), (65, 2560, 2112, False),
-    (100, 2552, 576, False), (128, 8192, 1024, True), (64, 64, 64, True)])
+    (129, 64, 320, True), (128, 56, 256, False), (65, 2816, 2048, True), (65, 2816, 2112, False),
+    (100, 2808, 576, False), (128, 8192, 1024, True), (64, 64, 64, True)])
 def test_line_to_the_library(m, n, k, own):
     x, w = _inputs(m, n, k)
     got = ops._hip.own_product(x, w, 0)
     assert (got is not None) == own
     strided = torch.cat([x, x], 1)[:, :k]  # rows apart
     _check(ops.linear(strided, w), x.double() @ w.double().t())
+
+
+@pytest.mark.parametrize("m,n,k,own", [
+    (512, 3584, 2048, True), (512, 2816, 4096, False), (512, 2816, 2048, True),
+    (384, 3584, 4096, True), (512, 3328, 4096, False), (512, 3584, 4096, True),
+    (300, 4608, 3584, False), (1000, 1536, 5632, False), (256, 8192, 4096, True)])
+def test_line_of_long_rows(m, n, k, own):
+    """Workgroups of one round and more, blocks of a tile on few XCDs and many."""
+    x, w = _inputs(m, n, k)
+    assert (ops._hip.own_product(x, w, 0) is not None) == own
+    _check(ops.linear(x, w), x.double() @ w.double().t())
 
 
 @pytest.mark.parametrize("m", [2, 33, 65, 128])

@@ -105,8 +105,24 @@ def test_idle_rows(idle, dtype):
 
 
 @pytest.mark.gpu
+def test_refused_forms_run_as_two():
+    """Widths, pages and layouts without a form."""
+    args = dict(parts=0, biased=False, dtype=torch.bfloat16, dev="cuda")
+    for D, page in ((96, 32), (64, 16)):
+        qkv, bias, at, slots, cs, kc, vc, bt, ctx = _case(3, [5, 9, 14], 4, 2, D, **args)
+        kc, vc = (c.reshape(-1, 2, page, D).contiguous() if page == 32 else
+                  c[:, :, :page].contiguous() for c in (kc, vc))
+        slots = bt[:, 0] * page + ctx - 1
+        assert ops._hip.fresh_attention_decode(qkv, bias, cs, kc, vc, bt, ctx, 4, 0.1,
+                                               None) is None
+        if D == 64:
+            out = ops.fresh_attention_decode(qkv, bias, at, slots, cs, kc, vc, bt, ctx, 4, 0.1)
+            assert torch.isfinite(out).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,page", [(64, 16), (128, 16)])
-def test_refused_forms_run_as_two(D, page):
+def test_refused_pages(D, page):
     """Pages without a form: the reference's results and cache."""
     qkv, bias, at, slots, cs, kc, vc, bt, ctx = _case(3, [5, 9, 14], 4, 2, D, 0, True,
                                                       torch.bfloat16, "cuda")
@@ -122,13 +138,6 @@ def test_refused_forms_run_as_two(D, page):
         got, held = got.float().cpu(), held.float()
         assert ((got - held).abs() <= 2 ** -7 * held.abs() + 1e-6).all()
     assert ((out - want).abs() <= 2 ** -6 * host[6].float().abs().max()).all()
-
-
-@pytest.mark.gpu
-def test_refused_width():
-    qkv, bias, _, _, cs, kc, vc, bt, ctx = _case(3, [5, 9, 14], 4, 2, 96, 0, True, torch.bfloat16,
-                                                 "cuda")
-    assert ops._hip.fresh_attention_decode(qkv, bias, cs, kc, vc, bt, ctx, 4, 0.1, None) is None
 
 
 def test_reference():
