@@ -17,7 +17,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from .. import ops
-from ..parallel.tp import is_plain
+from ..parallel.tp import is_method, is_plain
 from .config import ModelSpec, get_spec
 
 
@@ -134,10 +134,15 @@ class SentenceEncoder(nn.Module):
         in_order = maxp <= TURNED_TOKENS or max(map(len, batches), default=0) <= TURNED_TOKENS
         x = self.embed(ids)
         delta = None
-        plain = [is_plain(layer, EncoderLayer) for layer in self.layers] + [True]
+        plain = [is_plain(layer, EncoderLayer) for layer in self.layers]
+        # a step of a user's own knows nothing of parts: it neither is asked for them nor gets them
+        known = [a and is_method(layer, EncoderLayer, "step")
+                 for a, layer in zip(plain, self.layers)] + [True]
         for i, layer in enumerate(self.layers):
-            if plain[i]:
-                x, delta = layer.step(x, delta, self.cos_sin, pos_t, cu_t, in_order, plain[i + 1])
+            if known[i]:
+                x, delta = layer.step(x, delta, self.cos_sin, pos_t, cu_t, in_order, known[i + 1])
+            elif plain[i]:
+                x, delta = layer.step(x, delta, self.cos_sin, pos_t, cu_t, in_order)
             else:  # somebody watches it or has replaced it
                 x, delta = x if delta is None else x + delta, None
                 x = layer(x, self.cos_sin, pos_t, cu_t)

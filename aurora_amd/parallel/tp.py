@@ -37,15 +37,19 @@ def is_plain(module: nn.Module, kind: type) -> bool:
                 or _global_backward_hooks or _global_backward_pre_hooks)
 
 
+def is_method(module: nn.Module, kind: type, name: str) -> bool:
+    """True where ``module``'s method of a name is ``kind``'s, not its own or a subclass's."""
+    return (name not in module.__dict__
+            and getattr(type(module), name, None) is getattr(kind, name))
+
+
 def told(m: nn.Module, x, kind: type, steady: bool, name: str = "") -> torch.Tensor:
     """``m(x)``, or its method ``name`` of x, which is told ``steady`` (see ``ops.linear``) where
     it is ``kind``'s, whoever watches it; one of a user's own is given what it always was."""
     step = getattr(m, name) if name else m
-    if not steady:
-        return step(x)
-    at = name or "forward"
-    own = at in m.__dict__ or getattr(type(m), at, None) is not getattr(kind, at)
-    return step(x) if own else step(x, steady=True)
+    if steady and is_method(m, kind, name or "forward"):
+        return step(x, steady=True)
+    return step(x)
 
 
 class ColumnParallelLinear(nn.Module):
