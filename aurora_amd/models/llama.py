@@ -32,6 +32,7 @@ from ..parallel.tp import (
     column_parts,
     column_silu_mul,
     column_weight,
+    is_method,
     is_plain,
     row,
     row_parts,
@@ -319,9 +320,10 @@ class MoEMLP(nn.Module):
         weights = weights.softmax(-1).to(x.dtype)  # [T, k]
         if self.ep_size > 1:
             from ..parallel import ep as pep
-            return pep.ep_moe_forward(x, weights, sel, self.n_experts,
-                                      partial(self._local_expert_fn, steady=True) if steady
-                                      else self._local_expert_fn)
+            local = self._local_expert_fn
+            if steady and is_method(self, MoEMLP, "_local_expert_fn"):
+                local = partial(local, steady=True)
+            return pep.ep_moe_forward(x, weights, sel, self.n_experts, local)
         if T <= 256:
             return self._forward_batched(x, weights, sel)
         # prefill: per-expert token batches are large, so plain per-expert

@@ -2,7 +2,10 @@
 import pytest
 import torch
 
+from aurora_amd.models.config import ModelSpec
 from aurora_amd.models.encoder import EncoderLayer, SentenceEncoder
+from aurora_amd.models.llama import MoEMLP
+from aurora_amd.parallel import ep
 
 DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
 
@@ -51,3 +54,23 @@ def _as(layer):
     other = _Step.__new__(_Step)
     other.__dict__ = {k: v for k, v in layer.__dict__.items() if k != "step"}
     return other
+
+
+class _Experts(MoEMLP):
+    def _local_expert_fn(self, xp, local_sel):
+        return xp * 2
+
+
+@pytest.mark.parametrize("kind", [_Experts, MoEMLP])
+@pytest.mark.parametrize("steady", [False, True])
+def test_local_experts(kind, steady, monkeypatch):
+    spec = ModelSpec(name="t", vocab_size=64, hidden_size=64, n_layers=1, n_heads=1, n_kv_heads=1,
+                     head_dim=64, intermediate_size=64, n_experts=4)
+    monkeypatch.setattr(ep, "ep_size", lambda: 2)
+    monkeypatch.setattr(ep, "ep_moe_forward", lambda x, w, sel, n, fn: fn(x, sel[:, 0] % 2))
+    m = kind(spec, torch.float32)
+    for p in m.parameters():
+        torch.nn.init.normal_(p, std=0.1, generator=torch.Generator().manual_seed(0))
+    x = torch.randn(5, 64, generator=torch.Generator().manual_seed(1))
+    y = m(x, steady=True) if steady else m(x)
+    assert torch.equal(y, x * 2) == (kind is _Experts) and torch.equal(y, m(x))
