@@ -269,9 +269,11 @@ bool rotates_by_eight(long T, long width);  // defined in elementwise.hip
 // new key and value, which it writes to the cache and takes from LDS where the cache would still
 // have what was there before. While parts and rotations are on their way so are its first keys.
 // After a kernel of its own for that and with it in here, 32 heads over 8, us: one sequence of
-// 777, 128 wide, 12.0 and 10.1; 8 of 300 to 1500 17.2 and 14.7; 96 of 500 to 2900 125.3 and
-// 123.2; 41 of 700 to 2600 71.0 and 68.7; 23 of 300 to 5000 in fp8 48.3 and 45.5, 64 wide 27.1
-// and 25.0.
+// 777, 128 wide, 12.0 and 10.1; 8 of 300 to 1500 17.2 and 14.7; 41 of 700 to 2600 71.0 and 68.7;
+// 23 of 300 to 5000 in fp8 48.3 and 45.5, 64 wide 27.1 and 25.0. Where whole contexts fill the chip
+// the work takes as long here (96 of 500 to 2900 124.5 and 4.8, in one 129.2) and what goes is the
+// launch between: captured steps of 8 layers 4096 wide 2316 and 2302, 64 sequences 1998 and
+// 1957, 128 of 300 to 1500 2247 and 2230, in fp8 1950 and 1901.
 // (Four columns and partners a lane in all waves, with 64-bit addresses, gave half of that.)
 template <int D, int DV, bool FP8, int BIAS, bool PAGED, bool CUT, int FRESH = 0>
 __global__ __launch_bounds__(256, FRESH && D == 64 ? 4 : 2) void paged_decode_kernel(
